@@ -46,7 +46,7 @@ KERNEL_SOURCES = {
     "paged_decode_latent16_kernel": ["decode_wide.hip", "decode_common.h", "common.h"],
     "paged_decode_latent128_kernel": ["decode_wide.hip", "gen_latent_frag.py", "decode_common.h", "common.h"],
     "latent_prefill_kernel": ["decode_wide.hip", "gen_latent_frag.py", "decode_common.h", "common.h"],
-    "prefill_kernel": ["prefill.hip", "gen_prefill_stream.py", "common.h"],
+    "prefill_stream_kernel": ["prefill_stream.hip", "prefill_common.h", "gen_prefill_stream.py", "common.h"],
 }
 MEASURED_TRAFFIC = {
     # workload: (kernel, hash of its sources, HBM bytes per launch: FETCH_SIZE and WRITE_SIZE of the
@@ -55,7 +55,7 @@ MEASURED_TRAFFIC = {
     "config2": ("paged_decode_mfma16_kernel", "8ba1b647faebb44c", 310422335),
     "config5": ("paged_decode_mfma16_kernel", "8ba1b647faebb44c", 168457090),
     "config4": ("paged_decode_mfma16_kernel", "8ba1b647faebb44c", 3415575936),
-    "config3": ("prefill_kernel", "9e5dc9fce6518e7f", 244468287),
+    "config3": ("prefill_stream_kernel", "9e5dc9fce6518e7f", 244468287),
     "latent": ("paged_decode_latent16_kernel", "cb2ca9fa245030d1", 654198293),
     "latent128": ("paged_decode_latent128_kernel", "b26a62d6c1d0a108", 739381753),
     "latent-prefill": ("latent_prefill_kernel", "b26a62d6c1d0a108", 332193335),
@@ -643,10 +643,10 @@ def run_prefill(args):
         "tokens_per_s": w.users * w.seq / (ms * 1e-3),
         "fill_bytes_per_step": w.fill_bytes(),
         "roofline": {
-            "kernel": "prefill_kernel", "bound": "mfma", "achieved": achieved,
+            "kernel": "prefill_stream_kernel", "bound": "mfma", "achieved": achieved,
             "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
-            "frac": achieved / MFMA_BF16_PEAK_TFLOPS, "traffic": measured_traffic("config3", "prefill_kernel"),
-            "kernel_source_hash": kernel_source_hash("prefill_kernel"),
+            "frac": achieved / MFMA_BF16_PEAK_TFLOPS, "traffic": measured_traffic("config3", "prefill_stream_kernel"),
+            "kernel_source_hash": kernel_source_hash("prefill_stream_kernel"),
             "kernel_us": kern_ms * 1e3, "kernel_us_min": min(d for d, _ in durs) * 1e3,
             "flops_per_launch": flops, "timed_launches": len(durs),
             "note": "useful (causal) FLOPs only; the dense 4*B*Hq*S^2*D figure is twice this; the launch "

@@ -1,0 +1,50 @@
+"""The forms of the streaming prefill kernel (head size 128) at the sizes where they can go wrong:
+one, two and four query heads of a KV head per workgroup (row blocks of one workgroup that end at
+different keys, row blocks that do not exist), K / V of an odd number of 32-key blocks, sliding
+windows whose lower edge falls on, before and behind a block boundary.  Oracle and tolerance as in
+test_gpu_prefill.py."""
+
+import pytest
+import torch
+
+import test_gpu_prefill as P
+from oracle import paged_ops as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _pkg():
+    P.entry.ensure_built()
+    import tt_xla_amd  # noqa: F401
+
+
+@pytest.mark.parametrize("b,hq,hkv,s,window", [
+    (1, 1, 1, 32, 0), (2, 3, 3, 160, 0), (1, 5, 5, 288, 0),      # one head: 128 rows of it per workgroup
+    (1, 2, 1, 32, 0), (2, 6, 3, 96, 0), (1, 4, 2, 352, 0),       # two heads: 64 rows
+    (1, 4, 1, 32, 0), (2, 8, 2, 96, 0), (1, 4, 1, 416, 0),       # four heads: 32 rows, odd numbers of blocks
+    (1, 2, 2, 416, 31), (1, 2, 2, 416, 32), (1, 2, 2, 416, 33), (1, 3, 3, 288, 1), (2, 2, 2, 160, 200),
+    (1, 4, 2, 416, 64), (1, 6, 3, 224, 97), (1, 4, 1, 416, 65), (1, 8, 2, 288, 128),
+])
+def test_dense_forms(b, hq, hkv, s, window):
+    g = torch.Generator().manual_seed(b + hq + s + window)
+    q, k, v = P._bf(g, b, hq, s, 128), P._bf(g, b, hkv, s, 128), P._bf(g, b, hkv, s, 128)
+    want = O.sdpa_windowed(q, k, v, sliding_window=window) if window else O.sdpa(q, k, v, None, True, None)
+    got = torch.ops.tt.scaled_dot_product_attention(q.cuda(), k.cuda(), v.cuda(), is_causal=True,
+                                                    sliding_window_size=window or None)
+    P._check(f"dense b{b} h{hq}x{hkv} s{s} window{window}", got.cpu(), want)
+
+
+@pytest.mark.parametrize("hq,hkv,bs,start,lc", [
+    (3, 3, 64, 64, 130), (2, 1, 64, 192, 33), (4, 2, 128, 128, 200), (1, 1, 64, 0, 32), (10, 2, 64, 37, 129),
+])
+def test_paged_forms(hq, hkv, bs, start, lc):
+    g = torch.Generator().manual_seed(hq + bs + start)
+    users, nbpu = 2, -(-(start + lc) // bs) + 1
+    key, value, table = P._paged(g, users, nbpu, hkv, bs, 128, False)
+    q = P._bf(g, users, hq, lc, 128)
+    st = torch.tensor([start], dtype=torch.int32)
+    want = O.chunked_sdpa(q, key, value, table, st, 128**-0.5)
+    got = torch.ops.tt.chunked_scaled_dot_product_attention(
+        q.cuda(), key.cuda(), value.cuda(), table.cuda(), st.cuda(), 128**-0.5)
+    P._check(f"paged h{hq}x{hkv} bs{bs} start{start} len{lc}", got.cpu(), want)

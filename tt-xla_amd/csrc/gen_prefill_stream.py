@@ -1,7 +1,8 @@
 #!/usr/bin/env python3
-"""Writes the hand-scheduled loop of the prefill kernel (head size 128, four query heads of one KV
-head per workgroup, 32 query rows per wavefront, two workgroups per CU) as one block of gfx950
-assembly per K / V source: build/prefill_stream_asm.h, included by prefill.hip.
+"""Writes the hand-scheduled loop of the streaming prefill kernel (head size 128, 32 query rows of one
+head per wavefront, two workgroups of four wavefronts per CU) as one block of gfx950 assembly per
+form of the loop: build/prefill_stream_asm.h, included by prefill_stream.hip.  The forms: dense
+K / V, dense with a sliding window, paged K / V.
 
 Why assembly: the loop wants the matrix pipe and the vector ALU of a SIMD busy at the same time
 from one instruction stream, with every register chosen by hand (256 per wavefront at two
@@ -22,13 +23,17 @@ block reaches 2, which is one OR over the packed probabilities and one test of b
 bfloat16: p >= 2 exactly when the score exceeds the reference's maximum by 2^8, the lazy rule of
 the plain loop.  The block then takes the slow path at the end of the iteration: true row maximum,
 new reference, accumulators and row sum rescaled, probabilities of the block recomputed.  The first
-block of a row always does (the reference starts at -inf).
+block of a row always does: the reference starts at the lowest finite float, so that every real score
+lies above it by more than any exponent, while a masked one (-inf) still becomes a zero and not a NaN
+(a block may be masked for all keys of a row: wavefronts of one workgroup may hold different row
+blocks, and a window may start behind the first block).
 
 Masks: a lane holds the keys key0 + 4 h + {0..3, 8..11, 16..19, 24..27} of a block (h = lane / 32)
 for query row lane % 32, and may see keys up to its limit (causal diagonal, end of K / V).  Blocks
 from key `mask_from` on are masked in place, at the start of their iteration, before anything reads
 the scores: 16 compares of the key constants against limit - 4 h - key0 and 16 selects of -inf.
-Blocks in front of it skip that with one scalar branch.
+Blocks in front of it skip that with one scalar branch.  With a sliding window a lane also has a
+lowest key; blocks whose first key is below `low_to` are masked from below in the same way.
 
 LDS: a ring of NS slots of 8 KiB (32 rows) for K blocks and one for V blocks; block j lives in
 slot j % NS.  Iteration i reads K block i + 1 and V block i - 1 and, through the running fragment
@@ -50,7 +55,8 @@ d = k spg + (k even ? j : spg - 1 - j), as long as d < nqt.  Row blocks are deal
 alternating direction, so that with causal masking every workgroup gets about the same number of
 key blocks.  The launcher's default is one item per workgroup (spg = nqt: the hardware deals the
 workgroups as slots free up, which measured faster than one static round), several when the row
-blocks weigh the same and divide evenly over one round.  Per item the block does everything
+blocks weigh the same and divide evenly over one round.  (Only where the four wavefronts share their
+rows, and not with a window, whose row blocks start at different keys.)  Per item the block does everything
 between the Q fragments and the stored output rows: its first requests (K blocks 0..NS-1, V blocks
 0..NS-3; for the first item they are a block of assembly of their own, so that the caller's Q loads
 overlap them), all blocks, the last PV, normalisation and store; then the next item's Q fragments
@@ -80,12 +86,13 @@ MC, LRUN, LSUM, ALPHA = 196, 197, 198, 199   # MC, LRUN: inputs / outputs
 T = [200, 201, 202, 203]
 ORV, MLOC, MB, MCN = 204, 205, 206, 207
 PTREQ = 208                    # paged: the requested block-table entry (input)
+LOWEST, LOWREL = 209, 210      # window: first visible key of the lane's row, minus 4 h (input); relative to the block
 LIMIT = 212                    # last visible key of the lane's row, minus 4 h (input)
 LIMREL, NEGINF, VZERO = 213, 214, 215
 QBASE, OUTBASE = 216, 218      # per lane, 64-bit: q / out of row 0 of the lane's head, at the lane's 8 h / 4 h elements (inputs)
 VN, V4H = 220, 221             # lane % 32 and 4 (lane / 32) (inputs)
 OUTP, PTMP, VT0, VROW = 222, 224, 226, 227
-CLOBBERED = (list(range(0, QF)) + list(range(S[0], RING + 4 * NSLOT)) + list(range(MC, MCN + 1)) + [209, 210, 211, LIMIT, LIMREL, NEGINF, VZERO]
+CLOBBERED = (list(range(0, QF)) + list(range(S[0], RING + 4 * NSLOT)) + list(range(MC, MCN + 1)) + [LOWREL, 211, LIMIT, LIMREL, NEGINF, VZERO]
              + list(range(OUTP, VROW + 1)))
 
 # ---- scalar registers ---------------------------------------------------------------------------
@@ -98,7 +105,8 @@ S_KLEFT = "s71"                # K blocks left to request
 S_M0B = "s72"                  # LDS address of this wavefront's first 1 KiB segment in K slot 0
 S_VLEFT = "s73"                # V blocks left to request
 S_MASKFROM = "s74"             # blocks whose first key is >= this are masked
-S_KEY0 = "s75"                 # first key of the block whose softmax comes next
+S_KEY0 = "s75"                 # first key of the block whose softmax comes next (input: of the first block)
+S_LOWTO = "s34"                # window: blocks whose first key is < this are masked from below (input)
 # paged only
 S_HKV, S_HK, S_NCB, S_TPB = "s76", "s77", "s78", "s79"  # kv heads, this kv head, cache blocks, tiles per cache block
 S_CIN = "s80"                  # tile-in-cache-block index of the tile whose entry is read next
@@ -117,13 +125,25 @@ S_QTS, S_OTS = "s48", "s49"    # bytes from a query / output row to the next
 S_ROW0 = "s57"                 # first query row of the item
 S_STOREMASK = "s[60:61]"
 # temporaries s[88:95], s[62:63]
-SCALAR_CLOBBERS = [f"s{r}" for r in list(range(88, 96)) + [60, 61, 62, 63, 74, 75]]
+SCALAR_CLOBBERS = [f"s{r}" for r in list(range(88, 96)) + [60, 61, 62, 63, 74]]
 
 NS = 5                         # slots per ring
 UNROLL = 10                    # lcm(2, NS): score bank and slots repeat
 SLOT = 8192
 VRING = NS * SLOT              # LDS offset of the V ring; VOFF carries it
 KEY_CONST = [8 * (r // 4) + r % 4 for r in range(16)]
+
+
+class Form:
+    """What one block of assembly serves."""
+
+    def __init__(self, name, paged=False, window=False):
+        self.name, self.paged, self.window = name, paged, window
+        self.items = not window  # several row blocks in turn
+
+
+FORMS = [Form("DENSE"), Form("DENSE_WINDOW", window=True), Form("PAGED", paged=True)]
+START_REFERENCE = "0xff7fffff"  # the lowest finite float
 
 
 class Out:
@@ -240,22 +260,32 @@ def iteration_pairs(p, has_pv=True):
     return pairs
 
 
-def mask_block(o, q, tag):
+def mask_block(o, f, q, tag):
     """Start of the iteration whose softmax reads bank q: masks the block in place if it needs it."""
     s = S[q]
+    if f.window:
+        o.e(f"s_cmp_lt_i32 {S_KEY0}, {S_LOWTO}")
+        o.e(f"s_cbranch_scc1 L_mask_{tag}%=")
     o.e(f"s_cmp_lt_i32 {S_KEY0}, {S_MASKFROM}")
     o.e(f"s_cbranch_scc1 L_nomask_{tag}%=")
+    if f.window:
+        o.label(f"L_mask_{tag}")
     o.e("s_nop 15")  # the last matrix instruction into this bank has written
     o.e(f"v_subrev_u32 v{LIMREL}, {S_KEY0}, v{LIMIT}")  # limit - 4 h - key0
     o.e(f"v_mov_b32 v{NEGINF}, 0xff800000")
     sel = lambda r: f"v_cndmask_b32_e64 v{s + r}, v{s + r}, v{NEGINF}, s[{88 + 2 * (r % 4)}:{89 + 2 * (r % 4)}]"
-    for r in range(16):
-        o.e(f"v_cmp_gt_i32_e64 s[{88 + 2 * (r % 4)}:{89 + 2 * (r % 4)}], {KEY_CONST[r]}, v{LIMREL}")
-        if r >= 3:  # a select reads its mask three instructions after the compare that wrote it
-            o.e(sel(r - 3))
-    o.e("s_nop 1")
-    for r in range(13, 16):
-        o.e(sel(r))
+    sides = [("v_cmp_gt_i32_e64", LIMREL)]
+    if f.window:
+        o.e(f"v_subrev_u32 v{LOWREL}, {S_KEY0}, v{LOWEST}")
+        sides.append(("v_cmp_lt_i32_e64", LOWREL))
+    for compare, bound in sides:
+        for r in range(16):
+            o.e(f"{compare} s[{88 + 2 * (r % 4)}:{89 + 2 * (r % 4)}], {KEY_CONST[r]}, v{bound}")
+            if r >= 3:  # a select reads its mask three instructions after the compare that wrote it
+                o.e(sel(r - 3))
+        o.e("s_nop 1")
+        for r in range(13, 16):
+            o.e(sel(r))
     o.label(f"L_nomask_{tag}")
     o.e(f"s_add_u32 {S_KEY0}, {S_KEY0}, 32")
 
@@ -357,9 +387,10 @@ def next_tile(o, tag):
     o.label(f"L_noreq_{tag}")
 
 
-def iteration_head(o, p, tag, paged):
+def iteration_head(o, f, p, tag):
     """Mask, barrier and requests of iteration i = p (mod UNROLL)."""
-    mask_block(o, p % 2, tag)
+    paged = f.paged
+    mask_block(o, f, p % 2, tag)
     # requests of the last two barriers may stay in flight, unless some were skipped
     o.e(f"s_cmp_eq_u32 {S_KLEFT}, 0")
     o.e(f"s_cbranch_scc1 L_all_{tag}%=")
@@ -410,8 +441,9 @@ def item_setup(o, tag):
     o.label(f"L_causal_{tag}")
     o.e(f"v_sub_u32 v{LIMIT}, v{VT0}, v{V4H}")
     o.e(f"s_sub_u32 {S_MASKFROM}, s88, 30")
-    o.e(f"s_mov_b32 {S_KEY0}, 0")
-    o.e(f"v_mov_b32 v{MC}, 0xff800000")
+    if tag != "first":  # (several row blocks in turn: all of them start at key 0)
+        o.e(f"s_mov_b32 {S_KEY0}, 0")
+    o.e(f"v_mov_b32 v{MC}, {START_REFERENCE}")
     o.e(f"v_mov_b32 v{LRUN}, 0")
     for r in range(64):
         o.e(f"v_mov_b32 v{r}, 0")
@@ -555,7 +587,7 @@ def generate_first(paged, suffix=""):
     return o.lines
 
 
-def generate(paged):
+def generate(f):
     o = Out()
     assert NS == 5 and UNROLL == 10
     o.e(f"v_mov_b32 v{VZERO}, 0")
@@ -569,14 +601,14 @@ def generate(paged):
     stream(o, pairs, [[] for _ in pairs], False, [f for _, f in it0])
     # ---- iteration 0: S(1), sm(0) ---------------------------------------------------------------
     o.e("s_nop 7")
-    iteration_head(o, 0, "i0", paged)
+    iteration_head(o, f, 0, "i0")
     stream(o, it0, spread(softmax_ops(0), 8), True, first_frags(1))
     iteration_tail(o, "i0", "L_exit0")
     # ---- iterations 1 .. : ten in a row, then round again -------------------------------------------
     for k in range(UNROLL):
         p = (k + 1) % UNROLL
         o.label(f"L_it{p}")
-        iteration_head(o, p, f"p{p}", paged)
+        iteration_head(o, f, p, f"p{p}")
         stream(o, iteration_pairs(p), spread(softmax_ops(p % 2), 16), True, first_frags(p + 1))
         iteration_tail(o, f"p{p}", f"L_exit{p}")
     o.e("s_branch L_it1%=")
@@ -604,7 +636,10 @@ def generate(paged):
     o.label("L_end")
     o.e("s_nop 15")
     o.e("s_nop 15")
-    next_item(o, paged)
+    if f.items:
+        next_item(o, f.paged)
+    else:
+        epilogue(o)
     return o.lines
 
 
@@ -612,9 +647,9 @@ def main():
     out = sys.argv[1] if len(sys.argv) > 1 else "/dev/stdout"
     with open(out, "w") as f:
         f.write("// Generated by gen_prefill_stream.py; do not edit.\n#pragma once\n")
-        for name, paged in (("DENSE", False), ("PAGED", True)):
-            for macro, lines in ((f"TTPA_STREAM_FIRST_TEXT_{name}", generate_first(paged)),
-                                 (f"TTPA_STREAM_LOOP_TEXT_{name}", generate(paged))):
+        for form in FORMS:
+            for macro, lines in ((f"TTPA_STREAM_FIRST_TEXT_{form.name}", generate_first(form.paged)),
+                                 (f"TTPA_STREAM_LOOP_TEXT_{form.name}", generate(form))):
                 f.write(f"#define {macro} \\\n")
                 for ln in lines:
                     f.write(f'  "{ln}\\n\\t" \\\n')

@@ -23,84 +23,13 @@
 // unpadded in LDS; bank conflicts are avoided by an XOR swizzle of the 16-byte chunk
 // position inside a row, applied on the global side (which chunk a lane fetches) and again
 // when fragments are read.
-#include "common.h"
-#include "build/prefill_stream_asm.h"
+#include "prefill_common.h"
 
 #include <algorithm>
 #include <cstdlib>
 
 namespace ttpa {
 namespace {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef short shortx4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-constexpr int kKeysPerTile = 64;
-constexpr int kRowsPerWave = 32;
-
-struct PrefillArgs {
-  uint16_t *out;
-  int64_t out_bs, out_hs, out_ts;
-  const uint16_t *q;
-  int64_t q_bs, q_hs, q_ts;
-  const uint16_t *k, *v;
-  int64_t kv_bs, kv_hs, kv_ts;  // dense form
-  const int32_t *pt;            // paged form when non-null
-  int64_t pt_rs;
-  const int32_t *chunk_start;
-  const uint16_t *mask;
-  int64_t mask_bs, mask_rs;
-  int batch, hq, hkv, sq, skv, bs, w, nb, causal;
-  uint32_t bs_magic;  // floor(2^32 / bs) + 1: key / bs = mulhi(key, bs_magic) while key * bs < 2^32 (bs >= 2)
-  // Dense form with a cache fill in the same launch (fill_kc != null): k / v are also written
-  // to the paged caches through fill_pt, by workgroups n_attn ... of the grid.  bs / nb /
-  // bs_magic describe the caches; table row of batch entry i = fill_bidx[i] (or i == 0).
-  uint16_t *fill_kc, *fill_vc;
-  const int32_t *fill_pt;
-  int64_t fill_pt_rs;
-  const void *fill_bidx;
-  int fill_bidx_i64, fill_rows;
-  // Grid layout with a fill: fill_groups super-groups of (8 * attn_per_fill attention
-  // workgroups, then 8 fill workgroups), then the remaining attention workgroups.  Groups of 8
-  // keep an attention workgroup's index congruent to its hardware index modulo 8 (its XCD).
-  int fill_groups, attn_per_fill, n_fill;
-  int window;  // > 0 (causal only): row i attends keys offset + i - window < j <= offset + i
-  float scale_log2e;
-  int kv_bfp8;  // paged form: the caches are block-float-8 (mode 4, or expanded into `expand` first)
-  void *expand; // scratch for bfloat16 copies of the block-float-8 blocks of this pass, or null
-  int stream;   // the hand-scheduled loop serves this launch (head size 128, 4 heads per workgroup, whole blocks)
-  int spg;      // ... with this many workgroups per (batch entry, head group), each taking several row blocks
-  int spg_even; // > 0: when the row blocks weigh about the same, only this many of them work (equal shares)
-};
-
-// key / block_size without a division instruction sequence (about 30 instructions each, and the
-// paged tile loads need several per tile).
-__device__ __forceinline__ int div_block(const PrefillArgs &a, int key) {
-  return a.bs == 1 ? key : (int)__umulhi((uint32_t)key, a.bs_magic);
-}
-
-// LDS geometry of one stage: the K tile (64 rows of D elements) followed by the V tile.
-// Chunk c (16 bytes) of row r is stored at chunk position c ^ swz(r).
-//   K fragments are read by 16 lanes of consecutive rows at one logical chunk: the 16
-//   positions must differ (rows of >= 256 bytes) or, for 128-byte rows, differ within each
-//   pair of rows that shares a 256-byte bank line.
-//   V fragments are read, per 32 lanes, as 4 consecutive rows x 4 consecutive chunks.
-template <int D>
-struct Tile {
-  static constexpr int RB = 2 * D;                 // row bytes
-  static constexpr int CPR = D / 8;                // 16-byte chunks per row
-  static constexpr int RPI = 1024 / RB;            // rows covered by one wavefront load
-  static constexpr int NI = kKeysPerTile / RPI / 4;  // loads per wavefront per tile and tensor
-  static constexpr int TILE_BYTES = kKeysPerTile * RB;
-  static constexpr int STAGE_BYTES = 2 * TILE_BYTES;
-  __device__ static constexpr int swz_k(int r) { return RB >= 256 ? (r & 15) : ((r >> 1) & 7); }
-  __device__ static constexpr int swz_v(int r) { return RB >= 256 ? 4 * (r & 3) : 4 * ((r >> 1) & 1); }
-};
 
 // v_max3_f32 without the input canonicalisation the compiler adds around fmaxf (scores are
 // never signalling NaNs).  Callers order it after a compiler-visible read of the matrix
@@ -109,54 +38,6 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
   float d;
   asm("v_max3_f32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
   return d;
-}
-
-// The cache fill that rides along with a dense prefill: workgroup f (counted from the end of
-// the attention workgroups) copies fill_rows_per_wg(D) token rows (128 KiB) of one (tensor, batch entry, KV head)
-// from the dense K / V operand into the paged cache, with the semantics of the fill operator
-// (rows whose table row or block is out of range are skipped).  Pure memory work that runs in
-// the shadow of the matrix-bound attention workgroups; nothing in this launch reads the caches.
-constexpr int kFillPasses = 32;  // 16-byte loads in flight per thread
-constexpr int fill_rows_per_wg(int d) { return kFillPasses * (256 / (d / 8)); }
-
-template <int D>
-__device__ __forceinline__ void fill_workgroup(const PrefillArgs &a, int f) {
-  constexpr int CPR = D / 8;        // 16-byte chunks per row
-  constexpr int RPP = 256 / CPR;    // rows per pass of the 256 threads
-  constexpr int NP = kFillPasses;
-  constexpr int kFillRows = fill_rows_per_wg(D);
-  const int chunks = (a.skv + kFillRows - 1) / kFillRows;
-  const int c0 = f % chunks;
-  int r = f / chunks;
-  const int h = r % a.hkv;
-  r /= a.hkv;
-  const int b = r % a.batch;
-  const bool is_v = r / a.batch != 0;
-  int64_t row = a.fill_bidx ? load_index(a.fill_bidx, a.fill_bidx_i64, b) : 0;
-  if (row < 0 || row >= a.fill_rows) return;
-  const uint16_t *src = (is_v ? a.v : a.k) + b * a.kv_bs + h * a.kv_hs;
-  uint16_t *cache = is_v ? a.fill_vc : a.fill_kc;
-  const int32_t *pt = a.fill_pt + row * a.fill_pt_rs;
-  const int t0 = c0 * kFillRows + (int)threadIdx.x / CPR, c = (int)threadIdx.x % CPR;
-  // every load (rows and table entries) is requested before the first store: the compiler
-  // cannot move a load across a store that might alias it, and a table entry per pass would
-  // otherwise cost a round trip each
-  u32x4 val[NP];
-  int phys[NP];
-#pragma unroll
-  for (int p = 0; p < NP; ++p) {
-    const int t = min(t0 + p * RPP, a.skv - 1);
-    val[p] = *reinterpret_cast<const u32x4 *>(src + (int64_t)t * a.kv_ts + 8 * c);
-    phys[p] = pt[div_block(a, t)];
-  }
-#pragma unroll
-  for (int p = 0; p < NP; ++p) {
-    const int t = t0 + p * RPP;
-    const int off = t - div_block(a, t) * a.bs;
-    // (no early exit from the loop: the arrays must stay in registers)
-    if (t < a.skv && (unsigned)phys[p] < (unsigned)a.nb)
-      __builtin_nontemporal_store(val[p], reinterpret_cast<u32x4 *>(cache + (((int64_t)phys[p] * a.hkv + h) * a.bs + off) * D + 8 * c));
-  }
 }
 
 // Expansion of the block-float-8 blocks a chunk pass reads into bfloat16 copies, so that the
@@ -211,102 +92,6 @@ __global__ __launch_bounds__(256) void bfp8_expand_kernel(ExpandArgs e) {
   }
 }
 
-// ---------------------------------------------------------------------------------------------
-// The hand-scheduled loop over whole unmasked tiles (head size 128, 32 rows per wavefront): one
-// block of assembly, written by gen_prefill_stream.py, which documents the schedule and the
-// state on entry and exit.  Everything the block touches is bound to the registers its text
-// names; the compiler moves values in and out around it and keeps its own out of the clobbered
-// ones.  Entered with K(0), V(0), K(1) requested and K(0) published; handles tiles 0 .. n - 1.
-typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x16 __attribute__((ext_vector_type(16)));
-
-// The requests of a workgroup's first blocks are a block of assembly of their own, issued in front
-// of the Q loads so that the two round trips to memory overlap.  (Scalars only: with the per-lane
-// offsets in the same struct the compiler keeps the whole of it in vector registers.)
-struct StreamRequests {
-  uint64_t kbase, vbase;       // dense: block 0 of K / V; paged: the caches (both minus 1024 bytes)
-  uint32_t stride;             // dense: bytes from a 32-key block to the next; paged: bytes of a (cache block, head) slab
-  uint32_t m0_base;            // LDS address of the wavefront's first segment in K slot 0
-  int k_requests, v_requests;  // blocks not requested yet
-  uint64_t off0, off1, off2;   // paged: byte offsets of tiles 0, 1, 2 in a cache
-};
-
-__device__ __forceinline__ void stream_first_dense(StreamRequests &r, const u32x2 &ldk, const u32x2 &ldv) {
-  asm volatile(TTPA_STREAM_FIRST_TEXT_DENSE
-               : "+{s[64:65]}"(r.kbase), "+{s[66:67]}"(r.vbase), "+{s71}"(r.k_requests), "+{s73}"(r.v_requests)
-               : "{v[188:189]}"(ldk), "{v[190:191]}"(ldv), "{s68}"(r.stride), "{s72}"(r.m0_base)
-               : "memory", "scc", "m0");
-}
-
-__device__ __forceinline__ void stream_first_paged(StreamRequests &r, const u32x2 &ldk, const u32x2 &ldv) {
-  asm volatile(TTPA_STREAM_FIRST_TEXT_PAGED
-               : "+{s71}"(r.k_requests), "+{s73}"(r.v_requests)
-               : "{v[188:189]}"(ldk), "{v[190:191]}"(ldv), "{s[64:65]}"(r.kbase), "{s[66:67]}"(r.vbase),
-                 "{s72}"(r.m0_base), "{s[84:85]}"(r.off1), "{s[86:87]}"(r.off2), "{s[98:99]}"(r.off0)
-               : "memory", "scc", "m0", "s90", "s91");
-}
-
-// The items of a workgroup (see gen_prefill_stream.py): which row blocks, and what the block needs
-// to set one up.
-// Values the compiler may hold in vector registers although they are the same in every lane: the
-// block binds them to scalar registers.
-__device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
-__device__ __forceinline__ uint32_t uni(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
-__device__ __forceinline__ uint64_t uni(uint64_t x) {
-  return address_from_words(__builtin_amdgcn_readfirstlane((int)(uint32_t)x), __builtin_amdgcn_readfirstlane((int)(uint32_t)(x >> 32)));
-}
-
-struct StreamItems {
-  int k, j, spg, nqt;          // item counter (starts at 0), the workgroup's slot, slots, row blocks
-  int sq, skv, offset, causal;
-  uint32_t q_row_bytes, out_row_bytes;
-  int row0;                    // first query row of item 0
-};
-
-#define TTPA_STREAM_COMMON_OUT                                                                        \
-  "+{v[64:79]}"(q_lo), "+{v[80:95]}"(q_hi), "+{s[64:65]}"(r.kbase), "+{s[66:67]}"(r.vbase), "+{s70}"(nblk), \
-      "+{s71}"(r.k_requests), "+{s73}"(r.v_requests), "+{s40}"(it.k), "+{s57}"(it.row0)
-#define TTPA_STREAM_COMMON_IN                                                                       \
-  "{v[176:183]}"(koff), "{v[184:187]}"(voff), "{v[188:189]}"(ldk), "{v[190:191]}"(ldv),         \
-      "{v[216:217]}"(q_base), "{v[218:219]}"(out_base), "{v220}"(lane_n), "{v221}"(lane_h4),       \
-      "{s68}"(r.stride), "{s69}"(c), "{s72}"(r.m0_base), "{s41}"(it.j), "{s42}"(it.spg), "{s43}"(it.nqt), \
-      "{s44}"(it.sq), "{s45}"(it.skv), "{s46}"(it.offset), "{s47}"(it.causal), "{s48}"(it.q_row_bytes),  \
-      "{s49}"(it.out_row_bytes)
-
-// Everything behind the first requests of item 0, through the stored output rows of the last item.
-// q_lo / q_hi: the eight Q fragments of item 0; koff / voff: the lane's LDS addresses of its K and
-// V^T fragments in slot 0 of the K and V rings; nblk: the 32-key blocks of item 0; kbase0 / vbase0:
-// block 0 of K / V again, for the items that follow.
-__device__ __forceinline__ void stream_items_dense(StreamRequests &r, StreamItems &it, u32x16 q_lo, u32x16 q_hi,
-                                                   const u32x8 &koff, const u32x4 &voff, const u32x2 &ldk,
-                                                   const u32x2 &ldv, uint64_t q_base, uint64_t out_base, int lane_n,
-                                                   int lane_h4, float c, int nblk, uint64_t kbase0, uint64_t vbase0) {
-  asm volatile(TTPA_STREAM_LOOP_TEXT_DENSE
-               : TTPA_STREAM_COMMON_OUT
-               : TTPA_STREAM_COMMON_IN, "{s[50:51]}"(kbase0), "{s[52:53]}"(vbase0)
-               : "memory", "vcc", "scc", "m0", "v208", TTPA_STREAM_LOOP_CLOBBERS);
-}
-
-// Paged: entry is the raw table entry of tile 3, entry_ptr the address of tile 4's.
-__device__ __forceinline__ void stream_items_paged(StreamRequests &r, StreamItems &it, u32x16 q_lo, u32x16 q_hi,
-                                                   const u32x8 &koff, const u32x4 &voff, const u32x2 &ldk,
-                                                   const u32x2 &ldv, uint64_t q_base, uint64_t out_base, int lane_n,
-                                                   int lane_h4, float c, int nblk, int kv_heads, int kv_head, int num_blocks, int tiles_per_block,
-                                                   int entry, uint64_t entry_ptr) {
-  int read_in_block = 3 % tiles_per_block, request_in_block = 4 % tiles_per_block;
-  const int read_in_block0 = read_in_block, request_in_block0 = request_in_block, entry0 = entry;
-  const uint64_t entry_ptr0 = entry_ptr, off1 = r.off1, off2 = r.off2;
-  int entry_requests = max((nblk - 1) / 2 - 3, 0);
-  asm volatile(TTPA_STREAM_LOOP_TEXT_PAGED
-               : TTPA_STREAM_COMMON_OUT, "+{s80}"(read_in_block), "+{s81}"(request_in_block),
-                 "+{s[82:83]}"(entry_ptr), "+{s[84:85]}"(r.off1), "+{s[86:87]}"(r.off2), "+{s96}"(entry_requests),
-                 "+{v208}"(entry)
-               : TTPA_STREAM_COMMON_IN, "{s76}"(kv_heads), "{s77}"(kv_head), "{s78}"(num_blocks),
-                 "{s79}"(tiles_per_block), "{s[98:99]}"(r.off0), "{s[50:51]}"(off1), "{s[52:53]}"(off2),
-                 "{s54}"(entry0), "{s55}"(read_in_block0), "{s56}"(request_in_block0), "{s[58:59]}"(entry_ptr0)
-               : "memory", "vcc", "scc", "m0", TTPA_STREAM_LOOP_CLOBBERS);
-}
-
 // MODE 0: dense K/V; 1: paged, block_size a multiple of 64 (a tile lies in one block);
 // 3: paged, block_size a multiple of the rows one wavefront load covers (1 KiB: 8 / 4 / 2 rows
 // for head sizes 64 / 128 / 256): one wavefront-uniform table lookup per load; 2: paged, any
@@ -342,20 +127,8 @@ __global__ __launch_bounds__(256, prefill_wgs_per_cu<RH>(D, MODE)) void prefill_
 
   int wg = blockIdx.x;  // index among the attention workgroups
   if constexpr (MODE == 0) {
-    if (a.fill_kc != nullptr) {
-      const int per = 8 * (a.attn_per_fill + 1);
-      const int sg = wg / per, m = wg - sg * per;
-      if (sg < a.fill_groups) {
-        if (m >= 8 * a.attn_per_fill) {
-          const int f = sg * 8 + (m - 8 * a.attn_per_fill);
-          if (f < a.n_fill) fill_workgroup<D>(a, f);
-          return;
-        }
-        wg = sg * 8 * a.attn_per_fill + m;
-      } else {
-        wg -= 8 * a.fill_groups;
-      }
-    }
+    wg = attention_workgroup<D>(a, wg);
+    if (wg < 0) return;
   }
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -368,15 +141,11 @@ __global__ __launch_bounds__(256, prefill_wgs_per_cu<RH>(D, MODE)) void prefill_
   // while its query tiles stream through.
   const int nqt = (a.sq + ROWS * RPW - 1) / (ROWS * RPW);
   const int groups = a.hq / HPW;
-  // (the hand-scheduled loop: a.spg workgroups per group, each taking several row blocks, heavy first)
-  constexpr bool kStreams = D == 128 && HPW == 4 && RH == 1 && (MODE == 0 || MODE == 1);
-  const bool streamed = kStreams && a.stream != 0;
-  const int per_group = streamed ? a.spg : nqt;
   const int xcd = wg & 7, slot = wg >> 3;
-  const int yl = slot / per_group;
+  const int yl = slot / nqt;
   const int y = yl * 8 + xcd;
   if (y >= a.batch * groups) return;  // grid is padded to a multiple of 8 groups
-  const int qt = nqt - 1 - (slot - yl * per_group);  // heavy (late) tiles are scheduled first
+  const int qt = nqt - 1 - (slot - yl * nqt);  // heavy (late) tiles are scheduled first
   const int b = y / groups;
   const int hq0 = (y - b * groups) * HPW;
   const int g = a.hq / a.hkv;
@@ -395,106 +164,6 @@ __global__ __launch_bounds__(256, prefill_wgs_per_cu<RH>(D, MODE)) void prefill_
   const int wg_first_key = a.window > 0 ? max(0, offset + qt * ROWS * RPW - a.window + 1) : 0;
   const int wave_first_key = a.window > 0 ? max(0, offset + row0 - a.window + 1) : 0;
   const int first_tile = wg_first_key / kKeysPerTile;
-
-  // ---- the hand-scheduled loop: its first requests go out now, in front of the Q loads ----------
-  StreamRequests sreq;
-  u32x2 stream_ldk = {0, 0}, stream_ldv = {0, 0};
-  int stream_entry = 0;
-  if constexpr (kStreams) {
-    if (streamed) {
-      int spg = a.spg;
-      if (a.spg_even > 0) {
-        const int lightest = a.causal ? min(offset + ROWS, a.skv) : a.skv;
-        const int heaviest = a.causal ? min(offset + a.sq, a.skv) : a.skv;
-        if (4 * lightest >= 3 * heaviest) {
-          spg = a.spg_even;
-          if (slot - yl * per_group >= spg) return;
-        }
-      }
-      const uint32_t lds0 = lds_address(smem);
-      const uint32_t row_bytes = MODE == 0 ? 2u * (uint32_t)a.kv_ts : (uint32_t)T::RB;
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        // a block is 8 segments of 1 KiB; wavefront w requests segments 2 w and 2 w + 1
-        const int r = (2 * wave + j) * T::RPI + lane / T::CPR, cp = lane % T::CPR;
-        stream_ldk[j] = (uint32_t)r * row_bytes + 16u * (uint32_t)(cp ^ T::swz_k(r)) + 1024u - 1024u * j;
-        stream_ldv[j] = (uint32_t)r * row_bytes + 16u * (uint32_t)(cp ^ T::swz_v(r)) + 1024u - 1024u * j;
-      }
-      sreq.m0_base = uni(lds0 + 2048u * (uint32_t)wave);
-      sreq.k_requests = sreq.v_requests = __builtin_amdgcn_readfirstlane((kv_end_wg + 31) / 32);
-      sreq.off0 = sreq.off1 = sreq.off2 = 0;
-      if constexpr (MODE == 0) {
-        const int64_t head = b * a.kv_bs + hk * a.kv_hs;
-        sreq.kbase = uni(reinterpret_cast<uint64_t>(a.k + head) - 1024u);
-        sreq.vbase = uni(reinterpret_cast<uint64_t>(a.v + head) - 1024u);
-        sreq.stride = (uint32_t)(64 * a.kv_ts);
-        stream_first_dense(sreq, stream_ldk, stream_ldv);
-      } else {
-        const int tpb = a.bs / kKeysPerTile, last = a.w * tpb - 1;  // (entries exist for every tile of the table)
-        sreq.kbase = reinterpret_cast<uint64_t>(a.k) - 1024u;
-        sreq.vbase = reinterpret_cast<uint64_t>(a.v) - 1024u;
-        sreq.stride = (uint32_t)a.bs * (uint32_t)T::RB;
-        int raw[4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) raw[t] = a.pt[(int64_t)b * a.pt_rs + min(t, last) / tpb];
-        uint64_t off[3];
-#pragma unroll
-        for (int t = 0; t < 3; ++t) {
-          int phys = __builtin_amdgcn_readfirstlane(raw[t]);
-          if ((unsigned)phys >= (unsigned)a.nb) phys = 0;
-          off[t] = (uint64_t)((int64_t)phys * a.hkv + hk) * sreq.stride + (uint64_t)(min(t, last) % tpb) * T::TILE_BYTES;
-        }
-        sreq.off0 = uni(off[0]), sreq.off1 = uni(off[1]), sreq.off2 = uni(off[2]);
-        stream_entry = raw[3];
-        stream_first_paged(sreq, stream_ldk, stream_ldv);
-      }
-      // Q fragments behind the requests (B operand: lane n = query row, 8 head-dim elements per k-step)
-      u32x16 q_lo, q_hi;
-      {
-        const int qrow = min(row0 + n, a.sq - 1);
-        const uint16_t *qp = a.q + b * a.q_bs + hq * a.q_hs + (int64_t)qrow * a.q_ts + 8 * h;
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          const uint4 lo = *reinterpret_cast<const uint4 *>(qp + 16 * s), hi = *reinterpret_cast<const uint4 *>(qp + 16 * (s + 4));
-          q_lo[4 * s] = lo.x, q_lo[4 * s + 1] = lo.y, q_lo[4 * s + 2] = lo.z, q_lo[4 * s + 3] = lo.w;
-          q_hi[4 * s] = hi.x, q_hi[4 * s + 1] = hi.y, q_hi[4 * s + 2] = hi.z, q_hi[4 * s + 3] = hi.w;
-        }
-      }
-      // LDS operand addresses of the lane inside slot 0 of the K ring and of the V ring (the formulas
-      // of the plain loop below: K fragment of k-step s, V^T fragment of output block db)
-      u32x8 ko;
-#pragma unroll
-      for (int s = 0; s < 8; ++s) ko[s] = lds0 + (uint32_t)(n * T::RB + 16 * ((2 * s + h) ^ T::swz_k(n)));
-      u32x4 vo;
-      {
-        const int grp = lane >> 4, a16 = lane & 15, vr = 4 * (grp >> 1) + (a16 >> 2);
-#pragma unroll
-        for (int db = 0; db < 4; ++db) {
-          const int c = 4 * db + 2 * (grp & 1) + ((a16 & 3) >> 1);
-          vo[db] = lds0 + TTPA_STREAM_V_RING + (uint32_t)(vr * T::RB + 16 * (c ^ T::swz_v(vr)) + 8 * (a16 & 1));
-        }
-      }
-      StreamItems it;
-      it.k = 0, it.j = uni(slot - yl * per_group), it.spg = uni(spg), it.nqt = uni(nqt);
-      it.sq = uni(a.sq), it.skv = uni(a.skv), it.offset = uni(offset), it.causal = uni(a.causal);
-      it.q_row_bytes = uni(2u * (uint32_t)a.q_ts), it.out_row_bytes = uni(2u * (uint32_t)a.out_ts);
-      it.row0 = __builtin_amdgcn_readfirstlane(row0);
-      // per lane: row 0 of the lane's head, at the lane's 8 (lane / 32) / 4 (lane / 32) elements
-      const uint64_t q_base = reinterpret_cast<uint64_t>(a.q + b * a.q_bs + hq * a.q_hs + 8 * h);
-      const uint64_t out_base = reinterpret_cast<uint64_t>(a.out + b * a.out_bs + hq * a.out_hs + 8 * h);
-      const int nblk = __builtin_amdgcn_readfirstlane((kv_end_wg + 31) / 32);
-      if constexpr (MODE == 0) {
-        const int64_t head = b * a.kv_bs + hk * a.kv_hs;
-        stream_items_dense(sreq, it, q_lo, q_hi, ko, vo, stream_ldk, stream_ldv, q_base, out_base, n, 4 * h, a.scale_log2e, nblk,
-                           uni(reinterpret_cast<uint64_t>(a.k + head) - 1024u), uni(reinterpret_cast<uint64_t>(a.v + head) - 1024u));
-      } else {
-        const int tpb = a.bs / kKeysPerTile;
-        stream_items_paged(sreq, it, q_lo, q_hi, ko, vo, stream_ldk, stream_ldv, q_base, out_base, n, 4 * h, a.scale_log2e, nblk, uni(a.hkv), uni(hk), uni(a.nb), uni(tpb), stream_entry,
-                           uni(reinterpret_cast<uint64_t>(a.pt + (int64_t)b * a.pt_rs + 4 / tpb)));
-      }
-      return;
-    }
-  }
 
   // ---- Q fragments (B operand: lane n = query row, 8 head-dim elements per k-step) -----
   static_assert(RH == 1, "one block of 32 query rows per wavefront");
@@ -930,60 +599,21 @@ int launch_mode(const PrefillArgs &a, hipStream_t st) {
   constexpr int RPW = 4 / HPW;
   constexpr int ROWS = kRowsPerWave * RH;
   const int nqt = (a.sq + ROWS * RPW - 1) / (ROWS * RPW);
-  // two stages of a K and a V tile
-  // (the hand-scheduled loop keeps two rings of five 8 KiB blocks)
-  constexpr bool kStreams = D == 128 && HPW == 4 && RH == 1 && (MODE == 0 || MODE == 1);
-  const size_t lds = kStreams ? (size_t)TTPA_STREAM_LDS_BYTES : 2 * Tile<D>::STAGE_BYTES;
+  const size_t lds = 2 * Tile<D>::STAGE_BYTES;  // two stages of a K and a V tile
   static std::atomic<uint64_t> lds_ready{0};
   if (!ensure_dynamic_lds(reinterpret_cast<const void *>(&prefill_kernel<D, HPW, MODE, RH>), lds, lds_ready))
     return fail(TTPA_ERR_LAUNCH, "prefill: cannot reserve %zu bytes of LDS", lds);
   const int ny8 = (a.batch * (a.hq / HPW) + 7) / 8;
   PrefillArgs b = a;
-  // The hand-scheduled loop takes launches of whole 32-key blocks without a window or an explicit mask
-  // (a dense K / V that ends inside a 64-key tile goes through the plain loop).  One workgroup per
-  // block of 32 query rows and head group, heavy blocks first, and the dispatcher deals them to the CUs
-  // as slots free up: the loop can also give a workgroup several row blocks (spg workgroups per group,
-  // TTPA_PREFILL_WGS_PER_GROUP), but one round of two workgroups per CU measured 204 us against 150 on
-  // the 4 x 2048-token causal workload (a change of row block costs a workgroup about 4 us in which
-  // nothing of its own overlaps, and a static deal cannot make up for workgroups that start late).
-  b.stream = kStreams && a.stream && a.window == 0 && a.mask == nullptr && (MODE == 1 || a.skv % kKeysPerTile == 0);
-  b.spg = b.spg_even = 0;
-  int per_group = nqt;
-  if (b.stream) {
-    b.spg = nqt;
-    // Row blocks of nearly one weight (a chunk far into its sequence, or no causal mask) that fill the
-    // chip more than once: one round of workgroups with equal shares instead, which saves the later
-    // rounds' start-up (267 -> 261 us on 4 x 512-token chunks behind 4096 tokens, 64 heads).  The
-    // chunk's start is in device memory, so the kernel decides: the workgroups past the round exit.
-    int cus = device_cus();
-    if (cus <= 0) cus = 256;
-    const int one_round = (2 * cus + ny8 * 8 - 1) / (ny8 * 8);
-    b.spg_even = one_round < nqt && nqt % one_round == 0 ? one_round : 0;
-    if (const char *e = getenv("TTPA_PREFILL_WGS_PER_GROUP")) {  // (read on every call) an experiment's override
-      if (atoi(e) > 0) b.spg = std::min(nqt, atoi(e)), b.spg_even = 0;
-    }
-    per_group = b.spg;
-  }
-  int grid = per_group * ny8 * 8;
-  if (MODE == 0 && a.fill_kc) {
-    // The fill workgroups are spread over the launch in groups of 8, one group behind every
-    // attn_per_fill groups of attention workgroups, so that their memory traffic runs while the
-    // neighbouring workgroups keep the matrix pipes busy (all of them at the end of the launch
-    // cost as much as two separate fills).
-    b.n_fill = 2 * a.batch * a.hkv * ((a.skv + fill_rows_per_wg(D) - 1) / fill_rows_per_wg(D));
-    const int fg = (b.n_fill + 7) / 8, ag = grid / 8;
-    b.fill_groups = fg;
-    b.attn_per_fill = ag >= fg ? ag / fg : 1;
-    // fewer attention groups than fill groups: one of each per super-group, and the attention
-    // slots past the last real one exit at once (the kernel's range check)
-    grid = ag >= fg ? grid + 8 * fg : 16 * fg;
-  }
+  int grid = nqt * ny8 * 8;
+  if (MODE == 0 && a.fill_kc) grid = grid_with_fill(b, grid, D);
   launch_dominant(&prefill_kernel<D, HPW, MODE, RH>, dim3(grid), dim3(256), lds, st, b);
   return check_launch("sdpa_prefill");
 }
 
 template <int D, int HPW, int RH>
 int launch_rh(const PrefillArgs &a, hipStream_t st) {
+  if (stream_serves(a, D)) return launch_stream(a, st);
   if (!a.pt) return launch_mode<D, HPW, 0, RH>(a, st);
   if (a.bs % kKeysPerTile == 0) return launch_mode<D, HPW, 1, RH>(a, st);
   if (a.bs % Tile<D>::RPI == 0) return launch_mode<D, HPW, 3, RH>(a, st);
@@ -1003,8 +633,7 @@ int launch(const PrefillArgs &a, hipStream_t st) {
     // With scratch from the caller, a pass that the hand-scheduled loop can serve reads bfloat16
     // copies of its blocks (written by one launch in front of it) instead of expanding every
     // tile once per workgroup on its way into LDS.
-    constexpr bool kStreams = D == 128 && HPW == 4;
-    if (kStreams && a.expand && a.stream && a.window == 0 && a.mask == nullptr && a.bs % kKeysPerTile == 0) {
+    if (a.expand && a.bs % kKeysPerTile == 0 && stream_serves(a, D)) {
       const int64_t blocks = (int64_t)a.batch * a.w;
       const int64_t cache_elems = blocks * a.hkv * a.bs * D;
       ExpandArgs e;
@@ -1025,7 +654,7 @@ int launch(const PrefillArgs &a, hipStream_t st) {
       if (after) arm_profile_events(nullptr, after);
       PrefillArgs b = a;
       b.k = e.k, b.v = e.v, b.pt = e.table, b.pt_rs = a.w, b.nb = (int)blocks, b.kv_bfp8 = 0, b.expand = nullptr;
-      return launch_mode<D, HPW, 1, 1>(b, st);
+      return launch_stream(b, st);
     }
     return launch_mode<D, HPW, 4, 1>(a, st);
   }

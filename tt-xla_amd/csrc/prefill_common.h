@@ -1,0 +1,163 @@
+// What the two prefill kernels (prefill.hip: the compiler-scheduled loop; prefill_stream.hip: the
+// hand-scheduled one) share: the arguments, the LDS swizzle of a K / V tile and the cache fill that
+// rides along with a dense launch.
+#pragma once
+
+#include "common.h"
+
+namespace ttpa {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef short shortx4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x16 __attribute__((ext_vector_type(16)));
+
+constexpr int kKeysPerTile = 64;
+constexpr int kRowsPerWave = 32;
+
+struct PrefillArgs {
+  uint16_t *out;
+  int64_t out_bs, out_hs, out_ts;
+  const uint16_t *q;
+  int64_t q_bs, q_hs, q_ts;
+  const uint16_t *k, *v;
+  int64_t kv_bs, kv_hs, kv_ts;  // dense form
+  const int32_t *pt;            // paged form when non-null
+  int64_t pt_rs;
+  const int32_t *chunk_start;
+  const uint16_t *mask;
+  int64_t mask_bs, mask_rs;
+  int batch, hq, hkv, sq, skv, bs, w, nb, causal;
+  uint32_t bs_magic;  // floor(2^32 / bs) + 1: key / bs = mulhi(key, bs_magic) while key * bs < 2^32 (bs >= 2)
+  // Dense form with a cache fill in the same launch (fill_kc != null): k / v are also written
+  // to the paged caches through fill_pt, by workgroups n_attn ... of the grid.  bs / nb /
+  // bs_magic describe the caches; table row of batch entry i = fill_bidx[i] (or i == 0).
+  uint16_t *fill_kc, *fill_vc;
+  const int32_t *fill_pt;
+  int64_t fill_pt_rs;
+  const void *fill_bidx;
+  int fill_bidx_i64, fill_rows;
+  // Grid layout with a fill: fill_groups super-groups of (8 * attn_per_fill attention
+  // workgroups, then 8 fill workgroups), then the remaining attention workgroups.  Groups of 8
+  // keep an attention workgroup's index congruent to its hardware index modulo 8 (its XCD).
+  int fill_groups, attn_per_fill, n_fill;
+  int window;  // > 0 (causal only): row i attends keys offset + i - window < j <= offset + i
+  float scale_log2e;
+  int kv_bfp8;  // paged form: the caches are block-float-8 (mode 4, or expanded into `expand` first)
+  void *expand; // scratch for bfloat16 copies of the block-float-8 blocks of this pass, or null
+  int stream;   // 0: the plain loop whatever the shape (TTPA_PREFILL_STREAM=0)
+  // The streaming kernel: workgroups per (batch entry, head group), each taking one or several row blocks
+  int spg;
+  int spg_even; // > 0: when the row blocks weigh about the same, only this many of them work (equal shares)
+};
+
+// key / block_size without a division instruction sequence (about 30 instructions each, and the
+// paged tile loads need several per tile).
+__device__ __forceinline__ int div_block(const PrefillArgs &a, int key) {
+  return a.bs == 1 ? key : (int)__umulhi((uint32_t)key, a.bs_magic);
+}
+
+// LDS geometry of one stage: the K tile (64 rows of D elements) followed by the V tile.
+// Chunk c (16 bytes) of row r is stored at chunk position c ^ swz(r).
+//   K fragments are read by 16 lanes of consecutive rows at one logical chunk: the 16
+//   positions must differ (rows of >= 256 bytes) or, for 128-byte rows, differ within each
+//   pair of rows that shares a 256-byte bank line.
+//   V fragments are read, per 32 lanes, as 4 consecutive rows x 4 consecutive chunks.
+template <int D>
+struct Tile {
+  static constexpr int RB = 2 * D;                 // row bytes
+  static constexpr int CPR = D / 8;                // 16-byte chunks per row
+  static constexpr int RPI = 1024 / RB;            // rows covered by one wavefront load
+  static constexpr int NI = kKeysPerTile / RPI / 4;  // loads per wavefront per tile and tensor
+  static constexpr int TILE_BYTES = kKeysPerTile * RB;
+  static constexpr int STAGE_BYTES = 2 * TILE_BYTES;
+  __device__ static constexpr int swz_k(int r) { return RB >= 256 ? (r & 15) : ((r >> 1) & 7); }
+  __device__ static constexpr int swz_v(int r) { return RB >= 256 ? 4 * (r & 3) : 4 * ((r >> 1) & 1); }
+};
+
+// The cache fill that rides along with a dense prefill: workgroup f (counted from the end of
+// the attention workgroups) copies fill_rows_per_wg(D) token rows (128 KiB) of one (tensor, batch entry, KV head)
+// from the dense K / V operand into the paged cache, with the semantics of the fill operator
+// (rows whose table row or block is out of range are skipped).  Pure memory work that runs in
+// the shadow of the matrix-bound attention workgroups; nothing in this launch reads the caches.
+constexpr int kFillPasses = 32;  // 16-byte loads in flight per thread
+constexpr int fill_rows_per_wg(int d) { return kFillPasses * (256 / (d / 8)); }
+
+template <int D>
+__device__ __forceinline__ void fill_workgroup(const PrefillArgs &a, int f) {
+  constexpr int CPR = D / 8;        // 16-byte chunks per row
+  constexpr int RPP = 256 / CPR;    // rows per pass of the 256 threads
+  constexpr int NP = kFillPasses;
+  constexpr int kFillRows = fill_rows_per_wg(D);
+  const int chunks = (a.skv + kFillRows - 1) / kFillRows;
+  const int c0 = f % chunks;
+  int r = f / chunks;
+  const int h = r % a.hkv;
+  r /= a.hkv;
+  const int b = r % a.batch;
+  const bool is_v = r / a.batch != 0;
+  int64_t row = a.fill_bidx ? load_index(a.fill_bidx, a.fill_bidx_i64, b) : 0;
+  if (row < 0 || row >= a.fill_rows) return;
+  const uint16_t *src = (is_v ? a.v : a.k) + b * a.kv_bs + h * a.kv_hs;
+  uint16_t *cache = is_v ? a.fill_vc : a.fill_kc;
+  const int32_t *pt = a.fill_pt + row * a.fill_pt_rs;
+  const int t0 = c0 * kFillRows + (int)threadIdx.x / CPR, c = (int)threadIdx.x % CPR;
+  // every load (rows and table entries) is requested before the first store: the compiler
+  // cannot move a load across a store that might alias it, and a table entry per pass would
+  // otherwise cost a round trip each
+  u32x4 val[NP];
+  int phys[NP];
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    const int t = min(t0 + p * RPP, a.skv - 1);
+    val[p] = *reinterpret_cast<const u32x4 *>(src + (int64_t)t * a.kv_ts + 8 * c);
+    phys[p] = pt[div_block(a, t)];
+  }
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    const int t = t0 + p * RPP;
+    const int off = t - div_block(a, t) * a.bs;
+    // (no early exit from the loop: the arrays must stay in registers)
+    if (t < a.skv && (unsigned)phys[p] < (unsigned)a.nb)
+      __builtin_nontemporal_store(val[p], reinterpret_cast<u32x4 *>(cache + (((int64_t)phys[p] * a.hkv + h) * a.bs + off) * D + 8 * c));
+  }
+}
+
+// Index of this workgroup among the attention workgroups of a dense launch that may carry a fill;
+// negative: it was a fill workgroup and is done.
+template <int D>
+__device__ __forceinline__ int attention_workgroup(const PrefillArgs &a, int wg) {
+  if (a.fill_kc == nullptr) return wg;
+  const int per = 8 * (a.attn_per_fill + 1);
+  const int sg = wg / per, m = wg - sg * per;
+  if (sg >= a.fill_groups) return wg - 8 * a.fill_groups;
+  if (m < 8 * a.attn_per_fill) return sg * 8 * a.attn_per_fill + m;
+  const int f = sg * 8 + (m - 8 * a.attn_per_fill);
+  if (f < a.n_fill) fill_workgroup<D>(a, f);
+  return -1;
+}
+
+// The grid of a dense launch with a fill, from its attention workgroups (a multiple of 8): the fill
+// workgroups are spread over the launch in groups of 8, one group behind every attn_per_fill groups
+// of attention workgroups, so that their memory traffic runs while the neighbouring workgroups keep
+// the matrix pipes busy (all of them at the end of the launch cost as much as two separate fills).
+inline int grid_with_fill(PrefillArgs &b, int grid, int d) {
+  b.n_fill = 2 * b.batch * b.hkv * ((b.skv + fill_rows_per_wg(d) - 1) / fill_rows_per_wg(d));
+  const int fg = (b.n_fill + 7) / 8, ag = grid / 8;
+  b.fill_groups = fg;
+  b.attn_per_fill = ag >= fg ? ag / fg : 1;
+  // fewer attention groups than fill groups: one of each per super-group, and the attention
+  // slots past the last real one exit at once (the kernels' range check)
+  return ag >= fg ? grid + 8 * fg : 16 * fg;
+}
+
+// prefill_stream.hip: whether the streaming kernel serves this launch, and the launch.
+bool stream_serves(const PrefillArgs &a, int head_size);
+int launch_stream(const PrefillArgs &a, hipStream_t st);
+
+}  // namespace ttpa
