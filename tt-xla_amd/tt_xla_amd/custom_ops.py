@@ -29,7 +29,9 @@ _BFP8_GROUP = 16
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """Handle of the current stream of the current device (the raw query: a Stream object costs
+    more than a kernel launch)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _ptr(t: Optional[torch.Tensor]) -> int:
@@ -432,9 +434,11 @@ def _workspace(nbytes: int, device) -> torch.Tensor:
     an eager serving loop pays no allocator round trip per layer and step.  Under graph capture the
     allocation has to belong to the graph's pool, and a call on another stream must not share the
     buffer, so both get a fresh tensor."""
-    if torch.cuda.is_current_stream_capturing() or torch.cuda.current_stream(device) != torch.cuda.default_stream(device):
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    # (the default stream's handle is 0, and it cannot be captured)
+    if torch._C._cuda_getCurrentRawStream(index) != 0 or torch.cuda.is_current_stream_capturing():
         return torch.empty(nbytes, dtype=torch.uint8, device=device)
-    key = (device.type, device.index if device.index is not None else torch.cuda.current_device())
+    key = (device.type, index)
     ws = _WORKSPACES.get(key)
     if ws is None or ws.numel() < nbytes:
         ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
