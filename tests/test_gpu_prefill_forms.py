@@ -48,3 +48,24 @@ def test_paged_forms(hq, hkv, bs, start, lc):
     got = torch.ops.tt.chunked_scaled_dot_product_attention(
         q.cuda(), key.cuda(), value.cuda(), table.cuda(), st.cuda(), 128**-0.5)
     P._check(f"paged h{hq}x{hkv} bs{bs} start{start} len{lc}", got.cpu(), want)
+
+
+@pytest.mark.parametrize("users,hq,hkv,bs,start,lc", [
+    (2, 4, 1, 32, 0, 32), (2, 4, 1, 32, 160, 33), (1, 2, 1, 96, 96, 130), (1, 3, 3, 32, 224, 64), (2, 8, 2, 160, 320, 96),
+    # split over the keys: an uneven last part, parts behind the causal limit of the first rows, one row block
+    # only, a start inside a block, 64-token blocks, fewer parts than the table's width allows, several row
+    # blocks per workgroup of which some do not exist
+    (1, 4, 1, 32, 2048, 32), (1, 4, 1, 32, 1000, 96), (1, 8, 2, 32, 512, 300), (1, 4, 1, 64, 4096, 1), (1, 4, 1, 64, 1100, 200),
+    (1, 2, 1, 32, 1536, 96), (2, 3, 3, 32, 700, 200), (1, 5, 5, 128, 1280, 129),
+])
+def test_blocks_of_32_and_parts(users, hq, hkv, bs, start, lc):
+    g = torch.Generator().manual_seed(hq + bs + start + lc)
+    for spare in (1, 40):  # columns behind the pass: the host sees the table, the device the keys
+        nbpu = -(-(start + lc) // bs) + spare
+        key, value, table = P._paged(g, users, nbpu, hkv, bs, 128, False)
+        q = P._bf(g, users, hq, lc, 128)
+        st = torch.tensor([start], dtype=torch.int32)
+        want = O.chunked_sdpa(q, key, value, table, st, 128**-0.5)
+        got = torch.ops.tt.chunked_scaled_dot_product_attention(
+            q.cuda(), key.cuda(), value.cuda(), table.cuda(), st.cuda(), 128**-0.5)
+        P._check(f"paged h{hq}x{hkv} bs{bs} start{start} len{lc} spare{spare}", got.cpu(), want)

@@ -2,7 +2,8 @@
 """Writes the hand-scheduled loop of the streaming prefill kernel (head size 128, 32 query rows of one
 head per wavefront, two workgroups of four wavefronts per CU) as one block of gfx950 assembly per
 form of the loop: build/prefill_stream_asm.h, included by prefill_stream.hip.  The forms: dense
-K / V, dense with a sliding window, paged K / V.
+K / V, dense with a sliding window, paged K / V in cache blocks of whole 64-key tiles, and in cache
+blocks of whole 32-key blocks.
 
 Why assembly: the loop wants the matrix pipe and the vector ALU of a SIMD busy at the same time
 from one instruction stream, with every register chosen by hand (256 per wavefront at two
@@ -47,7 +48,14 @@ is for everything.  Dense K / V: a block is `stride` bytes behind the one before
 size a multiple of 64): two blocks are a tile, a tile lies in one cache block; the table entry of
 the tile K enters two iterations from now is requested in front of the tile requests of every
 odd iteration (so the same wait covers it) and read at the next odd one.  Entries outside
-[0, num_blocks) read cache block 0.
+[0, num_blocks) read cache block 0.  Cache blocks of a multiple of 32 keys: every block has an entry
+of its own; the one of K block i + NS is read in iteration i and was requested in iteration i - 2 in
+front of the tile requests, so the same wait covers it (vmcnt(8), not 10: near the end an iteration
+requests no entry any more).  V follows two blocks behind K, so two byte offsets wait in a queue.
+
+A workgroup may take only a part of the keys (paged forms): it starts at any block, and if the base
+of a partial result is given, the accumulators go out as they are, with the reference and the sum of
+every row, for a merge kernel.
 
 A workgroup takes one or several ITEMS (blocks of 32 query rows of its four heads) one after the
 other: item k of the workgroup in slot j of `spg` slots is row block nqt - 1 - d with
@@ -86,13 +94,14 @@ MC, LRUN, LSUM, ALPHA = 196, 197, 198, 199   # MC, LRUN: inputs / outputs
 T = [200, 201, 202, 203]
 ORV, MLOC, MB, MCN = 204, 205, 206, 207
 PTREQ = 208                    # paged: the requested block-table entry (input)
+PTREQ2 = 211                   # blocks of 32: the entry requested in odd iterations (input)
 LOWEST, LOWREL = 209, 210      # window: first visible key of the lane's row, minus 4 h (input); relative to the block
 LIMIT = 212                    # last visible key of the lane's row, minus 4 h (input)
 LIMREL, NEGINF, VZERO = 213, 214, 215
 QBASE, OUTBASE = 216, 218      # per lane, 64-bit: q / out of row 0 of the lane's head, at the lane's 8 h / 4 h elements (inputs)
 VN, V4H = 220, 221             # lane % 32 and 4 (lane / 32) (inputs)
 OUTP, PTMP, VT0, VROW = 222, 224, 226, 227
-CLOBBERED = (list(range(0, QF)) + list(range(S[0], RING + 4 * NSLOT)) + list(range(MC, MCN + 1)) + [LOWREL, 211, LIMIT, LIMREL, NEGINF, VZERO]
+CLOBBERED = (list(range(0, QF)) + list(range(S[0], RING + 4 * NSLOT)) + list(range(MC, MCN + 1)) + [LOWREL, LIMIT, LIMREL, NEGINF, VZERO]
              + list(range(OUTP, VROW + 1)))
 
 # ---- scalar registers ---------------------------------------------------------------------------
@@ -106,6 +115,7 @@ S_M0B = "s72"                  # LDS address of this wavefront's first 1 KiB seg
 S_VLEFT = "s73"                # V blocks left to request
 S_MASKFROM = "s74"             # blocks whose first key is >= this are masked
 S_KEY0 = "s75"                 # first key of the block whose softmax comes next (input: of the first block)
+S_STATS, S_PART = "s[36:37]", "s[38:39]"  # paged: where (reference, sum) and the accumulators of a part go (0: the whole result)
 S_LOWTO = "s34"                # window: blocks whose first key is < this are masked from below (input)
 # paged only
 S_HKV, S_HK, S_NCB, S_TPB = "s76", "s77", "s78", "s79"  # kv heads, this kv head, cache blocks, tiles per cache block
@@ -122,6 +132,8 @@ S_SQ, S_SKV, S_OFFSET, S_CAUSAL = "s44", "s45", "s46", "s47"
 S_QTS, S_OTS = "s48", "s49"    # bytes from a query / output row to the next
 # dense: s[50:51], s[52:53] K / V block 0 (minus 1024); paged: tile 1 and 2 offsets, s54 entry of tile 3,
 # s55 / s56 tile-in-cache-block of tiles 3 / 4, s[58:59] address of tile 4's entry
+# blocks of 32: s[50:51], s[52:53], s[58:59] byte offsets of blocks 0, 1, 2, s[84:85] and s[98:99] of blocks 3
+# and 4 (later: the next two V blocks), s[86:87] the K block's; S_TPB, S_CIN, S_RIN count 32-key blocks
 S_ROW0 = "s57"                 # first query row of the item
 S_STOREMASK = "s[60:61]"
 # temporaries s[88:95], s[62:63]
@@ -137,12 +149,13 @@ KEY_CONST = [8 * (r // 4) + r % 4 for r in range(16)]
 class Form:
     """What one block of assembly serves."""
 
-    def __init__(self, name, paged=False, window=False):
-        self.name, self.paged, self.window = name, paged, window
-        self.items = not window  # several row blocks in turn
+    def __init__(self, name, paged=0, window=False):
+        self.name, self.paged, self.window = name, paged, window  # paged: 0 or the keys that share a table entry
+        self.items = not window and paged != 32  # several row blocks in turn
+        self.parts = paged > 0  # may take a part of the keys
 
 
-FORMS = [Form("DENSE"), Form("DENSE_WINDOW", window=True), Form("PAGED", paged=True)]
+FORMS = [Form("DENSE"), Form("DENSE_WINDOW", window=True), Form("PAGED", paged=64), Form("PAGED32", paged=32)]
 START_REFERENCE = "0xff7fffff"  # the lowest finite float
 
 
@@ -387,6 +400,36 @@ def next_tile(o, tag):
     o.label(f"L_noreq_{tag}")
 
 
+def next_block(o, p, tag):
+    """Blocks of 32, every iteration: the byte offset of the K block from its table entry; the entry of
+    the K block two iterations on is requested."""
+    req = PTREQ2 if p % 2 else PTREQ
+    o.e(f"v_readfirstlane_b32 s88, v{req}")
+    o.e(f"s_cmp_lt_u32 s88, {S_NCB}")
+    o.e("s_cselect_b32 s88, s88, 0")
+    o.e(f"s_mul_i32 s88, s88, {S_HKV}")
+    o.e(f"s_add_u32 s90, s88, {S_HK}")
+    o.e(f"s_mul_hi_u32 s87, s90, {S_STRIDE}")
+    o.e(f"s_mul_i32 s86, s90, {S_STRIDE}")
+    o.e(f"s_lshl_b32 s90, {S_CIN}, 13")           # 32 tokens of 256 bytes per block inside the cache block
+    o.e("s_add_u32 s86, s86, s90")
+    o.e("s_addc_u32 s87, s87, 0")
+    o.e(f"s_add_u32 {S_CIN}, {S_CIN}, 1")
+    o.e(f"s_cmp_eq_u32 {S_CIN}, {S_TPB}")
+    o.e(f"s_cselect_b32 {S_CIN}, 0, {S_CIN}")
+    o.e(f"s_cmp_eq_u32 {S_RLEFT}, 0")
+    o.e(f"s_cbranch_scc1 L_noreq_{tag}%=")
+    o.e(f"global_load_dword v{req}, v{VZERO}, {S_RPTR}")
+    o.e(f"s_sub_u32 {S_RLEFT}, {S_RLEFT}, 1")
+    o.e(f"s_add_u32 {S_RIN}, {S_RIN}, 1")
+    o.e(f"s_cmp_lg_u32 {S_RIN}, {S_TPB}")
+    o.e(f"s_cbranch_scc1 L_noreq_{tag}%=")
+    o.e(f"s_mov_b32 {S_RIN}, 0")
+    o.e("s_add_u32 s82, s82, 4")
+    o.e("s_addc_u32 s83, s83, 0")
+    o.label(f"L_noreq_{tag}")
+
+
 def iteration_head(o, f, p, tag):
     """Mask, barrier and requests of iteration i = p (mod UNROLL)."""
     paged = f.paged
@@ -400,11 +443,17 @@ def iteration_head(o, f, p, tag):
     o.e("s_waitcnt vmcnt(0)")
     o.label(f"L_bar_{tag}")
     o.e("s_barrier")
-    if paged and p % 2 == 1:
+    if paged == 64 and p % 2 == 1:
         next_tile(o, tag)
+    if paged == 32:
+        next_block(o, p, tag)
     # K block i + NS is half (i + NS) % 2 of its tile, V block i + NS - 2 the same half of its own
-    request_block(o, "K", p % NS, tag, paged, (p + NS) % 2)
-    request_block(o, "V", (p + NS - 2) % NS, tag, paged, (p + NS) % 2)
+    half = (p + NS) % 2 if paged == 64 else 0
+    request_block(o, "K", p % NS, tag, paged, half)
+    request_block(o, "V", (p + NS - 2) % NS, tag, paged, half)
+    if paged == 32:
+        o.e("s_mov_b64 s[84:85], s[98:99]")
+        o.e("s_mov_b64 s[98:99], s[86:87]")
 
 
 def iteration_tail(o, tag, exit_label):
@@ -497,9 +546,42 @@ def epilogue(o):
     o.e("s_nop 1")
 
 
-def next_item(o, paged):
+def partial_epilogue(o):
+    """The accumulators of a part of the keys as floats, register group by register group in the order in
+    which the lanes hold them (a store writes 1 KiB), and (reference, sum) per row."""
+    o.e(f"v_mov_b32 v{MB}, v{LRUN}")
+    o.e("s_nop 1")
+    o.e(f"v_permlane32_swap_b32 v{LRUN}, v{MB}")
+    o.e("s_nop 1")
+    o.e(f"v_add_f32 v{S[0] + 1}, v{LRUN}, v{MB}")
+    o.e(f"v_mov_b32 v{S[0]}, v{MC}")
+    o.e(f"v_lshlrev_b32 v{VT0}, 3, v{VN}")
+    o.e(f"v_lshlrev_b32 v{PTMP}, 4, v{VN}")
+    o.e(f"v_lshl_add_u32 v{PTMP}, v{V4H}, 7, v{PTMP}")      # 16 times the lane
+    for g in range(16):
+        if g and g % 4 == 0:
+            o.e("s_add_u32 s38, s38, 4096")
+            o.e("s_addc_u32 s39, s39, 0")
+        o.e(f"global_store_dwordx4 v{PTMP}, v[{4 * g}:{4 * g + 3}], {S_PART} offset:{1024 * (g % 4)}")
+    o.e(f"global_store_dwordx2 v{VT0}, v[{S[0]}:{S[0] + 1}], {S_STATS}")   # (both lanes of a row: the same values)
+
+
+def last_epilogue(o, f):
+    if f.parts:
+        o.e(f"s_cmp_lg_u64 {S_PART}, 0")
+        o.e("s_cbranch_scc1 L_partial%=")
+    epilogue(o)
+    if f.parts:
+        o.e("s_branch L_done%=")
+        o.label("L_partial")
+        partial_epilogue(o)
+        o.label("L_done")
+
+
+def next_item(o, f):
     """Behind the last PV of an item: is there another one?  Its Q fragments and first requests go
     out first, then the finished item is stored, then the state of the new one is set up."""
+    paged = f.paged
     o.e(f"s_add_u32 {S_K}, {S_K}, 1")
     o.e(f"s_mul_i32 s88, {S_K}, {S_SPG}")
     o.e(f"s_sub_u32 s89, {S_SPG}, 1")
@@ -541,7 +623,10 @@ def next_item(o, paged):
     item_setup(o, "nx")
     o.e("s_branch L_item_top%=")
     o.label("L_last_item")
-    epilogue(o)
+    last_epilogue(o, f)
+
+
+FIRST32 = ("s[50:51]", "s[52:53]", "s[58:59]", "s[84:85]", "s[98:99]")  # blocks of 32: the first five byte offsets
 
 
 def generate_first(paged, suffix=""):
@@ -549,14 +634,14 @@ def generate_first(paged, suffix=""):
     the caller can put its Q loads behind them)."""
     o = Out()
     for j in range(NS):
-        if paged:  # tiles 0, 1, 2 at S_OFF0, S_OFFV, S_OFFK
-            src = ("s[98:99]", S_OFFV, S_OFFK)[j // 2]
+        if paged:  # tiles 0, 1, 2 at S_OFF0, S_OFFV, S_OFFK; blocks of 32: 0 .. 4
+            src = ("s[98:99]", S_OFFV, S_OFFK)[j // 2] if paged == 64 else FIRST32[j]
             lo = int(src[2:4])
             o.e(f"s_cmp_eq_u32 {S_KLEFT}, 0")
             o.e(f"s_cbranch_scc1 L_noK_pro{j}{suffix}%=")
             o.e(f"s_add_u32 s90, s64, s{lo}")
             o.e(f"s_addc_u32 s91, s65, s{lo + 1}")
-            if j % 2:
+            if j % 2 and paged == 64:
                 o.e(f"s_add_u32 s90, s90, {SLOT}")
                 o.e("s_addc_u32 s91, s91, 0")
             o.e(f"s_add_u32 m0, {S_M0B}, {j * SLOT}")
@@ -568,13 +653,13 @@ def generate_first(paged, suffix=""):
             request_block(o, "K", j, f"pro{j}{suffix}", False, 0)
     for j in range(NS - 2):
         if paged:
-            src = ("s[98:99]", S_OFFV)[j // 2]
+            src = ("s[98:99]", S_OFFV)[j // 2] if paged == 64 else FIRST32[j]
             lo = int(src[2:4])
             o.e(f"s_cmp_eq_u32 {S_VLEFT}, 0")
             o.e(f"s_cbranch_scc1 L_noV_pro{j}{suffix}%=")
             o.e(f"s_add_u32 s90, s66, s{lo}")
             o.e(f"s_addc_u32 s91, s67, s{lo + 1}")
-            if j % 2:
+            if j % 2 and paged == 64:
                 o.e(f"s_add_u32 s90, s90, {SLOT}")
                 o.e("s_addc_u32 s91, s91, 0")
             o.e(f"s_add_u32 m0, {S_M0B}, {VRING + j * SLOT}")
@@ -637,9 +722,9 @@ def generate(f):
     o.e("s_nop 15")
     o.e("s_nop 15")
     if f.items:
-        next_item(o, f.paged)
+        next_item(o, f)
     else:
-        epilogue(o)
+        last_epilogue(o, f)
     return o.lines
 
 

@@ -633,7 +633,7 @@ int launch(const PrefillArgs &a, hipStream_t st) {
     // With scratch from the caller, a pass that the hand-scheduled loop can serve reads bfloat16
     // copies of its blocks (written by one launch in front of it) instead of expanding every
     // tile once per workgroup on its way into LDS.
-    if (a.expand && a.bs % kKeysPerTile == 0 && stream_serves(a, D)) {
+    if (a.expand && stream_serves(a, D)) {
       const int64_t blocks = (int64_t)a.batch * a.w;
       const int64_t cache_elems = blocks * a.hkv * a.bs * D;
       ExpandArgs e;
@@ -754,10 +754,15 @@ static int prefill_impl(void *out, int64_t out_batch_stride, int64_t out_head_st
       return fail(TTPA_ERR_UNSUPPORTED, "prefill: a block-float-8 cache needs block_size %% 16 == 0");
     TTPA_REQUIRE(workspace_bytes >= 0 && (workspace != nullptr || workspace_bytes == 0),
                  "prefill: workspace_bytes %lld with a null workspace", (long long)workspace_bytes);
-    if (workspace && aligned16(workspace) && (int64_t)batch * table_width < (1ll << 31) &&
-        workspace_bytes >= expand_bytes(batch, table_width, kv_heads, block_size, head_size))
+    const int64_t need = expand_bytes(batch, table_width, kv_heads, block_size, head_size);
+    if (workspace && aligned16(workspace) && (int64_t)batch * table_width < (1ll << 31) && workspace_bytes >= need) {
       a.expand = workspace;  // (a smaller one is not an error: the pass expands tile by tile instead)
+      workspace = static_cast<unsigned char *>(workspace) + need;
+      workspace_bytes -= need;
+    }
   }
+  a.part_acc = nullptr, a.part_bytes = 0, a.parts = 1;
+  if (page_table && workspace && aligned16(workspace)) a.part_acc = static_cast<float *>(workspace), a.part_bytes = workspace_bytes;
   {
     // (TTPA_PREFILL_STREAM=0, read on every call, sends every shape through the plain loop)
     const char *e = getenv("TTPA_PREFILL_STREAM");
@@ -819,6 +824,17 @@ extern "C" int64_t ttpa_sdpa_prefill_workspace_bytes(int32_t batch, int32_t kv_h
   if (kv_format != TTPA_KV_BFP8 || batch <= 0 || kv_heads <= 0 || head_size <= 0 || block_size <= 0 || table_width <= 0)
     return 0;
   return expand_bytes(batch, table_width, kv_heads, block_size, head_size);
+}
+
+extern "C" int64_t ttpa_sdpa_prefill_scratch_bytes(int32_t batch, int32_t q_heads, int32_t kv_heads, int32_t q_len, int32_t head_size,
+                                                   int32_t block_size, int32_t table_width, int32_t kv_format) {
+  if (batch <= 0 || q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads || q_len <= 0 || head_size <= 0 || block_size <= 0 || table_width <= 0)
+    return 0;
+  const int32_t some_table = 0;
+  PrefillArgs a = {};
+  a.pt = &some_table, a.stream = 1;
+  a.batch = batch, a.hq = q_heads, a.hkv = kv_heads, a.sq = q_len, a.bs = block_size, a.w = table_width;
+  return ttpa_sdpa_prefill_workspace_bytes(batch, kv_heads, head_size, block_size, table_width, kv_format) + stream_part_bytes(a, head_size);
 }
 
 extern "C" int ttpa_sdpa_prefill_fill(

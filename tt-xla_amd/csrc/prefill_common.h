@@ -54,6 +54,10 @@ struct PrefillArgs {
   // The streaming kernel: workgroups per (batch entry, head group), each taking one or several row blocks
   int spg;
   int spg_even; // > 0: when the row blocks weigh about the same, only this many of them work (equal shares)
+  // ... and, paged, several workgroups per row block, each with a part of the keys (scratch from the caller or null)
+  float *part_acc;
+  int64_t part_bytes;
+  int parts;
 };
 
 // key / block_size without a division instruction sequence (about 30 instructions each, and the
@@ -158,6 +162,8 @@ inline int grid_with_fill(PrefillArgs &b, int grid, int d) {
 
 // prefill_stream.hip: whether the streaming kernel serves this launch, and the launch.
 bool stream_serves(const PrefillArgs &a, int head_size);
+// Bytes of scratch with which it splits the launch over the keys (0: it would not); stream_serves launches only.
+int64_t stream_part_bytes(const PrefillArgs &a, int head_size);
 int launch_stream(const PrefillArgs &a, hipStream_t st);
 
 }  // namespace ttpa

@@ -1,5 +1,5 @@
 // Streaming prefill attention for gfx950: head size 128, no explicit mask, K / V readable in whole
-// blocks of 32 keys (dense, or paged with a block size that is a multiple of 64).  The matrix pipe bounds it:
+// blocks of 32 keys (dense, or paged with a block size that is a multiple of 32).  The matrix pipe bounds it:
 // 16 v_mfma_f32_32x32x16_bf16 per block of 32 keys and wavefront, with the vector work of the softmax
 // between them.
 //
@@ -11,6 +11,13 @@
 // keys, 2 x 4096 tokens, 32 / 8 heads 160 -> 137 us; 4 x 2048 tokens, 16 / 16 heads 118 -> 98 us and 16 / 8
 // heads 99 -> 83 us; 2 x 2048 tokens, 40 / 8 heads 126 -> 103 us; 2 x 512-token chunks behind 4096 tokens,
 // 16 / 16 heads 103 -> 81 us.
+//
+// A launch of few row blocks over many keys (the chunk of one request far into its sequence: 128
+// workgroups for 512 rows of 32 / 8 heads, on 256 CUs that hold two each) is split over the keys:
+// several workgroups per row block, each with a share of the 32-key blocks, hand float accumulators
+// to prefill_merge_kernel.  512 rows behind 8192 tokens: blocks of 64 139 -> 80 us for the pass, blocks of 32
+// 231 -> 81 us (unsplit on the plain loop before); 256 rows of 16 / 16 heads behind 8192 228 -> 67 us.  Blocks
+// of 32 alone, where nothing is split: 4 x 512 rows behind 4096 tokens 180 -> 144 us.
 #include "prefill_common.h"
 #include "build/prefill_stream_asm.h"
 
@@ -23,7 +30,9 @@ namespace {
 constexpr int kD = 128;
 constexpr int kBlockKeys = 32;
 
-enum StreamForm { kDense = 0, kDenseWindow = 1, kPaged = 2 };
+// kPaged: cache blocks of whole 64-key tiles (two 32-key blocks share a table entry); kPaged32: of whole
+// 32-key blocks (an entry per block costs scalar instructions in every iteration, not in every other one)
+enum StreamForm { kDense = 0, kDenseWindow = 1, kPaged = 2, kPaged32 = 3 };
 
 // The assembly is bound to the registers its text names through constraint strings; everything else it
 // touches is on the clobber list.  The requests of a workgroup's first blocks are a block of assembly of their own, issued in front
@@ -58,6 +67,15 @@ __device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlan
 __device__ __forceinline__ uint32_t uni(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
 __device__ __forceinline__ uint64_t uni(uint64_t x) {
   return address_from_words(__builtin_amdgcn_readfirstlane((int)(uint32_t)x), __builtin_amdgcn_readfirstlane((int)(uint32_t)(x >> 32)));
+}
+
+__device__ __forceinline__ void stream_first_paged32(StreamRequests &r, const u32x2 &ldk, const u32x2 &ldv, const uint64_t (&off)[5]) {
+  asm volatile(TTPA_STREAM_FIRST_TEXT_PAGED32
+               : "+{s71}"(r.k_requests), "+{s73}"(r.v_requests)
+               : "{v[188:189]}"(ldk), "{v[190:191]}"(ldv), "{s[64:65]}"(r.kbase), "{s[66:67]}"(r.vbase),
+                 "{s72}"(r.m0_base), "{s[50:51]}"(off[0]), "{s[52:53]}"(off[1]), "{s[58:59]}"(off[2]), "{s[84:85]}"(off[3]),
+                 "{s[98:99]}"(off[4])
+               : "memory", "scc", "m0", "s90", "s91");
 }
 
 // What a workgroup works on (see gen_prefill_stream.py): which row blocks, and what the block of
@@ -106,31 +124,81 @@ __device__ __forceinline__ void stream_items_window(StreamRequests &r, StreamIte
                : "memory", "vcc", "scc", "m0", "v208", TTPA_STREAM_LOOP_CLOBBERS);
 }
 
-// Paged: entry is the raw table entry of tile 3, entry_ptr the address of tile 4's.
-__device__ __forceinline__ void stream_items_paged(StreamRequests &r, StreamItems &it, u32x16 q_lo, u32x16 q_hi,
-                                                   const u32x8 &koff, const u32x4 &voff, const u32x2 &ldk,
+// Where a workgroup that takes a part of the keys leaves its result (0: the whole result goes to the output).
+struct StreamPart {
+  uint64_t stats, acc;
+};
+
+// The block-table state of the paged forms: table entries per cache block, the raw entry (blocks of 32:
+// the two raw entries) that follow the first requests, where they and the next requested one lie in their
+// cache blocks, the address of the latter, and how many are left to request.
+struct StreamTable {
+  int kv_heads, kv_head, num_blocks, per_block;
+  int entry, entry2;
+  int read_in_block, request_in_block;
+  uint64_t entry_ptr;
+  int entry_requests;
+};
+
+__device__ __forceinline__ void stream_items_paged(StreamRequests &r, StreamItems &it, StreamTable &t, StreamPart &part,
+                                                   u32x16 q_lo, u32x16 q_hi, const u32x8 &koff, const u32x4 &voff, const u32x2 &ldk,
                                                    const u32x2 &ldv, uint64_t q_base, uint64_t out_base, int lane_n,
-                                                   int lane_h4, float c, int nblk, int kv_heads, int kv_head, int num_blocks, int tiles_per_block,
-                                                   int entry, uint64_t entry_ptr) {
-  int read_in_block = 3 % tiles_per_block, request_in_block = 4 % tiles_per_block;
-  const int read_in_block0 = read_in_block, request_in_block0 = request_in_block, entry0 = entry;
-  const uint64_t entry_ptr0 = entry_ptr, off1 = r.off1, off2 = r.off2;
-  int entry_requests = max((nblk - 1) / 2 - 3, 0);
+                                                   int lane_h4, float c, int nblk) {
+  const int read_in_block0 = t.read_in_block, request_in_block0 = t.request_in_block, entry0 = t.entry;
+  const uint64_t entry_ptr0 = t.entry_ptr, off1 = r.off1, off2 = r.off2;
   asm volatile(TTPA_STREAM_LOOP_TEXT_PAGED
-               : TTPA_STREAM_COMMON_OUT, "+{s80}"(read_in_block), "+{s81}"(request_in_block),
-                 "+{s[82:83]}"(entry_ptr), "+{s[84:85]}"(r.off1), "+{s[86:87]}"(r.off2), "+{s96}"(entry_requests),
-                 "+{v208}"(entry)
-               : TTPA_STREAM_COMMON_IN, "{s76}"(kv_heads), "{s77}"(kv_head), "{s78}"(num_blocks),
-                 "{s79}"(tiles_per_block), "{s[98:99]}"(r.off0), "{s[50:51]}"(off1), "{s[52:53]}"(off2),
-                 "{s54}"(entry0), "{s55}"(read_in_block0), "{s56}"(request_in_block0), "{s[58:59]}"(entry_ptr0)
+               : TTPA_STREAM_COMMON_OUT, "+{s80}"(t.read_in_block), "+{s81}"(t.request_in_block),
+                 "+{s[82:83]}"(t.entry_ptr), "+{s[84:85]}"(r.off1), "+{s[86:87]}"(r.off2), "+{s96}"(t.entry_requests),
+                 "+{v208}"(t.entry), "+{s[38:39]}"(part.acc)
+               : TTPA_STREAM_COMMON_IN, "{s76}"(t.kv_heads), "{s77}"(t.kv_head), "{s78}"(t.num_blocks),
+                 "{s79}"(t.per_block), "{s[98:99]}"(r.off0), "{s[50:51]}"(off1), "{s[52:53]}"(off2),
+                 "{s54}"(entry0), "{s55}"(read_in_block0), "{s56}"(request_in_block0), "{s[58:59]}"(entry_ptr0),
+                 "{s[36:37]}"(part.stats)
                : "memory", "vcc", "scc", "m0", TTPA_STREAM_LOOP_CLOBBERS);
+}
+
+__device__ __forceinline__ void stream_items_paged32(StreamRequests &r, StreamItems &it, StreamTable &t, StreamPart &part, uint64_t off3,
+                                                     uint64_t off4, u32x16 q_lo, u32x16 q_hi, const u32x8 &koff, const u32x4 &voff,
+                                                     const u32x2 &ldk, const u32x2 &ldv, uint64_t q_base, uint64_t out_base,
+                                                     int lane_n, int lane_h4, float c, int nblk) {
+  asm volatile(TTPA_STREAM_LOOP_TEXT_PAGED32
+               : TTPA_STREAM_COMMON_OUT, "+{s80}"(t.read_in_block), "+{s81}"(t.request_in_block),
+                 "+{s[82:83]}"(t.entry_ptr), "+{s[84:85]}"(off3), "+{s[98:99]}"(off4), "+{s96}"(t.entry_requests),
+                 "+{v208}"(t.entry), "+{v211}"(t.entry2), "+{s[38:39]}"(part.acc)
+               : TTPA_STREAM_COMMON_IN, "{s76}"(t.kv_heads), "{s77}"(t.kv_head), "{s78}"(t.num_blocks),
+                 "{s79}"(t.per_block), "{s[36:37]}"(part.stats)
+               : "memory", "vcc", "scc", "m0", "s86", "s87", TTPA_STREAM_LOOP_CLOBBERS);
+}
+
+// ---- splitting over the keys --------------------------------------------------------------------
+// A part is at least this many 32-key blocks: below it a workgroup's start and its float accumulators
+// cost more than the matrix work that they spread.
+constexpr int kMinPartBlocks = 8;
+constexpr int kMaxParts = 16;
+constexpr int kPartAccFloats = kRowsPerWave * kD;  // accumulators of one (part, head, row block)
+
+// The share of `nblk` blocks that part `part` of at most `parts` takes; the merge kernel asks the same
+// question.  Shares are whole 64-key tiles.
+__device__ __forceinline__ int blocks_per_part(int nblk, int parts) {
+  return max((((nblk + parts - 1) / parts) + 1) & ~1, kMinPartBlocks);
+}
+
+// Accumulators and (reference, sum) rows of the parts: [part][batch][head][row block], the statistics
+// behind all accumulators.
+struct PartLayout {
+  int64_t slots;  // (part, batch entry, head, row block) combinations
+  int row_blocks;
+};
+__host__ __device__ inline PartLayout part_layout(const PrefillArgs &a, int rows_per_wg) {
+  const int rb = (a.sq + rows_per_wg - 1) / rows_per_wg * (rows_per_wg / kRowsPerWave);
+  return {(int64_t)a.parts * a.batch * a.hq * rb, rb};
 }
 
 template <int HPW, int FORM>
 __global__ __launch_bounds__(256, 2) void prefill_stream_kernel(PrefillArgs a) {
   constexpr int RPW = 4 / HPW;  // row blocks per workgroup
   constexpr int D = kD;
-  constexpr bool PAGED = FORM == kPaged;
+  constexpr bool PAGED = FORM == kPaged || FORM == kPaged32;
   using T = Tile<D>;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
 
@@ -145,10 +213,13 @@ __global__ __launch_bounds__(256, 2) void prefill_stream_kernel(PrefillArgs a) {
   const int nqt = (a.sq + kRowsPerWave * RPW - 1) / (kRowsPerWave * RPW);
   const int groups = a.hq / HPW;
   const int xcd = wg & 7, slot = wg >> 3;
-  const int yl = slot / a.spg;
+  const int per_group = PAGED ? a.spg * a.parts : a.spg;
+  const int yl = slot / per_group;
   const int y = yl * 8 + xcd;
   if (y >= a.batch * groups) return;  // grid is padded to a multiple of 8 groups
-  const int qt = nqt - 1 - (slot - yl * a.spg);
+  const int item0 = PAGED ? (slot - yl * per_group) / a.parts : slot - yl * per_group;
+  const int part = PAGED ? slot - yl * per_group - item0 * a.parts : 0;
+  const int qt = nqt - 1 - item0;
   const int b = y / groups;
   const int hq0 = (y - b * groups) * HPW;
   const int hk = hq0 / (a.hq / a.hkv);
@@ -159,8 +230,18 @@ __global__ __launch_bounds__(256, 2) void prefill_stream_kernel(PrefillArgs a) {
   // keys the workgroup can see, in blocks of 32
   const int wg_last_row = min(a.sq, (qt + 1) * kRowsPerWave * RPW) - 1;
   const int kv_end = a.causal ? min(a.skv, offset + wg_last_row + 1) : a.skv;
-  const int first_block = FORM == kDenseWindow ? max(0, offset + qt * kRowsPerWave * RPW - a.window + 1) / kBlockKeys : 0;
-  const int nblk = __builtin_amdgcn_readfirstlane((kv_end + kBlockKeys - 1) / kBlockKeys - first_block);
+  int first_block = FORM == kDenseWindow ? max(0, offset + qt * kRowsPerWave * RPW - a.window + 1) / kBlockKeys : 0;
+  int nblk = __builtin_amdgcn_readfirstlane((kv_end + kBlockKeys - 1) / kBlockKeys - first_block);
+  bool whole = true;  // this workgroup sees all keys of its rows
+  if constexpr (PAGED) {
+    if (a.parts > 1) {
+      const int share = __builtin_amdgcn_readfirstlane(blocks_per_part(nblk, a.parts));
+      whole = share >= nblk;
+      first_block = part * share;
+      nblk = min(share, nblk - first_block);
+      if (nblk <= 0) return;
+    }
+  }
 
   int spg = a.spg;
   if (a.spg_even > 0) {
@@ -168,7 +249,7 @@ __global__ __launch_bounds__(256, 2) void prefill_stream_kernel(PrefillArgs a) {
     const int heaviest = a.causal ? min(offset + a.sq, a.skv) : a.skv;
     if (4 * lightest >= 3 * heaviest) {
       spg = a.spg_even;
-      if (slot - yl * a.spg >= spg) return;
+      if (item0 >= spg) return;
     }
   }
 
@@ -187,7 +268,9 @@ __global__ __launch_bounds__(256, 2) void prefill_stream_kernel(PrefillArgs a) {
   sreq.m0_base = uni(lds0 + 2048u * (uint32_t)wave);
   sreq.k_requests = sreq.v_requests = nblk;
   sreq.off0 = sreq.off1 = sreq.off2 = 0;
-  int entry = 0;
+  StreamTable tab;
+  StreamPart out_part = {0, 0};
+  uint64_t off[5];
   uint64_t kbase0 = 0, vbase0 = 0;
   if constexpr (!PAGED) {
     const int64_t head = b * a.kv_bs + hk * a.kv_hs + (int64_t)first_block * kBlockKeys * a.kv_ts;
@@ -197,23 +280,42 @@ __global__ __launch_bounds__(256, 2) void prefill_stream_kernel(PrefillArgs a) {
     sreq.stride = (uint32_t)(2 * kBlockKeys * a.kv_ts);
     stream_first_dense(sreq, ldk, ldv);
   } else {
-    const int tpb = a.bs / kKeysPerTile, last = a.w * tpb - 1;  // (entries exist for every tile of the table)
+    // keys that share a table entry are a multiple of a unit (a 64-key tile, a 32-key block); the first FIRST
+    // units are requested here, the loop takes raw entries from there on
+    constexpr int UNIT = FORM == kPaged ? kKeysPerTile : kBlockKeys;
+    constexpr int FIRST = FORM == kPaged ? 3 : 5, RAW = FORM == kPaged ? 1 : 2;
+    const int per = a.bs / UNIT, last = a.w * per - 1;  // (entries exist for every unit of the table)
+    const int unit0 = first_block * kBlockKeys / UNIT;
     sreq.kbase = reinterpret_cast<uint64_t>(a.k) - 1024u;
     sreq.vbase = reinterpret_cast<uint64_t>(a.v) - 1024u;
     sreq.stride = (uint32_t)a.bs * (uint32_t)T::RB;
-    int raw[4];
+    int raw[FIRST + RAW];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) raw[t] = a.pt[(int64_t)b * a.pt_rs + min(t, last) / tpb];
-    uint64_t off[3];
+    for (int t = 0; t < FIRST + RAW; ++t) raw[t] = a.pt[(int64_t)b * a.pt_rs + min(unit0 + t, last) / per];
 #pragma unroll
-    for (int t = 0; t < 3; ++t) {
+    for (int t = 0; t < FIRST; ++t) {
       int phys = __builtin_amdgcn_readfirstlane(raw[t]);
       if ((unsigned)phys >= (unsigned)a.nb) phys = 0;
-      off[t] = (uint64_t)((int64_t)phys * a.hkv + hk) * sreq.stride + (uint64_t)(min(t, last) % tpb) * T::TILE_BYTES;
+      off[t] = uni((uint64_t)((int64_t)phys * a.hkv + hk) * sreq.stride + (uint64_t)(min(unit0 + t, last) % per) * (UNIT * T::RB));
     }
-    sreq.off0 = uni(off[0]), sreq.off1 = uni(off[1]), sreq.off2 = uni(off[2]);
-    entry = raw[3];
-    stream_first_paged(sreq, ldk, ldv);
+    tab.kv_heads = uni(a.hkv), tab.kv_head = uni(hk), tab.num_blocks = uni(a.nb), tab.per_block = uni(per);
+    tab.entry = raw[FIRST], tab.entry2 = raw[FIRST + RAW - 1];
+    const int next = unit0 + FIRST;
+    tab.read_in_block = uni(next % per), tab.request_in_block = uni((next + RAW) % per);
+    tab.entry_ptr = uni(reinterpret_cast<uint64_t>(a.pt + (int64_t)b * a.pt_rs + (next + RAW) / per));
+    tab.entry_requests = uni(max((nblk - 1) / (UNIT / kBlockKeys) + 1 - FIRST - RAW, 0));
+    if constexpr (FORM == kPaged) {
+      sreq.off0 = off[0], sreq.off1 = off[1], sreq.off2 = off[2];
+      stream_first_paged(sreq, ldk, ldv);
+    } else {
+      stream_first_paged32(sreq, ldk, ldv, off);
+    }
+    if (!whole) {
+      const PartLayout lay = part_layout(a, kRowsPerWave * RPW);
+      const int64_t at = (((int64_t)part * a.batch + b) * a.hq + hq) * lay.row_blocks + qt * RPW + wave / HPW;
+      out_part.acc = uni(reinterpret_cast<uint64_t>(a.part_acc + at * kPartAccFloats));
+      out_part.stats = uni(reinterpret_cast<uint64_t>(a.part_acc + lay.slots * kPartAccFloats + at * (2 * kRowsPerWave)));
+    }
   }
   // Q fragments behind the requests (B operand: lane n = query row, 8 head-dim elements per k-step)
   u32x16 q_lo, q_hi;
@@ -242,7 +344,7 @@ __global__ __launch_bounds__(256, 2) void prefill_stream_kernel(PrefillArgs a) {
     }
   }
   StreamItems it;
-  it.k = 0, it.j = uni(slot - yl * a.spg), it.spg = uni(spg), it.nqt = uni(nqt);
+  it.k = 0, it.j = uni(item0), it.spg = uni(spg), it.nqt = uni(nqt);
   it.sq = uni(a.sq), it.skv = uni(a.skv), it.offset = uni(offset), it.causal = uni(a.causal);
   it.q_row_bytes = uni(2u * (uint32_t)a.q_ts), it.out_row_bytes = uni(2u * (uint32_t)a.out_ts);
   it.row0 = __builtin_amdgcn_readfirstlane(row0);
@@ -256,11 +358,100 @@ __global__ __launch_bounds__(256, 2) void prefill_stream_kernel(PrefillArgs a) {
     const int lowest = offset + min(row0 + n, a.sq - 1) - a.window + 1 - 4 * h;
     const int low_to = uni(offset + row0 + kRowsPerWave - a.window);
     stream_items_window(sreq, it, q_lo, q_hi, ko, vo, ldk, ldv, q_base, out_base, n, 4 * h, a.scale_log2e, nblk, lowest, low_to);
+  } else if constexpr (FORM == kPaged) {
+    stream_items_paged(sreq, it, tab, out_part, q_lo, q_hi, ko, vo, ldk, ldv, q_base, out_base, n, 4 * h, a.scale_log2e, nblk);
   } else {
-    const int tpb = a.bs / kKeysPerTile;
-    stream_items_paged(sreq, it, q_lo, q_hi, ko, vo, ldk, ldv, q_base, out_base, n, 4 * h, a.scale_log2e, nblk, uni(a.hkv), uni(hk), uni(a.nb), uni(tpb), entry,
-                       uni(reinterpret_cast<uint64_t>(a.pt + (int64_t)b * a.pt_rs + 4 / tpb)));
+    stream_items_paged32(sreq, it, tab, out_part, off[3], off[4], q_lo, q_hi, ko, vo, ldk, ldv, q_base, out_base, n, 4 * h, a.scale_log2e, nblk);
   }
+}
+
+// Merges the parts of a row block: out = sum_p 2^(m_p - M) acc_p / sum_p 2^(m_p - M) l_p.  One workgroup per
+// (row block, head, batch entry); thread (n, g) takes row n and head-dim elements 16 g .. 16 g + 15, which lie in
+// register groups 2 g and 2 g + 1 of lanes n and n + 32 (prefill_stream_kernel's lane holds elements
+// 8 group + 4 (lane / 32) .. + 3): 512 consecutive bytes per read of 32 lanes, whole 32-byte pieces of a row per
+// write.  Memory bound: 34 MB of accumulators (512 rows, 32 heads, 4 parts) in 7.9 us.
+template <int RPW>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
+  const int rb = blockIdx.x, hq = blockIdx.y, b = blockIdx.z;
+  const int qt = rb / RPW;
+  const int n = threadIdx.x & 31, g = threadIdx.x >> 5;
+  const int offset = a.causal ? (a.chunk_start ? a.chunk_start[0] : 0) : 0;
+  const int wg_last_row = min(a.sq, (qt + 1) * kRowsPerWave * RPW) - 1;
+  const int kv_end = a.causal ? min(a.skv, offset + wg_last_row + 1) : a.skv;
+  const int nblk = (kv_end + kBlockKeys - 1) / kBlockKeys;
+  const int share = blocks_per_part(nblk, a.parts);
+  if (share >= nblk) return;  // one workgroup saw all keys and wrote the output
+  const int active = (nblk + share - 1) / share;
+  const PartLayout lay = part_layout(a, kRowsPerWave * RPW);
+  const int64_t step = (int64_t)a.batch * a.hq * lay.row_blocks;
+  const int64_t at = ((int64_t)b * a.hq + hq) * lay.row_blocks + rb;
+  const float *acc = a.part_acc + at * kPartAccFloats + (8 * g) * 64 + 4 * n;
+  const float *stats = a.part_acc + lay.slots * kPartAccFloats + at * (2 * kRowsPerWave) + 2 * n;
+  float m[kMaxParts], l[kMaxParts];
+  float top = -INFINITY;
+#pragma unroll
+  for (int p = 0; p < kMaxParts; ++p) {
+    const int q = min(p, active - 1);
+    const float2 s = *reinterpret_cast<const float2 *>(stats + q * step * (2 * kRowsPerWave));
+    m[p] = s.x, l[p] = p < active ? s.y : 0.f;
+    top = fmaxf(top, m[p]);
+  }
+  float sum = 0.f;
+  float o[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) o[i] = 0.f;
+  // four parts' accumulators in flight at a time; parts past the last repeat it with weight 0
+  for (int p0 = 0; p0 < active; p0 += 4) {
+    float4 v[4][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float *src = acc + min(p0 + j, active - 1) * step * kPartAccFloats;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[j][i] = *reinterpret_cast<const float4 *>(src + (i >> 1) * 256 + (i & 1) * 128);  // group 2 g + i / 2, lane half i % 2
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float w = 0.f;
+#pragma unroll
+      for (int p = 0; p < kMaxParts; ++p)
+        if (p == p0 + j && p < active) w = __builtin_amdgcn_exp2f(m[p] - top), sum = fmaf(w, l[p], sum);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        o[4 * i] = fmaf(w, v[j][i].x, o[4 * i]), o[4 * i + 1] = fmaf(w, v[j][i].y, o[4 * i + 1]);
+        o[4 * i + 2] = fmaf(w, v[j][i].z, o[4 * i + 2]), o[4 * i + 3] = fmaf(w, v[j][i].w, o[4 * i + 3]);
+      }
+    }
+  }
+  const int row = rb * kRowsPerWave + n;
+  if (row >= a.sq) return;
+  const float inv = 1.0f / sum;
+  uint16_t *op = a.out + b * a.out_bs + hq * a.out_hs + (int64_t)row * a.out_ts + 16 * g;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    *reinterpret_cast<uint2 *>(op + 4 * i) = make_uint2(pack_bf16x2(o[4 * i] * inv, o[4 * i + 1] * inv), pack_bf16x2(o[4 * i + 2] * inv, o[4 * i + 3] * inv));
+}
+
+// Parts a launch is split into: as many as fill the two workgroup slots of every CU once, if its row blocks leave
+// at least half of them empty.  Only the host's view: how many keys there are is in device memory, and
+// the kernel takes fewer parts where they would get short.
+int launch_parts(const PrefillArgs &a, int heads_per_wg) {
+  int cus = device_cus();
+  if (cus <= 0) cus = 256;
+  const int rows = kRowsPerWave * 4 / heads_per_wg;
+  const int64_t wgs = (int64_t)a.batch * (a.hq / heads_per_wg) * ((a.sq + rows - 1) / rows);
+  const int most = (a.w * (a.bs / kBlockKeys) + kMinPartBlocks - 1) / kMinPartBlocks;
+  return (int)std::max<int64_t>(1, std::min<int64_t>({2 * cus / wgs, kMaxParts, most}));
+}
+
+int64_t part_bytes(PrefillArgs a, int heads_per_wg) {
+  a.parts = launch_parts(a, heads_per_wg);
+  if (a.parts <= 1) return 0;
+  return part_layout(a, kRowsPerWave * 4 / heads_per_wg).slots * (kPartAccFloats + 2 * kRowsPerWave) * (int64_t)sizeof(float);
+}
+
+int heads_per_workgroup(const PrefillArgs &a) {
+  const int g = a.hq / a.hkv;
+  return g % 4 == 0 ? 4 : g % 2 == 0 ? 2 : 1;
 }
 
 template <int HPW, int FORM>
@@ -278,7 +469,10 @@ int launch_form(const PrefillArgs &a, hipStream_t st) {
   // the 4 x 2048-token causal workload (a change of row block costs a workgroup about 4 us in which
   // nothing of its own overlaps, and a static deal cannot make up for workgroups that start late).
   b.spg = nqt, b.spg_even = 0;
-  if (HPW == 4 && FORM != kDenseWindow) {
+  b.parts = 1;
+  constexpr bool PAGED = FORM == kPaged || FORM == kPaged32;
+  if (PAGED && a.part_acc && a.part_bytes >= part_bytes(a, HPW)) b.parts = launch_parts(a, HPW);
+  if (HPW == 4 && (FORM == kDense || FORM == kPaged) && b.parts == 1) {
     // Row blocks of nearly one weight (a chunk far into its sequence, or no causal mask) that fill the
     // chip more than once: one round of workgroups with equal shares instead, which saves the later
     // rounds' start-up (267 -> 261 us on 4 x 512-token chunks behind 4096 tokens, 64 heads).  The
@@ -291,15 +485,20 @@ int launch_form(const PrefillArgs &a, hipStream_t st) {
       if (atoi(e) > 0) b.spg = std::min(nqt, atoi(e)), b.spg_even = 0;
     }
   }
-  int grid = b.spg * ny8 * 8;
-  if (FORM != kPaged && a.fill_kc) grid = grid_with_fill(b, grid, kD);
+  int grid = b.spg * b.parts * ny8 * 8;
+  if (!PAGED && a.fill_kc) grid = grid_with_fill(b, grid, kD);
   launch_dominant(&prefill_stream_kernel<HPW, FORM>, dim3(grid), dim3(256), (size_t)TTPA_STREAM_LDS_BYTES, st, b);
-  return check_launch("sdpa_prefill");
+  if (const int rc = check_launch("sdpa_prefill")) return rc;
+  if (b.parts > 1) {
+    prefill_merge_kernel<RPW><<<dim3((b.sq + kRowsPerWave - 1) / kRowsPerWave, b.hq, b.batch), dim3(256), 0, st>>>(b);
+    return check_launch("sdpa_prefill (merge of the parts)");
+  }
+  return TTPA_OK;
 }
 
 template <int HPW>
 int launch_heads(const PrefillArgs &a, hipStream_t st) {
-  if (a.pt) return launch_form<HPW, kPaged>(a, st);
+  if (a.pt) return a.bs % kKeysPerTile == 0 ? launch_form<HPW, kPaged>(a, st) : launch_form<HPW, kPaged32>(a, st);
   return a.window > 0 ? launch_form<HPW, kDenseWindow>(a, st) : launch_form<HPW, kDense>(a, st);
 }
 
@@ -311,15 +510,20 @@ int launch_heads(const PrefillArgs &a, hipStream_t st) {
 // faster (above) or, on passes of a few microseconds, equal.
 bool stream_serves(const PrefillArgs &a, int head_size) {
   if (!a.stream || head_size != kD || a.mask != nullptr) return false;
-  if (a.pt) return a.bs % kKeysPerTile == 0 && a.window == 0;
+  if (a.pt) return a.bs % kBlockKeys == 0 && a.window == 0;
   return a.skv % kBlockKeys == 0;
 }
 
+int64_t stream_part_bytes(const PrefillArgs &a, int head_size) {
+  return a.pt && stream_serves(a, head_size) ? part_bytes(a, heads_per_workgroup(a)) : 0;
+}
+
 int launch_stream(const PrefillArgs &a, hipStream_t st) {
-  const int g = a.hq / a.hkv;
-  if (g % 4 == 0) return launch_heads<4>(a, st);
-  if (g % 2 == 0) return launch_heads<2>(a, st);
-  return launch_heads<1>(a, st);
+  switch (heads_per_workgroup(a)) {
+    case 4: return launch_heads<4>(a, st);
+    case 2: return launch_heads<2>(a, st);
+    default: return launch_heads<1>(a, st);
+  }
 }
 
 }  // namespace ttpa

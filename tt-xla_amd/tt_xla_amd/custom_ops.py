@@ -655,11 +655,11 @@ def _prefill(query, key, value, page_table, chunk_start, attn_mask, is_causal, s
         if m.stride(-1) != 1:
             m = m.contiguous()
         mask_ptr, mask_bs, mask_rs = m.data_ptr(), m.stride(0), m.stride(2)
-    # block-float-8 caches: scratch for bfloat16 copies of the blocks the pass reads (the library uses
-    # it for the shapes its fastest loop serves and ignores it otherwise)
+    # scratch for what the library's fastest loop can use it for: bfloat16 copies of the blocks that a pass
+    # over block-float-8 caches reads, partial results where few query rows meet many keys
     ws_ptr, ws_bytes = 0, 0
-    if fmt == N.KV_BFP8 and d == 128 and (hq // hkv) % 4 == 0 and bs % 64 == 0 and not window and attn_mask is None:
-        need = int(N.lib().ttpa_sdpa_prefill_workspace_bytes(b, hkv, d, bs, w, fmt))
+    if page_table is not None and d == 128 and bs % 32 == 0 and not window and attn_mask is None:
+        need = int(N.lib().ttpa_sdpa_prefill_scratch_bytes(b, hq, hkv, s, d, bs, w, fmt))
         if 0 < need <= _EXPANSION_LIMIT:
             ws = _workspace(need, q.device)
             ws_ptr, ws_bytes = ws.data_ptr(), need
