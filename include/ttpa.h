@@ -485,6 +485,37 @@ int ttpa_latent_prefill(void *out, int64_t out_batch_stride, int64_t out_head_st
                         int32_t seq_len, int32_t head_size, int32_t head_dim_v, int32_t causal,
                         float scale, void *stream);
 
+/*
+ * Causal prefill attention with keys of 128 + 64 features in two parts (a part without and a part with
+ * position) and values of 128: out[b, h, i] = softmax_j<=i(scale * (q_nope[b, h, i] . k_nope[b, h / G, j] +
+ * q_rope[b, h, i] . k_rope[b, h / G, j])) . v[b, h / G, j].  The prompt form of a latent layer whose K and V
+ * have been expanded per head (head_size 192, head_dim_v 128; a k_rope that the heads share has head
+ * stride 0), and tt::flash_mla_prefill with a V of its own at that size (reference custom_ops.py:223-378).
+ * All operands bfloat16 [batch, heads, seq_len, part] by element strides (multiples of 8, out's of 4; innermost
+ * dimension contiguous); seq_len a multiple of 32.
+ */
+int ttpa_split_key_prefill(void *out, int64_t out_batch_stride, int64_t out_head_stride, int64_t out_token_stride,
+                           const void *q_nope, int64_t q_nope_batch_stride, int64_t q_nope_head_stride,
+                           int64_t q_nope_token_stride, const void *q_rope, int64_t q_rope_batch_stride,
+                           int64_t q_rope_head_stride, int64_t q_rope_token_stride, const void *k_nope,
+                           int64_t k_nope_batch_stride, int64_t k_nope_head_stride, int64_t k_nope_token_stride,
+                           const void *k_rope, int64_t k_rope_batch_stride, int64_t k_rope_head_stride,
+                           int64_t k_rope_token_stride, const void *v, int64_t v_batch_stride,
+                           int64_t v_head_stride, int64_t v_token_stride, int32_t batch, int32_t q_heads,
+                           int32_t kv_heads, int32_t seq_len, float scale, void *stream);
+
+/*
+ * paged_fill_cache of latent rows that are still in two parts: row t of user u, [latent_size] from `latent` and
+ * [rope_size] from `rope` behind it, goes to position t of page-table row u in a cache
+ * [num_blocks, 1, block_size, latent_size + rope_size] (what the latent backend builds with a concatenation and
+ * a fill: attention_mla.py:246-248, :337-359).  Rows and blocks out of range are skipped, as in the fill.
+ */
+int ttpa_paged_fill_latent(void *cache, const void *latent, int64_t latent_user_stride, int64_t latent_token_stride,
+                           const void *rope, int64_t rope_user_stride, int64_t rope_token_stride,
+                           const int32_t *page_table, int64_t page_table_row_stride, int32_t users,
+                           int32_t table_rows, int32_t seq_len, int32_t block_size, int32_t latent_size,
+                           int32_t rope_size, int32_t table_width, int32_t num_blocks, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

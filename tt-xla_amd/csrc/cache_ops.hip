@@ -109,6 +109,10 @@ struct FillArgs {
   const void *bidx;
   int bidx_i64;
   int fill_users, table_rows, hkv, s, bs, d, w, nb;
+  // latent rows: elements from head_elems on come from here, and fill row i belongs to table row i; or null
+  const uint16_t *tail;
+  int64_t tail_us, tail_ts;
+  int head_elems;
   // floor(2^32 / divisor) + 1 for the two per-thread divisions (by the threads of a token row
   // and by the block size), or 0 where the multiply-high quotient would not be exact
   uint32_t tpr_magic, bs_magic;
@@ -125,7 +129,7 @@ inline uint32_t magic_for(int64_t max_dividend, int d) {
 
 // Block of token t of fill row i, and the token's row inside it.
 __device__ __forceinline__ bool resolve_fill(const FillArgs &a, int i, int t, int &phys, int &off) {
-  int64_t b = a.bidx ? load_index(a.bidx, a.bidx_i64, i) : 0;
+  int64_t b = a.bidx ? load_index(a.bidx, a.bidx_i64, i) : a.tail ? i : 0;
   if (b < 0 || b >= a.table_rows) return false;
   const int col = fast_div(t, a.bs, a.bs_magic);
   off = t - col * a.bs;
@@ -147,6 +151,7 @@ __global__ __launch_bounds__(256) void fill_bf16_kernel(FillArgs a) {
   int phys, off;
   if (!resolve_fill(a, i, t, phys, off)) return;
   const uint16_t *src = (second ? a.fill2 : a.fill) + i * a.fill_us + h * a.fill_hs + t * a.fill_ts + chunk * VEC;
+  if (a.tail && chunk * VEC >= a.head_elems) src = a.tail + i * a.tail_us + t * a.tail_ts + (chunk * VEC - a.head_elems);
   uint16_t *dst = static_cast<uint16_t *>(second ? a.cache2 : a.cache) +
                   (((int64_t)phys * a.hkv + h) * a.bs + off) * a.d + chunk * VEC;
   if constexpr (VEC == 8) {
@@ -285,7 +290,7 @@ static int launch_fill(void *cache, void *cache2, const void *fill, const void *
              page_table, page_table_row_stride,
              batch_idx,  batch_idx_is_i64,
              fill_users, table_rows, kv_heads, seq_len, block_size, head_size, table_width,
-             num_blocks, 0u, 0u};
+             num_blocks, nullptr, 0, 0, 0, 0u, 0u};
   hipStream_t st = static_cast<hipStream_t>(stream);
   const bool vec_ok = head_size % 8 == 0 && aligned16(cache) && aligned16(fill) &&
                       (!cache2 || (aligned16(cache2) && aligned16(fill2))) &&
@@ -343,4 +348,32 @@ extern "C" int ttpa_paged_fill_cache_kv(void *k_cache, void *v_cache, const void
                      fill_token_stride, page_table, page_table_row_stride, batch_idx,
                      batch_idx_is_i64, fill_users, table_rows, kv_heads, seq_len, block_size,
                      head_size, table_width, num_blocks, kv_format, stream);
+}
+
+extern "C" int ttpa_paged_fill_latent(void *cache, const void *latent, int64_t latent_user_stride, int64_t latent_token_stride,
+                                      const void *rope, int64_t rope_user_stride, int64_t rope_token_stride,
+                                      const int32_t *page_table, int64_t page_table_row_stride, int32_t users, int32_t table_rows,
+                                      int32_t seq_len, int32_t block_size, int32_t latent_size, int32_t rope_size,
+                                      int32_t table_width, int32_t num_blocks, void *stream) {
+  const int32_t row = latent_size + rope_size;
+  if (int rc = common_checks(cache, latent, page_table, 1, block_size, row, table_width, num_blocks, TTPA_KV_BF16)) return rc;
+  TTPA_REQUIRE(rope && latent_size > 0 && rope_size > 0, "latent fill: missing part");
+  TTPA_REQUIRE(users >= 0 && seq_len >= 0 && table_rows > 0, "bad users / seq_len / table_rows");
+  TTPA_REQUIRE((int64_t)seq_len <= (int64_t)table_width * block_size, "seq_len %d does not fit %d page-table columns of %d tokens",
+               seq_len, table_width, block_size);
+  TTPA_REQUIRE(latent_size % 8 == 0 && rope_size % 8 == 0 && aligned16(cache) && aligned16(latent) && aligned16(rope) &&
+                   latent_user_stride % 8 == 0 && latent_token_stride % 8 == 0 && rope_user_stride % 8 == 0 && rope_token_stride % 8 == 0,
+               "latent fill: rows must be 16-byte aligned");
+  const int64_t threads = (int64_t)seq_len * (row / 8);
+  TTPA_REQUIRE(threads < (int64_t)1 << 31 && users <= 65535, "fill too large for one launch");
+  if (users == 0 || seq_len == 0) return TTPA_OK;
+  FillArgs a{};
+  a.cache = cache, a.fill = static_cast<const uint16_t *>(latent);
+  a.fill_us = latent_user_stride, a.fill_ts = latent_token_stride;
+  a.tail = static_cast<const uint16_t *>(rope), a.tail_us = rope_user_stride, a.tail_ts = rope_token_stride, a.head_elems = latent_size;
+  a.pt = page_table, a.pt_rs = page_table_row_stride;
+  a.fill_users = users, a.table_rows = table_rows, a.hkv = 1, a.s = seq_len, a.bs = block_size, a.d = row, a.w = table_width, a.nb = num_blocks;
+  a.tpr_magic = magic_for(threads, row / 8), a.bs_magic = magic_for(seq_len, block_size);
+  fill_bf16_kernel<8><<<dim3((unsigned)((threads + 255) / 256), 1, (unsigned)users), dim3(256), 0, static_cast<hipStream_t>(stream)>>>(a);
+  return check_launch("paged_fill_latent");
 }

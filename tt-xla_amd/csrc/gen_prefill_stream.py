@@ -2,8 +2,9 @@
 """Writes the hand-scheduled loop of the streaming prefill kernel (head size 128, 32 query rows of one
 head per wavefront, two workgroups of four wavefronts per CU) as one block of gfx950 assembly per
 form of the loop: build/prefill_stream_asm.h, included by prefill_stream.hip.  The forms: dense
-K / V, dense with a sliding window, paged K / V in cache blocks of whole 64-key tiles, and in cache
-blocks of whole 32-key blocks.
+K / V, dense with a sliding window, dense with keys of 128 + 64 features (the second part, the rotary
+one, with base and strides of its own), paged K / V in cache blocks of whole 64-key tiles, and in
+cache blocks of whole 32-key blocks.
 
 Why assembly: the loop wants the matrix pipe and the vector ALU of a SIMD busy at the same time
 from one instruction stream, with every register chosen by hand (256 per wavefront at two
@@ -41,7 +42,7 @@ slot j % NS.  Iteration i reads K block i + 1 and V block i - 1 and, through the
 reads, the first fragments of K block i + 2 and V block i.  Its barrier, at its start, says that
 nobody reads K block i and V block i - 2 any more; K block i + NS and V block i + NS - 2 are
 requested into their slots (LDS-DMA loads, two per tensor and wavefront).  A request has to have
-landed NS - 2 barriers later: the wait in front of a barrier lets the requests of the last two
+landed NS - 2 barriers later: the wait in front of a barrier lets the requests of the last NS - 3
 barriers stay in flight (vmcnt(8)), so a tile has three iterations to arrive with NS = 5, where
 two stages of whole tiles gave it two.  Once requests have been skipped (no such block) the wait
 is for everything.  Dense K / V: a block is `stride` bytes behind the one before.  Paged (block
@@ -52,6 +53,10 @@ odd iteration (so the same wait covers it) and read at the next odd one.  Entrie
 of its own; the one of K block i + NS is read in iteration i and was requested in iteration i - 2 in
 front of the tile requests, so the same wait covers it (vmcnt(8), not 10: near the end an iteration
 requests no entry any more).  V follows two blocks behind K, so two byte offsets wait in a queue.
+
+Keys of 128 + 64 features: S(i) is 12 matrix instructions, an iteration 20; a block of the second part
+is 4 KiB (one load per wavefront), in a ring of its own behind the other two.  With rings of NS = 4
+the three still fit 80 KiB, half of a CU's LDS, and a request has two iterations to arrive.
 
 A workgroup may take only a part of the keys (paged forms): it starts at any block, and if the base
 of a partial result is given, the accumulators go out as they are, with the reference and the sum of
@@ -100,6 +105,7 @@ LIMIT = 212                    # last visible key of the lane's row, minus 4 h (
 LIMREL, NEGINF, VZERO = 213, 214, 215
 QBASE, OUTBASE = 216, 218      # per lane, 64-bit: q / out of row 0 of the lane's head, at the lane's 8 h / 4 h elements (inputs)
 VN, V4H = 220, 221             # lane % 32 and 4 (lane / 32) (inputs)
+QFP, KOFFP, LDKP = 228, 244, 248  # keys of 128 + 64: Q fragments, LDS addresses and global offsets of the second part (inputs)
 OUTP, PTMP, VT0, VROW = 222, 224, 226, 227
 CLOBBERED = (list(range(0, QF)) + list(range(S[0], RING + 4 * NSLOT)) + list(range(MC, MCN + 1)) + [LOWREL, LIMIT, LIMREL, NEGINF, VZERO]
              + list(range(OUTP, VROW + 1)))
@@ -117,6 +123,8 @@ S_MASKFROM = "s74"             # blocks whose first key is >= this are masked
 S_KEY0 = "s75"                 # first key of the block whose softmax comes next (input: of the first block)
 S_STATS, S_PART = "s[36:37]", "s[38:39]"  # paged: where (reference, sum) and the accumulators of a part go (0: the whole result)
 S_LOWTO = "s34"                # window: blocks whose first key is < this are masked from below (input)
+# keys of 128 + 64 only: the second part of K, its bytes per block and the LDS address of the wavefront's segment; V's bytes per block
+S_PBASE, S_PSTRIDE, S_M0P, S_VSTRIDE = "s[30:31]", "s32", "s33", "s35"
 # paged only
 S_HKV, S_HK, S_NCB, S_TPB = "s76", "s77", "s78", "s79"  # kv heads, this kv head, cache blocks, tiles per cache block
 S_CIN = "s80"                  # tile-in-cache-block index of the tile whose entry is read next
@@ -139,23 +147,27 @@ S_STOREMASK = "s[60:61]"
 # temporaries s[88:95], s[62:63]
 SCALAR_CLOBBERS = [f"s{r}" for r in list(range(88, 96)) + [60, 61, 62, 63, 74]]
 
-NS = 5                         # slots per ring
-UNROLL = 10                    # lcm(2, NS): score bank and slots repeat
-SLOT = 8192
-VRING = NS * SLOT              # LDS offset of the V ring; VOFF carries it
+SLOT, PSLOT = 8192, 4096       # bytes of a block of K or V, of the second part of K
 KEY_CONST = [8 * (r // 4) + r % 4 for r in range(16)]
 
 
 class Form:
     """What one block of assembly serves."""
 
-    def __init__(self, name, paged=0, window=False):
+    def __init__(self, name, paged=0, window=False, wide=False):
         self.name, self.paged, self.window = name, paged, window  # paged: 0 or the keys that share a table entry
-        self.items = not window and paged != 32  # several row blocks in turn
+        self.wide = wide                    # keys of 128 + 64 features
+        self.ns = 4 if wide else 5          # slots per ring
+        self.unroll = 4 if wide else 10     # lcm(2, ns): score bank and slots repeat
+        self.vring = self.ns * SLOT         # LDS offset of the V ring (VOFF carries it), of the second part's ring (KOFFP)
+        self.pring = 2 * self.vring
+        self.loads = 5 if wide else 4       # tile loads of an iteration
+        self.items = not window and not wide and paged != 32  # several row blocks in turn
         self.parts = paged > 0  # may take a part of the keys
 
 
-FORMS = [Form("DENSE"), Form("DENSE_WINDOW", window=True), Form("PAGED", paged=64), Form("PAGED32", paged=32)]
+FORMS = [Form("DENSE"), Form("DENSE_WINDOW", window=True), Form("DENSE_WIDE", wide=True), Form("PAGED", paged=64),
+         Form("PAGED32", paged=32)]
 START_REFERENCE = "0xff7fffff"  # the lowest finite float
 
 
@@ -178,6 +190,8 @@ def frag_reads(frag, slot):
     """LDS read instructions of a fragment into ring slot `slot`.
     ("K", LDS slot, k-step) or ("V", LDS slot, key step 0 / 1, output block)."""
     base = RING + 4 * slot
+    if frag[0] == "K" and frag[2] >= 8:
+        return [f"ds_read_b128 {vr(base, 4)}, v{KOFFP + frag[2] - 8} offset:{frag[1] * PSLOT}"]
     if frag[0] == "K":
         _, ls, ks = frag
         return [f"ds_read_b128 {vr(base, 4)}, v{KOFF + ks} offset:{ls * SLOT}"]
@@ -192,7 +206,8 @@ def mfma(m, slot):
     if m[0] == "S":
         _, bank, ks = m
         d = vr(S[bank], 16)
-        return f"v_mfma_f32_32x32x16_bf16 {d}, {a}, {vr(QF + 4 * ks, 4)}, {'0' if ks == 0 else d}"
+        q = QF + 4 * ks if ks < 8 else QFP + 4 * (ks - 8)
+        return f"v_mfma_f32_32x32x16_bf16 {d}, {a}, {vr(q, 4)}, {'0' if ks == 0 else d}"
     _, db, bank, k4p = m
     d = vr(ACC[db], 16)
     return f"v_mfma_f32_32x32x16_bf16 {d}, {a}, {vr(P[bank] + 4 * k4p, 4)}, {d}"
@@ -237,40 +252,48 @@ def spread(ops, nslots, first=0):
     return out
 
 
-def stream(o, pairs, valu_chunks, in_flight, tail):
+def stream(o, pairs, valu_chunks, phase, in_flight, tail):
     """pairs: [(matrix instruction, fragment)].  Per pair: wait for its fragment, the matrix
-    instruction, the read of the fragment NSLOT pairs on, the vector chunk.  in_flight: the first
-    NSLOT fragments have been requested by the code in front (else they are requested here);
-    tail: the fragments requested behind the last NSLOT pairs (the next iteration's first ones)."""
+    instruction, the read of the fragment NSLOT pairs on, the vector chunk.  phase: the ring slot of the
+    first pair's fragment; in_flight: the first NSLOT fragments have been requested by the code in front
+    (else they are requested here); tail: the fragments requested behind the last NSLOT pairs (the next
+    iteration's first ones).  Returns the next phase."""
     frags = [f for _, f in pairs] + list(tail)
     n = len(pairs)
     count = lambda f: len(frag_reads(frags[f], 0))
     if not in_flight:
         for f in range(min(NSLOT, len(frags))):
-            for x in frag_reads(frags[f], f % NSLOT):
+            for x in frag_reads(frags[f], (phase + f) % NSLOT):
                 o.e(x)
     for j in range(n):
         after = sum(count(f) for f in range(j + 1, min(j + NSLOT, len(frags))))
         assert after <= 15
         o.e(f"s_waitcnt lgkmcnt({after})")
-        o.e(mfma(pairs[j][0], j % NSLOT))
+        o.e(mfma(pairs[j][0], (phase + j) % NSLOT))
         if j + NSLOT < len(frags):
-            for x in frag_reads(frags[j + NSLOT], j % NSLOT):
+            for x in frag_reads(frags[j + NSLOT], (phase + j) % NSLOT):
                 o.e(x)
         for x in valu_chunks[j]:
             o.e(x)
+    return (phase + n) % NSLOT
 
 
-def iteration_pairs(p, has_pv=True):
-    """Iteration i = p (mod UNROLL): S(i + 1) into bank 1 - q from K block i + 1, PV(i - 1) from
+def score_pairs(bank, slot, f):
+    return [(("S", bank, x), ("K", slot, x)) for x in range(12 if f.wide else 8)]
+
+
+def iteration_pairs(p, f, has_pv=True):
+    """Iteration i = p (mod f.unroll): S(i + 1) into bank 1 - q from K block i + 1, PV(i - 1) from
     bank 1 - q of the probabilities and V block i - 1."""
     q = p % 2
-    pairs = []
-    for x in range(8):
-        pairs.append((("S", 1 - q, x), ("K", (p + 1) % NS, x)))
-        if has_pv:
-            pairs.append((("PV", x % 4, 1 - q, x // 4), ("V", (p - 1) % NS, x // 4, x % 4)))
-    return pairs
+    scores = score_pairs(1 - q, (p + 1) % f.ns, f)
+    if not has_pv:
+        return scores
+    pv = [(("PV", x % 4, 1 - q, x // 4), ("V", (p - 1) % f.ns, x // 4, x % 4)) for x in range(8)]
+    order = "SPSSPSPSSPSPSSPSPSSP" if f.wide else "SP" * 8
+    assert order.count("S") == len(scores) and order.count("P") == 8
+    scores, pv = iter(scores), iter(pv)
+    return [next(scores if x == "S" else pv) for x in order]
 
 
 def mask_block(o, f, q, tag):
@@ -345,10 +368,11 @@ def two_loads(o, lane_regs, base):
         o.e(f"global_load_lds_dwordx4 v{lane_regs + j}, {base} offset:{1024 * j}")
 
 
-def request_block(o, which, slot, tag, paged, half):
+def request_block(o, f, which, slot, tag, half):
     """One K or V block into LDS slot `slot` of its ring, if there is one left to request.
     paged: the block is half `half` of the tile at S_OFFK / S_OFFV."""
-    left, lane, base, ring = (S_KLEFT, LDK, S_KBASE, 0) if which == "K" else (S_VLEFT, LDV, S_VBASE, VRING)
+    paged = f.paged
+    left, lane, base, ring = (S_KLEFT, LDK, S_KBASE, 0) if which == "K" else (S_VLEFT, LDV, S_VBASE, f.vring)
     o.e(f"s_cmp_eq_u32 {left}, 0")
     o.e(f"s_cbranch_scc1 L_no{which}_{tag}%=")
     if paged:
@@ -364,8 +388,14 @@ def request_block(o, which, slot, tag, paged, half):
     two_loads(o, lane, "s[90:91]" if paged else base)
     if not paged:
         b0 = int(base[2:4])
-        o.e(f"s_add_u32 s{b0}, s{b0}, {S_STRIDE}")
+        o.e(f"s_add_u32 s{b0}, s{b0}, {S_VSTRIDE if f.wide and which == 'V' else S_STRIDE}")
         o.e(f"s_addc_u32 s{b0 + 1}, s{b0 + 1}, 0")
+    if f.wide and which == "K":
+        o.e(f"s_add_u32 m0, {S_M0P}, {slot * PSLOT}")
+        o.e("s_nop 0")
+        o.e(f"global_load_lds_dwordx4 v{LDKP}, {S_PBASE}")
+        o.e(f"s_add_u32 s30, s30, {S_PSTRIDE}")
+        o.e("s_addc_u32 s31, s31, 0")
     o.e(f"s_sub_u32 {left}, {left}, 1")
     o.label(f"L_no{which}_{tag}")
 
@@ -431,13 +461,13 @@ def next_block(o, p, tag):
 
 
 def iteration_head(o, f, p, tag):
-    """Mask, barrier and requests of iteration i = p (mod UNROLL)."""
-    paged = f.paged
+    """Mask, barrier and requests of iteration i = p (mod f.unroll)."""
+    paged, ns = f.paged, f.ns
     mask_block(o, f, p % 2, tag)
-    # requests of the last two barriers may stay in flight, unless some were skipped
+    # requests of the last ns - 3 barriers may stay in flight, unless some were skipped
     o.e(f"s_cmp_eq_u32 {S_KLEFT}, 0")
     o.e(f"s_cbranch_scc1 L_all_{tag}%=")
-    o.e("s_waitcnt vmcnt(8)")
+    o.e(f"s_waitcnt vmcnt({(ns - 3) * f.loads})")
     o.e(f"s_branch L_bar_{tag}%=")
     o.label(f"L_all_{tag}")
     o.e("s_waitcnt vmcnt(0)")
@@ -448,9 +478,9 @@ def iteration_head(o, f, p, tag):
     if paged == 32:
         next_block(o, p, tag)
     # K block i + NS is half (i + NS) % 2 of its tile, V block i + NS - 2 the same half of its own
-    half = (p + NS) % 2 if paged == 64 else 0
-    request_block(o, "K", p % NS, tag, paged, half)
-    request_block(o, "V", (p + NS - 2) % NS, tag, paged, half)
+    half = (p + ns) % 2 if paged == 64 else 0
+    request_block(o, f, "K", p % ns, tag, half)
+    request_block(o, f, "V", (p + ns - 2) % ns, tag, half)
     if paged == 32:
         o.e("s_mov_b64 s[84:85], s[98:99]")
         o.e("s_mov_b64 s[98:99], s[86:87]")
@@ -465,9 +495,9 @@ def iteration_tail(o, tag, exit_label):
     o.e(f"s_cbranch_scc1 {exit_label}%=")
 
 
-def first_frags(p):
-    """The first NSLOT fragments of iteration p (mod UNROLL)."""
-    return [f for _, f in iteration_pairs(p % UNROLL)[:NSLOT]]
+def first_frags(p, f):
+    """The first NSLOT fragments of iteration p (mod f.unroll)."""
+    return [frag for _, frag in iteration_pairs(p % f.unroll, f)[:NSLOT]]
 
 
 def item_setup(o, tag):
@@ -617,7 +647,7 @@ def next_item(o, f):
     else:
         o.e("s_mov_b64 s[64:65], s[50:51]")
         o.e("s_mov_b64 s[66:67], s[52:53]")
-    for ln in generate_first(paged, "nx"):
+    for ln in generate_first(f, "nx"):
         o.lines.append(ln)
     epilogue(o)
     item_setup(o, "nx")
@@ -629,11 +659,12 @@ def next_item(o, f):
 FIRST32 = ("s[50:51]", "s[52:53]", "s[58:59]", "s[84:85]", "s[98:99]")  # blocks of 32: the first five byte offsets
 
 
-def generate_first(paged, suffix=""):
-    """The first requests: K blocks 0 .. NS - 1, V blocks 0 .. NS - 3 (a block of its own, so that
+def generate_first(f, suffix=""):
+    """The first requests: K blocks 0 .. ns - 1, V blocks 0 .. ns - 3 (a block of its own, so that
     the caller can put its Q loads behind them)."""
     o = Out()
-    for j in range(NS):
+    paged = f.paged
+    for j in range(f.ns):
         if paged:  # tiles 0, 1, 2 at S_OFF0, S_OFFV, S_OFFK; blocks of 32: 0 .. 4
             src = ("s[98:99]", S_OFFV, S_OFFK)[j // 2] if paged == 64 else FIRST32[j]
             lo = int(src[2:4])
@@ -650,8 +681,8 @@ def generate_first(paged, suffix=""):
             o.e(f"s_sub_u32 {S_KLEFT}, {S_KLEFT}, 1")
             o.label(f"L_noK_pro{j}{suffix}")
         else:
-            request_block(o, "K", j, f"pro{j}{suffix}", False, 0)
-    for j in range(NS - 2):
+            request_block(o, f, "K", j, f"pro{j}{suffix}", 0)
+    for j in range(f.ns - 2):
         if paged:
             src = ("s[98:99]", S_OFFV)[j // 2] if paged == 64 else FIRST32[j]
             lo = int(src[2:4])
@@ -662,61 +693,69 @@ def generate_first(paged, suffix=""):
             if j % 2 and paged == 64:
                 o.e(f"s_add_u32 s90, s90, {SLOT}")
                 o.e("s_addc_u32 s91, s91, 0")
-            o.e(f"s_add_u32 m0, {S_M0B}, {VRING + j * SLOT}")
+            o.e(f"s_add_u32 m0, {S_M0B}, {f.vring + j * SLOT}")
             o.e("s_nop 0")
             two_loads(o, LDV, "s[90:91]")
             o.e(f"s_sub_u32 {S_VLEFT}, {S_VLEFT}, 1")
             o.label(f"L_noV_pro{j}{suffix}")
         else:
-            request_block(o, "V", j, f"pro{j}{suffix}", False, 0)
+            request_block(o, f, "V", j, f"pro{j}{suffix}", 0)
     return o.lines
 
 
 def generate(f):
     o = Out()
-    assert NS == 5 and UNROLL == 10
+    assert (f.ns, f.unroll) in ((5, 10), (4, 4))
     o.e(f"v_mov_b32 v{VZERO}, 0")
     item_setup(o, "first")
     o.label("L_item_top")
     o.e("s_waitcnt vmcnt(0)")
     o.e("s_barrier")
     # ---- S(0) from K block 0; behind it the fragments of iteration 0 (K block 1) ------------------
-    pairs = [(("S", 0, x), ("K", 0, x)) for x in range(8)]
-    it0 = iteration_pairs(0, has_pv=False)
-    stream(o, pairs, [[] for _ in pairs], False, [f for _, f in it0])
+    pairs = score_pairs(0, 0, f)
+    it0 = iteration_pairs(0, f, has_pv=False)
+    phase = stream(o, pairs, [[] for _ in pairs], 0, False, [frag for _, frag in it0[:NSLOT]])
     # ---- iteration 0: S(1), sm(0) ---------------------------------------------------------------
     o.e("s_nop 7")
     iteration_head(o, f, 0, "i0")
-    stream(o, it0, spread(softmax_ops(0), 8), True, first_frags(1))
+    phase = stream(o, it0, spread(softmax_ops(0), len(it0)), phase, True, first_frags(1, f))
     iteration_tail(o, "i0", "L_exit0")
-    # ---- iterations 1 .. : ten in a row, then round again -------------------------------------------
-    for k in range(UNROLL):
-        p = (k + 1) % UNROLL
+    phases = {0: phase}  # ring slot of the next iteration's first fragment, behind iteration p
+    # ---- iterations 1 .. : `unroll` in a row, then round again -----------------------------------------
+    for k in range(f.unroll):
+        p = (k + 1) % f.unroll
         o.label(f"L_it{p}")
         iteration_head(o, f, p, f"p{p}")
-        stream(o, iteration_pairs(p), spread(softmax_ops(p % 2), 16), True, first_frags(p + 1))
+        pairs = iteration_pairs(p, f)
+        phase = stream(o, pairs, spread(softmax_ops(p % 2), len(pairs)), phase, True, first_frags(p + 1, f))
+        assert phases.setdefault(p, phase) == phase  # (iteration 0 and iteration `unroll` share an exit)
         iteration_tail(o, f"p{p}", f"L_exit{p}")
     o.e("s_branch L_it1%=")
 
-    # ---- exits: PV of the last block i = p (mod UNROLL) -----------------------------------------------
-    # The ring holds the first eight fragments of the iteration that is not coming: slots 1, 3, 5, 7
-    # are V block i, key step 0, output blocks 0..3; slots 0, 2, 4, 6 (K fragments nobody needs) take
-    # key step 1.
-    for p in range(UNROLL):
+    # ---- exits: PV of the last block i = p (mod unroll) -----------------------------------------------
+    # The ring holds the first fragments of the iteration that is not coming, some of V block i among
+    # them; the others take the slots of the K fragments nobody needs.
+    for p in range(f.unroll):
         o.label(f"L_exit{p}")
         o.e("s_waitcnt lgkmcnt(0)")
-        for db in range(4):
-            for x in frag_reads(("V", p % NS, 1, db), 2 * db):
+        held = {frag: (phases[p] + j) % NSLOT for j, frag in enumerate(first_frags(p + 1, f)) if frag[0] == "V"}
+        wanted = [("V", p % f.ns, x // 4, x % 4) for x in range(8)]
+        free = [x for x in range(NSLOT) if x not in held.values()]
+        missing = [frag for frag in wanted if frag not in held]
+        slots = dict(held)
+        for frag in missing:
+            slots[frag] = free.pop(0)
+            for x in frag_reads(frag, slots[frag]):
                 o.e(x)
-        for db in range(4):
-            o.e(mfma(("PV", db, p % 2, 0), 2 * db + 1))
+        for frag in sorted(held, key=wanted.index):
+            o.e(mfma(("PV", frag[3], p % 2, frag[2]), slots[frag]))
         o.e("s_waitcnt lgkmcnt(0)")
-        for db in range(4):
-            o.e(mfma(("PV", db, p % 2, 1), 2 * db))
+        for frag in missing:
+            o.e(mfma(("PV", frag[3], p % 2, frag[2]), slots[frag]))
         o.e("s_branch L_end%=")
 
     slow_path(o, 0, "L_slow_i0", "L_join_i0")
-    for p in range(UNROLL):
+    for p in range(f.unroll):
         slow_path(o, p % 2, f"L_slow_p{p}", f"L_join_p{p}")
     o.label("L_end")
     o.e("s_nop 15")
@@ -733,7 +772,7 @@ def main():
     with open(out, "w") as f:
         f.write("// Generated by gen_prefill_stream.py; do not edit.\n#pragma once\n")
         for form in FORMS:
-            for macro, lines in ((f"TTPA_STREAM_FIRST_TEXT_{form.name}", generate_first(form.paged)),
+            for macro, lines in ((f"TTPA_STREAM_FIRST_TEXT_{form.name}", generate_first(form)),
                                  (f"TTPA_STREAM_LOOP_TEXT_{form.name}", generate(form))):
                 f.write(f"#define {macro} \\\n")
                 for ln in lines:
@@ -741,7 +780,11 @@ def main():
                 f.write('  ""\n')
         regs = ", ".join([f'"v{r}"' for r in CLOBBERED] + [f'"{r}"' for r in SCALAR_CLOBBERS])
         f.write(f"#define TTPA_STREAM_LOOP_CLOBBERS {regs}\n")
-        f.write(f"#define TTPA_STREAM_LDS_BYTES {2 * NS * SLOT}\n#define TTPA_STREAM_V_RING {VRING}\n")
+        lds = {form.pring + (form.ns * PSLOT if form.wide else 0) for form in FORMS}
+        assert len(lds) == 1  # every form takes half of a CU's LDS
+        wide = next(form for form in FORMS if form.wide)
+        f.write(f"#define TTPA_STREAM_LDS_BYTES {lds.pop()}\n#define TTPA_STREAM_V_RING {FORMS[0].vring}\n"
+                f"#define TTPA_STREAM_WIDE_V_RING {wide.vring}\n#define TTPA_STREAM_WIDE_P_RING {wide.pring}\n")
 
 
 if __name__ == "__main__":

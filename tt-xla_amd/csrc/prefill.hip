@@ -862,3 +862,47 @@ extern "C" int ttpa_sdpa_prefill_fill(
                       q_len, kv_len, head_size, block_size, table_width, num_blocks, causal, scale,
                       sliding_window, stream, &fill);
 }
+
+extern "C" int ttpa_split_key_prefill(
+    void *out, int64_t out_batch_stride, int64_t out_head_stride, int64_t out_token_stride, const void *q_nope,
+    int64_t q_nope_batch_stride, int64_t q_nope_head_stride, int64_t q_nope_token_stride, const void *q_rope,
+    int64_t q_rope_batch_stride, int64_t q_rope_head_stride, int64_t q_rope_token_stride, const void *k_nope,
+    int64_t k_nope_batch_stride, int64_t k_nope_head_stride, int64_t k_nope_token_stride, const void *k_rope,
+    int64_t k_rope_batch_stride, int64_t k_rope_head_stride, int64_t k_rope_token_stride, const void *v,
+    int64_t v_batch_stride, int64_t v_head_stride, int64_t v_token_stride, int32_t batch, int32_t q_heads,
+    int32_t kv_heads, int32_t seq_len, float scale, void *stream) {
+  TTPA_REQUIRE(out && q_nope && q_rope && k_nope && k_rope && v, "null pointer argument");
+  TTPA_REQUIRE(batch > 0 && q_heads > 0 && kv_heads > 0 && seq_len > 0, "non-positive dimension");
+  TTPA_REQUIRE(q_heads % kv_heads == 0, "q_heads %d not divisible by kv_heads %d", q_heads, kv_heads);
+  TTPA_REQUIRE(seq_len % 32 == 0, "split-key prefill: seq_len %d is not a multiple of 32", seq_len);
+  TTPA_REQUIRE(scale > 0.f, "split-key prefill: scale %g must be positive", (double)scale);
+  TTPA_REQUIRE(aligned16(out) && aligned16(q_nope) && aligned16(q_rope) && aligned16(k_nope) && aligned16(k_rope) && aligned16(v),
+               "split-key prefill: operands must be 16-byte aligned");
+  const int64_t strides[] = {q_nope_batch_stride, q_nope_head_stride, q_nope_token_stride, q_rope_batch_stride, q_rope_head_stride,
+                             q_rope_token_stride, k_nope_batch_stride, k_nope_head_stride, k_nope_token_stride, k_rope_batch_stride,
+                             k_rope_head_stride, k_rope_token_stride, v_batch_stride, v_head_stride, v_token_stride};
+  for (int64_t s : strides) TTPA_REQUIRE(s % 8 == 0, "split-key prefill: operand strides must be multiples of 8 elements");
+  TTPA_REQUIRE(out_batch_stride % 4 == 0 && out_head_stride % 4 == 0 && out_token_stride % 4 == 0,
+               "split-key prefill: out strides must be multiples of 4 elements");
+  TTPA_REQUIRE(k_nope_token_stride < (1 << 24) && k_rope_token_stride < (1 << 24) && v_token_stride < (1 << 24) &&
+                   q_nope_token_stride < (1ll << 31) && out_token_stride < (1ll << 31),
+               "split-key prefill: token stride out of range");
+  TTPA_REQUIRE((int64_t)batch * q_heads * ((seq_len + 31) / 32) < (1ll << 30),
+               "split-key prefill: batch * heads * query tiles too large for one launch");
+  PrefillArgs a = {};
+  a.out = static_cast<uint16_t *>(out);
+  a.out_bs = out_batch_stride, a.out_hs = out_head_stride, a.out_ts = out_token_stride;
+  a.q = static_cast<const uint16_t *>(q_nope);
+  a.q_bs = q_nope_batch_stride, a.q_hs = q_nope_head_stride, a.q_ts = q_nope_token_stride;
+  a.q2 = static_cast<const uint16_t *>(q_rope);
+  a.q2_bs = q_rope_batch_stride, a.q2_hs = q_rope_head_stride, a.q2_ts = q_rope_token_stride;
+  a.k = static_cast<const uint16_t *>(k_nope);
+  a.kv_bs = k_nope_batch_stride, a.kv_hs = k_nope_head_stride, a.kv_ts = k_nope_token_stride;
+  a.k2 = static_cast<const uint16_t *>(k_rope);
+  a.k2_bs = k_rope_batch_stride, a.k2_hs = k_rope_head_stride, a.k2_ts = k_rope_token_stride;
+  a.v = static_cast<const uint16_t *>(v);
+  a.v_bs = v_batch_stride, a.v_hs = v_head_stride, a.v_ts = v_token_stride;
+  a.batch = batch, a.hq = q_heads, a.hkv = kv_heads, a.sq = seq_len, a.skv = seq_len, a.causal = 1, a.parts = 1;
+  a.scale_log2e = scale * 1.4426950408889634f;
+  return launch_stream_wide(a, static_cast<hipStream_t>(stream));
+}

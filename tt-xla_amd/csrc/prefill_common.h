@@ -54,6 +54,9 @@ struct PrefillArgs {
   // The streaming kernel: workgroups per (batch entry, head group), each taking one or several row blocks
   int spg;
   int spg_even; // > 0: when the row blocks weigh about the same, only this many of them work (equal shares)
+  // ... with keys of 128 + 64 features: the second part of q and k, and V's own strides
+  const uint16_t *q2, *k2;
+  int64_t q2_bs, q2_hs, q2_ts, k2_bs, k2_hs, k2_ts, v_bs, v_hs, v_ts;
   // ... and, paged, several workgroups per row block, each with a part of the keys (scratch from the caller or null)
   float *part_acc;
   int64_t part_bytes;
@@ -165,5 +168,7 @@ bool stream_serves(const PrefillArgs &a, int head_size);
 // Bytes of scratch with which it splits the launch over the keys (0: it would not); stream_serves launches only.
 int64_t stream_part_bytes(const PrefillArgs &a, int head_size);
 int launch_stream(const PrefillArgs &a, hipStream_t st);
+// The streaming kernel for keys of 128 + 64 features (dense, causal or not, kv length a multiple of 32).
+int launch_stream_wide(const PrefillArgs &a, hipStream_t st);
 
 }  // namespace ttpa

@@ -32,7 +32,10 @@ constexpr int kBlockKeys = 32;
 
 // kPaged: cache blocks of whole 64-key tiles (two 32-key blocks share a table entry); kPaged32: of whole
 // 32-key blocks (an entry per block costs scalar instructions in every iteration, not in every other one)
-enum StreamForm { kDense = 0, kDenseWindow = 1, kPaged = 2, kPaged32 = 3 };
+// kDenseWide: keys of 128 + 64 features (the latent layers' prompts with K and V expanded per head): 20 matrix
+// instructions per block of 32 keys; 4 x 2048 tokens, 16 heads: 8.6e10 flop in 100 us, where the absorbed form's
+// 2.9e11 took 281
+enum StreamForm { kDense = 0, kDenseWindow = 1, kPaged = 2, kPaged32 = 3, kDenseWide = 4 };
 
 // The assembly is bound to the registers its text names through constraint strings; everything else it
 // touches is on the clobber list.  The requests of a workgroup's first blocks are a block of assembly of their own, issued in front
@@ -78,6 +81,21 @@ __device__ __forceinline__ void stream_first_paged32(StreamRequests &r, const u3
                : "memory", "scc", "m0", "s90", "s91");
 }
 
+// The second part of the keys: its first block, bytes from a block to the next, the LDS address of the
+// wavefront's segment, V's bytes per block, the lane's offset inside a block.
+struct StreamWide {
+  uint64_t base;
+  uint32_t stride, m0, v_stride;
+};
+
+__device__ __forceinline__ void stream_first_wide(StreamRequests &r, StreamWide &w, const u32x2 &ldk, const u32x2 &ldv, uint32_t ldp) {
+  asm volatile(TTPA_STREAM_FIRST_TEXT_DENSE_WIDE
+               : "+{s[64:65]}"(r.kbase), "+{s[66:67]}"(r.vbase), "+{s[30:31]}"(w.base), "+{s71}"(r.k_requests), "+{s73}"(r.v_requests)
+               : "{v[188:189]}"(ldk), "{v[190:191]}"(ldv), "{v248}"(ldp), "{s68}"(r.stride), "{s72}"(r.m0_base),
+                 "{s32}"(w.stride), "{s33}"(w.m0), "{s35}"(w.v_stride)
+               : "memory", "scc", "m0");
+}
+
 // What a workgroup works on (see gen_prefill_stream.py): which row blocks, and what the block of
 // assembly needs to set one up.
 struct StreamItems {
@@ -121,6 +139,17 @@ __device__ __forceinline__ void stream_items_window(StreamRequests &r, StreamIte
   asm volatile(TTPA_STREAM_LOOP_TEXT_DENSE_WINDOW
                : TTPA_STREAM_COMMON_OUT
                : TTPA_STREAM_COMMON_IN, "{v209}"(lowest), "{s34}"(low_to)
+               : "memory", "vcc", "scc", "m0", "v208", TTPA_STREAM_LOOP_CLOBBERS);
+}
+
+__device__ __forceinline__ void stream_items_wide(StreamRequests &r, StreamItems &it, StreamWide &w, u32x16 q_lo, u32x16 q_hi,
+                                                  u32x16 q_second, const u32x8 &koff, const u32x4 &poff, const u32x4 &voff,
+                                                  const u32x2 &ldk, const u32x2 &ldv, uint32_t ldp, uint64_t q_base, uint64_t out_base,
+                                                  int lane_n, int lane_h4, float c, int nblk) {
+  asm volatile(TTPA_STREAM_LOOP_TEXT_DENSE_WIDE
+               : TTPA_STREAM_COMMON_OUT, "+{s[30:31]}"(w.base)
+               : TTPA_STREAM_COMMON_IN, "{v[228:243]}"(q_second), "{v[244:247]}"(poff), "{v248}"(ldp), "{s32}"(w.stride),
+                 "{s33}"(w.m0), "{s35}"(w.v_stride)
                : "memory", "vcc", "scc", "m0", "v208", TTPA_STREAM_LOOP_CLOBBERS);
 }
 
@@ -198,12 +227,12 @@ template <int HPW, int FORM>
 __global__ __launch_bounds__(256, 2) void prefill_stream_kernel(PrefillArgs a) {
   constexpr int RPW = 4 / HPW;  // row blocks per workgroup
   constexpr int D = kD;
-  constexpr bool PAGED = FORM == kPaged || FORM == kPaged32;
+  constexpr bool PAGED = FORM == kPaged || FORM == kPaged32, WIDE = FORM == kDenseWide;
   using T = Tile<D>;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
 
   int wg = blockIdx.x;
-  if constexpr (!PAGED) {
+  if constexpr (!PAGED && !WIDE) {
     wg = attention_workgroup<D>(a, wg);
     if (wg < 0) return;
   }
@@ -263,7 +292,17 @@ __global__ __launch_bounds__(256, 2) void prefill_stream_kernel(PrefillArgs a) {
     // a block is 8 segments of 1 KiB; wavefront w requests segments 2 w and 2 w + 1
     const int r = (2 * wave + j) * T::RPI + lane / T::CPR, cp = lane % T::CPR;
     ldk[j] = (uint32_t)r * row_bytes + 16u * (uint32_t)(cp ^ T::swz_k(r)) + 1024u - 1024u * j;
-    ldv[j] = (uint32_t)r * row_bytes + 16u * (uint32_t)(cp ^ T::swz_v(r)) + 1024u - 1024u * j;
+    ldv[j] = (uint32_t)r * (WIDE ? 2u * (uint32_t)a.v_ts : row_bytes) + 16u * (uint32_t)(cp ^ T::swz_v(r)) + 1024u - 1024u * j;
+  }
+  StreamWide wide;
+  uint32_t ldp = 0;
+  if constexpr (WIDE) {
+    // a block of the second part is 4 segments of eight 128-byte rows, one per wavefront
+    const int r = 8 * wave + (lane >> 3);
+    ldp = (uint32_t)r * 2u * (uint32_t)a.k2_ts + 16u * (uint32_t)((lane & 7) ^ Tile<64>::swz_k(r));
+    wide.base = uni(reinterpret_cast<uint64_t>(a.k2 + b * a.k2_bs + hk * a.k2_hs));
+    wide.stride = (uint32_t)(2 * kBlockKeys * a.k2_ts), wide.v_stride = (uint32_t)(2 * kBlockKeys * a.v_ts);
+    wide.m0 = uni(lds0 + TTPA_STREAM_WIDE_P_RING + 1024u * (uint32_t)wave);
   }
   sreq.m0_base = uni(lds0 + 2048u * (uint32_t)wave);
   sreq.k_requests = sreq.v_requests = nblk;
@@ -275,10 +314,11 @@ __global__ __launch_bounds__(256, 2) void prefill_stream_kernel(PrefillArgs a) {
   if constexpr (!PAGED) {
     const int64_t head = b * a.kv_bs + hk * a.kv_hs + (int64_t)first_block * kBlockKeys * a.kv_ts;
     kbase0 = uni(reinterpret_cast<uint64_t>(a.k + head) - 1024u);
-    vbase0 = uni(reinterpret_cast<uint64_t>(a.v + head) - 1024u);
+    vbase0 = uni(reinterpret_cast<uint64_t>(a.v + (WIDE ? b * a.v_bs + hk * a.v_hs : head)) - 1024u);
     sreq.kbase = kbase0, sreq.vbase = vbase0;
     sreq.stride = (uint32_t)(2 * kBlockKeys * a.kv_ts);
-    stream_first_dense(sreq, ldk, ldv);
+    if constexpr (WIDE) stream_first_wide(sreq, wide, ldk, ldv, ldp);
+    else stream_first_dense(sreq, ldk, ldv);
   } else {
     // keys that share a table entry are a multiple of a unit (a 64-key tile, a 32-key block); the first FIRST
     // units are requested here, the loop takes raw entries from there on
@@ -329,6 +369,17 @@ __global__ __launch_bounds__(256, 2) void prefill_stream_kernel(PrefillArgs a) {
       q_hi[4 * s] = hi.x, q_hi[4 * s + 1] = hi.y, q_hi[4 * s + 2] = hi.z, q_hi[4 * s + 3] = hi.w;
     }
   }
+  u32x16 q_second;
+  u32x4 po;
+  if constexpr (WIDE) {
+    const uint16_t *qp = a.q2 + b * a.q2_bs + hq * a.q2_hs + (int64_t)min(row0 + n, a.sq - 1) * a.q2_ts + 8 * h;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const uint4 x = *reinterpret_cast<const uint4 *>(qp + 16 * s);
+      q_second[4 * s] = x.x, q_second[4 * s + 1] = x.y, q_second[4 * s + 2] = x.z, q_second[4 * s + 3] = x.w;
+      po[s] = lds0 + TTPA_STREAM_WIDE_P_RING + (uint32_t)(n * 128 + 16 * ((2 * s + h) ^ Tile<64>::swz_k(n)));
+    }
+  }
   // LDS operand addresses of the lane inside slot 0 of the K ring and of the V ring: K fragment of k-step
   // s, V^T fragment of output block db (through the transposing LDS load; the layout of prefill.hip)
   u32x8 ko;
@@ -340,7 +391,7 @@ __global__ __launch_bounds__(256, 2) void prefill_stream_kernel(PrefillArgs a) {
 #pragma unroll
     for (int db = 0; db < 4; ++db) {
       const int c = 4 * db + 2 * (grp & 1) + ((a16 & 3) >> 1);
-      vo[db] = lds0 + TTPA_STREAM_V_RING + (uint32_t)(vr * T::RB + 16 * (c ^ T::swz_v(vr)) + 8 * (a16 & 1));
+      vo[db] = lds0 + (WIDE ? TTPA_STREAM_WIDE_V_RING : TTPA_STREAM_V_RING) + (uint32_t)(vr * T::RB + 16 * (c ^ T::swz_v(vr)) + 8 * (a16 & 1));
     }
   }
   StreamItems it;
@@ -358,6 +409,8 @@ __global__ __launch_bounds__(256, 2) void prefill_stream_kernel(PrefillArgs a) {
     const int lowest = offset + min(row0 + n, a.sq - 1) - a.window + 1 - 4 * h;
     const int low_to = uni(offset + row0 + kRowsPerWave - a.window);
     stream_items_window(sreq, it, q_lo, q_hi, ko, vo, ldk, ldv, q_base, out_base, n, 4 * h, a.scale_log2e, nblk, lowest, low_to);
+  } else if constexpr (WIDE) {
+    stream_items_wide(sreq, it, wide, q_lo, q_hi, q_second, ko, po, vo, ldk, ldv, ldp, q_base, out_base, n, 4 * h, a.scale_log2e, nblk);
   } else if constexpr (FORM == kPaged) {
     stream_items_paged(sreq, it, tab, out_part, q_lo, q_hi, ko, vo, ldk, ldv, q_base, out_base, n, 4 * h, a.scale_log2e, nblk);
   } else {
@@ -486,7 +539,7 @@ int launch_form(const PrefillArgs &a, hipStream_t st) {
     }
   }
   int grid = b.spg * b.parts * ny8 * 8;
-  if (!PAGED && a.fill_kc) grid = grid_with_fill(b, grid, kD);
+  if (!PAGED && FORM != kDenseWide && a.fill_kc) grid = grid_with_fill(b, grid, kD);
   launch_dominant(&prefill_stream_kernel<HPW, FORM>, dim3(grid), dim3(256), (size_t)TTPA_STREAM_LDS_BYTES, st, b);
   if (const int rc = check_launch("sdpa_prefill")) return rc;
   if (b.parts > 1) {
@@ -516,6 +569,14 @@ bool stream_serves(const PrefillArgs &a, int head_size) {
 
 int64_t stream_part_bytes(const PrefillArgs &a, int head_size) {
   return a.pt && stream_serves(a, head_size) ? part_bytes(a, heads_per_workgroup(a)) : 0;
+}
+
+int launch_stream_wide(const PrefillArgs &a, hipStream_t st) {
+  switch (heads_per_workgroup(a)) {
+    case 4: return launch_form<4, kDenseWide>(a, st);
+    case 2: return launch_form<2, kDenseWide>(a, st);
+    default: return launch_form<1, kDenseWide>(a, st);
+  }
 }
 
 int launch_stream(const PrefillArgs &a, hipStream_t st) {

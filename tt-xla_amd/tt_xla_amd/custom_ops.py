@@ -1044,6 +1044,10 @@ def flash_mla_prefill(
             mask_ptr, *mask_strides, b, hq, key.shape[1], s, dh, head_dim_v, int(is_causal), float(scale), _stream(),
         )
         return out
+    if v is not None and (dh, head_dim_v) == (192, 128) and attn_mask is None and scale > 0:
+        # keys of 128 + 64 features: the streaming prefill kernel, 128 or 32 query rows per K / V block
+        _split_key_prefill(q[..., :128], q[..., 128:], k[..., :128], k[..., 128:], v, out, scale)
+        return out
     # other shapes, and a separate V: the decode kernels, query row i of a sequence being a user at
     # position i whose cache is the sequence itself (one block of s tokens, a one-column page table)
     table = torch.zeros((s, 1), dtype=torch.int32, device=query.device)
@@ -1067,6 +1071,75 @@ def flash_mla_prefill(
         _mla_decode_launch(out[i].transpose(0, 1), q[i].transpose(0, 1), k[i : i + 1],
                            None if v is None else v[i : i + 1], table, cur, head_dim_v, scale, None, rows)
     return out
+
+
+def _split_key_prefill(q_nope, q_rope, k_nope, k_rope, value, out, scale):
+    """q_nope [b, heads, s, 128], q_rope [b, heads, s, 64], k_nope [b, kv heads, s, 128], k_rope
+    [b, kv heads or 1, s, 64], value / out [b, kv heads / heads, s, 128], by strides."""
+    b, hq, s, _ = q_nope.shape
+    hkv = k_nope.shape[1]
+    q_nope, q_rope, k_nope, k_rope, value = map(_rows_contiguous, (q_nope, q_rope, k_nope, k_rope, value))
+    _check_out(out, (b, hq, s, 128), "split-key prefill")
+    N.call(
+        "ttpa_split_key_prefill",
+        out.data_ptr(), out.stride(0), out.stride(1), out.stride(2),
+        q_nope.data_ptr(), q_nope.stride(0), q_nope.stride(1), q_nope.stride(2),
+        q_rope.data_ptr(), q_rope.stride(0), q_rope.stride(1), q_rope.stride(2),
+        k_nope.data_ptr(), k_nope.stride(0), k_nope.stride(1), k_nope.stride(2),
+        k_rope.data_ptr(), k_rope.stride(0), k_rope.stride(1) if k_rope.shape[1] == hkv and hkv > 1 else 0, k_rope.stride(2),
+        value.data_ptr(), value.stride(0), value.stride(1), value.stride(2),
+        b, hq, hkv, s, float(scale), _stream(),
+    )
+
+
+@torch.library.custom_op("tt::split_key_prefill_out", mutates_args=["out"], device_types=["cuda"])
+def split_key_prefill_out(
+    q_nope: torch.Tensor,
+    q_rope: torch.Tensor,
+    k_nope: torch.Tensor,
+    k_rope: torch.Tensor,
+    value: torch.Tensor,
+    out: torch.Tensor,
+    scale: float,
+) -> None:
+    """Causal prefill attention with keys in two parts, the prompt pass of a latent layer whose keys and
+    values are expanded per head: scores (q_nope . k_nope + q_rope . k_rope) * scale, q_nope [b, heads, s,
+    128], q_rope [b, heads, s, 64], k_nope [b, kv_heads, s, 128], k_rope [b, kv_heads or 1, s, 64], value
+    [b, kv_heads, s, 128]; writes out [b, heads, s, 128] (any batch / head / token strides).  No counterpart
+    as one operator in the reference (attention_mla.py:230-335 computes the same in absorbed form)."""
+    b, hq, s, d = q_nope.shape
+    hkv = k_nope.shape[1]
+    if (d, q_rope.shape[-1], value.shape[-1]) != (128, 64, 128):
+        raise ValueError(f"built for parts of 128 + 64 features and values of 128, got {d} + {q_rope.shape[-1]} and {value.shape[-1]}")
+    if q_rope.shape[:3] != (b, hq, s) or k_nope.shape != (b, hkv, s, 128) or value.shape != (b, hkv, s, 128) \
+            or k_rope.shape not in ((b, hkv, s, 64), (b, 1, s, 64)) or hq % hkv:
+        raise ValueError("query, key and value shapes do not match")
+    if s % 32:
+        raise ValueError(f"query sequence length must be divisible by 32 but got {s}.")
+    if any(t.dtype != torch.bfloat16 for t in (q_nope, q_rope, k_nope, k_rope, value)):
+        raise ValueError("query, key and value must be bfloat16")
+    _split_key_prefill(q_nope, q_rope, k_nope, k_rope, value, out, scale)
+
+
+@torch.library.custom_op("tt::paged_fill_latent_cache_", mutates_args=["cache"], device_types=["cuda"])
+def paged_fill_latent_cache_(cache: torch.Tensor, latent: torch.Tensor, rope: torch.Tensor, page_table: torch.Tensor) -> None:
+    """``paged_fill_cache_`` of latent rows in two parts: latent [users, s, L] and rope [users, s, R] go to
+    positions 0 .. s - 1 of table rows 0 .. users - 1 of cache [blocks, 1, block_size, L + R] (reference
+    attention_mla.py:246-248, :337-359, without the concatenated copy)."""
+    nb, hkv, bs, d, fmt = _cache_geometry(cache)
+    users, s, lat = latent.shape
+    if fmt != N.KV_BF16 or hkv != 1 or lat + rope.shape[-1] != d or rope.shape[:2] != (users, s):
+        raise ValueError(f"latent {tuple(latent.shape)} and rope {tuple(rope.shape)} do not match the cache {tuple(cache.shape)}")
+    if latent.dtype != cache.dtype or rope.dtype != cache.dtype:
+        raise ValueError("fill_value dtype must match the cache")
+    if page_table.dim() != 2 or s > page_table.shape[1] * bs:
+        raise ValueError(f"{s} tokens do not fit a page table of shape {tuple(page_table.shape)}")
+    latent, rope, pt = _rows_contiguous(latent), _rows_contiguous(rope), _table(page_table)
+    N.call(
+        "ttpa_paged_fill_latent",
+        cache.data_ptr(), latent.data_ptr(), latent.stride(0), latent.stride(1), rope.data_ptr(), rope.stride(0), rope.stride(1),
+        pt.data_ptr(), pt.stride(0), users, pt.shape[0], s, bs, lat, rope.shape[-1], pt.shape[1], nb, _stream(),
+    )
 
 
 @flash_mla_prefill.register_fake
