@@ -43,7 +43,7 @@ struct DecodeArgs {
   const float *sink;  // [q_heads] extra logit per head in the softmax denominator, or null
   // Fused cache update (16x16x32 kernel only): the token at cur_pos of every user is taken from
   // k_new / v_new [users][>= hkv heads][head_size] instead of the cache, and written to it.
-  const uint16_t *k_new, *v_new;
+  const uint16_t *k_new = nullptr, *v_new = nullptr;
   int64_t new_us, new_hs;
   // Additive mask on the scaled scores (bfloat16, natural-log units), or null: the element for
   // (user, query head, position) is mask[user * mask_us + head * mask_hs + position].  Applied by the
@@ -365,6 +365,56 @@ __device__ __forceinline__ void write_partial(float *slot, int g, int G, int r, 
   }
 }
 
+// Where the fresh token of a user with a negative position goes: position -k counts from the end of
+// the user's table (the update operator's floor rule: column = floor(pos / bs) taken from the end
+// once, row = pos mod bs).  False: not negative, or outside the table or the cache (skipped).
+__device__ inline bool negative_slot(const DecodeArgs &a, int u, int &phys, int &row) {
+  const int64_t pos = load_index(a.cur, a.cur_i64, u);
+  if (pos >= 0) return false;
+  int64_t col = pos / a.bs, rem = pos - col * a.bs;
+  if (rem < 0) rem += a.bs, col -= 1;
+  col += a.w;
+  if (col < 0 || col >= a.w) return false;
+  phys = a.pt[(int64_t)u * a.pt_rs + col];
+  row = (int)rem;
+  return (unsigned)phys < (unsigned)a.nb;
+}
+
+// The cache write of a user with a negative position when the step's update is part of the launch: by
+// the 256 threads of a merge workgroup, which has nothing to merge for such a user.  Parked rows of a
+// batch usually share one slot of the null block: the last user wins, as if they wrote in turn.  (As
+// the first wavefront's business, ahead of its tiles, five parked block-float-8 rows of 32 users made
+// the whole attention kernel wait 13 us for that wavefront.)
+__device__ inline void write_negative_position(const DecodeArgs &a, int seg, int D) {
+  const int u = seg / a.hkv, h = seg - u * a.hkv;
+  int phys, row;
+  if (!negative_slot(a, u, phys, row)) return;  // (the same for the whole workgroup)
+  bool later = false;
+  for (int v = u + 1 + (int)threadIdx.x; v < a.users; v += 256) {
+    int p2, r2;
+    later |= negative_slot(a, v, p2, r2) && p2 == phys && r2 == row;
+  }
+  if (__syncthreads_or(later)) return;
+  const int64_t slot = (int64_t)phys * a.hkv + h;
+  for (int i = threadIdx.x; i < 2 * (D / 16); i += 256) {
+    const int t = i / (D / 16), grp = i - t * (D / 16);
+    const uint16_t *src = (t ? a.v_new : a.k_new) + u * a.new_us + h * a.new_hs + 16 * grp;
+    uint8_t *dst = const_cast<uint8_t *>(t ? a.v : a.k);
+    const uint4 lo = *reinterpret_cast<const uint4 *>(src), hi = *reinterpret_cast<const uint4 *>(src + 8);
+    if (a.kv_format == TTPA_KV_BFP8) {
+      uint8_t *slab = dst + slot * (int64_t)(a.bs + a.bs / 16) * D;
+      const uint32_t w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+      uint32_t bytes[4];
+      const uint32_t e = bfp8_encode16(w, bytes);
+      *reinterpret_cast<uint4 *>(slab + (int64_t)row * D + 16 * grp) = make_uint4(bytes[0], bytes[1], bytes[2], bytes[3]);
+      slab[(int64_t)a.bs * D + (int64_t)row * (D / 16) + grp] = (uint8_t)e;
+    } else {
+      uint4 *p = reinterpret_cast<uint4 *>(dst + ((slot * a.bs + row) * D + 16 * grp) * 2);
+      p[0] = lo, p[1] = hi;
+    }
+  }
+}
+
 // Merges the partials of one (user, kv_head) segment and writes bfloat16 output.
 // Partials are read eight at a time so that their loads overlap (with four wavefronts per CU
 // and at least one segment per CU, a segment has about five): the kernel is a chain of
@@ -393,6 +443,7 @@ __global__ inline __launch_bounds__(256) void decode_combine_kernel(DecodeArgs a
   if (nw == 0) {  // padded row: no attended position -> NaN like softmax over nothing
     for (int i = i_begin; i < i_end; i += 256)
       out[(int64_t)(h * G + head_of(i)) * a.out_hs + elem_of(i)] = 0x7fc0;
+    if (a.k_new != nullptr && blockIdx.y == 0) write_negative_position(a, seg, D);
     return;
   }
   constexpr int kBatch = 8;

@@ -20,9 +20,8 @@
 // depends on a separate update launch.  The fresh rows of a segment's (user, head) are
 // requested where its Q rows are, once per segment (that block has its own waits; a request
 // inside the per-tile path would make the wait-count pass drain the tile loads in the
-// steady-state loop).  Users whose position is negative (padded rows) attend nothing; their
-// write follows the update operator's rule for negative positions and is done by the thread
-// that publishes their segment.
+// steady-state loop).  Users whose position is negative (padded rows) attend nothing; their write
+// is the merge kernel's (write_negative_position).
 //
 // v_mfma_f32_16x16x32_{f16,bf16} with the heads as the 16-wide N dimension:
 //   S^T block b (16 keys):  A = K rows 16 b + lane%16, 8 elements per lane and k-step
@@ -87,45 +86,6 @@ __device__ __forceinline__ floatx4 mma16(const u32x4 &x, const u32x4 &y, const f
                                                    __builtin_bit_cast(bf16x8, y), c, 0, 0, 0);
 }
 
-// The cache write of a user whose position is negative, by one thread per (user, kv head):
-// position -k counts from the end of the user's table (the update operator's floor rule:
-// column = floor(pos / bs) taken from the end once, row = pos mod bs); positions that still fall
-// outside the table and blocks outside the cache are skipped.
-template <bool BFP8, int D>
-__device__ inline void write_negative_position(const DecodeArgs &a, const int32_t *page_table,
-                                               const void *cur_pos, int seg) {
-  if (seg >= a.users * a.hkv) return;
-  const int u = seg / a.hkv, h = seg - u * a.hkv;
-  const int64_t pos = load_index(cur_pos, a.cur_i64, u);
-  if (pos >= 0) return;
-  int64_t col = pos / a.bs, rem = pos - col * a.bs;
-  if (rem < 0) rem += a.bs, col -= 1;
-  col += a.w;
-  if (col < 0 || col >= a.w) return;
-  const int phys = page_table[(int64_t)u * a.pt_rs + col];
-  if ((unsigned)phys >= (unsigned)a.nb) return;
-  const uint16_t *src[2] = {a.k_new + u * a.new_us + h * a.new_hs, a.v_new + u * a.new_us + h * a.new_hs};
-  uint8_t *dst[2] = {const_cast<uint8_t *>(a.k), const_cast<uint8_t *>(a.v)};
-  for (int t = 0; t < 2; ++t) {
-    if constexpr (BFP8) {
-      uint8_t *slab = dst[t] + ((int64_t)phys * a.hkv + h) * (int64_t)(a.bs + a.bs / 16) * D;
-      for (int grp = 0; grp < D / 16; ++grp) {
-        const uint4 lo = *reinterpret_cast<const uint4 *>(src[t] + 16 * grp);
-        const uint4 hi = *reinterpret_cast<const uint4 *>(src[t] + 16 * grp + 8);
-        const uint32_t w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-        uint32_t bytes[4];
-        const uint32_t e = bfp8_encode16(w, bytes);
-        *reinterpret_cast<uint4 *>(slab + rem * D + 16 * grp) = make_uint4(bytes[0], bytes[1], bytes[2], bytes[3]);
-        slab[(int64_t)a.bs * D + rem * (D / 16) + grp] = (uint8_t)e;
-      }
-    } else {
-      uint16_t *row = reinterpret_cast<uint16_t *>(dst[t]) + (((int64_t)phys * a.hkv + h) * a.bs + rem) * D;
-      for (int c = 0; c < D / 8; ++c)
-        *reinterpret_cast<uint4 *>(row + 8 * c) = *reinterpret_cast<const uint4 *>(src[t] + 8 * c);
-    }
-  }
-}
-
 // RUNS: 1, 2, 4, or 0 for one run per load.  MASKED: an additive mask row per (user, head) joins the
 // scores (a.mask; the form of a pass that is not causal, built with RUNS = 0 and without the update).
 template <int D, bool BFP8, int RUNS, bool FUSED, bool MASKED = false>
@@ -167,7 +127,6 @@ __global__ __launch_bounds__(256, 1) void paged_decode_mfma16_kernel(
   const int64_t total = (int64_t)total_units * a.hkv;
   const int64_t max_ranges = total / (seg_units + 1);
   const int n_eff = (int)(max_ranges < a.n_waves ? max_ranges : a.n_waves);
-  if constexpr (FUSED) write_negative_position<BFP8, D>(a, page_table, cur_pos, blockIdx.x * 256 + threadIdx.x);
   if (total == 0 || wave >= n_eff) {
     publish_segment_row(a, s_pref, total, n_eff, seg_units);
     return;
