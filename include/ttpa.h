@@ -505,6 +505,30 @@ int ttpa_split_key_prefill(void *out, int64_t out_batch_stride, int64_t out_head
                            int32_t kv_heads, int32_t seq_len, float scale, void *stream);
 
 /*
+ * The decode step of a latent layer in one call (reference attention_mla.py:230-248, :379-422: query absorption,
+ * cache write of the new token's latent key at cur_pos, paged latent attention, output expansion), for heads of
+ * 128 + 64 query features over a latent width of 512 and values of 128:
+ *   q_lat[u, n] = (q_nope[u, n] . W_UK[n], q_rope[u, n]) rounded to bfloat16;
+ *   cache[slot(cur_pos[u])] = (latent[u], rope[u]) as ttpa_paged_update_cache writes it;
+ *   o_lat = ttpa_paged_mla_decode(q_lat, cache, V = the 512 leading features);
+ *   out[u, n] = o_lat[u, n] . W_UV[n].
+ * w_uk [heads, 128, 512] and w_uv [heads, 512, 128] by head and row strides (innermost contiguous), the
+ * activations by user (and head) strides; strides multiples of 8 elements (out's of 4), 16-byte aligned pointers.
+ * Four or five launches on the stream; the scratch (256-byte aligned, the size below; 0: these head counts are
+ * not built) holds nothing between calls.
+ */
+int ttpa_latent_decode_step(void *out, int64_t out_user_stride, int64_t out_head_stride, const void *q_nope,
+                            int64_t q_nope_user_stride, int64_t q_nope_head_stride, const void *q_rope,
+                            int64_t q_rope_user_stride, int64_t q_rope_head_stride, const void *latent,
+                            int64_t latent_user_stride, const void *rope, int64_t rope_user_stride, const void *w_uk,
+                            int64_t w_uk_head_stride, int64_t w_uk_row_stride, const void *w_uv,
+                            int64_t w_uv_head_stride, int64_t w_uv_row_stride, void *cache, const int32_t *page_table,
+                            int64_t page_table_row_stride, const void *cur_pos, int cur_pos_is_i64, int32_t users,
+                            int32_t heads, int32_t block_size, int32_t table_width, int32_t num_blocks, float scale,
+                            void *workspace, size_t workspace_bytes, void *stream);
+size_t ttpa_latent_decode_step_workspace_bytes(int32_t users, int32_t heads);
+
+/*
  * paged_fill_cache of latent rows that are still in two parts: row t of user u, [latent_size] from `latent` and
  * [rope_size] from `rope` behind it, goes to position t of page-table row u in a cache
  * [num_blocks, 1, block_size, latent_size + rope_size] (what the latent backend builds with a concatenation and

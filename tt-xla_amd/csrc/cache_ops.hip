@@ -25,18 +25,7 @@ struct UpdateArgs {
 
 // Resolves (user) -> (physical block, row offset); false = skip this user.
 __device__ __forceinline__ bool resolve_update(const UpdateArgs &a, int u, int &phys, int &off) {
-  int64_t pos = load_index(a.idx, a.idx_i64, u);
-  int64_t col = pos / a.bs;
-  int64_t rem = pos - col * a.bs;
-  if (rem < 0) {  // floor semantics for negative positions
-    rem += a.bs;
-    col -= 1;
-  }
-  if (col < 0) col += a.w;  // a negative column indexes from the end, once
-  if (col < 0 || col >= a.w) return false;
-  phys = a.pt[(int64_t)u * a.pt_rs + col];
-  off = (int)rem;
-  return (unsigned)phys < (unsigned)a.nb;
+  return update_slot(a.idx, a.idx_i64, a.pt, a.pt_rs, a.bs, a.w, a.nb, u, phys, off);
 }
 
 template <int VEC>  // VEC = 8 (16-byte chunks) or 1 (element-wise, unaligned operands)

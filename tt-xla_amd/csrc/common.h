@@ -91,6 +91,21 @@ __device__ __forceinline__ int64_t load_index(const void *p, int is_i64, int64_t
                 : static_cast<int64_t>(static_cast<const int32_t *>(p)[i]);
 }
 
+// Where the token that user u writes at its position goes (the update operator's rule): the row of the
+// block that the table names for column floor(pos / bs); a negative column counts from the end,
+// once.  False: outside the table or the cache, the user writes nothing.
+__device__ __forceinline__ bool update_slot(const void *pos_ptr, int pos_i64, const int32_t *pt, int64_t pt_rs, int bs, int w, int nb,
+                                            int u, int &phys, int &row) {
+  const int64_t pos = load_index(pos_ptr, pos_i64, u);
+  int64_t col = pos / bs, rem = pos - col * bs;
+  if (rem < 0) rem += bs, col -= 1;
+  if (col < 0) col += w;
+  if (col < 0 || col >= w) return false;
+  phys = pt[(int64_t)u * pt_rs + col];
+  row = (int)rem;
+  return (unsigned)phys < (unsigned)nb;
+}
+
 // ---- block-float-8 ---------------------------------------------------------
 // A group of 16 values shares the exponent byte e (largest biased bfloat16 exponent of the
 // group); an element byte is 128 + v with the signed mantissa v in [-127, 127] and decodes

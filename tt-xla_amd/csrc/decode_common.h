@@ -365,19 +365,10 @@ __device__ __forceinline__ void write_partial(float *slot, int g, int G, int r, 
   }
 }
 
-// Where the fresh token of a user with a negative position goes: position -k counts from the end of
-// the user's table (the update operator's floor rule: column = floor(pos / bs) taken from the end
-// once, row = pos mod bs).  False: not negative, or outside the table or the cache (skipped).
+// Where the fresh token of a user with a negative position goes (update_slot); false: not negative, or
+// nowhere.
 __device__ inline bool negative_slot(const DecodeArgs &a, int u, int &phys, int &row) {
-  const int64_t pos = load_index(a.cur, a.cur_i64, u);
-  if (pos >= 0) return false;
-  int64_t col = pos / a.bs, rem = pos - col * a.bs;
-  if (rem < 0) rem += a.bs, col -= 1;
-  col += a.w;
-  if (col < 0 || col >= a.w) return false;
-  phys = a.pt[(int64_t)u * a.pt_rs + col];
-  row = (int)rem;
-  return (unsigned)phys < (unsigned)a.nb;
+  return load_index(a.cur, a.cur_i64, u) < 0 && update_slot(a.cur, a.cur_i64, a.pt, a.pt_rs, a.bs, a.w, a.nb, u, phys, row);
 }
 
 // The cache write of a user with a negative position when the step's update is part of the launch: by

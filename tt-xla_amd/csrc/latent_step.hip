@@ -1,0 +1,221 @@
+// The decode step of a latent layer in one call: around the latent attention kernels (decode_wide.hip)
+// the projections of the layer, without the concatenated copies in between.
+//
+//   latent_query_kernel  q_lat[u, n] = (q_nope[u, n] . W_UK[n], q_rope[u, n]), and the new token's row
+//                        (latent, rope) of every user goes into the paged cache
+//   latent attention     o_lat[u, n] over the paged cache (its own launches)
+//   latent_value_kernel  out[u, n] = o_lat[u, n] . W_UV[n]
+//
+// Both kernels are short: 2 MB of weights and 2 - 4 MB of activations for 128 users of 16 heads, bounded by
+// the trip to memory and back.  So the split is for many small workgroups: (128 latent columns, head, 32
+// users) for the query, (32 value columns, head, 32 users) with the contraction over the latent width cut
+// between the four wavefronts for the value.  A weight tile travels memory -> LDS directly and is read
+// through the transposing LDS load, so that v_mfma_f32_32x32x16_bf16 gets the users as its columns and
+// the activations go from memory to registers as they are.  128 users, 16 heads: 8.2 and 5.0 us, where two
+// batched library products, two concatenations, the cache write and the copy to the output took 41 us in six
+// launches; the whole pass over contexts of 512 .. 8192 168 -> 94 us, of one user over 512 tokens 149 -> 37 us.
+#include "common.h"
+
+#include <algorithm>
+
+namespace ttpa {
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef short shortx4 __attribute__((ext_vector_type(4)));
+
+constexpr int kNope = 128, kRope = 64, kLatent = 512, kValue = 128;
+constexpr int kRow = kLatent + kRope;
+constexpr int kUsers = 32;  // users per workgroup: the 32-wide dimension of the matrix instruction
+
+struct StepArgs {
+  const uint16_t *q_nope, *q_rope, *latent, *rope, *w_uk, *w_uv;
+  int64_t qn_us, qn_hs, qr_us, qr_hs, latent_us, rope_us, uk_hs, uk_rs, uv_hs, uv_rs;
+  uint16_t *q_lat, *o_lat;  // [users][heads][kRow], [users][heads][kLatent]
+  uint16_t *out;
+  int64_t out_us, out_hs;
+  uint16_t *cache;
+  const int32_t *pt;
+  int64_t pt_rs;
+  const void *pos;
+  int pos_i64;
+  int users, heads, bs, w, nb;
+};
+
+// A operand of a 32x32x16 instruction from rows 16 s .. 16 s + 15 (k) and 32 columns (m) of a weight tile in LDS:
+// lane (m, h) receives column m of rows 8 h .. 8 h + 7.  `first` addresses the lane's 8 bytes of rows
+// 8 h .. 8 h + 3 (row 8 h + (lane % 16) / 4), `half` is the byte distance of four rows.
+__device__ __forceinline__ bf16x8 read_transposed(const unsigned char *first, int half) {
+  typedef __attribute__((address_space(3))) shortx4 *lds_v4;
+  const shortx4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4)first);
+  const shortx4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4)(first + half));
+  struct {
+    shortx4 a, b;
+  } t = {lo, hi};
+  return __builtin_bit_cast(bf16x8, t);
+}
+
+__global__ __launch_bounds__(256) void latent_query_kernel(StepArgs a) {
+  __shared__ __attribute__((aligned(1024))) unsigned char tile[kNope * 256];  // 128 rows of 128 columns
+  const int col0 = blockIdx.x * 128, head = blockIdx.y, u0 = blockIdx.z * kUsers;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 31, h = lane >> 5;
+
+  // weights: 32 segments of four rows; 16-byte chunk c of row r lies at chunk position c ^ 4 (r % 4), which puts the
+  // four rows of a transposing read in different banks
+  const uint16_t *w = a.w_uk + head * a.uk_hs + col0;
+  const uint32_t lane_bytes = (uint32_t)(lane >> 4) * (uint32_t)(2 * a.uk_rs) + 16u * (uint32_t)((lane & 15) ^ (4 * (lane >> 4)));
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int seg = 8 * wave + j;
+    dma16_uniform(w + (int64_t)(4 * seg) * a.uk_rs, lane_bytes, lds_address(tile) + 1024u * (uint32_t)seg);
+  }
+  const int u = min(u0 + n, a.users - 1);
+  bf16x8 q[8];
+  const uint16_t *qp = a.q_nope + u * a.qn_us + head * a.qn_hs + 8 * h;
+#pragma unroll
+  for (int s = 0; s < 8; ++s) q[s] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(qp + 16 * s));
+
+  if (blockIdx.x == 0) {  // the rotary part of the query, as it is: 8 chunks per user
+    const int v = u0 + (tid >> 3), c = 8 * (tid & 7);
+    if (v < a.users)
+      *reinterpret_cast<uint4 *>(a.q_lat + ((int64_t)v * a.heads + head) * kRow + kLatent + c) =
+          *reinterpret_cast<const uint4 *>(a.q_rope + v * a.qr_us + head * a.qr_hs + c);
+  }
+  if (head == 0) {  // the new token's row: 128 latent columns per workgroup, the rotary part with the first
+    const int chunks = 16 + (blockIdx.x == 0 ? 8 : 0);
+    for (int i = tid; i < kUsers * chunks; i += 256) {
+      const int v = u0 + i / chunks, c = i % chunks;
+      int phys, row;
+      if (v >= a.users || !update_slot(a.pos, a.pos_i64, a.pt, a.pt_rs, a.bs, a.w, a.nb, v, phys, row)) continue;
+      const int at = c < 16 ? col0 + 8 * c : kLatent + 8 * (c - 16);
+      const uint16_t *src = c < 16 ? a.latent + v * a.latent_us + at : a.rope + v * a.rope_us + 8 * (c - 16);
+      *reinterpret_cast<uint4 *>(a.cache + ((int64_t)phys * a.bs + row) * kRow + at) = *reinterpret_cast<const uint4 *>(src);
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's segments have landed
+  __syncthreads();
+
+  floatx16 acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  const int grp = lane >> 4, a16 = lane & 15;
+  const int row = 8 * (grp >> 1) + (a16 >> 2), chunk = 4 * wave + 2 * (grp & 1) + ((a16 & 3) >> 1);
+  const unsigned char *first = tile + row * 256 + 16 * (chunk ^ (4 * (row & 3))) + 8 * (a16 & 1);
+#pragma unroll
+  for (int s = 0; s < 8; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(read_transposed(first + s * 16 * 256, 4 * 256), q[s], acc, 0, 0, 0);
+  if (u0 + n >= a.users) return;
+  uint16_t *dst = a.q_lat + ((int64_t)(u0 + n) * a.heads + head) * kRow + col0 + 32 * wave + 4 * h;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    *reinterpret_cast<uint2 *>(dst + 8 * j) = make_uint2(pack_bf16x2(acc[4 * j], acc[4 * j + 1]), pack_bf16x2(acc[4 * j + 2], acc[4 * j + 3]));
+}
+
+__global__ __launch_bounds__(256) void latent_value_kernel(StepArgs a) {
+  constexpr int kPitch = 36;  // floats of a user's partial sums: rows of 16-byte writes in different banks
+  __shared__ __attribute__((aligned(1024))) unsigned char tile[kLatent * 64];  // 512 rows of 32 columns, 128 per wavefront
+  __shared__ __attribute__((aligned(16))) float sums[4][kUsers * kPitch];
+  const int col0 = blockIdx.x * 32, head = blockIdx.y, u0 = blockIdx.z * kUsers;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 31, h = lane >> 5;
+  // weights: 8 segments of sixteen 64-byte rows per wavefront (four rows of a transposing read are 256 consecutive bytes)
+  const uint16_t *w = a.w_uv + head * a.uv_hs + (int64_t)(128 * wave) * a.uv_rs + col0;
+  const uint32_t lane_bytes = (uint32_t)(lane >> 2) * (uint32_t)(2 * a.uv_rs) + 16u * (uint32_t)(lane & 3);
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+    dma16_uniform(w + (int64_t)(16 * j) * a.uv_rs, lane_bytes, lds_address(tile) + 8192u * (uint32_t)wave + 1024u * j);
+  const int u = min(u0 + n, a.users - 1);
+  bf16x8 o[8];
+  const uint16_t *op = a.o_lat + ((int64_t)u * a.heads + head) * kLatent + 128 * wave + 8 * h;
+#pragma unroll
+  for (int s = 0; s < 8; ++s) o[s] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(op + 16 * s));
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // a wavefront reads the segments that it requested
+
+  floatx16 acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  const int grp = lane >> 4, a16 = lane & 15;
+  const unsigned char *first = tile + 8192 * wave + (8 * (grp >> 1) + (a16 >> 2)) * 64 + 32 * (grp & 1) + 8 * (a16 & 3);
+#pragma unroll
+  for (int s = 0; s < 8; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(read_transposed(first + s * 16 * 64, 4 * 64), o[s], acc, 0, 0, 0);
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    *reinterpret_cast<float4 *>(&sums[wave][n * kPitch + 8 * j + 4 * h]) = make_float4(acc[4 * j], acc[4 * j + 1], acc[4 * j + 2], acc[4 * j + 3]);
+  __syncthreads();
+  const int v = tid >> 3, c = 4 * (tid & 7);
+  if (u0 + v >= a.users) return;
+  float4 t = *reinterpret_cast<const float4 *>(&sums[0][v * kPitch + c]);
+#pragma unroll
+  for (int k = 1; k < 4; ++k) {
+    const float4 x = *reinterpret_cast<const float4 *>(&sums[k][v * kPitch + c]);
+    t.x += x.x, t.y += x.y, t.z += x.z, t.w += x.w;
+  }
+  *reinterpret_cast<uint2 *>(a.out + (u0 + v) * a.out_us + head * a.out_hs + col0 + c) = make_uint2(pack_bf16x2(t.x, t.y), pack_bf16x2(t.z, t.w));
+}
+
+inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
+
+}  // namespace
+}  // namespace ttpa
+
+using namespace ttpa;
+
+extern "C" size_t ttpa_latent_decode_step_workspace_bytes(int32_t users, int32_t heads) {
+  if (users <= 0 || heads <= 0) return 0;
+  const size_t attn = ttpa_paged_mla_decode_workspace_bytes(users, heads, 1, kLatent);
+  if (attn == 0) return 0;
+  return align256(attn) + align256((size_t)users * heads * kRow * 2) + align256((size_t)users * heads * kLatent * 2);
+}
+
+extern "C" int ttpa_latent_decode_step(
+    void *out, int64_t out_user_stride, int64_t out_head_stride, const void *q_nope, int64_t q_nope_user_stride,
+    int64_t q_nope_head_stride, const void *q_rope, int64_t q_rope_user_stride, int64_t q_rope_head_stride, const void *latent,
+    int64_t latent_user_stride, const void *rope, int64_t rope_user_stride, const void *w_uk, int64_t w_uk_head_stride,
+    int64_t w_uk_row_stride, const void *w_uv, int64_t w_uv_head_stride, int64_t w_uv_row_stride, void *cache,
+    const int32_t *page_table, int64_t page_table_row_stride, const void *cur_pos, int cur_pos_is_i64, int32_t users,
+    int32_t heads, int32_t block_size, int32_t table_width, int32_t num_blocks, float scale, void *workspace,
+    size_t workspace_bytes, void *stream) {
+  TTPA_REQUIRE(out && q_nope && q_rope && latent && rope && w_uk && w_uv && cache && page_table && cur_pos, "null pointer argument");
+  TTPA_REQUIRE(users > 0 && heads > 0 && block_size > 0 && table_width > 0 && num_blocks > 0, "non-positive dimension");
+  TTPA_REQUIRE(aligned16(q_nope) && aligned16(q_rope) && aligned16(latent) && aligned16(rope) && aligned16(w_uk) && aligned16(w_uv) &&
+                   aligned16(cache) && (reinterpret_cast<uintptr_t>(out) & 7u) == 0,
+               "latent step: operands must be 16-byte aligned");
+  const int64_t strides[] = {q_nope_user_stride, q_nope_head_stride, q_rope_user_stride, q_rope_head_stride, latent_user_stride,
+                             rope_user_stride, w_uk_head_stride, w_uk_row_stride, w_uv_head_stride, w_uv_row_stride};
+  for (int64_t s : strides) TTPA_REQUIRE(s % 8 == 0, "latent step: strides must be multiples of 8 elements");
+  TTPA_REQUIRE(out_user_stride % 4 == 0 && out_head_stride % 4 == 0, "latent step: out strides must be multiples of 4 elements");
+  TTPA_REQUIRE(w_uk_row_stride > 0 && w_uk_row_stride < (1 << 24) && w_uv_row_stride > 0 && w_uv_row_stride < (1 << 24),
+               "latent step: weight row stride out of range");
+  TTPA_REQUIRE(heads <= 65535 && (users + kUsers - 1) / kUsers <= 65535, "latent step: too many heads or users for one launch");
+  const size_t need = ttpa_latent_decode_step_workspace_bytes(users, heads);
+  if (need == 0) return fail(TTPA_ERR_UNSUPPORTED, "latent step: %d heads are not built", heads);
+  if (!workspace || workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 255u))
+    return fail(TTPA_ERR_WORKSPACE, "latent step: workspace of %zu bytes (256-byte aligned) required, got %zu", need, workspace_bytes);
+  const size_t attn = align256(ttpa_paged_mla_decode_workspace_bytes(users, heads, 1, kLatent));
+  StepArgs a;
+  a.q_nope = static_cast<const uint16_t *>(q_nope), a.qn_us = q_nope_user_stride, a.qn_hs = q_nope_head_stride;
+  a.q_rope = static_cast<const uint16_t *>(q_rope), a.qr_us = q_rope_user_stride, a.qr_hs = q_rope_head_stride;
+  a.latent = static_cast<const uint16_t *>(latent), a.latent_us = latent_user_stride;
+  a.rope = static_cast<const uint16_t *>(rope), a.rope_us = rope_user_stride;
+  a.w_uk = static_cast<const uint16_t *>(w_uk), a.uk_hs = w_uk_head_stride, a.uk_rs = w_uk_row_stride;
+  a.w_uv = static_cast<const uint16_t *>(w_uv), a.uv_hs = w_uv_head_stride, a.uv_rs = w_uv_row_stride;
+  a.q_lat = reinterpret_cast<uint16_t *>(static_cast<unsigned char *>(workspace) + attn);
+  a.o_lat = reinterpret_cast<uint16_t *>(reinterpret_cast<unsigned char *>(a.q_lat) + align256((size_t)users * heads * kRow * 2));
+  a.out = static_cast<uint16_t *>(out), a.out_us = out_user_stride, a.out_hs = out_head_stride;
+  a.cache = static_cast<uint16_t *>(cache);
+  a.pt = page_table, a.pt_rs = page_table_row_stride, a.pos = cur_pos, a.pos_i64 = cur_pos_is_i64;
+  a.users = users, a.heads = heads, a.bs = block_size, a.w = table_width, a.nb = num_blocks;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const unsigned tiles = (unsigned)((users + kUsers - 1) / kUsers);
+  latent_query_kernel<<<dim3(kLatent / 128, (unsigned)heads, tiles), dim3(256), 0, st>>>(a);
+  if (int rc = check_launch("latent_decode_step (query)")) return rc;
+  if (int rc = ttpa_paged_mla_decode(a.o_lat, (int64_t)heads * kLatent, kLatent, a.q_lat, (int64_t)heads * kRow, kRow, cache, nullptr,
+                                     page_table, page_table_row_stride, cur_pos, cur_pos_is_i64, users, heads, 1, kRow, kLatent,
+                                     block_size, table_width, num_blocks, scale, nullptr, workspace, attn, stream))
+    return rc;
+  latent_value_kernel<<<dim3(kValue / 32, (unsigned)heads, tiles), dim3(256), 0, st>>>(a);
+  return check_launch("latent_decode_step (value)");
+}

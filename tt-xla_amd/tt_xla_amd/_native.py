@@ -105,6 +105,12 @@ SIGNATURES = {
          _i64, _i64, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _f32, _i32, _i32, _p, _i64, _p],
     ),
     "ttpa_sdpa_prefill_workspace_bytes": (_i64, [_i32, _i32, _i32, _i32, _i32, _i32]),
+    "ttpa_latent_decode_step_workspace_bytes": (_sz, [_i32, _i32]),
+    "ttpa_latent_decode_step": (
+        _int,
+        [_p, _i64, _i64, _p, _i64, _i64, _p, _i64, _i64, _p, _i64, _p, _i64, _p, _i64, _i64, _p, _i64, _i64,
+         _p, _p, _i64, _p, _int, _i32, _i32, _i32, _i32, _i32, _f32, _p, _sz, _p],
+    ),
     "ttpa_split_key_prefill": (
         _int, [_p, _i64, _i64, _i64] * 6 + [_i32, _i32, _i32, _i32, _f32, _p],
     ),

@@ -21,7 +21,9 @@ What a forward pass does, in the order of the reference:
 Differences from the reference, invisible in results: a causal prompt pass at the head shape
 128 + 64 / 128 expands K and V per head instead of absorbing the query (``_expands_prompts``: the same
 sums with the products grouped the other way; four prompts of 2048 tokens, 16 heads: 763 -> 164 us, and
-the error against a 64-bit evaluation stays at 3.4e-3 of the output); the cache writes use the in-place
+the error against a 64-bit evaluation stays at 3.4e-3 of the output); a causal decode pass at that shape and a
+latent width of 512 is one operator (``tt::latent_decode_step_``: the same steps and roundings without the
+copies between them; 128 users, 16 heads: 168 -> 94 us); the cache writes use the in-place
 operators (one batched fill instead of a per-user loop over functional fills followed by a
 copy of the whole cache); ``functional_cache_ops=True`` restores the reference's call sequence.
 
@@ -167,6 +169,13 @@ class TTMLAAttentionBackendImpl(_ImplBase):
             self._forward_prefill_expanded(q_nope, q_pe, kv_c_normed, k_pe, kv_cache, attn_metadata, layer, s, users, output)
             return
 
+        if not prefill and self._steps_at_once(q_nope, q_pe, kv_c_normed, k_pe, kv_cache, attn_metadata, layer, output):
+            # projections, cache write and attention without the copies in between
+            torch.ops.tt.latent_decode_step_(
+                q_nope, q_pe, kv_c_normed.view(users, lat), k_pe.view(users, rope), layer.W_UK_T, layer.W_UV, kv_cache,
+                attn_metadata.page_table, attn_metadata.cache_position, output.view(users, n, self.v_head_dim), float(self.scale))
+            return
+
         act_dtype, device = q_pe.dtype, q_nope.device
         # W_UK_T is a plain attribute of the layer, not a parameter: it may still sit elsewhere
         w_uk_t = layer.W_UK_T.to(device=device)
@@ -197,6 +206,20 @@ class TTMLAAttentionBackendImpl(_ImplBase):
     def _expand(self, out_lat: torch.Tensor, layer, pattern: str) -> torch.Tensor:
         return torch.einsum(pattern, out_lat, layer.W_UV.to(device=out_lat.device))
 
+    def _bf16_on_gpu(self, *tensors) -> bool:
+        return all(t.device.type == "cuda" and t.dtype == torch.bfloat16 for t in tensors)
+
+    def _steps_at_once(self, q_nope, q_pe, kv_c_normed, k_pe, kv_cache, attn_metadata, layer, output) -> bool:
+        """Whether a decode pass is one ``tt::latent_decode_step_``: the head shape it is built for, causal, with a
+        cache to write.  (Without a cache the pass is a profiling run, which the operators in turn refuse.)"""
+        if (self.qk_nope_head_dim, self.qk_rope_head_dim, self.kv_lora_rank, self.v_head_dim) != (128, 64, 512, 128):
+            return False
+        if self.functional_cache_ops or not attn_metadata.is_causal or not self._has_cache(kv_cache) or not kv_cache.is_contiguous():
+            return False
+        if not self._bf16_on_gpu(q_nope, q_pe, kv_c_normed, k_pe, layer.W_UK_T, layer.W_UV, kv_cache, output):
+            return False
+        return output.is_contiguous() and output.data_ptr() % 16 == 0
+
     def _expands_prompts(self, q_nope, q_pe, kv_c_normed, k_pe, kv_cache, attn_metadata, layer, s, output) -> bool:
         """A prompt pass attends only its own tokens, so K and V can be expanded per head (scores over
         nope + rope features, values of v_head_dim) where the absorbed form works on kv_lora_rank +
@@ -206,8 +229,7 @@ class TTMLAAttentionBackendImpl(_ImplBase):
             return False
         if attn_metadata is not None and (attn_metadata.attn_mask is not None or not attn_metadata.is_causal):
             return False
-        tensors = (q_nope, q_pe, kv_c_normed, k_pe, layer.W_UK_T, layer.W_UV, output)
-        if not all(t.device.type == "cuda" and t.dtype == torch.bfloat16 for t in tensors) or not self.scale > 0:
+        if not self._bf16_on_gpu(q_nope, q_pe, kv_c_normed, k_pe, layer.W_UK_T, layer.W_UV, output) or not self.scale > 0:
             return False
         if attn_metadata is not None and self._has_cache(kv_cache) and kv_cache.dtype != torch.bfloat16:
             return False

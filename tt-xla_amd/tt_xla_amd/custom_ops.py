@@ -1121,6 +1121,57 @@ def split_key_prefill_out(
     _split_key_prefill(q_nope, q_rope, k_nope, k_rope, value, out, scale)
 
 
+@torch.library.custom_op("tt::latent_decode_step_", mutates_args=["cache", "out"], device_types=["cuda"])
+def latent_decode_step_(
+    q_nope: torch.Tensor,
+    q_rope: torch.Tensor,
+    latent: torch.Tensor,
+    rope: torch.Tensor,
+    w_uk_t: torch.Tensor,
+    w_uv: torch.Tensor,
+    cache: torch.Tensor,
+    page_table: torch.Tensor,
+    cur_pos_tensor: torch.Tensor,
+    out: torch.Tensor,
+    scale: float,
+) -> None:
+    """The decode step of a latent layer as one operator (reference attention_mla.py:230-248, :379-422): absorbs
+    w_uk_t [heads, 128, 512] into q_nope [users, heads, 128], writes (latent [users, 512], rope [users, 64]) to
+    the cache [blocks, 1, block_size, 576] at cur_pos_tensor, attends, and writes the expansion with w_uv
+    [heads, 512, 128] to out [users, heads, 128].  The same roundings as the operators in turn (the absorbed
+    query and the latent output are bfloat16)."""
+    users, heads, nope = q_nope.shape
+    nb, nkv, bs, row = cache.shape
+    if (nope, q_rope.shape[-1], latent.shape[-1], w_uv.shape[-1], nkv, row) != (128, 64, 512, 128, 1, 576):
+        raise ValueError("the latent step is built for 128 + 64 query features, a latent width of 512 and values of 128")
+    if (q_rope.shape[:2] != (users, heads) or latent.shape[0] != users or rope.shape != (users, 64)
+            or w_uk_t.shape != (heads, 128, 512) or w_uv.shape != (heads, 512, 128) or out.shape != (users, heads, 128)):
+        raise ValueError("query, weight and output shapes do not match")
+    if any(t.dtype != torch.bfloat16 for t in (q_nope, q_rope, latent, rope, w_uk_t, w_uv, cache, out)) or not cache.is_contiguous():
+        raise ValueError("the latent step takes bfloat16 tensors and a contiguous cache")
+    if page_table.dim() != 2 or page_table.shape[0] != users or cur_pos_tensor.shape != (users,):
+        raise ValueError("page_table / cur_pos_tensor must have one row per user")
+    q_nope, q_rope, latent, rope, w_uk_t, w_uv = map(_rows_contiguous, (q_nope, q_rope, latent, rope, w_uk_t, w_uv))
+    if out.stride(-1) != 1 or out.data_ptr() % 16 or out.stride(0) % 4 or out.stride(1) % 4:
+        raise ValueError("latent step: out needs contiguous 16-byte aligned rows and strides that are multiples of 4")
+    pt, cur = _table(page_table), _index_tensor(cur_pos_tensor)
+    for u0 in range(0, users, _MLA_MAX_USERS):
+        n = min(_MLA_MAX_USERS, users - u0)
+        ws_bytes = N.lib().ttpa_latent_decode_step_workspace_bytes(n, heads)
+        if ws_bytes == 0:
+            raise NotImplementedError(f"latent attention with {heads} query heads over one KV head is not built")
+        ws = _workspace(ws_bytes, out.device)
+        at = lambda t: t.data_ptr() + u0 * t.stride(0) * t.element_size()  # noqa: E731
+        N.call(
+            "ttpa_latent_decode_step",
+            at(out), out.stride(0), out.stride(1), at(q_nope), q_nope.stride(0), q_nope.stride(1),
+            at(q_rope), q_rope.stride(0), q_rope.stride(1), at(latent), latent.stride(0), at(rope), rope.stride(0),
+            w_uk_t.data_ptr(), w_uk_t.stride(0), w_uk_t.stride(1), w_uv.data_ptr(), w_uv.stride(0), w_uv.stride(1),
+            cache.data_ptr(), at(pt), pt.stride(0), at(cur), int(cur.dtype == torch.int64), n, heads, bs, pt.shape[1], nb,
+            float(scale), ws.data_ptr(), ws_bytes, _stream(),
+        )
+
+
 @torch.library.custom_op("tt::paged_fill_latent_cache_", mutates_args=["cache"], device_types=["cuda"])
 def paged_fill_latent_cache_(cache: torch.Tensor, latent: torch.Tensor, rope: torch.Tensor, page_table: torch.Tensor) -> None:
     """``paged_fill_cache_`` of latent rows in two parts: latent [users, s, L] and rope [users, s, R] go to
