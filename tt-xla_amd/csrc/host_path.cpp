@@ -1,0 +1,178 @@
+// The eager host path of the attention backend: one Python call takes the tensors of a pass to the C ABI.
+//
+// A pass of a few microseconds of GPU time (a short prompt, one user's decode step) is bound by the host:
+// through Python views, the operator registry and ctypes it issues in 33 .. 55 us.  This module reads
+// addresses, sizes and strides from the tensors directly and calls the same entry points with the same
+// arguments.  It serves exactly the ordinary form of a pass (plain bfloat16 rows on the current device, the
+// caches' layouts, int32 tables); for anything else it answers None before it has issued anything, and the
+// caller's general path takes the pass, raises what is to be raised and converts what is to be
+// converted.  Scratch comes from the caching allocator on the current stream, call by call: nothing is kept
+// between calls, so streams, threads and graph captures need no care of their own.
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <ATen/ATen.h>
+#include <ATen/core/grad_mode.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+
+#include "ttpa.h"
+
+namespace {
+
+// Largest scratch a pass may ask for (the operators' limit).
+constexpr int64_t kScratchLimit = int64_t(8) << 30;
+
+struct Pass {
+  int device;
+  bool grad;
+
+  // A plain tensor on the current device that autograd does not watch; null otherwise.
+  const at::Tensor *plain(PyObject *o) const {
+    if (!THPVariable_CheckExact(o)) return nullptr;
+    const at::Tensor &t = THPVariable_Unpack(o);
+    if (!t.defined() || !t.is_cuda() || t.get_device() != device || t.layout() != at::kStrided) return nullptr;
+    if (grad && t.requires_grad()) return nullptr;
+    return &t;
+  }
+  // [rows, cols] bfloat16 with contiguous, 16-byte aligned rows.
+  const at::Tensor *rows(PyObject *o, int64_t cols) const {
+    const at::Tensor *t = plain(o);
+    if (!t || t->scalar_type() != at::kBFloat16 || t->dim() != 2 || t->size(1) != cols || t->stride(1) != 1 || t->stride(0) % 8 ||
+        reinterpret_cast<uintptr_t>(t->data_ptr()) % 16)
+      return nullptr;
+    return t;
+  }
+  const at::Tensor *table(PyObject *o) const {
+    const at::Tensor *t = plain(o);
+    return t && t->scalar_type() == at::kInt && t->dim() == 2 && t->stride(1) == 1 ? t : nullptr;
+  }
+  // `n` whole numbers, int32 or int64.
+  const at::Tensor *numbers(PyObject *o, int64_t n) const {
+    const at::Tensor *t = plain(o);
+    if (!t || (t->scalar_type() != at::kInt && t->scalar_type() != at::kLong) || t->dim() != 1 || t->size(0) != n || !t->is_contiguous())
+      return nullptr;
+    return t;
+  }
+};
+
+inline void *at_ptr(const at::Tensor *t) { return t ? t->data_ptr() : nullptr; }
+inline int is_i64(const at::Tensor *t) { return t && t->scalar_type() == at::kLong; }
+inline void written(const at::Tensor *t) {
+  if (!t->is_inference()) t->unsafeGetTensorImpl()->bump_version();
+}
+inline at::Tensor scratch(int64_t bytes, const at::Tensor *like) {
+  return at::empty({bytes}, like->options().dtype(at::kByte));
+}
+
+// attention_pass(query, key, value, k_cache, v_cache, page_table, cache_position, fill_page_table, batch_idx, chunk_start,
+//                sinks, output, users, heads, kv_heads, head_size, scale, window)
+// -> status of the last entry point called, or None: not an ordinary pass, nothing was issued.
+PyObject *attention_pass(PyObject *, PyObject *const *v, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 18) {
+    PyErr_SetString(PyExc_TypeError, "attention_pass takes 18 arguments");
+    return nullptr;
+  }
+  if (c10::impl::TorchDispatchModeTLS::any_modes_set()) Py_RETURN_NONE;
+  if (!THPVariable_CheckExact(v[0]) || !THPVariable_Unpack(v[0]).is_cuda()) Py_RETURN_NONE;  // (ahead of any question to the device)
+  for (int i = 12; i < 18; ++i)
+    if (i == 16 ? !PyFloat_Check(v[i]) : !PyLong_Check(v[i])) Py_RETURN_NONE;
+  const int64_t users = PyLong_AsLongLong(v[12]), hq = PyLong_AsLongLong(v[13]), hkv = PyLong_AsLongLong(v[14]);
+  const int64_t d = PyLong_AsLongLong(v[15]), window = PyLong_AsLongLong(v[17]);
+  const float scale = (float)PyFloat_AsDouble(v[16]);
+  if (users <= 0 || hq <= 0 || hkv <= 0 || d <= 0 || d % 8 || hq % hkv || window < 0) Py_RETURN_NONE;
+
+  const Pass p{(int)c10::hip::current_device(), at::GradMode::is_enabled()};
+  const at::Tensor *q = p.rows(v[0], hq * d), *k = p.rows(v[1], hkv * d), *val = p.rows(v[2], hkv * d);
+  if (!q || !k || !val) Py_RETURN_NONE;
+  const int64_t tokens = q->size(0);
+  if (tokens == 0 || tokens % users || k->size(0) != tokens || val->size(0) != tokens || k->stride(0) != val->stride(0)) Py_RETURN_NONE;
+  const int64_t s = tokens / users;
+  const at::Tensor *out = p.plain(v[11]);
+  if (!out || out->scalar_type() != at::kBFloat16 || !out->is_contiguous() || out->numel() != tokens * hq * d ||
+      reinterpret_cast<uintptr_t>(out->data_ptr()) % 16)
+    Py_RETURN_NONE;
+
+  const at::Tensor *kc = p.plain(v[3]), *vc = p.plain(v[4]);
+  if (!kc || !vc || kc->dim() != 4 || kc->sizes() != vc->sizes() || kc->scalar_type() != vc->scalar_type() || !kc->is_contiguous() ||
+      !vc->is_contiguous() || kc->size(0) == 0 || kc->size(1) != hkv || kc->size(3) != d)
+    Py_RETURN_NONE;
+  const bool bfp8 = kc->scalar_type() == at::kByte;
+  if (!bfp8 && kc->scalar_type() != at::kBFloat16) Py_RETURN_NONE;
+  const int64_t nb = kc->size(0);
+  int64_t bs = kc->size(2);
+  if (bfp8) {
+    if (bs % 17) Py_RETURN_NONE;
+    bs = bs / 17 * 16;
+  }
+  const int fmt = bfp8 ? TTPA_KV_BFP8 : TTPA_KV_BF16;
+  void *stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)p.device).stream();
+
+  if (s == 1) {  // decode step: cache update and attention
+    const at::Tensor *pt = p.table(v[5]), *pos = p.numbers(v[6], users), *sinks = nullptr;
+    if (!pt || pt->size(0) != users || !pos) Py_RETURN_NONE;
+    if (v[10] != Py_None) {
+      sinks = p.plain(v[10]);
+      if (!sinks || sinks->scalar_type() != at::kFloat || sinks->numel() != hq || !sinks->is_contiguous()) Py_RETURN_NONE;
+    }
+    const size_t bytes = ttpa_paged_decode_workspace_bytes((int32_t)users, (int32_t)hq, (int32_t)hkv, (int32_t)d);
+    if (bytes == 0) Py_RETURN_NONE;
+    const at::Tensor ws = scratch((int64_t)bytes, out);
+    written(kc), written(vc), written(out);
+    const int rc = ttpa_paged_update_decode(
+        out->data_ptr(), hq * d, d, q->data_ptr(), q->stride(0), d, kc->data_ptr(), vc->data_ptr(), k->data_ptr(), val->data_ptr(),
+        k->stride(0), d, static_cast<const int32_t *>(pt->data_ptr()), pt->stride(0), pos->data_ptr(), is_i64(pos), (int32_t)users,
+        (int32_t)hq, (int32_t)hkv, (int32_t)d, (int32_t)bs, (int32_t)pt->size(1), (int32_t)nb, scale, fmt, (int32_t)window,
+        static_cast<const float *>(at_ptr(sinks)), ws.data_ptr(), bytes, stream);
+    return PyLong_FromLong(rc);
+  }
+
+  // prefill: fill through the fill table, attention on the fresh K / V or on the cache
+  if (v[10] != Py_None || !(scale > 0.f)) Py_RETURN_NONE;
+  const at::Tensor *fill = p.table(v[7]), *bidx = p.numbers(v[8], users);
+  if (!fill || !bidx || fill->size(0) == 0 || s > fill->size(1) * bs) Py_RETURN_NONE;
+  const int32_t *fill_pt = static_cast<const int32_t *>(fill->data_ptr());
+  if (v[9] == Py_None) {
+    if (bfp8 || s % 32) Py_RETURN_NONE;
+    written(kc), written(vc), written(out);
+    const int rc = ttpa_sdpa_prefill_fill(
+        out->data_ptr(), s * hq * d, d, hq * d, q->data_ptr(), s * q->stride(0), d, q->stride(0), k->data_ptr(), val->data_ptr(),
+        s * k->stride(0), d, k->stride(0), (int32_t)users, (int32_t)hq, (int32_t)hkv, (int32_t)s, (int32_t)s, (int32_t)d, 1, scale,
+        (int32_t)window, kc->data_ptr(), vc->data_ptr(), fill_pt, fill->stride(0), bidx->data_ptr(), is_i64(bidx),
+        (int32_t)fill->size(0), (int32_t)bs, (int32_t)fill->size(1), (int32_t)nb, stream);
+    return PyLong_FromLong(rc);
+  }
+  const at::Tensor *pt = p.table(v[5]), *start = p.numbers(v[9], 1);
+  if (!pt || pt->size(0) != users || !start || is_i64(start)) Py_RETURN_NONE;
+  int64_t bytes = 0;
+  if (d == 128 && bs % 32 == 0) {
+    bytes = ttpa_sdpa_prefill_scratch_bytes((int32_t)users, (int32_t)hq, (int32_t)hkv, (int32_t)s, (int32_t)d, (int32_t)bs,
+                                            (int32_t)pt->size(1), fmt);
+    if (bytes < 0 || bytes > kScratchLimit) bytes = 0;
+  }
+  at::Tensor ws;
+  if (bytes) ws = scratch(bytes, out);
+  written(kc), written(vc), written(out);
+  int rc = ttpa_paged_fill_cache_kv(kc->data_ptr(), vc->data_ptr(), k->data_ptr(), val->data_ptr(), s * k->stride(0), d, k->stride(0),
+                                    fill_pt, fill->stride(0), bidx->data_ptr(), is_i64(bidx), (int32_t)users, (int32_t)fill->size(0),
+                                    (int32_t)hkv, (int32_t)s, (int32_t)bs, (int32_t)d, (int32_t)fill->size(1), (int32_t)nb, fmt, stream);
+  if (rc == TTPA_OK)
+    rc = ttpa_sdpa_prefill_expanded(
+        out->data_ptr(), s * hq * d, d, hq * d, q->data_ptr(), s * q->stride(0), d, q->stride(0), kc->data_ptr(), vc->data_ptr(), 0, 0,
+        0, static_cast<const int32_t *>(pt->data_ptr()), pt->stride(0), static_cast<const int32_t *>(start->data_ptr()), nullptr, 0, 0,
+        (int32_t)users, (int32_t)hq, (int32_t)hkv, (int32_t)s, (int32_t)(pt->size(1) * bs), (int32_t)d, (int32_t)bs,
+        (int32_t)pt->size(1), (int32_t)nb, 1, scale, 0, fmt, bytes ? ws.data_ptr() : nullptr, bytes, stream);
+  return PyLong_FromLong(rc);
+  END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef methods[] = {
+    {"attention_pass", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(attention_pass)), METH_FASTCALL,
+     "One pass of an attention layer from its tensors; None if it is not an ordinary one."},
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "ttpa_host", "Eager host path of the attention backend.", -1, methods};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit_ttpa_host() { return PyModule_Create(&module); }

@@ -3,11 +3,13 @@
 from __future__ import annotations
 
 import ctypes as C
+import importlib.util
 import os
 from typing import Optional
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libttpa.so")
+HOST_PATH = os.path.join(_HERE, "lib", "ttpa_host.so")
 CSRC_DIR = os.path.normpath(os.path.join(_HERE, "..", "csrc"))
 
 OK = 0
@@ -164,6 +166,29 @@ def lib() -> C.CDLL:
             raise RuntimeError("libttpa.so ABI version mismatch; rebuild it")
         _lib = handle
     return _lib
+
+
+_host = None
+
+
+def host():
+    """The eager host path (csrc/host_path.cpp), loaded once.  Raises if it has not been built."""
+    global _host
+    if _host is None:
+        lib()  # the module is linked against the library at this path
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError(f"{HOST_PATH} is missing; build it with `make -C {CSRC_DIR}`")
+        spec = importlib.util.spec_from_file_location("ttpa_host", HOST_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _host = module
+    return _host
+
+
+def check(name: str, rc: int) -> None:
+    """Raises TtpaError for a negative status."""
+    if rc != OK:
+        raise TtpaError(name, rc, lib().ttpa_last_error().decode("utf-8", "replace"))
 
 
 def call(name: str, *args) -> None:
