@@ -96,6 +96,10 @@ def test_other_passes_are_left_to_the_operators():
     refused(kv=[kv[0], kv[1][1:]])
     refused(kv=[torch.tensor([]), torch.tensor([])])
     refused(kv=[kv[0].transpose(1, 2), kv[1].transpose(1, 2)])
+    refused(q=torch._neg_view(q))
+    with torch.autograd.forward_ad.dual_level():
+        refused(q=torch.autograd.forward_ad.make_dual(q, torch.ones_like(q)))
+    torch.vmap(lambda x: (refused(q=x), x)[1])(torch.stack([q, q]))
     md.num_users = None
     refused()
     md.num_users = 3

@@ -11,6 +11,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/ATen.h>
+#include <ATen/TracerMode.h>
 #include <ATen/core/grad_mode.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
@@ -23,16 +24,24 @@ namespace {
 // Largest scratch a pass may ask for (the operators' limit).
 constexpr int64_t kScratchLimit = int64_t(8) << 30;
 
+constexpr c10::DispatchKeySet kWrapped({c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                        c10::DispatchKey::Functionalize, c10::DispatchKey::Python, c10::DispatchKey::ZeroTensor,
+                                        c10::DispatchKey::Negative, c10::DispatchKey::Conjugate});
+
 struct Pass {
   int device;
   bool grad;
 
-  // A plain tensor on the current device that autograd does not watch; null otherwise.
+  // A plain tensor on the current device that autograd does not watch; null otherwise.  (A tensor inside vmap or
+  // a functional transform, one to be functionalized and one with a lazy sign are plain Python tensors whose memory is not theirs to read;
+  // one with a forward-mode tangent would lose it.)
   const at::Tensor *plain(PyObject *o) const {
     if (!THPVariable_CheckExact(o)) return nullptr;
     const at::Tensor &t = THPVariable_Unpack(o);
     if (!t.defined() || !t.is_cuda() || t.get_device() != device || t.layout() != at::kStrided) return nullptr;
+    if (t.unsafeGetTensorImpl()->key_set().has_any(kWrapped) || !t.has_storage()) return nullptr;
     if (grad && t.requires_grad()) return nullptr;
+    if (t.unsafeGetTensorImpl()->autograd_meta() && t._fw_grad(0).defined()) return nullptr;
     return &t;
   }
   // [rows, cols] bfloat16 with contiguous, 16-byte aligned rows.
@@ -74,7 +83,7 @@ PyObject *attention_pass(PyObject *, PyObject *const *v, Py_ssize_t n) {
     PyErr_SetString(PyExc_TypeError, "attention_pass takes 18 arguments");
     return nullptr;
   }
-  if (c10::impl::TorchDispatchModeTLS::any_modes_set()) Py_RETURN_NONE;
+  if (c10::impl::TorchDispatchModeTLS::any_modes_set() || at::tracer::impl::is_dispatch_enabled()) Py_RETURN_NONE;
   if (!THPVariable_CheckExact(v[0]) || !THPVariable_Unpack(v[0]).is_cuda()) Py_RETURN_NONE;  // (ahead of any question to the device)
   for (int i = 12; i < 18; ++i)
     if (i == 16 ? !PyFloat_Check(v[i]) : !PyLong_Check(v[i])) Py_RETURN_NONE;

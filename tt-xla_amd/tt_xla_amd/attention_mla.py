@@ -207,7 +207,9 @@ class TTMLAAttentionBackendImpl(_ImplBase):
         return torch.einsum(pattern, out_lat, layer.W_UV.to(device=out_lat.device))
 
     def _bf16_on_gpu(self, *tensors) -> bool:
-        return all(t.device.type == "cuda" and t.dtype == torch.bfloat16 for t in tensors)
+        """bfloat16 on one GPU.  (The weights are plain attributes and may sit elsewhere: such a pass moves them.)"""
+        device = tensors[0].device
+        return device.type == "cuda" and all(t.device == device and t.dtype == torch.bfloat16 for t in tensors)
 
     def _steps_at_once(self, q_nope, q_pe, kv_c_normed, k_pe, kv_cache, attn_metadata, layer, output) -> bool:
         """Whether a decode pass is one ``tt::latent_decode_step_``: the head shape it is built for, causal, with a
