@@ -3,8 +3,8 @@
 // to half precision) or a bfloat16 cache.
 //
 // Work decomposition, partial slots and merge kernel are those of decode.hip, with tiles of
-// 16 KiB of 16-bit elements (128, 64 or 32 tokens at head size 64, 128, 256; 8 KiB = 32 tokens
-// for a bfloat16 cache with head size 128, see tile_bytes).  Inside a wavefront a tile of K,
+// 16 KiB of 16-bit elements (128, 64 or 32 tokens at head size 64, 128, 256; 8 KiB = 64 / 32 tokens
+// for a bfloat16 cache with head size 64 / 128, see tile_bytes).  Inside a wavefront a tile of K,
 // then of V, goes global -> registers -> a wave-private LDS buffer of that size that both
 // tensors use in turn:
 //   stage K(t) | prefetch K(t+1) | S^T = K Q^T | softmax | stage V(t) | prefetch V(t+1) | O^T += V^T P^T
@@ -41,9 +41,9 @@
 // banks and the keys are taken from row / 2: (row / 2) & 7 and y = (row / 2) & 3.
 //
 // Where a tile's rows sit in the cache (RUNS): one run of consecutive rows when a block holds
-// whole tiles; two runs of half a tile when block_size is a multiple of half a tile (block size
-// 32 with head size 128, the serving default; 64 with 64; 16 with 256); four runs of a quarter
-// tile when it is a multiple of a quarter tile (16 with 128; 32 with 64; 8 with 256); otherwise
+// whole tiles; two runs of half a tile when block_size is a multiple of half a tile (the serving
+// default of 32 with head size 64, or with 128 and block-float-8; 16 with 256); four runs of a quarter
+// tile when it is a multiple of a quarter tile (16 with 64; 8 with 128 and 256); otherwise
 // one run per load instruction.  A run costs a block-table lookup and a 64-bit base, which are
 // scalar registers, the resource this kernel is short of.
 //
@@ -64,16 +64,20 @@ typedef short shortx4 __attribute__((ext_vector_type(4)));
 
 constexpr int kMaxUsers16 = kMaxUsers;  // the library-wide limit: 16 KiB of prefix tables
 // Bytes of a tile's K (or V) rows as 16-bit elements, i.e. of a wavefront's LDS buffer: 16 KiB
-// (128 / 64 / 32 tokens at head size 64 / 128 / 256), except 8 KiB (32 tokens) for a bfloat16
-// cache with head size 128.  A wavefront has one tile of K and one of V in flight; the kernel
+// (128 / 64 / 32 tokens at head size 64 / 128 / 256), except 8 KiB (64 / 32 tokens) for a bfloat16
+// cache with head size 64 or 128.  A wavefront has one tile of K and one of V in flight; the kernel
 // ends when the slowest wavefront has drained its last tile, and wavefronts of one launch finish
 // several microseconds apart (the XCDs do not get equal shares of the HBM bandwidth), so a
 // shorter tile shortens that tail: config 2's step 58.7 -> 57.8 us, config 4's 549 -> 543 us.
-// The block-float-8 cache moves half the bytes per token and loses with the shorter tile
-// (44.1 -> 46.2 us on config 5).
+// At head size 64 (64 / 8 heads, us per layer of a replayed step): a window of 1024 over 37 users 25.2 ->
+// 23.1 (its two ends waste less, too), 32 users with 512 ... 4096 tokens 27.7 -> 26.5, 8 users with
+// 128 ... 1024 15.0 -> 11.6, 128 users with 256 ... 32768 274 -> 272; 4 KiB: 23.6, 26.9, 10.8.
+// The block-float-8 cache moves half the bytes per token and loses with the shorter tile where there is
+// much to read (head size 128, 64 users with 1024 ... 16384 tokens: 138 -> 150 us; head size 64, 100 users
+// with 1024 ... 8192: 78 -> 84), and how much there is only the device knows.
 template <int D, bool BFP8>
 constexpr int tile_bytes() {
-  return (D == 128 && !BFP8) ? 8192 : 16384;
+  return (D <= 128 && !BFP8) ? 8192 : 16384;
 }
 
 template <bool F16>
