@@ -554,7 +554,7 @@ static int decode_impl(void *out, int64_t out_user_stride, int64_t out_head_stri
   if (ev1) (void)hipEventRecord(ev1, st);
   if (use_mfma16) take_profile_events(ev0, ev1);  // still armed only if the launch did not happen
   if (rc) return rc;
-  decode_combine_kernel<<<dim3(users * kv_heads, combine_pieces(g, head_size)), dim3(256), 0, st>>>(a, g, head_size);
+  launch_combine(a, users * kv_heads, g, head_size, st);
   return check_launch("paged_sdpa_decode");
 }
 

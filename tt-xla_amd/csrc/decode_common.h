@@ -417,13 +417,35 @@ __device__ inline void write_negative_position(const DecodeArgs &a, int seg, int
 // decode shape, whose step is 0.7 us shorter than with one piece of 512; a latent segment of
 // 16 heads x 512 values is 32 pieces, and as one workgroup per segment its merge took as long as
 // the attention itself).
-constexpr int kCombinePiece = 256;
-inline int combine_pieces(int g, int d) { return (g * d + kCombinePiece - 1) / kCombinePiece; }
+// SLICES > 1: the workgroup's threads are kCombinePiece / SLICES elements times SLICES; a slice takes every
+// SLICES-th batch of the partials and the slices meet in LDS.  One long segment cut into a hundred ranges
+// is otherwise a chain of a dozen round trips on a nearly empty chip, as long as the attention.  Four layers of a
+// replayed step: one user of 16/8 heads over 9148 tokens (96 ranges a segment) 83.1 -> 57.9 us, of 32/8 heads over
+// 16384 block-float-8 tokens 116 -> 80.2, three users of 40/8 heads 73.2 -> 56.3; a latent step of one user over
+// 32768 tokens 91.3 -> 42.0.
+constexpr int kCombinePiece = 256, kCombineSlices = 8;
+inline int combine_pieces(int n, int slices) {
+  const int piece = kCombinePiece / slices;
+  return (n + piece - 1) / piece;
+}
+// A segment has at most as many partials as there are ranges, and on average n_waves / segments where
+// contexts are long: from two batches on, the slices save a round trip.  At the line both forms are level (6 users
+// of 8 KV heads with 4096 tokens 100.8 -> 99.6 us, with 512 ... 4096 tokens 69.7 -> 63.2; latent, 40 users 59.5 -> 59.1);
+// one user with 512 tokens, whose partials are one batch, 45.2 -> 44.1.
+inline bool combine_sliced(const DecodeArgs &a, int segments) { return a.n_waves >= 16 * segments; }
 
-__global__ inline __launch_bounds__(256) void decode_combine_kernel(DecodeArgs a, int G, int D) {
+// What the weights of the partials seen so far are relative to.  With an explicit mask they may all be fully
+// masked (maximum -inf) where their segment is not: their weights are zeros, not exp2(-inf + inf).
+__device__ __forceinline__ float merge_reference(float m) { return m == -INFINITY ? 0.f : m; }
+
+template <int SLICES>
+__global__ __launch_bounds__(256) void decode_combine_kernel(DecodeArgs a, int G, int D) {
+  constexpr int kElems = kCombinePiece / SLICES;
   const int seg = blockIdx.x;
-  const int i_begin = blockIdx.y * kCombinePiece + threadIdx.x;
-  const int i_end = min(G * D, (int)(blockIdx.y + 1) * kCombinePiece);
+  const int slice = SLICES == 1 ? 0 : (int)threadIdx.x / kElems;
+  const int i_own = blockIdx.y * kElems + ((int)threadIdx.x - slice * kElems);
+  const int i = min(i_own, G * D - 1);
+  const bool stores = slice == 0 && i_own < G * D;
   const int u = seg / a.hkv, h = seg % a.hkv;
   const bool pow2 = (D & (D - 1)) == 0;
   const int dshift = __builtin_ctz(D);
@@ -432,48 +454,76 @@ __global__ inline __launch_bounds__(256) void decode_combine_kernel(DecodeArgs a
   const int first = a.ws_seg[2 * seg], nw = a.ws_seg[2 * seg + 1];
   uint16_t *out = a.out + u * a.out_us;
   if (nw == 0) {  // padded row: no attended position -> NaN like softmax over nothing
-    for (int i = i_begin; i < i_end; i += 256)
-      out[(int64_t)(h * G + head_of(i)) * a.out_hs + elem_of(i)] = 0x7fc0;
+    if (stores) out[(int64_t)(h * G + head_of(i)) * a.out_hs + elem_of(i)] = 0x7fc0;
     if (a.k_new != nullptr && blockIdx.y == 0) write_negative_position(a, seg, D);
     return;
   }
   constexpr int kBatch = 8;
   const float *base = a.ws_slots + (int64_t)first * a.slot_floats;
-  for (int i = i_begin; i < i_end; i += 256) {
-    const int g = head_of(i);
-    float mall = -INFINITY, num = 0.f, den = 0.f;
-    for (int w = 0; w < nw; w += kBatch) {
-      float mv[kBatch], lv[kBatch], av[kBatch];
+  const int g = head_of(i);
+  float mall = -INFINITY, num = 0.f, den = 0.f;
+  for (int w = slice * kBatch; w < nw; w += SLICES * kBatch) {
+    float mv[kBatch], lv[kBatch], av[kBatch];
 #pragma unroll
-      for (int j = 0; j < kBatch; ++j) {
-        const float *sl = base + (int64_t)min(w + j, nw - 1) * a.slot_floats;
-        mv[j] = (w + j < nw) ? sl[G * D + g] : -INFINITY;
-        lv[j] = sl[G * D + G + g];
-        av[j] = sl[i];
-      }
-      float mnew = mall;
-#pragma unroll
-      for (int j = 0; j < kBatch; ++j) mnew = fmaxf(mnew, mv[j]);
-      float resc = __builtin_amdgcn_exp2f(mall - mnew);
-      num *= resc;
-      den *= resc;
-#pragma unroll
-      for (int j = 0; j < kBatch; ++j) {
-        float wgt = __builtin_amdgcn_exp2f(mv[j] - mnew);  // 0 for the padding entries
-        num = fmaf(wgt, av[j], num);
-        den = fmaf(wgt, lv[j], den);
-      }
-      mall = mnew;
+    for (int j = 0; j < kBatch; ++j) {
+      const float *sl = base + (int64_t)min(w + j, nw - 1) * a.slot_floats;
+      mv[j] = (w + j < nw) ? sl[G * D + g] : -INFINITY;
+      lv[j] = sl[G * D + G + g];
+      av[j] = sl[i];
     }
-    if (a.sink) {  // the sink logit (natural-log units, not scaled) only enlarges the normaliser
-      const float sk = a.sink[h * G + g] * 1.4426950408889634f;
-      const float mnew = fmaxf(mall, sk);
-      const float resc = __builtin_amdgcn_exp2f(mall - mnew);
-      num *= resc;
-      den = den * resc + __builtin_amdgcn_exp2f(sk - mnew);
+    float mnew = mall;
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) mnew = fmaxf(mnew, mv[j]);
+    const float ref = merge_reference(mnew);
+    const float resc = __builtin_amdgcn_exp2f(mall - ref);
+    num *= resc;
+    den *= resc;
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      const float wgt = __builtin_amdgcn_exp2f(mv[j] - ref);  // 0 for the padding entries
+      num = fmaf(wgt, av[j], num);
+      den = fmaf(wgt, lv[j], den);
     }
-    out[(int64_t)(h * G + g) * a.out_hs + elem_of(i)] = (uint16_t)f32_to_bf16_bits(num / den);
+    mall = mnew;
   }
+  if constexpr (SLICES > 1) {
+    if (nw > kBatch) {  // (the same for the whole workgroup; the first slice has it all otherwise)
+      __shared__ float s_part[3][kCombinePiece];
+      s_part[0][threadIdx.x] = mall, s_part[1][threadIdx.x] = num, s_part[2][threadIdx.x] = den;
+      __syncthreads();
+      if (slice == 0) {
+        float mnew = mall;
+#pragma unroll
+        for (int j = 1; j < SLICES; ++j) mnew = fmaxf(mnew, s_part[0][threadIdx.x + j * kElems]);
+        const float ref = merge_reference(mnew);
+        const float resc = __builtin_amdgcn_exp2f(mall - ref);
+        num *= resc, den *= resc, mall = mnew;
+#pragma unroll
+        for (int j = 1; j < SLICES; ++j) {
+          const int at = threadIdx.x + j * kElems;
+          const float wgt = __builtin_amdgcn_exp2f(s_part[0][at] - ref);  // 0 for a slice without a partial
+          num = fmaf(wgt, s_part[1][at], num);
+          den = fmaf(wgt, s_part[2][at], den);
+        }
+      }
+    }
+  }
+  if (!stores) return;
+  if (a.sink) {  // the sink logit (natural-log units, not scaled) only enlarges the normaliser
+    const float sk = a.sink[h * G + g] * 1.4426950408889634f;
+    const float mnew = fmaxf(mall, sk);
+    const float resc = __builtin_amdgcn_exp2f(mall - mnew);
+    num *= resc;
+    den = den * resc + __builtin_amdgcn_exp2f(sk - mnew);
+  }
+  out[(int64_t)(h * G + g) * a.out_hs + elem_of(i)] = (uint16_t)f32_to_bf16_bits(num / den);
+}
+
+inline void launch_combine(const DecodeArgs &a, int segments, int g, int d, hipStream_t st) {
+  if (combine_sliced(a, segments))
+    decode_combine_kernel<kCombineSlices><<<dim3(segments, combine_pieces(g * d, kCombineSlices)), dim3(256), 0, st>>>(a, g, d);
+  else
+    decode_combine_kernel<1><<<dim3(segments, combine_pieces(g * d, 1)), dim3(256), 0, st>>>(a, g, d);
 }
 
 // The same merge over partials whose values are bfloat16 (DecodeArgs::partial_bf16).  They lie in
@@ -483,26 +533,29 @@ __global__ inline __launch_bounds__(256) void decode_combine_kernel(DecodeArgs a
 // thread owns W consecutive 32-bit words of every partial, in that order, and stores its 2 W
 // neighbouring output elements at once: W = 4 (16 bytes per load and store) where output rows start
 // on 16-byte boundaries, W = 1 where only on 4-byte ones (the caller checks).
-// Grid: x = segment, y = piece of kCombinePiece threads.
-template <int W>
-__global__ inline __launch_bounds__(256) void decode_combine_bf16_kernel(DecodeArgs a, int G, int D) {
+// Grid: x = segment, y = piece of kCombinePiece / SLICES threads, times SLICES as above.
+template <int W, int SLICES>
+__global__ __launch_bounds__(256) void decode_combine_bf16_kernel(DecodeArgs a, int G, int D) {
   static_assert(W == 1 || W == 4, "a thread's words stay inside one head's eight");
   typedef uint32_t words_t __attribute__((ext_vector_type(W)));
   const int seg = blockIdx.x;
   const int pairs = (G + 15) / 16 * 16 * D / 2;  // words of values in a partial
-  const int p = W * (blockIdx.y * kCombinePiece + threadIdx.x);
-  if (p >= pairs) return;
+  constexpr int kElems = kCombinePiece / SLICES;
+  const int slice = SLICES == 1 ? 0 : (int)threadIdx.x / kElems;
+  const int p_own = W * (blockIdx.y * kElems + ((int)threadIdx.x - slice * kElems));
+  const int p = min(p_own, pairs - W);
   const int u = seg / a.hkv, h = seg % a.hkv;
   const int blk = p >> 7, in_blk = p & 127;  // a block: 16 heads x 8 words
   const int g = 16 * (blk / (D / 16)) + (in_blk >> 3), e = 16 * (blk % (D / 16)) + 2 * (in_blk & 7);
-  if (g >= G) return;
+  const bool live = p_own < pairs && g < G;  // (the slices of an element meet at a barrier: nobody leaves before it)
+  if (SLICES == 1 && !live) return;
   const int first = a.ws_seg[2 * seg], nw = a.ws_seg[2 * seg + 1];
   words_t *out = reinterpret_cast<words_t *>(a.out + u * a.out_us + (int64_t)(h * G + g) * a.out_hs + e);
   if (nw == 0) {  // padded row: no attended position -> NaN like softmax over nothing
     words_t nan;
 #pragma unroll
     for (int k = 0; k < W; ++k) nan[k] = 0x7fc07fc0u;
-    *out = nan;
+    if (live && slice == 0) *out = nan;
     return;
   }
   const float *base = a.ws_slots + (int64_t)first * a.slot_floats;
@@ -513,7 +566,7 @@ __global__ inline __launch_bounds__(256) void decode_combine_bf16_kernel(DecodeA
   // 128-head latent form: two or three) takes batches of its size instead of eight mostly repeated loads
   auto merge = [&](auto batch_tag) {
     constexpr int kBatch = decltype(batch_tag)::value;
-    for (int w = 0; w < nw; w += kBatch) {
+    for (int w = live ? slice * kBatch : nw; w < nw; w += SLICES * kBatch) {
       float mv[kBatch], lv[kBatch];
       words_t av[kBatch];
 #pragma unroll
@@ -526,13 +579,14 @@ __global__ inline __launch_bounds__(256) void decode_combine_bf16_kernel(DecodeA
       float mnew = mall;
 #pragma unroll
       for (int j = 0; j < kBatch; ++j) mnew = fmaxf(mnew, mv[j]);
-      const float resc = __builtin_amdgcn_exp2f(mall - mnew);
+      const float ref = merge_reference(mnew);
+      const float resc = __builtin_amdgcn_exp2f(mall - ref);
       den *= resc;
 #pragma unroll
       for (int k = 0; k < 2 * W; ++k) num[k] *= resc;
 #pragma unroll
       for (int j = 0; j < kBatch; ++j) {
-        const float wgt = __builtin_amdgcn_exp2f(mv[j] - mnew);  // 0 for the padding entries
+        const float wgt = __builtin_amdgcn_exp2f(mv[j] - ref);  // 0 for the padding entries
 #pragma unroll
         for (int k = 0; k < W; ++k) {
           num[2 * k] = fmaf(wgt, bf16_lo(av[j][k]), num[2 * k]);
@@ -546,6 +600,34 @@ __global__ inline __launch_bounds__(256) void decode_combine_bf16_kernel(DecodeA
   if (nw <= 2) merge(std::integral_constant<int, 2>{});
   else if (nw <= 4) merge(std::integral_constant<int, 4>{});
   else merge(std::integral_constant<int, 8>{});
+  if constexpr (SLICES > 1) {
+    if (nw > 8) {  // (the same for the whole workgroup; the first slice has it all otherwise)
+      __shared__ float s_part[2 + 2 * W][kCombinePiece];
+      s_part[0][threadIdx.x] = mall, s_part[1][threadIdx.x] = den;
+#pragma unroll
+      for (int k = 0; k < 2 * W; ++k) s_part[2 + k][threadIdx.x] = num[k];
+      __syncthreads();
+      if (slice == 0) {
+        float mnew = mall;
+#pragma unroll
+        for (int j = 1; j < SLICES; ++j) mnew = fmaxf(mnew, s_part[0][threadIdx.x + j * kElems]);
+        const float ref = merge_reference(mnew);
+        const float resc = __builtin_amdgcn_exp2f(mall - ref);
+        den *= resc, mall = mnew;
+#pragma unroll
+        for (int k = 0; k < 2 * W; ++k) num[k] *= resc;
+#pragma unroll
+        for (int j = 1; j < SLICES; ++j) {
+          const int at = threadIdx.x + j * kElems;
+          const float wgt = __builtin_amdgcn_exp2f(s_part[0][at] - ref);  // 0 for a slice without a partial
+          den = fmaf(wgt, s_part[1][at], den);
+#pragma unroll
+          for (int k = 0; k < 2 * W; ++k) num[k] = fmaf(wgt, s_part[2 + k][at], num[k]);
+        }
+      }
+    }
+    if (!live || slice != 0) return;
+  }
   if (a.sink) {
     const float sk = a.sink[h * G + g] * 1.4426950408889634f;
     const float mnew = fmaxf(mall, sk);

@@ -1317,10 +1317,13 @@ using namespace ttpa::decode;
 static void launch_combine_bf16(const DecodeArgs &a, int segments, int gseg, int head_dim_v, const void *out, int64_t out_user_stride,
                                 int64_t out_head_stride, hipStream_t st) {
   const int words = (gseg + 15) / 16 * 16 * head_dim_v / 2;
-  if (out_user_stride % 8 == 0 && out_head_stride % 8 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0)
-    decode_combine_bf16_kernel<4><<<dim3(segments, combine_pieces(words / 4, 1)), dim3(256), 0, st>>>(a, gseg, head_dim_v);
-  else
-    decode_combine_bf16_kernel<1><<<dim3(segments, combine_pieces(words, 1)), dim3(256), 0, st>>>(a, gseg, head_dim_v);
+  const bool wide = out_user_stride % 8 == 0 && out_head_stride % 8 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
+  const int slices = combine_sliced(a, segments) ? kCombineSlices : 1;
+  const dim3 grid(segments, combine_pieces(wide ? words / 4 : words, slices));
+  if (slices > 1 && wide) decode_combine_bf16_kernel<4, kCombineSlices><<<grid, dim3(256), 0, st>>>(a, gseg, head_dim_v);
+  else if (slices > 1) decode_combine_bf16_kernel<1, kCombineSlices><<<grid, dim3(256), 0, st>>>(a, gseg, head_dim_v);
+  else if (wide) decode_combine_bf16_kernel<4, 1><<<grid, dim3(256), 0, st>>>(a, gseg, head_dim_v);
+  else decode_combine_bf16_kernel<1, 1><<<grid, dim3(256), 0, st>>>(a, gseg, head_dim_v);
 }
 
 static int wide_geometry(int32_t q_heads, int32_t kv_heads, int32_t &nhb, int32_t &gseg) {
@@ -1472,7 +1475,7 @@ static int mla_decode_impl(void *out, int64_t out_user_stride, int64_t out_head_
     if (a.partial_bf16)
       launch_combine_bf16(a, users * kv_heads * nhb, gseg, head_dim_v, out, out_user_stride, out_head_stride, st);
     else
-      decode_combine_kernel<<<dim3(users * kv_heads * nhb, combine_pieces(gseg, head_dim_v)), dim3(256), 0, st>>>(a, gseg, head_dim_v);
+      launch_combine(a, users * kv_heads * nhb, gseg, head_dim_v, st);
     return check_launch("paged_mla_decode");
   }
   // The 16-head form: V taken from K, one head block of up to 16 heads, tiles inside one block.
@@ -1510,7 +1513,7 @@ static int mla_decode_impl(void *out, int64_t out_user_stride, int64_t out_head_
       if (a.partial_bf16)
         launch_combine_bf16(a, users * kv_heads, gseg, head_dim_v, out, out_user_stride, out_head_stride, st);
       else
-        decode_combine_kernel<<<dim3(users * kv_heads, combine_pieces(gseg, head_dim_v)), dim3(256), 0, st>>>(a, gseg, head_dim_v);
+        launch_combine(a, users * kv_heads, gseg, head_dim_v, st);
       return check_launch("paged_mla_decode");
     }
     a.n_waves = cus;
@@ -1538,7 +1541,7 @@ static int mla_decode_impl(void *out, int64_t out_user_stride, int64_t out_head_
   if (!ok) return fail(TTPA_ERR_LAUNCH, "latent decode: cannot configure the kernel");
   if (ev1) (void)hipEventRecord(ev1, st);
   if (int rc = check_launch("paged_mla_decode")) return rc;
-  decode_combine_kernel<<<dim3(users * kv_heads * nhb, combine_pieces(gseg, head_dim_v)), dim3(256), 0, st>>>(a, gseg, head_dim_v);
+  launch_combine(a, users * kv_heads * nhb, gseg, head_dim_v, st);
   return check_launch("paged_mla_decode");
 }
 
