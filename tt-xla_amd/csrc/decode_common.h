@@ -429,10 +429,12 @@ inline int combine_pieces(int n, int slices) {
   return (n + piece - 1) / piece;
 }
 // A segment has at most as many partials as there are ranges, and on average n_waves / segments where
-// contexts are long: from two batches on, the slices save a round trip.  At the line both forms are level (6 users
-// of 8 KV heads with 4096 tokens 100.8 -> 99.6 us, with 512 ... 4096 tokens 69.7 -> 63.2; latent, 40 users 59.5 -> 59.1);
-// one user with 512 tokens, whose partials are one batch, 45.2 -> 44.1.
-inline bool combine_sliced(const DecodeArgs &a, int segments) { return a.n_waves >= 16 * segments; }
+// contexts are long; ragged ones have several times that for the longest users, whom the merge waits for.  Lines at
+// 16 / 8 / 4 ranges per segment (four layers, us): 8 users of 8 KV heads with 256 ... 32768 tokens 173.4 / 162.6 / 162.9,
+// 32 users of 8/2 heads at head size 64 56.2 / 49.8 / 49.9, 16 users with 2048 tokens 117.5 / 117.1 / 119.9, 24 with
+// 1024 tokens 100.4 / 100.3 / 105.4: below eight the segments' workgroups fill the chip as they are, and cutting
+// them only makes more of them.  One user with 512 tokens, whose partials are one batch, 45.2 -> 44.1.
+inline bool combine_sliced(const DecodeArgs &a, int segments) { return a.n_waves >= 8 * segments; }
 
 // What the weights of the partials seen so far are relative to.  With an explicit mask they may all be fully
 // masked (maximum -inf) where their segment is not: their weights are zeros, not exp2(-inf + inf).
