@@ -89,3 +89,31 @@ def test_as_close_to_64_bits_as_the_plain_loop(hq, hkv, s, window, monkeypatch):
         err.append(((got[0].double() - want).norm() / want.norm()).item())
     print(f"h{hq}x{hkv} s{s} window{window}: plain {err[0]:.4e} stream {err[1]:.4e} ratio {err[1] / err[0]:.4f}", flush=True)
     assert err[1] < 1.002 * err[0]
+
+
+@pytest.mark.parametrize("hq,hkv,bs,bfp8", [(3, 3, 32, False), (4, 2, 64, False), (8, 2, 32, False), (8, 2, 64, False), (8, 2, 64, True)])
+@pytest.mark.parametrize("start,lc", [(-40, 96), (-1000, 96), (-32, 32), (-2000000000, 33), (2000000000, 33)])
+def test_chunk_that_starts_outside_the_sequence(hq, hkv, bs, bfp8, start, lc):
+    """Row i sees keys up to start + i: none is NaN (softmax over nothing), as in the plain loop.  The start is in
+    device memory, so no check of the host's sees it; a block count of
+    zero or less would never count down to zero."""
+    g = torch.Generator().manual_seed(hq + bs + lc)
+    users, nbpu = 2, 20
+    key, value, table = P._paged(g, users, nbpu, hkv, bs, 128, False)
+    q = P._bf(g, users, hq, lc, 128)
+    k, v = key.cuda(), value.cuda()
+    if bfp8:
+        from tt_xla_amd import custom_ops as ops
+        k, v = ops.bfp8_pack_cache(k), ops.bfp8_pack_cache(v)
+        key, value = ops.bfp8_unpack_cache(k).cpu(), ops.bfp8_unpack_cache(v).cpu()
+    got = torch.ops.tt.chunked_scaled_dot_product_attention(
+        q.cuda(), k, v, table.cuda(), torch.tensor([start], dtype=torch.int32).cuda(), 128**-0.5).cpu()
+    if start > 0:  # every row sees the whole table
+        want = O.chunked_sdpa(q, key, value, table, torch.tensor([nbpu * bs], dtype=torch.int32), 128**-0.5)
+        P._check(f"h{hq}x{hkv} bs{bs} start{start}", got, want)
+        return
+    blind = min(lc, -start)
+    assert got[:, :, :blind].isnan().all()
+    if blind < lc:  # the other rows are a chunk that starts at 0
+        want = O.chunked_sdpa(q[:, :, blind:].contiguous(), key, value, table, torch.tensor([0], dtype=torch.int32), 128**-0.5)
+        P._check(f"h{hq}x{hkv} bs{bs} start{start}", got[:, :, blind:].contiguous(), want)

@@ -63,7 +63,7 @@ __global__ __launch_bounds__(256) void bfp8_expand_kernel(ExpandArgs e) {
   const bool is_v = blockIdx.y & 1;
   if (blockIdx.y == 0 && threadIdx.x == 0) e.table[x] = x;
   const int skv = e.w * e.bs;
-  const int kv_end = e.causal ? min(skv, (e.chunk_start ? e.chunk_start[0] : 0) + e.sq) : skv;
+  const int kv_end = e.causal ? min(skv, chunk_offset(e.chunk_start, e.sq, skv) + e.sq) : skv;
   if (j * e.bs >= kv_end) return;
   int phys = e.pt[(int64_t)b * e.pt_rs + j];
   if ((unsigned)phys >= (unsigned)e.nb) phys = 0;  // (as the attention kernels treat a bad entry)

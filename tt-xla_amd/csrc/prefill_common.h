@@ -69,6 +69,13 @@ __device__ __forceinline__ int div_block(const PrefillArgs &a, int key) {
   return a.bs == 1 ? key : (int)__umulhi((uint32_t)key, a.bs_magic);
 }
 
+// Position of the first query row.  It is in device memory, where no check of the host's sees it: below -sq no row
+// sees a key and from skv on every row sees all of them, so the value is held between the two, and sums with
+// row numbers stay small.
+__device__ __forceinline__ int chunk_offset(const int32_t *chunk_start, int sq, int skv) {
+  return chunk_start ? min(max(chunk_start[0], -sq), skv) : 0;
+}
+
 // LDS geometry of one stage: the K tile (64 rows of D elements) followed by the V tile.
 // Chunk c (16 bytes) of row r is stored at chunk position c ^ swz(r).
 //   K fragments are read by 16 lanes of consecutive rows at one logical chunk: the 16

@@ -254,13 +254,15 @@ __global__ __launch_bounds__(256, 2) void prefill_stream_kernel(PrefillArgs a) {
   const int hk = hq0 / (a.hq / a.hkv);
   const int hq = hq0 + wave % HPW;
   const int row0 = (qt * RPW + wave / HPW) * kRowsPerWave;  // first query row of the wavefront
-  const int offset = a.causal ? (a.chunk_start ? a.chunk_start[0] : 0) : 0;
+  const int offset = a.causal ? chunk_offset(a.chunk_start, a.sq, a.skv) : 0;
 
   // keys the workgroup can see, in blocks of 32
   const int wg_last_row = min(a.sq, (qt + 1) * kRowsPerWave * RPW) - 1;
   const int kv_end = a.causal ? min(a.skv, offset + wg_last_row + 1) : a.skv;
   int first_block = FORM == kDenseWindow ? max(0, offset + qt * kRowsPerWave * RPW - a.window + 1) / kBlockKeys : 0;
-  int nblk = __builtin_amdgcn_readfirstlane((kv_end + kBlockKeys - 1) / kBlockKeys - first_block);
+  // (at least one: the loop counts blocks down to zero.  Where no row sees a key, a chunk that starts at a negative
+  // position, block 0 is read and masked, and the rows come out as NaN, softmax over nothing)
+  int nblk = __builtin_amdgcn_readfirstlane(max((kv_end + kBlockKeys - 1) / kBlockKeys - first_block, 1));
   bool whole = true;  // this workgroup sees all keys of its rows
   if constexpr (PAGED) {
     if (a.parts > 1) {
@@ -428,7 +430,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
   const int rb = blockIdx.x, hq = blockIdx.y, b = blockIdx.z;
   const int qt = rb / RPW;
   const int n = threadIdx.x & 31, g = threadIdx.x >> 5;
-  const int offset = a.causal ? (a.chunk_start ? a.chunk_start[0] : 0) : 0;
+  const int offset = a.causal ? chunk_offset(a.chunk_start, a.sq, a.skv) : 0;
   const int wg_last_row = min(a.sq, (qt + 1) * kRowsPerWave * RPW) - 1;
   const int kv_end = a.causal ? min(a.skv, offset + wg_last_row + 1) : a.skv;
   const int nblk = (kv_end + kBlockKeys - 1) / kBlockKeys;
