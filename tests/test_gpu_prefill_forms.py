@@ -117,3 +117,24 @@ def test_chunk_that_starts_outside_the_sequence(hq, hkv, bs, bfp8, start, lc):
     if blind < lc:  # the other rows are a chunk that starts at 0
         want = O.chunked_sdpa(q[:, :, blind:].contiguous(), key, value, table, torch.tensor([0], dtype=torch.int32), 128**-0.5)
         P._check(f"h{hq}x{hkv} bs{bs} start{start}", got[:, :, blind:].contiguous(), want)
+
+
+@pytest.mark.parametrize("users,hq,hkv,nbpu,start,lc", [(2, 32, 8, 8, 256, 256), (2, 64, 8, 6, 192, 192), (1, 16, 4, 9, 293, 200)])
+@pytest.mark.parametrize("slots", ["2", "3"])
+def test_several_row_blocks_per_workgroup_are_not_split(users, hq, hkv, nbpu, start, lc, slots, monkeypatch):
+    """TTPA_PREFILL_WGS_PER_GROUP has a workgroup walk its row blocks over all of their keys, also where the launch would
+    otherwise split the keys: every row comes out of the same operations as with a workgroup per row block and no
+    scratch to split with, bit for bit.  (Parts merged in float round differently.)"""
+    from tt_xla_amd import custom_ops as ops
+
+    g = torch.Generator().manual_seed(hq + start)
+    key, value, table = P._paged(g, users, nbpu, hkv, 64, 128, False)
+    args = [t.cuda() for t in (P._bf(g, users, hq, lc, 128), key, value, table, torch.tensor([start], dtype=torch.int32))]
+    split = torch.ops.tt.chunked_scaled_dot_product_attention(*args, 128**-0.5)
+    monkeypatch.setattr(ops, "_EXPANSION_LIMIT", 0)
+    whole = torch.ops.tt.chunked_scaled_dot_product_attention(*args, 128**-0.5)
+    monkeypatch.undo()
+    monkeypatch.setenv("TTPA_PREFILL_WGS_PER_GROUP", slots)
+    walked = torch.ops.tt.chunked_scaled_dot_product_attention(*args, 128**-0.5)
+    assert not torch.equal(split, whole)  # (what the next line would not tell from a split)
+    assert torch.equal(walked, whole)

@@ -1,9 +1,11 @@
-"""GPU parity for the two inner loops of the prefill kernel.  Shapes with head size 128 and a multiple
-of four query heads per KV head, causal or unmasked, dense or paged bfloat16, run the hand-scheduled
-loop (32-key blocks in LDS rings, written as one assembly block by csrc/gen_prefill_stream.py);
-TTPA_PREFILL_STREAM=0, read on every call, sends them through the compiler-scheduled loop that serves
-every other shape, and TTPA_PREFILL_WGS_PER_GROUP=n makes a workgroup of the hand-scheduled loop walk
-several blocks of query rows in turn instead of one.  Every case runs under each setting.  Same
+"""GPU parity for the two inner loops of the prefill kernel.  Shapes with head size 128
+run the hand-scheduled loop (32-key blocks in LDS rings, written as one assembly block by
+csrc/gen_prefill_stream.py): here those with a multiple of four query heads per KV head, the other
+forms in test_gpu_prefill_forms.py.  TTPA_PREFILL_STREAM=0, read on every call, sends them through the
+compiler-scheduled loop that serves every other shape, and TTPA_PREFILL_WGS_PER_GROUP=n makes a
+workgroup of the hand-scheduled loop walk several blocks of query rows in turn, each over all of its
+keys, instead of one (dense, and cache blocks of whole 64-key tiles).  Every case runs under each
+setting.  Same
 oracle, inputs and bar (atol = rtol = 2e-2) as tests/test_gpu_prefill.py, on the shapes of that file
 and of tests/test_gpu_window_sink.py, plus shapes chosen for the loops' corners: an odd number of
 32-key blocks, a single block, fewer blocks than the rings hold, query lengths that are not multiples

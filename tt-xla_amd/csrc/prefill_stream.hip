@@ -526,8 +526,13 @@ int launch_form(const PrefillArgs &a, hipStream_t st) {
   b.spg = nqt, b.spg_even = 0;
   b.parts = 1;
   constexpr bool PAGED = FORM == kPaged || FORM == kPaged32;
-  if (PAGED && a.part_acc && a.part_bytes >= part_bytes(a, HPW)) b.parts = launch_parts(a, HPW);
-  if (HPW == 4 && (FORM == kDense || FORM == kPaged) && b.parts == 1) {
+  // (read on every call) an experiment's override: several row blocks per workgroup, each over all of its keys
+  const char *e = HPW == 4 && (FORM == kDense || FORM == kPaged) ? getenv("TTPA_PREFILL_WGS_PER_GROUP") : nullptr;
+  const int per_group = e ? atoi(e) : 0;
+  if (PAGED && per_group <= 0 && a.part_acc && a.part_bytes >= part_bytes(a, HPW)) b.parts = launch_parts(a, HPW);
+  if (per_group > 0) {
+    b.spg = std::min(nqt, per_group);
+  } else if (HPW == 4 && (FORM == kDense || FORM == kPaged) && b.parts == 1) {
     // Row blocks of nearly one weight (a chunk far into its sequence, or no causal mask) that fill the
     // chip more than once: one round of workgroups with equal shares instead, which saves the later
     // rounds' start-up (267 -> 261 us on 4 x 512-token chunks behind 4096 tokens, 64 heads).  The
@@ -536,9 +541,6 @@ int launch_form(const PrefillArgs &a, hipStream_t st) {
     if (cus <= 0) cus = 256;
     const int one_round = (2 * cus + ny8 * 8 - 1) / (ny8 * 8);
     b.spg_even = one_round < nqt && nqt % one_round == 0 ? one_round : 0;
-    if (const char *e = getenv("TTPA_PREFILL_WGS_PER_GROUP")) {  // (read on every call) an experiment's override
-      if (atoi(e) > 0) b.spg = std::min(nqt, atoi(e)), b.spg_even = 0;
-    }
   }
   int grid = b.spg * b.parts * ny8 * 8;
   if (!PAGED && FORM != kDenseWide && a.fill_kc) grid = grid_with_fill(b, grid, kD);
