@@ -93,10 +93,12 @@ def test_as_close_to_64_bits_as_the_plain_loop(hq, hkv, s, window, monkeypatch):
 
 @pytest.mark.parametrize("hq,hkv,bs,bfp8", [(3, 3, 32, False), (4, 2, 64, False), (8, 2, 32, False), (8, 2, 64, False), (8, 2, 64, True)])
 @pytest.mark.parametrize("start,lc", [(-40, 96), (-1000, 96), (-32, 32), (-2000000000, 33), (2000000000, 33)])
-def test_chunk_that_starts_outside_the_sequence(hq, hkv, bs, bfp8, start, lc):
+@pytest.mark.parametrize("slots", [None, "1"])  # a workgroup per row block; one that walks them all, the blind ones last
+def test_chunk_that_starts_outside_the_sequence(hq, hkv, bs, bfp8, start, lc, slots, monkeypatch):
     """Row i sees keys up to start + i: none is NaN (softmax over nothing), as in the plain loop.  The start is in
-    device memory, so no check of the host's sees it; a block count of
-    zero or less would never count down to zero."""
+    device memory, so no check of the host's sees it; a block count of zero or less would never count down to zero."""
+    if slots:
+        monkeypatch.setenv("TTPA_PREFILL_WGS_PER_GROUP", slots)
     g = torch.Generator().manual_seed(hq + bs + lc)
     users, nbpu = 2, 20
     key, value, table = P._paged(g, users, nbpu, hkv, bs, 128, False)

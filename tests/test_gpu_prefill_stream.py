@@ -5,8 +5,7 @@ forms in test_gpu_prefill_forms.py.  TTPA_PREFILL_STREAM=0, read on every call, 
 compiler-scheduled loop that serves every other shape, and TTPA_PREFILL_WGS_PER_GROUP=n makes a
 workgroup of the hand-scheduled loop walk several blocks of query rows in turn, each over all of its
 keys, instead of one (dense, and cache blocks of whole 64-key tiles).  Every case runs under each
-setting.  Same
-oracle, inputs and bar (atol = rtol = 2e-2) as tests/test_gpu_prefill.py, on the shapes of that file
+setting.  Same oracle, inputs and bar (atol = rtol = 2e-2) as tests/test_gpu_prefill.py, on the shapes of that file
 and of tests/test_gpu_window_sink.py, plus shapes chosen for the loops' corners: an odd number of
 32-key blocks, a single block, fewer blocks than the rings hold, query lengths that are not multiples
 of 64, an additive mask, the ragged end of K / V inside a block, paged blocks smaller than a tile."""

@@ -559,6 +559,7 @@ def item_blocks(o):
     o.e(f"s_min_i32 s88, s88, {S_SKV}")
     o.e(f"s_cmp_eq_u32 {S_CAUSAL}, 0")
     o.e(f"s_cselect_b32 s88, {S_SKV}, s88")
+    o.e("s_max_i32 s88, s88, 1")                        # (at least one block: they are counted down to zero)
     o.e("s_add_u32 s88, s88, 31")
     o.e(f"s_lshr_b32 {S_NB}, s88, 5")
     o.e(f"s_mov_b32 {S_KLEFT}, {S_NB}")
