@@ -346,6 +346,13 @@ def _check_out(out, shape, name):
     return out
 
 
+def _storable(out):
+    """``out`` if the kernels' vector stores can write it, else a fresh tensor of its shape, for the caller to copy back."""
+    if out.stride(-1) != 1 or out.data_ptr() % 16 or any(st % 4 for st in out.stride()[:-1]):
+        return torch.empty(out.shape, dtype=out.dtype, device=out.device)
+    return out
+
+
 def _decode(query, key, value, page_table, is_causal, attn_mask, cur_pos_tensor, attention_sink, scale,
             sliding_window_size, k_new, v_new, out=None):
     """Checks and launch shared by the decode operator and the fused update + decode operator
@@ -1118,7 +1125,12 @@ def split_key_prefill_out(
         raise ValueError(f"query sequence length must be divisible by 32 but got {s}.")
     if any(t.dtype != torch.bfloat16 for t in (q_nope, q_rope, k_nope, k_rope, value)):
         raise ValueError("query, key and value must be bfloat16")
-    _split_key_prefill(q_nope, q_rope, k_nope, k_rope, value, out, scale)
+    if out.dtype != torch.bfloat16 or out.shape != (b, hq, s, 128):
+        raise ValueError(f"out must be bfloat16 of shape {(b, hq, s, 128)}, got {out.dtype} {tuple(out.shape)}")
+    target = _storable(out)
+    _split_key_prefill(q_nope, q_rope, k_nope, k_rope, value, target, scale)
+    if target is not out:
+        out.copy_(target)
 
 
 @torch.library.custom_op("tt::latent_decode_step_", mutates_args=["cache", "out"], device_types=["cuda"])
@@ -1152,8 +1164,7 @@ def latent_decode_step_(
     if page_table.dim() != 2 or page_table.shape[0] != users or cur_pos_tensor.shape != (users,):
         raise ValueError("page_table / cur_pos_tensor must have one row per user")
     q_nope, q_rope, latent, rope, w_uk_t, w_uv = map(_rows_contiguous, (q_nope, q_rope, latent, rope, w_uk_t, w_uv))
-    if out.stride(-1) != 1 or out.data_ptr() % 16 or out.stride(0) % 4 or out.stride(1) % 4:
-        raise ValueError("latent step: out needs contiguous 16-byte aligned rows and strides that are multiples of 4")
+    target = _storable(out)
     pt, cur = _table(page_table), _index_tensor(cur_pos_tensor)
     for u0 in range(0, users, _MLA_MAX_USERS):
         n = min(_MLA_MAX_USERS, users - u0)
@@ -1164,12 +1175,14 @@ def latent_decode_step_(
         at = lambda t: t.data_ptr() + u0 * t.stride(0) * t.element_size()  # noqa: E731
         N.call(
             "ttpa_latent_decode_step",
-            at(out), out.stride(0), out.stride(1), at(q_nope), q_nope.stride(0), q_nope.stride(1),
+            at(target), target.stride(0), target.stride(1), at(q_nope), q_nope.stride(0), q_nope.stride(1),
             at(q_rope), q_rope.stride(0), q_rope.stride(1), at(latent), latent.stride(0), at(rope), rope.stride(0),
             w_uk_t.data_ptr(), w_uk_t.stride(0), w_uk_t.stride(1), w_uv.data_ptr(), w_uv.stride(0), w_uv.stride(1),
             cache.data_ptr(), at(pt), pt.stride(0), at(cur), int(cur.dtype == torch.int64), n, heads, bs, pt.shape[1], nb,
             float(scale), ws.data_ptr(), ws_bytes, _stream(),
         )
+    if target is not out:
+        out.copy_(target)
 
 
 @torch.library.custom_op("tt::paged_fill_latent_cache_", mutates_args=["cache"], device_types=["cuda"])
