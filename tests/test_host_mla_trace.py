@@ -1,5 +1,7 @@
-"""The latent backend's forward is one graph to a tracer: decode step and prompt pass of the head shape
-with operators of its own, and of another one, on fake tensors of the GPU type (nothing is computed)."""
+"""The latent backend's forward under a tracer and under differentiation, on fake tensors of the GPU type
+(nothing is computed): decode step and prompt pass of the head shape with operators of its own, and of
+another one, are one graph; where something looks at the weights' derivative or maps over them, the pass
+goes through the operators in turn, whose output expansion is an ordinary product."""
 
 import types
 
@@ -50,3 +52,30 @@ def test_one_graph_of_operators(s):
         forward, _, args = _forward(2, s, nope=64)
         torch._dynamo.reset()
         torch.compile(forward, fullgraph=True, backend="eager")(*args)
+
+
+@pytest.mark.parametrize("s", [1, 64])
+def test_output_depends_on_the_weights(s):
+    with FakeTensorMode():
+        forward, layer, args = _forward(2, s)
+        layer.W_UV.requires_grad_()
+        assert forward(*args).requires_grad
+        with torch.no_grad():
+            assert not forward(*args[:4], torch.empty_like(args[4])).requires_grad
+
+
+@pytest.mark.parametrize("s", [1, 64])
+def test_forward_mode_and_vmap(s):
+    fw = torch.autograd.forward_ad
+    with FakeTensorMode():
+        forward, layer, args = _forward(2, s)
+        plain = layer.W_UV
+        with fw.dual_level():
+            layer.W_UV = fw.make_dual(plain, torch.empty_like(plain))
+            assert fw.unpack_dual(forward(*args)).tangent is not None
+
+        def one(w_uv, out):
+            layer.W_UV = w_uv
+            return forward(*args[:4], out)
+
+        assert torch.vmap(one)(torch.stack([plain] * 3), torch.stack([args[4]] * 3)).shape == (3,) + args[4].shape

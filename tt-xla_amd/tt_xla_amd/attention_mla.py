@@ -207,9 +207,16 @@ class TTMLAAttentionBackendImpl(_ImplBase):
         return torch.einsum(pattern, out_lat, layer.W_UV.to(device=out_lat.device))
 
     def _bf16_on_gpu(self, *tensors) -> bool:
-        """bfloat16 on one GPU.  (The weights are plain attributes and may sit elsewhere: such a pass moves them.)"""
+        """bfloat16 on one GPU.  (The weights are plain attributes and may sit elsewhere: such a pass moves them.)
+        Not if autograd, a forward-mode derivative or a functional transform may look at one of them: the operators
+        that take a pass at once have no derivative, while the products around the attention have."""
         device = tensors[0].device
-        return device.type == "cuda" and all(t.device == device and t.dtype == torch.bfloat16 for t in tensors)
+        if device.type != "cuda" or not all(t.device == device and t.dtype == torch.bfloat16 for t in tensors):
+            return False
+        if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+            return False
+        return torch.compiler.is_compiling() or (
+            torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None)
 
     def _steps_at_once(self, q_nope, q_pe, kv_c_normed, k_pe, kv_cache, attn_metadata, layer, output) -> bool:
         """Whether a decode pass is one ``tt::latent_decode_step_``: the head shape it is built for, causal, with a
