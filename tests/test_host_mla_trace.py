@@ -10,7 +10,7 @@ import torch
 from torch._subclasses import FakeTensorMode
 
 
-def _forward(users, s, n=16, nope=128, rope=64, lat=512, vd=128):
+def _forward(users, s, n=16, nope=128, rope=64, lat=512, vd=128, **kw):
     import __graft_entry__  # noqa: F401  (puts the package on sys.path)
     from tt_xla_amd import attention_mla as M
     from tt_xla_amd.attention import TTMetadata
@@ -18,9 +18,9 @@ def _forward(users, s, n=16, nope=128, rope=64, lat=512, vd=128):
     new = lambda *shape, dtype=torch.bfloat16: torch.empty(*shape, dtype=dtype, device="cuda")  # noqa: E731
     layer = types.SimpleNamespace(W_UK_T=new(n, nope, lat), W_UV=new(n, lat, vd))
     impl = M.TTMLAAttentionBackendImpl(
-        num_heads=n, head_size=lat + rope, scale=(nope + rope) ** -0.5, num_kv_heads=1, alibi_slopes=None, sliding_window=None,
-        kv_cache_dtype="auto", logits_soft_cap=None, attn_type="decoder", kv_sharing_target_layer_name=None, kv_lora_rank=lat,
-        qk_nope_head_dim=nope, qk_rope_head_dim=rope, qk_head_dim=nope + rope, v_head_dim=vd)
+        **{**dict(num_heads=n, head_size=lat + rope, scale=(nope + rope) ** -0.5, num_kv_heads=1, alibi_slopes=None, sliding_window=None,
+                  kv_cache_dtype="auto", logits_soft_cap=None, attn_type="decoder", kv_sharing_target_layer_name=None, kv_lora_rank=lat,
+                  qk_nope_head_dim=nope, qk_rope_head_dim=rope, qk_head_dim=nope + rope, v_head_dim=vd), **kw})
     meta = TTMetadata(cache_position=new(users, dtype=torch.int32), page_table=new(users, 4, dtype=torch.int32), is_causal=True)
     cache, t = new(9, 1, 32, lat + rope), users * s
 
@@ -79,3 +79,11 @@ def test_forward_mode_and_vmap(s):
             return forward(*args[:4], out)
 
         assert torch.vmap(one)(torch.stack([plain] * 3), torch.stack([args[4]] * 3)).shape == (3,) + args[4].shape
+
+
+@pytest.mark.parametrize("s", [1, 64])
+def test_scale_of_the_operators(s):
+    """Without a scale of its own the layer uses the operators' default."""
+    with FakeTensorMode():
+        forward, _, args = _forward(2, s, scale=None)
+        forward(*args)

@@ -225,6 +225,8 @@ class TTMLAAttentionBackendImpl(_ImplBase):
             return False
         if self.functional_cache_ops or not attn_metadata.is_causal or not self._has_cache(kv_cache) or not kv_cache.is_contiguous():
             return False
+        if self.scale is None:  # (the operators' default is theirs to choose)
+            return False
         if not self._bf16_on_gpu(q_nope, q_pe, kv_c_normed, k_pe, layer.W_UK_T, layer.W_UV, kv_cache, output):
             return False
         return output.is_contiguous()  # (its address is the operator's business: a traced tensor has none)
@@ -238,7 +240,7 @@ class TTMLAAttentionBackendImpl(_ImplBase):
             return False
         if attn_metadata is not None and (attn_metadata.attn_mask is not None or not attn_metadata.is_causal):
             return False
-        if not self._bf16_on_gpu(q_nope, q_pe, kv_c_normed, k_pe, layer.W_UK_T, layer.W_UV, output) or not self.scale > 0:
+        if not self._bf16_on_gpu(q_nope, q_pe, kv_c_normed, k_pe, layer.W_UK_T, layer.W_UV, output) or self.scale is None or not self.scale > 0:
             return False
         if attn_metadata is not None and self._has_cache(kv_cache) and kv_cache.dtype != torch.bfloat16:
             return False
