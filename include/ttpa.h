@@ -527,6 +527,22 @@ int ttpa_latent_decode_step(void *out, int64_t out_user_stride, int64_t out_head
                             int32_t heads, int32_t block_size, int32_t table_width, int32_t num_blocks, float scale,
                             void *workspace, size_t workspace_bytes, void *stream);
 size_t ttpa_latent_decode_step_workspace_bytes(int32_t users, int32_t heads);
+/*
+ * The same step with weights read as they lie, also where they are transposed views: w_uk [heads, 128, 512] and w_uv
+ * [heads, 512, 128] by head, row and column strides, of which the column stride (rows contiguous) or the row stride
+ * (columns contiguous) is 1.  Either layout of either weight costs the same.
+ */
+int ttpa_latent_decode_step_strided(void *out, int64_t out_user_stride, int64_t out_head_stride, const void *q_nope,
+                                    int64_t q_nope_user_stride, int64_t q_nope_head_stride, const void *q_rope,
+                                    int64_t q_rope_user_stride, int64_t q_rope_head_stride, const void *latent,
+                                    int64_t latent_user_stride, const void *rope, int64_t rope_user_stride,
+                                    const void *w_uk, int64_t w_uk_head_stride, int64_t w_uk_row_stride,
+                                    int64_t w_uk_column_stride, const void *w_uv, int64_t w_uv_head_stride,
+                                    int64_t w_uv_row_stride, int64_t w_uv_column_stride, void *cache,
+                                    const int32_t *page_table, int64_t page_table_row_stride, const void *cur_pos,
+                                    int cur_pos_is_i64, int32_t users, int32_t heads, int32_t block_size,
+                                    int32_t table_width, int32_t num_blocks, float scale, void *workspace,
+                                    size_t workspace_bytes, void *stream);
 
 /*
  * paged_fill_cache of latent rows that are still in two parts: row t of user u, [latent_size] from `latent` and

@@ -1,4 +1,4 @@
-"""The latent backend's passes in the forms that its own operators take or leave: outputs that are not
+"""The latent backend's passes in the forms that its own operators take or leave: weights in every layout, outputs that are not
 aligned.  Compared with the same pass in its ordinary form, bit for bit."""
 
 import math
@@ -63,3 +63,43 @@ def test_output_that_is_not_aligned(s):
     room = torch.zeros(want.numel() + 1, dtype=torch.bfloat16, device="cuda")
     got, cache = _run(impl, p, out=room[1:].view(want.shape))
     assert torch.equal(got, want) and torch.equal(cache, want_cache) and room[0] == 0
+
+
+def _as_projection_leaves_them(layer, joint):
+    """The same weights as views of one joint projection: [512, heads, 256] (W_UK_T's columns are contiguous) or
+    [heads * 256, 512] (W_UV's are)."""
+    n = layer.W_UK_T.shape[0]
+    uk, uv = layer.W_UK_T.permute(2, 0, 1), layer.W_UV.permute(1, 0, 2)  # [512, heads, 128]
+    if joint == "latent first":
+        both = torch.cat([uk, uv], -1).contiguous()
+    else:
+        both = torch.cat([uk, uv], -1).permute(1, 2, 0).reshape(n * 256, 512).contiguous().t().view(512, n, 256)
+    uk, uv = both.split([128, 128], -1)
+    return types.SimpleNamespace(W_UK_T=uk.permute(1, 2, 0), W_UV=uv.transpose(0, 1))
+
+
+@pytest.mark.parametrize("joint", ["latent first", "heads first"])
+@pytest.mark.parametrize("n,users", [(16, 1), (16, 32), (3, 33), (16, 130), (128, 5)])
+def test_weights_are_read_as_they_lie(n, users, joint):
+    """Views of a joint projection: the same products in the same order, and no copy of a weight."""
+    p, impl = _pass(users, n, users, 1), _impl(n)
+    want, want_cache = _run(impl, p)
+    layer = _as_projection_leaves_them(p.layer, joint)
+    assert torch.equal(layer.W_UK_T, p.layer.W_UK_T) and torch.equal(layer.W_UV, p.layer.W_UV)
+    assert not (layer.W_UK_T.stride(2) == 1 and layer.W_UV.stride(2) == 1)
+    cache, got = p.cache.clone(), torch.zeros_like(want)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    _run(impl, p, out=got, layer=layer, cache=cache)
+    torch.cuda.synchronize()
+    assert torch.cuda.max_memory_allocated() - before < 2 * n * 128 * 512
+    assert torch.equal(got, want) and torch.equal(cache, want_cache)
+
+
+def test_weights_of_any_other_layout():
+    p, impl = _pass(9, 16, 3, 1), _impl(16)
+    want, _ = _run(impl, p)
+    spread = lambda t: torch.stack([t, t], -1)[..., 0]  # noqa: E731  (no dimension contiguous)
+    got, _ = _run(impl, p, layer=types.SimpleNamespace(W_UK_T=spread(p.layer.W_UK_T), W_UV=spread(p.layer.W_UV)))
+    assert torch.equal(got, want)

@@ -11,7 +11,13 @@
 // users) for the query, (32 value columns, head, 32 users) with the contraction over the latent width cut
 // between the four wavefronts for the value.  A weight tile travels memory -> LDS directly and is read
 // through the transposing LDS load, so that v_mfma_f32_32x32x16_bf16 gets the users as its columns and
-// the activations go from memory to registers as they are.  128 users, 16 heads: 8.2 and 5.0 us, where two
+// the activations go from memory to registers as they are.
+// A weight whose contracted dimension is the contiguous one (how a joint projection [heads * (128 + 128), 512] leaves W_UV
+// after a split and a transposition, and [512, heads, 128 + 128] leaves W_UK) is the operand that the matrix instruction
+// wants: lane (column, half) takes 8 consecutive elements per step, from memory to registers, without LDS.  (A copy into
+// the other layout took a pass over the weights, 2 MB at 16 heads and 16 MB at 128, in front of every step: captured steps
+// with either of these layouts, one user over 512 tokens at 16 heads 33.8 -> 27.1 us, 128 users 86.4 -> 79.4, one user at 128
+// heads 83.2 -> 52.0 and 81.1 -> 48.4; with rows contiguous 26.7, 78.8 and 49.9.)  128 users, 16 heads: 8.2 and 5.0 us, where two
 // batched library products, two concatenations, the cache write and the copy to the output took 41 us in six
 // launches; the whole pass over contexts of 512 .. 8192 168 -> 94 us, of one user over 512 tokens 149 -> 37 us.
 #include "common.h"
@@ -31,7 +37,8 @@ constexpr int kUsers = 32;  // users per workgroup: the 32-wide dimension of the
 
 struct StepArgs {
   const uint16_t *q_nope, *q_rope, *latent, *rope, *w_uk, *w_uv;
-  int64_t qn_us, qn_hs, qr_us, qr_hs, latent_us, rope_us, uk_hs, uk_rs, uv_hs, uv_rs;
+  int64_t qn_us, qn_hs, qr_us, qr_hs, latent_us, rope_us;
+  int64_t uk_hs, uk_ld, uv_hs, uv_ld;  // head stride, and the stride of the dimension that is not contiguous
   uint16_t *q_lat, *o_lat;  // [users][heads][kRow], [users][heads][kLatent]
   uint16_t *out;
   int64_t out_us, out_hs;
@@ -56,8 +63,17 @@ __device__ __forceinline__ bf16x8 read_transposed(const unsigned char *first, in
   return __builtin_bit_cast(bf16x8, t);
 }
 
+// The eight A operands of a wavefront where the contracted dimension is contiguous: `column` is the lane's column (32 of
+// them `ld` elements apart), at the lane's first element of the contracted dimension.
+__device__ __forceinline__ void load_columns(bf16x8 (&w)[8], const uint16_t *column) {
+#pragma unroll
+  for (int s = 0; s < 8; ++s) w[s] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(column + 16 * s));
+}
+
+// COLUMNS: the weight's contracted dimension is contiguous (else its columns are).
+template <bool COLUMNS>
 __global__ __launch_bounds__(256) void latent_query_kernel(StepArgs a) {
-  __shared__ __attribute__((aligned(1024))) unsigned char tile[kNope * 256];  // 128 rows of 128 columns
+  __shared__ __attribute__((aligned(1024))) unsigned char tile[COLUMNS ? 1024 : kNope * 256];  // 128 rows of 128 columns
   const int col0 = blockIdx.x * 128, head = blockIdx.y, u0 = blockIdx.z * kUsers;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -65,12 +81,17 @@ __global__ __launch_bounds__(256) void latent_query_kernel(StepArgs a) {
 
   // weights: 32 segments of four rows; 16-byte chunk c of row r lies at chunk position c ^ 4 (r % 4), which puts the
   // four rows of a transposing read in different banks
-  const uint16_t *w = a.w_uk + head * a.uk_hs + col0;
-  const uint32_t lane_bytes = (uint32_t)(lane >> 4) * (uint32_t)(2 * a.uk_rs) + 16u * (uint32_t)((lane & 15) ^ (4 * (lane >> 4)));
+  bf16x8 columns[8];
+  if constexpr (COLUMNS) {
+    load_columns(columns, a.w_uk + head * a.uk_hs + (int64_t)(col0 + 32 * wave + n) * a.uk_ld + 8 * h);
+  } else {
+    const uint16_t *w = a.w_uk + head * a.uk_hs + col0;
+    const uint32_t lane_bytes = (uint32_t)(lane >> 4) * (uint32_t)(2 * a.uk_ld) + 16u * (uint32_t)((lane & 15) ^ (4 * (lane >> 4)));
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const int seg = 8 * wave + j;
-    dma16_uniform(w + (int64_t)(4 * seg) * a.uk_rs, lane_bytes, lds_address(tile) + 1024u * (uint32_t)seg);
+    for (int j = 0; j < 8; ++j) {
+      const int seg = 8 * wave + j;
+      dma16_uniform(w + (int64_t)(4 * seg) * a.uk_ld, lane_bytes, lds_address(tile) + 1024u * (uint32_t)seg);
+    }
   }
   const int u = min(u0 + n, a.users - 1);
   bf16x8 q[8];
@@ -95,8 +116,10 @@ __global__ __launch_bounds__(256) void latent_query_kernel(StepArgs a) {
       *reinterpret_cast<uint4 *>(a.cache + ((int64_t)phys * a.bs + row) * kRow + at) = *reinterpret_cast<const uint4 *>(src);
     }
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's segments have landed
-  __syncthreads();
+  if constexpr (!COLUMNS) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's segments have landed
+    __syncthreads();
+  }
 
   floatx16 acc;
 #pragma unroll
@@ -105,7 +128,12 @@ __global__ __launch_bounds__(256) void latent_query_kernel(StepArgs a) {
   const int row = 8 * (grp >> 1) + (a16 >> 2), chunk = 4 * wave + 2 * (grp & 1) + ((a16 & 3) >> 1);
   const unsigned char *first = tile + row * 256 + 16 * (chunk ^ (4 * (row & 3))) + 8 * (a16 & 1);
 #pragma unroll
-  for (int s = 0; s < 8; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(read_transposed(first + s * 16 * 256, 4 * 256), q[s], acc, 0, 0, 0);
+  for (int s = 0; s < 8; ++s) {
+    bf16x8 w;
+    if constexpr (COLUMNS) w = columns[s];
+    else w = read_transposed(first + s * 16 * 256, 4 * 256);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, q[s], acc, 0, 0, 0);
+  }
   if (u0 + n >= a.users) return;
   uint16_t *dst = a.q_lat + ((int64_t)(u0 + n) * a.heads + head) * kRow + col0 + 32 * wave + 4 * h;
 #pragma unroll
@@ -113,26 +141,32 @@ __global__ __launch_bounds__(256) void latent_query_kernel(StepArgs a) {
     *reinterpret_cast<uint2 *>(dst + 8 * j) = make_uint2(pack_bf16x2(acc[4 * j], acc[4 * j + 1]), pack_bf16x2(acc[4 * j + 2], acc[4 * j + 3]));
 }
 
+template <bool COLUMNS>
 __global__ __launch_bounds__(256) void latent_value_kernel(StepArgs a) {
   constexpr int kPitch = 36;  // floats of a user's partial sums: rows of 16-byte writes in different banks
-  __shared__ __attribute__((aligned(1024))) unsigned char tile[kLatent * 64];  // 512 rows of 32 columns, 128 per wavefront
+  __shared__ __attribute__((aligned(1024))) unsigned char tile[COLUMNS ? 1024 : kLatent * 64];  // 512 rows of 32 columns, 128 per wavefront
   __shared__ __attribute__((aligned(16))) float sums[4][kUsers * kPitch];
   const int col0 = blockIdx.x * 32, head = blockIdx.y, u0 = blockIdx.z * kUsers;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, h = lane >> 5;
   // weights: 8 segments of sixteen 64-byte rows per wavefront (four rows of a transposing read are 256 consecutive bytes)
-  const uint16_t *w = a.w_uv + head * a.uv_hs + (int64_t)(128 * wave) * a.uv_rs + col0;
-  const uint32_t lane_bytes = (uint32_t)(lane >> 2) * (uint32_t)(2 * a.uv_rs) + 16u * (uint32_t)(lane & 3);
+  bf16x8 columns[8];
+  if constexpr (COLUMNS) {
+    load_columns(columns, a.w_uv + head * a.uv_hs + (int64_t)(col0 + n) * a.uv_ld + 128 * wave + 8 * h);
+  } else {
+    const uint16_t *w = a.w_uv + head * a.uv_hs + (int64_t)(128 * wave) * a.uv_ld + col0;
+    const uint32_t lane_bytes = (uint32_t)(lane >> 2) * (uint32_t)(2 * a.uv_ld) + 16u * (uint32_t)(lane & 3);
 #pragma unroll
-  for (int j = 0; j < 8; ++j)
-    dma16_uniform(w + (int64_t)(16 * j) * a.uv_rs, lane_bytes, lds_address(tile) + 8192u * (uint32_t)wave + 1024u * j);
+    for (int j = 0; j < 8; ++j)
+      dma16_uniform(w + (int64_t)(16 * j) * a.uv_ld, lane_bytes, lds_address(tile) + 8192u * (uint32_t)wave + 1024u * j);
+  }
   const int u = min(u0 + n, a.users - 1);
   bf16x8 o[8];
   const uint16_t *op = a.o_lat + ((int64_t)u * a.heads + head) * kLatent + 128 * wave + 8 * h;
 #pragma unroll
   for (int s = 0; s < 8; ++s) o[s] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(op + 16 * s));
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // a wavefront reads the segments that it requested
+  if constexpr (!COLUMNS) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // a wavefront reads the segments that it requested
 
   floatx16 acc;
 #pragma unroll
@@ -140,7 +174,12 @@ __global__ __launch_bounds__(256) void latent_value_kernel(StepArgs a) {
   const int grp = lane >> 4, a16 = lane & 15;
   const unsigned char *first = tile + 8192 * wave + (8 * (grp >> 1) + (a16 >> 2)) * 64 + 32 * (grp & 1) + 8 * (a16 & 3);
 #pragma unroll
-  for (int s = 0; s < 8; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(read_transposed(first + s * 16 * 64, 4 * 64), o[s], acc, 0, 0, 0);
+  for (int s = 0; s < 8; ++s) {
+    bf16x8 w;
+    if constexpr (COLUMNS) w = columns[s];
+    else w = read_transposed(first + s * 16 * 64, 4 * 64);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, o[s], acc, 0, 0, 0);
+  }
 #pragma unroll
   for (int j = 0; j < 4; ++j)
     *reinterpret_cast<float4 *>(&sums[wave][n * kPitch + 8 * j + 4 * h]) = make_float4(acc[4 * j], acc[4 * j + 1], acc[4 * j + 2], acc[4 * j + 3]);
@@ -170,25 +209,43 @@ extern "C" size_t ttpa_latent_decode_step_workspace_bytes(int32_t users, int32_t
   return align256(attn) + align256((size_t)users * heads * kRow * 2) + align256((size_t)users * heads * kLatent * 2);
 }
 
-extern "C" int ttpa_latent_decode_step(
-    void *out, int64_t out_user_stride, int64_t out_head_stride, const void *q_nope, int64_t q_nope_user_stride,
-    int64_t q_nope_head_stride, const void *q_rope, int64_t q_rope_user_stride, int64_t q_rope_head_stride, const void *latent,
-    int64_t latent_user_stride, const void *rope, int64_t rope_user_stride, const void *w_uk, int64_t w_uk_head_stride,
-    int64_t w_uk_row_stride, const void *w_uv, int64_t w_uv_head_stride, int64_t w_uv_row_stride, void *cache,
-    const int32_t *page_table, int64_t page_table_row_stride, const void *cur_pos, int cur_pos_is_i64, int32_t users,
-    int32_t heads, int32_t block_size, int32_t table_width, int32_t num_blocks, float scale, void *workspace,
-    size_t workspace_bytes, void *stream) {
+#define TTPA_LATENT_STEP_HEAD                                                                                          \
+  void *out, int64_t out_user_stride, int64_t out_head_stride, const void *q_nope, int64_t q_nope_user_stride,          \
+      int64_t q_nope_head_stride, const void *q_rope, int64_t q_rope_user_stride, int64_t q_rope_head_stride,           \
+      const void *latent, int64_t latent_user_stride, const void *rope, int64_t rope_user_stride, const void *w_uk
+#define TTPA_LATENT_STEP_TAIL                                                                                          \
+  void *cache, const int32_t *page_table, int64_t page_table_row_stride, const void *cur_pos, int cur_pos_is_i64,       \
+      int32_t users, int32_t heads, int32_t block_size, int32_t table_width, int32_t num_blocks, float scale,           \
+      void *workspace, size_t workspace_bytes, void *stream
+
+extern "C" int ttpa_latent_decode_step(TTPA_LATENT_STEP_HEAD, int64_t w_uk_head_stride, int64_t w_uk_row_stride, const void *w_uv,
+                                       int64_t w_uv_head_stride, int64_t w_uv_row_stride, TTPA_LATENT_STEP_TAIL) {
+  return ttpa_latent_decode_step_strided(
+      out, out_user_stride, out_head_stride, q_nope, q_nope_user_stride, q_nope_head_stride, q_rope, q_rope_user_stride,
+      q_rope_head_stride, latent, latent_user_stride, rope, rope_user_stride, w_uk, w_uk_head_stride, w_uk_row_stride, 1, w_uv,
+      w_uv_head_stride, w_uv_row_stride, 1, cache, page_table, page_table_row_stride, cur_pos, cur_pos_is_i64, users, heads,
+      block_size, table_width, num_blocks, scale, workspace, workspace_bytes, stream);
+}
+
+extern "C" int ttpa_latent_decode_step_strided(TTPA_LATENT_STEP_HEAD, int64_t w_uk_head_stride, int64_t w_uk_row_stride,
+                                               int64_t w_uk_column_stride, const void *w_uv, int64_t w_uv_head_stride,
+                                               int64_t w_uv_row_stride, int64_t w_uv_column_stride, TTPA_LATENT_STEP_TAIL) {
   TTPA_REQUIRE(out && q_nope && q_rope && latent && rope && w_uk && w_uv && cache && page_table && cur_pos, "null pointer argument");
   TTPA_REQUIRE(users > 0 && heads > 0 && block_size > 0 && table_width > 0 && num_blocks > 0, "non-positive dimension");
   TTPA_REQUIRE(aligned16(q_nope) && aligned16(q_rope) && aligned16(latent) && aligned16(rope) && aligned16(w_uk) && aligned16(w_uv) &&
                    aligned16(cache) && (reinterpret_cast<uintptr_t>(out) & 7u) == 0,
                "latent step: operands must be 16-byte aligned");
   const int64_t strides[] = {q_nope_user_stride, q_nope_head_stride, q_rope_user_stride, q_rope_head_stride, latent_user_stride,
-                             rope_user_stride, w_uk_head_stride, w_uk_row_stride, w_uv_head_stride, w_uv_row_stride};
+                             rope_user_stride, w_uk_head_stride, w_uv_head_stride};
   for (int64_t s : strides) TTPA_REQUIRE(s % 8 == 0, "latent step: strides must be multiples of 8 elements");
   TTPA_REQUIRE(out_user_stride % 4 == 0 && out_head_stride % 4 == 0, "latent step: out strides must be multiples of 4 elements");
-  TTPA_REQUIRE(w_uk_row_stride > 0 && w_uk_row_stride < (1 << 24) && w_uv_row_stride > 0 && w_uv_row_stride < (1 << 24),
-               "latent step: weight row stride out of range");
+  // one of a weight's two inner dimensions is contiguous, the other's stride whole 16-byte pieces
+  const bool uk_columns = w_uk_column_stride != 1, uv_columns = w_uv_column_stride != 1;
+  const int64_t uk_ld = uk_columns ? w_uk_column_stride : w_uk_row_stride, uv_ld = uv_columns ? w_uv_column_stride : w_uv_row_stride;
+  TTPA_REQUIRE((!uk_columns || w_uk_row_stride == 1) && (!uv_columns || w_uv_row_stride == 1),
+               "latent step: the rows or the columns of a weight must be contiguous");
+  TTPA_REQUIRE(uk_ld % 8 == 0 && uv_ld % 8 == 0, "latent step: strides must be multiples of 8 elements");
+  TTPA_REQUIRE(uk_ld > 0 && uk_ld < (1 << 24) && uv_ld > 0 && uv_ld < (1 << 24), "latent step: weight row stride out of range");
   TTPA_REQUIRE(heads <= 65535 && (users + kUsers - 1) / kUsers <= 65535, "latent step: too many heads or users for one launch");
   const size_t need = ttpa_latent_decode_step_workspace_bytes(users, heads);
   if (need == 0) return fail(TTPA_ERR_UNSUPPORTED, "latent step: %d heads are not built", heads);
@@ -200,8 +257,8 @@ extern "C" int ttpa_latent_decode_step(
   a.q_rope = static_cast<const uint16_t *>(q_rope), a.qr_us = q_rope_user_stride, a.qr_hs = q_rope_head_stride;
   a.latent = static_cast<const uint16_t *>(latent), a.latent_us = latent_user_stride;
   a.rope = static_cast<const uint16_t *>(rope), a.rope_us = rope_user_stride;
-  a.w_uk = static_cast<const uint16_t *>(w_uk), a.uk_hs = w_uk_head_stride, a.uk_rs = w_uk_row_stride;
-  a.w_uv = static_cast<const uint16_t *>(w_uv), a.uv_hs = w_uv_head_stride, a.uv_rs = w_uv_row_stride;
+  a.w_uk = static_cast<const uint16_t *>(w_uk), a.uk_hs = w_uk_head_stride, a.uk_ld = uk_ld;
+  a.w_uv = static_cast<const uint16_t *>(w_uv), a.uv_hs = w_uv_head_stride, a.uv_ld = uv_ld;
   a.q_lat = reinterpret_cast<uint16_t *>(static_cast<unsigned char *>(workspace) + attn);
   a.o_lat = reinterpret_cast<uint16_t *>(reinterpret_cast<unsigned char *>(a.q_lat) + align256((size_t)users * heads * kRow * 2));
   a.out = static_cast<uint16_t *>(out), a.out_us = out_user_stride, a.out_hs = out_head_stride;
@@ -210,12 +267,15 @@ extern "C" int ttpa_latent_decode_step(
   a.users = users, a.heads = heads, a.bs = block_size, a.w = table_width, a.nb = num_blocks;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const unsigned tiles = (unsigned)((users + kUsers - 1) / kUsers);
-  latent_query_kernel<<<dim3(kLatent / 128, (unsigned)heads, tiles), dim3(256), 0, st>>>(a);
+  const dim3 query_grid(kLatent / 128, (unsigned)heads, tiles), value_grid(kValue / 32, (unsigned)heads, tiles);
+  if (uk_columns) latent_query_kernel<true><<<query_grid, dim3(256), 0, st>>>(a);
+  else latent_query_kernel<false><<<query_grid, dim3(256), 0, st>>>(a);
   if (int rc = check_launch("latent_decode_step (query)")) return rc;
   if (int rc = ttpa_paged_mla_decode(a.o_lat, (int64_t)heads * kLatent, kLatent, a.q_lat, (int64_t)heads * kRow, kRow, cache, nullptr,
                                      page_table, page_table_row_stride, cur_pos, cur_pos_is_i64, users, heads, 1, kRow, kLatent,
                                      block_size, table_width, num_blocks, scale, nullptr, workspace, attn, stream))
     return rc;
-  latent_value_kernel<<<dim3(kValue / 32, (unsigned)heads, tiles), dim3(256), 0, st>>>(a);
+  if (uv_columns) latent_value_kernel<true><<<value_grid, dim3(256), 0, st>>>(a);
+  else latent_value_kernel<false><<<value_grid, dim3(256), 0, st>>>(a);
   return check_launch("latent_decode_step (value)");
 }

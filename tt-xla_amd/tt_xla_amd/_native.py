@@ -113,6 +113,11 @@ SIGNATURES = {
         [_p, _i64, _i64, _p, _i64, _i64, _p, _i64, _i64, _p, _i64, _p, _i64, _p, _i64, _i64, _p, _i64, _i64,
          _p, _p, _i64, _p, _int, _i32, _i32, _i32, _i32, _i32, _f32, _p, _sz, _p],
     ),
+    "ttpa_latent_decode_step_strided": (
+        _int,
+        [_p, _i64, _i64, _p, _i64, _i64, _p, _i64, _i64, _p, _i64, _p, _i64, _p, _i64, _i64, _i64, _p, _i64, _i64, _i64,
+         _p, _p, _i64, _p, _int, _i32, _i32, _i32, _i32, _i32, _f32, _p, _sz, _p],
+    ),
     "ttpa_split_key_prefill": (
         _int, [_p, _i64, _i64, _i64] * 6 + [_i32, _i32, _i32, _i32, _f32, _p],
     ),

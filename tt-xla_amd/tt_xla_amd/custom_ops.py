@@ -1133,6 +1133,16 @@ def split_key_prefill_out(
         out.copy_(target)
 
 
+def _weight(t: torch.Tensor) -> torch.Tensor:
+    """A weight [heads, rows, columns] as the latent step reads it: rows or columns contiguous, every other stride a
+    multiple of 8 elements, 16-byte base.  Both are what a split of a joint projection leaves; anything else is copied."""
+    hs, rs, cs = t.stride()
+    other = rs if cs == 1 else cs
+    if 1 not in (rs, cs) or hs % 8 or other % 8 or not 0 < other < 1 << 24 or t.data_ptr() % 16:
+        return t.contiguous()
+    return t
+
+
 @torch.library.custom_op("tt::latent_decode_step_", mutates_args=["cache", "out"], device_types=["cuda"])
 def latent_decode_step_(
     q_nope: torch.Tensor,
@@ -1163,7 +1173,8 @@ def latent_decode_step_(
         raise ValueError("the latent step takes bfloat16 tensors and a contiguous cache")
     if page_table.dim() != 2 or page_table.shape[0] != users or cur_pos_tensor.shape != (users,):
         raise ValueError("page_table / cur_pos_tensor must have one row per user")
-    q_nope, q_rope, latent, rope, w_uk_t, w_uv = map(_rows_contiguous, (q_nope, q_rope, latent, rope, w_uk_t, w_uv))
+    q_nope, q_rope, latent, rope = map(_rows_contiguous, (q_nope, q_rope, latent, rope))
+    w_uk_t, w_uv = _weight(w_uk_t), _weight(w_uv)
     target = _storable(out)
     pt, cur = _table(page_table), _index_tensor(cur_pos_tensor)
     for u0 in range(0, users, _MLA_MAX_USERS):
@@ -1174,10 +1185,10 @@ def latent_decode_step_(
         ws = _workspace(ws_bytes, out.device)
         at = lambda t: t.data_ptr() + u0 * t.stride(0) * t.element_size()  # noqa: E731
         N.call(
-            "ttpa_latent_decode_step",
+            "ttpa_latent_decode_step_strided",
             at(target), target.stride(0), target.stride(1), at(q_nope), q_nope.stride(0), q_nope.stride(1),
             at(q_rope), q_rope.stride(0), q_rope.stride(1), at(latent), latent.stride(0), at(rope), rope.stride(0),
-            w_uk_t.data_ptr(), w_uk_t.stride(0), w_uk_t.stride(1), w_uv.data_ptr(), w_uv.stride(0), w_uv.stride(1),
+            w_uk_t.data_ptr(), *w_uk_t.stride(), w_uv.data_ptr(), *w_uv.stride(),
             cache.data_ptr(), at(pt), pt.stride(0), at(cur), int(cur.dtype == torch.int64), n, heads, bs, pt.shape[1], nb,
             float(scale), ws.data_ptr(), ws_bytes, _stream(),
         )
