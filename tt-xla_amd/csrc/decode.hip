@@ -554,7 +554,8 @@ static int decode_impl(void *out, int64_t out_user_stride, int64_t out_head_stri
   if (ev1) (void)hipEventRecord(ev1, st);
   if (use_mfma16) take_profile_events(ev0, ev1);  // still armed only if the launch did not happen
   if (rc) return rc;
-  launch_combine(a, users * kv_heads, g, head_size, st);
+  if (a.k_new) launch_combine<true>(a, users * kv_heads, g, head_size, st);
+  else launch_combine(a, users * kv_heads, g, head_size, st);
   return check_launch("paged_sdpa_decode");
 }
 

@@ -440,7 +440,9 @@ inline bool combine_sliced(const DecodeArgs &a, int segments) { return a.n_waves
 // masked (maximum -inf) where their segment is not: their weights are zeros, not exp2(-inf + inf).
 __device__ __forceinline__ float merge_reference(float m) { return m == -INFINITY ? 0.f : m; }
 
-template <int SLICES>
+// PARKED: the step's cache update is part of the launch, so the rows of users with a negative position are written here.  (A
+// form of its own: with the write as a run-time branch every merge carries its registers, its barrier and its LDS.)
+template <int SLICES, bool PARKED>
 __global__ __launch_bounds__(256) void decode_combine_kernel(DecodeArgs a, int G, int D) {
   constexpr int kElems = kCombinePiece / SLICES;
   const int seg = blockIdx.x;
@@ -457,7 +459,9 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(DecodeArgs a, int G
   uint16_t *out = a.out + u * a.out_us;
   if (nw == 0) {  // padded row: no attended position -> NaN like softmax over nothing
     if (stores) out[(int64_t)(h * G + head_of(i)) * a.out_hs + elem_of(i)] = 0x7fc0;
-    if (a.k_new != nullptr && blockIdx.y == 0) write_negative_position(a, seg, D);
+    if constexpr (PARKED) {
+      if (blockIdx.y == 0) write_negative_position(a, seg, D);
+    }
     return;
   }
   constexpr int kBatch = 8;
@@ -521,11 +525,12 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(DecodeArgs a, int G
   out[(int64_t)(h * G + g) * a.out_hs + elem_of(i)] = (uint16_t)f32_to_bf16_bits(num / den);
 }
 
+template <bool PARKED = false>
 inline void launch_combine(const DecodeArgs &a, int segments, int g, int d, hipStream_t st) {
   if (combine_sliced(a, segments))
-    decode_combine_kernel<kCombineSlices><<<dim3(segments, combine_pieces(g * d, kCombineSlices)), dim3(256), 0, st>>>(a, g, d);
+    decode_combine_kernel<kCombineSlices, PARKED><<<dim3(segments, combine_pieces(g * d, kCombineSlices)), dim3(256), 0, st>>>(a, g, d);
   else
-    decode_combine_kernel<1><<<dim3(segments, combine_pieces(g * d, 1)), dim3(256), 0, st>>>(a, g, d);
+    decode_combine_kernel<1, PARKED><<<dim3(segments, combine_pieces(g * d, 1)), dim3(256), 0, st>>>(a, g, d);
 }
 
 // The same merge over partials whose values are bfloat16 (DecodeArgs::partial_bf16).  They lie in
