@@ -117,3 +117,23 @@ def test_another_stream():
         got = _run(impl, args, True)[2]
     torch.cuda.current_stream().wait_stream(side)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("case,op", [
+    (dict(users=2, s=1, d=128, bs=32, start=40), "paged_update_kv_decode_out_"),
+    (dict(users=1, s=32, d=128, bs=32, start=0), "paged_fill_kv_prefill_out_"),
+    (dict(users=1, s=32, d=128, bs=32, start=64), "chunked_scaled_dot_product_attention_out"),
+])
+def test_a_function_mode_sees_the_operators(case, op):
+    from torch.overrides import TorchFunctionMode
+
+    class Watch(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    impl, (q, k, v, kv, md, out) = _pass(3, **case)
+    seen = []
+    with Watch():
+        impl.forward(None, q, k, v, kv, md, output=out)
+    assert any(op in name for name in seen), seen

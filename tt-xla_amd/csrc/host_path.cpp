@@ -4,13 +4,14 @@
 // through Python views, the operator registry and ctypes it issues in 33 .. 55 us.  This module reads
 // addresses, sizes and strides from the tensors directly and calls the same entry points with the same
 // arguments.  It serves exactly the ordinary form of a pass (plain bfloat16 rows on the current device, the
-// caches' layouts, int32 tables); for anything else it answers None before it has issued anything, and the
+// caches' layouts, int32 tables; nobody watching operators: no dispatch mode, function mode or trace); for anything else it answers None before it has issued anything, and the
 // caller's general path takes the pass, raises what is to be raised and converts what is to be
 // converted.  Scratch comes from the caching allocator on the current stream, call by call: nothing is kept
 // between calls, so streams, threads and graph captures need no care of their own.
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/TracerMode.h>
 #include <ATen/core/grad_mode.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
@@ -83,7 +84,9 @@ PyObject *attention_pass(PyObject *, PyObject *const *v, Py_ssize_t n) {
     PyErr_SetString(PyExc_TypeError, "attention_pass takes 18 arguments");
     return nullptr;
   }
-  if (c10::impl::TorchDispatchModeTLS::any_modes_set() || at::tracer::impl::is_dispatch_enabled()) Py_RETURN_NONE;
+  if (c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled() ||
+      at::tracer::impl::is_dispatch_enabled())
+    Py_RETURN_NONE;
   if (!THPVariable_CheckExact(v[0]) || !THPVariable_Unpack(v[0]).is_cuda()) Py_RETURN_NONE;  // (ahead of any question to the device)
   for (int i = 12; i < 18; ++i)
     if (i == 16 ? !PyFloat_Check(v[i]) : !PyLong_Check(v[i])) Py_RETURN_NONE;
