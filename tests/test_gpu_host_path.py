@@ -57,9 +57,11 @@ def _run(impl, args, native):
     if native:
         assert impl._native_pass(q, k, v, kv, md, out)
     else:
-        keep, impl._native_pass = impl._native_pass, lambda *a: False
-        impl.forward(None, q, k, v, kv, md, output=out)
-        impl._native_pass = keep
+        impl._native_pass = lambda *a: False
+        try:
+            impl.forward(None, q, k, v, kv, md, output=out)
+        finally:
+            del impl._native_pass
     assert _native.host() is not None
     return kv[0], kv[1], out
 
@@ -137,3 +139,31 @@ def test_a_function_mode_sees_the_operators(case, op):
     with Watch():
         impl.forward(None, q, k, v, kv, md, output=out)
     assert any(op in name for name in seen), seen
+
+
+@pytest.mark.parametrize("case,names", [
+    (dict(users=2, s=1, d=128, bs=32, start=40), ["tt::paged_update_kv_decode_out_"]),
+    (dict(users=1, s=32, d=128, bs=32, start=0), ["tt::paged_fill_kv_prefill_out_"]),
+    (dict(users=1, s=32, d=128, bs=32, start=64), ["tt::paged_fill_kv_cache_", "tt::chunked_scaled_dot_product_attention_out"]),
+])
+def test_a_profiler_names_the_operators(case, names):
+    impl, (q, k, v, kv, md, out) = _pass(4, **case)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        assert impl._native_pass(q, k, v, kv, md, out)
+    got = [e.name for e in prof.events()]
+    assert [n for n in got if n.startswith("tt::")] == names
+
+
+@pytest.mark.parametrize("case", [dict(users=2, s=1, d=96, bs=32, start=40), dict(users=1, s=32, d=96, bs=32, start=0),
+                                  dict(users=1, s=32, d=96, bs=32, start=64)])
+def test_an_error_names_the_entry_point(case):
+    """A head size that is not built: refused on the host, in the words of the operators' error."""
+    from tt_xla_amd import _native
+
+    impl, args = _pass(5, **case)
+    said = []
+    for native in (True, False):
+        with pytest.raises(_native.TtpaError) as error:
+            _run(impl, args, native)
+        said.append(str(error.value))
+    assert said[0] == said[1]

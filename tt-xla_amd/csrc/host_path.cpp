@@ -14,6 +14,7 @@
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/TracerMode.h>
 #include <ATen/core/grad_mode.h>
+#include <ATen/record_function.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
@@ -75,9 +76,12 @@ inline at::Tensor scratch(int64_t bytes, const at::Tensor *like) {
   return at::empty({bytes}, like->options().dtype(at::kByte));
 }
 
+PyObject *result(const char *entry, int rc) { return rc == TTPA_OK ? PyLong_FromLong(0) : Py_BuildValue("(si)", entry, rc); }
+
 // attention_pass(query, key, value, k_cache, v_cache, page_table, cache_position, fill_page_table, batch_idx, chunk_start,
 //                sinks, output, users, heads, kv_heads, head_size, scale, window)
-// -> status of the last entry point called, or None: not an ordinary pass, nothing was issued.
+// -> 0, (name, status) of the entry point that failed, or None: not an ordinary pass, nothing was issued.  A profiler
+// sees the names of the operators that the pass stands for.
 PyObject *attention_pass(PyObject *, PyObject *const *v, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (n != 18) {
@@ -130,6 +134,7 @@ PyObject *attention_pass(PyObject *, PyObject *const *v, Py_ssize_t n) {
     }
     const size_t bytes = ttpa_paged_decode_workspace_bytes((int32_t)users, (int32_t)hq, (int32_t)hkv, (int32_t)d);
     if (bytes == 0) Py_RETURN_NONE;
+    RECORD_FUNCTION("tt::paged_update_kv_decode_out_", std::vector<c10::IValue>());
     const at::Tensor ws = scratch((int64_t)bytes, out);
     written(kc), written(vc), written(out);
     const int rc = ttpa_paged_update_decode(
@@ -137,7 +142,7 @@ PyObject *attention_pass(PyObject *, PyObject *const *v, Py_ssize_t n) {
         k->stride(0), d, static_cast<const int32_t *>(pt->data_ptr()), pt->stride(0), pos->data_ptr(), is_i64(pos), (int32_t)users,
         (int32_t)hq, (int32_t)hkv, (int32_t)d, (int32_t)bs, (int32_t)pt->size(1), (int32_t)nb, scale, fmt, (int32_t)window,
         static_cast<const float *>(at_ptr(sinks)), ws.data_ptr(), bytes, stream);
-    return PyLong_FromLong(rc);
+    return result("ttpa_paged_update_decode", rc);
   }
 
   // prefill: fill through the fill table, attention on the fresh K / V or on the cache
@@ -147,13 +152,14 @@ PyObject *attention_pass(PyObject *, PyObject *const *v, Py_ssize_t n) {
   const int32_t *fill_pt = static_cast<const int32_t *>(fill->data_ptr());
   if (v[9] == Py_None) {
     if (bfp8 || s % 32) Py_RETURN_NONE;
+    RECORD_FUNCTION("tt::paged_fill_kv_prefill_out_", std::vector<c10::IValue>());
     written(kc), written(vc), written(out);
     const int rc = ttpa_sdpa_prefill_fill(
         out->data_ptr(), s * hq * d, d, hq * d, q->data_ptr(), s * q->stride(0), d, q->stride(0), k->data_ptr(), val->data_ptr(),
         s * k->stride(0), d, k->stride(0), (int32_t)users, (int32_t)hq, (int32_t)hkv, (int32_t)s, (int32_t)s, (int32_t)d, 1, scale,
         (int32_t)window, kc->data_ptr(), vc->data_ptr(), fill_pt, fill->stride(0), bidx->data_ptr(), is_i64(bidx),
         (int32_t)fill->size(0), (int32_t)bs, (int32_t)fill->size(1), (int32_t)nb, stream);
-    return PyLong_FromLong(rc);
+    return result("ttpa_sdpa_prefill_fill", rc);
   }
   const at::Tensor *pt = p.table(v[5]), *start = p.numbers(v[9], 1);
   if (!pt || pt->size(0) != users || !start || is_i64(start)) Py_RETURN_NONE;
@@ -166,16 +172,21 @@ PyObject *attention_pass(PyObject *, PyObject *const *v, Py_ssize_t n) {
   at::Tensor ws;
   if (bytes) ws = scratch(bytes, out);
   written(kc), written(vc), written(out);
-  int rc = ttpa_paged_fill_cache_kv(kc->data_ptr(), vc->data_ptr(), k->data_ptr(), val->data_ptr(), s * k->stride(0), d, k->stride(0),
-                                    fill_pt, fill->stride(0), bidx->data_ptr(), is_i64(bidx), (int32_t)users, (int32_t)fill->size(0),
-                                    (int32_t)hkv, (int32_t)s, (int32_t)bs, (int32_t)d, (int32_t)fill->size(1), (int32_t)nb, fmt, stream);
-  if (rc == TTPA_OK)
-    rc = ttpa_sdpa_prefill_expanded(
-        out->data_ptr(), s * hq * d, d, hq * d, q->data_ptr(), s * q->stride(0), d, q->stride(0), kc->data_ptr(), vc->data_ptr(), 0, 0,
-        0, static_cast<const int32_t *>(pt->data_ptr()), pt->stride(0), static_cast<const int32_t *>(start->data_ptr()), nullptr, 0, 0,
-        (int32_t)users, (int32_t)hq, (int32_t)hkv, (int32_t)s, (int32_t)(pt->size(1) * bs), (int32_t)d, (int32_t)bs,
-        (int32_t)pt->size(1), (int32_t)nb, 1, scale, 0, fmt, bytes ? ws.data_ptr() : nullptr, bytes, stream);
-  return PyLong_FromLong(rc);
+  {
+    RECORD_FUNCTION("tt::paged_fill_kv_cache_", std::vector<c10::IValue>());
+    const int rc =
+        ttpa_paged_fill_cache_kv(kc->data_ptr(), vc->data_ptr(), k->data_ptr(), val->data_ptr(), s * k->stride(0), d, k->stride(0),
+                                 fill_pt, fill->stride(0), bidx->data_ptr(), is_i64(bidx), (int32_t)users, (int32_t)fill->size(0),
+                                 (int32_t)hkv, (int32_t)s, (int32_t)bs, (int32_t)d, (int32_t)fill->size(1), (int32_t)nb, fmt, stream);
+    if (rc != TTPA_OK) return result("ttpa_paged_fill_cache_kv", rc);
+  }
+  RECORD_FUNCTION("tt::chunked_scaled_dot_product_attention_out", std::vector<c10::IValue>());
+  const int rc = ttpa_sdpa_prefill_expanded(
+      out->data_ptr(), s * hq * d, d, hq * d, q->data_ptr(), s * q->stride(0), d, q->stride(0), kc->data_ptr(), vc->data_ptr(), 0, 0, 0,
+      static_cast<const int32_t *>(pt->data_ptr()), pt->stride(0), static_cast<const int32_t *>(start->data_ptr()), nullptr, 0, 0,
+      (int32_t)users, (int32_t)hq, (int32_t)hkv, (int32_t)s, (int32_t)(pt->size(1) * bs), (int32_t)d, (int32_t)bs,
+      (int32_t)pt->size(1), (int32_t)nb, 1, scale, 0, fmt, bytes ? ws.data_ptr() : nullptr, bytes, stream);
+  return result("ttpa_sdpa_prefill_expanded", rc);
   END_HANDLE_TH_ERRORS
 }
 

@@ -344,7 +344,8 @@ class TTAttentionBackendImpl(_ImplBase):
         )
         if status is None:
             return False
-        _native.check("attention pass", status)
+        if status != 0:
+            _native.check(*status)
         return True
 
     def _output_view(self, output: torch.Tensor, inputs) -> Optional[torch.Tensor]:
