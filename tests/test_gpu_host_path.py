@@ -167,3 +167,46 @@ def test_an_error_names_the_entry_point(case):
             _run(impl, args, native)
         said.append(str(error.value))
     assert said[0] == said[1]
+
+
+def test_other_threads_run_while_a_launch_waits():
+    """Behind a kernel that keeps the GPU busy the queue fills up and a launch waits for room: not with the
+    interpreter lock held.  (The other thread's longest pause is compared with the longest wait of this one.)"""
+    import threading
+    import time
+
+    impl, (q, k, v, kv, md, out) = _pass(6, users=1, s=1, d=64, bs=32, start=30)
+    impl.forward(None, q, k, v, kv, md, output=out)
+    torch.cuda.synchronize()
+    pauses, stop = [], threading.Event()
+
+    def tick():
+        last = time.perf_counter()
+        while not stop.is_set():
+            time.sleep(1e-3)
+            now = time.perf_counter()
+            pauses.append((now - last, last))
+            last = now
+
+    other = threading.Thread(target=tick)
+    other.start()
+    t0 = time.perf_counter()
+    torch.cuda._sleep(10**6)
+    torch.cuda.synchronize()
+    cycles = int(10**6 * min(0.6 / max(time.perf_counter() - t0, 1e-4), 2000))  # about 0.6 s
+    waits, begin = [], time.perf_counter()
+    torch.cuda._sleep(cycles)
+    while time.perf_counter() - begin < 2 and not any(w > 0.03 for w, _ in waits):
+        t0 = time.perf_counter()
+        impl.forward(None, q, k, v, kv, md, output=out)
+        waits.append((time.perf_counter() - t0, t0))
+    stop.set()
+    other.join()
+    torch.cuda.synchronize()
+    wait, t0 = max(waits)
+    print(f"{len(waits)} passes behind {cycles} cycles, longest {wait:.3f} s", flush=True)
+    if wait < 0.03:
+        pytest.skip("no launch had to wait")
+    during = [p for p, at in pauses if at + p > t0 and at < t0 + wait]
+    print(f"longest wait of a pass {wait:.3f} s, pauses of the other thread meanwhile up to {max(during):.3f} s", flush=True)
+    assert max(during) < wait / 2

@@ -72,6 +72,17 @@ inline int is_i64(const at::Tensor *t) { return t && t->scalar_type() == at::kLo
 inline void written(const at::Tensor *t) {
   if (!t->is_inference()) t->unsafeGetTensorImpl()->bump_version();
 }
+// The interpreter lock is not held while scratch is allocated and kernels are launched: either may wait (a launch for a
+// full queue, as long as the GPU takes), and other Python threads run meanwhile, as they do through ctypes.
+class Unlocked {
+ public:
+  Unlocked() : state_(PyEval_SaveThread()) {}
+  ~Unlocked() { PyEval_RestoreThread(state_); }
+  Unlocked(const Unlocked &) = delete;
+
+ private:
+  PyThreadState *state_;
+};
 inline at::Tensor scratch(int64_t bytes, const at::Tensor *like) {
   return at::empty({bytes}, like->options().dtype(at::kByte));
 }
@@ -135,14 +146,17 @@ PyObject *attention_pass(PyObject *, PyObject *const *v, Py_ssize_t n) {
     const size_t bytes = ttpa_paged_decode_workspace_bytes((int32_t)users, (int32_t)hq, (int32_t)hkv, (int32_t)d);
     if (bytes == 0) Py_RETURN_NONE;
     RECORD_FUNCTION("tt::paged_update_kv_decode_out_", std::vector<c10::IValue>());
-    const at::Tensor ws = scratch((int64_t)bytes, out);
     written(kc), written(vc), written(out);
-    const int rc = ttpa_paged_update_decode(
-        out->data_ptr(), hq * d, d, q->data_ptr(), q->stride(0), d, kc->data_ptr(), vc->data_ptr(), k->data_ptr(), val->data_ptr(),
-        k->stride(0), d, static_cast<const int32_t *>(pt->data_ptr()), pt->stride(0), pos->data_ptr(), is_i64(pos), (int32_t)users,
-        (int32_t)hq, (int32_t)hkv, (int32_t)d, (int32_t)bs, (int32_t)pt->size(1), (int32_t)nb, scale, fmt, (int32_t)window,
-        static_cast<const float *>(at_ptr(sinks)), ws.data_ptr(), bytes, stream);
-    return result("ttpa_paged_update_decode", rc);
+    const auto launch = [&] {
+      const Unlocked unlocked;
+      const at::Tensor ws = scratch((int64_t)bytes, out);
+      return ttpa_paged_update_decode(
+          out->data_ptr(), hq * d, d, q->data_ptr(), q->stride(0), d, kc->data_ptr(), vc->data_ptr(), k->data_ptr(), val->data_ptr(),
+          k->stride(0), d, static_cast<const int32_t *>(pt->data_ptr()), pt->stride(0), pos->data_ptr(), is_i64(pos), (int32_t)users,
+          (int32_t)hq, (int32_t)hkv, (int32_t)d, (int32_t)bs, (int32_t)pt->size(1), (int32_t)nb, scale, fmt, (int32_t)window,
+          static_cast<const float *>(at_ptr(sinks)), ws.data_ptr(), bytes, stream);
+    };
+    return result("ttpa_paged_update_decode", launch());
   }
 
   // prefill: fill through the fill table, attention on the fresh K / V or on the cache
@@ -154,12 +168,15 @@ PyObject *attention_pass(PyObject *, PyObject *const *v, Py_ssize_t n) {
     if (bfp8 || s % 32) Py_RETURN_NONE;
     RECORD_FUNCTION("tt::paged_fill_kv_prefill_out_", std::vector<c10::IValue>());
     written(kc), written(vc), written(out);
-    const int rc = ttpa_sdpa_prefill_fill(
-        out->data_ptr(), s * hq * d, d, hq * d, q->data_ptr(), s * q->stride(0), d, q->stride(0), k->data_ptr(), val->data_ptr(),
-        s * k->stride(0), d, k->stride(0), (int32_t)users, (int32_t)hq, (int32_t)hkv, (int32_t)s, (int32_t)s, (int32_t)d, 1, scale,
-        (int32_t)window, kc->data_ptr(), vc->data_ptr(), fill_pt, fill->stride(0), bidx->data_ptr(), is_i64(bidx),
-        (int32_t)fill->size(0), (int32_t)bs, (int32_t)fill->size(1), (int32_t)nb, stream);
-    return result("ttpa_sdpa_prefill_fill", rc);
+    const auto launch = [&] {
+      const Unlocked unlocked;
+      return ttpa_sdpa_prefill_fill(
+          out->data_ptr(), s * hq * d, d, hq * d, q->data_ptr(), s * q->stride(0), d, q->stride(0), k->data_ptr(), val->data_ptr(),
+          s * k->stride(0), d, k->stride(0), (int32_t)users, (int32_t)hq, (int32_t)hkv, (int32_t)s, (int32_t)s, (int32_t)d, 1, scale,
+          (int32_t)window, kc->data_ptr(), vc->data_ptr(), fill_pt, fill->stride(0), bidx->data_ptr(), is_i64(bidx),
+          (int32_t)fill->size(0), (int32_t)bs, (int32_t)fill->size(1), (int32_t)nb, stream);
+    };
+    return result("ttpa_sdpa_prefill_fill", launch());
   }
   const at::Tensor *pt = p.table(v[5]), *start = p.numbers(v[9], 1);
   if (!pt || pt->size(0) != users || !start || is_i64(start)) Py_RETURN_NONE;
@@ -169,24 +186,29 @@ PyObject *attention_pass(PyObject *, PyObject *const *v, Py_ssize_t n) {
                                             (int32_t)pt->size(1), fmt);
     if (bytes < 0 || bytes > kScratchLimit) bytes = 0;
   }
-  at::Tensor ws;
-  if (bytes) ws = scratch(bytes, out);
   written(kc), written(vc), written(out);
   {
     RECORD_FUNCTION("tt::paged_fill_kv_cache_", std::vector<c10::IValue>());
-    const int rc =
-        ttpa_paged_fill_cache_kv(kc->data_ptr(), vc->data_ptr(), k->data_ptr(), val->data_ptr(), s * k->stride(0), d, k->stride(0),
-                                 fill_pt, fill->stride(0), bidx->data_ptr(), is_i64(bidx), (int32_t)users, (int32_t)fill->size(0),
-                                 (int32_t)hkv, (int32_t)s, (int32_t)bs, (int32_t)d, (int32_t)fill->size(1), (int32_t)nb, fmt, stream);
-    if (rc != TTPA_OK) return result("ttpa_paged_fill_cache_kv", rc);
+    const auto launch = [&] {
+      const Unlocked unlocked;
+      return ttpa_paged_fill_cache_kv(
+          kc->data_ptr(), vc->data_ptr(), k->data_ptr(), val->data_ptr(), s * k->stride(0), d, k->stride(0), fill_pt, fill->stride(0),
+          bidx->data_ptr(), is_i64(bidx), (int32_t)users, (int32_t)fill->size(0), (int32_t)hkv, (int32_t)s, (int32_t)bs, (int32_t)d,
+          (int32_t)fill->size(1), (int32_t)nb, fmt, stream);
+    };
+    if (const int rc = launch()) return result("ttpa_paged_fill_cache_kv", rc);
   }
   RECORD_FUNCTION("tt::chunked_scaled_dot_product_attention_out", std::vector<c10::IValue>());
-  const int rc = ttpa_sdpa_prefill_expanded(
-      out->data_ptr(), s * hq * d, d, hq * d, q->data_ptr(), s * q->stride(0), d, q->stride(0), kc->data_ptr(), vc->data_ptr(), 0, 0, 0,
-      static_cast<const int32_t *>(pt->data_ptr()), pt->stride(0), static_cast<const int32_t *>(start->data_ptr()), nullptr, 0, 0,
-      (int32_t)users, (int32_t)hq, (int32_t)hkv, (int32_t)s, (int32_t)(pt->size(1) * bs), (int32_t)d, (int32_t)bs,
-      (int32_t)pt->size(1), (int32_t)nb, 1, scale, 0, fmt, bytes ? ws.data_ptr() : nullptr, bytes, stream);
-  return result("ttpa_sdpa_prefill_expanded", rc);
+  const auto launch = [&] {
+    const Unlocked unlocked;
+    const at::Tensor ws = bytes ? scratch(bytes, out) : at::Tensor();
+    return ttpa_sdpa_prefill_expanded(
+        out->data_ptr(), s * hq * d, d, hq * d, q->data_ptr(), s * q->stride(0), d, q->stride(0), kc->data_ptr(), vc->data_ptr(), 0, 0,
+        0, static_cast<const int32_t *>(pt->data_ptr()), pt->stride(0), static_cast<const int32_t *>(start->data_ptr()), nullptr, 0, 0,
+        (int32_t)users, (int32_t)hq, (int32_t)hkv, (int32_t)s, (int32_t)(pt->size(1) * bs), (int32_t)d, (int32_t)bs,
+        (int32_t)pt->size(1), (int32_t)nb, 1, scale, 0, fmt, bytes ? ws.data_ptr() : nullptr, bytes, stream);
+  };
+  return result("ttpa_sdpa_prefill_expanded", launch());
   END_HANDLE_TH_ERRORS
 }
 
