@@ -211,10 +211,12 @@ class TTMLAAttentionBackendImpl(_ImplBase):
         Not if autograd, a forward-mode derivative or a functional transform may look at one of them: the operators
         that take a pass at once have no derivative, while the products around the attention have."""
         device = tensors[0].device
-        if device.type != "cuda" or not all(t.device == device and t.dtype == torch.bfloat16 for t in tensors):
+        if device.type != "cuda":
             return False
-        if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
-            return False
+        bf16, watched = torch.bfloat16, torch.is_grad_enabled()
+        for t in tensors:  # (a loop: a short prompt is bound by the host)
+            if t.dtype is not bf16 or t.device != device or (watched and t.requires_grad):
+                return False
         return torch.compiler.is_compiling() or (
             torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None)
 

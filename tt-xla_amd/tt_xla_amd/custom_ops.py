@@ -40,8 +40,12 @@ def _ptr(t: Optional[torch.Tensor]) -> int:
 
 def _rows_contiguous(t: torch.Tensor) -> torch.Tensor:
     """Last dim contiguous, every other stride a multiple of 8 elements, 16-byte base."""
-    if t.stride(-1) != 1 or t.data_ptr() % 16 or any(s % 8 for s in t.stride()[:-1]):
+    strides = t.stride()
+    if strides[-1] != 1 or t.data_ptr() % 16:
         return t.contiguous()
+    for s in strides[:-1]:
+        if s % 8:
+            return t.contiguous()
     return t
 
 
@@ -348,9 +352,11 @@ def _check_out(out, shape, name):
 
 def _storable(out):
     """``out`` if the kernels' vector stores can write it, else a fresh tensor of its shape, for the caller to copy back."""
-    if out.stride(-1) != 1 or out.data_ptr() % 16 or any(st % 4 for st in out.stride()[:-1]):
-        return torch.empty(out.shape, dtype=out.dtype, device=out.device)
-    return out
+    strides = out.stride()
+    storable = strides[-1] == 1 and out.data_ptr() % 16 == 0
+    for s in strides[:-1]:
+        storable = storable and s % 4 == 0
+    return out if storable else torch.empty(out.shape, dtype=out.dtype, device=out.device)
 
 
 def _decode(query, key, value, page_table, is_causal, attn_mask, cur_pos_tensor, attention_sink, scale,
@@ -1082,11 +1088,10 @@ def flash_mla_prefill(
 
 def _split_key_prefill(q_nope, q_rope, k_nope, k_rope, value, out, scale):
     """q_nope [b, heads, s, 128], q_rope [b, heads, s, 64], k_nope [b, kv heads, s, 128], k_rope
-    [b, kv heads or 1, s, 64], value / out [b, kv heads / heads, s, 128], by strides."""
+    [b, kv heads or 1, s, 64], value / out [b, kv heads / heads, s, 128], by strides; out storable."""
     b, hq, s, _ = q_nope.shape
     hkv = k_nope.shape[1]
     q_nope, q_rope, k_nope, k_rope, value = map(_rows_contiguous, (q_nope, q_rope, k_nope, k_rope, value))
-    _check_out(out, (b, hq, s, 128), "split-key prefill")
     N.call(
         "ttpa_split_key_prefill",
         out.data_ptr(), out.stride(0), out.stride(1), out.stride(2),
