@@ -96,3 +96,13 @@ def test_backend_prompt_forms_agree(n, users, s):
         got.append((out.float(), cache))
     assert torch.equal(got[0][1], got[1][1])
     torch.testing.assert_close(got[0][0], got[1][0], atol=2e-2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("dh", [192, 128])  # the split-key kernel's shape, and one of the decode kernels'
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32, torch.uint8])
+def test_value_of_another_type_is_refused(dh, dtype):
+    """The kernels read V as bfloat16: another type's bits would be taken for numbers, a one-byte V read past its end."""
+    g = torch.Generator().manual_seed(1)
+    q, k = _bf(g, 1, 2, 32, dh).cuda(), _bf(g, 1, 2, 32, dh).cuda()
+    with pytest.raises(ValueError, match="bfloat16"):
+        torch.ops.tt.flash_mla_prefill(q, k, 128, torch.zeros(1, 2, 32, 128, dtype=dtype, device="cuda"))

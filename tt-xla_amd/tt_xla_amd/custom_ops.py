@@ -1029,8 +1029,8 @@ def flash_mla_prefill(
         assert attn_mask.shape[0] == query.shape[0], "attention mask batch size must match query batch size."
     else:
         assert is_causal == True, "is_causal must be True if attn_mask is not provided"  # noqa: E712
-    if query.dtype != torch.bfloat16 or key.dtype != torch.bfloat16:
-        raise ValueError("query and key must be bfloat16")
+    if query.dtype != torch.bfloat16 or key.dtype != torch.bfloat16 or (value is not None and value.dtype != torch.bfloat16):
+        raise ValueError("query, key and value must be bfloat16")
     b, hq, s, dh = query.shape
     if scale is None:
         scale = 1.0 / math.sqrt(dh)
