@@ -51,15 +51,18 @@ def test_shared_rotary_part_and_strides():
     torch.testing.assert_close(out.cpu().transpose(1, 2).float(), want.float(), atol=2e-2, rtol=2e-2)
 
 
-@pytest.mark.parametrize("users,s,bs,lat,rope", [(1, 1, 16, 512, 64), (3, 77, 32, 512, 64), (2, 130, 64, 64, 8)])
-def test_two_part_fill(users, s, bs, lat, rope):
+@pytest.mark.parametrize("users,s,bs,lat,rope,aligned", [
+    (1, 1, 16, 512, 64, True), (3, 77, 32, 512, 64, True), (2, 130, 64, 64, 8, True),
+    (3, 77, 32, 512, 64, False), (2, 33, 16, 60, 12, True),  # what does not come in 16-byte pieces
+])
+def test_two_part_fill(users, s, bs, lat, rope, aligned):
     g = torch.Generator().manual_seed(users + s)
     w = -(-s // bs) + 1
     nb = users * w + 2
     table = (torch.randperm(nb, generator=g)[: users * w]).view(users, w).to(torch.int32)
     table[0, 0] = nb + 5  # out of range: skipped
     cache, latent, rotary = _bf(g, nb, 1, bs, lat + rope), _bf(g, users, s, lat), _bf(g, users, s, rope)
-    dev = cache.cuda()
+    dev = cache.cuda() if aligned else torch.zeros(cache.numel() + 1, dtype=cache.dtype, device="cuda")[1:].view(cache.shape).copy_(cache)
     torch.ops.tt.paged_fill_latent_cache_(dev, latent.cuda(), rotary.cuda(), table.cuda())
     rows = torch.cat([latent, rotary], -1)
     for u in range(users):

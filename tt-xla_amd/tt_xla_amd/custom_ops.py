@@ -1214,6 +1214,10 @@ def paged_fill_latent_cache_(cache: torch.Tensor, latent: torch.Tensor, rope: to
         raise ValueError("fill_value dtype must match the cache")
     if page_table.dim() != 2 or s > page_table.shape[1] * bs:
         raise ValueError(f"{s} tokens do not fit a page table of shape {tuple(page_table.shape)}")
+    if cache.data_ptr() % 16 or lat % 8 or d % 8:  # not in 16-byte pieces: rows in one part, element by element
+        rows = torch.cat([latent, rope], -1).unsqueeze(1)
+        _fill_inplace(cache, rows, page_table, torch.arange(users, dtype=torch.int32, device=cache.device))
+        return
     latent, rope, pt = _rows_contiguous(latent), _rows_contiguous(rope), _table(page_table)
     N.call(
         "ttpa_paged_fill_latent",
