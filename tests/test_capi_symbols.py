@@ -104,3 +104,16 @@ def test_latent_decode_refuses_more_segments_than_the_grid_has_threads(native, m
     rc = lib.ttpa_paged_mla_decode(256, 8 * d, d, 256, 8 * d, d, 256, None, 256, 1, 256, 0, users, hq, hkv, d, d,
                                    32, 1, 4, 1.0, None, 256, need, None)
     assert rc == native.ERR_UNSUPPORTED and b"segments" in lib.ttpa_last_error()
+
+
+@pytest.mark.parametrize("missing", ["LIB_PATH", "HOST_PATH"])
+def test_a_missing_library_is_built(native, missing, monkeypatch, tmp_path):
+    """Every ordinary forward needs both: the kernels and the eager host path."""
+    built = []
+    monkeypatch.setattr(entry, "build", lambda: built.append(missing))
+    entry.ensure_built()
+    assert not built
+    monkeypatch.setattr(native, missing, str(tmp_path / "none.so"))
+    entry.ensure_built()
+    assert built == [missing]
+    assert hasattr(native.host(), "attention_pass")
