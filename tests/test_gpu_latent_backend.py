@@ -103,3 +103,18 @@ def test_weights_of_any_other_layout():
     spread = lambda t: torch.stack([t, t], -1)[..., 0]  # noqa: E731  (no dimension contiguous)
     got, _ = _run(impl, p, layer=types.SimpleNamespace(W_UK_T=spread(p.layer.W_UK_T), W_UV=spread(p.layer.W_UV)))
     assert torch.equal(got, want)
+
+
+def test_every_token_of_a_step_is_written_before_any_is_attended():
+    """More users than one launch takes; rows of one sequence far apart in the batch (drafted tokens): user 0, in the
+    first launch, attends the token that the last user, in the second one, writes in the same step.  Against the operators
+    in turn, within the bfloat16 roundings of their intermediates."""
+    n, users = 16, 1100
+    p = _pass(11, n, users, 1, bs=32, ctx=20)
+    p.meta.page_table[0] = p.meta.page_table[users - 1]
+    p.meta.cache_position[users - 1], p.meta.cache_position[0] = 2, 3
+    p.kv_c[users - 1] *= 8
+    got, cache = _run(_impl(n), p)
+    want, want_cache = _run(_impl(n, functional_cache_ops=True), p)
+    assert torch.equal(cache, want_cache)
+    torch.testing.assert_close(got.float(), want.float(), atol=2e-2, rtol=2e-2)

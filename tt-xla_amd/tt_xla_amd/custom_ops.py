@@ -1182,6 +1182,9 @@ def latent_decode_step_(
     w_uk_t, w_uv = _weight(w_uk_t), _weight(w_uv)
     target = _storable(out)
     pt, cur = _table(page_table), _index_tensor(cur_pos_tensor)
+    if users > _MLA_MAX_USERS:
+        # several calls, each of which writes its users' tokens: the first one's users see the last one's tokens too
+        _update_inplace(cache, torch.cat([latent, rope], -1).view(1, users, 1, row), cur, pt)
     for u0 in range(0, users, _MLA_MAX_USERS):
         n = min(_MLA_MAX_USERS, users - u0)
         ws_bytes = N.lib().ttpa_latent_decode_step_workspace_bytes(n, heads)
