@@ -1,5 +1,6 @@
 """The latent backend's passes in the forms that its own operators take or leave: weights in every layout, outputs that are not
-aligned.  Compared with the same pass in its ordinary form, bit for bit."""
+aligned, other streams and graphs, compared with the same pass in its ordinary form bit for bit; and the
+ordinary form against 64 bits."""
 
 import math
 import types
@@ -118,3 +119,63 @@ def test_every_token_of_a_step_is_written_before_any_is_attended():
     want, want_cache = _run(_impl(n, functional_cache_ops=True), p)
     assert torch.equal(cache, want_cache)
     torch.testing.assert_close(got.float(), want.float(), atol=2e-2, rtol=2e-2)
+
+
+def _in_64_bits(p, n, s):
+    """The output of a pass, [tokens, heads, 128]; the cache holds the step's tokens."""
+    f = lambda t: t.double()  # noqa: E731
+    users = p.meta.cache_position.shape[0]
+    qn, qr, uk, uv = f(p.q[0]), f(p.q[1]), f(p.layer.W_UK_T), f(p.layer.W_UV)
+    out = torch.empty(users * s, n, 128, dtype=torch.float64, device="cuda")
+    for u in range(users):
+        if s == 1:
+            t = int(p.meta.cache_position[u]) + 1
+            rows = f(p.cache[p.meta.page_table[u].long()].reshape(-1, 576)[:t])
+        else:
+            t, rows = s, torch.cat([f(p.kv_c), f(p.k_pe[:, 0])], 1)[u * s : (u + 1) * s]
+        mine = slice(u * s, (u + 1) * s)
+        seen = torch.arange(t, device="cuda")[None] <= torch.arange(s, device="cuda")[:, None] + t - s
+        for h in range(n):
+            scores = (qn[mine, h] @ uk[h] @ rows[:, :512].T + qr[mine, h] @ rows[:, 512:].T) * 192**-0.5
+            out[mine, h] = torch.softmax(scores.masked_fill(~seen, float("-inf")), -1) @ rows[:, :512] @ uv[h]
+    return out
+
+
+@pytest.mark.parametrize("n,users,s", [(16, 33, 1), (128, 3, 1), (3, 2, 96), (16, 1, 256)])
+def test_against_64_bits(n, users, s):
+    """Four values on the way to an output element are rounded to bfloat16 (step: absorbed query, probability, latent
+    output, output; prompt: K, probability, V, output), each within 2^-9 of itself."""
+    p = _pass(n + s, n, users, s, ctx=300)
+    got, _ = _run(_impl(n), p, cache=p.cache)
+    want = _in_64_bits(p, n, s)
+    rel = ((got.view(want.shape).double() - want).norm() / want.norm()).item()
+    print(f"latent heads{n} users{users} tokens{s}: relative error {rel:.2e}", flush=True)
+    assert rel < 4 * 2**-9
+
+
+@pytest.mark.parametrize("n,users,s", [(16, 5, 1), (128, 2, 1), (16, 2, 64)])
+def test_another_stream_and_replays(n, users, s):
+    p, impl = _pass(n + users, n, users, s), _impl(n)
+    want, want_cache = _run(impl, p)
+    out, cache = torch.zeros_like(want), p.cache.clone()
+
+    def check():
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and torch.equal(cache, want_cache)
+        out.zero_()
+        cache.copy_(p.cache)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        _run(impl, p, out=out, cache=cache)
+    torch.cuda.current_stream().wait_stream(side)
+    check()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        _run(impl, p, out=out, cache=cache)
+    for i in range(4):
+        graph.replay()
+        check()
+        _run(impl, _pass(i, n, users + 1, s))  # the program's own work in between
+        torch.cuda.synchronize()

@@ -140,3 +140,34 @@ def test_several_row_blocks_per_workgroup_are_not_split(users, hq, hkv, nbpu, st
     walked = torch.ops.tt.chunked_scaled_dot_product_attention(*args, 128**-0.5)
     assert not torch.equal(split, whole)  # (what the next line would not tell from a split)
     assert torch.equal(walked, whole)
+
+
+@pytest.mark.parametrize("bs,bfp8", [(32, False), (64, False), (32, True)])
+def test_parts_on_another_stream_and_replayed(bs, bfp8):
+    """A chunk that is split over the keys: its partial results are scratch of the stream's, or of the graph's own."""
+    from tt_xla_amd import custom_ops as ops
+
+    g = torch.Generator().manual_seed(bs)
+    key, value, table = P._paged(g, 1, 2048 // bs, 2, bs, 128, False)
+    kv = [ops.bfp8_pack_cache(t.cuda()) if bfp8 else t.cuda() for t in (key, value)]
+    args = (P._bf(g, 1, 8, 96, 128).cuda(), *kv, table.cuda(), torch.tensor([1500], dtype=torch.int32, device="cuda"))
+    other = (P._bf(g, 1, 8, 160, 128).cuda(),) + args[1:]
+    run = lambda a=args: torch.ops.tt.chunked_scaled_dot_product_attention(*a, 128**-0.5)  # noqa: E731
+    want = run()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        got = run()
+    run(other)
+    torch.cuda.current_stream().wait_stream(side)
+    assert torch.equal(got, want)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = run()
+    for _ in range(4):
+        got.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+        run(other)
+        torch.cuda.synchronize()
