@@ -210,3 +210,10 @@ def test_other_threads_run_while_a_launch_waits():
     during = [p for p, at in pauses if at + p > t0 and at < t0 + wait]
     print(f"longest wait of a pass {wait:.3f} s, pauses of the other thread meanwhile up to {max(during):.3f} s", flush=True)
     assert max(during) < wait / 2
+
+
+def test_a_window_that_is_no_64_bit_number_is_the_operators_to_refuse():
+    impl, (q, k, v, kv, md, out) = _pass(7, users=2, s=1, d=128, bs=32, start=40, window=2**70)
+    assert not impl._native_pass(q, k, v, kv, md, out)
+    with pytest.raises((RuntimeError, OverflowError)):
+        impl.forward(None, q, k, v, kv, md, output=out)

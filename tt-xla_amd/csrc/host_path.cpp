@@ -108,6 +108,10 @@ PyObject *attention_pass(PyObject *, PyObject *const *v, Py_ssize_t n) {
   const int64_t users = PyLong_AsLongLong(v[12]), hq = PyLong_AsLongLong(v[13]), hkv = PyLong_AsLongLong(v[14]);
   const int64_t d = PyLong_AsLongLong(v[15]), window = PyLong_AsLongLong(v[17]);
   const float scale = (float)PyFloat_AsDouble(v[16]);
+  if (PyErr_Occurred()) {  // a number that does not fit 64 bits
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
   if (users <= 0 || hq <= 0 || hkv <= 0 || d <= 0 || d % 8 || hq % hkv || window < 0) Py_RETURN_NONE;
 
   const Pass p{(int)c10::hip::current_device(), at::GradMode::is_enabled()};
