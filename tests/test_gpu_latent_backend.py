@@ -57,7 +57,7 @@ def _run(impl, p, out=None, layer=None, cache=None):
     return out, cache
 
 
-@pytest.mark.parametrize("s", [1, 32])
+@pytest.mark.parametrize("s", [1, 32, 96])
 def test_output_that_is_not_aligned(s):
     p, impl = _pass(s, 16, 3, s), _impl(16)
     want, want_cache = _run(impl, p)
@@ -141,7 +141,7 @@ def _in_64_bits(p, n, s):
     return out
 
 
-@pytest.mark.parametrize("n,users,s", [(16, 33, 1), (128, 3, 1), (3, 2, 96), (16, 1, 256)])
+@pytest.mark.parametrize("n,users,s", [(16, 33, 1), (128, 3, 1), (3, 2, 64), (3, 2, 96), (16, 1, 256)])
 def test_against_64_bits(n, users, s):
     """Four values on the way to an output element are rounded to bfloat16 (step: absorbed query, probability, latent
     output, output; prompt: K, probability, V, output), each within 2^-9 of itself."""
@@ -153,7 +153,22 @@ def test_against_64_bits(n, users, s):
     assert rel < 4 * 2**-9
 
 
-@pytest.mark.parametrize("n,users,s", [(16, 5, 1), (128, 2, 1), (16, 2, 64)])
+@pytest.mark.parametrize("users,s", [(1, 32), (3, 32), (1, 64), (2, 96), (1, 256)])
+def test_prompts_are_as_close_to_64_bits_as_the_operators_in_turn(users, s):
+    """Whichever way the products are grouped.  (Expanded, prompts of 32 and 64 tokens were 0.5 - 0.7 % further off, longer
+    ones are closer.  The mean of these inputs' errors has a spread of 0.2 % where the two sides round differently.)"""
+    n, err = 16, [0.0, 0.0]
+    for seed in range(24 if s <= 64 else 8):
+        p = _pass(seed, n, users, s)
+        for i, functional in enumerate((True, False)):
+            got, _ = _run(_impl(n, functional_cache_ops=functional), p)
+            want = _in_64_bits(p, n, s)
+            err[i] += ((got.view(want.shape).double() - want).norm() / want.norm()).item()
+    print(f"latent users{users} tokens{s}: ratio of the errors {err[1] / err[0]:.4f}", flush=True)
+    assert err[1] < 1.002 * err[0]
+
+
+@pytest.mark.parametrize("n,users,s", [(16, 5, 1), (128, 2, 1), (16, 2, 64), (16, 2, 96)])
 def test_another_stream_and_replays(n, users, s):
     p, impl = _pass(n + users, n, users, s), _impl(n)
     want, want_cache = _run(impl, p)

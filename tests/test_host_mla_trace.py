@@ -31,7 +31,9 @@ def _forward(users, s, n=16, nope=128, rope=64, lat=512, vd=128, **kw):
     return forward, layer, (new(t, n, nope), new(t, n, rope), new(t, lat), new(t, 1, rope), new(t, n * vd))
 
 
-@pytest.mark.parametrize("s,ops", [(1, ["tt.latent_decode_step_"]), (64, ["tt.split_key_prefill_out", "tt.paged_fill_latent_cache_"])])
+@pytest.mark.parametrize("s,ops", [
+    (1, ["tt.latent_decode_step_"]), (64, ["tt.flash_mla_prefill", "tt.paged_fill_latent_cache_"]),
+    (96, ["tt.split_key_prefill_out", "tt.paged_fill_latent_cache_"])])
 def test_one_graph(s, ops):
     seen = []
 
@@ -46,7 +48,7 @@ def test_one_graph(s, ops):
     assert seen == [ops]
 
 
-@pytest.mark.parametrize("s", [1, 64])
+@pytest.mark.parametrize("s", [1, 64, 96])
 def test_one_graph_of_operators(s):
     with FakeTensorMode():
         forward, _, args = _forward(2, s, nope=64)
@@ -54,7 +56,7 @@ def test_one_graph_of_operators(s):
         torch.compile(forward, fullgraph=True, backend="eager")(*args)
 
 
-@pytest.mark.parametrize("s", [1, 64])
+@pytest.mark.parametrize("s", [1, 64, 96])
 def test_output_depends_on_the_weights(s):
     with FakeTensorMode():
         forward, layer, args = _forward(2, s)
@@ -64,7 +66,7 @@ def test_output_depends_on_the_weights(s):
             assert not forward(*args[:4], torch.empty_like(args[4])).requires_grad
 
 
-@pytest.mark.parametrize("s", [1, 64])
+@pytest.mark.parametrize("s", [1, 64, 96])
 def test_forward_mode_and_vmap(s):
     fw = torch.autograd.forward_ad
     with FakeTensorMode():
@@ -81,7 +83,7 @@ def test_forward_mode_and_vmap(s):
         assert torch.vmap(one)(torch.stack([plain] * 3), torch.stack([args[4]] * 3)).shape == (3,) + args[4].shape
 
 
-@pytest.mark.parametrize("s", [1, 64])
+@pytest.mark.parametrize("s", [1, 64, 96])
 def test_scale_of_the_operators(s):
     """Without a scale of its own the layer uses the operators' default."""
     with FakeTensorMode():

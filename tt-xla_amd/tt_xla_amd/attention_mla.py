@@ -18,10 +18,10 @@ What a forward pass does, in the order of the reference:
      (:379-389), then ``tt::paged_flash_mla_decode`` attends over the paged cache (:394-405);
   3. expand the latent output with ``W_UV`` and write ``[tokens, N * v_head_dim]`` (:322-335,
      :408-422).
-Differences from the reference, invisible in results: a causal prompt pass at the head shape
-128 + 64 / 128 expands K and V per head instead of absorbing the query (``_expands_prompts``: the same
-sums with the products grouped the other way; four prompts of 2048 tokens, 16 heads: 763 -> 164 us, and
-the error against a 64-bit evaluation stays at 3.4e-3 of the output); a causal decode pass at that shape and a
+Differences from the reference, invisible in results: a causal prompt pass of more than 64 tokens at the
+head shape 128 + 64 / 128 expands K and V per head instead of absorbing the query (``_expands_prompts``: the
+same sums with the products grouped the other way; four prompts of 2048 tokens, 16 heads: 763 -> 164 us, and
+the error against a 64-bit evaluation is 3.37e-3 of the output where the absorbed form's is 3.45e-3); a causal decode pass at that shape and a
 latent width of 512 is one operator (``tt::latent_decode_step_``: the same steps and roundings without the
 copies between them; 128 users, 16 heads: 168 -> 94 us); the cache writes use the in-place
 operators (one batched fill instead of a per-user loop over functional fills followed by a
@@ -166,7 +166,8 @@ class TTMLAAttentionBackendImpl(_ImplBase):
         n, lat, rope, nope = self.num_heads, self.kv_lora_rank, self.qk_rope_head_dim, self.qk_nope_head_dim
 
         if prefill and self._expands_prompts(q_nope, q_pe, kv_c_normed, k_pe, kv_cache, attn_metadata, layer, s, output):
-            self._forward_prefill_expanded(q_nope, q_pe, kv_c_normed, k_pe, kv_cache, attn_metadata, layer, s, users, output)
+            form = self._forward_prefill_short if s <= 64 else self._forward_prefill_expanded
+            form(q_nope, q_pe, kv_c_normed, k_pe, kv_cache, attn_metadata, layer, s, users, output)
             return
 
         if not prefill and self._steps_at_once(q_nope, q_pe, kv_c_normed, k_pe, kv_cache, attn_metadata, layer, output):
@@ -247,6 +248,23 @@ class TTMLAAttentionBackendImpl(_ImplBase):
         if attn_metadata is not None and self._has_cache(kv_cache) and kv_cache.dtype != torch.bfloat16:
             return False
         return output.is_contiguous()  # (its address is the operator's business: a traced tensor has none)
+
+    def _forward_prefill_short(self, q_nope, q_pe, kv_c_normed, k_pe, kv_cache, attn_metadata, layer, s, users, output):
+        """A prompt of up to 64 tokens in the absorbed form: its error against a 64-bit evaluation is smaller there (a latent
+        output of few keys is rounded less than each of their values; 16 heads, 32 / 64 / 96 / 160 tokens: 2.851e-3 / 2.975e-3 /
+        3.062e-3 / 3.155e-3 against 2.871e-3 / 2.993e-3 / 3.056e-3 / 3.140e-3 expanded), and so short a pass is bound by
+        the host: the steps of the operators in turn in fewer calls, one prompt of 32 tokens 165 -> 112 us (100 expanded)."""
+        n, lat, rope = self.num_heads, self.kv_lora_rank, self.qk_rope_head_dim
+        rows = lambda w: w if w.stride(-1) == 1 else w.contiguous()  # noqa: E731  (no batched product with a transposed right operand)
+        latent, rotary = kv_c_normed.view(users, s, lat), k_pe.view(users, s, rope)
+        heads = lambda t, width: t.view(users * s, n, width).transpose(0, 1)  # noqa: E731
+        q_abs = torch.bmm(heads(q_nope, self.qk_nope_head_dim), rows(layer.W_UK_T))             # [N, tokens, L]
+        q_lat = torch.cat([q_abs, heads(q_pe, rope)], -1).view(n, users, s, lat + rope).transpose(0, 1)
+        out_lat = _ops.flash_mla_prefill(query=q_lat, key=torch.cat([latent, rotary], -1).unsqueeze(1), head_dim_v=lat, scale=self.scale)
+        out = torch.bmm(out_lat.transpose(0, 1).reshape(n, users * s, lat), rows(layer.W_UV))   # [N, tokens, V]
+        heads(output, self.v_head_dim).copy_(out)
+        if attn_metadata is not None and self._has_cache(kv_cache):
+            torch.ops.tt.paged_fill_latent_cache_(kv_cache, latent, rotary, attn_metadata.fill_page_table)
 
     def _forward_prefill_expanded(self, q_nope, q_pe, kv_c_normed, k_pe, kv_cache, attn_metadata, layer, s, users, output):
         n, lat, rope, nope, vd = self.num_heads, self.kv_lora_rank, self.qk_rope_head_dim, self.qk_nope_head_dim, self.v_head_dim
