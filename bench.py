@@ -37,7 +37,7 @@ for _p in (ROOT, os.path.join(ROOT, "tt-xla_amd")):
 HBM_PEAK_GBPS = 8000.0      # MI355X published HBM3E bandwidth
 MFMA_BF16_PEAK_TFLOPS = 2500.0  # MI355X published dense bf16 MFMA rate
 # HBM bytes per launch of the dominant kernel, from rocprofv3 FETCH_SIZE / WRITE_SIZE counter runs
-# of this script scaled by a plain copy of known size (profiles/*_hbm_traffic_*.md).  A counter run
+# of this script scaled by a plain copy of known size (profiles/hbm_traffic_all_workloads.md).  A counter run
 # cannot share a process with the timed run, so the figures are carried here, each with the hash
 # of the kernel sources it was measured on (the first 16 hex digits of the SHA-256 over the files
 # listed): when the sources have changed since, `roofline.traffic` is null instead of stale.
@@ -52,13 +52,13 @@ MEASURED_TRAFFIC = {
     # workload: (kernel, hash of its sources, HBM bytes per launch: FETCH_SIZE and WRITE_SIZE of the
     # kernel, each scaled by what the same counter reads for a plain copy of known size, mean over
     # the rotating workload copies; the summaries under profiles/ hold the runs)
-    "config2": ("paged_decode_mfma16_kernel", "8ba1b647faebb44c", 310422335),
-    "config5": ("paged_decode_mfma16_kernel", "8ba1b647faebb44c", 168457090),
-    "config4": ("paged_decode_mfma16_kernel", "8ba1b647faebb44c", 3415575936),
-    "config3": ("prefill_stream_kernel", "9e5dc9fce6518e7f", 244468287),
-    "latent": ("paged_decode_latent16_kernel", "cb2ca9fa245030d1", 654198293),
-    "latent128": ("paged_decode_latent128_kernel", "b26a62d6c1d0a108", 739381753),
-    "latent-prefill": ("latent_prefill_kernel", "b26a62d6c1d0a108", 332193335),
+    "config2": ("paged_decode_mfma16_kernel", "410306992a9b7e9b", 310401868),
+    "config5": ("paged_decode_mfma16_kernel", "410306992a9b7e9b", 168429482),
+    "config4": ("paged_decode_mfma16_kernel", "410306992a9b7e9b", 3415531104),
+    "config3": ("prefill_stream_kernel", "d622c3aa465eb385", 244949812),
+    "latent": ("paged_decode_latent16_kernel", "611a48caa3e35aca", 654199369),
+    "latent128": ("paged_decode_latent128_kernel", "75ff2b818e7d1cd4", 739359975),
+    "latent-prefill": ("latent_prefill_kernel", "75ff2b818e7d1cd4", 332250064),
 }
 DECODE_KERNEL_NAME = {"config2": "paged_decode_mfma16_kernel", "config4": "paged_decode_mfma16_kernel",
                       "config5": "paged_decode_mfma16_kernel"}
