@@ -105,7 +105,9 @@ __global__ __launch_bounds__(256) void latent_query_kernel(StepArgs a) {
       *reinterpret_cast<uint4 *>(a.q_lat + ((int64_t)v * a.heads + head) * kRow + kLatent + c) =
           *reinterpret_cast<const uint4 *>(a.q_rope + v * a.qr_us + head * a.qr_hs + c);
   }
-  if (head == 0) {  // the new token's row: 128 latent columns per workgroup, the rotary part with the first
+  // The new token's row: 128 latent columns per workgroup, the rotary part with the first.  (Parked users that share a
+  // slot of the null block write it in any order.)
+  if (head == 0) {
     const int chunks = 16 + (blockIdx.x == 0 ? 8 : 0);
     for (int i = tid; i < kUsers * chunks; i += 256) {
       const int v = u0 + i / chunks, c = i % chunks;
