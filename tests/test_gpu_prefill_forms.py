@@ -121,7 +121,7 @@ def test_chunk_that_starts_outside_the_sequence(hq, hkv, bs, bfp8, start, lc, sl
         P._check(f"h{hq}x{hkv} bs{bs} start{start}", got[:, :, blind:].contiguous(), want)
 
 
-@pytest.mark.parametrize("users,hq,hkv,nbpu,start,lc", [(2, 32, 8, 8, 256, 256), (2, 64, 8, 6, 192, 192), (1, 16, 4, 9, 293, 200)])
+@pytest.mark.parametrize("users,hq,hkv,nbpu,start,lc", [(1, 32, 8, 17, 960, 128), (1, 64, 8, 17, 900, 96), (1, 16, 4, 9, 330, 200)])
 @pytest.mark.parametrize("slots", ["2", "3"])
 def test_several_row_blocks_per_workgroup_are_not_split(users, hq, hkv, nbpu, start, lc, slots, monkeypatch):
     """TTPA_PREFILL_WGS_PER_GROUP has a workgroup walk its row blocks over all of their keys, also where the launch would
@@ -171,3 +171,31 @@ def test_parts_on_another_stream_and_replayed(bs, bfp8):
         assert torch.equal(got, want)
         run(other)
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("users,hq,hkv,lc,blocks", [
+    # 32-key blocks from which on the last row block is split: 16, or 7 / 16 of the workgroups of the launch, or (above half of
+    # the 256 CUs) half of them
+    (1, 8, 2, 32, 16), (2, 2, 2, 40, 16), (1, 4, 2, 64, 16), (4, 32, 8, 64, 28), (1, 64, 8, 256, 56), (1, 64, 8, 288, 72),
+    (1, 64, 8, 512, 128),
+])
+@pytest.mark.parametrize("bs", [32, 64])
+def test_where_the_split_begins(users, hq, hkv, lc, blocks, bs, monkeypatch):
+    """Under a page table far wider than the pass, one block in front of the line every row comes out of the same
+    operations as without scratch to split with, bit for bit; on the line not, but within the roundings of the parts."""
+    from tt_xla_amd import custom_ops as ops
+
+    g = torch.Generator().manual_seed(hq + lc + bs)
+    width = 32 * blocks // bs + 200
+    key, value, _ = P._paged(g, 1, 64, hkv, bs, 128, False)
+    table = torch.randint(0, 65, (users, width), generator=g).to(torch.int32).cuda()
+    q, key, value = P._bf(g, users, hq, lc, 128).cuda(), key.cuda(), value.cuda()
+    for n in (blocks - 1, blocks):
+        start = torch.tensor([32 * n - lc], dtype=torch.int32, device="cuda")
+        args = (q, key, value, table, start, 128**-0.5)
+        got = torch.ops.tt.chunked_scaled_dot_product_attention(*args)
+        with monkeypatch.context() as m:
+            m.setattr(ops, "_EXPANSION_LIMIT", 0)
+            whole = torch.ops.tt.chunked_scaled_dot_product_attention(*args)
+        assert torch.equal(got, whole) == (n < blocks)
+        torch.testing.assert_close(got.float(), whole.float(), atol=2e-2, rtol=2e-2)

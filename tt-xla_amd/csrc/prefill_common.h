@@ -60,7 +60,9 @@ struct PrefillArgs {
   // ... and, paged, several workgroups per row block, each with a part of the keys (scratch from the caller or null)
   float *part_acc;
   int64_t part_bytes;
-  int parts;
+  int parts, parts_one;  // shares of the keys at most; with one workgroup per CU
+  int split_from;        // launches whose last row block has fewer 32-key blocks are not split
+  int part_stride;       // workgroups per part
 };
 
 // key / block_size without a division instruction sequence (about 30 instructions each, and the

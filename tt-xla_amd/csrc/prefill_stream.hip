@@ -200,16 +200,35 @@ __device__ __forceinline__ void stream_items_paged32(StreamRequests &r, StreamIt
 }
 
 // ---- splitting over the keys --------------------------------------------------------------------
-// A part is at least this many 32-key blocks: below it a workgroup's start and its float accumulators
-// cost more than the matrix work that they spread.
-constexpr int kMinPartBlocks = 8;
+// Splitting costs a second launch (1.4 us, also where the kernel then does not split), the start of more
+// workgroups, and 64 KiB of float accumulators written and read per part and workgroup; it saves about 0.48 us per
+// 32-key block that a workgroup need not walk.  How many blocks there are is in device memory (the host sees the
+// page table's width), so the host launches the most parts that may be wanted and the kernel decides, as does the
+// merge kernel with the same function.  Attention of a pass in us, unsplit / split, by workgroups of the unsplit launch:
+//    8 (32 rows, 32 / 8 heads):   10 blocks 12.8 / 13.6, 16 blocks 15.9 / 13.7, 64 blocks 38.9 / 16.1
+//   32 (128 rows, 32 / 8 heads):  10 blocks 12.9 / 14.7, 16 blocks 16.0 / 15.2, 64 blocks 39.4 / 23.8
+//   64 (4 x 64 rows, 32 / 8):     16 blocks 16.1 / 17.7, 32 blocks 24.0 / 21.9, 64 blocks 39.4 / 23.7
+//  128 (512 rows, 32 / 8 heads):  32 blocks 23.6 / 27.1, 64 blocks 38.5 / 35.0, 128 blocks 68.8 / 46.9
+//  192 (3 x 256 rows, 32 / 8):    64 blocks 40.0 / 41.8, 96 blocks 55.1 / 53.8, 256 blocks 131 / 115
+//  256 (512 rows, 64 / 8 heads):  64 blocks 41.2 / 47.3, 128 blocks 76.9 / 77.8, 256 blocks 145 / 138
+// so from 16 blocks on, or 7 / 16 of the number of workgroups, or half of it where a split leaves no CU to itself.  The last
+// row block decides for all: where some are split and others are not, the launch is as long as without a split and the merge comes
+// on top (4 x 64 rows of 32 / 8 heads, 23 and 24 blocks, the pass 27 us, 22 without a split).
+constexpr int kMinPartBlocks = 8, kMinSplitBlocks = 16;
+// Parts up to one workgroup per CU; twice as many, which then share a CU's matrix pipes, from this many blocks per part
+// on (128 workgroups, 2 / 4 parts: 64 blocks 35.0 / 35.6 us, 80 blocks 43.5 / 41.5, 96 blocks 43.6 / 40.8, 256 blocks
+// 82.5 / 77.3).
+constexpr int kSharedPartBlocks = 20;
 constexpr int kMaxParts = 16;
 constexpr int kPartAccFloats = kRowsPerWave * kD;  // accumulators of one (part, head, row block)
 
-// The share of `nblk` blocks that part `part` of at most `parts` takes; the merge kernel asks the same
-// question.  Shares are whole 64-key tiles.
-__device__ __forceinline__ int blocks_per_part(int nblk, int parts) {
-  return max((((nblk + parts - 1) / parts) + 1) & ~1, kMinPartBlocks);
+// Blocks of a part (whole 64-key tiles) in a launch whose first query row is at `offset`; a row block of no more is not split.
+__device__ __forceinline__ int blocks_per_part(const PrefillArgs &a, int offset) {
+  const int most = max(((a.causal ? min(a.skv, offset + a.sq) : a.skv) + kBlockKeys - 1) / kBlockKeys, 1);  // of the last row block
+  if (most < a.split_from) return most;
+  const int shared = (most + a.parts - 1) / a.parts;
+  const int share = shared >= kSharedPartBlocks ? shared : max((most + a.parts_one - 1) / a.parts_one, kMinPartBlocks);
+  return (share + 1) & ~1;
 }
 
 // Accumulators and (reference, sum) rows of the parts: [part][batch][head][row block], the statistics
@@ -241,13 +260,16 @@ __global__ __launch_bounds__(256, 2) void prefill_stream_kernel(PrefillArgs a) {
   const int n = lane & 31, h = lane >> 5;
   const int nqt = (a.sq + kRowsPerWave * RPW - 1) / (kRowsPerWave * RPW);
   const int groups = a.hq / HPW;
+  // The part is the slowest index: the workgroups of part 0, the only ones with work where the keys are few, are dealt over the
+  // XCDs and CUs as in a launch that is not split.  (As the fastest index, they met on half of the CUs or a quarter: 256
+  // workgroups over 512 keys 20.5 us, 16.3 this way.)
+  const int part = PAGED ? wg / a.part_stride : 0;
+  if (PAGED) wg -= part * a.part_stride;
   const int xcd = wg & 7, slot = wg >> 3;
-  const int per_group = PAGED ? a.spg * a.parts : a.spg;
-  const int yl = slot / per_group;
+  const int yl = slot / a.spg;
   const int y = yl * 8 + xcd;
   if (y >= a.batch * groups) return;  // grid is padded to a multiple of 8 groups
-  const int item0 = PAGED ? (slot - yl * per_group) / a.parts : slot - yl * per_group;
-  const int part = PAGED ? slot - yl * per_group - item0 * a.parts : 0;
+  const int item0 = slot - yl * a.spg;
   const int qt = nqt - 1 - item0;
   const int b = y / groups;
   const int hq0 = (y - b * groups) * HPW;
@@ -266,7 +288,7 @@ __global__ __launch_bounds__(256, 2) void prefill_stream_kernel(PrefillArgs a) {
   bool whole = true;  // this workgroup sees all keys of its rows
   if constexpr (PAGED) {
     if (a.parts > 1) {
-      const int share = __builtin_amdgcn_readfirstlane(blocks_per_part(nblk, a.parts));
+      const int share = __builtin_amdgcn_readfirstlane(blocks_per_part(a, offset));
       whole = share >= nblk;
       first_block = part * share;
       nblk = min(share, nblk - first_block);
@@ -434,7 +456,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
   const int wg_last_row = min(a.sq, (qt + 1) * kRowsPerWave * RPW) - 1;
   const int kv_end = a.causal ? min(a.skv, offset + wg_last_row + 1) : a.skv;
   const int nblk = (kv_end + kBlockKeys - 1) / kBlockKeys;
-  const int share = blocks_per_part(nblk, a.parts);
+  const int share = blocks_per_part(a, offset);
   if (share >= nblk) return;  // one workgroup saw all keys and wrote the output
   const int active = (nblk + share - 1) / share;
   const PartLayout lay = part_layout(a, kRowsPerWave * RPW);
@@ -486,20 +508,22 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
     *reinterpret_cast<uint2 *>(op + 4 * i) = make_uint2(pack_bf16x2(o[4 * i] * inv, o[4 * i + 1] * inv), pack_bf16x2(o[4 * i + 2] * inv, o[4 * i + 3] * inv));
 }
 
-// Parts a launch is split into: as many as fill the two workgroup slots of every CU once, if its row blocks leave
-// at least half of them empty.  Only the host's view: how many keys there are is in device memory, and
-// the kernel takes fewer parts where they would get short.
-int launch_parts(const PrefillArgs &a, int heads_per_wg) {
+// Workgroups of the launch without a split, and what it may be split into: as many parts as fill the two workgroup slots of
+// every CU once, if its row blocks leave at least half of them empty and its page table is wide enough to be split at all.
+void set_parts(PrefillArgs &a, int heads_per_wg) {
   int cus = device_cus();
   if (cus <= 0) cus = 256;
   const int rows = kRowsPerWave * 4 / heads_per_wg;
   const int64_t wgs = (int64_t)a.batch * (a.hq / heads_per_wg) * ((a.sq + rows - 1) / rows);
-  const int most = (a.w * (a.bs / kBlockKeys) + kMinPartBlocks - 1) / kMinPartBlocks;
-  return (int)std::max<int64_t>(1, std::min<int64_t>({2 * cus / wgs, kMaxParts, most}));
+  const int blocks = a.w * (a.bs / kBlockKeys);
+  const int most = std::min(kMaxParts, (blocks + kMinPartBlocks - 1) / kMinPartBlocks);
+  a.split_from = (int)std::max<int64_t>(kMinSplitBlocks, 2 * wgs <= cus ? 7 * wgs / 16 : std::min<int64_t>(wgs, 2 * cus) / 2);
+  a.parts = blocks < a.split_from ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>(2 * cus / wgs, most));
+  a.parts_one = (int)std::max<int64_t>(1, std::min<int64_t>(cus / wgs, most));
 }
 
 int64_t part_bytes(PrefillArgs a, int heads_per_wg) {
-  a.parts = launch_parts(a, heads_per_wg);
+  set_parts(a, heads_per_wg);
   if (a.parts <= 1) return 0;
   return part_layout(a, kRowsPerWave * 4 / heads_per_wg).slots * (kPartAccFloats + 2 * kRowsPerWave) * (int64_t)sizeof(float);
 }
@@ -529,7 +553,7 @@ int launch_form(const PrefillArgs &a, hipStream_t st) {
   // (read on every call) an experiment's override: several row blocks per workgroup, each over all of its keys
   const char *e = HPW == 4 && (FORM == kDense || FORM == kPaged) ? getenv("TTPA_PREFILL_WGS_PER_GROUP") : nullptr;
   const int per_group = e ? atoi(e) : 0;
-  if (PAGED && per_group <= 0 && a.part_acc && a.part_bytes >= part_bytes(a, HPW)) b.parts = launch_parts(a, HPW);
+  if (PAGED && per_group <= 0 && a.part_acc && a.part_bytes >= part_bytes(a, HPW)) set_parts(b, HPW);
   if (per_group > 0) {
     b.spg = std::min(nqt, per_group);
   } else if (HPW == 4 && (FORM == kDense || FORM == kPaged) && b.parts == 1) {
@@ -542,7 +566,8 @@ int launch_form(const PrefillArgs &a, hipStream_t st) {
     const int one_round = (2 * cus + ny8 * 8 - 1) / (ny8 * 8);
     b.spg_even = one_round < nqt && nqt % one_round == 0 ? one_round : 0;
   }
-  int grid = b.spg * b.parts * ny8 * 8;
+  b.part_stride = b.spg * ny8 * 8;
+  int grid = b.part_stride * b.parts;
   if (!PAGED && FORM != kDenseWide && a.fill_kc) grid = grid_with_fill(b, grid, kD);
   launch_dominant(&prefill_stream_kernel<HPW, FORM>, dim3(grid), dim3(256), (size_t)TTPA_STREAM_LDS_BYTES, st, b);
   if (const int rc = check_launch("sdpa_prefill")) return rc;
