@@ -190,6 +190,13 @@ def host():
     return _host
 
 
+def attention_pass(*args):
+    """The host path's entry; the first call puts the extension's own function in its place."""
+    global attention_pass
+    attention_pass = host().attention_pass
+    return attention_pass(*args)
+
+
 def check(name: str, rc: int) -> None:
     """Raises TtpaError for a negative status."""
     if rc != OK:

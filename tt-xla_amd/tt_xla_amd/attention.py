@@ -336,7 +336,7 @@ class TTAttentionBackendImpl(_ImplBase):
             or torch.compiler.is_compiling()
         ):
             return False
-        status = _native.host().attention_pass(
+        status = _native.attention_pass(
             query, key, value, kv_cache[0], kv_cache[1], attn_metadata.page_table, attn_metadata.cache_position,
             attn_metadata.fill_page_table, attn_metadata.batch_idx, attn_metadata.chunk_start_idx, self.sinks, output,
             attn_metadata.num_users, self.num_heads, self.num_kv_heads, self.head_size, self.scale,
