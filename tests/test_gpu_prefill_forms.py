@@ -199,3 +199,22 @@ def test_where_the_split_begins(users, hq, hkv, lc, blocks, bs, monkeypatch):
             whole = torch.ops.tt.chunked_scaled_dot_product_attention(*args)
         assert torch.equal(got, whole) == (n < blocks)
         torch.testing.assert_close(got.float(), whole.float(), atol=2e-2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("hq,hkv,bs", [(2, 2, 32), (4, 1, 64)])
+@pytest.mark.parametrize("users,lc,width,start", [(1, 32, 8, 90), (3, 128, 40, 1000), (1, 100, 300, 64), (2, 200, 12, 150)])
+def test_block_float_8_chunks(hq, hkv, bs, users, lc, width, start):
+    """Through bfloat16 copies (walked by a fixed number of workgroups, only the columns that the pass reads) or tile by
+    tile, whichever the pass takes: the attention over the values that the cache holds."""
+    from tt_xla_amd import custom_ops as ops
+
+    if start + lc > width * bs:
+        width = -(-(start + lc) // bs)
+    g = torch.Generator().manual_seed(lc + width)
+    key, value = (ops.bfp8_pack_cache(P._bf(g, 60, hkv, bs, 128).cuda()) for _ in range(2))
+    table = torch.randint(-1, 61, (users, width), generator=g).to(torch.int32)  # (ids outside the cache read block 0)
+    q, st = P._bf(g, users, hq, lc, 128), torch.tensor([start], dtype=torch.int32)
+    want = O.chunked_sdpa(q, ops.bfp8_unpack_cache(key).cpu(), ops.bfp8_unpack_cache(value).cpu(),
+                          torch.where((table < 0) | (table >= 60), 0, table), st, 128**-0.5)
+    got = torch.ops.tt.chunked_scaled_dot_product_attention(q.cuda(), key, value, table.cuda(), st.cuda(), 128**-0.5)
+    P._check(f"bfp8 h{hq}x{hkv} bs{bs} u{users} len{lc} width{width}", got.cpu(), want)

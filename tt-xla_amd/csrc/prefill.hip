@@ -42,10 +42,13 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
 
 // Expansion of the block-float-8 blocks a chunk pass reads into bfloat16 copies, so that the
 // hand-scheduled loop (which wants bfloat16 blocks it can request straight into LDS) serves a
-// block-float-8 cache too: workgroup (x, y) expands the slab of table entry x = batch entry * width
-// + column and of (KV head, K or V) y into block x of a scratch cache, and writes entry x of the
-// identity table that goes with it.  Columns behind the last key of the pass are skipped.  Memory
-// work (1 byte in, 2 out per element) of about a tenth of the attention's time.
+// block-float-8 cache too: the slab of table entry x = batch entry * width + column and of a (KV head, K or V)
+// goes to block x of a scratch cache, and entry x of the identity table that goes with it is written.  Memory work (1 byte
+// in, 2 out per element) of about a tenth of the attention's time.  How many columns the pass reads is in device memory, so
+// a fixed number of workgroups (eight per CU, what fits) walks the slabs there are: one workgroup per slab of the page table cost
+// 0.25 ns each where most had nothing to do (4 x 64 rows behind 256 tokens, 16 / 16 heads, blocks of 32 under 32768 columns:
+// the pass 60.9 -> 25.4 us).
+constexpr int kExpandWorkgroups = 2048;
 struct ExpandArgs {
   const uint8_t *kc, *vc;  // the block-float-8 caches
   uint16_t *k, *v;         // scratch caches [batch * width][KV heads][block size][D]
@@ -53,42 +56,46 @@ struct ExpandArgs {
   const int32_t *pt;
   int64_t pt_rs;
   const int32_t *chunk_start;
-  int w, hkv, bs, nb, sq, causal;
+  int batch, w, hkv, bs, nb, sq, causal;
 };
 
 template <int D>
 __global__ __launch_bounds__(256) void bfp8_expand_kernel(ExpandArgs e) {
-  const int x = blockIdx.x, b = x / e.w, j = x - b * e.w;
-  const int h = blockIdx.y >> 1;
-  const bool is_v = blockIdx.y & 1;
-  if (blockIdx.y == 0 && threadIdx.x == 0) e.table[x] = x;
   const int skv = e.w * e.bs;
   const int kv_end = e.causal ? min(skv, chunk_offset(e.chunk_start, e.sq, skv) + e.sq) : skv;
-  if (j * e.bs >= kv_end) return;
-  int phys = e.pt[(int64_t)b * e.pt_rs + j];
-  if ((unsigned)phys >= (unsigned)e.nb) phys = 0;  // (as the attention kernels treat a bad entry)
-  const int64_t slab = (int64_t)(e.bs + e.bs / 16) * D;
-  const uint8_t *src = (is_v ? e.vc : e.kc) + ((int64_t)phys * e.hkv + h) * slab;
-  const uint8_t *exps = src + (int64_t)e.bs * D;
-  uint16_t *dst = (is_v ? e.v : e.k) + ((int64_t)x * e.hkv + h) * e.bs * D;
-  const int groups = e.bs * D / 16;
-  for (int g = threadIdx.x; g < groups; g += 256) {
-    const u32x4 bytes = *reinterpret_cast<const u32x4 *>(src + 16 * g);
-    const float sc = bfp8_group_scale(exps[g]), off = -128.f * sc;
-    u32x4 lo, hi;
+  const int cols = (kv_end + e.bs - 1) / e.bs;  // page-table columns that the pass reads
+  const int blocks = e.batch * cols, items = kv_end > 0 ? blocks * 2 * e.hkv : 0;
+  for (int item = blockIdx.x; item < items; item += gridDim.x) {
+    const int part = item / blocks, r = item - part * blocks;  // (K or V, KV head); block of the pass
+    const int b = r / cols, j = r - b * cols, x = b * e.w + j;
+    const int h = part >> 1;
+    const bool is_v = part & 1;
+    if (part == 0 && threadIdx.x == 0) e.table[x] = x;
+    int phys = e.pt[(int64_t)b * e.pt_rs + j];
+    if ((unsigned)phys >= (unsigned)e.nb) phys = 0;  // (as the attention kernels treat a bad entry)
+    const int64_t slab = (int64_t)(e.bs + e.bs / 16) * D;
+    const uint8_t *src = (is_v ? e.vc : e.kc) + ((int64_t)phys * e.hkv + h) * slab;
+    const uint8_t *exps = src + (int64_t)e.bs * D;
+    uint16_t *dst = (is_v ? e.v : e.k) + ((int64_t)x * e.hkv + h) * e.bs * D;
+    const int groups = e.bs * D / 16;
+    for (int g = threadIdx.x; g < groups; g += 256) {
+      const u32x4 bytes = *reinterpret_cast<const u32x4 *>(src + 16 * g);
+      const float sc = bfp8_group_scale(exps[g]), off = -128.f * sc;
+      u32x4 lo, hi;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const uint32_t v = bytes[w];
-      const float f0 = fmaf((float)(v & 0xffu), sc, off), f1 = fmaf((float)((v >> 8) & 0xffu), sc, off);
-      const float f2 = fmaf((float)((v >> 16) & 0xffu), sc, off), f3 = fmaf((float)(v >> 24), sc, off);
-      // the products are exact in bfloat16: their upper halves are the elements
-      const uint32_t p0 = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, f1), __builtin_bit_cast(uint32_t, f0), 0x07060302u);
-      const uint32_t p1 = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, f3), __builtin_bit_cast(uint32_t, f2), 0x07060302u);
-      if (w < 2) lo[2 * w] = p0, lo[2 * w + 1] = p1;
-      else hi[2 * (w - 2)] = p0, hi[2 * (w - 2) + 1] = p1;
+      for (int w = 0; w < 4; ++w) {
+        const uint32_t v = bytes[w];
+        const float f0 = fmaf((float)(v & 0xffu), sc, off), f1 = fmaf((float)((v >> 8) & 0xffu), sc, off);
+        const float f2 = fmaf((float)((v >> 16) & 0xffu), sc, off), f3 = fmaf((float)(v >> 24), sc, off);
+        // the products are exact in bfloat16: their upper halves are the elements
+        const uint32_t p0 = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, f1), __builtin_bit_cast(uint32_t, f0), 0x07060302u);
+        const uint32_t p1 = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, f3), __builtin_bit_cast(uint32_t, f2), 0x07060302u);
+        if (w < 2) lo[2 * w] = p0, lo[2 * w + 1] = p1;
+        else hi[2 * (w - 2)] = p0, hi[2 * (w - 2) + 1] = p1;
+      }
+      *reinterpret_cast<u32x4 *>(dst + 16 * g) = lo;
+      *reinterpret_cast<u32x4 *>(dst + 16 * g + 8) = hi;
     }
-    *reinterpret_cast<u32x4 *>(dst + 16 * g) = lo;
-    *reinterpret_cast<u32x4 *>(dst + 16 * g + 8) = hi;
   }
 }
 
@@ -633,7 +640,7 @@ int launch(const PrefillArgs &a, hipStream_t st) {
     // With scratch from the caller, a pass that the hand-scheduled loop can serve reads bfloat16
     // copies of its blocks (written by one launch in front of it) instead of expanding every
     // tile once per workgroup on its way into LDS.
-    if (a.expand && stream_serves(a, D)) {
+    if (a.expand && stream_expands(a, D)) {
       const int64_t blocks = (int64_t)a.batch * a.w;
       const int64_t cache_elems = blocks * a.hkv * a.bs * D;
       ExpandArgs e;
@@ -641,11 +648,11 @@ int launch(const PrefillArgs &a, hipStream_t st) {
       e.k = static_cast<uint16_t *>(a.expand), e.v = e.k + cache_elems;
       e.table = reinterpret_cast<int32_t *>(e.v + cache_elems);
       e.pt = a.pt, e.pt_rs = a.pt_rs, e.chunk_start = a.chunk_start;
-      e.w = a.w, e.hkv = a.hkv, e.bs = a.bs, e.nb = a.nb, e.sq = a.sq, e.causal = a.causal;
+      e.batch = a.batch, e.w = a.w, e.hkv = a.hkv, e.bs = a.bs, e.nb = a.nb, e.sq = a.sq, e.causal = a.causal;
       // armed events: the pair brackets both launches
       hipEvent_t before, after;
       take_profile_events(before, after);
-      const dim3 grid((unsigned)blocks, (unsigned)(2 * a.hkv));
+      const dim3 grid((unsigned)std::min<int64_t>(blocks * 2 * a.hkv, kExpandWorkgroups));
       if (before)
         hipExtLaunchKernelGGL(bfp8_expand_kernel<D>, grid, dim3(256), 0u, st, before, nullptr, 0u, e);
       else
@@ -834,7 +841,9 @@ extern "C" int64_t ttpa_sdpa_prefill_scratch_bytes(int32_t batch, int32_t q_head
   PrefillArgs a = {};
   a.pt = &some_table, a.stream = 1;
   a.batch = batch, a.hq = q_heads, a.hkv = kv_heads, a.sq = q_len, a.bs = block_size, a.w = table_width;
-  return ttpa_sdpa_prefill_workspace_bytes(batch, kv_heads, head_size, block_size, table_width, kv_format) + stream_part_bytes(a, head_size);
+  const int64_t expansion = stream_expands(a, head_size)
+      ? ttpa_sdpa_prefill_workspace_bytes(batch, kv_heads, head_size, block_size, table_width, kv_format) : 0;
+  return kv_format == TTPA_KV_BFP8 && expansion == 0 ? 0 : expansion + stream_part_bytes(a, head_size);
 }
 
 extern "C" int ttpa_sdpa_prefill_fill(

@@ -600,6 +600,16 @@ int64_t stream_part_bytes(const PrefillArgs &a, int head_size) {
   return a.pt && stream_serves(a, head_size) ? part_bytes(a, heads_per_workgroup(a)) : 0;
 }
 
+// A pass of one workgroup per head group reads every block once, so mode 4's expansion on the way into LDS is not repeated either:
+// the copies, a trip through memory in front of the attention, pay where they are few or where the keys may be split
+// (16 / 16 heads, copies / mode 4: 1 x 128 rows over 256 keys 17.4 / 19.3 us, 4 x 64 rows over 320 keys 22.7 / 20.5; 1 x 128
+// rows over 2176 keys, where the copies let it be split, 32.0 / 78.6).
+bool stream_expands(const PrefillArgs &a, int head_size) {
+  if (!stream_serves(a, head_size)) return false;
+  const int hpw = heads_per_workgroup(a);
+  return a.sq > kRowsPerWave * 4 / hpw || (int64_t)a.batch * a.w * a.bs * a.hkv <= 8192 || part_bytes(a, hpw) > 0;
+}
+
 int launch_stream_wide(const PrefillArgs &a, hipStream_t st) {
   switch (heads_per_workgroup(a)) {
     case 4: return launch_form<4, kDenseWide>(a, st);
