@@ -218,3 +218,38 @@ def test_block_float_8_chunks(hq, hkv, bs, users, lc, width, start):
                           torch.where((table < 0) | (table >= 60), 0, table), st, 128**-0.5)
     got = torch.ops.tt.chunked_scaled_dot_product_attention(q.cuda(), key, value, table.cuda(), st.cuda(), 128**-0.5)
     P._check(f"bfp8 h{hq}x{hkv} bs{bs} u{users} len{lc} width{width}", got.cpu(), want)
+
+
+@pytest.mark.parametrize("native", [False, True])
+def test_a_pass_without_room_for_scratch_runs(native):
+    """The scratch is sized by the page table, which is as wide as the longest sequence may be; memory is what the
+    caches leave.  A pass that cannot have it runs without."""
+    from tt_xla_amd import TTAttentionBackendImpl, TTMetadata
+    from tt_xla_amd import custom_ops as ops
+
+    g = torch.Generator().manual_seed(3)
+    users, rows, start, bs, width = 2, 64, 96, 32, 4096
+    kc, vc = (ops.bfp8_pack_cache(P._bf(g, 12, 2, bs, 128).cuda()) for _ in range(2))
+    table = torch.zeros(users, width, dtype=torch.int32)
+    table[:, :5] = torch.arange(10).view(2, 5) + 1
+    q, k, v = (P._bf(g, users * rows, n * 128).cuda() for n in (2, 2, 2))
+    md = TTMetadata(page_table=table.cuda(), fill_page_table=torch.roll(table, -3, 1).cuda(), num_users=users,
+                    batch_idx=torch.arange(users, dtype=torch.int32).cuda(), chunk_start_idx=torch.tensor([start], dtype=torch.int32).cuda())
+    impl = TTAttentionBackendImpl(2, 128, 128**-0.5, 2, None, None, "auto")
+    if not native:
+        impl._native_pass = lambda *a: False
+    outs = []
+    for room in (True, False):
+        out = torch.zeros_like(q)
+        ops._WORKSPACES.clear()
+        torch.cuda.empty_cache()
+        if not room:  # 64 MiB where the copies of 2 x 4096 blocks would be 268
+            total = torch.cuda.get_device_properties(0).total_memory
+            torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (64 << 20)) / total)
+        try:
+            impl.forward(None, q, k, v, [kc, vc], md, output=out)
+            torch.cuda.synchronize()
+        finally:
+            torch.cuda.set_per_process_memory_fraction(1.0)
+        outs.append(out)
+    torch.testing.assert_close(outs[1].float(), outs[0].float(), atol=1e-2, rtol=1e-2)

@@ -205,7 +205,14 @@ PyObject *attention_pass(PyObject *, PyObject *const *v, Py_ssize_t n) {
   RECORD_FUNCTION("tt::chunked_scaled_dot_product_attention_out", std::vector<c10::IValue>());
   const auto launch = [&] {
     const Unlocked unlocked;
-    const at::Tensor ws = bytes ? scratch(bytes, out) : at::Tensor();
+    at::Tensor ws;
+    if (bytes) {
+      try {
+        ws = scratch(bytes, out);
+      } catch (const c10::OutOfMemoryError &) {  // sized by the page table, not by the pass: it runs without, too
+        bytes = 0;
+      }
+    }
     return ttpa_sdpa_prefill_expanded(
         out->data_ptr(), s * hq * d, d, hq * d, q->data_ptr(), s * q->stride(0), d, q->stride(0), kc->data_ptr(), vc->data_ptr(), 0, 0,
         0, static_cast<const int32_t *>(pt->data_ptr()), pt->stride(0), static_cast<const int32_t *>(start->data_ptr()), nullptr, 0, 0,
