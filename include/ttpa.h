@@ -420,8 +420,9 @@ int64_t ttpa_sdpa_prefill_workspace_bytes(int32_t batch, int32_t kv_heads, int32
 /* Bytes of scratch with which ttpa_sdpa_prefill_expanded runs these dimensions fastest: the above, and, for
  * either cache format, room for float partial results where a pass of few query rows over many keys is
  * split over the keys (head size 128, block_size a multiple of 32; at most 16 parts, 34 MB for 512 rows of 32
- * heads).  With less, a null or a smaller workspace the pass runs unsplit.  Scratch for the expansion comes
- * first; what is behind it is used for the parts. */
+ * heads).  0 where neither would pay (a table too narrow to be split; over block-float-8 caches, one workgroup per
+ * head group and many copies).  With less, a null or a smaller workspace the pass runs unsplit.  Scratch for the
+ * expansion comes first; what is behind it is used for the parts. */
 int64_t ttpa_sdpa_prefill_scratch_bytes(int32_t batch, int32_t q_heads, int32_t kv_heads, int32_t q_len,
                                         int32_t head_size, int32_t block_size, int32_t table_width,
                                         int32_t kv_format);
