@@ -52,13 +52,13 @@ MEASURED_TRAFFIC = {
     # workload: (kernel, hash of its sources, HBM bytes per launch: FETCH_SIZE and WRITE_SIZE of the
     # kernel, each scaled by what the same counter reads for a plain copy of known size, mean over
     # the rotating workload copies; the summaries under profiles/ hold the runs)
-    "config2": ("paged_decode_mfma16_kernel", "410306992a9b7e9b", 310401700),
-    "config5": ("paged_decode_mfma16_kernel", "410306992a9b7e9b", 168429392),
-    "config4": ("paged_decode_mfma16_kernel", "410306992a9b7e9b", 3415529248),
-    "config3": ("prefill_stream_kernel", "810acb56ec44bcd9", 244818087),
-    "latent": ("paged_decode_latent16_kernel", "611a48caa3e35aca", 654199020),
-    "latent128": ("paged_decode_latent128_kernel", "75ff2b818e7d1cd4", 739359598),
-    "latent-prefill": ("latent_prefill_kernel", "75ff2b818e7d1cd4", 332249956),
+    "config2": ("paged_decode_mfma16_kernel", "410306992a9b7e9b", 310401819),
+    "config5": ("paged_decode_mfma16_kernel", "410306992a9b7e9b", 168429456),
+    "config4": ("paged_decode_mfma16_kernel", "410306992a9b7e9b", 3415530563),
+    "config3": ("prefill_stream_kernel", "4aae0c7b51b8339c", 244868493),
+    "latent": ("paged_decode_latent16_kernel", "611a48caa3e35aca", 654199267),
+    "latent128": ("paged_decode_latent128_kernel", "75ff2b818e7d1cd4", 739359865),
+    "latent-prefill": ("latent_prefill_kernel", "75ff2b818e7d1cd4", 332250032),
 }
 DECODE_KERNEL_NAME = {"config2": "paged_decode_mfma16_kernel", "config4": "paged_decode_mfma16_kernel",
                       "config5": "paged_decode_mfma16_kernel"}
