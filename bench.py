@@ -17,7 +17,7 @@ Other workloads (same JSON contract):
            useful TFLOP/s
 
 Prints ONE JSON line.  `roofline` is the dominant kernel alone, timed by a HIP event
-pair that its launch carries inside the library; `cpu_baseline` is the CPU oracle timed on this box's host cores on a
+pair that its launch carries inside the library; `cpu_baseline` is the CPU oracle timed on this host's cores on a
 bounded sample of the same workload.
 """
 
@@ -62,7 +62,7 @@ MEASURED_TRAFFIC = {
 }
 DECODE_KERNEL_NAME = {"config2": "paged_decode_mfma16_kernel", "config4": "paged_decode_mfma16_kernel",
                       "config5": "paged_decode_mfma16_kernel"}
-CPU_THREADS_CAP = 16        # host cores a one-GPU box grants, whatever os.cpu_count() says
+CPU_THREADS_CAP = 16        # host cores a one-GPU share of a host grants, whatever os.cpu_count() says
 
 
 def kernel_source_hash(kernel):
