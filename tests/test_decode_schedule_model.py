@@ -1,5 +1,5 @@
 """Host-side model of the split-K schedule of the decode kernels (tt-xla_amd/csrc/decode_common.h:
-build_prefix, locate_unit, publish_segment_row; the range walk that every decode kernel repeats).
+build_prefix, share_of, locate_unit, publish_segment_row; the range walk that every decode kernel repeats).
 
 The flat list holds, per (user, kv head) segment with at least one tile, `extra` leading units that
 carry no work and then the segment's tiles; it is cut into n_eff equal ranges of units.  The model
@@ -10,6 +10,7 @@ processed one of its tiles.  Pure integers, no GPU: it guards the formulas, not 
 
 import random
 
+import numpy as np
 import pytest
 
 
@@ -141,3 +142,73 @@ def test_weighted_ranges_balance_cost():
         opened = sum(1 for (_, _, rel) in mine[1:] if rel == 0)
         cost.append(len(mine) + opened)
     assert max(cost) - min(cost) <= 2
+
+
+# --------------------------------------------------------------------------- #
+# the forms that replace 64-bit divisions and the interval search (share_of, publish_segment_row, locate_unit)
+# --------------------------------------------------------------------------- #
+U32 = 1 << 32
+
+
+def short_share(total, n_ranges, extra, index):
+    """share_of below 2^31 units and 2^15 ranges, in 32-bit words."""
+    room = extra + 1
+    assert n_ranges * room < U32
+    n = n_ranges if total >= n_ranges * room else total // room
+    if index >= n:
+        return n, 0, 0
+    q, r = divmod(total, n)
+    for word in ((index + 1) * q, (index + 1) * r):
+        assert word < U32
+    return n, index * q + index * r // n, (index + 1) * q + (index + 1) * r // n
+
+
+def short_owner(x, n, total):
+    """The wavefront that owns unit x: a float quotient, off by one at most."""
+    p = (x + 1) * n - 1
+    w = int(np.float32(p) / np.float32(total))
+    assert abs(w - p // total) <= 1
+    if w * total > p:
+        w -= 1
+    elif (w + 1) * total <= p:
+        w += 1
+    return w
+
+
+def lane_search(pref, hkv, x):
+    """locate_unit's search: 64 lanes compare an entry each, above 64 users every `step`-th first."""
+    users = len(pref) - 1
+    lo, step, count = 0, (users + 63) // 64, users
+    if step > 1:
+        lo = (sum(1 for lane in range(64) if lane * step < users and pref[min(lane * step, users - 1)] * hkv <= x) - 1) * step
+        count = min(step, users - lo)
+    assert 1 <= count <= 64
+    return lo + sum(1 for lane in range(64) if lane < count and pref[lo + min(lane, count - 1)] * hkv <= x) - 1
+
+
+@pytest.mark.parametrize("extra", [0, 1, 4, 64])
+def test_short_forms_of_the_cut(extra):
+    rng = random.Random(23 + extra)
+    totals = [1, 2, extra + 1, extra + 2, (1 << 31) - 1, 1 << 24] + [int(2 ** rng.uniform(0, 31)) for _ in range(60)]
+    for total in totals:
+        for n_ranges in (1, 4, 192, 768, 1024, 2048, 32768):
+            n = min(total // (extra + 1), n_ranges)
+            for index in {0, 1, n // 2, n - 2, n - 1, n, n_ranges - 1} | {rng.randrange(n_ranges) for _ in range(4)}:
+                if index < 0:
+                    continue
+                got = short_share(total, n_ranges, extra, index)
+                assert got == ((n, index * total // n, (index + 1) * total // n) if index < n else (n, 0, 0))
+            if n:
+                for x in {0, total - 1, total // 2} | {rng.randrange(total) for _ in range(6)}:
+                    assert short_owner(x, n, total) == ((x + 1) * n + total - 1) // total - 1
+
+
+@pytest.mark.parametrize("users", [1, 2, 63, 64, 65, 66, 127, 128, 129, 1000, 1985, 2047, 2048])
+def test_lane_search_finds_the_users_segment(users):
+    rng = random.Random(users)
+    for zeros in (0.0, 0.4):
+        pref = prefix([0 if rng.random() < zeros else rng.randint(1, 50) for _ in range(users)], 1)
+        hkv = rng.choice([1, 2, 8])
+        total = pref[-1] * hkv
+        for x in {0, total - 1} | {rng.randrange(total) for _ in range(40)} if total else ():
+            assert lane_search(pref, hkv, x) == locate(pref, hkv, x, 1)[0]

@@ -60,16 +60,16 @@ __global__ __launch_bounds__(256, (D <= 128 && G <= 4) ? 2 : 1) void paged_decod
   // The flat list in units: per segment `seg_units` units that stand for the cost of opening it,
   // then its tiles.  A range of more than seg_units units holds at least one tile.
   const int total_units = __builtin_amdgcn_readfirstlane(s_pref[a.users]);
-  const int64_t total = (int64_t)total_units * a.hkv;
-  const int64_t max_ranges = total / (seg_units + 1);
-  const int n_eff = (int)(max_ranges < a.n_waves ? max_ranges : a.n_waves);  // wavefronts that get work
+  const Share share = share_of(total_units, a.hkv, a.n_waves, seg_units, wave);
+  const int64_t total = share.total;
+  const int n_eff = share.n_eff;  // wavefronts that get work
   if (total == 0 || wave >= n_eff) {  // idle wavefronts still do their share of the table
     publish_segment_row(a, s_pref, total, n_eff, seg_units);
     return;
   }
-  const int64_t x_lo = (int64_t)wave * total / n_eff;
+  const int64_t x_lo = share.lo;
   int64_t x = x_lo;  // set below to the unit of the first tile at or behind x_lo
-  const int64_t x_hi = (int64_t)(wave + 1) * total / n_eff;
+  const int64_t x_hi = share.hi;
   lds_u16 *plds = s_p[wib];
   const int my_step = bitrev4(c);
   const uint16_t *kb = reinterpret_cast<const uint16_t *>(a.k);
@@ -427,6 +427,7 @@ static int decode_impl(void *out, int64_t out_user_stride, int64_t out_head_stri
   a.cur = cur_pos, a.cur_i64 = cur_pos_is_i64;
   a.users = users, a.hq = q_heads, a.hkv = kv_heads, a.bs = block_size, a.w = table_width;
   a.nb = num_blocks;
+  a.bs_magic = block_magic((int64_t)table_width * block_size, block_size);
   a.scale_log2e = scale * 1.4426950408889634f;
   a.ws_seg = static_cast<int *>(workspace);
   a.ws_slots = reinterpret_cast<float *>(static_cast<uint8_t *>(workspace) + header_bytes(users, kv_heads));

@@ -58,16 +58,16 @@ __global__ __launch_bounds__(256, 2) void paged_decode_bfp8_kernel(
   // The flat list in units: per segment `seg_units` units that stand for the cost of opening it,
   // then its tiles.  A range of more than seg_units units holds at least one tile.
   const int total_units = __builtin_amdgcn_readfirstlane(s_pref[a.users]);
-  const int64_t total = (int64_t)total_units * a.hkv;
-  const int64_t max_ranges = total / (seg_units + 1);
-  const int n_eff = (int)(max_ranges < a.n_waves ? max_ranges : a.n_waves);  // wavefronts that get work
+  const Share share = share_of(total_units, a.hkv, a.n_waves, seg_units, wave);
+  const int64_t total = share.total;
+  const int n_eff = share.n_eff;  // wavefronts that get work
   if (total == 0 || wave >= n_eff) {
     publish_segment_row(a, s_pref, total, n_eff, seg_units);
     return;
   }
-  const int64_t x_lo = (int64_t)wave * total / n_eff;
+  const int64_t x_lo = share.lo;
   int64_t x = x_lo;  // set below to the unit of the first tile at or behind x_lo
-  const int64_t x_hi = (int64_t)(wave + 1) * total / n_eff;
+  const int64_t x_hi = share.hi;
   lds_u16 *plds = s_p[wib];
   const int my_step = bitrev4(c);
   const int grp = (c * EPL) / 16;                              // exponent group of this lane

@@ -128,15 +128,15 @@ __global__ __launch_bounds__(256, 1) void paged_decode_mfma16_kernel(
   // The flat list in units: per segment `seg_units` units that stand for the cost of opening it,
   // then its tiles.  A range of more than seg_units units holds at least one tile.
   const int total_units = __builtin_amdgcn_readfirstlane(s_pref[a.users]);
-  const int64_t total = (int64_t)total_units * a.hkv;
-  const int64_t max_ranges = total / (seg_units + 1);
-  const int n_eff = (int)(max_ranges < a.n_waves ? max_ranges : a.n_waves);
+  const Share share = share_of(total_units, a.hkv, a.n_waves, seg_units, wave);
+  const int64_t total = share.total;
+  const int n_eff = share.n_eff;
   if (total == 0 || wave >= n_eff) {
     publish_segment_row(a, s_pref, total, n_eff, seg_units);
     return;
   }
-  const int64_t x_lo = (int64_t)wave * total / n_eff;
-  const int64_t x_hi = (int64_t)(wave + 1) * total / n_eff;
+  const int64_t x_lo = share.lo;
+  const int64_t x_hi = share.hi;
   int64_t x = x_lo;  // set below to the unit of the first tile at or behind x_lo
   uint8_t *tile = tiles + wib * kTileBytes;
   const int G = a.hq / a.hkv;
@@ -191,7 +191,7 @@ __global__ __launch_bounds__(256, 1) void paged_decode_mfma16_kernel(
     const int tok0 = cu.t * TILE;
     // a run never crosses a block (block_size is a multiple of the run length), so block and
     // row advance without a division; the table is read again only where the block changes
-    int col = tok0 / a.bs, row = tok0 - col * a.bs;
+    int col = block_of(a, tok0), row = tok0 - col * a.bs;
     int64_t base = 0;
 #pragma unroll
     for (int i = 0; i < NOFF; ++i) {

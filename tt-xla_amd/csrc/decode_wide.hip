@@ -69,14 +69,15 @@ __global__ __launch_bounds__(256, 1) void paged_decode_wide_kernel(
   const int n = lane & 31, h = lane >> 5;
   const int wg = blockIdx.x;
   const int total_tiles = __builtin_amdgcn_readfirstlane(s_pref[a.users]);
-  const int64_t total = (int64_t)total_tiles * a.hkv;
-  const int n_eff = (int)(total < a.n_waves ? total : a.n_waves);  // workgroups that get work
+  const Share share = share_of(total_tiles, a.hkv, a.n_waves, 0, wg);
+  const int64_t total = share.total;
+  const int n_eff = share.n_eff;  // workgroups that get work
   if (total == 0 || wg >= n_eff) {
     publish_segment_row(a, s_pref, total, n_eff);
     return;
   }
-  int64_t x = (int64_t)wg * total / n_eff;
-  const int64_t x_hi = (int64_t)(wg + 1) * total / n_eff;
+  int64_t x = share.lo;
+  const int64_t x_hi = share.hi;
   const int G = w.gseg;
   const int v_row_bytes = 2 * w.dv;                    // separate V cache: bytes per token row
   const int v_lds_row = v_row_bytes + 16;
@@ -405,15 +406,15 @@ __global__ __launch_bounds__(256, 1) void paged_decode_latent16_kernel(
   // The flat list in units: per segment `seg_units` units that stand for the cost of opening it,
   // then its tiles.  A range of more than seg_units units holds at least one tile.
   const int total_units = __builtin_amdgcn_readfirstlane(s_pref[a.users]);
-  const int64_t total = (int64_t)total_units * a.hkv;
-  const int64_t max_ranges = total / (seg_units + 1);
-  const int n_eff = (int)(max_ranges < a.n_waves ? max_ranges : a.n_waves);
+  const Share share = share_of(total_units, a.hkv, a.n_waves, seg_units, wave);
+  const int64_t total = share.total;
+  const int n_eff = share.n_eff;
   if (total == 0 || wave >= n_eff) {
     publish_segment_row(a, s_pref, total, n_eff, seg_units);
     return;
   }
-  const int64_t x_lo = (int64_t)wave * total / n_eff;
-  const int64_t x_hi = (int64_t)(wave + 1) * total / n_eff;
+  const int64_t x_lo = share.lo;
+  const int64_t x_hi = share.hi;
   int64_t x = x_lo;  // set below to the unit of the first tile at or behind x_lo
   const int G = w.gseg;
   unsigned char *my_lds = smem + wib * L::WAVE_LDS;
@@ -831,15 +832,15 @@ __global__ __launch_bounds__(256) void paged_decode_latent128_kernel(
   // partial, the next segment's Q), then its tiles.  A range of more than seg_units units holds at
   // least one tile.
   const int total_units = __builtin_amdgcn_readfirstlane(s_pref[a.users]);
-  const int64_t total = (int64_t)total_units * a.hkv;
-  const int64_t max_ranges = total / (seg_units + 1);
-  const int n_eff = (int)(max_ranges < a.n_waves ? max_ranges : a.n_waves);  // workgroups that get work
+  const Share share = share_of(total_units, a.hkv, a.n_waves, seg_units, wg);
+  const int64_t total = share.total;
+  const int n_eff = share.n_eff;  // workgroups that get work
   if (total == 0 || wg >= n_eff) {
     publish_segment_row(a, s_pref, total, n_eff, seg_units);
     return;
   }
-  const int64_t x_lo = (int64_t)wg * total / n_eff;
-  const int64_t x_hi = (int64_t)(wg + 1) * total / n_eff;
+  const int64_t x_lo = share.lo;
+  const int64_t x_hi = share.hi;
   int64_t x = x_lo;  // set below to the unit of the first tile at or behind x_lo
   const int G = w.gseg;
 
