@@ -364,6 +364,28 @@ int launch_g(const DecodeArgs &a, int g, hipStream_t st) {
 using namespace ttpa;
 using namespace ttpa::decode;
 
+// Wavefronts of a workgroup that reads a whole (user, KV head) segment, writes the output itself and leaves nothing to
+// merge; 0: the segments are cut into equal ranges (decode_common.h).  A step of few tokens spends its time on what
+// the cut needs: the prefix over all users, the search, partials, the merge launch and the gap in front of it (us per
+// layer of a replayed step, cut / whole: one user of 8/8 heads at head size 64 over 128 tokens 11.8 / 6.1; eight of
+// 32/8 heads at 128 over 256 tokens 11.8 / 9.2; 37 of 64/8 heads at 64 in a window of 1024 23.1 / 21.8; block-float-8, 24 users of
+// 32/8 heads over 256 / 1024 tokens 16.8 / 10.7 and 23.9 / 17.1; 150 users 38.7 / 33.1 and 77.6 / 69.0).  A CU streams
+// 57 - 60 KB per us whatever the number of its wavefronts, so a whole segment costs 6 us and its
+// bytes at that rate, and a cut one about 11.  How long contexts are only the device knows; the host knows what a
+// user can attend at most, by the window and by the width of the page table: up to 272 KB per segment (512 bfloat16 tokens of 128
+// values, 1024 block-float-8 ones) the whole segment is no slower whoever has how much (one user at 256 KB: 11.0 / 10.5;
+// 512 KB: 11.2 / 15.0).  Eight wavefronts hide more of a tile's chain (one user over 1024 block-float-8 tokens 18.2 / 15.2
+// with four / eight), but four leave room for two workgroups on a CU, which more segments than CUs need (296
+// segments of 128 tokens: 10.7 / 14.7); a segment of four tiles has no work for more.
+static int direct_waves(int users, int kv_heads, int head_size, int kv_format, int64_t tokens, bool forced) {
+  const int tile_tokens = 4096 / head_size;
+  const int64_t bytes = tokens * head_size * (kv_format == TTPA_KV_BFP8 ? 2 : 4);
+  if (!forced && bytes > 272 * 1024) return 0;
+  int cus = device_cus();
+  if (cus <= 0) cus = 256;
+  return (int64_t)users * kv_heads > cus || tokens <= 4 * tile_tokens ? 4 : 8;
+}
+
 // wavefronts per CU of the largest grid a decode launch uses (the VALU kernel on a block-float-8 cache)
 static constexpr double kLargestGrid = 8.0;
 
@@ -453,26 +475,31 @@ static int decode_impl(void *out, int64_t out_user_stride, int64_t out_head_stri
   // heads), 32x32x16 kernel for wider groups (up to 32 heads), VALU kernel for the rest.  The block-float-8 cache goes to a matrix-core kernel
   // whenever one applies: there the byte expansion costs one VALU operation per element and the
   // products none, while the VALU kernel pays for both.
-  // TTPA_DECODE_KERNEL=valu|mfma|mfma16 overrides the choice.
+  // TTPA_DECODE_KERNEL=valu|mfma|mfma16|ranges|direct overrides the choice (the last two: the 16x16x32 kernel on
+  // ranges, or with one workgroup per segment whatever its length).
   // read on every call (a getenv is negligible next to a launch) so that a process can
   // exercise every kernel
   const char *forced_name = getenv("TTPA_DECODE_KERNEL");
   const int forced = !forced_name ? 0
                      : !strcmp(forced_name, "valu") ? 1
                      : !strcmp(forced_name, "mfma") ? 2
-                     : !strcmp(forced_name, "mfma16") ? 3 : 0;
+                     : !strcmp(forced_name, "mfma16") ? 3
+                     : !strcmp(forced_name, "ranges") ? 4
+                     : !strcmp(forced_name, "direct") ? 5 : 0;
   const bool mfma_ok = mfma_decode_supported(a, head_size, g);
   const bool mfma16_ok = mfma16_decode_supported(a, head_size, g);
-  // As a step (update + attention) the 16x16x32 kernel with the update inside already wins at 2
-  // and 3 heads per group (1 - 6 % and 2 - 11 % per step against update launch + VALU kernel; at
-  // 1 head the two are within 2.5 % of each other either way).
-  const int g_min16 = k_new ? 2 : 4;
+  // As a step (update + attention) the 16x16x32 kernel with the update inside wins at any group width
+  // (1 - 6 % and 2 - 11 % per step at 2 and 3 heads against update launch + VALU kernel; at 1 head, us per layer of a
+  // replayed step, head size 128: one user over 1024 tokens 12.9 -> 11.4, 32 users with 512 ... 4096 81.8 -> 78.0, 150
+  // with 512 ... 2048 228 -> 220; head size 64: 12.3 -> 11.1, 30.3 -> 26.6, 67.9 -> 64.4).
+  // The attention alone with one head per group goes the same way, so that a step gives what its operators give in turn.
+  const int g_min16 = k_new || g == 1 ? 1 : 4;
   bool use_mfma16 = mfma16_ok && (g >= g_min16 || kv_format == TTPA_KV_BFP8 || head_size == 256);
   bool use_mfma = !use_mfma16 && mfma_ok && (g >= 5 || kv_format == TTPA_KV_BFP8);
   // a forced kernel that is not built for the shape leaves the default choice in place
   if (forced == 1 && g <= 8 && !(kv_format == TTPA_KV_BFP8 && head_size == 256)) use_mfma = use_mfma16 = false;
   if (forced == 2 && mfma_ok) use_mfma = true, use_mfma16 = false;
-  if (forced == 3 && mfma16_ok) use_mfma16 = true, use_mfma = false;
+  if (forced >= 3 && mfma16_ok) use_mfma16 = true, use_mfma = false;
   if (mask) {
     // A mask is applied by the dot-product kernel (bfloat16 caches, up to 8 heads per group) and by
     // the matrix-core kernels (either format; 16x16x32 up to 16 heads, 32x32x16 up to 32); a forced
@@ -483,12 +510,22 @@ static int decode_impl(void *out, int64_t out_user_stride, int64_t out_head_stri
                   "masked decode: %d query heads per KV head with this cache format, head size and block size is not "
                   "built (bfloat16 up to 8, or up to 32 on the matrix-core kernels' shapes)", g);
     if (forced == 2 && mfma_ok) use_mfma = true, use_mfma16 = false;
-    else if (forced == 3 && mfma16_ok) use_mfma = false, use_mfma16 = true;
+    else if (forced >= 3 && mfma16_ok) use_mfma = false, use_mfma16 = true;
     else if (forced == 1 && valu_ok) use_mfma = use_mfma16 = false;
     else {
       use_mfma16 = mfma16_ok && (g >= 4 || !valu_ok);
       use_mfma = !use_mfma16 && !valu_ok;
     }
+  }
+  // A step whose new rows cannot be read in 16-byte pieces is an update launch and the attention behind it.
+  const bool vec_ok = !k_new || (aligned16(k_new) && aligned16(v_new) && new_user_stride % 8 == 0 && new_head_stride % 8 == 0);
+  // (an explicit grid asks for ranges)
+  if (!mask && mfma16_ok && head_size <= 128 && block_size % (4096 / head_size / 2) == 0 &&
+      (forced == 5 || ((forced == 0 || forced == 3) && !getenv("TTPA_DECODE_WAVES_PER_CU")))) {
+    int64_t tokens = (int64_t)table_width * block_size;
+    if (sliding_window > 0) tokens = std::min<int64_t>(tokens, sliding_window);
+    a.direct = direct_waves(users, kv_heads, head_size, kv_format, tokens, forced == 5);
+    if (a.direct) use_mfma16 = true, use_mfma = false;
   }
   // The matrix-core kernels get at most one workgroup per CU whatever the cache format: the 32x32
   // kernel fills the CU's LDS with one, and the 16x16 kernel streams as fast with one as with the
@@ -513,14 +550,12 @@ static int decode_impl(void *out, int64_t out_user_stride, int64_t out_head_stri
   // 0 / 1 / 2).  TTPA_DECODE_SEG_UNITS (read on every call) overrides.
   a.seg_units = segment_units(use_mfma16 ? 1 : use_mfma ? 2 : 0);
   // one thread of the main grid per segment publishes the segment's partial slots
-  if ((int64_t)users * kv_heads > (int64_t)a.n_waves * kWave)
+  if (!a.direct && (int64_t)users * kv_heads > (int64_t)a.n_waves * kWave)
     return fail(TTPA_ERR_UNSUPPORTED, "decode: %d x %d segments need a grid of more than %d wavefronts",
                 users, kv_heads, a.n_waves);
   if (k_new) {
     // The step's cache update: inside the 16x16 kernel when that is the kernel of this shape,
     // as a launch of its own in front of the attention otherwise.
-    const bool vec_ok = aligned16(k_new) && aligned16(v_new) && new_user_stride % 8 == 0 &&
-                        new_head_stride % 8 == 0;
     if (use_mfma16 && vec_ok) {
       a.k_new = static_cast<const uint16_t *>(k_new);
       a.v_new = static_cast<const uint16_t *>(v_new);
@@ -555,6 +590,7 @@ static int decode_impl(void *out, int64_t out_user_stride, int64_t out_head_stri
   if (ev1) (void)hipEventRecord(ev1, st);
   if (use_mfma16) take_profile_events(ev0, ev1);  // still armed only if the launch did not happen
   if (rc) return rc;
+  if (a.direct) return check_launch("paged_sdpa_decode");
   if (a.k_new) launch_combine<true>(a, users * kv_heads, g, head_size, st);
   else launch_combine(a, users * kv_heads, g, head_size, st);
   return check_launch("paged_sdpa_decode");

@@ -75,9 +75,11 @@ constexpr int kMaxUsers16 = kMaxUsers;  // the library-wide limit: 16 KiB of pre
 // The block-float-8 cache moves half the bytes per token and loses with the shorter tile where there is
 // much to read (head size 128, 64 users with 1024 ... 16384 tokens: 138 -> 150 us; head size 64, 100 users
 // with 1024 ... 8192: 78 -> 84), and how much there is only the device knows.
-template <int D, bool BFP8>
+// With one workgroup per segment (DIRECT) the short tile for both formats: the wavefronts of a workgroup
+// take the tiles in turn, so a short context reaches more of them, and two wavefronts share a SIMD's registers.
+template <int D, bool BFP8, int DIRECT = 0>
 constexpr int tile_bytes() {
-  return (D <= 128 && !BFP8) ? 8192 : 16384;
+  return (D <= 128 && (!BFP8 || DIRECT)) ? 8192 : 16384;
 }
 
 template <bool F16>
@@ -90,13 +92,73 @@ __device__ __forceinline__ floatx4 mma16(const u32x4 &x, const u32x4 &y, const f
                                                    __builtin_bit_cast(bf16x8, y), c, 0, 0, 0);
 }
 
+// The end of a segment that one workgroup of WAVES wavefronts has read (`active` of them had a tile): the
+// wavefronts' results meet in LDS, each in its own tile buffer, whose last tile it has consumed; then every
+// thread merges, normalises and stores four neighbouring elements of a head.  A wavefront's values lie as
+// its lanes hold them, [element / 4][head][4], so its stores are 1 KiB in a row.
+template <int D, int WAVES>
+__device__ __forceinline__ void merge_waves(const DecodeArgs &a, int u, int h, int G, int active, uint8_t *own, const uint8_t *all,
+                                            int pitch, const floatx4 (&acc)[D / 16], float vout, float m, float l) {
+  __shared__ float s_m[WAVES][16], s_l[WAVES][16];
+  const int lane = threadIdx.x & 63, wib = threadIdx.x >> 6;
+  if (wib < active) {
+#pragma unroll
+    for (int db = 0; db < D / 16; ++db)
+      *reinterpret_cast<float4 *>(own + db * 1024 + lane * 16) =
+          make_float4(acc[db][0] * vout, acc[db][1] * vout, acc[db][2] * vout, acc[db][3] * vout);
+    if (lane < 16) s_m[wib][lane] = m, s_l[wib][lane] = l;
+  }
+  __syncthreads();
+  const int gshift = G <= 1 ? 0 : 32 - __builtin_clz(G - 1);
+  const bool wide_stores = ((a.out_us | a.out_hs) & 3) == 0;
+  for (int i = threadIdx.x; i < (D / 4) << gshift; i += kWave * WAVES) {
+    const int g = i & ((1 << gshift) - 1), d4 = i >> gshift;
+    if (g >= G) continue;
+    float mall = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w)
+      if (w < active) mall = fmaxf(mall, s_m[w][g]);
+    const float ref = merge_reference(mall);
+    float num[4] = {0.f, 0.f, 0.f, 0.f}, den = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w)
+      if (w < active) {
+        const float wgt = __builtin_amdgcn_exp2f(s_m[w][g] - ref);
+        const float4 x = *reinterpret_cast<const float4 *>(all + w * pitch + d4 * 256 + g * 16);
+        num[0] = fmaf(wgt, x.x, num[0]), num[1] = fmaf(wgt, x.y, num[1]);
+        num[2] = fmaf(wgt, x.z, num[2]), num[3] = fmaf(wgt, x.w, num[3]);
+        den = fmaf(wgt, s_l[w][g], den);
+      }
+    if (a.sink) {  // the sink logit (natural-log units, not scaled) only enlarges the normaliser
+      const float sk = a.sink[h * G + g] * 1.4426950408889634f;
+      const float mnew = fmaxf(mall, sk);
+      const float resc = __builtin_amdgcn_exp2f(mall - mnew);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) num[r] *= resc;
+      den = den * resc + __builtin_amdgcn_exp2f(sk - mnew);
+    }
+    uint16_t *dst = a.out + u * a.out_us + (int64_t)(h * G + g) * a.out_hs + 4 * d4;
+    uint32_t b[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) b[r] = f32_to_bf16_bits(num[r] / den);
+    if (wide_stores) {
+      *reinterpret_cast<uint2 *>(dst) = make_uint2(b[0] | (b[1] << 16), b[2] | (b[3] << 16));
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) dst[r] = (uint16_t)b[r];
+    }
+  }
+}
+
 // RUNS: 1, 2, 4, or 0 for one run per load.  MASKED: an additive mask row per (user, head) joins the
 // scores (a.mask; the form of a pass that is not causal, built with RUNS = 0 and without the update).
-template <int D, bool BFP8, int RUNS, bool FUSED, bool MASKED = false>
-__global__ __launch_bounds__(256, 1) void paged_decode_mfma16_kernel(
+// DIRECT: a workgroup of DIRECT wavefronts owns the whole segment blockIdx.x (chosen by direct_waves, decode.hip): no prefix, no
+// search, no partials, no merge launch.  Its wavefronts take the segment's tiles in turn.
+template <int D, bool BFP8, int RUNS, bool FUSED, bool MASKED = false, int DIRECT = 0>
+__global__ __launch_bounds__(DIRECT ? kWave *DIRECT : 256, DIRECT && D <= 128 ? 2 : 1) void paged_decode_mfma16_kernel(
     DecodeArgs a, const int32_t *__restrict__ page_table, const void *__restrict__ cur_pos) {
   static_assert(D == 64 || D == 128 || D == 256, "shapes built");
-  constexpr int kTileBytes = tile_bytes<D, BFP8>();
+  constexpr int kTileBytes = tile_bytes<D, BFP8, DIRECT>();
   constexpr int TILE = kTileBytes / (2 * D);  // tokens per tile
   constexpr int ROWB = 2 * D;                 // bytes of a tile row in LDS
   constexpr int KSTEPS = D / 32, DBLK = D / 16;
@@ -113,30 +175,46 @@ __global__ __launch_bounds__(256, 1) void paged_decode_mfma16_kernel(
   constexpr int LPO = NL / NOFF;               // loads per run
   static_assert(NL % NOFF == 0, "a run is a whole number of loads");
 
-  __shared__ int s_pref[kMaxUsers16 + 1];
-  __shared__ int s_len[kMaxUsers16];
+  __shared__ int s_pref[DIRECT ? 1 : kMaxUsers16 + 1];
+  __shared__ int s_len[DIRECT ? 1 : kMaxUsers16];
   __shared__ int s_wsum[kWavesPerBlock];
   extern __shared__ __attribute__((aligned(16))) uint8_t tiles[];
 
   const int seg_units = a.seg_units;
-  build_prefix<TILE>(a, cur_pos, s_pref, s_len, s_wsum, seg_units);
-
+  if constexpr (DIRECT == 0) build_prefix<TILE>(a, cur_pos, s_pref, s_len, s_wsum, seg_units);
   const int lane = threadIdx.x & 63;
   const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 15, quad = lane >> 4;
   const int wave = blockIdx.x * kWavesPerBlock + wib;
-  // The flat list in units: per segment `seg_units` units that stand for the cost of opening it,
-  // then its tiles.  A range of more than seg_units units holds at least one tile.
-  const int total_units = __builtin_amdgcn_readfirstlane(s_pref[a.users]);
-  const Share share = share_of(total_units, a.hkv, a.n_waves, seg_units, wave);
-  const int64_t total = share.total;
-  const int n_eff = share.n_eff;
-  if (total == 0 || wave >= n_eff) {
-    publish_segment_row(a, s_pref, total, n_eff, seg_units);
-    return;
+  int64_t total = 0, x_lo = 0, x_hi = 0;
+  int n_eff = 0, n_tiles = 0;
+  Cursor cur;
+  if constexpr (DIRECT > 0) {
+    cur.u = (int)blockIdx.x / a.hkv;
+    cur.h = (int)blockIdx.x - cur.u * a.hkv;
+    n_tiles = tiles_of_user<TILE>(a, cur_pos, cur.u, cur.len);
+    if (n_tiles == 0) {  // a padded row: NaN like softmax over nothing, and the parked token's cache write
+      const int g_all = a.hq / a.hkv;
+      for (int i = threadIdx.x; i < g_all * D; i += kWave * DIRECT)
+        a.out[cur.u * a.out_us + (int64_t)(cur.h * g_all + i / D) * a.out_hs + i % D] = 0x7fc0;
+      if constexpr (FUSED) write_negative_position(a, blockIdx.x, D);
+      return;
+    }
+    cur.lo = window_lo(a, cur.len);
+    cur.t = cur.lo / TILE + wib;
+    cur.tiles_left = n_tiles - wib;
+  } else {
+    // The flat list in units: per segment `seg_units` units that stand for the cost of opening it,
+    // then its tiles.  A range of more than seg_units units holds at least one tile.
+    const int total_units = __builtin_amdgcn_readfirstlane(s_pref[a.users]);
+    const Share share = share_of(total_units, a.hkv, a.n_waves, seg_units, wave);
+    total = share.total, n_eff = share.n_eff;
+    if (total == 0 || wave >= n_eff) {
+      publish_segment_row(a, s_pref, total, n_eff, seg_units);
+      return;
+    }
+    x_lo = share.lo, x_hi = share.hi;
   }
-  const int64_t x_lo = share.lo;
-  const int64_t x_hi = share.hi;
   int64_t x = x_lo;  // set below to the unit of the first tile at or behind x_lo
   uint8_t *tile = tiles + wib * kTileBytes;
   const int G = a.hq / a.hkv;
@@ -335,22 +413,25 @@ __global__ __launch_bounds__(256, 1) void paged_decode_mfma16_kernel(
     }
   };
 
-  Cursor cur = locate_unit<TILE>(a, s_pref, s_len, x_lo, seg_units, &x);
+  if constexpr (DIRECT == 0) cur = locate_unit<TILE>(a, s_pref, s_len, x_lo, seg_units, &x);
   int64_t eo[NOFF], xo[NOFF];
   u32x4 kraw[NL], vraw[NL];
   uint32_t kex[NL], vex[NL];
   u32x4 qf[KSTEPS];
   Fresh kfresh = {}, vfresh = {};
   uint32_t bad_cur = 0;  // the current tile's runs that read block 0 in place of a block out of range
-  tile_offsets(cur, eo, xo, bad_cur);
-  fetch(a.k, eo, xo, kraw, kex);
-  fetch(a.v, eo, xo, vraw, vex);
-  if constexpr (FUSED) {
-    kfresh = fetch_fresh(a.k_new, cur);
-    vfresh = fetch_fresh(a.v_new, cur);
+  const bool works = DIRECT == 0 || cur.tiles_left > 0;  // (a short segment leaves wavefronts without a tile)
+  if (works) {
+    tile_offsets(cur, eo, xo, bad_cur);
+    fetch(a.k, eo, xo, kraw, kex);
+    fetch(a.v, eo, xo, vraw, vex);
+    if constexpr (FUSED) {
+      kfresh = fetch_fresh(a.k_new, cur);
+      vfresh = fetch_fresh(a.v_new, cur);
+    }
+    load_q(cur, qf);
   }
-  load_q(cur, qf);
-  publish_segment_row(a, s_pref, total, n_eff, seg_units);
+  if constexpr (DIRECT == 0) publish_segment_row(a, s_pref, total, n_eff, seg_units);
 
   floatx4 acc[DBLK];
 #pragma unroll
@@ -363,7 +444,7 @@ __global__ __launch_bounds__(256, 1) void paged_decode_mfma16_kernel(
     const int nvalid = cur.len - cur.t * TILE;
     const bool partial = nvalid < TILE;
     const int nbelow = cur.lo - cur.t * TILE;  // sliding window: > 0 only in a segment's first tile
-    const bool same_seg = has_next && cur.tiles_left > 1;
+    const bool same_seg = DIRECT > 0 || (has_next && cur.tiles_left > 1);
     Cursor nxt = cur;
 
     // ---- K: registers -> LDS, then the next tile's K: global -> registers -------------------
@@ -396,8 +477,9 @@ __global__ __launch_bounds__(256, 1) void paged_decode_mfma16_kernel(
     stage(false, kraw, kex, eref_k, nvalid, false);
     if constexpr (has_next) {
       if (same_seg) {
-        nxt.t = cur.t + 1;
-        nxt.tiles_left = cur.tiles_left - 1;
+        constexpr int kStep = DIRECT > 0 ? DIRECT : 1;
+        nxt.t = cur.t + kStep;
+        nxt.tiles_left = cur.tiles_left - kStep;
       } else {
         nxt = locate(x + 1);
       }
@@ -489,10 +571,10 @@ __global__ __launch_bounds__(256, 1) void paged_decode_mfma16_kernel(
         for (int r = 0; r < 4; r += 2) {
           const float p0 = __builtin_amdgcn_exp2f(fmaf(st[b][r], scale, -m_safe));
           const float p1 = __builtin_amdgcn_exp2f(fmaf(st[b][r + 1], scale, -m_safe));
-          const floatx2 pp = {p0, p1};
-          const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(pp, bf16x2));
+          const uint32_t w = pack_bf16x2(p0, p1);
           lsum += bf16_lo(w) + bf16_hi(w);  // the normaliser sums the weights that multiply V
           pf[b >> 1][2 * (b & 1) + (r >> 1)] = w;
+          st[b][r] = p0 - bf16_lo(w), st[b][r + 1] = p1 - bf16_hi(w);  // what the rounding took
         }
     }
     l_run = l_run * alpha + lsum;
@@ -501,17 +583,38 @@ __global__ __launch_bounds__(256, 1) void paged_decode_mfma16_kernel(
       for (int i = 0; i < DBLK; ++i) acc[i] *= alpha_acc;
     }
     // ---- O^T += V^T . P^T ------------------------------------------------------------------------
+    auto second_product = [&]() {
 #pragma unroll
-    for (int s = 0; s < PSTEPS; ++s)
+      for (int s = 0; s < PSTEPS; ++s)
 #pragma unroll
-      for (int db = 0; db < DBLK; ++db) {
-        typedef __attribute__((address_space(3))) shortx4 *lds_v4;
-        const uint8_t *vp = tile + vr[db] + s * (32 * ROWB);
-        shortx4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4)(vp));
-        shortx4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4)(vp + 16 * ROWB));
-        const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
-        acc[db] = mma16<BFP8>(u32x4{l2.x, l2.y, h2.x, h2.y}, pf[s], acc[db]);
+        for (int db = 0; db < DBLK; ++db) {
+          typedef __attribute__((address_space(3))) shortx4 *lds_v4;
+          const uint8_t *vp = tile + vr[db] + s * (32 * ROWB);
+          shortx4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4)(vp));
+          shortx4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4)(vp + 16 * ROWB));
+          const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
+          acc[db] = mma16<BFP8>(u32x4{l2.x, l2.y, h2.x, h2.y}, pf[s], acc[db]);
+        }
+    };
+    second_product();
+    // One query head per KV head: the weights in two bfloat16 parts.  The dot-product kernel, which serves such groups
+    // otherwise, keeps a running maximum per sixteen of a tile's tokens, so more of its weights are exact; rounded once, this
+    // kernel's results were 4 - 7 % further from a 64-bit evaluation than that one's (2.09e-3 against 1.97e-3, 128 tokens of 8 / 8
+    // heads), in two parts they are 15 - 17 % closer (1.66e-3).
+    if constexpr (!BFP8) {
+      if (G == 1) {
+        float low = 0.f;
+#pragma unroll
+        for (int b = 0; b < KBLK; ++b)
+#pragma unroll
+          for (int r = 0; r < 4; r += 2) {
+            low += st[b][r] + st[b][r + 1];
+            pf[b >> 1][2 * (b & 1) + (r >> 1)] = pack_bf16x2(st[b][r], st[b][r + 1]);
+          }
+        l_run += low;
+        second_product();
       }
+    }
 
     // ---- close the segment --------------------------------------------------------------------
     if (!same_seg) {
@@ -545,22 +648,38 @@ __global__ __launch_bounds__(256, 1) void paged_decode_mfma16_kernel(
     cur = nxt;
     x += same_seg ? 1 : 1 + seg_units;
   };
+  if constexpr (DIRECT > 0) {
+    if (works) {
+      while (cur.tiles_left > DIRECT) process_tile(std::true_type{});
+      process_tile(std::false_type{});
+    }
+    merge_waves<D, DIRECT>(a, cur.u, cur.h, G, std::min(n_tiles, DIRECT), tile, tiles, kTileBytes, acc,
+                           BFP8 ? __builtin_ldexpf(1.f, ev_run - 133) : 1.f, m_run, sum_over_quads(l_run));
+    return;
+  }
   // the unit of the tile behind the current one: the next, or behind the next segment's leading units
   auto next_tile_unit = [&]() { return x + (cur.tiles_left > 1 ? 1 : 1 + seg_units); };
   while (next_tile_unit() < x_hi) process_tile(std::true_type{});
   process_tile(std::false_type{});
 }
 
-template <int D, bool BFP8, int RUNS, bool FUSED, bool MASKED = false>
+template <int D, bool BFP8, int RUNS, bool FUSED, bool MASKED = false, int DIRECT = 0>
 bool launch(const DecodeArgs &a, hipStream_t st) {
-  const int blocks = a.n_waves / kWavesPerBlock;
-  const size_t lds = (size_t)kWavesPerBlock * tile_bytes<D, BFP8>();
+  constexpr int kWaves = DIRECT ? DIRECT : kWavesPerBlock;
+  const int blocks = DIRECT ? a.users * a.hkv : a.n_waves / kWavesPerBlock;
+  const size_t lds = (size_t)kWaves * tile_bytes<D, BFP8, DIRECT>();
   static std::atomic<uint64_t> lds_ready{0};
-  if (!ensure_dynamic_lds(reinterpret_cast<const void *>(&paged_decode_mfma16_kernel<D, BFP8, RUNS, FUSED, MASKED>), lds,
-                          lds_ready))
-    return false;
-  launch_dominant(&paged_decode_mfma16_kernel<D, BFP8, RUNS, FUSED, MASKED>, dim3(blocks), dim3(256), lds, st, a, a.pt, a.cur);
+  const auto kernel = &paged_decode_mfma16_kernel<D, BFP8, RUNS, FUSED, MASKED, DIRECT>;
+  if (!ensure_dynamic_lds(reinterpret_cast<const void *>(kernel), lds, lds_ready)) return false;
+  launch_dominant(kernel, dim3(blocks), dim3(kWave * kWaves), lds, st, a, a.pt, a.cur);
   return true;
+}
+
+// One workgroup per segment (a.direct).
+template <int D, bool BFP8, bool FUSED, int DIRECT>
+bool launch_direct(const DecodeArgs &a, hipStream_t st) {
+  constexpr int TILE = tile_bytes<D, BFP8, DIRECT>() / (2 * D);
+  return a.bs % TILE == 0 ? launch<D, BFP8, 1, FUSED, false, DIRECT>(a, st) : launch<D, BFP8, 2, FUSED, false, DIRECT>(a, st);
 }
 
 // Picks the variant for the block size and for a.k_new (set: the launch also performs the
@@ -569,6 +688,10 @@ template <int D, bool BFP8>
 bool launch_for_block_size(const DecodeArgs &a, hipStream_t st) {
   constexpr int TILE = tile_bytes<D, BFP8>() / (2 * D);
   const bool fused = a.k_new != nullptr;
+  if constexpr (D <= 128) {
+    if (a.direct == 4) return fused ? launch_direct<D, BFP8, true, 4>(a, st) : launch_direct<D, BFP8, false, 4>(a, st);
+    if (a.direct == 8) return fused ? launch_direct<D, BFP8, true, 8>(a, st) : launch_direct<D, BFP8, false, 8>(a, st);
+  }
   if (a.mask != nullptr) return !fused && launch<D, BFP8, 0, false, true>(a, st);
   if (a.bs % TILE == 0) return fused ? launch<D, BFP8, 1, true>(a, st) : launch<D, BFP8, 1, false>(a, st);
   if (a.bs % (TILE / 2) == 0) return fused ? launch<D, BFP8, 2, true>(a, st) : launch<D, BFP8, 2, false>(a, st);
