@@ -546,6 +546,27 @@ int ttpa_latent_decode_step_strided(void *out, int64_t out_user_stride, int64_t 
                                     size_t workspace_bytes, void *stream);
 
 /*
+ * The causal prompt pass of a latent layer in one call (reference attention_mla.py:230-359: new tokens' latent keys into the
+ * cache, attention of the prompt over itself, output expansion) for the same head shape, users x seq_len tokens (a
+ * multiple of 32).  Up to 64 tokens per user in the absorbed form, as the step; longer prompts with
+ * k[t, n] = latent[t] . W_UK[n] and v[t, n] = latent[t] . W_UV[n] rounded to bfloat16 and ttpa_split_key_prefill over them.
+ * Activations and out [tokens, heads, part] by token and head strides (multiples of 8 elements, the latent's below 2^23),
+ * weights as in ttpa_latent_decode_step_strided (strides below 2^23), 16-byte aligned pointers.  cache null: nothing is
+ * written; otherwise row t of user u goes to position t of page-table row u, rows and blocks out of range are skipped.
+ * Two or three launches; the scratch (256-byte aligned, the size below) holds nothing between calls.
+ */
+int ttpa_latent_prompt(void *out, int64_t out_token_stride, int64_t out_head_stride, const void *q_nope,
+                       int64_t q_nope_token_stride, int64_t q_nope_head_stride, const void *q_rope,
+                       int64_t q_rope_token_stride, int64_t q_rope_head_stride, const void *latent,
+                       int64_t latent_token_stride, const void *rope, int64_t rope_token_stride, const void *w_uk,
+                       int64_t w_uk_head_stride, int64_t w_uk_row_stride, int64_t w_uk_column_stride, const void *w_uv,
+                       int64_t w_uv_head_stride, int64_t w_uv_row_stride, int64_t w_uv_column_stride, void *cache,
+                       const int32_t *page_table, int64_t page_table_row_stride, int32_t users, int32_t table_rows,
+                       int32_t heads, int32_t seq_len, int32_t block_size, int32_t table_width, int32_t num_blocks,
+                       float scale, void *workspace, int64_t workspace_bytes, void *stream);
+int64_t ttpa_latent_prompt_workspace_bytes(int32_t users, int32_t heads, int32_t seq_len);
+
+/*
  * paged_fill_cache of latent rows that are still in two parts: row t of user u, [latent_size] from `latent` and
  * [rope_size] from `rope` behind it, goes to position t of page-table row u in a cache
  * [num_blocks, 1, block_size, latent_size + rope_size] (what the latent backend builds with a concatenation and

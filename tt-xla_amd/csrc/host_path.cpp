@@ -223,7 +223,124 @@ PyObject *attention_pass(PyObject *, PyObject *const *v, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// A weight [heads, rows, columns] as the latent kernels read it: rows or columns contiguous, every other stride whole
+// 16-byte pieces, aligned.
+const at::Tensor *weight(const Pass &p, PyObject *o, int64_t heads, int64_t rows, int64_t columns) {
+  const at::Tensor *t = p.plain(o);
+  if (!t || t->scalar_type() != at::kBFloat16 || t->dim() != 3 || t->size(0) != heads || t->size(1) != rows || t->size(2) != columns) return nullptr;
+  const int64_t rs = t->stride(1), cs = t->stride(2), other = cs == 1 ? rs : cs;
+  if ((rs != 1 && cs != 1) || t->stride(0) % 8 || other % 8 || other <= 0 || other >= (1 << 23) || reinterpret_cast<uintptr_t>(t->data_ptr()) % 16)
+    return nullptr;
+  return t;
+}
+
+// latent_pass(q_nope, q_rope, latent, rope, cache, page_table, cache_position, fill_page_table, w_uk_t, w_uv, output, heads, scale,
+//             workspace)
+// The pass of a latent layer (128 + 64 query features, latent width 512, values of 128; causal): decode step or prompt.
+// -> as attention_pass.  workspace(bytes, device) is the operators' own scratch of a decode step, which is sized for the
+// largest grid and not for the pass.
+PyObject *latent_pass(PyObject *, PyObject *const *v, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 14) {
+    PyErr_SetString(PyExc_TypeError, "latent_pass takes 14 arguments");
+    return nullptr;
+  }
+  if (c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled() ||
+      at::tracer::impl::is_dispatch_enabled())
+    Py_RETURN_NONE;
+  if (!THPVariable_CheckExact(v[0]) || !THPVariable_Unpack(v[0]).is_cuda()) Py_RETURN_NONE;  // (ahead of any question to the device)
+  if (!PyLong_Check(v[11]) || !PyFloat_Check(v[12])) Py_RETURN_NONE;
+  const int64_t heads = PyLong_AsLongLong(v[11]);
+  const float scale = (float)PyFloat_AsDouble(v[12]);
+  if (PyErr_Occurred()) {  // a number that does not fit 64 bits
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
+  if (heads <= 0 || heads > 65535) Py_RETURN_NONE;
+  const Pass p{(int)c10::hip::current_device(), at::GradMode::is_enabled()};
+  // [tokens, heads, width] with contiguous, 16-byte aligned rows
+  const auto parts = [&](PyObject *o, int64_t per_token, int64_t width) -> const at::Tensor * {
+    const at::Tensor *t = p.plain(o);
+    return t && t->scalar_type() == at::kBFloat16 && t->dim() == 3 && t->size(1) == per_token && t->size(2) == width && t->stride(2) == 1 &&
+                   t->stride(0) % 8 == 0 && t->stride(1) % 8 == 0 && reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0
+               ? t
+               : nullptr;
+  };
+  const at::Tensor *qn = parts(v[0], heads, 128), *qr = parts(v[1], heads, 64), *lat = p.rows(v[2], 512), *rope = parts(v[3], 1, 64);
+  if (!qn || !qr || !lat || !rope) Py_RETURN_NONE;
+  const int64_t tokens = qn->size(0);
+  if (tokens == 0 || qr->size(0) != tokens || lat->size(0) != tokens || rope->size(0) != tokens) Py_RETURN_NONE;
+  const at::Tensor *pos = p.plain(v[6]);
+  if (!pos || pos->dim() != 1 || pos->size(0) == 0 || tokens % pos->size(0)) Py_RETURN_NONE;
+  const int64_t users = pos->size(0), s = tokens / users;
+  const at::Tensor *cache = p.plain(v[4]);
+  if (!cache || cache->scalar_type() != at::kBFloat16 || cache->dim() != 4 || cache->size(0) == 0 || cache->size(1) != 1 || cache->size(2) == 0 ||
+      cache->size(3) != 576 || !cache->is_contiguous() || reinterpret_cast<uintptr_t>(cache->data_ptr()) % 16)
+    Py_RETURN_NONE;
+  const int64_t nb = cache->size(0), bs = cache->size(2);
+  const at::Tensor *uk = weight(p, v[8], heads, 128, 512), *uv = weight(p, v[9], heads, 512, 128), *out = p.plain(v[10]);
+  if (!uk || !uv || !out || out->scalar_type() != at::kBFloat16 || !out->is_contiguous() || out->numel() != tokens * heads * 128) Py_RETURN_NONE;
+  // (an output that the kernels' stores cannot take is copied to)
+  const bool storable = reinterpret_cast<uintptr_t>(out->data_ptr()) % 16 == 0;
+  void *stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)p.device).stream();
+
+  if (s == 1) {
+    const at::Tensor *pt = p.table(v[5]);
+    pos = p.numbers(v[6], users);
+    if (!pt || pt->size(0) != users || pt->size(1) == 0 || !pos || users > 1024) Py_RETURN_NONE;
+    const size_t bytes = ttpa_latent_decode_step_workspace_bytes((int32_t)users, (int32_t)heads);
+    if (bytes == 0) Py_RETURN_NONE;
+    PyObject *const device = PyObject_GetAttrString(v[10], "device");
+    if (!device) return nullptr;
+    PyObject *const kept = PyObject_CallFunction(v[13], "nO", (Py_ssize_t)bytes, device);
+    Py_DECREF(device);
+    if (!kept) return nullptr;
+    const at::Tensor ws = THPVariable_Check(kept) ? THPVariable_Unpack(kept) : at::Tensor();
+    Py_DECREF(kept);
+    if (!ws.defined() || !ws.is_cuda() || ws.get_device() != p.device || ws.nbytes() < bytes) Py_RETURN_NONE;
+    RECORD_FUNCTION("tt::latent_decode_step_", std::vector<c10::IValue>());
+    written(cache), written(out);
+    const auto launch = [&] {
+      const Unlocked unlocked;
+      const at::Tensor target = storable ? *out : at::empty(out->sizes(), out->options());
+      const int rc = ttpa_latent_decode_step_strided(
+          target.data_ptr(), heads * 128, 128, qn->data_ptr(), qn->stride(0), qn->stride(1), qr->data_ptr(), qr->stride(0), qr->stride(1),
+          lat->data_ptr(), lat->stride(0), rope->data_ptr(), rope->stride(0), uk->data_ptr(), uk->stride(0), uk->stride(1), uk->stride(2),
+          uv->data_ptr(), uv->stride(0), uv->stride(1), uv->stride(2), cache->data_ptr(), static_cast<const int32_t *>(pt->data_ptr()),
+          pt->stride(0), pos->data_ptr(), is_i64(pos), (int32_t)users, (int32_t)heads, (int32_t)bs, (int32_t)pt->size(1), (int32_t)nb, scale,
+          ws.data_ptr(), bytes, stream);
+      if (!storable && rc == TTPA_OK) out->copy_(target);
+      return rc;
+    };
+    return result("ttpa_latent_decode_step_strided", launch());
+  }
+
+  const at::Tensor *fill = p.table(v[7]);
+  if (!(scale > 0.f) || s % 32 || !fill || fill->size(0) == 0 || s > fill->size(1) * bs || lat->stride(0) <= 0 || lat->stride(0) >= (1 << 23))
+    Py_RETURN_NONE;
+  const int64_t bytes = ttpa_latent_prompt_workspace_bytes((int32_t)users, (int32_t)heads, (int32_t)s);
+  if (tokens > 65535 * 32 || bytes <= 0 || bytes > kScratchLimit) Py_RETURN_NONE;
+  RECORD_FUNCTION("tt::latent_prompt", std::vector<c10::IValue>());
+  written(cache), written(out);
+  const auto launch = [&] {
+    const Unlocked unlocked;
+    const at::Tensor ws = scratch(bytes, out), target = storable ? *out : at::empty(out->sizes(), out->options());
+    const int rc = ttpa_latent_prompt(
+        target.data_ptr(), heads * 128, 128, qn->data_ptr(), qn->stride(0), qn->stride(1), qr->data_ptr(), qr->stride(0), qr->stride(1),
+        lat->data_ptr(), lat->stride(0), rope->data_ptr(), rope->stride(0), uk->data_ptr(), uk->stride(0), uk->stride(1), uk->stride(2),
+        uv->data_ptr(), uv->stride(0), uv->stride(1), uv->stride(2), cache->data_ptr(), static_cast<const int32_t *>(fill->data_ptr()),
+        fill->stride(0), (int32_t)users, (int32_t)fill->size(0), (int32_t)heads, (int32_t)s, (int32_t)bs, (int32_t)fill->size(1), (int32_t)nb,
+        scale, ws.data_ptr(), bytes, stream);
+    if (!storable && rc == TTPA_OK) out->copy_(target);
+    return rc;
+  };
+  return result("ttpa_latent_prompt", launch());
+  END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef methods[] = {
+    {"latent_pass", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(latent_pass)), METH_FASTCALL,
+     "One pass of a latent layer from its tensors; None if it is not an ordinary one."},
     {"attention_pass", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(attention_pass)), METH_FASTCALL,
      "One pass of an attention layer from its tensors; None if it is not an ordinary one."},
     {nullptr, nullptr, 0, nullptr}};

@@ -20,9 +20,16 @@
 // heads 83.2 -> 52.0 and 81.1 -> 48.4; with rows contiguous 26.7, 78.8 and 49.9.)  128 users, 16 heads: 8.2 and 5.0 us, where two
 // batched library products, two concatenations, the cache write and the copy to the output took 41 us in six
 // launches; the whole pass over contexts of 512 .. 8192 168 -> 94 us, of one user over 512 tokens 149 -> 37 us.
+//
+// And the prompt pass of a latent layer in one call.  Up to 64 tokens in the absorbed form (two kernels of the step around
+// ttpa_latent_prefill, with the tokens as users), longer ones with K and V expanded per head:
+//
+//   latent_expand_kernel  k[t, n] = latent[t] . W_UK[n], v[t, n] = latent[t] . W_UV[n], and the prompt's rows go into the cache
+//   ttpa_split_key_prefill over (k, rope) and v
 #include "common.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace ttpa {
 namespace {
@@ -30,6 +37,7 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef short shortx4 __attribute__((ext_vector_type(4)));
+typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
 
 constexpr int kNope = 128, kRope = 64, kLatent = 512, kValue = 128;
 constexpr int kRow = kLatent + kRope;
@@ -48,7 +56,18 @@ struct StepArgs {
   const void *pos;
   int pos_i64;
   int users, heads, bs, w, nb;
+  // prompt: the rows are tokens, `seq` to a user, and belong to positions 0 .. seq - 1 of the users' table rows
+  int seq, table_rows;
+  uint16_t *k_lat;  // [rows][kRow]
 };
+
+// Block and row of the cache for row v of a prompt pass (the fill's rule); false: outside the table or the cache.
+__device__ __forceinline__ bool prompt_slot(const StepArgs &a, int v, int &phys, int &row) {
+  const int u = v / a.seq, t = v - u * a.seq, col = t / a.bs;
+  if (!a.cache || u >= a.table_rows) return false;
+  phys = a.pt[u * a.pt_rs + col], row = t - col * a.bs;
+  return (unsigned)phys < (unsigned)a.nb;
+}
 
 // A operand of a 32x32x16 instruction from rows 16 s .. 16 s + 15 (k) and 32 columns (m) of a weight tile in LDS:
 // lane (m, h) receives column m of rows 8 h .. 8 h + 7.  `first` addresses the lane's 8 bytes of rows
@@ -70,8 +89,9 @@ __device__ __forceinline__ void load_columns(bf16x8 (&w)[8], const uint16_t *col
   for (int s = 0; s < 8; ++s) w[s] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(column + 16 * s));
 }
 
-// COLUMNS: the weight's contracted dimension is contiguous (else its columns are).
-template <bool COLUMNS>
+// COLUMNS: the weight's contracted dimension is contiguous (else its columns are).  PROMPT: the rows' latent keys go to a.k_lat
+// as well, in one piece for the attention.
+template <bool COLUMNS, bool PROMPT = false>
 __global__ __launch_bounds__(256) void latent_query_kernel(StepArgs a) {
   __shared__ __attribute__((aligned(1024))) unsigned char tile[COLUMNS ? 1024 : kNope * 256];  // 128 rows of 128 columns
   const int col0 = blockIdx.x * 128, head = blockIdx.y, u0 = blockIdx.z * kUsers;
@@ -112,10 +132,16 @@ __global__ __launch_bounds__(256) void latent_query_kernel(StepArgs a) {
     for (int i = tid; i < kUsers * chunks; i += 256) {
       const int v = u0 + i / chunks, c = i % chunks;
       int phys, row;
-      if (v >= a.users || !update_slot(a.pos, a.pos_i64, a.pt, a.pt_rs, a.bs, a.w, a.nb, v, phys, row)) continue;
+      if (v >= a.users) continue;
+      if (!PROMPT && !update_slot(a.pos, a.pos_i64, a.pt, a.pt_rs, a.bs, a.w, a.nb, v, phys, row)) continue;
       const int at = c < 16 ? col0 + 8 * c : kLatent + 8 * (c - 16);
       const uint16_t *src = c < 16 ? a.latent + v * a.latent_us + at : a.rope + v * a.rope_us + 8 * (c - 16);
-      *reinterpret_cast<uint4 *>(a.cache + ((int64_t)phys * a.bs + row) * kRow + at) = *reinterpret_cast<const uint4 *>(src);
+      const uint4 piece = *reinterpret_cast<const uint4 *>(src);
+      if constexpr (PROMPT) {
+        *reinterpret_cast<uint4 *>(a.k_lat + (int64_t)v * kRow + at) = piece;
+        if (!prompt_slot(a, v, phys, row)) continue;
+      }
+      *reinterpret_cast<uint4 *>(a.cache + ((int64_t)phys * a.bs + row) * kRow + at) = piece;
     }
   }
   if constexpr (!COLUMNS) {
@@ -195,6 +221,163 @@ __global__ __launch_bounds__(256) void latent_value_kernel(StepArgs a) {
     t.x += x.x, t.y += x.y, t.z += x.z, t.w += x.w;
   }
   *reinterpret_cast<uint2 *>(a.out + (u0 + v) * a.out_us + head * a.out_hs + col0 + c) = make_uint2(pack_bf16x2(t.x, t.y), pack_bf16x2(t.z, t.w));
+}
+
+// K and V of a prompt, expanded per head, and the fill of the cache in the same launch (34 GFLOP at 8192 tokens of 16 heads, 75 MB
+// moved: 52 us, where two library products, a copy of W_UV, the fill and the gaps between them took 61).  Bound by the way of the
+// operands from L2 into LDS, about 44 bytes per ns and CU: without its products the launch takes 45 us.  A workgroup
+// computes 128 tokens x the 128 features of K or of V of a head, in steps of 32 latent values; both operands travel
+// memory -> LDS directly, 16 KiB per step, in a ring of four steps, one barrier per step; 64 KiB, so two workgroups share a CU.  A
+// half step's fragments are read while the products of the half before run.  A wavefront takes 64 x 64 as 2 x 2
+// v_mfma_f32_32x32x16_bf16 tiles, features as rows, tokens as columns; the results meet in LDS so that stores are whole rows (57 us
+// with 16 bytes per row and store).  Workgroups are ordered weights first: with the round-robin deal an XCD's L2 holds an
+// eighth of the weights, and the tokens pass through it.  Not better: 256 tokens x K and V per workgroup, with half the bytes
+// (49 us, but one workgroup per CU: 20 against 14 us for a pass of 96 tokens), and two workgroups per CU that go
+// through their items without emptying the ring (56 us).
+struct ExpandArgs {
+  StepArgs s;                // latent, rope, weights, cache, table, rows (users), seq
+  uint16_t *k, *v;           // [rows][heads][128]
+  int uk_rows, uv_rows;      // the weight's contracted dimension is contiguous (else its features are)
+  int items;                 // workgroups behind them write rows of the cache, 8 threads to a row
+};
+
+constexpr int kExpTokens = 128, kExpStep = 32, kExpStages = 4, kExpSteps = kLatent / kExpStep;
+constexpr int kExpHalf = 8192, kExpStage = 2 * kExpHalf;  // bytes of the tokens' and of the weight's part of a step
+constexpr int kExpPitch = 272;    // bytes of a result row in LDS: 8-byte writes of 32 rows spread over the banks
+static_assert(kExpTokens * kExpPitch <= kExpStages * kExpStage, "the results take the ring's place");
+
+// Rows of 64 bytes (32 values of the contracted dimension): 16-byte chunk c of row r lies at chunk position c ^ (r / 4 % 4),
+// so the 16 lanes that LDS serves together find their chunks in different banks.
+__device__ __forceinline__ bf16x8 read_row_chunk(const unsigned char *tile, int row, int chunk) {
+  return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(tile + row * 64 + 16 * (chunk ^ ((row >> 2) & 3))));
+}
+
+// part: 0 for K, 1 for V; ROWS: its weight's contracted dimension is contiguous.
+template <bool ROWS>
+__device__ __forceinline__ void expand_item(const ExpandArgs &a, unsigned char *ring, int head, int part, int row0) {
+  const StepArgs &p = a.s;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  // Requests: the first two wavefronts bring the tokens' part of a step, the others the weight's, 4 KiB each as four
+  // consecutive pieces.  Piece i of rows of 64 bytes holds rows 16 i ..., of rows of 256 bytes rows 4 i ...
+  const int first = 4 * (wave & 1);
+  const bool weights = wave >= 2, by_row = !weights || ROWS;
+  const int64_t ld = part ? p.uv_ld : p.uk_ld;
+  const uint16_t *weight = part ? p.w_uv + head * p.uv_hs : p.w_uk + head * p.uk_hs;
+  const uint64_t at = reinterpret_cast<uint64_t>(weights ? weight : p.latent + row0 * p.latent_us);
+  const unsigned char *base = reinterpret_cast<const unsigned char *>(
+      address_from_words(__builtin_amdgcn_readfirstlane((int)(uint32_t)at), __builtin_amdgcn_readfirstlane((int)(uint32_t)(at >> 32))));
+  const int64_t step_bytes = by_row ? 2 * kExpStep : 2 * ld * kExpStep;
+  uint32_t lane_bytes[4];
+  {
+    const uint32_t pitch = (uint32_t)(weights ? 2 * ld : 2 * p.latent_us);
+    const int last = weights ? kLatent : min(kExpTokens, p.users - row0) - 1;  // (rows behind the prompt repeat its last)
+    const int per = by_row ? 16 : 4, in = by_row ? lane >> 2 : lane >> 4;
+    const uint32_t chunk = by_row ? (lane & 3) ^ ((lane >> 4) & 3) : (lane & 15) ^ (4 * (lane >> 4));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) lane_bytes[i] = (uint32_t)min(per * (first + i) + in, last) * pitch + 16u * chunk;
+  }
+  const uint32_t to = lds_address(ring) + 1024u * (uint32_t)first + (weights ? kExpHalf : 0u);
+  auto request = [&](int step) {  // called for the steps in turn
+    const void *const bases[4] = {base, base - 1024, base - 2048, base - 3072};
+    dma16_quad(bases, lane_bytes, (uint32_t)__builtin_amdgcn_readfirstlane((int)(to + (uint32_t)(step % kExpStages) * kExpStage)));
+    base += step_bytes;
+  };
+
+  const int n = lane & 31, h = lane >> 5, grp = lane >> 4, a16 = lane & 15;
+  const int f0 = 64 * (wave & 1), t0 = 64 * (wave >> 1);  // the wavefront's features and tokens
+  const int trow = 8 * (grp >> 1) + (a16 >> 2), tchunk = f0 / 8 + 2 * (grp & 1) + ((a16 & 3) >> 1);
+  floatx16 acc[2][2];
+  bf16x8 w[2][2], x[2][2];  // the fragments of a step's two halves
+  auto read = [&](int step, int half) {
+    const unsigned char *tokens = ring + step % kExpStages * kExpStage, *wtile = tokens + kExpHalf;
+#pragma unroll
+    for (int g = 0; g < 2; ++g) x[half][g] = read_row_chunk(tokens, t0 + 32 * g + n, 2 * half + h);
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+      if constexpr (ROWS) w[half][f] = read_row_chunk(wtile, f0 + 32 * f + n, 2 * half + h);
+      else w[half][f] = read_transposed(wtile + (16 * half + trow) * 256 + 16 * ((tchunk + 4 * f) ^ (4 * (trow & 3))) + 8 * (a16 & 1), 4 * 256);
+  };
+  auto products = [&](int half) {
+    __builtin_amdgcn_sched_barrier(0);  // (the scheduler would put the reads of the other half behind these products)
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+      for (int g = 0; g < 2; ++g) acc[f][g] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[half][f], x[half][g], acc[f][g], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+#pragma unroll
+  for (int f = 0; f < 2; ++f)
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[f][g][r] = 0.f;
+#pragma unroll
+  for (int step = 0; step < kExpStages; ++step) request(step);
+  asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  read(0, 0);
+#pragma unroll
+  for (int step = 0; step < kExpSteps; ++step) {
+    read(step, 1);
+    products(0);
+    if (step + 1 < kExpSteps) {
+      // This wavefront's requests of the next step have landed and its reads of this one have returned; behind the
+      // barrier that holds for everybody: the next step can be read, and this one's place filled.
+      if (step + 3 < kExpSteps) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
+      else if (step + 2 < kExpSteps) asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
+      else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      if (step + kExpStages < kExpSteps) request(step + kExpStages);
+      read(step + 1, 0);
+    }
+    products(1);
+  }
+  // lane (n, h) holds features 8 j + 4 h ... + 3 of token n; the results meet in LDS so that stores are whole rows
+  __syncthreads();
+#pragma unroll
+  for (int f = 0; f < 2; ++f)
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        *reinterpret_cast<uint2 *>(ring + (t0 + 32 * g + n) * kExpPitch + 2 * (f0 + 32 * f + 8 * j + 4 * h)) =
+            make_uint2(pack_bf16x2(acc[f][g][4 * j], acc[f][g][4 * j + 1]), pack_bf16x2(acc[f][g][4 * j + 2], acc[f][g][4 * j + 3]));
+  __syncthreads();
+  uint16_t *out = (part ? a.v : a.k) + head * 128 + 8 * (tid & 15);
+#pragma unroll
+  for (int i = 0; i < kExpTokens / 16; ++i) {
+    const int r = (tid >> 4) + 16 * i;
+    if (row0 + r < p.users)
+      *reinterpret_cast<uint4 *>(out + (int64_t)(row0 + r) * p.heads * 128) = *reinterpret_cast<const uint4 *>(ring + r * kExpPitch + 16 * (tid & 15));
+  }
+}
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void latent_expand_kernel(ExpandArgs a) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char ring[];
+  const StepArgs &p = a.s;
+  if ((int)blockIdx.x >= a.items) {
+    const int tid = threadIdx.x, v = 32 * ((int)blockIdx.x - a.items) + (tid >> 3);
+    int phys, row;
+    if (v >= p.users || !prompt_slot(p, v, phys, row)) return;
+    uint16_t *dst = p.cache + ((int64_t)phys * p.bs + row) * kRow + 8 * (tid & 7);
+    const uint16_t *lat = p.latent + v * p.latent_us + 8 * (tid & 7);
+    uintx4 piece[8];
+    const uintx4 last = *reinterpret_cast<const uintx4 *>(p.rope + v * p.rope_us + 8 * (tid & 7));
+#pragma unroll
+    for (int c = 0; c < 8; ++c) piece[c] = *reinterpret_cast<const uintx4 *>(lat + 64 * c);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) *reinterpret_cast<uintx4 *>(dst + 64 * c) = piece[c];
+    *reinterpret_cast<uintx4 *>(dst + kLatent) = last;
+    return;
+  }
+  const int wt = 2 * p.heads, which = (int)blockIdx.x % wt, row0 = (int)blockIdx.x / wt * kExpTokens;
+  const int head = which >> 1, part = which & 1;
+  if (part ? a.uv_rows : a.uk_rows) expand_item<true>(a, ring, head, part, row0);
+  else expand_item<false>(a, ring, head, part, row0);
 }
 
 inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -280,4 +463,98 @@ extern "C" int ttpa_latent_decode_step_strided(TTPA_LATENT_STEP_HEAD, int64_t w_
   if (uv_columns) latent_value_kernel<true><<<value_grid, dim3(256), 0, st>>>(a);
   else latent_value_kernel<false><<<value_grid, dim3(256), 0, st>>>(a);
   return check_launch("latent_decode_step (value)");
+}
+
+// Prompts of up to this many tokens are absorbed: their error against 64 bits is smaller there than expanded (16 heads, 32 / 64
+// tokens 2.851e-3 / 2.975e-3 against 2.871e-3 / 2.993e-3; 96 / 512 tokens 3.062e-3 / 3.336e-3 against 3.056e-3 / 3.305e-3).
+static constexpr int kAbsorbedTokens = 64;
+
+extern "C" int64_t ttpa_latent_prompt_workspace_bytes(int32_t users, int32_t heads, int32_t seq_len) {
+  if (users <= 0 || heads <= 0 || seq_len <= 0) return 0;
+  const size_t rows = (size_t)users * seq_len, row = (size_t)heads * rows * 2;
+  if (seq_len <= kAbsorbedTokens) return (int64_t)(align256(rows * kRow * 2) + align256(row * kRow) + align256(row * kLatent));
+  return (int64_t)(2 * align256(row * 128));
+}
+
+extern "C" int ttpa_latent_prompt(void *out, int64_t out_token_stride, int64_t out_head_stride, const void *q_nope,
+                                  int64_t q_nope_token_stride, int64_t q_nope_head_stride, const void *q_rope,
+                                  int64_t q_rope_token_stride, int64_t q_rope_head_stride, const void *latent,
+                                  int64_t latent_token_stride, const void *rope, int64_t rope_token_stride, const void *w_uk,
+                                  int64_t w_uk_head_stride, int64_t w_uk_row_stride, int64_t w_uk_column_stride,
+                                  const void *w_uv, int64_t w_uv_head_stride, int64_t w_uv_row_stride,
+                                  int64_t w_uv_column_stride, void *cache, const int32_t *page_table,
+                                  int64_t page_table_row_stride, int32_t users, int32_t table_rows, int32_t heads,
+                                  int32_t seq_len, int32_t block_size, int32_t table_width, int32_t num_blocks, float scale,
+                                  void *workspace, int64_t workspace_bytes, void *stream) {
+  TTPA_REQUIRE(out && q_nope && q_rope && latent && rope && w_uk && w_uv, "null pointer argument");
+  TTPA_REQUIRE(users > 0 && heads > 0 && seq_len > 0 && seq_len % 32 == 0, "latent prompt: bad users, heads or tokens");
+  TTPA_REQUIRE(!cache || (page_table && table_rows > 0 && block_size > 0 && table_width > 0 && num_blocks > 0 &&
+                          (int64_t)seq_len <= (int64_t)table_width * block_size),
+               "latent prompt: %d tokens do not fit the page table", seq_len);
+  TTPA_REQUIRE(aligned16(q_nope) && aligned16(q_rope) && aligned16(latent) && aligned16(rope) && aligned16(w_uk) && aligned16(w_uv) &&
+                   aligned16(cache) && aligned16(out),
+               "latent prompt: operands must be 16-byte aligned");
+  const int64_t strides[] = {out_token_stride, out_head_stride, q_nope_token_stride, q_nope_head_stride, q_rope_token_stride, q_rope_head_stride,
+                             latent_token_stride, rope_token_stride, w_uk_head_stride, w_uv_head_stride};
+  for (int64_t s : strides) TTPA_REQUIRE(s % 8 == 0, "latent prompt: strides must be multiples of 8 elements");
+  const bool uk_columns = w_uk_column_stride != 1, uv_columns = w_uv_column_stride != 1;
+  const int64_t uk_ld = uk_columns ? w_uk_column_stride : w_uk_row_stride, uv_ld = uv_columns ? w_uv_column_stride : w_uv_row_stride;
+  TTPA_REQUIRE((!uk_columns || w_uk_row_stride == 1) && (!uv_columns || w_uv_row_stride == 1),
+               "latent prompt: the rows or the columns of a weight must be contiguous");
+  TTPA_REQUIRE(uk_ld % 8 == 0 && uv_ld % 8 == 0 && uk_ld > 0 && uk_ld < (1 << 23) && uv_ld > 0 && uv_ld < (1 << 23) &&
+                   latent_token_stride > 0 && latent_token_stride < (1 << 23),
+               "latent prompt: row strides must be multiples of 8 elements below 2^23");
+  const int64_t rows = (int64_t)users * seq_len, token_tiles = (rows + kExpTokens - 1) / kExpTokens;
+  TTPA_REQUIRE(heads <= 65535 && rows <= (int64_t)65535 * kUsers && token_tiles * 2 * heads + rows < (int64_t)1 << 31,
+               "latent prompt: too many heads or tokens for one launch");
+  const int64_t need = ttpa_latent_prompt_workspace_bytes(users, heads, seq_len);
+  if (!workspace || workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 255u))
+    return fail(TTPA_ERR_WORKSPACE, "latent prompt: workspace of %lld bytes (256-byte aligned) required, got %lld", (long long)need,
+                (long long)workspace_bytes);
+  unsigned char *ws = static_cast<unsigned char *>(workspace);
+  ExpandArgs e{};
+  StepArgs &a = e.s;
+  a.q_nope = static_cast<const uint16_t *>(q_nope), a.qn_us = q_nope_token_stride, a.qn_hs = q_nope_head_stride;
+  a.q_rope = static_cast<const uint16_t *>(q_rope), a.qr_us = q_rope_token_stride, a.qr_hs = q_rope_head_stride;
+  a.latent = static_cast<const uint16_t *>(latent), a.latent_us = latent_token_stride;
+  a.rope = static_cast<const uint16_t *>(rope), a.rope_us = rope_token_stride;
+  a.w_uk = static_cast<const uint16_t *>(w_uk), a.uk_hs = w_uk_head_stride, a.uk_ld = uk_ld;
+  a.w_uv = static_cast<const uint16_t *>(w_uv), a.uv_hs = w_uv_head_stride, a.uv_ld = uv_ld;
+  a.out = static_cast<uint16_t *>(out), a.out_us = out_token_stride, a.out_hs = out_head_stride;
+  a.cache = static_cast<uint16_t *>(cache), a.pt = page_table, a.pt_rs = page_table_row_stride;
+  a.users = (int)rows, a.heads = heads, a.bs = block_size, a.w = table_width, a.nb = num_blocks;
+  a.seq = seq_len, a.table_rows = table_rows;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (seq_len > kAbsorbedTokens) {
+    e.k = reinterpret_cast<uint16_t *>(ws), e.v = reinterpret_cast<uint16_t *>(ws + align256((size_t)rows * heads * 256));
+    e.uk_rows = !uk_columns, e.uv_rows = uv_columns;
+    e.items = (int)(token_tiles * 2 * heads);
+    const int64_t groups = e.items + (cache ? (rows + 31) / 32 : 0);
+    constexpr size_t kLds = (size_t)kExpStages * kExpStage;
+    static std::atomic<uint64_t> lds_ready{0};
+    if (!ensure_dynamic_lds(reinterpret_cast<const void *>(&latent_expand_kernel), kLds, lds_ready))
+      return fail(TTPA_ERR_LAUNCH, "latent prompt: cannot configure the expansion kernel");
+    latent_expand_kernel<<<dim3((unsigned)groups), dim3(256), kLds, st>>>(e);
+    if (int rc = check_launch("latent_prompt (expansion)")) return rc;
+    const int64_t hd = (int64_t)heads * 128, sl = seq_len;
+    return ttpa_split_key_prefill(out, sl * out_token_stride, out_head_stride, out_token_stride, q_nope, sl * q_nope_token_stride,
+                                  q_nope_head_stride, q_nope_token_stride, q_rope, sl * q_rope_token_stride, q_rope_head_stride,
+                                  q_rope_token_stride, e.k, sl * hd, 128, hd, rope, sl * rope_token_stride, 0, rope_token_stride, e.v,
+                                  sl * hd, 128, hd, users, heads, heads, seq_len, scale, stream);
+  }
+  a.k_lat = reinterpret_cast<uint16_t *>(ws);
+  a.q_lat = reinterpret_cast<uint16_t *>(ws + align256((size_t)rows * kRow * 2));
+  a.o_lat = reinterpret_cast<uint16_t *>(reinterpret_cast<unsigned char *>(a.q_lat) + align256((size_t)rows * heads * kRow * 2));
+  const unsigned tiles = (unsigned)((rows + kUsers - 1) / kUsers);
+  const dim3 query_grid(kLatent / 128, (unsigned)heads, tiles), value_grid(kValue / 32, (unsigned)heads, tiles);
+  if (uk_columns) latent_query_kernel<true, true><<<query_grid, dim3(256), 0, st>>>(a);
+  else latent_query_kernel<false, true><<<query_grid, dim3(256), 0, st>>>(a);
+  if (int rc = check_launch("latent_prompt (query)")) return rc;
+  const int64_t ql = (int64_t)heads * kRow, ol = (int64_t)heads * kLatent;
+  if (int rc = ttpa_latent_prefill(a.o_lat, seq_len * ol, kLatent, ol, a.q_lat, seq_len * ql, kRow, ql, a.k_lat, (int64_t)seq_len * kRow, 0, kRow,
+                                   nullptr, 0, 0, 0, users, heads, 1, seq_len, kRow, kLatent, 1, scale, stream))
+    return rc;
+  if (uv_columns) latent_value_kernel<true><<<value_grid, dim3(256), 0, st>>>(a);
+  else latent_value_kernel<false><<<value_grid, dim3(256), 0, st>>>(a);
+  return check_launch("latent_prompt (value)");
 }

@@ -118,6 +118,12 @@ SIGNATURES = {
         [_p, _i64, _i64, _p, _i64, _i64, _p, _i64, _i64, _p, _i64, _p, _i64, _p, _i64, _i64, _i64, _p, _i64, _i64, _i64,
          _p, _p, _i64, _p, _int, _i32, _i32, _i32, _i32, _i32, _f32, _p, _sz, _p],
     ),
+    "ttpa_latent_prompt_workspace_bytes": (_i64, [_i32, _i32, _i32]),
+    "ttpa_latent_prompt": (
+        _int,
+        [_p, _i64, _i64, _p, _i64, _i64, _p, _i64, _i64, _p, _i64, _p, _i64, _p, _i64, _i64, _i64, _p, _i64, _i64, _i64,
+         _p, _p, _i64, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _f32, _p, _i64, _p],
+    ),
     "ttpa_split_key_prefill": (
         _int, [_p, _i64, _i64, _i64] * 6 + [_i32, _i32, _i32, _i32, _f32, _p],
     ),
@@ -195,6 +201,13 @@ def attention_pass(*args):
     global attention_pass
     attention_pass = host().attention_pass
     return attention_pass(*args)
+
+
+def latent_pass(*args):
+    """The same for a latent layer's pass."""
+    global latent_pass
+    latent_pass = host().latent_pass
+    return latent_pass(*args)
 
 
 def check(name: str, rc: int) -> None:

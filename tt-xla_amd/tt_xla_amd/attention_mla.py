@@ -36,7 +36,8 @@ from typing import List, Optional, Tuple
 
 import torch
 
-from . import custom_ops  # noqa: F401  (registers torch.ops.tt.*)
+from . import _native
+from . import custom_ops  # (registers torch.ops.tt.*)
 from .attention import TTAttentionMetadataBuilder, TTMetadata
 
 # the operator namespace, looked up once: host-logic tests substitute it
@@ -155,6 +156,8 @@ class TTMLAAttentionBackendImpl(_ImplBase):
         into ``output`` [tokens, N * v_head_dim].  ``layer`` carries ``W_UK_T`` [N, P, L] and
         ``W_UV`` [N, L, V]."""
         assert output is not None, "TTMLAAttentionBackendImpl.forward requires an output tensor."
+        if self._forward_native(q, kv_c_normed, k_pe, kv_cache, attn_metadata, layer, output):
+            return
         q_nope, q_pe = q
         prefill = self._infer_is_prefill(q_nope, attn_metadata)
         users = 1
@@ -189,6 +192,28 @@ class TTMLAAttentionBackendImpl(_ImplBase):
         else:
             out = self._forward_decode(q_lat, k_lat, kv_cache, attn_metadata, layer, users)
         output.copy_(out.to(act_dtype).reshape_as(output))
+
+    def _forward_native(self, q, kv_c_normed, k_pe, kv_cache, attn_metadata, layer, output) -> bool:
+        """The ordinary eager pass (causal, the head shape that the operators below are built for, with a cache) as one native
+        call; False: not such a pass, nothing has been issued.  A prompt of 32 tokens took 100 us through views, batched
+        products and operators, whatever the GPU did meanwhile."""
+        if (
+            attn_metadata is None
+            or self.functional_cache_ops
+            or (self.qk_nope_head_dim, self.qk_rope_head_dim, self.kv_lora_rank, self.v_head_dim) != (128, 64, 512, 128)
+            or attn_metadata.attn_mask is not None
+            or not attn_metadata.is_causal
+            or torch.compiler.is_compiling()
+        ):
+            return False
+        status = _native.latent_pass(
+            q[0], q[1], kv_c_normed, k_pe, kv_cache, attn_metadata.page_table, attn_metadata.cache_position, attn_metadata.fill_page_table,
+            layer.W_UK_T, layer.W_UV, output, self.num_heads, self.scale, custom_ops._workspace)
+        if status is None:
+            return False
+        if status != 0:
+            _native.check(*status)
+        return True
 
     @staticmethod
     def _infer_is_prefill(q_nope: torch.Tensor, attn_metadata: Optional[TTMetadata]) -> bool:
