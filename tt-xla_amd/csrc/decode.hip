@@ -527,16 +527,22 @@ static int decode_impl(void *out, int64_t out_user_stride, int64_t out_head_stri
     a.direct = direct_waves(users, kv_heads, head_size, kv_format, tokens, forced == 5);
     if (a.direct) use_mfma16 = true, use_mfma = false;
   }
-  // The matrix-core kernels get at most one workgroup per CU whatever the cache format: the 32x32
+  // The matrix-core kernels get at most one workgroup per CU on a bfloat16 cache: the 32x32
   // kernel fills the CU's LDS with one, and the 16x16 kernel streams as fast with one as with the
-  // two that would fit, while twice the partials cost the merge kernel more.  On a bfloat16 cache
+  // two that would fit, while twice the partials cost the merge kernel more.  There
   // the 16x16 kernel is fastest with three quarters of the CUs (measured in one process, grids of
   // 2.5 ... 4 wavefronts per CU: 56.0-56.9 us per step at 2.75 ... 3.75 against 57.3-57.7 at 4 on
   // the 32-user workload, 531 against 544 us on the 128-user one: the streams of 192 workgroups
   // already hold the memory system's latency in bytes, and every further wavefront is one more
-  // partial and one more share in the contention); on a block-float-8 cache it wants all of them
-  // (50.4 against 43.9 us).
+  // partial and one more share in the contention).  On a block-float-8 cache it wants two workgroups
+  // per CU up to head size 128 (tile_bytes), if they have something to do: where no more than six tiles per range
+  // can be attended, the partials of twice the ranges cost more than the chains that they hide (us per layer at one / two: 2
+  // users of 64/8 heads with 3327 ... 6987 tokens 16.4 / 17.5, one of 32/8 heads over 16384 19.2 / 20.0, 27 with 512 ... 4096 32.5 / 30.5).
+  const int64_t seen = sliding_window > 0 ? std::min<int64_t>((int64_t)table_width * block_size, sliding_window) : (int64_t)table_width * block_size;
+  const bool two_per_cu = use_mfma16 && kv_format == TTPA_KV_BFP8 && head_size <= 128 &&
+                          (int64_t)users * kv_heads * (seen * head_size / 4096) >= 6 * (int64_t)waves_for_device(8.0);
   a.n_waves = waves_for_device(use_mfma16 && kv_format == TTPA_KV_BF16 ? 3.0
+                               : two_per_cu                             ? 8.0
                                : (use_mfma || use_mfma16)               ? 4.0
                                : kv_format == TTPA_KV_BFP8              ? kLargestGrid
                                                                         : 4.0);

@@ -3,8 +3,7 @@
 // to half precision) or a bfloat16 cache.
 //
 // Work decomposition, partial slots and merge kernel are those of decode.hip, with tiles of
-// 16 KiB of 16-bit elements (128, 64 or 32 tokens at head size 64, 128, 256; 8 KiB = 64 / 32 tokens
-// for a bfloat16 cache with head size 64 / 128, see tile_bytes).  Inside a wavefront a tile of K,
+// 64, 32 or 32 tokens at head size 64, 128, 256 (tile_bytes).  Inside a wavefront a tile of K,
 // then of V, goes global -> registers -> a wave-private LDS buffer of that size that both
 // tensors use in turn:
 //   stage K(t) | prefetch K(t+1) | S^T = K Q^T | softmax | stage V(t) | prefetch V(t+1) | O^T += V^T P^T
@@ -64,22 +63,20 @@ typedef short shortx4 __attribute__((ext_vector_type(4)));
 
 constexpr int kMaxUsers16 = kMaxUsers;  // the library-wide limit: 16 KiB of prefix tables
 // Bytes of a tile's K (or V) rows as 16-bit elements, i.e. of a wavefront's LDS buffer: 16 KiB
-// (128 / 64 / 32 tokens at head size 64 / 128 / 256), except 8 KiB (64 / 32 tokens) for a bfloat16
-// cache with head size 64 or 128.  A wavefront has one tile of K and one of V in flight; the kernel
-// ends when the slowest wavefront has drained its last tile, and wavefronts of one launch finish
+// (32 tokens) at head size 256, 8 KiB (64 / 32 tokens) at head size 64 / 128.  A wavefront has one
+// tile of K and one of V in flight; the kernel ends when the slowest wavefront has drained its last tile, and wavefronts of one launch finish
 // several microseconds apart (the XCDs do not get equal shares of the HBM bandwidth), so a
 // shorter tile shortens that tail: config 2's step 58.7 -> 57.8 us, config 4's 549 -> 543 us.
 // At head size 64 (64 / 8 heads, us per layer of a replayed step): a window of 1024 over 37 users 25.2 ->
 // 23.1 (its two ends waste less, too), 32 users with 512 ... 4096 tokens 27.7 -> 26.5, 8 users with
 // 128 ... 1024 15.0 -> 11.6, 128 users with 256 ... 32768 274 -> 272; 4 KiB: 23.6, 26.9, 10.8.
-// The block-float-8 cache moves half the bytes per token and loses with the shorter tile where there is
-// much to read (head size 128, 64 users with 1024 ... 16384 tokens: 138 -> 150 us; head size 64, 100 users
-// with 1024 ... 8192: 78 -> 84), and how much there is only the device knows.
-// With one workgroup per segment (DIRECT) the short tile for both formats: the wavefronts of a workgroup
-// take the tiles in turn, so a short context reaches more of them, and two wavefronts share a SIMD's registers.
-template <int D, bool BFP8, int DIRECT = 0>
+// A block-float-8 tile is half the bytes behind the same chain of steps, so that kernel is bound by the chain.  With 16 KiB it
+// needed 316 registers, one wavefront per SIMD; with 8 KiB two share a SIMD and a launch has twice the wavefronts (us per layer,
+// 64 users with 1024 ... 16384 tokens, 32/8 heads at head size 128: 144 -> 137; 100 users with 1024 ... 8192, 64/8 heads at 64: 92 ->
+// 78; 40 users of 16/16 heads with 512 ... 4096: 68 -> 61).  Head size 256 has 32-token tiles either way.
+template <int D>
 constexpr int tile_bytes() {
-  return (D <= 128 && (!BFP8 || DIRECT)) ? 8192 : 16384;
+  return D <= 128 ? 8192 : 16384;
 }
 
 template <bool F16>
@@ -155,10 +152,10 @@ __device__ __forceinline__ void merge_waves(const DecodeArgs &a, int u, int h, i
 // DIRECT: a workgroup of DIRECT wavefronts owns the whole segment blockIdx.x (chosen by direct_waves, decode.hip): no prefix, no
 // search, no partials, no merge launch.  Its wavefronts take the segment's tiles in turn.
 template <int D, bool BFP8, int RUNS, bool FUSED, bool MASKED = false, int DIRECT = 0>
-__global__ __launch_bounds__(DIRECT ? kWave *DIRECT : 256, DIRECT && D <= 128 ? 2 : 1) void paged_decode_mfma16_kernel(
+__global__ __launch_bounds__(DIRECT ? kWave *DIRECT : 256, (DIRECT || BFP8) && D <= 128 ? 2 : 1) void paged_decode_mfma16_kernel(
     DecodeArgs a, const int32_t *__restrict__ page_table, const void *__restrict__ cur_pos) {
   static_assert(D == 64 || D == 128 || D == 256, "shapes built");
-  constexpr int kTileBytes = tile_bytes<D, BFP8, DIRECT>();
+  constexpr int kTileBytes = tile_bytes<D>();
   constexpr int TILE = kTileBytes / (2 * D);  // tokens per tile
   constexpr int ROWB = 2 * D;                 // bytes of a tile row in LDS
   constexpr int KSTEPS = D / 32, DBLK = D / 16;
@@ -667,7 +664,7 @@ template <int D, bool BFP8, int RUNS, bool FUSED, bool MASKED = false, int DIREC
 bool launch(const DecodeArgs &a, hipStream_t st) {
   constexpr int kWaves = DIRECT ? DIRECT : kWavesPerBlock;
   const int blocks = DIRECT ? a.users * a.hkv : a.n_waves / kWavesPerBlock;
-  const size_t lds = (size_t)kWaves * tile_bytes<D, BFP8, DIRECT>();
+  const size_t lds = (size_t)kWaves * tile_bytes<D>();
   static std::atomic<uint64_t> lds_ready{0};
   const auto kernel = &paged_decode_mfma16_kernel<D, BFP8, RUNS, FUSED, MASKED, DIRECT>;
   if (!ensure_dynamic_lds(reinterpret_cast<const void *>(kernel), lds, lds_ready)) return false;
@@ -678,7 +675,7 @@ bool launch(const DecodeArgs &a, hipStream_t st) {
 // One workgroup per segment (a.direct).
 template <int D, bool BFP8, bool FUSED, int DIRECT>
 bool launch_direct(const DecodeArgs &a, hipStream_t st) {
-  constexpr int TILE = tile_bytes<D, BFP8, DIRECT>() / (2 * D);
+  constexpr int TILE = tile_bytes<D>() / (2 * D);
   return a.bs % TILE == 0 ? launch<D, BFP8, 1, FUSED, false, DIRECT>(a, st) : launch<D, BFP8, 2, FUSED, false, DIRECT>(a, st);
 }
 
@@ -686,7 +683,7 @@ bool launch_direct(const DecodeArgs &a, hipStream_t st) {
 // cache update of the step).
 template <int D, bool BFP8>
 bool launch_for_block_size(const DecodeArgs &a, hipStream_t st) {
-  constexpr int TILE = tile_bytes<D, BFP8>() / (2 * D);
+  constexpr int TILE = tile_bytes<D>() / (2 * D);
   const bool fused = a.k_new != nullptr;
   if constexpr (D <= 128) {
     if (a.direct == 4) return fused ? launch_direct<D, BFP8, true, 4>(a, st) : launch_direct<D, BFP8, false, 4>(a, st);
