@@ -389,8 +389,8 @@ int ttpa_sdpa_prefill_format(void *out, int64_t out_batch_stride, int64_t out_he
 /*
  * ttpa_sdpa_prefill_format with scratch memory from the caller.  With kv_format = TTPA_KV_BFP8 and
  * at least ttpa_sdpa_prefill_workspace_bytes(...) bytes of 16-byte aligned device memory, a pass
- * over head size 128 with a multiple of four query heads per KV head, block_size a multiple of 64,
- * no window and no mask first expands the block-float-8 blocks it will read into bfloat16 copies
+ * over head size 128, block_size a multiple of 32, no window and no mask, whose blocks are read by more than two
+ * workgroups each, first expands the block-float-8 blocks it will read into bfloat16 copies
  * in the scratch (one launch; the decode is exact, so the result is the same) and then runs the
  * bfloat16 attention kernel over the copies: measured 1.7 times faster than expanding every tile
  * once per workgroup on 4 x 512-token chunks behind 2048 cached tokens.  Every other shape, a null
@@ -417,12 +417,11 @@ int ttpa_sdpa_prefill_expanded(void *out, int64_t out_batch_stride, int64_t out_
 int64_t ttpa_sdpa_prefill_workspace_bytes(int32_t batch, int32_t kv_heads, int32_t head_size,
                                           int32_t block_size, int32_t table_width, int32_t kv_format);
 
-/* Bytes of scratch with which ttpa_sdpa_prefill_expanded runs these dimensions fastest: the above, and, for
- * either cache format, room for float partial results where a pass of few query rows over many keys is
- * split over the keys (head size 128, block_size a multiple of 32; at most 16 parts, 34 MB for 512 rows of 32
- * heads).  0 where neither would pay (a table too narrow to be split; over block-float-8 caches, one workgroup per
- * head group and many copies).  With less, a null or a smaller workspace the pass runs unsplit.  Scratch for the
- * expansion comes first; what is behind it is used for the parts. */
+/* Bytes of scratch with which ttpa_sdpa_prefill_expanded runs these dimensions fastest: the above where the pass reads
+ * copies, and, for either cache format, room for float partial results where a pass of few query rows over many keys
+ * is split over the keys (at most 16 parts, 34 MB for 512 rows of 32 heads of 128).  0 where neither would pay (a table
+ * too narrow to be split).  With less, a null or a smaller workspace the pass runs unsplit.  Scratch for the expansion
+ * comes first; what is behind it is used for the parts. */
 int64_t ttpa_sdpa_prefill_scratch_bytes(int32_t batch, int32_t q_heads, int32_t kv_heads, int32_t q_len,
                                         int32_t head_size, int32_t block_size, int32_t table_width,
                                         int32_t kv_format);

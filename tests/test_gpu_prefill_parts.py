@@ -1,0 +1,119 @@
+"""Chunk passes of the compiler-scheduled prefill loop split over the keys (head sizes 64 and 256, cache blocks that the
+streaming loop does not take, block-float-8 tiles): sizes where a split begins and ends, parts that lie behind the causal
+limit of the first rows, wavefronts without rows, row blocks without keys.  Tolerance as in test_gpu_prefill.py: a bfloat16
+output and bfloat16 probabilities, split or not."""
+
+import pytest
+import torch
+
+import test_gpu_prefill as P
+from oracle import bfp8_codec
+from oracle import paged_ops as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _pkg():
+    P.entry.ensure_built()
+    import tt_xla_amd  # noqa: F401
+
+
+def _pass(q, key, value, table, start, scale):
+    return torch.ops.tt.chunked_scaled_dot_product_attention(q, key, value, table, start, scale)
+
+
+@pytest.mark.parametrize("users,hq,hkv,d,bs,start,lc", [
+    # head size 64: blocks of whole tiles, of whole loads, smaller ones; no split, an uneven last part, a start inside a block
+    (1, 8, 8, 64, 64, 1216, 224), (1, 8, 8, 64, 32, 320, 608), (2, 4, 1, 64, 64, 0, 40), (1, 8, 2, 64, 128, 4001, 33),
+    (1, 2, 1, 64, 8, 700, 100), (1, 4, 1, 64, 4, 600, 50), (3, 6, 3, 64, 64, 1500, 70),
+    (1, 4, 1, 64, 64, 511, 1), (1, 4, 1, 64, 64, 479, 1), (1, 4, 1, 64, 64, 512, 200),  # 16 key blocks, 15, parts behind early rows
+    # head size 128 outside the streaming loop's blocks
+    (1, 4, 1, 128, 16, 2048, 32), (1, 3, 3, 128, 48, 1000, 130), (2, 8, 2, 128, 2, 650, 60),
+    # head size 256: one workgroup per CU
+    (1, 16, 8, 256, 32, 832, 192), (1, 4, 1, 256, 64, 3000, 65), (2, 2, 2, 256, 16, 640, 20),
+])
+def test_split_chunks(users, hq, hkv, d, bs, start, lc):
+    g = torch.Generator().manual_seed(hq + bs + start + d)
+    nbpu = -(-(start + lc) // bs) + 1
+    key, value, table = P._paged(g, users, nbpu, hkv, bs, d, False)
+    q = P._bf(g, users, hq, lc, d)
+    st = torch.tensor([start], dtype=torch.int32)
+    want = O.chunked_sdpa(q, key, value, table, st, d**-0.5)
+    got = _pass(q.cuda(), key.cuda(), value.cuda(), table.cuda(), st.cuda(), d**-0.5)
+    P._check(f"split u{users} h{hq}x{hkv} d{d} bs{bs} start{start} len{lc}", got.cpu(), want)
+
+
+@pytest.mark.parametrize("users,hq,hkv,d,bs,start,lc", [
+    (1, 8, 8, 64, 32, 1300, 96), (2, 8, 2, 64, 64, 700, 33), (1, 64, 8, 128, 64, 2368, 32), (3, 4, 4, 128, 32, 900, 40),
+    (1, 4, 1, 128, 16, 1100, 100),
+])
+def test_split_chunks_over_block_float_8(users, hq, hkv, d, bs, start, lc):
+    g = torch.Generator().manual_seed(hq + bs + start + d)
+    nbpu = -(-(start + lc) // bs) + 1
+    key, value, table = P._paged(g, users, nbpu, hkv, bs, d, False)
+    q = P._bf(g, users, hq, lc, d)
+    st = torch.tensor([start], dtype=torch.int32)
+    packed = [bfp8_codec.pack_cache(t) for t in (key, value)]
+    want = O.chunked_sdpa(q, *[bfp8_codec.unpack_cache(t, bs).to(torch.bfloat16) for t in packed], table, st, d**-0.5)
+    got = _pass(q.cuda(), packed[0].cuda(), packed[1].cuda(), table.cuda(), st.cuda(), d**-0.5)
+    P._check(f"split bfp8 u{users} h{hq}x{hkv} d{d} bs{bs} start{start} len{lc}", got.cpu(), want)
+
+
+@pytest.mark.parametrize("d,bs", [(64, 64), (64, 32), (128, 16), (256, 32)])
+def test_split_closeness_and_replay(d, bs, monkeypatch):
+    """Against 64 bits a split pass is as close as an unsplit one (the same probabilities, float accumulators; a quarter
+    more allows for the other references of the parts), and a captured one gives the eager bits on every replay."""
+    from tt_xla_amd import _native as N
+
+    g = torch.Generator().manual_seed(d + bs)
+    hq, hkv, start, lc = 4, 2, 1600, 96
+    nbpu = -(-(start + lc) // bs)
+    key, value, table = P._paged(g, 1, nbpu, hkv, bs, d, False)
+    q = P._bf(g, 1, hq, lc, d)
+    st = torch.tensor([start], dtype=torch.int32)
+    k = key[table[0].long()].permute(1, 0, 2, 3).reshape(hkv, -1, d).double().repeat_interleave(hq // hkv, 0)
+    v = value[table[0].long()].permute(1, 0, 2, 3).reshape(hkv, -1, d).double().repeat_interleave(hq // hkv, 0)
+    s = q[0].double() @ k.transpose(1, 2) * d**-0.5
+    s = s.masked_fill(torch.arange(k.shape[1])[None] > start + torch.arange(lc)[:, None], -torch.inf)
+    want = (s.softmax(-1) @ v)[None]
+    args = [t.cuda() for t in (q, key, value, table, st)]
+    got = _pass(*args, d**-0.5)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        replayed = _pass(*args, d**-0.5)
+    for _ in range(3):
+        replayed.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(replayed, got)
+    assert N.lib().ttpa_sdpa_prefill_scratch_bytes(1, hq, hkv, lc, d, bs, nbpu, 0) > 0
+    call = N.call
+
+    def without_scratch(name, *a):
+        return call(name, *(a[:-3] + (0, 0, a[-1]) if name == "ttpa_sdpa_prefill_expanded" else a))
+
+    monkeypatch.setattr(N, "call", without_scratch)
+    unsplit = _pass(*args, d**-0.5)
+    err = [((t.cpu().double() - want).norm() / want.norm()).item() for t in (got, unsplit)]
+    print(f"d{d} bs{bs}: split {err[0]:.3e}, unsplit {err[1]:.3e}")
+    assert not torch.equal(got, unsplit), "the pass was not split"
+    assert err[0] <= 1.25 * err[1]
+
+
+@pytest.mark.parametrize("d,bs", [(64, 32), (128, 16), (256, 64)])
+@pytest.mark.parametrize("start", [-40, -1000, -2000000000, 2000000000])
+def test_chunks_that_start_outside_the_sequence(d, bs, start):
+    """Rows without a key come out as NaN, a start behind the table lets every row see all of it; as in the streaming loop."""
+    g = torch.Generator().manual_seed(d)
+    lc, nbpu = 96, 1280 // bs
+    key, value, table = P._paged(g, 1, nbpu, 1, bs, d, False)
+    q = P._bf(g, 1, 2, lc, d)
+    st = torch.tensor([start], dtype=torch.int32)
+    got = _pass(q.cuda(), key.cuda(), value.cuda(), table.cuda(), st.cuda(), d**-0.5).cpu()
+    blind = min(max(-start, 0), lc)
+    assert got[:, :, :blind].isnan().all()
+    if blind < lc:
+        held = torch.tensor([min(start, 1280)], dtype=torch.int32)
+        want = O.chunked_sdpa(q[:, :, blind:], key, value, table, torch.clamp(held + blind, 0), d**-0.5)
+        P._check(f"start {start} d{d}", got[:, :, blind:], want)

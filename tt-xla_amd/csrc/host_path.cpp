@@ -184,12 +184,9 @@ PyObject *attention_pass(PyObject *, PyObject *const *v, Py_ssize_t n) {
   }
   const at::Tensor *pt = p.table(v[5]), *start = p.numbers(v[9], 1);
   if (!pt || pt->size(0) != users || !start || is_i64(start)) Py_RETURN_NONE;
-  int64_t bytes = 0;
-  if (d == 128 && bs % 32 == 0) {
-    bytes = ttpa_sdpa_prefill_scratch_bytes((int32_t)users, (int32_t)hq, (int32_t)hkv, (int32_t)s, (int32_t)d, (int32_t)bs,
-                                            (int32_t)pt->size(1), fmt);
-    if (bytes < 0 || bytes > kScratchLimit) bytes = 0;
-  }
+  int64_t bytes = ttpa_sdpa_prefill_scratch_bytes((int32_t)users, (int32_t)hq, (int32_t)hkv, (int32_t)s, (int32_t)d, (int32_t)bs,
+                                                  (int32_t)pt->size(1), fmt);
+  if (bytes < 0 || bytes > kScratchLimit) bytes = 0;
   written(kc), written(vc), written(out);
   {
     RECORD_FUNCTION("tt::paged_fill_kv_cache_", std::vector<c10::IValue>());

@@ -23,7 +23,7 @@
 // unpadded in LDS; bank conflicts are avoided by an XOR swizzle of the 16-byte chunk
 // position inside a row, applied on the global side (which chunk a lane fetches) and again
 // when fragments are read.
-#include "prefill_common.h"
+#include "prefill_parts.h"
 
 #include <algorithm>
 #include <cstdlib>
@@ -137,6 +137,8 @@ __global__ __launch_bounds__(256, prefill_wgs_per_cu<RH>(D, MODE)) void prefill_
     wg = attention_workgroup<D>(a, wg);
     if (wg < 0) return;
   }
+  // (the slower index, so that part 0, alone with work where the keys are few, is on every XCD)
+  const int part = MODE != 0 ? blockIdx.y : 0;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -159,18 +161,29 @@ __global__ __launch_bounds__(256, prefill_wgs_per_cu<RH>(D, MODE)) void prefill_
   const int hk = hq0 / g;
   const int hq = hq0 + wave % HPW;
   const int row0 = (qt * RPW + wave / HPW) * ROWS;  // first query row of the wavefront
-  const int offset = a.causal ? (a.chunk_start ? a.chunk_start[0] : 0) : 0;
+  const int offset = a.causal ? chunk_offset(a.chunk_start, a.sq, a.skv) : 0;
 
   // keys this workgroup / this wavefront can see
   const int wg_last_row = min(a.sq, (qt + 1) * ROWS * RPW) - 1;
   const int kv_end_wg = a.causal ? min(a.skv, offset + wg_last_row + 1) : a.skv;
-  const int ntiles = (kv_end_wg + kKeysPerTile - 1) / kKeysPerTile;
+  // (at least one tile: where no row sees a key, tile 0 is read and no score of it is computed)
+  int ntiles = max((kv_end_wg + kKeysPerTile - 1) / kKeysPerTile, 1);
   const int wave_last_key = a.causal ? offset + min(a.sq - 1, row0 + ROWS - 1) : a.skv - 1;
   const bool wave_active = row0 < a.sq;
   // sliding window: first key any row of the workgroup / of this wavefront can see
   const int wg_first_key = a.window > 0 ? max(0, offset + qt * ROWS * RPW - a.window + 1) : 0;
   const int wave_first_key = a.window > 0 ? max(0, offset + row0 - a.window + 1) : 0;
-  const int first_tile = wg_first_key / kKeysPerTile;
+  int first_tile = wg_first_key / kKeysPerTile;
+  bool whole = true;  // this workgroup sees all keys of its rows
+  if constexpr (MODE != 0) {
+    if (a.parts > 1) {  // (no window, no mask)
+      const int share = __builtin_amdgcn_readfirstlane((blocks_per_part(a, offset) + 1) / 2);
+      whole = share >= ntiles;
+      first_tile = part * share;
+      ntiles = min(ntiles, first_tile + share);
+      if (first_tile >= ntiles) return;
+    }
+  }
 
   // ---- Q fragments (B operand: lane n = query row, 8 head-dim elements per k-step) -----
   static_assert(RH == 1, "one block of 32 query rows per wavefront");
@@ -373,7 +386,6 @@ __global__ __launch_bounds__(256, prefill_wgs_per_cu<RH>(D, MODE)) void prefill_
   constexpr int KPRE = MODE == 4 ? 4 : 6;  // K fragments
   constexpr int VPRE = MODE == 4 ? 2 : 4;  // V^T fragments
 
-  // ntiles >= 1 always (row 0 sees key 0).
   const int last_tile = ntiles - 1;
   // Block-table entries are vector loads (the load-to-LDS instruction is opaque to the
   // compiler, so it cannot prove the table unchanged and scalar), and waiting for one means
@@ -580,6 +592,26 @@ __global__ __launch_bounds__(256, prefill_wgs_per_cu<RH>(D, MODE)) void prefill_
   }
 
   // ---- normalise and store: lane (n, h) holds head-dim elements 32 db + 8 j + 4 h + i ----
+  if constexpr (MODE != 0) {
+    if (!whole) {
+      // a part's accumulators and (maximum, sum) per row: lane l's four elements of group 4 db + j at float 256 (4 db + j) + 4 l
+      // of the row block's, 1 KiB per store of the wavefront.  A row that sees none of the part's keys has maximum -inf, sum 0.
+      const float l_tot = l_run[0] + __shfl_xor(l_run[0], 32);
+      const PartLayout lay = part_layout(a, ROWS * RPW);
+      const int64_t at = (((int64_t)part * a.batch + b) * a.hq + hq) * lay.row_blocks + qt * RPW + wave / HPW;
+      float *dst = a.part_acc + at * part_acc_floats(D) + 4 * lane;
+#pragma unroll
+      for (int db = 0; db < DBLK; ++db)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          *reinterpret_cast<float4 *>(dst + 256 * (4 * db + j)) =
+              make_float4(acc[0][db][4 * j], acc[0][db][4 * j + 1], acc[0][db][4 * j + 2], acc[0][db][4 * j + 3]);
+      if (h == 0)
+        *reinterpret_cast<float2 *>(a.part_acc + lay.slots * part_acc_floats(D) + at * (2 * kRowsPerWave) + 2 * n) =
+            make_float2(m_run[0] * a.scale_log2e, l_tot);
+      return;
+    }
+  }
   if (!wave_active) return;
 #pragma unroll
   for (int x = 0; x < RH; ++x) {
@@ -601,6 +633,16 @@ __global__ __launch_bounds__(256, prefill_wgs_per_cu<RH>(D, MODE)) void prefill_
   }
 }
 
+// Whether the plain loop may split the keys of this launch: paged, each row sees all keys up to its own.
+inline bool plain_splits(const PrefillArgs &a) { return a.pt != nullptr && a.window == 0 && a.mask == nullptr; }
+
+// Bytes of scratch with which it does (0: it would not).
+inline int64_t plain_part_bytes(const PrefillArgs &a, int d, bool bfp8) {
+  if (!plain_splits(a)) return 0;
+  const int g = a.hq / a.hkv;
+  return part_bytes(a, g % 4 == 0 ? 4 : g % 2 == 0 ? 2 : 1, plain_split(d, bfp8), d);
+}
+
 template <int D, int HPW, int MODE, int RH>
 int launch_mode(const PrefillArgs &a, hipStream_t st) {
   constexpr int RPW = 4 / HPW;
@@ -613,9 +655,17 @@ int launch_mode(const PrefillArgs &a, hipStream_t st) {
   const int ny8 = (a.batch * (a.hq / HPW) + 7) / 8;
   PrefillArgs b = a;
   int grid = nqt * ny8 * 8;
+  b.parts = 1;
+  constexpr SplitRule kRule = plain_split(D, MODE == 4);
+  if (MODE != 0 && plain_splits(a) && a.part_acc && a.part_bytes >= part_bytes(a, HPW, kRule, D)) set_parts(b, HPW, kRule);
   if (MODE == 0 && a.fill_kc) grid = grid_with_fill(b, grid, D);
-  launch_dominant(&prefill_kernel<D, HPW, MODE, RH>, dim3(grid), dim3(256), lds, st, b);
-  return check_launch("sdpa_prefill");
+  launch_dominant(&prefill_kernel<D, HPW, MODE, RH>, dim3(grid, b.parts), dim3(256), lds, st, b);
+  if (const int rc = check_launch("sdpa_prefill")) return rc;
+  if (MODE != 0 && b.parts > 1) {
+    prefill_merge_kernel<D, RPW><<<dim3((b.sq + kRowsPerWave - 1) / kRowsPerWave, b.hq, b.batch), dim3(2 * D), 0, st>>>(b);
+    return check_launch("sdpa_prefill (merge of the parts)");
+  }
+  return TTPA_OK;
 }
 
 template <int D, int HPW, int RH>
@@ -751,6 +801,11 @@ static int prefill_impl(void *out, int64_t out_batch_stride, int64_t out_head_st
   a.bs = block_size, a.w = table_width, a.nb = num_blocks, a.causal = causal ? 1 : 0;
   a.window = sliding_window;
   a.scale_log2e = scale * 1.4426950408889634f;
+  {
+    // (TTPA_PREFILL_STREAM=0, read on every call, sends every shape through the plain loop)
+    const char *e = getenv("TTPA_PREFILL_STREAM");
+    a.stream = e ? atoi(e) : 1;
+  }
   if (kv_format != TTPA_KV_BF16 && kv_format != TTPA_KV_BFP8)
     return fail(TTPA_ERR_INVALID_ARGUMENT, "prefill: unknown kv_format %d", kv_format);
   a.kv_bfp8 = kv_format == TTPA_KV_BFP8;
@@ -762,7 +817,7 @@ static int prefill_impl(void *out, int64_t out_batch_stride, int64_t out_head_st
     TTPA_REQUIRE(workspace_bytes >= 0 && (workspace != nullptr || workspace_bytes == 0),
                  "prefill: workspace_bytes %lld with a null workspace", (long long)workspace_bytes);
     const int64_t need = expand_bytes(batch, table_width, kv_heads, block_size, head_size);
-    if (workspace && aligned16(workspace) && (int64_t)batch * table_width < (1ll << 31) && workspace_bytes >= need) {
+    if (stream_expands(a, head_size) && workspace && aligned16(workspace) && (int64_t)batch * table_width < (1ll << 31) && workspace_bytes >= need) {
       a.expand = workspace;  // (a smaller one is not an error: the pass expands tile by tile instead)
       workspace = static_cast<unsigned char *>(workspace) + need;
       workspace_bytes -= need;
@@ -770,11 +825,6 @@ static int prefill_impl(void *out, int64_t out_batch_stride, int64_t out_head_st
   }
   a.part_acc = nullptr, a.part_bytes = 0, a.parts = 1;
   if (page_table && workspace && aligned16(workspace)) a.part_acc = static_cast<float *>(workspace), a.part_bytes = workspace_bytes;
-  {
-    // (TTPA_PREFILL_STREAM=0, read on every call, sends every shape through the plain loop)
-    const char *e = getenv("TTPA_PREFILL_STREAM");
-    a.stream = e ? atoi(e) : 1;
-  }
   a.bs_magic = block_size >= 2 ? (uint32_t)((1ull << 32) / (uint32_t)block_size) + 1u : 0u;
   a.fill_kc = a.fill_vc = nullptr;
   a.fill_pt = nullptr, a.fill_pt_rs = 0, a.fill_bidx = nullptr, a.fill_bidx_i64 = 0, a.fill_rows = 0;
@@ -841,9 +891,11 @@ extern "C" int64_t ttpa_sdpa_prefill_scratch_bytes(int32_t batch, int32_t q_head
   PrefillArgs a = {};
   a.pt = &some_table, a.stream = 1;
   a.batch = batch, a.hq = q_heads, a.hkv = kv_heads, a.sq = q_len, a.bs = block_size, a.w = table_width;
-  const int64_t expansion = stream_expands(a, head_size)
-      ? ttpa_sdpa_prefill_workspace_bytes(batch, kv_heads, head_size, block_size, table_width, kv_format) : 0;
-  return kv_format == TTPA_KV_BFP8 && expansion == 0 ? 0 : expansion + stream_part_bytes(a, head_size);
+  if (kv_format == TTPA_KV_BFP8) {
+    if (!stream_expands(a, head_size)) return plain_part_bytes(a, head_size, true);
+    return ttpa_sdpa_prefill_workspace_bytes(batch, kv_heads, head_size, block_size, table_width, kv_format) + stream_part_bytes(a, head_size);
+  }
+  return stream_serves(a, head_size) ? stream_part_bytes(a, head_size) : plain_part_bytes(a, head_size, false);
 }
 
 extern "C" int ttpa_sdpa_prefill_fill(

@@ -62,7 +62,7 @@ struct PrefillArgs {
   int64_t part_bytes;
   int parts, parts_one;  // shares of the keys at most; with one workgroup per CU
   int split_from;        // launches whose last row block has fewer 32-key blocks are not split
-  int part_stride;       // workgroups per part
+  int part_min;          // 32-key blocks of a part at least
 };
 
 // key / block_size without a division instruction sequence (about 30 instructions each, and the

@@ -1,0 +1,162 @@
+// Prefill passes of few query rows over many cached keys, split over the keys: several workgroups per row block, each
+// with a share of the keys, hand float accumulators to prefill_merge_kernel.  Shared by the two loops
+// (prefill_stream.hip, prefill.hip), whose lanes hold the accumulators alike.
+#pragma once
+
+#include "prefill_common.h"
+
+#include <algorithm>
+
+namespace ttpa {
+namespace {
+
+// ---- splitting over the keys --------------------------------------------------------------------
+// Splitting costs a second launch (1.4 us, also where the kernel then does not split), the start of more
+// workgroups, and 64 KiB of float accumulators written and read per part and workgroup; it saves about 0.48 us per
+// 32-key block that a workgroup need not walk.  How many blocks there are is in device memory (the host sees the
+// page table's width), so the host launches the most parts that may be wanted and the kernel decides, as does the
+// merge kernel with the same function.  Attention of a pass in us, unsplit / split, by workgroups of the unsplit launch:
+//    8 (32 rows, 32 / 8 heads):   10 blocks 12.8 / 13.6, 16 blocks 15.9 / 13.7, 64 blocks 38.9 / 16.1
+//   32 (128 rows, 32 / 8 heads):  10 blocks 12.9 / 14.7, 16 blocks 16.0 / 15.2, 64 blocks 39.4 / 23.8
+//   64 (4 x 64 rows, 32 / 8):     16 blocks 16.1 / 17.7, 32 blocks 24.0 / 21.9, 64 blocks 39.4 / 23.7
+//  128 (512 rows, 32 / 8 heads):  32 blocks 23.6 / 27.1, 64 blocks 38.5 / 35.0, 128 blocks 68.8 / 46.9
+//  192 (3 x 256 rows, 32 / 8):    64 blocks 40.0 / 41.8, 96 blocks 55.1 / 53.8, 256 blocks 131 / 115
+//  256 (512 rows, 64 / 8 heads):  64 blocks 41.2 / 47.3, 128 blocks 76.9 / 77.8, 256 blocks 145 / 138
+// so (the streaming loop) from 16 blocks on, or 7 / 16 of the number of workgroups, or half of it where a split leaves no CU to itself.  The last
+// row block decides for all: where some are split and others are not, the launch is as long as without a split and the merge comes
+// on top (4 x 64 rows of 32 / 8 heads, 23 and 24 blocks, the pass 27 us, 22 without a split).
+// The plain loop's passes (prefill.hip) are longer per block: 0.49 us at head size 64, 1.2 at 256, 0.72 and 1.15 where it expands
+// block-float-8 blocks of 64 and 128 on their way into LDS.  So its parts may be shorter and a launch is split from fewer blocks:
+// whole passes (fill and attention), before there was a split / with it:
+//   head size 64, 8 / 8 heads:   1 x 224 rows behind 320 tokens 17.1 / 13.5, 1216 30.5 / 15.1, 8192 136 / 18.9; 4 x 64 behind 640 20.5 / 14.5
+//   head size 64, 64 / 8 heads:  1 x 128 rows behind 640 tokens 21.9 / 18.5, 2368 47.1 / 24.4
+//   head size 256, 16 / 8 heads: 5 x 192 rows behind 832 tokens 67 / 49; 1 x 32 behind 256 23.8 / 20.7, 2368 97.9 / 32.9
+//   block-float-8, 8 / 8 of 64:  1 x 128 rows behind 640 tokens 26.9 / 17.3, 2368 65 / 18.8
+// Under a page table that holds little more than the blocks to split from, the parts would be few and the merge launch (1.4 us)
+// be there for nothing where the pass reads less of it: 1 x 32 rows behind 128 tokens 10.4 us, 12.4 with.
+struct SplitRule {
+  int wgs_per_cu;               // workgroup slots of a CU
+  int min_part, min_split;      // 32-key blocks per part at least; blocks from which on a launch is split
+  int table_percent;            // the page table holds at least this many hundredths of the blocks to split from
+  int block_cost;               // of a 32-key block, in hundredths of the streaming loop's
+};
+constexpr SplitRule kStreamSplit = {2, 8, 16, 100, 100};  // (80 KiB of LDS per workgroup)
+constexpr SplitRule plain_split(int d, bool bfp8) { return {d <= 128 ? 2 : 1, 4, 8, bfp8 ? 125 : 150, d == 256 ? 300 : bfp8 ? 225 : 150}; }
+// Parts up to one workgroup per CU; twice as many, which then share a CU's matrix pipes, from this many blocks per part
+// on (128 workgroups, 2 / 4 parts: 64 blocks 35.0 / 35.6 us, 80 blocks 43.5 / 41.5, 96 blocks 43.6 / 40.8, 256 blocks
+// 82.5 / 77.3).
+constexpr int kSharedPartBlocks = 20;
+constexpr int kMaxParts = 16;
+constexpr int kBlockKeys = 32;
+constexpr int part_acc_floats(int d) { return kRowsPerWave * d; }  // accumulators of one (part, head, row block)
+
+// Blocks of a part (whole 64-key tiles) in a launch whose first query row is at `offset`; a row block of no more is not split.
+__device__ __forceinline__ int blocks_per_part(const PrefillArgs &a, int offset) {
+  const int most = max(((a.causal ? min(a.skv, offset + a.sq) : a.skv) + kBlockKeys - 1) / kBlockKeys, 1);  // of the last row block
+  if (most < a.split_from) return most;
+  const int shared = (most + a.parts - 1) / a.parts;
+  const int share = shared >= kSharedPartBlocks ? shared : max((most + a.parts_one - 1) / a.parts_one, a.part_min);
+  return (share + 1) & ~1;
+}
+
+// Accumulators and (reference, sum) rows of the parts: [part][batch][head][row block], the statistics
+// behind all accumulators.
+struct PartLayout {
+  int64_t slots;  // (part, batch entry, head, row block) combinations
+  int row_blocks;
+};
+__host__ __device__ inline PartLayout part_layout(const PrefillArgs &a, int rows_per_wg) {
+  const int rb = (a.sq + rows_per_wg - 1) / rows_per_wg * (rows_per_wg / kRowsPerWave);
+  return {(int64_t)a.parts * a.batch * a.hq * rb, rb};
+}
+
+// Merges the parts of a row block: out = sum_p 2^(m_p - M) acc_p / sum_p 2^(m_p - M) l_p.  One workgroup per
+// (row block, head, batch entry); thread (n, g) takes row n and head-dim elements 16 g .. 16 g + 15, which lie in
+// register groups 2 g and 2 g + 1 of lanes n and n + 32 (prefill_stream_kernel's lane holds elements
+// 8 group + 4 (lane / 32) .. + 3): 512 consecutive bytes per read of 32 lanes, whole 32-byte pieces of a row per
+// write.  Memory bound: 34 MB of accumulators (512 rows, 32 heads, 4 parts) in 7.9 us.
+template <int D, int RPW>
+__global__ __launch_bounds__(2 * D) void prefill_merge_kernel(PrefillArgs a) {
+  const int rb = blockIdx.x, hq = blockIdx.y, b = blockIdx.z;
+  const int qt = rb / RPW;
+  const int n = threadIdx.x & 31, g = threadIdx.x >> 5;
+  const int offset = a.causal ? chunk_offset(a.chunk_start, a.sq, a.skv) : 0;
+  const int wg_last_row = min(a.sq, (qt + 1) * kRowsPerWave * RPW) - 1;
+  const int kv_end = a.causal ? min(a.skv, offset + wg_last_row + 1) : a.skv;
+  const int nblk = (kv_end + kBlockKeys - 1) / kBlockKeys;
+  const int share = blocks_per_part(a, offset);
+  if (share >= nblk) return;  // one workgroup saw all keys and wrote the output
+  const int active = (nblk + share - 1) / share;
+  const PartLayout lay = part_layout(a, kRowsPerWave * RPW);
+  const int64_t step = (int64_t)a.batch * a.hq * lay.row_blocks;
+  const int64_t at = ((int64_t)b * a.hq + hq) * lay.row_blocks + rb;
+  const float *acc = a.part_acc + at * part_acc_floats(D) + (8 * g) * 64 + 4 * n;
+  const float *stats = a.part_acc + lay.slots * part_acc_floats(D) + at * (2 * kRowsPerWave) + 2 * n;
+  float m[kMaxParts], l[kMaxParts];
+  float top = -INFINITY;
+#pragma unroll
+  for (int p = 0; p < kMaxParts; ++p) {
+    const int q = min(p, active - 1);
+    const float2 s = *reinterpret_cast<const float2 *>(stats + q * step * (2 * kRowsPerWave));
+    m[p] = s.x, l[p] = p < active ? s.y : 0.f;
+    top = fmaxf(top, m[p]);
+  }
+  float sum = 0.f;
+  float o[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) o[i] = 0.f;
+  // four parts' accumulators in flight at a time; parts past the last repeat it with weight 0
+  for (int p0 = 0; p0 < active; p0 += 4) {
+    float4 v[4][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float *src = acc + min(p0 + j, active - 1) * step * part_acc_floats(D);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[j][i] = *reinterpret_cast<const float4 *>(src + (i >> 1) * 256 + (i & 1) * 128);  // group 2 g + i / 2, lane half i % 2
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float w = 0.f;
+#pragma unroll
+      for (int p = 0; p < kMaxParts; ++p)
+        if (p == p0 + j && p < active) w = __builtin_amdgcn_exp2f(m[p] - top), sum = fmaf(w, l[p], sum);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        o[4 * i] = fmaf(w, v[j][i].x, o[4 * i]), o[4 * i + 1] = fmaf(w, v[j][i].y, o[4 * i + 1]);
+        o[4 * i + 2] = fmaf(w, v[j][i].z, o[4 * i + 2]), o[4 * i + 3] = fmaf(w, v[j][i].w, o[4 * i + 3]);
+      }
+    }
+  }
+  const int row = rb * kRowsPerWave + n;
+  if (row >= a.sq) return;
+  const float inv = 1.0f / sum;
+  uint16_t *op = a.out + b * a.out_bs + hq * a.out_hs + (int64_t)row * a.out_ts + 16 * g;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    *reinterpret_cast<uint2 *>(op + 4 * i) = make_uint2(pack_bf16x2(o[4 * i] * inv, o[4 * i + 1] * inv), pack_bf16x2(o[4 * i + 2] * inv, o[4 * i + 3] * inv));
+}
+
+// Workgroups of the launch without a split, and what it may be split into: as many parts as fill the workgroup slots of
+// every CU once, if its row blocks leave at least half of them empty and its page table is wide enough to be split at all.
+inline void set_parts(PrefillArgs &a, int heads_per_wg, const SplitRule &rule) {
+  int cus = device_cus();
+  if (cus <= 0) cus = 256;
+  const int rows = kRowsPerWave * 4 / heads_per_wg;
+  const int64_t wgs = (int64_t)a.batch * (a.hq / heads_per_wg) * ((a.sq + rows - 1) / rows);
+  const int blocks = (int)(((int64_t)a.w * a.bs + kBlockKeys - 1) / kBlockKeys);
+  const int most = std::min(kMaxParts, (blocks + rule.min_part - 1) / rule.min_part);
+  const int64_t from = 2 * wgs <= cus ? 7 * wgs / 16 : std::min<int64_t>(wgs, rule.wgs_per_cu * cus) / 2;
+  a.split_from = (int)std::max<int64_t>(rule.min_split, 100 * from / rule.block_cost);
+  a.part_min = rule.min_part;
+  a.parts = blocks < a.split_from * rule.table_percent / 100 ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>(rule.wgs_per_cu * cus / wgs, most));
+  a.parts_one = (int)std::max<int64_t>(1, std::min<int64_t>(cus / wgs, most));
+}
+
+inline int64_t part_bytes(PrefillArgs a, int heads_per_wg, const SplitRule &rule, int d) {
+  set_parts(a, heads_per_wg, rule);
+  if (a.parts <= 1) return 0;
+  return part_layout(a, kRowsPerWave * 4 / heads_per_wg).slots * (part_acc_floats(d) + 2 * kRowsPerWave) * (int64_t)sizeof(float);
+}
+
+}  // namespace
+}  // namespace ttpa

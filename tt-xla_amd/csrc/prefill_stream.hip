@@ -18,7 +18,7 @@
 // to prefill_merge_kernel.  512 rows behind 8192 tokens: blocks of 64 139 -> 80 us for the pass, blocks of 32
 // 231 -> 81 us (unsplit on the plain loop before); 256 rows of 16 / 16 heads behind 8192 228 -> 67 us.  Blocks
 // of 32 alone, where nothing is split: 4 x 512 rows behind 4096 tokens 180 -> 144 us.
-#include "prefill_common.h"
+#include "prefill_parts.h"
 #include "build/prefill_stream_asm.h"
 
 #include <algorithm>
@@ -28,7 +28,6 @@ namespace ttpa {
 namespace {
 
 constexpr int kD = 128;
-constexpr int kBlockKeys = 32;
 
 // kPaged: cache blocks of whole 64-key tiles (two 32-key blocks share a table entry); kPaged32: of whole
 // 32-key blocks (an entry per block costs scalar instructions in every iteration, not in every other one)
@@ -199,49 +198,6 @@ __device__ __forceinline__ void stream_items_paged32(StreamRequests &r, StreamIt
                : "memory", "vcc", "scc", "m0", "s86", "s87", TTPA_STREAM_LOOP_CLOBBERS);
 }
 
-// ---- splitting over the keys --------------------------------------------------------------------
-// Splitting costs a second launch (1.4 us, also where the kernel then does not split), the start of more
-// workgroups, and 64 KiB of float accumulators written and read per part and workgroup; it saves about 0.48 us per
-// 32-key block that a workgroup need not walk.  How many blocks there are is in device memory (the host sees the
-// page table's width), so the host launches the most parts that may be wanted and the kernel decides, as does the
-// merge kernel with the same function.  Attention of a pass in us, unsplit / split, by workgroups of the unsplit launch:
-//    8 (32 rows, 32 / 8 heads):   10 blocks 12.8 / 13.6, 16 blocks 15.9 / 13.7, 64 blocks 38.9 / 16.1
-//   32 (128 rows, 32 / 8 heads):  10 blocks 12.9 / 14.7, 16 blocks 16.0 / 15.2, 64 blocks 39.4 / 23.8
-//   64 (4 x 64 rows, 32 / 8):     16 blocks 16.1 / 17.7, 32 blocks 24.0 / 21.9, 64 blocks 39.4 / 23.7
-//  128 (512 rows, 32 / 8 heads):  32 blocks 23.6 / 27.1, 64 blocks 38.5 / 35.0, 128 blocks 68.8 / 46.9
-//  192 (3 x 256 rows, 32 / 8):    64 blocks 40.0 / 41.8, 96 blocks 55.1 / 53.8, 256 blocks 131 / 115
-//  256 (512 rows, 64 / 8 heads):  64 blocks 41.2 / 47.3, 128 blocks 76.9 / 77.8, 256 blocks 145 / 138
-// so from 16 blocks on, or 7 / 16 of the number of workgroups, or half of it where a split leaves no CU to itself.  The last
-// row block decides for all: where some are split and others are not, the launch is as long as without a split and the merge comes
-// on top (4 x 64 rows of 32 / 8 heads, 23 and 24 blocks, the pass 27 us, 22 without a split).
-constexpr int kMinPartBlocks = 8, kMinSplitBlocks = 16;
-// Parts up to one workgroup per CU; twice as many, which then share a CU's matrix pipes, from this many blocks per part
-// on (128 workgroups, 2 / 4 parts: 64 blocks 35.0 / 35.6 us, 80 blocks 43.5 / 41.5, 96 blocks 43.6 / 40.8, 256 blocks
-// 82.5 / 77.3).
-constexpr int kSharedPartBlocks = 20;
-constexpr int kMaxParts = 16;
-constexpr int kPartAccFloats = kRowsPerWave * kD;  // accumulators of one (part, head, row block)
-
-// Blocks of a part (whole 64-key tiles) in a launch whose first query row is at `offset`; a row block of no more is not split.
-__device__ __forceinline__ int blocks_per_part(const PrefillArgs &a, int offset) {
-  const int most = max(((a.causal ? min(a.skv, offset + a.sq) : a.skv) + kBlockKeys - 1) / kBlockKeys, 1);  // of the last row block
-  if (most < a.split_from) return most;
-  const int shared = (most + a.parts - 1) / a.parts;
-  const int share = shared >= kSharedPartBlocks ? shared : max((most + a.parts_one - 1) / a.parts_one, kMinPartBlocks);
-  return (share + 1) & ~1;
-}
-
-// Accumulators and (reference, sum) rows of the parts: [part][batch][head][row block], the statistics
-// behind all accumulators.
-struct PartLayout {
-  int64_t slots;  // (part, batch entry, head, row block) combinations
-  int row_blocks;
-};
-__host__ __device__ inline PartLayout part_layout(const PrefillArgs &a, int rows_per_wg) {
-  const int rb = (a.sq + rows_per_wg - 1) / rows_per_wg * (rows_per_wg / kRowsPerWave);
-  return {(int64_t)a.parts * a.batch * a.hq * rb, rb};
-}
-
 template <int HPW, int FORM>
 __global__ __launch_bounds__(256, 2) void prefill_stream_kernel(PrefillArgs a) {
   constexpr int RPW = 4 / HPW;  // row blocks per workgroup
@@ -263,8 +219,7 @@ __global__ __launch_bounds__(256, 2) void prefill_stream_kernel(PrefillArgs a) {
   // The part is the slowest index: the workgroups of part 0, the only ones with work where the keys are few, are dealt over the
   // XCDs and CUs as in a launch that is not split.  (As the fastest index, they met on half of the CUs or a quarter: 256
   // workgroups over 512 keys 20.5 us, 16.3 this way.)
-  const int part = PAGED ? wg / a.part_stride : 0;
-  if (PAGED) wg -= part * a.part_stride;
+  const int part = PAGED ? blockIdx.y : 0;
   const int xcd = wg & 7, slot = wg >> 3;
   const int yl = slot / a.spg;
   const int y = yl * 8 + xcd;
@@ -377,8 +332,8 @@ __global__ __launch_bounds__(256, 2) void prefill_stream_kernel(PrefillArgs a) {
     if (!whole) {
       const PartLayout lay = part_layout(a, kRowsPerWave * RPW);
       const int64_t at = (((int64_t)part * a.batch + b) * a.hq + hq) * lay.row_blocks + qt * RPW + wave / HPW;
-      out_part.acc = uni(reinterpret_cast<uint64_t>(a.part_acc + at * kPartAccFloats));
-      out_part.stats = uni(reinterpret_cast<uint64_t>(a.part_acc + lay.slots * kPartAccFloats + at * (2 * kRowsPerWave)));
+      out_part.acc = uni(reinterpret_cast<uint64_t>(a.part_acc + at * part_acc_floats(D)));
+      out_part.stats = uni(reinterpret_cast<uint64_t>(a.part_acc + lay.slots * part_acc_floats(D) + at * (2 * kRowsPerWave)));
     }
   }
   // Q fragments behind the requests (B operand: lane n = query row, 8 head-dim elements per k-step)
@@ -442,92 +397,6 @@ __global__ __launch_bounds__(256, 2) void prefill_stream_kernel(PrefillArgs a) {
   }
 }
 
-// Merges the parts of a row block: out = sum_p 2^(m_p - M) acc_p / sum_p 2^(m_p - M) l_p.  One workgroup per
-// (row block, head, batch entry); thread (n, g) takes row n and head-dim elements 16 g .. 16 g + 15, which lie in
-// register groups 2 g and 2 g + 1 of lanes n and n + 32 (prefill_stream_kernel's lane holds elements
-// 8 group + 4 (lane / 32) .. + 3): 512 consecutive bytes per read of 32 lanes, whole 32-byte pieces of a row per
-// write.  Memory bound: 34 MB of accumulators (512 rows, 32 heads, 4 parts) in 7.9 us.
-template <int RPW>
-__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
-  const int rb = blockIdx.x, hq = blockIdx.y, b = blockIdx.z;
-  const int qt = rb / RPW;
-  const int n = threadIdx.x & 31, g = threadIdx.x >> 5;
-  const int offset = a.causal ? chunk_offset(a.chunk_start, a.sq, a.skv) : 0;
-  const int wg_last_row = min(a.sq, (qt + 1) * kRowsPerWave * RPW) - 1;
-  const int kv_end = a.causal ? min(a.skv, offset + wg_last_row + 1) : a.skv;
-  const int nblk = (kv_end + kBlockKeys - 1) / kBlockKeys;
-  const int share = blocks_per_part(a, offset);
-  if (share >= nblk) return;  // one workgroup saw all keys and wrote the output
-  const int active = (nblk + share - 1) / share;
-  const PartLayout lay = part_layout(a, kRowsPerWave * RPW);
-  const int64_t step = (int64_t)a.batch * a.hq * lay.row_blocks;
-  const int64_t at = ((int64_t)b * a.hq + hq) * lay.row_blocks + rb;
-  const float *acc = a.part_acc + at * kPartAccFloats + (8 * g) * 64 + 4 * n;
-  const float *stats = a.part_acc + lay.slots * kPartAccFloats + at * (2 * kRowsPerWave) + 2 * n;
-  float m[kMaxParts], l[kMaxParts];
-  float top = -INFINITY;
-#pragma unroll
-  for (int p = 0; p < kMaxParts; ++p) {
-    const int q = min(p, active - 1);
-    const float2 s = *reinterpret_cast<const float2 *>(stats + q * step * (2 * kRowsPerWave));
-    m[p] = s.x, l[p] = p < active ? s.y : 0.f;
-    top = fmaxf(top, m[p]);
-  }
-  float sum = 0.f;
-  float o[16];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) o[i] = 0.f;
-  // four parts' accumulators in flight at a time; parts past the last repeat it with weight 0
-  for (int p0 = 0; p0 < active; p0 += 4) {
-    float4 v[4][4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float *src = acc + min(p0 + j, active - 1) * step * kPartAccFloats;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[j][i] = *reinterpret_cast<const float4 *>(src + (i >> 1) * 256 + (i & 1) * 128);  // group 2 g + i / 2, lane half i % 2
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      float w = 0.f;
-#pragma unroll
-      for (int p = 0; p < kMaxParts; ++p)
-        if (p == p0 + j && p < active) w = __builtin_amdgcn_exp2f(m[p] - top), sum = fmaf(w, l[p], sum);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        o[4 * i] = fmaf(w, v[j][i].x, o[4 * i]), o[4 * i + 1] = fmaf(w, v[j][i].y, o[4 * i + 1]);
-        o[4 * i + 2] = fmaf(w, v[j][i].z, o[4 * i + 2]), o[4 * i + 3] = fmaf(w, v[j][i].w, o[4 * i + 3]);
-      }
-    }
-  }
-  const int row = rb * kRowsPerWave + n;
-  if (row >= a.sq) return;
-  const float inv = 1.0f / sum;
-  uint16_t *op = a.out + b * a.out_bs + hq * a.out_hs + (int64_t)row * a.out_ts + 16 * g;
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    *reinterpret_cast<uint2 *>(op + 4 * i) = make_uint2(pack_bf16x2(o[4 * i] * inv, o[4 * i + 1] * inv), pack_bf16x2(o[4 * i + 2] * inv, o[4 * i + 3] * inv));
-}
-
-// Workgroups of the launch without a split, and what it may be split into: as many parts as fill the two workgroup slots of
-// every CU once, if its row blocks leave at least half of them empty and its page table is wide enough to be split at all.
-void set_parts(PrefillArgs &a, int heads_per_wg) {
-  int cus = device_cus();
-  if (cus <= 0) cus = 256;
-  const int rows = kRowsPerWave * 4 / heads_per_wg;
-  const int64_t wgs = (int64_t)a.batch * (a.hq / heads_per_wg) * ((a.sq + rows - 1) / rows);
-  const int blocks = a.w * (a.bs / kBlockKeys);
-  const int most = std::min(kMaxParts, (blocks + kMinPartBlocks - 1) / kMinPartBlocks);
-  a.split_from = (int)std::max<int64_t>(kMinSplitBlocks, 2 * wgs <= cus ? 7 * wgs / 16 : std::min<int64_t>(wgs, 2 * cus) / 2);
-  a.parts = blocks < a.split_from ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>(2 * cus / wgs, most));
-  a.parts_one = (int)std::max<int64_t>(1, std::min<int64_t>(cus / wgs, most));
-}
-
-int64_t part_bytes(PrefillArgs a, int heads_per_wg) {
-  set_parts(a, heads_per_wg);
-  if (a.parts <= 1) return 0;
-  return part_layout(a, kRowsPerWave * 4 / heads_per_wg).slots * (kPartAccFloats + 2 * kRowsPerWave) * (int64_t)sizeof(float);
-}
-
 int heads_per_workgroup(const PrefillArgs &a) {
   const int g = a.hq / a.hkv;
   return g % 4 == 0 ? 4 : g % 2 == 0 ? 2 : 1;
@@ -553,7 +422,7 @@ int launch_form(const PrefillArgs &a, hipStream_t st) {
   // (read on every call) an experiment's override: several row blocks per workgroup, each over all of its keys
   const char *e = HPW == 4 && (FORM == kDense || FORM == kPaged) ? getenv("TTPA_PREFILL_WGS_PER_GROUP") : nullptr;
   const int per_group = e ? atoi(e) : 0;
-  if (PAGED && per_group <= 0 && a.part_acc && a.part_bytes >= part_bytes(a, HPW)) set_parts(b, HPW);
+  if (PAGED && per_group <= 0 && a.part_acc && a.part_bytes >= part_bytes(a, HPW, kStreamSplit, kD)) set_parts(b, HPW, kStreamSplit);
   if (per_group > 0) {
     b.spg = std::min(nqt, per_group);
   } else if (HPW == 4 && (FORM == kDense || FORM == kPaged) && b.parts == 1) {
@@ -566,13 +435,12 @@ int launch_form(const PrefillArgs &a, hipStream_t st) {
     const int one_round = (2 * cus + ny8 * 8 - 1) / (ny8 * 8);
     b.spg_even = one_round < nqt && nqt % one_round == 0 ? one_round : 0;
   }
-  b.part_stride = b.spg * ny8 * 8;
-  int grid = b.part_stride * b.parts;
+  int grid = b.spg * ny8 * 8;
   if (!PAGED && FORM != kDenseWide && a.fill_kc) grid = grid_with_fill(b, grid, kD);
-  launch_dominant(&prefill_stream_kernel<HPW, FORM>, dim3(grid), dim3(256), (size_t)TTPA_STREAM_LDS_BYTES, st, b);
+  launch_dominant(&prefill_stream_kernel<HPW, FORM>, dim3(grid, b.parts), dim3(256), (size_t)TTPA_STREAM_LDS_BYTES, st, b);
   if (const int rc = check_launch("sdpa_prefill")) return rc;
   if (b.parts > 1) {
-    prefill_merge_kernel<RPW><<<dim3((b.sq + kRowsPerWave - 1) / kRowsPerWave, b.hq, b.batch), dim3(256), 0, st>>>(b);
+    prefill_merge_kernel<kD, RPW><<<dim3((b.sq + kRowsPerWave - 1) / kRowsPerWave, b.hq, b.batch), dim3(2 * kD), 0, st>>>(b);
     return check_launch("sdpa_prefill (merge of the parts)");
   }
   return TTPA_OK;
@@ -597,17 +465,18 @@ bool stream_serves(const PrefillArgs &a, int head_size) {
 }
 
 int64_t stream_part_bytes(const PrefillArgs &a, int head_size) {
-  return a.pt && stream_serves(a, head_size) ? part_bytes(a, heads_per_workgroup(a)) : 0;
+  return a.pt && stream_serves(a, head_size) ? part_bytes(a, heads_per_workgroup(a), kStreamSplit, kD) : 0;
 }
 
-// A pass of one workgroup per head group reads every block once, so mode 4's expansion on the way into LDS is not repeated either:
-// the copies, a trip through memory in front of the attention, pay where they are few or where the keys may be split
-// (16 / 16 heads, copies / mode 4: 1 x 128 rows over 256 keys 17.4 / 19.3 us, 4 x 64 rows over 320 keys 22.7 / 20.5; 1 x 128
-// rows over 2176 keys, where the copies let it be split, 32.0 / 78.6).
+// Where a block is read by at most two workgroups (row blocks times head groups of a KV head), mode 4 expands it as it reads it:
+// split over the keys that costs less than the copies, a launch and a trip through memory in front of the attention.  Passes in
+// us, copies / mode 4: 1 x 32 rows behind 512 tokens, 64 / 8 heads 23.1 / 18.8; 4 x 32 rows of 32 / 8 behind 1024 32.1 / 25.3, 4096 49.3 /
+// 38.7; 8 x 128 of 16 / 16 behind 4096 167 / 75.6; two row blocks: 4 x 64 of 32 / 8 behind 512 29.5 / 24.9, 8 x 256 of 16 / 16 behind 512
+// 46.1 / 48.2, behind 4096 195 / 128.  Four workgroups: 2 x 64 of 64 / 8 behind 4096 49.5 / 55.6; three: 2 x 96 of 32 / 8 46.7 / 50.0.
 bool stream_expands(const PrefillArgs &a, int head_size) {
   if (!stream_serves(a, head_size)) return false;
-  const int hpw = heads_per_workgroup(a);
-  return a.sq > kRowsPerWave * 4 / hpw || (int64_t)a.batch * a.w * a.bs * a.hkv <= 8192 || part_bytes(a, hpw) > 0;
+  const int hpw = heads_per_workgroup(a), rows = kRowsPerWave * 4 / hpw;
+  return (int64_t)((a.sq + rows - 1) / rows) * (a.hq / hpw / a.hkv) > 2;
 }
 
 int launch_stream_wide(const PrefillArgs &a, hipStream_t st) {

@@ -671,7 +671,7 @@ def _prefill(query, key, value, page_table, chunk_start, attn_mask, is_causal, s
     # scratch for what the library's fastest loop can use it for: bfloat16 copies of the blocks that a pass
     # over block-float-8 caches reads, partial results where few query rows meet many keys
     ws_ptr, ws_bytes = 0, 0
-    if page_table is not None and d == 128 and bs % 32 == 0 and not window and attn_mask is None:
+    if page_table is not None and not window and attn_mask is None:
         need = int(N.lib().ttpa_sdpa_prefill_scratch_bytes(b, hq, hkv, s, d, bs, w, fmt))
         if 0 < need <= _EXPANSION_LIMIT:
             try:
