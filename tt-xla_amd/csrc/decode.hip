@@ -300,6 +300,8 @@ __global__ __launch_bounds__(256, (D <= 128 && G <= 4) ? 2 : 1) void paged_decod
   process_tile(std::false_type{});
 }
 
+bool segment_units_forced() { return getenv("TTPA_DECODE_SEG_UNITS") != nullptr; }
+
 int segment_units(int default_units) {
   const char *e = getenv("TTPA_DECODE_SEG_UNITS");
   const int v = e ? atoi(e) : default_units;

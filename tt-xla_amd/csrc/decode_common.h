@@ -37,6 +37,7 @@ struct DecodeArgs {
   // of segment costs (its partial, the search, the next Q rows), so that equal ranges of units
   // take about equal time.  0: the list holds tiles only.
   int seg_units = 0;
+  int seg_free_tiles = -1;  // >= 0: lists of at most that many tiles have no such units, longer ones up to seg_units (build_prefix_units)
   // Partial outputs stored as bfloat16 (16-head latent kernel: a partial there is 16 heads x 512
   // values): a slot is G * D bfloat16 values, then G running maxima and G running sums as floats.
   int partial_bf16 = 0;
@@ -138,6 +139,38 @@ __device__ inline void build_prefix(const DecodeArgs &a, const void *__restrict_
     pref[u + 1] = run;
   }
   __syncthreads();
+}
+
+// build_prefix with a number of leading units per segment that follows the length of the list, for kernels whose ranges are long
+// per tile (the latent layers).  The units keep segment changes from piling up on a range where ranges hold several tiles; a list
+// that does not fill the ranges has none to weigh, and as no range is shorter than a tile and its units, they only made it
+// run on a fifth of the chip.  So: none up to seg_free_tiles tiles, then one, and one more per n_ranges tiles up to the
+// kernel's own number.  Up to 64 users (a user per lane, nothing to wait for); returns the number.
+// us per decode step with 4 (128 heads) or 3 (16) / as chosen here: 128 heads, one user over 500 tokens 48.3 / 33.4, 6 users of
+// 146 ... 1229 50.1 / 36.7, 16 of 200 ... 3000 57.3 / 50.3, 7 of 1384 ... 7377 54.1 / 49.7; 32 heads, 6 of 500 ... 5000
+// 41.4 / 30.1; 16 heads, one user over 1000 27.9 / 21.3, 8 of 300 ... 3000 28.7 / 27.2.  With none throughout: 30 users of
+// 500 ... 4000, 128 heads 75.6 instead of 64.4 with three; one user over 16000, 16 heads 38.4 instead of 32.3.
+template <int TILE = kTile>
+__device__ __forceinline__ int build_prefix_units(const DecodeArgs &a, const void *__restrict__ cur, int *pref, int *lens, int *wave_sums,
+                                                  int n_ranges) {
+  if (a.seg_free_tiles < 0 || a.users > kWave) {
+    build_prefix<TILE>(a, cur, pref, lens, wave_sums, a.seg_units);
+    return a.seg_units;
+  }
+  const int u = threadIdx.x & (kWave - 1);
+  int len = 0, nt = 0;
+  if (u < a.users) nt = tiles_of_user<TILE>(a, cur, u, len);
+  const int tiles = wave_prefix_sum(nt);
+  const int64_t over = (int64_t)__builtin_amdgcn_readlane(tiles, kWave - 1) * a.hkv - a.seg_free_tiles;
+  int extra = 0;
+  for (int64_t at = 0; extra < a.seg_units && over > at; at += n_ranges) ++extra;
+  const int users_to = __builtin_popcountll(__builtin_amdgcn_ballot_w64(nt > 0) & (~0ull >> (kWave - 1 - u)));
+  if (u == 0) pref[0] = 0;
+  if (u < a.users) pref[u + 1] = tiles + extra * users_to, lens[u] = len;
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  return extra;
 }
 
 // LDS probabilities are written as 16-bit values and read back as 32-bit pairs
@@ -744,6 +777,7 @@ inline size_t header_bytes(int users, int hkv) { return (((size_t)users * hkv * 
 int waves_for_device(double default_per_cu);
 // Units in front of every segment of the flat list (TTPA_DECODE_SEG_UNITS overrides, 0 ... 64).
 int segment_units(int default_units);
+bool segment_units_forced();  // whether the override is set
 constexpr int kWavesPerBlockHost = kWavesPerBlock;
 
 // Launches the block-float-8 VALU main kernel (decode_bfp8.hip); false = shape not built.

@@ -364,8 +364,7 @@ __global__ __launch_bounds__(256, 1) void paged_decode_latent16_kernel(
   __shared__ int s_wsum[kWavesPerBlock];
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
-  const int seg_units = a.seg_units;
-  build_prefix<TILE>(a, cur_pos, s_pref, s_len, s_wsum, seg_units);
+  const int seg_units = build_prefix_units<TILE>(a, cur_pos, s_pref, s_len, s_wsum, a.n_waves);
 
   const int lane = threadIdx.x & 63;
   const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -821,8 +820,7 @@ __global__ __launch_bounds__(256) void paged_decode_latent128_kernel(
   __shared__ int s_wsum[NWAVES];
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
-  const int seg_units = a.seg_units;
-  build_prefix(a, cur_pos, s_pref, s_len, s_wsum, seg_units);
+  const int seg_units = build_prefix_units(a, cur_pos, s_pref, s_len, s_wsum, a.n_waves);
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1467,6 +1465,7 @@ static int mla_decode_impl(void *out, int64_t out_user_stride, int64_t out_head_
     // (the partial, the next segment's Q and first step; 128 users of 512 ... 8192 tokens: 180 us with none,
     // 167 with two, 163 with three to five)
     a.seg_units = segment_units(4);
+    if (!segment_units_forced()) a.seg_free_tiles = a.n_waves;  // (a tile of 64 tokens per workgroup)
     if (head_size == 576 && head_dim_v == 512) ok = launch_latent128<576, 512>(a, w, st);
     else if (head_size == 576 && head_dim_v == 384) ok = launch_latent128<576, 384>(a, w, st);
     else if (head_size == 192 && head_dim_v == 128) ok = launch_latent128<192, 128>(a, w, st);
@@ -1494,6 +1493,7 @@ static int mla_decode_impl(void *out, int64_t out_user_stride, int64_t out_head_
     // three units in front of every segment of the flat list (a partial here is 32 KiB, a tile
     // 18 KiB): 130 us per step against 131-134 with none
     a.seg_units = segment_units(3);
+    if (!segment_units_forced()) a.seg_free_tiles = a.n_waves / 4;  // (tiles of 16 tokens: a range for each costs more in partials)
     // partials as bfloat16 (TTPA_LATENT_PARTIALS=f32, read on every call, keeps floats): half the
     // bytes written here and read by the merge
     const char *pf = getenv("TTPA_LATENT_PARTIALS");
@@ -1518,7 +1518,7 @@ static int mla_decode_impl(void *out, int64_t out_user_stride, int64_t out_head_
       return check_launch("paged_mla_decode");
     }
     a.n_waves = cus;
-    a.seg_units = 0;
+    a.seg_units = 0, a.seg_free_tiles = -1;
     a.partial_bf16 = 0;
     a.slot_floats = slot_floats_for(gseg, head_dim_v);
   }
