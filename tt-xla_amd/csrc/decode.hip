@@ -557,6 +557,10 @@ static int decode_impl(void *out, int64_t out_user_stride, int64_t out_head_stri
   // 32.0 us at 0 / 1 / 2 / 3 / 4), the VALU kernels none (8 / 8 heads: 52.1 / 53.3 / 53.8 us at
   // 0 / 1 / 2).  TTPA_DECODE_SEG_UNITS (read on every call) overrides.
   a.seg_units = segment_units(use_mfma16 ? 1 : use_mfma ? 2 : 0);
+  // ... and the 16x16 kernel none where the tiles do not fill the ranges (up to 64 users: build_prefix_units).  us per layer
+  // with one / none: one user of 32/8 heads over 2000 tokens 11.0 / 9.8, of 8/8 heads of 64 over 4000 11.1 / 9.9, 3 users of 8/2 with
+  // 233 ... 1960 10.9 / 9.5, block-float-8 over 2000 12.5 / 10.9; beyond: one user of 64/8 over 4000 (1000 tiles, 768 ranges) 11.8 / 12.6.
+  if (use_mfma16 && !segment_units_forced()) a.seg_free_tiles = a.n_waves;
   // one thread of the main grid per segment publishes the segment's partial slots
   if (!a.direct && (int64_t)users * kv_heads > (int64_t)a.n_waves * kWave)
     return fail(TTPA_ERR_UNSUPPORTED, "decode: %d x %d segments need a grid of more than %d wavefronts",

@@ -164,7 +164,8 @@ __device__ __forceinline__ int build_prefix_units(const DecodeArgs &a, const voi
   const int64_t over = (int64_t)__builtin_amdgcn_readlane(tiles, kWave - 1) * a.hkv - a.seg_free_tiles;
   int extra = 0;
   for (int64_t at = 0; extra < a.seg_units && over > at; at += n_ranges) ++extra;
-  const int users_to = __builtin_popcountll(__builtin_amdgcn_ballot_w64(nt > 0) & (~0ull >> (kWave - 1 - u)));
+  const uint64_t some = __builtin_amdgcn_ballot_w64(nt > 0);  // users with tiles, up to and with this lane's:
+  const int users_to = __builtin_amdgcn_mbcnt_hi((uint32_t)(some >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)some, 0)) + (nt > 0);
   if (u == 0) pref[0] = 0;
   if (u < a.users) pref[u + 1] = tiles + extra * users_to, lens[u] = len;
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

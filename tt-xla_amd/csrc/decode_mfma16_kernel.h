@@ -177,8 +177,8 @@ __global__ __launch_bounds__(DIRECT ? kWave *DIRECT : 256, (DIRECT || BFP8) && D
   __shared__ int s_wsum[kWavesPerBlock];
   extern __shared__ __attribute__((aligned(16))) uint8_t tiles[];
 
-  const int seg_units = a.seg_units;
-  if constexpr (DIRECT == 0) build_prefix<TILE>(a, cur_pos, s_pref, s_len, s_wsum, seg_units);
+  int seg_units = 0;
+  if constexpr (DIRECT == 0) seg_units = build_prefix_units<TILE>(a, cur_pos, s_pref, s_len, s_wsum, a.n_waves);
   const int lane = threadIdx.x & 63;
   const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 15, quad = lane >> 4;
