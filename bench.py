@@ -46,19 +46,19 @@ KERNEL_SOURCES = {
     "paged_decode_latent16_kernel": ["decode_wide.hip", "decode_common.h", "common.h"],
     "paged_decode_latent128_kernel": ["decode_wide.hip", "gen_latent_frag.py", "decode_common.h", "common.h"],
     "latent_prefill_kernel": ["decode_wide.hip", "gen_latent_frag.py", "decode_common.h", "common.h"],
-    "prefill_stream_kernel": ["prefill_stream.hip", "prefill_common.h", "gen_prefill_stream.py", "common.h"],
+    "prefill_stream_kernel": ["prefill_stream.hip", "prefill_parts.h", "prefill_common.h", "gen_prefill_stream.py", "common.h"],
 }
 MEASURED_TRAFFIC = {
     # workload: (kernel, hash of its sources, HBM bytes per launch: FETCH_SIZE and WRITE_SIZE of the
     # kernel, each scaled by what the same counter reads for a plain copy of known size, mean over
     # the rotating workload copies; the summaries under profiles/ hold the runs)
-    "config2": ("paged_decode_mfma16_kernel", "410306992a9b7e9b", 310401819),
-    "config5": ("paged_decode_mfma16_kernel", "410306992a9b7e9b", 168429456),
-    "config4": ("paged_decode_mfma16_kernel", "410306992a9b7e9b", 3415530563),
-    "config3": ("prefill_stream_kernel", "4aae0c7b51b8339c", 244868493),
-    "latent": ("paged_decode_latent16_kernel", "611a48caa3e35aca", 654199267),
-    "latent128": ("paged_decode_latent128_kernel", "75ff2b818e7d1cd4", 739359865),
-    "latent-prefill": ("latent_prefill_kernel", "75ff2b818e7d1cd4", 332250032),
+    "config2": ("paged_decode_mfma16_kernel", "4ce6db6ba974355a", 310434376),
+    "config5": ("paged_decode_mfma16_kernel", "4ce6db6ba974355a", 169705302),
+    "config4": ("paged_decode_mfma16_kernel", "4ce6db6ba974355a", 3415566290),
+    "config3": ("prefill_stream_kernel", "71eb60990b4e7f24", 244768677),
+    "latent": ("paged_decode_latent16_kernel", "c6436ec19a280f84", 654181074),
+    "latent128": ("paged_decode_latent128_kernel", "f15376b0d1795d27", 739370325),
+    "latent-prefill": ("latent_prefill_kernel", "f15376b0d1795d27", 332232245),
 }
 DECODE_KERNEL_NAME = {"config2": "paged_decode_mfma16_kernel", "config4": "paged_decode_mfma16_kernel",
                       "config5": "paged_decode_mfma16_kernel"}
