@@ -117,3 +117,36 @@ def test_chunks_that_start_outside_the_sequence(d, bs, start):
         held = torch.tensor([min(start, 1280)], dtype=torch.int32)
         want = O.chunked_sdpa(q[:, :, blind:], key, value, table, torch.clamp(held + blind, 0), d**-0.5)
         P._check(f"start {start} d{d}", got[:, :, blind:], want)
+
+
+def test_block_float_8_with_room_for_the_copies_only(monkeypatch):
+    """Scratch of ttpa_sdpa_prefill_workspace_bytes holds the copies and not the parts: the pass reads copies, unsplit."""
+    from tt_xla_amd import _native as N
+
+    users, hq, hkv, d, bs, start, lc = 1, 8, 8, 128, 64, 500, 100
+    g = torch.Generator().manual_seed(5)
+    nbpu = -(-(start + lc) // bs)
+    key, value, table = P._paged(g, users, nbpu, hkv, bs, d, False)
+    q = P._bf(g, users, hq, lc, d)
+    st = torch.tensor([start], dtype=torch.int32)
+    packed = [bfp8_codec.pack_cache(t) for t in (key, value)]
+    want = O.chunked_sdpa(q, *[bfp8_codec.unpack_cache(t, bs).to(torch.bfloat16) for t in packed], table, st, d**-0.5)
+    room = int(N.lib().ttpa_sdpa_prefill_workspace_bytes(users, hkv, d, bs, nbpu, 1))
+    parts = int(N.lib().ttpa_sdpa_prefill_scratch_bytes(users, hq, hkv, lc, d, bs, nbpu, 1))
+    blocks = torch.zeros(room, dtype=torch.uint8, device="cuda")
+    call = N.call
+
+    def with_room(size):
+        def wrapped(name, *a):
+            if name == "ttpa_sdpa_prefill_expanded":
+                a = a[:-3] + (blocks.data_ptr(), size, a[-1])
+            return call(name, *a)
+        return wrapped
+
+    args = [t.cuda() for t in (q, packed[0], packed[1], table, st)]
+    assert room < parts
+    for size in (room, room - 256):  # copies; neither copies nor parts
+        blocks.zero_()
+        monkeypatch.setattr(N, "call", with_room(size))
+        got = _pass(*args, d**-0.5)
+        P._check(f"copies only, {size} of {room} bytes, parts {parts}", got.cpu(), want)

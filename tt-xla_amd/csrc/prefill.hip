@@ -690,7 +690,7 @@ int launch(const PrefillArgs &a, hipStream_t st) {
     // With scratch from the caller, a pass that the hand-scheduled loop can serve reads bfloat16
     // copies of its blocks (written by one launch in front of it) instead of expanding every
     // tile once per workgroup on its way into LDS.
-    if (a.expand && stream_expands(a, D)) {
+    if (a.expand) {
       const int64_t blocks = (int64_t)a.batch * a.w;
       const int64_t cache_elems = blocks * a.hkv * a.bs * D;
       ExpandArgs e;
@@ -817,7 +817,9 @@ static int prefill_impl(void *out, int64_t out_batch_stride, int64_t out_head_st
     TTPA_REQUIRE(workspace_bytes >= 0 && (workspace != nullptr || workspace_bytes == 0),
                  "prefill: workspace_bytes %lld with a null workspace", (long long)workspace_bytes);
     const int64_t need = expand_bytes(batch, table_width, kv_heads, block_size, head_size);
-    if (stream_expands(a, head_size) && workspace && aligned16(workspace) && (int64_t)batch * table_width < (1ll << 31) && workspace_bytes >= need) {
+    // (a pass that would be split where it stands, but has no room for its parts, reads copies too)
+    const bool copies = stream_expands(a, head_size) || (stream_serves(a, head_size) && workspace_bytes < plain_part_bytes(a, head_size, true));
+    if (copies && workspace && aligned16(workspace) && (int64_t)batch * table_width < (1ll << 31) && workspace_bytes >= need) {
       a.expand = workspace;  // (a smaller one is not an error: the pass expands tile by tile instead)
       workspace = static_cast<unsigned char *>(workspace) + need;
       workspace_bytes -= need;
