@@ -121,3 +121,23 @@ def test_whole_segments_with_rows_of_odd_strides_and_parked_users(d, bfp8):
         assert torch.equal(plain.nan_to_num(9.0), eager.nan_to_num(9.0))
         (dev.q.float() @ dev.q.float().transpose(-1, -2)).sum().item()
     del keep, keep2, keep3
+
+
+@pytest.mark.parametrize("hq,hkv,d,window", [(16, 8, 64, 0), (12, 4, 64, 256), (16, 8, 128, 0), (24, 8, 128, 256)])
+def test_attention_alone_over_two_or_three_heads_stays_with_the_dot_product_kernel(monkeypatch, hq, hkv, d, window):
+    """Whatever the page table's width or the window: its weights are rounded against the maxima of sixteen tokens, so it is
+    closer to 64 bits than a whole segment (tests of closeness would need a margin; the same kernel gives the same bits)."""
+    gen = torch.Generator().manual_seed(hq + d)
+    users, bs = 5, 32
+    width = 272 * 1024 // (4 * d * bs)
+    k = torch.randn(users * width, hkv, bs, d, generator=gen).to(torch.bfloat16).cuda()
+    v = torch.randn(users * width, hkv, bs, d, generator=gen).to(torch.bfloat16).cuda()
+    table = torch.arange(users * width, dtype=torch.int32).reshape(users, width).cuda()
+    q = torch.randn(1, users, hq, d, generator=gen).to(torch.bfloat16).cuda()
+    cur = torch.tensor([0, 63, 127, 300, width * bs - 1], dtype=torch.int32).cuda()
+    got = []
+    for kernel in (None, "valu"):
+        monkeypatch.setenv("TTPA_DECODE_KERNEL", kernel) if kernel else monkeypatch.delenv("TTPA_DECODE_KERNEL", raising=False)
+        got.append(torch.ops.tt.paged_scaled_dot_product_attention_decode(
+            q, k, v, table, is_causal=True, cur_pos_tensor=cur, scale=d**-0.5, sliding_window_size=window or None))
+    assert torch.equal(got[0], got[1])

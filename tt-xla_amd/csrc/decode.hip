@@ -521,13 +521,14 @@ static int decode_impl(void *out, int64_t out_user_stride, int64_t out_head_stri
   }
   // A step whose new rows cannot be read in 16-byte pieces is an update launch and the attention behind it.
   const bool vec_ok = !k_new || (aligned16(k_new) && aligned16(v_new) && new_user_stride % 8 == 0 && new_head_stride % 8 == 0);
-  // (an explicit grid asks for ranges)
-  if (!mask && mfma16_ok && head_size <= 128 && block_size % (4096 / head_size / 2) == 0 &&
+  // Whole segments are for the groups that the kernel serves anyway: the attention alone over two or three heads per group of a
+  // bfloat16 cache stays with the dot-product kernel, whose error against 64 bits is the smaller one (1.95e-3; whole segments
+  // 2.03e-3 ... 2.13e-3, over 128 ... 1001 tokens).  (An explicit grid asks for ranges.)
+  if (!mask && use_mfma16 && head_size <= 128 && block_size % (4096 / head_size / 2) == 0 &&
       (forced == 5 || ((forced == 0 || forced == 3) && !getenv("TTPA_DECODE_WAVES_PER_CU")))) {
     int64_t tokens = (int64_t)table_width * block_size;
     if (sliding_window > 0) tokens = std::min<int64_t>(tokens, sliding_window);
     a.direct = direct_waves(users, kv_heads, head_size, kv_format, tokens, forced == 5);
-    if (a.direct) use_mfma16 = true, use_mfma = false;
   }
   // The matrix-core kernels get at most one workgroup per CU on a bfloat16 cache: the 32x32
   // kernel fills the CU's LDS with one, and the 16x16 kernel streams as fast with one as with the
