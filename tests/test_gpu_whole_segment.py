@@ -141,3 +141,37 @@ def test_attention_alone_over_two_or_three_heads_stays_with_the_dot_product_kern
         got.append(torch.ops.tt.paged_scaled_dot_product_attention_decode(
             q, k, v, table, is_causal=True, cur_pos_tensor=cur, scale=d**-0.5, sliding_window_size=window or None))
     assert torch.equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("kernel", ["direct", "ranges"])
+@pytest.mark.parametrize("hq,d", [(4, 64), (4, 128), (16, 128)])  # one head per group, where the weights have two parts; four
+def test_infinite_values_stay_infinite(monkeypatch, kernel, hq, d):
+    """An infinite V element makes its output infinite, of the same sign, whatever its weight is rounded to; two of
+    opposite signs make NaN; one behind the context makes nothing.  (Not in a segment's last partial, which the merge of
+    the ranges repeats with weight 0.)"""
+    monkeypatch.setenv("TTPA_DECODE_KERNEL", kernel)
+    gen = torch.Generator().manual_seed(hq + d)
+    users, hkv, bs, width = 3, 4, 32, 12
+    k = torch.randn(users * width, hkv, bs, d, generator=gen).to(torch.bfloat16)
+    v = torch.randn(users * width, hkv, bs, d, generator=gen).to(torch.bfloat16)
+    table = torch.arange(users * width, dtype=torch.int32).reshape(users, width)
+    cur = torch.tensor([129, 200, width * bs - 2], dtype=torch.int32)
+    inf = float("inf")
+    for u in range(users):
+        at = lambda t: (u * width + t // bs, slice(None), t % bs)  # noqa: E731
+        for column, t in enumerate(range(0, 40, 3)):
+            v[at(t)][..., column] = inf if column % 2 else -inf
+        v[at(7)][..., 30], v[at(31)][..., 30] = inf, -inf
+        v[at(int(cur[u]) + 1)][...] = inf
+    q = torch.randn(1, users, hq, d, generator=gen).to(torch.bfloat16)
+    k_new, v_new = (torch.randn(1, users, hkv, d, generator=gen).to(torch.bfloat16) for _ in range(2))
+    if kernel == "direct":
+        v_new[..., 40], v_new[..., 41] = inf, -inf
+    dev = [t.cuda() for t in (q, k, v, k_new, v_new, table, cur)]
+    got = torch.ops.tt.paged_update_kv_decode_(*dev, None, d**-0.5).cpu()
+    alone = torch.ops.tt.paged_scaled_dot_product_attention_decode(
+        dev[0], dev[1], dev[2], dev[5], is_causal=True, cur_pos_tensor=dev[6], scale=d**-0.5).cpu()
+    want = O.textbook_decode_fp32(q, dev[1].cpu(), dev[2].cpu(), table, cur, d**-0.5)
+    assert want.isinf().any() and want.isnan().any()
+    for t in (got, alone):
+        torch.testing.assert_close(t.float(), want.reshape(t.shape).float(), atol=2e-2, rtol=2e-2, equal_nan=True)

@@ -89,6 +89,12 @@ __device__ __forceinline__ floatx4 mma16(const u32x4 &x, const u32x4 &y, const f
                                                    __builtin_bit_cast(bf16x8, y), c, 0, 0, 0);
 }
 
+// A pair of non-negative bfloat16 values less `n` units of their last place each (0 stays 0, NaN stays NaN).
+__device__ __forceinline__ uint32_t less_units(uint32_t pair, uint32_t n) {
+  typedef uint16_t ushort2_t __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(__builtin_bit_cast(ushort2_t, pair), __builtin_bit_cast(ushort2_t, n)));
+}
+
 // The end of a segment that one workgroup of WAVES wavefronts has read (`active` of them had a tile): the
 // wavefronts' results meet in LDS, each in its own tile buffer, whose last tile it has consumed; then every
 // thread merges, normalises and stores four neighbouring elements of a head.  A wavefront's values lie as
@@ -436,6 +442,8 @@ __global__ __launch_bounds__(DIRECT ? kWave *DIRECT : 256, (DIRECT || BFP8) && D
   float m_run = -INFINITY, l_run = 0.f;
   int ev_run = 0;  // reference exponent of the V accumulator
 
+  const uint32_t below = G == 1 ? 0x00010001u : 0u;  // what the first of two parts of a pair of weights is less
+
   auto process_tile = [&](auto has_next_tag) {
     constexpr bool has_next = decltype(has_next_tag)::value;
     const int nvalid = cur.len - cur.t * TILE;
@@ -568,10 +576,10 @@ __global__ __launch_bounds__(DIRECT ? kWave *DIRECT : 256, (DIRECT || BFP8) && D
         for (int r = 0; r < 4; r += 2) {
           const float p0 = __builtin_amdgcn_exp2f(fmaf(st[b][r], scale, -m_safe));
           const float p1 = __builtin_amdgcn_exp2f(fmaf(st[b][r + 1], scale, -m_safe));
-          const uint32_t w = pack_bf16x2(p0, p1);
+          const uint32_t w = less_units(pack_bf16x2(p0, p1), below);
           lsum += bf16_lo(w) + bf16_hi(w);  // the normaliser sums the weights that multiply V
           pf[b >> 1][2 * (b & 1) + (r >> 1)] = w;
-          st[b][r] = p0 - bf16_lo(w), st[b][r + 1] = p1 - bf16_hi(w);  // what the rounding took
+          st[b][r] = p0 - bf16_lo(w), st[b][r + 1] = p1 - bf16_hi(w);  // the second parts, where there are two
         }
     }
     l_run = l_run * alpha + lsum;
@@ -594,10 +602,11 @@ __global__ __launch_bounds__(DIRECT ? kWave *DIRECT : 256, (DIRECT || BFP8) && D
         }
     };
     second_product();
-    // One query head per KV head: the weights in two bfloat16 parts.  The dot-product kernel, which serves such groups
-    // otherwise, keeps a running maximum per sixteen of a tile's tokens, so more of its weights are exact; rounded once, this
+    // One query head per KV head: the weights in two bfloat16 parts.  The dot-product kernel, which serves such groups where this
+    // one is not built, keeps a running maximum per sixteen of a tile's tokens, so more of its weights are exact; rounded once, this
     // kernel's results were 4 - 7 % further from a 64-bit evaluation than that one's (2.09e-3 against 1.97e-3, 128 tokens of 8 / 8
-    // heads), in two parts they are 15 - 17 % closer (1.66e-3).
+    // heads), in two parts they are 15 - 17 % closer (1.66e-3).  The first part is the rounded weight less one unit of its last
+    // place, so that the second is positive: with zero or less, an infinite V element would come out as NaN.
     if constexpr (!BFP8) {
       if (G == 1) {
         float low = 0.f;
