@@ -149,4 +149,35 @@ def test_block_float_8_with_room_for_the_copies_only(monkeypatch):
         blocks.zero_()
         monkeypatch.setattr(N, "call", with_room(size))
         got = _pass(*args, d**-0.5)
+        assert bool(blocks.any()) == (size == room)
         P._check(f"copies only, {size} of {room} bytes, parts {parts}", got.cpu(), want)
+
+
+@pytest.mark.parametrize("users,hq,hkv,lc,nbpu,copies", [
+    (1, 16, 16, 32, 3, True), (1, 16, 16, 128, 3, True), (8, 16, 16, 256, 12, True),  # few rows to copy; two row blocks
+    (4, 40, 8, 64, 6, False),                                                         # one row block, and many rows
+])
+def test_block_float_8_under_tables_too_narrow_to_be_split(monkeypatch, users, hq, hkv, lc, nbpu, copies):
+    """Where neither loop is split, a pass reads copies if they are few or read more than once: its scratch is theirs,
+    and holds them behind the pass."""
+    from tt_xla_amd import _native as N
+
+    d, bs = 128, 64
+    g = torch.Generator().manual_seed(users + lc)
+    key, value, table = P._paged(g, users, nbpu, hkv, bs, d, False)
+    q = P._bf(g, users, hq, lc, d)
+    st = torch.tensor([nbpu * bs - lc], dtype=torch.int32)
+    packed = [bfp8_codec.pack_cache(t) for t in (key, value)]
+    want = O.chunked_sdpa(q, *[bfp8_codec.unpack_cache(t, bs).to(torch.bfloat16) for t in packed], table, st, d**-0.5)
+    room = int(N.lib().ttpa_sdpa_prefill_workspace_bytes(users, hkv, d, bs, nbpu, 1))
+    assert int(N.lib().ttpa_sdpa_prefill_scratch_bytes(users, hq, hkv, lc, d, bs, nbpu, 1)) == (room if copies else 0)
+    blocks = torch.zeros(room, dtype=torch.uint8, device="cuda")
+    call = N.call
+
+    def with_room(name, *a):
+        return call(name, *(a[:-3] + (blocks.data_ptr(), room, a[-1]) if name == "ttpa_sdpa_prefill_expanded" else a))
+
+    monkeypatch.setattr(N, "call", with_room)
+    got = _pass(*[t.cuda() for t in (q, packed[0], packed[1], table, st)], d**-0.5)
+    assert bool(blocks.any()) == copies
+    P._check(f"narrow u{users} h{hq}x{hkv} len{lc} width{nbpu}", got.cpu(), want)

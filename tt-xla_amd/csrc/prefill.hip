@@ -633,16 +633,6 @@ __global__ __launch_bounds__(256, prefill_wgs_per_cu<RH>(D, MODE)) void prefill_
   }
 }
 
-// Whether the plain loop may split the keys of this launch: paged, each row sees all keys up to its own.
-inline bool plain_splits(const PrefillArgs &a) { return a.pt != nullptr && a.window == 0 && a.mask == nullptr; }
-
-// Bytes of scratch with which it does (0: it would not).
-inline int64_t plain_part_bytes(const PrefillArgs &a, int d, bool bfp8) {
-  if (!plain_splits(a)) return 0;
-  const int g = a.hq / a.hkv;
-  return part_bytes(a, g % 4 == 0 ? 4 : g % 2 == 0 ? 2 : 1, plain_split(d, bfp8), d);
-}
-
 template <int D, int HPW, int MODE, int RH>
 int launch_mode(const PrefillArgs &a, hipStream_t st) {
   constexpr int RPW = 4 / HPW;
@@ -817,9 +807,7 @@ static int prefill_impl(void *out, int64_t out_batch_stride, int64_t out_head_st
     TTPA_REQUIRE(workspace_bytes >= 0 && (workspace != nullptr || workspace_bytes == 0),
                  "prefill: workspace_bytes %lld with a null workspace", (long long)workspace_bytes);
     const int64_t need = expand_bytes(batch, table_width, kv_heads, block_size, head_size);
-    // (a pass that would be split where it stands, but has no room for its parts, reads copies too)
-    const bool copies = stream_expands(a, head_size) || (stream_serves(a, head_size) && workspace_bytes < plain_part_bytes(a, head_size, true));
-    if (copies && workspace && aligned16(workspace) && (int64_t)batch * table_width < (1ll << 31) && workspace_bytes >= need) {
+    if (stream_expands(a, head_size, workspace_bytes) && workspace && aligned16(workspace) && (int64_t)batch * table_width < (1ll << 31) && workspace_bytes >= need) {
       a.expand = workspace;  // (a smaller one is not an error: the pass expands tile by tile instead)
       workspace = static_cast<unsigned char *>(workspace) + need;
       workspace_bytes -= need;
@@ -894,7 +882,7 @@ extern "C" int64_t ttpa_sdpa_prefill_scratch_bytes(int32_t batch, int32_t q_head
   a.pt = &some_table, a.stream = 1;
   a.batch = batch, a.hq = q_heads, a.hkv = kv_heads, a.sq = q_len, a.bs = block_size, a.w = table_width;
   if (kv_format == TTPA_KV_BFP8) {
-    if (!stream_expands(a, head_size)) return plain_part_bytes(a, head_size, true);
+    if (!stream_expands(a, head_size, INT64_MAX)) return plain_part_bytes(a, head_size, true);
     return ttpa_sdpa_prefill_workspace_bytes(batch, kv_heads, head_size, block_size, table_width, kv_format) + stream_part_bytes(a, head_size);
   }
   return stream_serves(a, head_size) ? stream_part_bytes(a, head_size) : plain_part_bytes(a, head_size, false);

@@ -158,5 +158,18 @@ inline int64_t part_bytes(PrefillArgs a, int heads_per_wg, const SplitRule &rule
   return part_layout(a, kRowsPerWave * 4 / heads_per_wg).slots * (part_acc_floats(d) + 2 * kRowsPerWave) * (int64_t)sizeof(float);
 }
 
+inline int heads_per_workgroup(const PrefillArgs &a) {
+  const int g = a.hq / a.hkv;
+  return g % 4 == 0 ? 4 : g % 2 == 0 ? 2 : 1;
+}
+
+// Whether the plain loop may split the keys of this launch: paged, each row sees all keys up to its own.
+inline bool plain_splits(const PrefillArgs &a) { return a.pt != nullptr && a.window == 0 && a.mask == nullptr; }
+
+// Bytes of scratch with which it does (0: it would not).
+inline int64_t plain_part_bytes(const PrefillArgs &a, int d, bool bfp8) {
+  return plain_splits(a) ? part_bytes(a, heads_per_workgroup(a), plain_split(d, bfp8), d) : 0;
+}
+
 }  // namespace
 }  // namespace ttpa

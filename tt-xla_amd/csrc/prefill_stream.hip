@@ -397,11 +397,6 @@ __global__ __launch_bounds__(256, 2) void prefill_stream_kernel(PrefillArgs a) {
   }
 }
 
-int heads_per_workgroup(const PrefillArgs &a) {
-  const int g = a.hq / a.hkv;
-  return g % 4 == 0 ? 4 : g % 2 == 0 ? 2 : 1;
-}
-
 template <int HPW, int FORM>
 int launch_form(const PrefillArgs &a, hipStream_t st) {
   constexpr int RPW = 4 / HPW;
@@ -468,15 +463,21 @@ int64_t stream_part_bytes(const PrefillArgs &a, int head_size) {
   return a.pt && stream_serves(a, head_size) ? part_bytes(a, heads_per_workgroup(a), kStreamSplit, kD) : 0;
 }
 
-// Where a block is read by at most two workgroups (row blocks times head groups of a KV head), mode 4 expands it as it reads it:
-// split over the keys that costs less than the copies, a launch and a trip through memory in front of the attention.  Passes in
-// us, copies / mode 4: 1 x 32 rows behind 512 tokens, 64 / 8 heads 23.1 / 18.8; 4 x 32 rows of 32 / 8 behind 1024 32.1 / 25.3, 4096 49.3 /
-// 38.7; 8 x 128 of 16 / 16 behind 4096 167 / 75.6; two row blocks: 4 x 64 of 32 / 8 behind 512 29.5 / 24.9, 8 x 256 of 16 / 16 behind 512
-// 46.1 / 48.2, behind 4096 195 / 128.  Four workgroups: 2 x 64 of 64 / 8 behind 4096 49.5 / 55.6; three: 2 x 96 of 32 / 8 46.7 / 50.0.
-bool stream_expands(const PrefillArgs &a, int head_size) {
+// A pass that reads a block once expands it no more often in mode 4, on its way into LDS, than into copies, a trip through memory in
+// front of the attention; the copies pay where there are several row blocks, where they are few, or where they let the keys be split
+// (16 / 16 heads, copies / mode 4: 1 x 128 rows behind 64 tokens 16.4 / 19.0 us, 8 x 256 behind 512 47.8 / 49.1; 40 / 8 heads, 4 x 64
+// behind 256 25.1 / 20.8).
+// Not where mode 4 itself is split and a block is read by at most two workgroups (row blocks times head groups of a KV head).
+// Passes in us, copies / mode 4: 1 x 32 rows behind 512 tokens, 64 / 8 heads 23.1 / 18.8; 4 x 32 rows of 32 / 8 behind 1024 32.1 / 25.3, 4096 49.3 /
+// 38.7; 8 x 128 of 16 / 16 behind 4096 167 / 75.6; two row blocks: 4 x 64 of 32 / 8 behind 512 29.5 / 24.9, 8 x 256 of 16 / 16 behind
+// 4096 195 / 128.  Four workgroups: 2 x 64 of 64 / 8 behind 4096 49.5 / 55.6; three: 2 x 96 of 32 / 8 46.7 / 50.0.
+bool stream_expands(const PrefillArgs &a, int head_size, int64_t room) {
   if (!stream_serves(a, head_size)) return false;
   const int hpw = heads_per_workgroup(a), rows = kRowsPerWave * 4 / hpw;
-  return (int64_t)((a.sq + rows - 1) / rows) * (a.hq / hpw / a.hkv) > 2;
+  const int64_t row_blocks = (a.sq + rows - 1) / rows;
+  const bool pays = row_blocks > 1 || (int64_t)a.batch * a.w * a.bs * a.hkv <= 8192 || part_bytes(a, hpw, kStreamSplit, kD) > 0;
+  const int64_t parts = plain_part_bytes(a, kD, true);
+  return pays && !(parts > 0 && parts <= room && row_blocks * (a.hq / hpw / a.hkv) <= 2);
 }
 
 int launch_stream_wide(const PrefillArgs &a, hipStream_t st) {
