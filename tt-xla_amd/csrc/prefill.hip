@@ -120,10 +120,14 @@ __global__ __launch_bounds__(256) void bfp8_expand_kernel(ExpandArgs e) {
 // RH: blocks of 32 query rows per wavefront; only 1 is built (a form with two, one workgroup per
 // CU and every K / V fragment feeding two matrix instructions, measured slower: with one wavefront
 // per SIMD nobody fills the waits for fragments and barriers).
+//
+// SPLIT: the keys of a row block are shared by a.parts > 1 workgroups (prefill_parts.h).  A kernel of its own: with the parts' way
+// out as a run-time branch an unsplit launch was 0.1 ... 0.7 us longer than without (1 x 512 rows of 64 / 8 heads of 64 behind 512
+// tokens 28.3 / 27.7 us, 8 x 256 of 16 / 8 of 256 behind 512 55.3 / 54.3), and a split one 0.3 us (1 x 32 of 16 / 8 of 256 22.5 / 22.2).
 template <int RH>
 constexpr int prefill_wgs_per_cu(int d, int mode) { return RH == 1 && d <= 128 ? 2 : 1; }
 
-template <int D, int HPW, int MODE, int RH>
+template <int D, int HPW, int MODE, int RH, bool SPLIT>
 __global__ __launch_bounds__(256, prefill_wgs_per_cu<RH>(D, MODE)) void prefill_kernel(PrefillArgs a) {
   constexpr int RPW = 4 / HPW;            // wavefront row slots per workgroup
   constexpr int ROWS = kRowsPerWave * RH;  // query rows per wavefront
@@ -138,7 +142,7 @@ __global__ __launch_bounds__(256, prefill_wgs_per_cu<RH>(D, MODE)) void prefill_
     if (wg < 0) return;
   }
   // (the slower index, so that part 0, alone with work where the keys are few, is on every XCD)
-  const int part = MODE != 0 ? blockIdx.y : 0;
+  const int part = SPLIT ? blockIdx.y : 0;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -175,14 +179,12 @@ __global__ __launch_bounds__(256, prefill_wgs_per_cu<RH>(D, MODE)) void prefill_
   const int wave_first_key = a.window > 0 ? max(0, offset + row0 - a.window + 1) : 0;
   int first_tile = wg_first_key / kKeysPerTile;
   bool whole = true;  // this workgroup sees all keys of its rows
-  if constexpr (MODE != 0) {
-    if (a.parts > 1) {  // (no window, no mask)
-      const int share = __builtin_amdgcn_readfirstlane((blocks_per_part(a, offset) + 1) / 2);
-      whole = share >= ntiles;
-      first_tile = part * share;
-      ntiles = min(ntiles, first_tile + share);
-      if (first_tile >= ntiles) return;
-    }
+  if constexpr (SPLIT) {  // (no window, no mask)
+    const int share = __builtin_amdgcn_readfirstlane((blocks_per_part(a, offset) + 1) / 2);
+    whole = share >= ntiles;
+    first_tile = part * share;
+    ntiles = min(ntiles, first_tile + share);
+    if (first_tile >= ntiles) return;
   }
 
   // ---- Q fragments (B operand: lane n = query row, 8 head-dim elements per k-step) -----
@@ -592,7 +594,7 @@ __global__ __launch_bounds__(256, prefill_wgs_per_cu<RH>(D, MODE)) void prefill_
   }
 
   // ---- normalise and store: lane (n, h) holds head-dim elements 32 db + 8 j + 4 h + i ----
-  if constexpr (MODE != 0) {
+  if constexpr (SPLIT) {
     if (!whole) {
       // a part's accumulators and (maximum, sum) per row: lane l's four elements of group 4 db + j at float 256 (4 db + j) + 4 l
       // of the row block's, 1 KiB per store of the wavefront.  A row that sees none of the part's keys has maximum -inf, sum 0.
@@ -633,29 +635,36 @@ __global__ __launch_bounds__(256, prefill_wgs_per_cu<RH>(D, MODE)) void prefill_
   }
 }
 
+template <int D, int HPW, int MODE, int RH, bool SPLIT>
+int launch_split(PrefillArgs &b, int grid, hipStream_t st) {
+  const size_t lds = 2 * Tile<D>::STAGE_BYTES;  // two stages of a K and a V tile
+  static std::atomic<uint64_t> lds_ready{0};
+  if (!ensure_dynamic_lds(reinterpret_cast<const void *>(&prefill_kernel<D, HPW, MODE, RH, SPLIT>), lds, lds_ready))
+    return fail(TTPA_ERR_LAUNCH, "prefill: cannot reserve %zu bytes of LDS", lds);
+  launch_dominant(&prefill_kernel<D, HPW, MODE, RH, SPLIT>, dim3(grid, b.parts), dim3(256), lds, st, b);
+  return check_launch("sdpa_prefill");
+}
+
 template <int D, int HPW, int MODE, int RH>
 int launch_mode(const PrefillArgs &a, hipStream_t st) {
   constexpr int RPW = 4 / HPW;
   constexpr int ROWS = kRowsPerWave * RH;
   const int nqt = (a.sq + ROWS * RPW - 1) / (ROWS * RPW);
-  const size_t lds = 2 * Tile<D>::STAGE_BYTES;  // two stages of a K and a V tile
-  static std::atomic<uint64_t> lds_ready{0};
-  if (!ensure_dynamic_lds(reinterpret_cast<const void *>(&prefill_kernel<D, HPW, MODE, RH>), lds, lds_ready))
-    return fail(TTPA_ERR_LAUNCH, "prefill: cannot reserve %zu bytes of LDS", lds);
   const int ny8 = (a.batch * (a.hq / HPW) + 7) / 8;
   PrefillArgs b = a;
   int grid = nqt * ny8 * 8;
   b.parts = 1;
-  constexpr SplitRule kRule = plain_split(D, MODE == 4);
-  if (MODE != 0 && plain_splits(a) && a.part_acc && a.part_bytes >= part_bytes(a, HPW, kRule, D)) set_parts(b, HPW, kRule);
-  if (MODE == 0 && a.fill_kc) grid = grid_with_fill(b, grid, D);
-  launch_dominant(&prefill_kernel<D, HPW, MODE, RH>, dim3(grid, b.parts), dim3(256), lds, st, b);
-  if (const int rc = check_launch("sdpa_prefill")) return rc;
-  if (MODE != 0 && b.parts > 1) {
-    prefill_merge_kernel<D, RPW><<<dim3((b.sq + kRowsPerWave - 1) / kRowsPerWave, b.hq, b.batch), dim3(2 * D), 0, st>>>(b);
-    return check_launch("sdpa_prefill (merge of the parts)");
+  if constexpr (MODE != 0) {
+    constexpr SplitRule kRule = plain_split(D, MODE == 4);
+    if (plain_splits(a) && a.part_acc && a.part_bytes >= part_bytes(a, HPW, kRule, D)) set_parts(b, HPW, kRule);
+    if (b.parts > 1) {
+      if (const int rc = launch_split<D, HPW, MODE, RH, true>(b, grid, st)) return rc;
+      prefill_merge_kernel<D, RPW><<<dim3((b.sq + kRowsPerWave - 1) / kRowsPerWave, b.hq, b.batch), dim3(2 * D), 0, st>>>(b);
+      return check_launch("sdpa_prefill (merge of the parts)");
+    }
   }
-  return TTPA_OK;
+  if (MODE == 0 && a.fill_kc) grid = grid_with_fill(b, grid, D);
+  return launch_split<D, HPW, MODE, RH, false>(b, grid, st);
 }
 
 template <int D, int HPW, int RH>
