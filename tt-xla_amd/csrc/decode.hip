@@ -542,7 +542,12 @@ static int decode_impl(void *out, int64_t out_user_stride, int64_t out_head_stri
   // can be attended, the partials of twice the ranges cost more than the chains that they hide (us per layer at one / two: 2
   // users of 64/8 heads with 3327 ... 6987 tokens 16.4 / 17.5, one of 32/8 heads over 16384 19.2 / 20.0, 27 with 512 ... 4096 32.5 / 30.5).
   const int64_t seen = sliding_window > 0 ? std::min<int64_t>((int64_t)table_width * block_size, sliding_window) : (int64_t)table_width * block_size;
-  const bool two_per_cu = use_mfma16 && kv_format == TTPA_KV_BFP8 && head_size <= 128 &&
+  // Groups whose partials are 1024 values or more at head size 128 (eight heads) keep tiles of 64 tokens and one workgroup per CU: there
+  // the short tiles' one costs more per byte, and two workgroups' partials more than they save (us per layer, short tiles one / two per
+  // CU, long: 40 users of 64/4 heads with 336 ... 1600 tokens 22.9 / 29.3 / 23.8, 1008 ... 4800 35.7 / 39.7 / 33.6, 3360 ... 16000 79.0 /
+  // 78.9 / 71.4; of 64/8, 105 ... 500 tokens 17.1 / 19.0 / 18.2, 1680 ... 8000 76.7 / 72.3 / 69.7; 40/8, 504 ... 2400 31.8 / 30.3 / 31.1).
+  a.long_tiles = use_mfma16 && kv_format == TTPA_KV_BFP8 && head_size == 128 && g * head_size >= 1024 && !mask && !a.direct;
+  const bool two_per_cu = use_mfma16 && kv_format == TTPA_KV_BFP8 && head_size <= 128 && !a.long_tiles &&
                           (int64_t)users * kv_heads * (seen * head_size / 4096) >= 6 * (int64_t)waves_for_device(8.0);
   a.n_waves = waves_for_device(use_mfma16 && kv_format == TTPA_KV_BF16 ? 3.0
                                : two_per_cu                             ? 8.0

@@ -46,6 +46,7 @@ struct DecodeArgs {
   // k_new / v_new [users][>= hkv heads][head_size] instead of the cache, and written to it.
   const uint16_t *k_new = nullptr, *v_new = nullptr;
   int64_t new_us, new_hs;
+  int long_tiles = 0;  // 16x16x32 kernel, block-float-8 at head size 128: tiles of 64 tokens instead of 32
   int direct = 0;  // wavefronts of the workgroup that owns a whole segment (16x16x32 kernel, fused step), or 0
   // Additive mask on the scaled scores (bfloat16, natural-log units), or null: the element for
   // (user, query head, position) is mask[user * mask_us + head * mask_hs + position].  Applied by the

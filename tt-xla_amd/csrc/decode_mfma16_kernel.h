@@ -3,7 +3,7 @@
 // to half precision) or a bfloat16 cache.
 //
 // Work decomposition, partial slots and merge kernel are those of decode.hip, with tiles of
-// 64, 32 or 32 tokens at head size 64, 128, 256 (tile_bytes).  Inside a wavefront a tile of K,
+// 64, 32 or 32 tokens at head size 64, 128, 256, or 64 at 128 (tile_bytes).  Inside a wavefront a tile of K,
 // then of V, goes global -> registers -> a wave-private LDS buffer of that size that both
 // tensors use in turn:
 //   stage K(t) | prefetch K(t+1) | S^T = K Q^T | softmax | stage V(t) | prefetch V(t+1) | O^T += V^T P^T
@@ -70,13 +70,14 @@ constexpr int kMaxUsers16 = kMaxUsers;  // the library-wide limit: 16 KiB of pre
 // At head size 64 (64 / 8 heads, us per layer of a replayed step): a window of 1024 over 37 users 25.2 ->
 // 23.1 (its two ends waste less, too), 32 users with 512 ... 4096 tokens 27.7 -> 26.5, 8 users with
 // 128 ... 1024 15.0 -> 11.6, 128 users with 256 ... 32768 274 -> 272; 4 KiB: 23.6, 26.9, 10.8.
-// A block-float-8 tile is half the bytes behind the same chain of steps, so that kernel is bound by the chain.  With 16 KiB it
+// A block-float-8 tile is half the bytes behind the same chain of steps, so that kernel is bound by the chain.  With 16 KiB (LONG) it
 // needed 316 registers, one wavefront per SIMD; with 8 KiB two share a SIMD and a launch has twice the wavefronts (us per layer,
 // 64 users with 1024 ... 16384 tokens, 32/8 heads at head size 128: 144 -> 137; 100 users with 1024 ... 8192, 64/8 heads at 64: 92 ->
-// 78; 40 users of 16/16 heads with 512 ... 4096: 68 -> 61).  Head size 256 has 32-token tiles either way.
-template <int D>
+// 78; 40 users of 16/16 heads with 512 ... 4096: 68 -> 61).  Wide groups keep 16 KiB (DecodeArgs::long_tiles).  Head size 256 has
+// 32-token tiles either way.
+template <int D, bool LONG = false>
 constexpr int tile_bytes() {
-  return D <= 128 ? 8192 : 16384;
+  return D <= 128 && !LONG ? 8192 : 16384;
 }
 
 template <bool F16>
@@ -156,12 +157,12 @@ __device__ __forceinline__ void merge_waves(const DecodeArgs &a, int u, int h, i
 // RUNS: 1, 2, 4, or 0 for one run per load.  MASKED: an additive mask row per (user, head) joins the
 // scores (a.mask; the form of a pass that is not causal, built with RUNS = 0 and without the update).
 // DIRECT: a workgroup of DIRECT wavefronts owns the whole segment blockIdx.x (chosen by direct_waves, decode.hip): no prefix, no
-// search, no partials, no merge launch.  Its wavefronts take the segment's tiles in turn.
-template <int D, bool BFP8, int RUNS, bool FUSED, bool MASKED = false, int DIRECT = 0>
-__global__ __launch_bounds__(DIRECT ? kWave *DIRECT : 256, (DIRECT || BFP8) && D <= 128 ? 2 : 1) void paged_decode_mfma16_kernel(
+// search, no partials, no merge launch.  Its wavefronts take the segment's tiles in turn.  LONG: tiles of 16 KiB (a.long_tiles).
+template <int D, bool BFP8, int RUNS, bool FUSED, bool MASKED = false, int DIRECT = 0, bool LONG = false>
+__global__ __launch_bounds__(DIRECT ? kWave *DIRECT : 256, (DIRECT || BFP8) && D <= 128 && !LONG ? 2 : 1) void paged_decode_mfma16_kernel(
     DecodeArgs a, const int32_t *__restrict__ page_table, const void *__restrict__ cur_pos) {
   static_assert(D == 64 || D == 128 || D == 256, "shapes built");
-  constexpr int kTileBytes = tile_bytes<D>();
+  constexpr int kTileBytes = tile_bytes<D, LONG>();
   constexpr int TILE = kTileBytes / (2 * D);  // tokens per tile
   constexpr int ROWB = 2 * D;                 // bytes of a tile row in LDS
   constexpr int KSTEPS = D / 32, DBLK = D / 16;
@@ -669,13 +670,13 @@ __global__ __launch_bounds__(DIRECT ? kWave *DIRECT : 256, (DIRECT || BFP8) && D
   process_tile(std::false_type{});
 }
 
-template <int D, bool BFP8, int RUNS, bool FUSED, bool MASKED = false, int DIRECT = 0>
+template <int D, bool BFP8, int RUNS, bool FUSED, bool MASKED = false, int DIRECT = 0, bool LONG = false>
 bool launch(const DecodeArgs &a, hipStream_t st) {
   constexpr int kWaves = DIRECT ? DIRECT : kWavesPerBlock;
   const int blocks = DIRECT ? a.users * a.hkv : a.n_waves / kWavesPerBlock;
-  const size_t lds = (size_t)kWaves * tile_bytes<D>();
+  const size_t lds = (size_t)kWaves * tile_bytes<D, LONG>();
   static std::atomic<uint64_t> lds_ready{0};
-  const auto kernel = &paged_decode_mfma16_kernel<D, BFP8, RUNS, FUSED, MASKED, DIRECT>;
+  const auto kernel = &paged_decode_mfma16_kernel<D, BFP8, RUNS, FUSED, MASKED, DIRECT, LONG>;
   if (!ensure_dynamic_lds(reinterpret_cast<const void *>(kernel), lds, lds_ready)) return false;
   launch_dominant(kernel, dim3(blocks), dim3(kWave * kWaves), lds, st, a, a.pt, a.cur);
   return true;
@@ -688,21 +689,29 @@ bool launch_direct(const DecodeArgs &a, hipStream_t st) {
   return a.bs % TILE == 0 ? launch<D, BFP8, 1, FUSED, false, DIRECT>(a, st) : launch<D, BFP8, 2, FUSED, false, DIRECT>(a, st);
 }
 
+// Equal ranges of the flat list.
+template <int D, bool BFP8, bool FUSED, bool LONG>
+bool launch_ranges(const DecodeArgs &a, hipStream_t st) {
+  constexpr int TILE = tile_bytes<D, LONG>() / (2 * D);
+  if (a.bs % TILE == 0) return launch<D, BFP8, 1, FUSED, false, 0, LONG>(a, st);
+  if (a.bs % (TILE / 2) == 0) return launch<D, BFP8, 2, FUSED, false, 0, LONG>(a, st);
+  if (LONG || a.bs % (TILE / 4) == 0) return launch<D, BFP8, 4, FUSED, false, 0, LONG>(a, st);  // (block-float-8: blocks of 16 tokens)
+  if constexpr (!LONG) return launch<D, BFP8, 0, FUSED, false, 0, LONG>(a, st);
+}
+
 // Picks the variant for the block size and for a.k_new (set: the launch also performs the
 // cache update of the step).
 template <int D, bool BFP8>
 bool launch_for_block_size(const DecodeArgs &a, hipStream_t st) {
-  constexpr int TILE = tile_bytes<D>() / (2 * D);
   const bool fused = a.k_new != nullptr;
   if constexpr (D <= 128) {
     if (a.direct == 4) return fused ? launch_direct<D, BFP8, true, 4>(a, st) : launch_direct<D, BFP8, false, 4>(a, st);
     if (a.direct == 8) return fused ? launch_direct<D, BFP8, true, 8>(a, st) : launch_direct<D, BFP8, false, 8>(a, st);
   }
   if (a.mask != nullptr) return !fused && launch<D, BFP8, 0, false, true>(a, st);
-  if (a.bs % TILE == 0) return fused ? launch<D, BFP8, 1, true>(a, st) : launch<D, BFP8, 1, false>(a, st);
-  if (a.bs % (TILE / 2) == 0) return fused ? launch<D, BFP8, 2, true>(a, st) : launch<D, BFP8, 2, false>(a, st);
-  if (a.bs % (TILE / 4) == 0) return fused ? launch<D, BFP8, 4, true>(a, st) : launch<D, BFP8, 4, false>(a, st);
-  return fused ? launch<D, BFP8, 0, true>(a, st) : launch<D, BFP8, 0, false>(a, st);
+  if constexpr (D == 128 && BFP8)
+    if (a.long_tiles) return fused ? launch_ranges<D, BFP8, true, true>(a, st) : launch_ranges<D, BFP8, false, true>(a, st);
+  return fused ? launch_ranges<D, BFP8, true, false>(a, st) : launch_ranges<D, BFP8, false, false>(a, st);
 }
 
 }  // namespace
