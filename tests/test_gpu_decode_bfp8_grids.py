@@ -1,5 +1,5 @@
 """GPU tests of how the 16x16 matrix kernel cuts a block-float-8 decode (csrc/decode.hip): long tiles and one workgroup per CU for
-wide groups.  A grid is told by its bits: the same list cut into the same ranges gives the same output, and into others
+wide groups, for the others one or two by the length of the list.  A grid is told by its bits: the same list cut into the same ranges gives the same output, and into others
 another one (partials are rounded against other maxima)."""
 
 import pytest
@@ -35,10 +35,10 @@ def _attend(q, k, v, table, cur, window=0, sink=None):
 
 
 @pytest.mark.parametrize("hq,hkv,bs,pos,window,with_sink", [
-    (64, 8, 64, [0, 63, 64, 65, 127, 128, -1, 1000], 0, False),  # borders of 64-token tiles, one block each
+    (72, 8, 64, [0, 63, 64, 65, 127, 128, -1, 1000], 0, False),  # borders of 64-token tiles, one block each
     (64, 4, 32, [0, 31, 32, 95, 96, 2047], 0, True),            # sixteen heads, tiles of two blocks
     (60, 4, 16, [15, 16, 63, 64, 500], 0, False),               # fifteen heads, tiles of four blocks
-    (64, 8, 128, [127, 128, 900, 1500], 200, True),             # a window: tiles cut at both ends
+    (128, 8, 128, [127, 128, 900, 1500], 200, True),            # a window: tiles cut at both ends
 ])
 def test_long_tiles_of_wide_groups(monkeypatch, hq, hkv, bs, pos, window, with_sink):
     monkeypatch.setenv("TTPA_DECODE_KERNEL", "ranges")
@@ -56,13 +56,36 @@ def test_long_tiles_of_wide_groups(monkeypatch, hq, hkv, bs, pos, window, with_s
         torch.testing.assert_close(got[:, live].float(), want.reshape(got[:, live].shape).float(), atol=2e-2, rtol=2e-2)
 
 
-@pytest.mark.parametrize("hq,hkv", [(64, 8), (64, 4)])
-def test_wide_groups_have_one_workgroup_per_cu(monkeypatch, hq, hkv):
-    users, width = 40, 128
-    args = _inputs(users, hq, hkv, 128, 64, [8000 - 77 * u for u in range(users)], width)
+@pytest.mark.parametrize("users,hq,hkv", [(40, 64, 4), (10, 64, 8)])
+def test_wide_groups_have_one_workgroup_per_cu(monkeypatch, users, hq, hkv):
+    args = _inputs(users, hq, hkv, 128, 64, [8000 - 77 * u for u in range(users)], 128)
     got = _attend(*args)
     outs = {}
     for waves in ("4", "8"):
         monkeypatch.setenv("TTPA_DECODE_WAVES_PER_CU", waves)
         outs[waves] = _attend(*args)
     assert torch.equal(got, outs["4"]) and not torch.equal(got, outs["8"])
+
+
+@pytest.mark.parametrize("users,hq,hkv,d,n_short,n_long", [
+    (16, 32, 8, 128, 31, 32),  # 512 values per partial: from 4096 tiles of 32 tokens on
+    (16, 40, 8, 128, 39, 40),  # 640: from 5120
+    (4, 64, 8, 64, 127, 128),  # tiles of 64 tokens
+    (8, 8, 8, 128, 43, 44),    # 128: from 2816
+    (65, 8, 8, 128, 4, 5),     # above 64 users the list counts the leading units as well: 5 and 6 per segment, 2816 / 520 = 5.4
+])
+def test_short_lists_have_one_workgroup_per_cu(monkeypatch, users, hq, hkv, d, n_short, n_long):
+    """Under one page table, by the tiles that there are: the border is where the grids change."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    if cus != 256:
+        pytest.skip("the cases are laid out for 256 CUs")
+    tile, width = 4096 // d, 512
+    for n, waves, other in ((n_short, "4", "8"), (n_long, "8", "4")):
+        q, k, v, table, cur = _inputs(users, hq, hkv, d, 64, [n * tile - 1] * users, width)
+        monkeypatch.delenv("TTPA_DECODE_WAVES_PER_CU", raising=False)
+        got = _attend(q, k, v, table, cur)
+        outs = {}
+        for w in (waves, other):
+            monkeypatch.setenv("TTPA_DECODE_WAVES_PER_CU", w)
+            outs[w] = _attend(q, k, v, table, cur)
+        assert torch.equal(got, outs[waves]) and not torch.equal(got, outs[other])

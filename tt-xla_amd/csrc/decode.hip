@@ -538,17 +538,25 @@ static int decode_impl(void *out, int64_t out_user_stride, int64_t out_head_stri
   // the 32-user workload, 531 against 544 us on the 128-user one: the streams of 192 workgroups
   // already hold the memory system's latency in bytes, and every further wavefront is one more
   // partial and one more share in the contention).  On a block-float-8 cache it wants two workgroups
-  // per CU up to head size 128 (tile_bytes), if they have something to do: where no more than six tiles per range
-  // can be attended, the partials of twice the ranges cost more than the chains that they hide (us per layer at one / two: 2
-  // users of 64/8 heads with 3327 ... 6987 tokens 16.4 / 17.5, one of 32/8 heads over 16384 19.2 / 20.0, 27 with 512 ... 4096 32.5 / 30.5).
+  // per CU up to head size 128 (tile_bytes), if they have something to do: in a short list the partials of twice the ranges cost more
+  // than the chains that they hide.  How long it is the kernel knows, and then leaves half of the ranges empty (few_ranges); the host
+  // launches the larger grid where the page tables or the window allow a list of that length.  us per layer at one / two, by the values of a
+  // partial: 64 (8/8 heads of 64, 16 ... 18 users) 2500 tiles 14.7 / 15.3, 3000 16.3 / 15.7, 4000 17.6 / 16.3; 512 (32/8 of 128, 16 and 40 users)
+  // 2500 tiles 15.5 / 16.5 and 15.2 / 16.7, 4000 18.3 / 18.0 and 18.5 / 18.8, 6000 21.6 / 20.3 and 21.6 / 21.4; 640 (40/8) 4000 19.3 / 19.3, 6000
+  // 22.3 / 21.9; 1024 (64/4 of 64, 16 users) 6000 22.2 / 23.1, 12000 31.6 / 30.7.
   const int64_t seen = sliding_window > 0 ? std::min<int64_t>((int64_t)table_width * block_size, sliding_window) : (int64_t)table_width * block_size;
-  // Groups whose partials are 1024 values or more at head size 128 (eight heads) keep tiles of 64 tokens and one workgroup per CU: there
-  // the short tiles' one costs more per byte, and two workgroups' partials more than they save (us per layer, short tiles one / two per
-  // CU, long: 40 users of 64/4 heads with 336 ... 1600 tokens 22.9 / 29.3 / 23.8, 1008 ... 4800 35.7 / 39.7 / 33.6, 3360 ... 16000 79.0 /
-  // 78.9 / 71.4; of 64/8, 105 ... 500 tokens 17.1 / 19.0 / 18.2, 1680 ... 8000 76.7 / 72.3 / 69.7; 40/8, 504 ... 2400 31.8 / 30.3 / 31.1).
-  a.long_tiles = use_mfma16 && kv_format == TTPA_KV_BFP8 && head_size == 128 && g * head_size >= 1024 && !mask && !a.direct;
-  const bool two_per_cu = use_mfma16 && kv_format == TTPA_KV_BFP8 && head_size <= 128 && !a.long_tiles &&
-                          (int64_t)users * kv_heads * (seen * head_size / 4096) >= 6 * (int64_t)waves_for_device(8.0);
+  const int segments = users * kv_heads, larger_grid = waves_for_device(8.0);
+  const int64_t most_tiles = (int64_t)segments * (seen * head_size / 4096);
+  // Groups of more than eight heads at head size 128 keep tiles of 64 tokens and one workgroup per CU: there the short tiles' one costs
+  // more per byte, and two workgroups' partials more than they save (us per layer, short tiles one / two per CU, long: 40 users of 64/4
+  // heads with 336 ... 1600 tokens 22.9 / 29.3 / 23.8, 1008 ... 4800 35.7 / 39.7 / 33.6, 3360 ... 16000 79.0 / 78.9 / 71.4).  With eight heads it is the
+  // better form of long lists of few segments (short tiles, long, 64/8 heads: 10 users, 9000 tiles 28.9 / 27.1, 20000 44.1 / 41.6, 3000 17.8 /
+  // 18.4, 6000 22.8 / 23.5; 16 users, 6000 tiles 22.5 / 24.9, 12000 31.9 / 32.6, 20000 43.1 / 43.2).
+  a.long_tiles = use_mfma16 && kv_format == TTPA_KV_BFP8 && head_size == 128 && !mask && !a.direct &&
+                 (g > 8 || (g == 8 && segments < 128 && most_tiles >= 8 * (int64_t)larger_grid));
+  a.many_from = (int64_t)larger_grid * std::max(352, g * head_size) / 256;
+  const bool two_per_cu = use_mfma16 && kv_format == TTPA_KV_BFP8 && head_size <= 128 && !a.long_tiles && most_tiles >= a.many_from;
+  if (two_per_cu) a.few_ranges = waves_for_device(4.0);
   a.n_waves = waves_for_device(use_mfma16 && kv_format == TTPA_KV_BF16 ? 3.0
                                : two_per_cu                             ? 8.0
                                : (use_mfma || use_mfma16)               ? 4.0

@@ -46,6 +46,8 @@ struct DecodeArgs {
   // k_new / v_new [users][>= hkv heads][head_size] instead of the cache, and written to it.
   const uint16_t *k_new = nullptr, *v_new = nullptr;
   int64_t new_us, new_hs;
+  int few_ranges = 0;  // > 0: lists of fewer than `many_from` tiles are cut into that many ranges instead of n_waves
+  int64_t many_from = 0;
   int long_tiles = 0;  // 16x16x32 kernel, block-float-8 at head size 128: tiles of 64 tokens instead of 32
   int direct = 0;  // wavefronts of the workgroup that owns a whole segment (16x16x32 kernel, fused step), or 0
   // Additive mask on the scaled scores (bfloat16, natural-log units), or null: the element for
@@ -151,18 +153,25 @@ __device__ inline void build_prefix(const DecodeArgs &a, const void *__restrict_
 // 146 ... 1229 50.1 / 36.7, 16 of 200 ... 3000 57.3 / 50.3, 7 of 1384 ... 7377 54.1 / 49.7; 32 heads, 6 of 500 ... 5000
 // 41.4 / 30.1; 16 heads, one user over 1000 27.9 / 21.3, 8 of 300 ... 3000 28.7 / 27.2.  With none throughout: 30 users of
 // 500 ... 4000, 128 heads 75.6 instead of 64.4 with three; one user over 16000, 16 heads 38.4 instead of 32.3.
-template <int TILE = kTile>
+// FEW: n_ranges, a.n_waves on entry, becomes a.few_ranges for a short list (above 64 users by its units).
+template <int TILE = kTile, bool FEW = false>
 __device__ __forceinline__ int build_prefix_units(const DecodeArgs &a, const void *__restrict__ cur, int *pref, int *lens, int *wave_sums,
-                                                  int n_ranges) {
+                                                  int &n_ranges) {
+  const auto choose = [&](int64_t tiles) {
+    if (FEW && a.few_ranges > 0 && tiles < a.many_from) n_ranges = a.few_ranges;
+  };
   if (a.seg_free_tiles < 0 || a.users > kWave) {
     build_prefix<TILE>(a, cur, pref, lens, wave_sums, a.seg_units);
+    choose((int64_t)__builtin_amdgcn_readfirstlane(pref[a.users]) * a.hkv);
     return a.seg_units;
   }
   const int u = threadIdx.x & (kWave - 1);
   int len = 0, nt = 0;
   if (u < a.users) nt = tiles_of_user<TILE>(a, cur, u, len);
   const int tiles = wave_prefix_sum(nt);
-  const int64_t over = (int64_t)__builtin_amdgcn_readlane(tiles, kWave - 1) * a.hkv - a.seg_free_tiles;
+  const int64_t list = (int64_t)__builtin_amdgcn_readlane(tiles, kWave - 1) * a.hkv;
+  choose(list);
+  const int64_t over = list - (FEW ? min(a.seg_free_tiles, n_ranges) : a.seg_free_tiles);
   int extra = 0;
   for (int64_t at = 0; extra < a.seg_units && over > at; at += n_ranges) ++extra;
   const uint64_t some = __builtin_amdgcn_ballot_w64(nt > 0);  // users with tiles, up to and with this lane's:
@@ -647,7 +656,10 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(DecodeArgs a, int G
 
 template <bool PARKED = false>
 inline void launch_combine(const DecodeArgs &a, int segments, int g, int d, hipStream_t st) {
-  if (combine_sliced(a, segments))
+  // (a block-float-8 list may have filled half of the ranges only: not where the slices' workgroups do not fit the chip at once, nine
+  // per CU, either: 32 users of 32/8 heads, 3000 ... 24000 tiles, sliced / not 18.2 / 16.7 ... 48.2 / 46.8 us per layer; 18 users 17.4 / 17.1, 46.4 / 46.7)
+  const bool fits = a.few_ranges == 0 || (int64_t)segments * combine_pieces(g * d, kCombineSlices) <= 9 * 256;
+  if (combine_sliced(a, segments) && fits)
     decode_combine_kernel<kCombineSlices, PARKED><<<dim3(segments, combine_pieces(g * d, kCombineSlices)), dim3(256), 0, st>>>(a, g, d);
   else
     decode_combine_kernel<1, PARKED><<<dim3(segments, combine_pieces(g * d, 1)), dim3(256), 0, st>>>(a, g, d);

@@ -184,8 +184,8 @@ __global__ __launch_bounds__(DIRECT ? kWave *DIRECT : 256, (DIRECT || BFP8) && D
   __shared__ int s_wsum[kWavesPerBlock];
   extern __shared__ __attribute__((aligned(16))) uint8_t tiles[];
 
-  int seg_units = 0;
-  if constexpr (DIRECT == 0) seg_units = build_prefix_units<TILE>(a, cur_pos, s_pref, s_len, s_wsum, a.n_waves);
+  int seg_units = 0, n_ranges = a.n_waves;
+  if constexpr (DIRECT == 0) seg_units = build_prefix_units<TILE, BFP8 && D <= 128 && !LONG>(a, cur_pos, s_pref, s_len, s_wsum, n_ranges);
   const int lane = threadIdx.x & 63;
   const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 15, quad = lane >> 4;
@@ -211,7 +211,7 @@ __global__ __launch_bounds__(DIRECT ? kWave *DIRECT : 256, (DIRECT || BFP8) && D
     // The flat list in units: per segment `seg_units` units that stand for the cost of opening it,
     // then its tiles.  A range of more than seg_units units holds at least one tile.
     const int total_units = __builtin_amdgcn_readfirstlane(s_pref[a.users]);
-    const Share share = share_of(total_units, a.hkv, a.n_waves, seg_units, wave);
+    const Share share = share_of(total_units, a.hkv, n_ranges, seg_units, wave);
     total = share.total, n_eff = share.n_eff;
     if (total == 0 || wave >= n_eff) {
       publish_segment_row(a, s_pref, total, n_eff, seg_units);

@@ -364,7 +364,8 @@ __global__ __launch_bounds__(256, 1) void paged_decode_latent16_kernel(
   __shared__ int s_wsum[kWavesPerBlock];
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
-  const int seg_units = build_prefix_units<TILE>(a, cur_pos, s_pref, s_len, s_wsum, a.n_waves);
+  int n_ranges = a.n_waves;
+  const int seg_units = build_prefix_units<TILE>(a, cur_pos, s_pref, s_len, s_wsum, n_ranges);
 
   const int lane = threadIdx.x & 63;
   const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -820,7 +821,8 @@ __global__ __launch_bounds__(256) void paged_decode_latent128_kernel(
   __shared__ int s_wsum[NWAVES];
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
-  const int seg_units = build_prefix_units(a, cur_pos, s_pref, s_len, s_wsum, a.n_waves);
+  int n_ranges = a.n_waves;
+  const int seg_units = build_prefix_units(a, cur_pos, s_pref, s_len, s_wsum, n_ranges);
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
