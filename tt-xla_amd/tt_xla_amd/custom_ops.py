@@ -16,6 +16,7 @@ implementation here: calling them with CPU tensors raises.
 from __future__ import annotations
 
 import math
+import threading
 from typing import Optional
 
 import torch
@@ -434,7 +435,17 @@ def _decode(query, key, value, page_table, is_causal, attn_mask, cur_pos_tensor,
     return out
 
 
-_WORKSPACES = {}
+class _Workspaces(threading.local):
+    """Scratch tensors of this thread, by device."""
+
+    def __init__(self):
+        self.kept = {}
+
+    def clear(self):
+        self.kept.clear()
+
+
+_WORKSPACES = _Workspaces()
 
 
 # Largest scratch a block-float-8 chunk pass may ask for (bfloat16 copies of its users' blocks).
@@ -442,20 +453,22 @@ _EXPANSION_LIMIT = 8 << 30
 
 
 def _workspace(nbytes: int, device) -> torch.Tensor:
-    """A per-device scratch tensor for the split-K partials of a decode launch, grown on demand and
+    """A scratch tensor per thread and device for the split-K partials of a decode launch, grown on demand and
     reused by later calls: launches of one stream run in order, so one buffer serves them all, and
-    an eager serving loop pays no allocator round trip per layer and step.  Under graph capture the
+    an eager serving loop pays no allocator round trip per layer and step.  (An entry point launches several kernels that
+    hand data through it, with the interpreter lock released: another thread's, between them, would take it from under
+    them.)  Under graph capture the
     allocation has to belong to the graph's pool, and a call on another stream must not share the
     buffer, so both get a fresh tensor."""
     index = device.index if device.index is not None else torch.cuda.current_device()
     # (the default stream's handle is 0, and it cannot be captured)
     if torch._C._cuda_getCurrentRawStream(index) != 0 or torch.cuda.is_current_stream_capturing():
         return torch.empty(nbytes, dtype=torch.uint8, device=device)
-    key = (device.type, index)
-    ws = _WORKSPACES.get(key)
+    kept = _WORKSPACES.kept
+    ws = kept.get(index)
     if ws is None or ws.numel() < nbytes:
         ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
-        _WORKSPACES[key] = ws
+        kept[index] = ws
     return ws
 
 
