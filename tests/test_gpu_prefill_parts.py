@@ -181,3 +181,24 @@ def test_block_float_8_under_tables_too_narrow_to_be_split(monkeypatch, users, h
     got = _pass(*[t.cuda() for t in (q, packed[0], packed[1], table, st)], d**-0.5)
     assert bool(blocks.any()) == copies
     P._check(f"narrow u{users} h{hq}x{hkv} len{lc} width{nbpu}", got.cpu(), want)
+
+
+@pytest.mark.parametrize("d,bs,start", [(64, 64, 640), (64, 32, 1216), (128, 64, 1216), (256, 32, 832)])
+def test_infinite_values_of_the_last_part_stay_infinite(d, bs, start):
+    """An infinite V element seen by every row makes its output infinite, in whichever part of the keys it lies (the merge
+    reads parts four at a time)."""
+    from tt_xla_amd import _native as N
+
+    g = torch.Generator().manual_seed(d + start)
+    lc, inf = 32, float("inf")
+    nbpu = -(-(start + lc) // bs)
+    key, value, table = P._paged(g, 1, nbpu, 2, bs, d, False)
+    for column, t in enumerate(range(0, start, 48)):
+        value[int(table[0, t // bs]), :, t % bs, column] = inf if column % 2 else -inf
+    q = P._bf(g, 1, 4, lc, d)
+    st = torch.tensor([start], dtype=torch.int32)
+    assert N.lib().ttpa_sdpa_prefill_scratch_bytes(1, 4, 2, lc, d, bs, nbpu, 0) > 0
+    got = _pass(q.cuda(), key.cuda(), value.cuda(), table.cuda(), st.cuda(), d**-0.5).cpu().float()
+    want = O.chunked_sdpa(q, key, value, table, st, d**-0.5).float()
+    assert want.isinf().any() and torch.equal(got.isinf(), want.isinf()) and not got.isnan().any()
+    torch.testing.assert_close(got, want.reshape(got.shape), atol=2e-2, rtol=2e-2)

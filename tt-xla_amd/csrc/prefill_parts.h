@@ -74,7 +74,8 @@ __host__ __device__ inline PartLayout part_layout(const PrefillArgs &a, int rows
 // (row block, head, batch entry); thread (n, g) takes row n and head-dim elements 16 g .. 16 g + 15, which lie in
 // register groups 2 g and 2 g + 1 of lanes n and n + 32 (prefill_stream_kernel's lane holds elements
 // 8 group + 4 (lane / 32) .. + 3): 512 consecutive bytes per read of 32 lanes, whole 32-byte pieces of a row per
-// write.  Memory bound: 34 MB of accumulators (512 rows, 32 heads, 4 parts) in 7.9 us.
+// write.  Memory bound: 34 MB of accumulators (512 rows, 32 heads, 4 parts) in 7.9 us.  Parts past the last are zeros: repeated
+// with weight 0 they needed as long at head sizes 64 and 128 and 5 us more at 256 (128 rows of 16/8 heads behind 2048 tokens 36.7 / 31.7).
 template <int D, int RPW>
 __global__ __launch_bounds__(2 * D) void prefill_merge_kernel(PrefillArgs a) {
   const int rb = blockIdx.x, hq = blockIdx.y, b = blockIdx.z;
@@ -105,7 +106,8 @@ __global__ __launch_bounds__(2 * D) void prefill_merge_kernel(PrefillArgs a) {
   float o[16];
 #pragma unroll
   for (int i = 0; i < 16; ++i) o[i] = 0.f;
-  // four parts' accumulators in flight at a time; parts past the last repeat it with weight 0
+  // four parts' accumulators in flight at a time; parts past the last are zeros with weight 0 (with the last one's values an
+  // infinite one would become NaN)
   for (int p0 = 0; p0 < active; p0 += 4) {
     float4 v[4][4];
 #pragma unroll
@@ -117,6 +119,10 @@ __global__ __launch_bounds__(2 * D) void prefill_merge_kernel(PrefillArgs a) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       float w = 0.f;
+      if (p0 + j >= active) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[j][i] = make_float4(0.f, 0.f, 0.f, 0.f);
+      }
 #pragma unroll
       for (int p = 0; p < kMaxParts; ++p)
         if (p == p0 + j && p < active) w = __builtin_amdgcn_exp2f(m[p] - top), sum = fmaf(w, l[p], sum);
