@@ -426,6 +426,25 @@ int64_t ttpa_sdpa_prefill_scratch_bytes(int32_t batch, int32_t q_heads, int32_t 
                                         int32_t head_size, int32_t block_size, int32_t table_width,
                                         int32_t kv_format);
 
+/* The two for a caller who knows that the last query row sees at most `most_keys` keys (chunk_start + q_len, of which the
+ * library knows only the page table's room): whether copies are read and the keys are split goes by that number.  It
+ * changes the launches and never which keys are attended; 0: by the page table, as above. */
+int ttpa_sdpa_prefill_bounded(void *out, int64_t out_batch_stride, int64_t out_head_stride,
+                              int64_t out_token_stride, const void *q, int64_t q_batch_stride,
+                              int64_t q_head_stride, int64_t q_token_stride, const void *k,
+                              const void *v, int64_t kv_batch_stride, int64_t kv_head_stride,
+                              int64_t kv_token_stride, const int32_t *page_table,
+                              int64_t page_table_row_stride, const int32_t *chunk_start,
+                              const void *mask, int64_t mask_batch_stride, int64_t mask_row_stride,
+                              int32_t batch, int32_t q_heads, int32_t kv_heads, int32_t q_len,
+                              int32_t kv_len, int32_t head_size, int32_t block_size,
+                              int32_t table_width, int32_t num_blocks, int32_t causal, float scale,
+                              int32_t sliding_window, int32_t kv_format, int64_t most_keys, void *workspace,
+                              int64_t workspace_bytes, void *stream);
+int64_t ttpa_sdpa_prefill_bounded_scratch_bytes(int32_t batch, int32_t q_heads, int32_t kv_heads, int32_t q_len,
+                                                int32_t head_size, int32_t block_size, int32_t table_width,
+                                                int32_t kv_format, int64_t most_keys);
+
 /*
  * The backend's first-chunk prefill pass in one call: ttpa_paged_fill_cache on K and on V
  * (attention.py:486-515: the prompt's keys and values go into the paged caches through the

@@ -202,3 +202,45 @@ def test_infinite_values_of_the_last_part_stay_infinite(d, bs, start):
     want = O.chunked_sdpa(q, key, value, table, st, d**-0.5).float()
     assert want.isinf().any() and torch.equal(got.isinf(), want.isinf()) and not got.isnan().any()
     torch.testing.assert_close(got, want.reshape(got.shape), atol=2e-2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("hq,hkv,d,rows,start,bfp8", [
+    (8, 8, 64, 32, 64, False), (64, 8, 64, 512, 512, False), (16, 8, 256, 128, 64, False), (8, 8, 64, 128, 64, True),
+    (16, 16, 128, 128, 64, True),  # split in place by the table, copies by the chunk
+    (32, 8, 128, 32, 96, False),   # the streaming loop
+])
+def test_a_pass_is_laid_out_for_the_chunk_and_not_for_the_table(hq, hkv, d, rows, start, bfp8):
+    """The metadata's chunk_end, which the builder knows: a wide page table makes an eager pass no other than a table that ends with
+    the chunk.  It is never what is attended: a smaller number gives the same result, and a captured pass goes by the table."""
+    from tt_xla_amd import TTAttentionBackendImpl, custom_ops
+    from tt_xla_amd import _native as N
+    from tt_xla_amd.metadata import PagedMetadataBuilder
+
+    bs, g = 64, torch.Generator().manual_seed(hq + d + rows)
+    blocks = -(-(start + rows) // bs)
+    scratch = [int(N.lib().ttpa_sdpa_prefill_bounded_scratch_bytes(1, hq, hkv, rows, d, bs, 128, int(bfp8), n)) for n in (0, start + rows)]
+    assert scratch[0] == int(N.lib().ttpa_sdpa_prefill_scratch_bytes(1, hq, hkv, rows, d, bs, 128, int(bfp8))) > 0
+    assert scratch[1] == (2 * 128 * hkv * bs * d * 2 + 512 if d == 128 and bfp8 else 0)
+    table = torch.arange(1, blocks + 1, dtype=torch.int32).view(1, blocks).numpy()
+    caches = [P._bf(g, blocks + 1, hkv, bs, d).cuda() for _ in range(2)]
+    if bfp8:
+        caches = [custom_ops.bfp8_pack_cache(t) for t in caches]
+    q, k, v = (P._bf(g, rows, n * d).cuda() for n in (hq, hkv, hkv))
+    impl = TTAttentionBackendImpl(hq, d, d**-0.5, hkv, None, None, "auto")
+    outs = {}
+    for name, width, end in (("narrow", blocks, None), ("told", 128, start + rows), ("told less", 128, 32), ("not told", 128, None)):
+        meta = PagedMetadataBuilder(bs, width, max(32, rows), device="cuda").prepare(table, [start], [rows]).metadata
+        assert meta.chunk_end == start + rows
+        meta.chunk_end = end
+        outs[name] = torch.zeros_like(q)
+        assert impl._native_pass(q, k, v, caches, meta, outs[name])
+    meta.chunk_end = start + rows
+    captured, graph = torch.zeros_like(q), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        impl.forward(None, q, k, v, caches, meta, output=captured)
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(outs["narrow"], outs["told"])
+    for name in ("told less", "not told"):
+        torch.testing.assert_close(outs[name].float(), outs["told"].float(), atol=2e-2, rtol=2e-2)
+    assert torch.equal(captured, outs["not told"])

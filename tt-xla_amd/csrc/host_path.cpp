@@ -17,6 +17,7 @@
 #include <ATen/record_function.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 
 #include "ttpa.h"
@@ -90,13 +91,13 @@ inline at::Tensor scratch(int64_t bytes, const at::Tensor *like) {
 PyObject *result(const char *entry, int rc) { return rc == TTPA_OK ? PyLong_FromLong(0) : Py_BuildValue("(si)", entry, rc); }
 
 // attention_pass(query, key, value, k_cache, v_cache, page_table, cache_position, fill_page_table, batch_idx, chunk_start,
-//                sinks, output, users, heads, kv_heads, head_size, scale, window)
+//                sinks, output, users, heads, kv_heads, head_size, scale, window, chunk_end)
 // -> 0, (name, status) of the entry point that failed, or None: not an ordinary pass, nothing was issued.  A profiler
 // sees the names of the operators that the pass stands for.
 PyObject *attention_pass(PyObject *, PyObject *const *v, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 18) {
-    PyErr_SetString(PyExc_TypeError, "attention_pass takes 18 arguments");
+  if (n != 19) {
+    PyErr_SetString(PyExc_TypeError, "attention_pass takes 19 arguments");
     return nullptr;
   }
   if (c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled() ||
@@ -108,6 +109,7 @@ PyObject *attention_pass(PyObject *, PyObject *const *v, Py_ssize_t n) {
   const int64_t users = PyLong_AsLongLong(v[12]), hq = PyLong_AsLongLong(v[13]), hkv = PyLong_AsLongLong(v[14]);
   const int64_t d = PyLong_AsLongLong(v[15]), window = PyLong_AsLongLong(v[17]);
   const float scale = (float)PyFloat_AsDouble(v[16]);
+  int64_t most_keys = PyLong_Check(v[18]) ? PyLong_AsLongLong(v[18]) : 0;
   if (PyErr_Occurred()) {  // a number that does not fit 64 bits
     PyErr_Clear();
     Py_RETURN_NONE;
@@ -184,8 +186,10 @@ PyObject *attention_pass(PyObject *, PyObject *const *v, Py_ssize_t n) {
   }
   const at::Tensor *pt = p.table(v[5]), *start = p.numbers(v[9], 1);
   if (!pt || pt->size(0) != users || !start || is_i64(start)) Py_RETURN_NONE;
-  int64_t bytes = ttpa_sdpa_prefill_scratch_bytes((int32_t)users, (int32_t)hq, (int32_t)hkv, (int32_t)s, (int32_t)d, (int32_t)bs,
-                                                  (int32_t)pt->size(1), fmt);
+  // (what a graph captures is replayed for other chunks)
+  if (most_keys <= 0 || c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) most_keys = 0;
+  int64_t bytes = ttpa_sdpa_prefill_bounded_scratch_bytes((int32_t)users, (int32_t)hq, (int32_t)hkv, (int32_t)s, (int32_t)d, (int32_t)bs,
+                                                          (int32_t)pt->size(1), fmt, most_keys);
   if (bytes < 0 || bytes > kScratchLimit) bytes = 0;
   written(kc), written(vc), written(out);
   {
@@ -210,13 +214,13 @@ PyObject *attention_pass(PyObject *, PyObject *const *v, Py_ssize_t n) {
         bytes = 0;
       }
     }
-    return ttpa_sdpa_prefill_expanded(
+    return ttpa_sdpa_prefill_bounded(
         out->data_ptr(), s * hq * d, d, hq * d, q->data_ptr(), s * q->stride(0), d, q->stride(0), kc->data_ptr(), vc->data_ptr(), 0, 0,
         0, static_cast<const int32_t *>(pt->data_ptr()), pt->stride(0), static_cast<const int32_t *>(start->data_ptr()), nullptr, 0, 0,
         (int32_t)users, (int32_t)hq, (int32_t)hkv, (int32_t)s, (int32_t)(pt->size(1) * bs), (int32_t)d, (int32_t)bs,
-        (int32_t)pt->size(1), (int32_t)nb, 1, scale, 0, fmt, bytes ? ws.data_ptr() : nullptr, bytes, stream);
+        (int32_t)pt->size(1), (int32_t)nb, 1, scale, 0, fmt, most_keys, bytes ? ws.data_ptr() : nullptr, bytes, stream);
   };
-  return result("ttpa_sdpa_prefill_expanded", launch());
+  return result("ttpa_sdpa_prefill_expanded", launch());  // (its bounded form; an error reads as the operators')
   END_HANDLE_TH_ERRORS
 }
 

@@ -751,7 +751,7 @@ static int prefill_impl(void *out, int64_t out_batch_stride, int64_t out_head_st
                                  int32_t block_size, int32_t table_width, int32_t num_blocks,
                                  int32_t causal, float scale, int32_t sliding_window, void *stream,
                                  const FillSpec *fill = nullptr, int32_t kv_format = TTPA_KV_BF16,
-                                 void *workspace = nullptr, int64_t workspace_bytes = 0) {
+                                 void *workspace = nullptr, int64_t workspace_bytes = 0, int64_t most_keys = 0) {
   TTPA_REQUIRE(out && q && k && v, "null pointer argument");
   TTPA_REQUIRE(sliding_window >= 0, "prefill: sliding_window %d is negative", sliding_window);
   TTPA_REQUIRE(sliding_window == 0 || causal, "prefill: a sliding window needs causal masking");
@@ -798,6 +798,7 @@ static int prefill_impl(void *out, int64_t out_batch_stride, int64_t out_head_st
   a.mask_bs = mask_batch_stride, a.mask_rs = mask_row_stride;
   a.batch = batch, a.hq = q_heads, a.hkv = kv_heads, a.sq = q_len, a.skv = kv_len;
   a.bs = block_size, a.w = table_width, a.nb = num_blocks, a.causal = causal ? 1 : 0;
+  a.keys_known = page_table && most_keys > 0, a.keys_bound = a.keys_known ? std::min<int64_t>(most_keys, kv_len) : kv_len;
   a.window = sliding_window;
   a.scale_log2e = scale * 1.4426950408889634f;
   {
@@ -875,6 +876,11 @@ extern "C" int ttpa_sdpa_prefill_expanded(TTPA_PREFILL_PARAMS, int32_t sliding_w
   return prefill_impl(TTPA_PREFILL_ARGS, sliding_window, stream, nullptr, kv_format, workspace, workspace_bytes);
 }
 
+extern "C" int ttpa_sdpa_prefill_bounded(TTPA_PREFILL_PARAMS, int32_t sliding_window, int32_t kv_format, int64_t most_keys,
+                                         void *workspace, int64_t workspace_bytes, void *stream) {
+  return prefill_impl(TTPA_PREFILL_ARGS, sliding_window, stream, nullptr, kv_format, workspace, workspace_bytes, most_keys);
+}
+
 extern "C" int64_t ttpa_sdpa_prefill_workspace_bytes(int32_t batch, int32_t kv_heads, int32_t head_size,
                                                      int32_t block_size, int32_t table_width, int32_t kv_format) {
   if (kv_format != TTPA_KV_BFP8 || batch <= 0 || kv_heads <= 0 || head_size <= 0 || block_size <= 0 || table_width <= 0)
@@ -884,12 +890,20 @@ extern "C" int64_t ttpa_sdpa_prefill_workspace_bytes(int32_t batch, int32_t kv_h
 
 extern "C" int64_t ttpa_sdpa_prefill_scratch_bytes(int32_t batch, int32_t q_heads, int32_t kv_heads, int32_t q_len, int32_t head_size,
                                                    int32_t block_size, int32_t table_width, int32_t kv_format) {
+  return ttpa_sdpa_prefill_bounded_scratch_bytes(batch, q_heads, kv_heads, q_len, head_size, block_size, table_width, kv_format, 0);
+}
+
+extern "C" int64_t ttpa_sdpa_prefill_bounded_scratch_bytes(int32_t batch, int32_t q_heads, int32_t kv_heads, int32_t q_len,
+                                                           int32_t head_size, int32_t block_size, int32_t table_width,
+                                                           int32_t kv_format, int64_t most_keys) {
   if (batch <= 0 || q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads || q_len <= 0 || head_size <= 0 || block_size <= 0 || table_width <= 0)
     return 0;
   const int32_t some_table = 0;
   PrefillArgs a = {};
   a.pt = &some_table, a.stream = 1;
   a.batch = batch, a.hq = q_heads, a.hkv = kv_heads, a.sq = q_len, a.bs = block_size, a.w = table_width;
+  a.keys_bound = (int64_t)table_width * block_size;
+  if (most_keys > 0) a.keys_known = 1, a.keys_bound = std::min(a.keys_bound, most_keys);
   if (kv_format == TTPA_KV_BFP8) {
     if (!stream_expands(a, head_size, INT64_MAX)) return plain_part_bytes(a, head_size, true);
     return ttpa_sdpa_prefill_workspace_bytes(batch, kv_heads, head_size, block_size, table_width, kv_format) + stream_part_bytes(a, head_size);

@@ -63,6 +63,8 @@ struct PrefillArgs {
   int parts, parts_one;  // shares of the keys at most; with one workgroup per CU
   int split_from;        // launches whose last row block has fewer 32-key blocks are not split
   int part_min;          // 32-key blocks of a part at least
+  int64_t keys_bound;    // keys of the last row at most, as far as the host knows: what the launch is laid out for (set_parts)
+  int keys_known;        // ... from the caller, and not from the page table's room
 };
 
 // key / block_size without a division instruction sequence (about 30 instructions each, and the

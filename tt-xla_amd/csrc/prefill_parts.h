@@ -32,12 +32,16 @@ namespace {
 //   head size 64, 64 / 8 heads:  1 x 128 rows behind 640 tokens 21.9 / 18.5, 2368 47.1 / 24.4
 //   head size 256, 16 / 8 heads: 5 x 192 rows behind 832 tokens 67 / 49; 1 x 32 behind 256 23.8 / 20.7, 2368 97.9 / 32.9
 //   block-float-8, 8 / 8 of 64:  1 x 128 rows behind 640 tokens 26.9 / 17.3, 2368 65 / 18.8
-// Under a page table that holds little more than the blocks to split from, the parts would be few and the merge launch (1.4 us)
-// be there for nothing where the pass reads less of it: 1 x 32 rows behind 128 tokens 10.4 us, 12.4 with.
+// The host knows how many blocks there may be from the page table, or closer from a caller who knows where the chunk lies
+// (a.keys_bound): by a table of 8192 tokens alone a pass that reads few of them prepares a split that it does not make, which costs
+// 1.5 us (whole passes, bounded / not: 32 rows of 8/8 heads of 64 behind 64 tokens 9.2 / 10.9, 512 rows of 64/8 behind 512 24.5 /
+// 26.2, block-float-8, 128 rows of 16/16 of 128 behind 64 16.2 / 19.3).  Where
+// a table holds little more than the blocks to split from, the parts would be few and the merge launch be there for nothing
+// where the pass reads less: 1 x 32 rows behind 128 tokens 10.4 us, 12.4 with.
 struct SplitRule {
   int wgs_per_cu;               // workgroup slots of a CU
   int min_part, min_split;      // 32-key blocks per part at least; blocks from which on a launch is split
-  int table_percent;            // the page table holds at least this many hundredths of the blocks to split from
+  int table_percent;            // a page table holds at least this many hundredths of the blocks to split from
   int block_cost;               // of a 32-key block, in hundredths of the streaming loop's
 };
 constexpr SplitRule kStreamSplit = {2, 8, 16, 100, 100};  // (80 KiB of LDS per workgroup)
@@ -143,18 +147,18 @@ __global__ __launch_bounds__(2 * D) void prefill_merge_kernel(PrefillArgs a) {
 }
 
 // Workgroups of the launch without a split, and what it may be split into: as many parts as fill the workgroup slots of
-// every CU once, if its row blocks leave at least half of them empty and its page table is wide enough to be split at all.
+// every CU once, if its row blocks leave at least half of them empty and its page keys may be enough to be split at all.
 inline void set_parts(PrefillArgs &a, int heads_per_wg, const SplitRule &rule) {
   int cus = device_cus();
   if (cus <= 0) cus = 256;
   const int rows = kRowsPerWave * 4 / heads_per_wg;
   const int64_t wgs = (int64_t)a.batch * (a.hq / heads_per_wg) * ((a.sq + rows - 1) / rows);
-  const int blocks = (int)(((int64_t)a.w * a.bs + kBlockKeys - 1) / kBlockKeys);
+  const int blocks = (int)((a.keys_bound + kBlockKeys - 1) / kBlockKeys);
   const int most = std::min(kMaxParts, (blocks + rule.min_part - 1) / rule.min_part);
   const int64_t from = 2 * wgs <= cus ? 7 * wgs / 16 : std::min<int64_t>(wgs, rule.wgs_per_cu * cus) / 2;
   a.split_from = (int)std::max<int64_t>(rule.min_split, 100 * from / rule.block_cost);
   a.part_min = rule.min_part;
-  a.parts = blocks < a.split_from * rule.table_percent / 100 ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>(rule.wgs_per_cu * cus / wgs, most));
+  a.parts = blocks < a.split_from * (a.keys_known ? 100 : rule.table_percent) / 100 ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>(rule.wgs_per_cu * cus / wgs, most));
   a.parts_one = (int)std::max<int64_t>(1, std::min<int64_t>(cus / wgs, most));
 }
 

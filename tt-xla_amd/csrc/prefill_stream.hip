@@ -475,7 +475,7 @@ bool stream_expands(const PrefillArgs &a, int head_size, int64_t room) {
   if (!stream_serves(a, head_size)) return false;
   const int hpw = heads_per_workgroup(a), rows = kRowsPerWave * 4 / hpw;
   const int64_t row_blocks = (a.sq + rows - 1) / rows;
-  const bool pays = row_blocks > 1 || (int64_t)a.batch * a.w * a.bs * a.hkv <= 8192 || part_bytes(a, hpw, kStreamSplit, kD) > 0;
+  const bool pays = row_blocks > 1 || a.batch * a.keys_bound * a.hkv <= 8192 || part_bytes(a, hpw, kStreamSplit, kD) > 0;
   const int64_t parts = plain_part_bytes(a, kD, true);
   return pays && !(parts > 0 && parts <= room && row_blocks * (a.hq / hpw / a.hkv) <= 2);
 }

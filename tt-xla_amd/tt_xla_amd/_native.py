@@ -106,6 +106,11 @@ SIGNATURES = {
         [_p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _p, _i64, _i64, _i64, _p, _i64, _p, _p,
          _i64, _i64, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _f32, _i32, _i32, _p, _i64, _p],
     ),
+    "ttpa_sdpa_prefill_bounded": (
+        _int,
+        [_p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _p, _i64, _i64, _i64, _p, _i64, _p, _p,
+         _i64, _i64, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _f32, _i32, _i32, _i64, _p, _i64, _p],
+    ),
     "ttpa_sdpa_prefill_workspace_bytes": (_i64, [_i32, _i32, _i32, _i32, _i32, _i32]),
     "ttpa_latent_decode_step_workspace_bytes": (_sz, [_i32, _i32]),
     "ttpa_latent_decode_step": (
@@ -132,6 +137,7 @@ SIGNATURES = {
         [_p, _p, _i64, _i64, _p, _i64, _i64, _p, _i64, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _p],
     ),
     "ttpa_sdpa_prefill_scratch_bytes": (_i64, [_i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32]),
+    "ttpa_sdpa_prefill_bounded_scratch_bytes": (_i64, [_i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i64]),
     "ttpa_latent_prefill": (
         _int,
         [_p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _i64, _i64, _i64,

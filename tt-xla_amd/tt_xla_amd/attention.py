@@ -76,6 +76,9 @@ class TTMetadata:
     chunk_start_idx [1] int32 = tokens already in the cache for a continuation chunk, or
                     None for a first / unchunked prefill.
     batch_idx       [users] int32 page-table row of each fill_value row.
+    chunk_end       position behind the last row of a continuation chunk, where the host knows it: eager passes are
+                    laid out for that many keys and not for all that the page table has room for.  Never what is
+                    attended: chunk_start_idx says that.
     """
 
     cache_position: Optional[torch.Tensor]
@@ -86,6 +89,7 @@ class TTMetadata:
     chunk_start_idx: Optional[torch.Tensor]
     batch_idx: Optional[torch.Tensor] = None
     num_users: Optional[int] = None
+    chunk_end: Optional[int] = None
 
     def __init__(
         self,
@@ -98,6 +102,7 @@ class TTMetadata:
         chunk_start_idx: Optional[torch.Tensor] = None,
         batch_idx: Optional[torch.Tensor] = None,
         num_users: Optional[int] = None,
+        chunk_end: Optional[int] = None,
     ):
         self.cache_position = cache_position
         self.attn_mask = attn_mask
@@ -108,6 +113,7 @@ class TTMetadata:
         self.chunk_start_idx = chunk_start_idx
         self.num_users = num_users
         self.batch_idx = batch_idx
+        self.chunk_end = chunk_end
 
 
 class TTAttentionMetadataBuilder:
@@ -341,6 +347,7 @@ class TTAttentionBackendImpl(_ImplBase):
             attn_metadata.fill_page_table, attn_metadata.batch_idx, attn_metadata.chunk_start_idx, self.sinks, output,
             attn_metadata.num_users, self.num_heads, self.num_kv_heads, self.head_size, self.scale,
             0 if self.sliding_window is None else self.sliding_window or -1,  # (0 is not a window: the operators say so)
+            getattr(attn_metadata, "chunk_end", None),
         )
         if status is None:
             return False

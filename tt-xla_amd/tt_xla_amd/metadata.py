@@ -271,7 +271,7 @@ class PagedMetadataBuilder:
         active_rows = np.nonzero(num_scheduled > 0)[0]
         active_computed = num_computed[active_rows]
         prefix_chunk_step = padded_tokens > 1 and bool(np.any(active_computed > 0))
-        chunk_start_idx = None
+        chunk_start_idx = chunk_end = None
         if prefix_chunk_step and (self.chunked_sdpa or self.spec_prefix_rows):
             active_starts = active_computed - lead[active_rows]
             offsets = {int(v) for v in active_starts}
@@ -284,6 +284,7 @@ class PagedMetadataBuilder:
                 )
             self._chunk_start_dev.copy_(torch.tensor([int(active_starts[0])], dtype=torch.int32))
             chunk_start_idx = self._chunk_start_dev
+            chunk_end = int(active_starts[0]) + padded_tokens
 
         copy_width = min(block_table.shape[1], self.read_width)
         page_table = torch.zeros((rows, self.read_width), dtype=torch.int32)
@@ -319,5 +320,6 @@ class PagedMetadataBuilder:
             chunk_start_idx=chunk_start_idx,
             batch_idx=batch_idx,
             num_users=rows,
+            chunk_end=chunk_end,
         )
         return PassPlan(metadata, lead, padded_tokens, positions, is_decode)
