@@ -48,7 +48,9 @@ def test_split_chunks(users, hq, hkv, d, bs, start, lc):
     (1, 8, 8, 64, 32, 1300, 96), (2, 8, 2, 64, 64, 700, 33), (1, 64, 8, 128, 64, 2368, 32), (3, 4, 4, 128, 32, 900, 40),
     (1, 4, 1, 128, 16, 1100, 100),
 ])
-def test_split_chunks_over_block_float_8(users, hq, hkv, d, bs, start, lc):
+def test_split_chunks_over_block_float_8(users, hq, hkv, d, bs, start, lc, monkeypatch):
+    from tt_xla_amd import _native as N
+
     g = torch.Generator().manual_seed(hq + bs + start + d)
     nbpu = -(-(start + lc) // bs) + 1
     key, value, table = P._paged(g, users, nbpu, hkv, bs, d, False)
@@ -56,8 +58,14 @@ def test_split_chunks_over_block_float_8(users, hq, hkv, d, bs, start, lc):
     st = torch.tensor([start], dtype=torch.int32)
     packed = [bfp8_codec.pack_cache(t) for t in (key, value)]
     want = O.chunked_sdpa(q, *[bfp8_codec.unpack_cache(t, bs).to(torch.bfloat16) for t in packed], table, st, d**-0.5)
-    got = _pass(q.cuda(), packed[0].cuda(), packed[1].cuda(), table.cuda(), st.cuda(), d**-0.5)
+    args = [t.cuda() for t in (q, packed[0], packed[1], table, st)]
+    got = _pass(*args, d**-0.5)
     P._check(f"split bfp8 u{users} h{hq}x{hkv} d{d} bs{bs} start{start} len{lc}", got.cpu(), want)
+    call = N.call
+    monkeypatch.setattr(N, "call", lambda name, *a: call(name, *(a[:-3] + (0, 0, a[-1]) if name == "ttpa_sdpa_prefill_expanded" else a)))
+    unsplit = _pass(*args, d**-0.5)
+    P._check("the same, unsplit", unsplit.cpu(), want)
+    assert not torch.equal(got, unsplit), "the pass was not split"
 
 
 @pytest.mark.parametrize("d,bs", [(64, 64), (64, 32), (128, 16), (256, 32)])
