@@ -158,7 +158,7 @@ __device__ __forceinline__ void merge_waves(const DecodeArgs &a, int u, int h, i
 // scores (a.mask; the form of a pass that is not causal, built with RUNS = 0 and without the update).
 // DIRECT: a workgroup of DIRECT wavefronts owns the whole segment blockIdx.x (chosen by direct_waves, decode.hip): no prefix, no
 // search, no partials, no merge launch.  Its wavefronts take the segment's tiles in turn.  LONG: tiles of 16 KiB (a.long_tiles).
-template <int D, bool BFP8, int RUNS, bool FUSED, bool MASKED = false, int DIRECT = 0, bool LONG = false>
+template <int D, bool BFP8, int RUNS, bool FUSED, bool MASKED = false, int DIRECT = 0, bool LONG = false, bool ONE = false>
 __global__ __launch_bounds__(DIRECT ? kWave *DIRECT : 256, (DIRECT || BFP8) && D <= 128 && !LONG ? 2 : 1) void paged_decode_mfma16_kernel(
     DecodeArgs a, const int32_t *__restrict__ page_table, const void *__restrict__ cur_pos) {
   static_assert(D == 64 || D == 128 || D == 256, "shapes built");
@@ -221,7 +221,7 @@ __global__ __launch_bounds__(DIRECT ? kWave *DIRECT : 256, (DIRECT || BFP8) && D
   }
   int64_t x = x_lo;  // set below to the unit of the first tile at or behind x_lo
   uint8_t *tile = tiles + wib * kTileBytes;
-  const int G = a.hq / a.hkv;
+  const int G = ONE ? 1 : a.hq / a.hkv;
 
   // staging lane mapping and swizzled write positions
   const int sr = lane / LPR, sc = lane % LPR;
@@ -443,8 +443,6 @@ __global__ __launch_bounds__(DIRECT ? kWave *DIRECT : 256, (DIRECT || BFP8) && D
   float m_run = -INFINITY, l_run = 0.f;
   int ev_run = 0;  // reference exponent of the V accumulator
 
-  const uint32_t below = G == 1 ? 0x00010001u : 0u;  // what the first of two parts of a pair of weights is less
-
   auto process_tile = [&](auto has_next_tag) {
     constexpr bool has_next = decltype(has_next_tag)::value;
     const int nvalid = cur.len - cur.t * TILE;
@@ -577,10 +575,11 @@ __global__ __launch_bounds__(DIRECT ? kWave *DIRECT : 256, (DIRECT || BFP8) && D
         for (int r = 0; r < 4; r += 2) {
           const float p0 = __builtin_amdgcn_exp2f(fmaf(st[b][r], scale, -m_safe));
           const float p1 = __builtin_amdgcn_exp2f(fmaf(st[b][r + 1], scale, -m_safe));
-          const uint32_t w = less_units(pack_bf16x2(p0, p1), below);
+          uint32_t w = pack_bf16x2(p0, p1);
+          if constexpr (ONE) w = less_units(w, 0x00010001u);
           lsum += bf16_lo(w) + bf16_hi(w);  // the normaliser sums the weights that multiply V
           pf[b >> 1][2 * (b & 1) + (r >> 1)] = w;
-          st[b][r] = p0 - bf16_lo(w), st[b][r + 1] = p1 - bf16_hi(w);  // the second parts, where there are two
+          if constexpr (ONE) st[b][r] = p0 - bf16_lo(w), st[b][r + 1] = p1 - bf16_hi(w);  // the second parts
         }
     }
     l_run = l_run * alpha + lsum;
@@ -603,24 +602,24 @@ __global__ __launch_bounds__(DIRECT ? kWave *DIRECT : 256, (DIRECT || BFP8) && D
         }
     };
     second_product();
-    // One query head per KV head: the weights in two bfloat16 parts.  The dot-product kernel, which serves such groups where this
+    // One query head per KV head (ONE): the weights in two bfloat16 parts.  The dot-product kernel, which serves such groups where this
     // one is not built, keeps a running maximum per sixteen of a tile's tokens, so more of its weights are exact; rounded once, this
     // kernel's results were 4 - 7 % further from a 64-bit evaluation than that one's (2.09e-3 against 1.97e-3, 128 tokens of 8 / 8
     // heads), in two parts they are 15 - 17 % closer (1.66e-3).  The first part is the rounded weight less one unit of its last
-    // place, so that the second is positive: with zero or less, an infinite V element would come out as NaN.
-    if constexpr (!BFP8) {
-      if (G == 1) {
-        float low = 0.f;
+    // place, so that the second is positive: with zero or less, an infinite V element would come out as NaN.  A kernel of its own: as a
+    // run-time branch the second parts cost every group 1 - 3 % (branch / kernels: 5 users of 32/8 heads in a window of 4096 19.1 / 18.9 us,
+    // 8 of 64/8 of 64 with 512 ... 4096 17.0 / 16.7, 37 of 8/8 of 64 in a window of 512 14.5 / 14.0).
+    if constexpr (ONE) {
+      float low = 0.f;
 #pragma unroll
-        for (int b = 0; b < KBLK; ++b)
+      for (int b = 0; b < KBLK; ++b)
 #pragma unroll
-          for (int r = 0; r < 4; r += 2) {
-            low += st[b][r] + st[b][r + 1];
-            pf[b >> 1][2 * (b & 1) + (r >> 1)] = pack_bf16x2(st[b][r], st[b][r + 1]);
-          }
-        l_run += low;
-        second_product();
-      }
+        for (int r = 0; r < 4; r += 2) {
+          low += st[b][r] + st[b][r + 1];
+          pf[b >> 1][2 * (b & 1) + (r >> 1)] = pack_bf16x2(st[b][r], st[b][r + 1]);
+        }
+      l_run += low;
+      second_product();
     }
 
     // ---- close the segment --------------------------------------------------------------------
@@ -670,48 +669,49 @@ __global__ __launch_bounds__(DIRECT ? kWave *DIRECT : 256, (DIRECT || BFP8) && D
   process_tile(std::false_type{});
 }
 
-template <int D, bool BFP8, int RUNS, bool FUSED, bool MASKED = false, int DIRECT = 0, bool LONG = false>
+template <int D, bool BFP8, int RUNS, bool FUSED, bool MASKED = false, int DIRECT = 0, bool LONG = false, bool ONE = false>
 bool launch(const DecodeArgs &a, hipStream_t st) {
   constexpr int kWaves = DIRECT ? DIRECT : kWavesPerBlock;
   const int blocks = DIRECT ? a.users * a.hkv : a.n_waves / kWavesPerBlock;
   const size_t lds = (size_t)kWaves * tile_bytes<D, LONG>();
   static std::atomic<uint64_t> lds_ready{0};
-  const auto kernel = &paged_decode_mfma16_kernel<D, BFP8, RUNS, FUSED, MASKED, DIRECT, LONG>;
+  const auto kernel = &paged_decode_mfma16_kernel<D, BFP8, RUNS, FUSED, MASKED, DIRECT, LONG, ONE>;
   if (!ensure_dynamic_lds(reinterpret_cast<const void *>(kernel), lds, lds_ready)) return false;
   launch_dominant(kernel, dim3(blocks), dim3(kWave * kWaves), lds, st, a, a.pt, a.cur);
   return true;
 }
 
-// One workgroup per segment (a.direct).
-template <int D, bool BFP8, bool FUSED, int DIRECT>
-bool launch_direct(const DecodeArgs &a, hipStream_t st) {
-  constexpr int TILE = tile_bytes<D>() / (2 * D);
-  return a.bs % TILE == 0 ? launch<D, BFP8, 1, FUSED, false, DIRECT>(a, st) : launch<D, BFP8, 2, FUSED, false, DIRECT>(a, st);
-}
-
-// Equal ranges of the flat list.
-template <int D, bool BFP8, bool FUSED, bool LONG>
-bool launch_ranges(const DecodeArgs &a, hipStream_t st) {
+// Equal ranges of the flat list, or one workgroup per segment (DIRECT); the variant for the block size.
+template <int D, bool BFP8, bool FUSED, int DIRECT, bool LONG, bool ONE>
+bool launch_runs(const DecodeArgs &a, hipStream_t st) {
   constexpr int TILE = tile_bytes<D, LONG>() / (2 * D);
-  if (a.bs % TILE == 0) return launch<D, BFP8, 1, FUSED, false, 0, LONG>(a, st);
-  if (a.bs % (TILE / 2) == 0) return launch<D, BFP8, 2, FUSED, false, 0, LONG>(a, st);
-  if (LONG || a.bs % (TILE / 4) == 0) return launch<D, BFP8, 4, FUSED, false, 0, LONG>(a, st);  // (block-float-8: blocks of 16 tokens)
-  if constexpr (!LONG) return launch<D, BFP8, 0, FUSED, false, 0, LONG>(a, st);
+  if (a.bs % TILE == 0) return launch<D, BFP8, 1, FUSED, false, DIRECT, LONG, ONE>(a, st);
+  if (DIRECT > 0 || a.bs % (TILE / 2) == 0) return launch<D, BFP8, 2, FUSED, false, DIRECT, LONG, ONE>(a, st);
+  if constexpr (DIRECT == 0) {
+    if (LONG || a.bs % (TILE / 4) == 0) return launch<D, BFP8, 4, FUSED, false, 0, LONG, ONE>(a, st);  // (block-float-8: blocks of 16 tokens)
+    if constexpr (!LONG) return launch<D, BFP8, 0, FUSED, false, 0, false, ONE>(a, st);
+  }
+  return false;
 }
 
-// Picks the variant for the block size and for a.k_new (set: the launch also performs the
-// cache update of the step).
+// FUSED (a.k_new set): the launch also performs the cache update of the step.
+template <int D, bool BFP8, bool FUSED>
+bool launch_form(const DecodeArgs &a, hipStream_t st) {
+  constexpr bool kOneHead = !BFP8;  // one query head per KV head has kernels of its own
+  const bool one = kOneHead && a.hq == a.hkv;
+  if constexpr (D <= 128) {
+    if (a.direct == 4) return one ? launch_runs<D, BFP8, FUSED, 4, false, kOneHead>(a, st) : launch_runs<D, BFP8, FUSED, 4, false, false>(a, st);
+    if (a.direct == 8) return one ? launch_runs<D, BFP8, FUSED, 8, false, kOneHead>(a, st) : launch_runs<D, BFP8, FUSED, 8, false, false>(a, st);
+  }
+  if constexpr (D == 128 && BFP8)
+    if (a.long_tiles) return launch_runs<D, BFP8, FUSED, 0, true, false>(a, st);
+  return one ? launch_runs<D, BFP8, FUSED, 0, false, kOneHead>(a, st) : launch_runs<D, BFP8, FUSED, 0, false, false>(a, st);
+}
+
 template <int D, bool BFP8>
 bool launch_for_block_size(const DecodeArgs &a, hipStream_t st) {
-  const bool fused = a.k_new != nullptr;
-  if constexpr (D <= 128) {
-    if (a.direct == 4) return fused ? launch_direct<D, BFP8, true, 4>(a, st) : launch_direct<D, BFP8, false, 4>(a, st);
-    if (a.direct == 8) return fused ? launch_direct<D, BFP8, true, 8>(a, st) : launch_direct<D, BFP8, false, 8>(a, st);
-  }
-  if (a.mask != nullptr) return !fused && launch<D, BFP8, 0, false, true>(a, st);
-  if constexpr (D == 128 && BFP8)
-    if (a.long_tiles) return fused ? launch_ranges<D, BFP8, true, true>(a, st) : launch_ranges<D, BFP8, false, true>(a, st);
-  return fused ? launch_ranges<D, BFP8, true, false>(a, st) : launch_ranges<D, BFP8, false, false>(a, st);
+  if (a.mask != nullptr) return a.k_new == nullptr && launch<D, BFP8, 0, false, true>(a, st);
+  return a.k_new ? launch_form<D, BFP8, true>(a, st) : launch_form<D, BFP8, false>(a, st);
 }
 
 }  // namespace
