@@ -163,7 +163,8 @@ def test_block_float_8_with_room_for_the_copies_only(monkeypatch):
 
 @pytest.mark.parametrize("users,hq,hkv,lc,nbpu,copies", [
     (1, 16, 16, 32, 3, True), (1, 16, 16, 128, 3, True), (8, 16, 16, 256, 12, True),  # few rows to copy; two row blocks
-    (4, 40, 8, 64, 6, False),                                                         # one row block, and many rows
+    (4, 40, 8, 64, 6, False), (5, 40, 8, 64, 10, True),                               # one row block, five readers of few keys, of many
+    (8, 16, 8, 128, 4, False), (1, 16, 16, 128, 4, True), (5, 16, 8, 64, 4, False),   # two row blocks over few keys; few rows, many
 ])
 def test_block_float_8_under_tables_too_narrow_to_be_split(monkeypatch, users, hq, hkv, lc, nbpu, copies):
     """Where neither loop is split, a pass reads copies if they are few or read more than once: its scratch is theirs,

@@ -42,10 +42,11 @@ struct SplitRule {
   int wgs_per_cu;               // workgroup slots of a CU
   int min_part, min_split;      // 32-key blocks per part at least; blocks from which on a launch is split
   int table_percent;            // a page table holds at least this many hundredths of the blocks to split from
+  int known_percent;            // ... or that the caller knows of: copies are better than the shortest split of block-float-8 blocks
   int block_cost;               // of a 32-key block, in hundredths of the streaming loop's
 };
-constexpr SplitRule kStreamSplit = {2, 8, 16, 100, 100};  // (80 KiB of LDS per workgroup)
-constexpr SplitRule plain_split(int d, bool bfp8) { return {d <= 128 ? 2 : 1, 4, 8, bfp8 ? 125 : 150, d == 256 ? 300 : bfp8 ? 225 : 150}; }
+constexpr SplitRule kStreamSplit = {2, 8, 16, 100, 100, 100};  // (80 KiB of LDS per workgroup)
+constexpr SplitRule plain_split(int d, bool bfp8) { return {d <= 128 ? 2 : 1, 4, 8, bfp8 ? 125 : 150, bfp8 && d == 128 ? 113 : 100, d == 256 ? 300 : bfp8 ? 225 : 150}; }
 // Parts up to one workgroup per CU; twice as many, which then share a CU's matrix pipes, from this many blocks per part
 // on (128 workgroups, 2 / 4 parts: 64 blocks 35.0 / 35.6 us, 80 blocks 43.5 / 41.5, 96 blocks 43.6 / 40.8, 256 blocks
 // 82.5 / 77.3).
@@ -158,7 +159,7 @@ inline void set_parts(PrefillArgs &a, int heads_per_wg, const SplitRule &rule) {
   const int64_t from = 2 * wgs <= cus ? 7 * wgs / 16 : std::min<int64_t>(wgs, rule.wgs_per_cu * cus) / 2;
   a.split_from = (int)std::max<int64_t>(rule.min_split, 100 * from / rule.block_cost);
   a.part_min = rule.min_part;
-  a.parts = blocks < a.split_from * (a.keys_known ? 100 : rule.table_percent) / 100 ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>(rule.wgs_per_cu * cus / wgs, most));
+  a.parts = blocks < a.split_from * (a.keys_known ? rule.known_percent : rule.table_percent) / 100 ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>(rule.wgs_per_cu * cus / wgs, most));
   a.parts_one = (int)std::max<int64_t>(1, std::min<int64_t>(cus / wgs, most));
 }
 

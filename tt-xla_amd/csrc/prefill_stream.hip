@@ -463,21 +463,27 @@ int64_t stream_part_bytes(const PrefillArgs &a, int head_size) {
   return a.pt && stream_serves(a, head_size) ? part_bytes(a, heads_per_workgroup(a), kStreamSplit, kD) : 0;
 }
 
-// A pass that reads a block once expands it no more often in mode 4, on its way into LDS, than into copies, a trip through memory in
-// front of the attention; the copies pay where there are several row blocks, where they are few, or where they let the keys be split
-// (16 / 16 heads, copies / mode 4: 1 x 128 rows behind 64 tokens 16.4 / 19.0 us, 8 x 256 behind 512 47.8 / 49.1; 40 / 8 heads, 4 x 64
-// behind 256 25.1 / 20.8).
-// Not where mode 4 itself is split and a block is read by at most two workgroups (row blocks times head groups of a KV head).
-// Passes in us, copies / mode 4: 1 x 32 rows behind 512 tokens, 64 / 8 heads 23.1 / 18.8; 4 x 32 rows of 32 / 8 behind 1024 32.1 / 25.3, 4096 49.3 /
-// 38.7; 8 x 128 of 16 / 16 behind 4096 167 / 75.6; two row blocks: 4 x 64 of 32 / 8 behind 512 29.5 / 24.9, 8 x 256 of 16 / 16 behind
-// 4096 195 / 128.  Four workgroups: 2 x 64 of 64 / 8 behind 4096 49.5 / 55.6; three: 2 x 96 of 32 / 8 46.7 / 50.0.
+// Whether a block-float-8 pass reads bfloat16 copies, written by a launch in front of it, or expands blocks on their way into
+// LDS (mode 4).  A block that one workgroup reads is expanded no more often in mode 4, and the copies are a trip through memory:
+// they pay where they are few, where they let the keys be split, and where several workgroups read a block of many: two if the keys
+// are 512, three if mode 4 is not split itself, four if it is.  us per pass, copies / mode 4: 16/16 heads, 1 x 128 rows behind 128 tokens
+// 17.2 / 18.0, 16/8 16.3 / 17.6, 5 x 64 of 16/8 17.8 / 16.7; 40/8 heads (five readers), 5 x 64 behind 128 20.6 / 17.6, 256 24.9 / 22.3, 576 31.1 / 34.4,
+// 1024 37.9 / 50.7; 8 x 128 behind 256 34.4 / 32.5, 576 42.3 / 47.3; two row blocks, 8 x 128 of 16/8 behind 128 22.7 / 21.3, 8 x 256 of 16/16
+// behind 512 47.8 / 49.1; where mode 4 is split, 24/8 heads, 4 x 64 behind 576 30.2 / 27.8, 40/8, 5 x 64 behind 1984 56.6 / 62.9.
+// Not where mode 4 is split and a block is read by at most two workgroups (row blocks times head groups of a KV head):
+// 1 x 32 rows behind 512 tokens, 64 / 8 heads 23.1 / 18.8; 4 x 32 rows of 32 / 8 behind 1024 32.1 / 25.3, 4096 49.3 / 38.7; 8 x 128 of 16 / 16 behind
+// 4096 167 / 75.6; two row blocks: 4 x 64 of 32 / 8 behind 512 29.5 / 24.9, 8 x 256 of 16 / 16 behind 4096 195 / 128.  Four workgroups: 2 x 64 of
+// 64 / 8 behind 4096 49.5 / 55.6; three: 2 x 96 of 32 / 8 46.7 / 50.0.
 bool stream_expands(const PrefillArgs &a, int head_size, int64_t room) {
   if (!stream_serves(a, head_size)) return false;
   const int hpw = heads_per_workgroup(a), rows = kRowsPerWave * 4 / hpw;
-  const int64_t row_blocks = (a.sq + rows - 1) / rows;
-  const bool pays = row_blocks > 1 || a.batch * a.keys_bound * a.hkv <= 8192 || part_bytes(a, hpw, kStreamSplit, kD) > 0;
+  const int64_t row_blocks = (a.sq + rows - 1) / rows, readers = row_blocks * (a.hq / hpw / a.hkv);
   const int64_t parts = plain_part_bytes(a, kD, true);
-  return pays && !(parts > 0 && parts <= room && row_blocks * (a.hq / hpw / a.hkv) <= 2);
+  const bool splits = parts > 0 && parts <= room;
+  // (a table has room for more keys than the chunk's: 8192 rows of it)
+  const bool few = a.batch * a.keys_bound * a.hkv <= (a.keys_known ? 5120 : 8192);
+  const bool pays = (row_blocks > 1 && (readers > 2 || a.keys_bound >= 512)) || few || part_bytes(a, hpw, kStreamSplit, kD) > 0 || (readers > (splits ? 3 : 2) && a.keys_bound >= 512);
+  return pays && !(splits && readers <= 2);
 }
 
 int launch_stream_wide(const PrefillArgs &a, hipStream_t st) {
