@@ -131,22 +131,26 @@ def test_what_is_left_to_the_operators():
 
 
 def test_no_thread_takes_another_ones_scratch(monkeypatch):
-    """A step's kernels hand data through scratch, and the interpreter lock is not held between their launches: the native call
-    allocates its own, and the operators' kept one belongs to a thread."""
+    """A step's kernels hand data through scratch, and the interpreter lock is not held between their launches: what is kept
+    belongs to a thread, for the operators and for the native call."""
     import threading
 
     from tt_xla_amd import custom_ops as ops
 
-    here, there = [ops._workspace(1 << 20, torch.device("cuda")) for _ in range(2)], []
-    thread = threading.Thread(target=lambda: there.append(ops._workspace(1 << 20, torch.device("cuda"))))
+    kept, taken = ops._workspace, []
+    monkeypatch.setattr(ops, "_workspace", lambda *a: taken.append(kept(*a)) or taken[-1])
+
+    def step():
+        for native in (True, False):
+            p, impl = _pass(4, 16, 3, 1), _impl(16)
+            if not native:
+                impl._forward_native = lambda *a: False
+            impl.forward(p.q, p.lat, p.rope, p.cache, p.meta, p.layer, output=torch.zeros(3, 2048, dtype=torch.bfloat16, device="cuda"))
+        torch.cuda.synchronize()
+
+    step()
+    thread = threading.Thread(target=step)
     thread.start()
     thread.join()
-    assert here[0] is here[1] and there[0].data_ptr() != here[0].data_ptr()
-
-    def refuse(*_):
-        raise AssertionError("the pass took the operators' scratch")
-
-    monkeypatch.setattr(ops, "_workspace", refuse)
-    for s in (1, 64, 96):
-        p = _pass(4, 16, 3, s)
-        assert _impl(16)._forward_native(p.q, p.lat, p.rope, p.cache, p.meta, p.layer, torch.zeros(3 * s, 2048, dtype=torch.bfloat16, device="cuda"))
+    assert len(taken) == 4 and taken[0] is taken[1] and taken[2] is taken[3]
+    assert taken[0].data_ptr() != taken[2].data_ptr()

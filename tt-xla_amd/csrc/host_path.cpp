@@ -7,7 +7,8 @@
 // caches' layouts, int32 tables; nobody watching operators: no dispatch mode, function mode or trace); for anything else it answers None before it has issued anything, and the
 // caller's general path takes the pass, raises what is to be raised and converts what is to be
 // converted.  Scratch comes from the caching allocator on the current stream, call by call: nothing is kept
-// between calls, so streams, threads and graph captures need no care of their own.
+// between calls, so streams, threads and graph captures need no care of their own.  (A latent step takes the operators', which
+// belongs to the calling thread and to the default stream outside a capture.)
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/ATen.h>
@@ -235,13 +236,15 @@ const at::Tensor *weight(const Pass &p, PyObject *o, int64_t heads, int64_t rows
   return t;
 }
 
-// latent_pass(q_nope, q_rope, latent, rope, cache, page_table, cache_position, fill_page_table, w_uk_t, w_uv, output, heads, scale)
+// latent_pass(q_nope, q_rope, latent, rope, cache, page_table, cache_position, fill_page_table, w_uk_t, w_uv, output, heads, scale,
+//             workspace)
 // The pass of a latent layer (128 + 64 query features, latent width 512, values of 128; causal): decode step or prompt.
-// -> as attention_pass.
+// -> as attention_pass.  workspace(bytes, device) is the operators' own scratch of a decode step, a thread's (the interpreter lock
+// is not held between the launches that hand data through it) and sized for the largest grid, not for the pass.
 PyObject *latent_pass(PyObject *, PyObject *const *v, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 13) {
-    PyErr_SetString(PyExc_TypeError, "latent_pass takes 13 arguments");
+  if (n != 14) {
+    PyErr_SetString(PyExc_TypeError, "latent_pass takes 14 arguments");
     return nullptr;
   }
   if (c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled() ||
@@ -289,11 +292,19 @@ PyObject *latent_pass(PyObject *, PyObject *const *v, Py_ssize_t n) {
     if (!pt || pt->size(0) != users || pt->size(1) == 0 || !pos || users > 1024) Py_RETURN_NONE;
     const size_t bytes = ttpa_latent_decode_step_workspace_bytes((int32_t)users, (int32_t)heads);
     if (bytes == 0) Py_RETURN_NONE;
+    PyObject *const device = PyObject_GetAttrString(v[10], "device");
+    if (!device) return nullptr;
+    PyObject *const kept = PyObject_CallFunction(v[13], "nO", (Py_ssize_t)bytes, device);
+    Py_DECREF(device);
+    if (!kept) return nullptr;
+    const at::Tensor ws = THPVariable_Check(kept) ? THPVariable_Unpack(kept) : at::Tensor();
+    Py_DECREF(kept);
+    if (!ws.defined() || !ws.is_cuda() || ws.get_device() != p.device || ws.nbytes() < bytes) Py_RETURN_NONE;
     RECORD_FUNCTION("tt::latent_decode_step_", std::vector<c10::IValue>());
     written(cache), written(out);
     const auto launch = [&] {
       const Unlocked unlocked;
-      const at::Tensor ws = scratch((int64_t)bytes, out), target = storable ? *out : at::empty(out->sizes(), out->options());
+      const at::Tensor target = storable ? *out : at::empty(out->sizes(), out->options());
       const int rc = ttpa_latent_decode_step_strided(
           target.data_ptr(), heads * 128, 128, qn->data_ptr(), qn->stride(0), qn->stride(1), qr->data_ptr(), qr->stride(0), qr->stride(1),
           lat->data_ptr(), lat->stride(0), rope->data_ptr(), rope->stride(0), uk->data_ptr(), uk->stride(0), uk->stride(1), uk->stride(2),

@@ -37,7 +37,7 @@ from typing import List, Optional, Tuple
 import torch
 
 from . import _native
-from . import custom_ops  # noqa: F401  (registers torch.ops.tt.*)
+from . import custom_ops  # (registers torch.ops.tt.*)
 from .attention import TTAttentionMetadataBuilder, TTMetadata
 
 # the operator namespace, looked up once: host-logic tests substitute it
@@ -208,7 +208,7 @@ class TTMLAAttentionBackendImpl(_ImplBase):
             return False
         status = _native.latent_pass(
             q[0], q[1], kv_c_normed, k_pe, kv_cache, attn_metadata.page_table, attn_metadata.cache_position, attn_metadata.fill_page_table,
-            layer.W_UK_T, layer.W_UV, output, self.num_heads, self.scale)
+            layer.W_UK_T, layer.W_UV, output, self.num_heads, self.scale, custom_ops._workspace)
         if status is None:
             return False
         if status != 0:
