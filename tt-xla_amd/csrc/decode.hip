@@ -467,14 +467,14 @@ static int decode_impl(void *out, int64_t out_user_stride, int64_t out_head_stri
   hipStream_t st = static_cast<hipStream_t>(stream);
   // Kernel choice.  The VALU kernel spends per-head work on every tile; the matrix-core kernels
   // do not (their cost per tile does not depend on the group width).  Measured on bfloat16
-  // caches with head size 128: at 1 and 2 query heads per KV head the VALU kernel is 2 - 19 %
-  // faster (the larger figure on launches of a few tiles), at 4 the 16x16x32 kernel is 2 - 8 %
+  // caches with head size 128: at 4 query heads per KV head the 16x16x32 kernel is 2 - 8 %
   // faster, at 8 the VALU kernel is 2.5 times slower.  With head size 256 the VALU kernel streams
   // at 3.8 TB/s with one head per group and at 1.2 TB/s with eight, the 16x16x32 kernel at 5.3 -
   // 5.6 TB/s with any.  Head size 64 behaves like 128 (block size 32, 4 heads: 47.6 us on the
   // 16x16x32 kernel, 50.0 us on the VALU kernel; block size 64: 47.5 and 46.7).  So: 16x16x32
-  // kernel for head sizes 64 / 128 and 4 ... 16 heads per group and for head size 256 (up to 16
-  // heads), 32x32x16 kernel for wider groups (up to 32 heads), VALU kernel for the rest.  The block-float-8 cache goes to a matrix-core kernel
+  // kernel for 1 and 4 ... 16 heads per group, as a step for 2 and 3 too (below), and for head size 256 (up to 16
+  // heads), 32x32x16 kernel for wider groups (up to 32 heads), VALU kernel for the rest: the attention alone over 2 and 3 heads, and
+  // blocks that the others do not read.  The block-float-8 cache goes to a matrix-core kernel
   // whenever one applies: there the byte expansion costs one VALU operation per element and the
   // products none, while the VALU kernel pays for both.
   // TTPA_DECODE_KERNEL=valu|mfma|mfma16|ranges|direct overrides the choice (the last two: the 16x16x32 kernel on

@@ -49,7 +49,7 @@ struct DecodeArgs {
   int few_ranges = 0;  // > 0: lists of fewer than `many_from` tiles are cut into that many ranges instead of n_waves
   int64_t many_from = 0;
   int long_tiles = 0;  // 16x16x32 kernel, block-float-8 at head size 128: tiles of 64 tokens instead of 32
-  int direct = 0;  // wavefronts of the workgroup that owns a whole segment (16x16x32 kernel, fused step), or 0
+  int direct = 0;  // wavefronts of the workgroup that owns a whole segment (16x16x32 kernel: the step, or the attention alone), or 0
   // Additive mask on the scaled scores (bfloat16, natural-log units), or null: the element for
   // (user, query head, position) is mask[user * mask_us + head * mask_hs + position].  Applied by the
   // dot-product kernel (decode.hip) and by the workgroup-shared latent kernel (decode_wide.hip); the

@@ -1,5 +1,5 @@
 // Paged decode attention on the 16x16x32 matrix-core shape: up to 16 query heads per KV head,
-// 80 KiB of LDS per workgroup; head sizes 64, 128 and 256 with a block-float-8 cache (expanded
+// 32 or 64 KiB of tiles in LDS per workgroup of four wavefronts, and 16 KiB of tables; head sizes 64, 128 and 256 with a block-float-8 cache (expanded
 // to half precision) or a bfloat16 cache.
 //
 // Work decomposition, partial slots and merge kernel are those of decode.hip, with tiles of
