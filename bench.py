@@ -52,13 +52,13 @@ MEASURED_TRAFFIC = {
     # workload: (kernel, hash of its sources, HBM bytes per launch: FETCH_SIZE and WRITE_SIZE of the
     # kernel, each scaled by what the same counter reads for a plain copy of known size, mean over
     # the rotating workload copies; the summaries under profiles/ hold the runs)
-    "config2": ("paged_decode_mfma16_kernel", "4ce6db6ba974355a", 310434376),
-    "config5": ("paged_decode_mfma16_kernel", "4ce6db6ba974355a", 169705302),
-    "config4": ("paged_decode_mfma16_kernel", "4ce6db6ba974355a", 3415566290),
-    "config3": ("prefill_stream_kernel", "71eb60990b4e7f24", 244768677),
-    "latent": ("paged_decode_latent16_kernel", "c6436ec19a280f84", 654181074),
-    "latent128": ("paged_decode_latent128_kernel", "f15376b0d1795d27", 739370325),
-    "latent-prefill": ("latent_prefill_kernel", "f15376b0d1795d27", 332232245),
+    "config2": ("paged_decode_mfma16_kernel", "e55932f41ec0da21", 310416688),
+    "config5": ("paged_decode_mfma16_kernel", "e55932f41ec0da21", 169723672),
+    "config4": ("paged_decode_mfma16_kernel", "e55932f41ec0da21", 3415574623),
+    "config3": ("prefill_stream_kernel", "9100e82cd57f3c5b", 244747201),
+    "latent": ("paged_decode_latent16_kernel", "ce690ec22bd340ff", 654190843),
+    "latent128": ("paged_decode_latent128_kernel", "c74b75a4a905f438", 739359376),
+    "latent-prefill": ("latent_prefill_kernel", "c74b75a4a905f438", 332218599),
 }
 DECODE_KERNEL_NAME = {"config2": "paged_decode_mfma16_kernel", "config4": "paged_decode_mfma16_kernel",
                       "config5": "paged_decode_mfma16_kernel"}
