@@ -159,7 +159,10 @@ __device__ __forceinline__ void merge_waves(const DecodeArgs &a, int u, int h, i
 // DIRECT: a workgroup of DIRECT wavefronts owns the whole segment blockIdx.x (chosen by direct_waves, decode.hip): no prefix, no
 // search, no partials, no merge launch.  Its wavefronts take the segment's tiles in turn.  LONG: tiles of 16 KiB (a.long_tiles).
 template <int D, bool BFP8, int RUNS, bool FUSED, bool MASKED = false, int DIRECT = 0, bool LONG = false, bool ONE = false>
-__global__ __launch_bounds__(DIRECT ? kWave *DIRECT : 256, (DIRECT || BFP8) && D <= 128 && !LONG ? 2 : 1) void paged_decode_mfma16_kernel(
+// (Whole bfloat16 segments: no more than two wavefronts per SIMD, or the compiler saves registers for a third that has no segment: 37 users
+// of 64/8 heads of 64 in a window of 1024 22.0 / 21.8 us per layer.  Block-float-8 ones use the third: 100 users of 64/8 of 64 19.4 / 16.5.)
+__global__ __launch_bounds__(DIRECT ? kWave *DIRECT : 256) __attribute__((amdgpu_waves_per_eu((DIRECT || BFP8) && D <= 128 && !LONG ? 2 : 1, DIRECT && !BFP8 ? 2 : 8)))
+void paged_decode_mfma16_kernel(
     DecodeArgs a, const int32_t *__restrict__ page_table, const void *__restrict__ cur_pos) {
   static_assert(D == 64 || D == 128 || D == 256, "shapes built");
   constexpr int kTileBytes = tile_bytes<D, LONG>();
