@@ -52,9 +52,9 @@ MEASURED_TRAFFIC = {
     # workload: (kernel, hash of its sources, HBM bytes per launch: FETCH_SIZE and WRITE_SIZE of the
     # kernel, each scaled by what the same counter reads for a plain copy of known size, mean over
     # the rotating workload copies; the summaries under profiles/ hold the runs)
-    "config2": ("paged_decode_mfma16_kernel", "e55932f41ec0da21", 310416688),
-    "config5": ("paged_decode_mfma16_kernel", "e55932f41ec0da21", 169723672),
-    "config4": ("paged_decode_mfma16_kernel", "e55932f41ec0da21", 3415574623),
+    "config2": ("paged_decode_mfma16_kernel", "d1ad07dcf65d7c97", 310416888),
+    "config5": ("paged_decode_mfma16_kernel", "d1ad07dcf65d7c97", 169724320),
+    "config4": ("paged_decode_mfma16_kernel", "d1ad07dcf65d7c97", 3415572133),
     "config3": ("prefill_stream_kernel", "9100e82cd57f3c5b", 244747201),
     "latent": ("paged_decode_latent16_kernel", "ce690ec22bd340ff", 654190843),
     "latent128": ("paged_decode_latent128_kernel", "c74b75a4a905f438", 739359376),
