@@ -250,3 +250,17 @@ def test_narrow_block_table_is_zero_padded():
     plan = b.prepare(_table(2, width=5), [0, 0], [1, 1])
     assert torch.equal(plan.metadata.page_table[:, :5], torch.from_numpy(_table(2, width=5)))
     assert not plan.metadata.page_table[:, 5:].any()
+
+
+@pytest.mark.parametrize("computed,scheduled,want", [
+    ([0, 0], [64, 40], None),        # a first chunk attends its own keys
+    ([96, 96], [1, 1], None),        # a decode step
+    ([96, 96], [64, 40], 96 + 64),   # behind the last row of the padded chunk
+    ([0, 512], [0, 33], 512 + 64),   # a parked row
+])
+def test_chunk_end_is_where_the_padded_chunk_ends(computed, scheduled, want):
+    builder = M.PagedMetadataBuilder(32, 64, 128)
+    table = np.arange(1, 129, dtype=np.int32).reshape(2, 64)
+    plan = builder.prepare(table, np.array(computed), np.array(scheduled))
+    assert plan.metadata.chunk_end == want
+    assert (plan.metadata.chunk_start_idx is None) == (want is None)
