@@ -1,14 +1,15 @@
 #!/usr/bin/env python3
-"""Writes the hand-scheduled loop of the streaming prefill kernel (head size 128, 32 query rows of one
-head per wavefront, two workgroups of four wavefronts per CU) as one block of gfx950 assembly per
-form of the loop: build/prefill_stream_asm.h, included by prefill_stream.hip.  The forms: dense
-K / V, dense with a sliding window, dense with keys of 128 + 64 features (the second part, the rotary
-one, with base and strides of its own), paged K / V in cache blocks of whole 64-key tiles, and in
-cache blocks of whole 32-key blocks.
+"""Writes the hand-scheduled loop of the streaming prefill kernel (32 query rows of one
+head per wavefront, workgroups of four wavefronts) as one block of gfx950 assembly per head size and
+form of the loop: build/prefill_stream_asm.h, included by prefill_stream_kernel.h.  Head sizes 64 (three
+workgroups per CU), 128 (two) and 256 (one: its 128 accumulators are accumulation registers).  The forms: dense
+K / V, dense with a sliding window, paged K / V in cache blocks of whole 64-key tiles, and in
+cache blocks of whole 32-key blocks; at 128 also dense with keys of 128 + 64 features (the second part, the rotary
+one, with base and strides of its own).  The numbers below are those of head size 128; at d, S(i) is d / 16
+matrix instructions, PV(i) d / 16, a block 64 d bytes.
 
 Why assembly: the loop wants the matrix pipe and the vector ALU of a SIMD busy at the same time
-from one instruction stream, with every register chosen by hand (256 per wavefront at two
-wavefronts per SIMD) and every wait counted.  The unit of work is a BLOCK of 32 keys:
+from one instruction stream, with every register chosen by hand (`Registers`) and every wait counted.  The unit of work is a BLOCK of 32 keys:
 
   S(i)   8 matrix instructions   S^T = K . Q^T of block i          (K fragments from LDS)
   sm(i)  ~56 vector instructions  p = exp2(s c - m), packed to bfloat16, row sum
@@ -38,7 +39,8 @@ the scores: 16 compares of the key constants against limit - 4 h - key0 and 16 s
 Blocks in front of it skip that with one scalar branch.  With a sliding window a lane also has a
 lowest key; blocks whose first key is below `low_to` are masked from below in the same way.
 
-LDS: a ring of NS slots of 8 KiB (32 rows) for K blocks and one for V blocks; block j lives in
+LDS: a ring of NS slots of 8 KiB (32 rows) for K blocks and one for V blocks (NS = 5; 4 at head size 256, whose five
+would be past what an LDS instruction's offset reaches); block j lives in
 slot j % NS.  Iteration i reads K block i + 1 and V block i - 1 and, through the running fragment
 reads, the first fragments of K block i + 2 and V block i.  Its barrier, at its start, says that
 nobody reads K block i and V block i - 2 any more; K block i + NS and V block i + NS - 2 are
@@ -82,34 +84,53 @@ it (the mask waits explicitly); a bank of probabilities is rewritten three matri
 after the last one that read it; the slow path and the exit wait out the matrix pipe with s_nop.
 """
 
+import re
 import sys
 
 
-# ---- register map (vector registers) ---------------------------------------------------------
-ACC = [0, 16, 32, 48]          # output accumulators, head-dim blocks 0..3 (inputs / outputs)
-QF = 64                        # Q fragments, k-step ks at QF + 4 ks (inputs)
-S = [96, 112]                  # score banks
-P = [128, 136]                 # probability banks (8 packed pairs each)
-RING = 144                     # 8 fragment slots of 4 registers
+# ---- vector registers ---------------------------------------------------------------------------
+class Registers:
+    """The vector register map of a head size; what is an operand of the block says `operands`."""
+
+    def __init__(self, d, wide):
+        self.acc_file = "a" if d == 256 else "v"   # file of the output accumulators
+        at = 0
+
+        def take(n):
+            nonlocal at
+            at += n
+            return at - n
+
+        # output accumulators, head-dim blocks 0 .. d / 32 - 1
+        self.ACC = [16 * db for db in range(d // 32)] if d == 256 else [take(16) for _ in range(d // 32)]
+        self.QF = take(d // 4)                     # Q fragments, k-step ks at QF + 4 ks
+        self.S = [take(16), take(16)]              # score banks (these, P and RING in one piece: the epilogue's packed rows)
+        self.P = [take(8), take(8)]                # probability banks (packed pairs)
+        self.RING = take(4 * NSLOT)                # fragment slots of 4 registers
+        self.KOFF = take(d // 16)                  # LDS byte address of the lane's K fragment in K slot 0, k-step ks
+        self.VOFF = take(d // 32)                  # ... of the lane's V^T fragment in V slot 0, output block db
+        self.LDK = take(d // 64)                   # per-lane global byte offsets of the K loads of a block
+        self.LDV = take(d // 64)                   # ... of the V loads
+        if d == 128:
+            at = 196
+        self.MC, self.LRUN, self.LSUM, self.ALPHA = (take(1) for _ in range(4))
+        self.T = [take(1) for _ in range(4)]
+        self.ORV, self.MLOC, self.MB, self.MCN = (take(1) for _ in range(4))
+        self.PTREQ = take(1)                       # paged: the requested block-table entry
+        self.LOWEST, self.LOWREL = take(1), take(1)  # window: first visible key of the lane's row, minus 4 h; relative to the block
+        self.PTREQ2 = take(1)                      # blocks of 32: the entry requested in odd iterations
+        self.LIMIT = take(1)                       # last visible key of the lane's row, minus 4 h
+        self.LIMREL, self.NEGINF, self.VZERO = (take(1) for _ in range(3))
+        self.QBASE, self.OUTBASE = take(2), take(2)  # per lane, 64-bit: q / out of row 0 of the lane's head, at the lane's 8 h elements
+        self.VN, self.V4H = take(1), take(1)       # lane % 32 and 4 (lane / 32)
+        self.OUTP, self.PTMP = take(2), take(2)
+        self.VT0, self.VROW = take(1), take(1)
+        if wide:                                   # keys of 128 + 64: Q fragments, LDS addresses and global offsets of the second part
+            self.QFP, self.KOFFP, self.LDKP = take(16), take(4), take(1)
+        self.count = at
+
+
 NSLOT = 8
-KOFF = 176                     # LDS byte address of the lane's K fragment in K slot 0, k-step ks (inputs)
-VOFF = 184                     # ... of the lane's V^T fragment in V slot 0, output block db (inputs)
-LDK = 188                      # per-lane global byte offsets of the 2 K loads of a block (inputs)
-LDV = 190                      # ... of the 2 V loads
-MC, LRUN, LSUM, ALPHA = 196, 197, 198, 199   # MC, LRUN: inputs / outputs
-T = [200, 201, 202, 203]
-ORV, MLOC, MB, MCN = 204, 205, 206, 207
-PTREQ = 208                    # paged: the requested block-table entry (input)
-PTREQ2 = 211                   # blocks of 32: the entry requested in odd iterations (input)
-LOWEST, LOWREL = 209, 210      # window: first visible key of the lane's row, minus 4 h (input); relative to the block
-LIMIT = 212                    # last visible key of the lane's row, minus 4 h (input)
-LIMREL, NEGINF, VZERO = 213, 214, 215
-QBASE, OUTBASE = 216, 218      # per lane, 64-bit: q / out of row 0 of the lane's head, at the lane's 8 h / 4 h elements (inputs)
-VN, V4H = 220, 221             # lane % 32 and 4 (lane / 32) (inputs)
-QFP, KOFFP, LDKP = 228, 244, 248  # keys of 128 + 64: Q fragments, LDS addresses and global offsets of the second part (inputs)
-OUTP, PTMP, VT0, VROW = 222, 224, 226, 227
-CLOBBERED = (list(range(0, QF)) + list(range(S[0], RING + 4 * NSLOT)) + list(range(MC, MCN + 1)) + [LOWREL, LIMIT, LIMREL, NEGINF, VZERO]
-             + list(range(OUTP, VROW + 1)))
 
 # ---- scalar registers ---------------------------------------------------------------------------
 S_KBASE = "s[64:65]"           # dense: next K block to request; paged: the K cache (both minus 1024, see dma)
@@ -146,29 +167,33 @@ S_QTS, S_OTS = "s48", "s49"    # bytes from a query / output row to the next
 S_ROW0 = "s57"                 # first query row of the item
 S_STOREMASK = "s[60:61]"
 # temporaries s[88:95], s[62:63]
-SCALAR_CLOBBERS = [f"s{r}" for r in list(range(88, 96)) + [60, 61, 62, 63, 74]]
 
-SLOT, PSLOT = 8192, 4096       # bytes of a block of K or V, of the second part of K
+PSLOT = 4096                   # bytes of a block of the second part of K
 KEY_CONST = [8 * (r // 4) + r % 4 for r in range(16)]
 
 
 class Form:
     """What one block of assembly serves."""
 
-    def __init__(self, name, paged=0, window=False, wide=False):
-        self.name, self.paged, self.window = name, paged, window  # paged: 0 or the keys that share a table entry
+    def __init__(self, name, d=128, paged=0, window=False, wide=False):
+        self.name, self.d = f"{name}_{d}", d
+        self.paged, self.window = paged, window  # paged: 0 or the keys that share a table entry
         self.wide = wide                    # keys of 128 + 64 features
-        self.ns = 4 if wide else 5          # slots per ring
-        self.unroll = 4 if wide else 10     # lcm(2, ns): score bank and slots repeat
-        self.vring = self.ns * SLOT         # LDS offset of the V ring (VOFF carries it), of the second part's ring (KOFFP)
+        self.ns = 4 if wide or d == 256 else 5  # slots per ring
+        self.unroll = 4 if self.ns == 4 else 10  # lcm(2, ns): score bank and slots repeat
+        self.SLOT = 64 * d                  # bytes of a block of K or V
+        self.tensor_loads = d // 64         # loads per wavefront of a block of K or V
+        self.__dict__.update(vars(Registers(d, wide)))
+        self.vring = self.ns * self.SLOT    # LDS offset of the V ring (VOFF carries it), of the second part's ring (KOFFP)
         self.pring = 2 * self.vring
-        self.loads = 5 if wide else 4       # tile loads of an iteration
-        self.items = not window and not wide and paged != 32  # several row blocks in turn
+        self.loads = 2 * self.tensor_loads + wide  # tile loads of an iteration
+        self.items = d == 128 and not window and not wide and paged != 32  # several row blocks in turn
         self.parts = paged > 0  # may take a part of the keys
 
 
-FORMS = [Form("DENSE"), Form("DENSE_WINDOW", window=True), Form("DENSE_WIDE", wide=True), Form("PAGED", paged=64),
-         Form("PAGED32", paged=32)]
+FORMS = [Form("DENSE_WIDE", wide=True)] + [
+    form for d in (64, 128, 256)
+    for form in (Form("DENSE", d), Form("DENSE_WINDOW", d, window=True), Form("PAGED", d, paged=64), Form("PAGED32", d, paged=32))]
 START_REFERENCE = "0xff7fffff"  # the lowest finite float
 
 
@@ -183,46 +208,46 @@ class Out:
         self.lines.append(name + "%=:")
 
 
-def vr(a, n=1):
-    return f"v{a}" if n == 1 else f"v[{a}:{a + n - 1}]"
+def vr(a, n=1, file="v"):
+    return f"{file}{a}" if n == 1 else f"{file}[{a}:{a + n - 1}]"
 
 
-def frag_reads(frag, slot):
+def frag_reads(f, frag, slot):
     """LDS read instructions of a fragment into ring slot `slot`.
     ("K", LDS slot, k-step) or ("V", LDS slot, key step 0 / 1, output block)."""
-    base = RING + 4 * slot
-    if frag[0] == "K" and frag[2] >= 8:
-        return [f"ds_read_b128 {vr(base, 4)}, v{KOFFP + frag[2] - 8} offset:{frag[1] * PSLOT}"]
+    base = f.RING + 4 * slot
+    if frag[0] == "K" and frag[2] >= f.d // 16:
+        return [f"ds_read_b128 {vr(base, 4)}, v{f.KOFFP + frag[2] - f.d // 16} offset:{frag[1] * PSLOT}"]
     if frag[0] == "K":
         _, ls, ks = frag
-        return [f"ds_read_b128 {vr(base, 4)}, v{KOFF + ks} offset:{ls * SLOT}"]
+        return [f"ds_read_b128 {vr(base, 4)}, v{f.KOFF + ks} offset:{ls * f.SLOT}"]
     _, ls, k4, db = frag
-    off = ls * SLOT + k4 * 4096
-    return [f"ds_read_b64_tr_b16 {vr(base, 2)}, v{VOFF + db} offset:{off}",
-            f"ds_read_b64_tr_b16 {vr(base + 2, 2)}, v{VOFF + db} offset:{off + 2048}"]
+    off = ls * f.SLOT + k4 * f.SLOT // 2
+    return [f"ds_read_b64_tr_b16 {vr(base, 2)}, v{f.VOFF + db} offset:{off}",
+            f"ds_read_b64_tr_b16 {vr(base + 2, 2)}, v{f.VOFF + db} offset:{off + f.SLOT // 4}"]
 
 
-def mfma(m, slot):
-    a = vr(RING + 4 * slot, 4)
+def mfma(f, m, slot):
+    a = vr(f.RING + 4 * slot, 4)
     if m[0] == "S":
         _, bank, ks = m
-        d = vr(S[bank], 16)
-        q = QF + 4 * ks if ks < 8 else QFP + 4 * (ks - 8)
+        d = vr(f.S[bank], 16)
+        q = f.QF + 4 * ks if ks < f.d // 16 else f.QFP + 4 * (ks - f.d // 16)
         return f"v_mfma_f32_32x32x16_bf16 {d}, {a}, {vr(q, 4)}, {'0' if ks == 0 else d}"
     _, db, bank, k4p = m
-    d = vr(ACC[db], 16)
-    return f"v_mfma_f32_32x32x16_bf16 {d}, {a}, {vr(P[bank] + 4 * k4p, 4)}, {d}"
+    d = vr(f.ACC[db], 16, f.acc_file)
+    return f"v_mfma_f32_32x32x16_bf16 {d}, {a}, {vr(f.P[bank] + 4 * k4p, 4)}, {d}"
 
 
-def softmax_ops(q, test=True):
+def softmax_ops(f, q, test=True):
     """Vector instructions of sm(i) on bank q, in an order that keeps one instruction between a
     transcendental and its first use."""
-    s, p = S[q], P[q]
-    A = lambda r: f"v_fma_f32 v{T[r % 4]}, v{s + r}, {S_C}, -v{MC}"
-    B = lambda r: f"v_exp_f32 v{T[r % 4]}, v{T[r % 4]}"
-    C = lambda j: f"v_cvt_pk_bf16_f32 v{p + j}, v{T[(2 * j) % 4]}, v{T[(2 * j + 1) % 4]}"
-    D = lambda j: f"v_dot2c_f32_bf16 v{LSUM}, 0x3f803f80, v{p + j}"
-    ops = [f"v_mov_b32 v{LSUM}, 0", A(0), A(1), B(0), B(1)]
+    s, p = f.S[q], f.P[q]
+    A = lambda r: f"v_fma_f32 v{f.T[r % 4]}, v{s + r}, {S_C}, -v{f.MC}"
+    B = lambda r: f"v_exp_f32 v{f.T[r % 4]}, v{f.T[r % 4]}"
+    C = lambda j: f"v_cvt_pk_bf16_f32 v{p + j}, v{f.T[(2 * j) % 4]}, v{f.T[(2 * j + 1) % 4]}"
+    D = lambda j: f"v_dot2c_f32_bf16 v{f.LSUM}, 0x3f803f80, v{p + j}"
+    ops = [f"v_mov_b32 v{f.LSUM}, 0", A(0), A(1), B(0), B(1)]
     for j in range(8):
         if j < 7:
             ops += [A(2 * j + 2), A(2 * j + 3)]
@@ -231,12 +256,12 @@ def softmax_ops(q, test=True):
             ops += [B(2 * j + 2), B(2 * j + 3)]
         ops.append(D(j))
     if test:
-        ops += [f"v_or3_b32 v{ORV}, v{p}, v{p + 1}, v{p + 2}",
-                f"v_or3_b32 v{ORV}, v{ORV}, v{p + 3}, v{p + 4}",
-                f"v_or3_b32 v{ORV}, v{ORV}, v{p + 5}, v{p + 6}",
-                f"v_or_b32 v{ORV}, v{ORV}, v{p + 7}",
-                f"v_and_b32 v{ORV}, 0x40004000, v{ORV}",
-                f"v_cmp_ne_u32 vcc, 0, v{ORV}"]
+        ops += [f"v_or3_b32 v{f.ORV}, v{p}, v{p + 1}, v{p + 2}",
+                f"v_or3_b32 v{f.ORV}, v{f.ORV}, v{p + 3}, v{p + 4}",
+                f"v_or3_b32 v{f.ORV}, v{f.ORV}, v{p + 5}, v{p + 6}",
+                f"v_or_b32 v{f.ORV}, v{f.ORV}, v{p + 7}",
+                f"v_and_b32 v{f.ORV}, 0x40004000, v{f.ORV}",
+                f"v_cmp_ne_u32 vcc, 0, v{f.ORV}"]
     for i, op in enumerate(ops[:-1]):  # a transcendental's result is not read by the next instruction
         if op.startswith("v_exp_f32"):
             dst = op.split()[1].rstrip(",")
@@ -253,7 +278,7 @@ def spread(ops, nslots, first=0):
     return out
 
 
-def stream(o, pairs, valu_chunks, phase, in_flight, tail):
+def stream(o, f, pairs, valu_chunks, phase, in_flight, tail):
     """pairs: [(matrix instruction, fragment)].  Per pair: wait for its fragment, the matrix
     instruction, the read of the fragment NSLOT pairs on, the vector chunk.  phase: the ring slot of the
     first pair's fragment; in_flight: the first NSLOT fragments have been requested by the code in front
@@ -261,18 +286,18 @@ def stream(o, pairs, valu_chunks, phase, in_flight, tail):
     iteration's first ones).  Returns the next phase."""
     frags = [f for _, f in pairs] + list(tail)
     n = len(pairs)
-    count = lambda f: len(frag_reads(frags[f], 0))
+    count = lambda k: len(frag_reads(f, frags[k], 0))
     if not in_flight:
-        for f in range(min(NSLOT, len(frags))):
-            for x in frag_reads(frags[f], (phase + f) % NSLOT):
+        for k in range(min(NSLOT, len(frags))):
+            for x in frag_reads(f, frags[k], (phase + k) % NSLOT):
                 o.e(x)
     for j in range(n):
-        after = sum(count(f) for f in range(j + 1, min(j + NSLOT, len(frags))))
+        after = sum(count(k) for k in range(j + 1, min(j + NSLOT, len(frags))))
         assert after <= 15
         o.e(f"s_waitcnt lgkmcnt({after})")
-        o.e(mfma(pairs[j][0], (phase + j) % NSLOT))
+        o.e(mfma(f, pairs[j][0], (phase + j) % NSLOT))
         if j + NSLOT < len(frags):
-            for x in frag_reads(frags[j + NSLOT], (phase + j) % NSLOT):
+            for x in frag_reads(f, frags[j + NSLOT], (phase + j) % NSLOT):
                 o.e(x)
         for x in valu_chunks[j]:
             o.e(x)
@@ -280,7 +305,7 @@ def stream(o, pairs, valu_chunks, phase, in_flight, tail):
 
 
 def score_pairs(bank, slot, f):
-    return [(("S", bank, x), ("K", slot, x)) for x in range(12 if f.wide else 8)]
+    return [(("S", bank, x), ("K", slot, x)) for x in range(f.d // 16 + 4 * f.wide)]
 
 
 def iteration_pairs(p, f, has_pv=True):
@@ -290,23 +315,24 @@ def iteration_pairs(p, f, has_pv=True):
     scores = score_pairs(1 - q, (p + 1) % f.ns, f)
     if not has_pv:
         return scores
-    pv = [(("PV", x % 4, 1 - q, x // 4), ("V", (p - 1) % f.ns, x // 4, x % 4)) for x in range(8)]
-    order = "SPSSPSPSSPSPSSPSPSSP" if f.wide else "SP" * 8
-    assert order.count("S") == len(scores) and order.count("P") == 8
+    db = f.d // 32
+    pv = [(("PV", x % db, 1 - q, x // db), ("V", (p - 1) % f.ns, x // db, x % db)) for x in range(2 * db)]
+    order = "SPSSPSPSSPSPSSPSPSSP" if f.wide else "SP" * len(pv)
+    assert order.count("S") == len(scores) and order.count("P") == len(pv)
     scores, pv = iter(scores), iter(pv)
     return [next(scores if x == "S" else pv) for x in order]
 
 
 def mask_selects(o, f, bank):
     """-inf in place of the scores of the block at S_KEY0 that a lane may not see; the bank has been written."""
-    s = S[bank]
-    o.e(f"v_subrev_u32 v{LIMREL}, {S_KEY0}, v{LIMIT}")  # limit - 4 h - key0
-    o.e(f"v_mov_b32 v{NEGINF}, 0xff800000")
-    sel = lambda r: f"v_cndmask_b32_e64 v{s + r}, v{s + r}, v{NEGINF}, s[{88 + 2 * (r % 4)}:{89 + 2 * (r % 4)}]"
-    sides = [("v_cmp_gt_i32_e64", LIMREL)]
+    s = f.S[bank]
+    o.e(f"v_subrev_u32 v{f.LIMREL}, {S_KEY0}, v{f.LIMIT}")  # limit - 4 h - key0
+    o.e(f"v_mov_b32 v{f.NEGINF}, 0xff800000")
+    sel = lambda r: f"v_cndmask_b32_e64 v{s + r}, v{s + r}, v{f.NEGINF}, s[{88 + 2 * (r % 4)}:{89 + 2 * (r % 4)}]"
+    sides = [("v_cmp_gt_i32_e64", f.LIMREL)]
     if f.window:
-        o.e(f"v_subrev_u32 v{LOWREL}, {S_KEY0}, v{LOWEST}")
-        sides.append(("v_cmp_lt_i32_e64", LOWREL))
+        o.e(f"v_subrev_u32 v{f.LOWREL}, {S_KEY0}, v{f.LOWEST}")
+        sides.append(("v_cmp_lt_i32_e64", f.LOWREL))
     for compare, bound in sides:
         for r in range(16):
             o.e(f"{compare} s[{88 + 2 * (r % 4)}:{89 + 2 * (r % 4)}], {KEY_CONST[r]}, v{bound}")
@@ -337,6 +363,22 @@ def mask_block(o, f, q, tag):
     o.e(f"s_add_u32 {S_KEY0}, {S_KEY0}, 32")
 
 
+def accumulators(f):
+    return range(f.ACC[0], f.ACC[0] + f.d // 2)
+
+
+def scale_accumulators(o, f):
+    """All of them by ALPHA."""
+    for r in accumulators(f):
+        if f.acc_file == "v":
+            o.e(f"v_mul_f32 v{r}, v{f.ALPHA}, v{r}")
+        else:  # (accumulation registers are the matrix instructions': a round trip through four registers in turn)
+            t = f.T[r % 4]
+            o.e(f"v_accvgpr_read_b32 v{t}, a{r}")
+            o.e(f"v_mul_f32 v{t}, v{f.ALPHA}, v{t}")
+            o.e(f"v_accvgpr_write_b32 a{r}, v{t}")
+
+
 def slow_path(o, f, q, name, join, first=False):
     """Bank q: true row maximum, new reference, rescale, probabilities again.  The scores of the next block are there
     already (bank 1 - q, S_KEY0 is its first key): the maximum is taken over both.  The weight that equals the
@@ -347,12 +389,12 @@ def slow_path(o, f, q, name, join, first=False):
     7.59 this way."""
     def row_max(bank, regs):
         for r in regs:
-            o.e(f"v_max3_f32 v{MLOC}, v{MLOC}, v{S[bank] + r}, v{S[bank] + r + 1}")
+            o.e(f"v_max3_f32 v{f.MLOC}, v{f.MLOC}, v{f.S[bank] + r}, v{f.S[bank] + r + 1}")
 
     o.label(name)
     o.e("s_nop 15")
     o.e("s_nop 15")
-    o.e(f"v_max_f32 v{MLOC}, v{S[q]}, v{S[q] + 1}")
+    o.e(f"v_max_f32 v{f.MLOC}, v{f.S[q]}, v{f.S[q] + 1}")
     row_max(q, range(2, 16, 2))
     o.e(f"s_cmp_lt_u32 {S_NB}, 2")              # no next block: its bank holds products of whatever the slot held
     o.e(f"s_cbranch_scc1 L_one_{name}%=")
@@ -361,38 +403,37 @@ def slow_path(o, f, q, name, join, first=False):
     o.label(f"L_nomask_{name}")
     row_max(1 - q, range(0, 16, 2))
     o.label(f"L_one_{name}")
-    o.e(f"v_mov_b32 v{MB}, v{MLOC}")
+    o.e(f"v_mov_b32 v{f.MB}, v{f.MLOC}")
     o.e("s_nop 1")
-    o.e(f"v_permlane32_swap_b32 v{MLOC}, v{MB}")
+    o.e(f"v_permlane32_swap_b32 v{f.MLOC}, v{f.MB}")
     o.e("s_nop 1")
-    o.e(f"v_max_f32 v{MLOC}, v{MLOC}, v{MB}")                 # row maximum (raw score)
-    o.e(f"v_fma_f32 v{MB}, v{MLOC}, {S_C}, -v{MC}")           # how far above the reference's zero
-    o.e(f"v_cmp_le_f32 vcc, 1.0, v{MB}")                      # p >= 2 somewhere in the row: move
-    o.e(f"v_mul_f32 v{MCN}, {S_C}, v{MLOC}")
-    o.e(f"v_add_f32 v{MCN}, 0x40e00000, v{MCN}")              # m c + 7
+    o.e(f"v_max_f32 v{f.MLOC}, v{f.MLOC}, v{f.MB}")                 # row maximum (raw score)
+    o.e(f"v_fma_f32 v{f.MB}, v{f.MLOC}, {S_C}, -v{f.MC}")           # how far above the reference's zero
+    o.e(f"v_cmp_le_f32 vcc, 1.0, v{f.MB}")                      # p >= 2 somewhere in the row: move
+    o.e(f"v_mul_f32 v{f.MCN}, {S_C}, v{f.MLOC}")
+    o.e(f"v_add_f32 v{f.MCN}, 0x40e00000, v{f.MCN}")              # m c + 7
     o.e("s_nop 1")
-    o.e(f"v_cndmask_b32 v{MCN}, v{MC}, v{MCN}, vcc")
+    o.e(f"v_cndmask_b32 v{f.MCN}, v{f.MC}, v{f.MCN}, vcc")
     if first:  # nothing is accumulated yet: no rescale
-        o.e(f"v_mov_b32 v{MC}, v{MCN}")
+        o.e(f"v_mov_b32 v{f.MC}, v{f.MCN}")
     else:
-        o.e(f"v_sub_f32 v{ALPHA}, v{MC}, v{MCN}")             # 0 where the reference stays
-        o.e(f"v_exp_f32 v{ALPHA}, v{ALPHA}")
-        o.e(f"v_mov_b32 v{MC}, v{MCN}")
+        o.e(f"v_sub_f32 v{f.ALPHA}, v{f.MC}, v{f.MCN}")             # 0 where the reference stays
+        o.e(f"v_exp_f32 v{f.ALPHA}, v{f.ALPHA}")
+        o.e(f"v_mov_b32 v{f.MC}, v{f.MCN}")
         o.e("s_nop 0")
-        o.e(f"v_mul_f32 v{LRUN}, v{LRUN}, v{ALPHA}")
-        for r in range(64):
-            o.e(f"v_mul_f32 v{r}, v{ALPHA}, v{r}")
-    for x in softmax_ops(q, test=False):
+        o.e(f"v_mul_f32 v{f.LRUN}, v{f.LRUN}, v{f.ALPHA}")
+        scale_accumulators(o, f)
+    for x in softmax_ops(f, q, test=False):
         o.e(x)
     o.e("s_nop 4")
     o.e(f"s_branch {join}%=")
 
 
-def two_loads(o, lane_regs, base):
+def block_loads(o, f, lane_regs, base):
     """The instruction offset moves the LDS address as well as the global one: load j lands 1024 j
     bytes behind M0 and reads base + lane offset + 1024 j, so the lane offsets carry
     1024 - 1024 j and the bases - 1024."""
-    for j in range(2):
+    for j in range(f.tensor_loads):
         o.e(f"global_load_lds_dwordx4 v{lane_regs + j}, {base} offset:{1024 * j}")
 
 
@@ -400,7 +441,7 @@ def request_block(o, f, which, slot, tag, half):
     """One K or V block into LDS slot `slot` of its ring, if there is one left to request.
     paged: the block is half `half` of the tile at S_OFFK / S_OFFV."""
     paged = f.paged
-    left, lane, base, ring = (S_KLEFT, LDK, S_KBASE, 0) if which == "K" else (S_VLEFT, LDV, S_VBASE, f.vring)
+    left, lane, base, ring = (S_KLEFT, f.LDK, S_KBASE, 0) if which == "K" else (S_VLEFT, f.LDV, S_VBASE, f.vring)
     o.e(f"s_cmp_eq_u32 {left}, 0")
     o.e(f"s_cbranch_scc1 L_no{which}_{tag}%=")
     if paged:
@@ -409,11 +450,11 @@ def request_block(o, f, which, slot, tag, half):
         o.e(f"s_add_u32 s90, s{b0}, s{lo}")
         o.e(f"s_addc_u32 s91, s{b0 + 1}, s{hi}")
         if half:
-            o.e(f"s_add_u32 s90, s90, {SLOT}")
+            o.e(f"s_add_u32 s90, s90, {f.SLOT}")
             o.e("s_addc_u32 s91, s91, 0")
-    o.e(f"s_add_u32 m0, {S_M0B}, {ring + slot * SLOT}")
+    o.e(f"s_add_u32 m0, {S_M0B}, {ring + slot * f.SLOT}")
     o.e("s_nop 0")
-    two_loads(o, lane, "s[90:91]" if paged else base)
+    block_loads(o, f, lane, "s[90:91]" if paged else base)
     if not paged:
         b0 = int(base[2:4])
         o.e(f"s_add_u32 s{b0}, s{b0}, {S_VSTRIDE if f.wide and which == 'V' else S_STRIDE}")
@@ -421,25 +462,25 @@ def request_block(o, f, which, slot, tag, half):
     if f.wide and which == "K":
         o.e(f"s_add_u32 m0, {S_M0P}, {slot * PSLOT}")
         o.e("s_nop 0")
-        o.e(f"global_load_lds_dwordx4 v{LDKP}, {S_PBASE}")
+        o.e(f"global_load_lds_dwordx4 v{f.LDKP}, {S_PBASE}")
         o.e(f"s_add_u32 s30, s30, {S_PSTRIDE}")
         o.e("s_addc_u32 s31, s31, 0")
     o.e(f"s_sub_u32 {left}, {left}, 1")
     o.label(f"L_no{which}_{tag}")
 
 
-def next_tile(o, tag):
+def next_tile(o, f, tag):
     """paged, odd iterations: V moves on to the tile K was in, K to the tile whose entry has
     arrived; the entry after that is requested."""
     o.e("s_mov_b64 s[84:85], s[86:87]")
-    o.e(f"v_readfirstlane_b32 s88, v{PTREQ}")
+    o.e(f"v_readfirstlane_b32 s88, v{f.PTREQ}")
     o.e(f"s_cmp_lt_u32 s88, {S_NCB}")
     o.e("s_cselect_b32 s88, s88, 0")
     o.e(f"s_mul_i32 s88, s88, {S_HKV}")
     o.e(f"s_add_u32 s90, s88, {S_HK}")            # cache block * kv_heads + kv_head
     o.e(f"s_mul_hi_u32 s87, s90, {S_STRIDE}")
     o.e(f"s_mul_i32 s86, s90, {S_STRIDE}")
-    o.e(f"s_lshl_b32 s90, {S_CIN}, 14")           # 64 tokens of 256 bytes per tile inside the cache block
+    o.e(f"s_lshl_b32 s90, {S_CIN}, {f.SLOT.bit_length()}")  # 64 tokens per tile inside the cache block
     o.e("s_add_u32 s86, s86, s90")
     o.e("s_addc_u32 s87, s87, 0")
     o.e(f"s_add_u32 {S_CIN}, {S_CIN}, 1")
@@ -447,7 +488,7 @@ def next_tile(o, tag):
     o.e(f"s_cselect_b32 {S_CIN}, 0, {S_CIN}")
     o.e(f"s_cmp_eq_u32 {S_RLEFT}, 0")
     o.e(f"s_cbranch_scc1 L_noreq_{tag}%=")
-    o.e(f"global_load_dword v{PTREQ}, v{VZERO}, {S_RPTR}")
+    o.e(f"global_load_dword v{f.PTREQ}, v{f.VZERO}, {S_RPTR}")
     o.e(f"s_sub_u32 {S_RLEFT}, {S_RLEFT}, 1")
     o.e(f"s_add_u32 {S_RIN}, {S_RIN}, 1")
     o.e(f"s_cmp_lg_u32 {S_RIN}, {S_TPB}")
@@ -458,10 +499,10 @@ def next_tile(o, tag):
     o.label(f"L_noreq_{tag}")
 
 
-def next_block(o, p, tag):
+def next_block(o, f, p, tag):
     """Blocks of 32, every iteration: the byte offset of the K block from its table entry; the entry of
     the K block two iterations on is requested."""
-    req = PTREQ2 if p % 2 else PTREQ
+    req = f.PTREQ2 if p % 2 else f.PTREQ
     o.e(f"v_readfirstlane_b32 s88, v{req}")
     o.e(f"s_cmp_lt_u32 s88, {S_NCB}")
     o.e("s_cselect_b32 s88, s88, 0")
@@ -469,7 +510,7 @@ def next_block(o, p, tag):
     o.e(f"s_add_u32 s90, s88, {S_HK}")
     o.e(f"s_mul_hi_u32 s87, s90, {S_STRIDE}")
     o.e(f"s_mul_i32 s86, s90, {S_STRIDE}")
-    o.e(f"s_lshl_b32 s90, {S_CIN}, 13")           # 32 tokens of 256 bytes per block inside the cache block
+    o.e(f"s_lshl_b32 s90, {S_CIN}, {f.SLOT.bit_length() - 1}")  # 32 tokens per block inside the cache block
     o.e("s_add_u32 s86, s86, s90")
     o.e("s_addc_u32 s87, s87, 0")
     o.e(f"s_add_u32 {S_CIN}, {S_CIN}, 1")
@@ -477,7 +518,7 @@ def next_block(o, p, tag):
     o.e(f"s_cselect_b32 {S_CIN}, 0, {S_CIN}")
     o.e(f"s_cmp_eq_u32 {S_RLEFT}, 0")
     o.e(f"s_cbranch_scc1 L_noreq_{tag}%=")
-    o.e(f"global_load_dword v{req}, v{VZERO}, {S_RPTR}")
+    o.e(f"global_load_dword v{req}, v{f.VZERO}, {S_RPTR}")
     o.e(f"s_sub_u32 {S_RLEFT}, {S_RLEFT}, 1")
     o.e(f"s_add_u32 {S_RIN}, {S_RIN}, 1")
     o.e(f"s_cmp_lg_u32 {S_RIN}, {S_TPB}")
@@ -501,10 +542,10 @@ def iteration_head(o, f, p, tag):
     o.e("s_waitcnt vmcnt(0)")
     o.label(f"L_bar_{tag}")
     o.e("s_barrier")
-    if paged == 64 and p % 2 == 1:
-        next_tile(o, tag)
+    if paged == 64 and (p + ns) % 2 == 0:
+        next_tile(o, f, tag)
     if paged == 32:
-        next_block(o, p, tag)
+        next_block(o, f, p, tag)
     # K block i + NS is half (i + NS) % 2 of its tile, V block i + NS - 2 the same half of its own
     half = (p + ns) % 2 if paged == 64 else 0
     request_block(o, f, "K", p % ns, tag, half)
@@ -514,10 +555,10 @@ def iteration_head(o, f, p, tag):
         o.e("s_mov_b64 s[98:99], s[86:87]")
 
 
-def iteration_tail(o, tag, exit_label):
+def iteration_tail(o, f, tag, exit_label):
     o.e(f"s_cbranch_vccnz L_slow_{tag}%=")
     o.label(f"L_join_{tag}")
-    o.e(f"v_add_f32 v{LRUN}, v{LRUN}, v{LSUM}")
+    o.e(f"v_add_f32 v{f.LRUN}, v{f.LRUN}, v{f.LSUM}")
     o.e(f"s_sub_u32 {S_NB}, {S_NB}, 1")
     o.e(f"s_cmp_eq_u32 {S_NB}, 0")
     o.e(f"s_cbranch_scc1 {exit_label}%=")
@@ -528,32 +569,32 @@ def first_frags(p, f):
     return [frag for _, frag in iteration_pairs(p % f.unroll, f)[:NSLOT]]
 
 
-def item_setup(o, tag):
+def item_setup(o, f, tag):
     """Per-item state from S_ROW0: output pointers, the rows' key limits, the mask threshold, cleared
     accumulators and softmax state."""
-    o.e(f"v_add_u32 v{VROW}, {S_ROW0}, v{VN}")                                   # the lane's query row
-    o.e(f"v_mad_u64_u32 v[{OUTP}:{OUTP + 1}], s[92:93], v{VROW}, {S_OTS}, v[{OUTBASE}:{OUTBASE + 1}]")
-    o.e(f"v_cmp_gt_i32_e64 {S_STOREMASK}, {S_SQ}, v{VROW}")                      # rows that exist are stored
+    o.e(f"v_add_u32 v{f.VROW}, {S_ROW0}, v{f.VN}")                                   # the lane's query row
+    o.e(f"v_mad_u64_u32 v[{f.OUTP}:{f.OUTP + 1}], s[92:93], v{f.VROW}, {S_OTS}, v[{f.OUTBASE}:{f.OUTBASE + 1}]")
+    o.e(f"v_cmp_gt_i32_e64 {S_STOREMASK}, {S_SQ}, v{f.VROW}")                      # rows that exist are stored
     o.e(f"s_sub_u32 s88, {S_SQ}, 1")
-    o.e(f"v_min_i32 v{VT0}, s88, v{VROW}")                                       # rows past the end repeat the last one
-    o.e(f"v_add_u32 v{VT0}, {S_OFFSET}, v{VT0}")
+    o.e(f"v_min_i32 v{f.VT0}, s88, v{f.VROW}")                                       # rows past the end repeat the last one
+    o.e(f"v_add_u32 v{f.VT0}, {S_OFFSET}, v{f.VT0}")
     o.e(f"s_sub_u32 s89, {S_SKV}, 1")
-    o.e(f"v_min_i32 v{VT0}, s89, v{VT0}")                                        # causal: min(offset + row, skv - 1)
+    o.e(f"v_min_i32 v{f.VT0}, s89, v{f.VT0}")                                        # causal: min(offset + row, skv - 1)
     o.e(f"s_add_u32 s88, {S_OFFSET}, {S_ROW0}")
     o.e("s_min_i32 s88, s88, s89")
     o.e(f"s_cmp_eq_u32 {S_CAUSAL}, 0")
     o.e("s_cselect_b32 s88, s89, s88")                                           # the first row's limit
     o.e(f"s_cbranch_scc0 L_causal_{tag}%=")
-    o.e(f"v_mov_b32 v{VT0}, s89")                                                # not causal: skv - 1 for every row
+    o.e(f"v_mov_b32 v{f.VT0}, s89")                                                # not causal: skv - 1 for every row
     o.label(f"L_causal_{tag}")
-    o.e(f"v_sub_u32 v{LIMIT}, v{VT0}, v{V4H}")
+    o.e(f"v_sub_u32 v{f.LIMIT}, v{f.VT0}, v{f.V4H}")
     o.e(f"s_sub_u32 {S_MASKFROM}, s88, 30")
     if tag != "first":  # (several row blocks in turn: all of them start at key 0)
         o.e(f"s_mov_b32 {S_KEY0}, 0")
-    o.e(f"v_mov_b32 v{MC}, {START_REFERENCE}")
-    o.e(f"v_mov_b32 v{LRUN}, 0")
-    for r in range(64):
-        o.e(f"v_mov_b32 v{r}, 0")
+    o.e(f"v_mov_b32 v{f.MC}, {START_REFERENCE}")
+    o.e(f"v_mov_b32 v{f.LRUN}, 0")
+    for r in accumulators(f):
+        o.e(f"v_mov_b32 v{r}, 0" if f.acc_file == "v" else f"v_accvgpr_write_b32 a{r}, 0")
 
 
 def item_blocks(o):
@@ -571,69 +612,76 @@ def item_blocks(o):
     o.e(f"s_mov_b32 {S_VLEFT}, {S_NB}")
 
 
-def epilogue(o):
+def epilogue(o, f):
     """Normalises the item's accumulators and stores its rows: lane (n, h) holds, in accumulator
     register 16 db + 4 j + i, head-dim element 32 db + 8 j + 4 h + i of query row n.  The output pointer
     of lane (n, h) is row n's plus 16 h bytes."""
-    o.e(f"v_mov_b32 v{MB}, v{LRUN}")
+    o.e(f"v_mov_b32 v{f.MB}, v{f.LRUN}")
     o.e("s_nop 1")
-    o.e(f"v_permlane32_swap_b32 v{LRUN}, v{MB}")
+    o.e(f"v_permlane32_swap_b32 v{f.LRUN}, v{f.MB}")
     o.e("s_nop 1")
-    o.e(f"v_add_f32 v{ALPHA}, v{LRUN}, v{MB}")          # the row's sum: both halves of its keys
-    o.e(f"v_rcp_f32 v{ALPHA}, v{ALPHA}")
+    o.e(f"v_add_f32 v{f.ALPHA}, v{f.LRUN}, v{f.MB}")          # the row's sum: both halves of its keys
+    o.e(f"v_rcp_f32 v{f.ALPHA}, v{f.ALPHA}")
     o.e("s_nop 1")
-    for r in range(64):
-        o.e(f"v_mul_f32 v{r}, v{ALPHA}, v{r}")
-    for i in range(32):
-        o.e(f"v_cvt_pk_bf16_f32 v{S[0] + i}, v{2 * i}, v{2 * i + 1}")
+    if f.acc_file == "v":
+        scale_accumulators(o, f)
+        for i in range(f.d // 4):
+            o.e(f"v_cvt_pk_bf16_f32 v{f.S[0] + i}, v{f.ACC[0] + 2 * i}, v{f.ACC[0] + 2 * i + 1}")
+    else:
+        for i in range(f.d // 4):
+            t = (f.T[2 * (i % 2)], f.T[2 * (i % 2) + 1])
+            for k in range(2):
+                o.e(f"v_accvgpr_read_b32 v{t[k]}, a{f.ACC[0] + 2 * i + k}")
+                o.e(f"v_mul_f32 v{t[k]}, v{f.ALPHA}, v{t[k]}")
+            o.e(f"v_cvt_pk_bf16_f32 v{f.S[0] + i}, v{t[0]}, v{t[1]}")
     o.e("s_nop 1")
     # The two lanes of a row trade halves, so that each stores 16 consecutive bytes (a row's 32 bytes per
     # instruction): lane (n, 0) keeps its block j and takes (n, 1)'s, lane (n, 1) ends with both blocks j + 1.
-    for db in range(4):
+    for db in range(f.d // 32):
         for jp in range(2):
-            x = S[0] + 8 * db + 4 * jp
+            x = f.S[0] + 8 * db + 4 * jp
             o.e(f"v_permlane32_swap_b32 v{x}, v{x + 2}")
             o.e(f"v_permlane32_swap_b32 v{x + 1}, v{x + 3}")
     o.e("s_nop 3")
     o.e(f"s_and_saveexec_b64 s[62:63], {S_STOREMASK}")
     o.e("s_nop 1")
-    for db in range(4):
+    for db in range(f.d // 32):
         for jp in range(2):
-            src = S[0] + 8 * db + 4 * jp
-            o.e(f"global_store_dwordx4 v[{OUTP}:{OUTP + 1}], v[{src}:{src + 3}], off offset:{64 * db + 32 * jp} nt")   # written once, read by a later kernel
+            src = f.S[0] + 8 * db + 4 * jp
+            o.e(f"global_store_dwordx4 v[{f.OUTP}:{f.OUTP + 1}], v[{src}:{src + 3}], off offset:{64 * db + 32 * jp} nt")   # written once, read by a later kernel
     o.e("s_mov_b64 exec, s[62:63]")
     o.e("s_nop 1")
 
 
-def partial_epilogue(o):
+def partial_epilogue(o, f):
     """The accumulators of a part of the keys as floats, register group by register group in the order in
     which the lanes hold them (a store writes 1 KiB), and (reference, sum) per row."""
-    o.e(f"v_mov_b32 v{MB}, v{LRUN}")
+    o.e(f"v_mov_b32 v{f.MB}, v{f.LRUN}")
     o.e("s_nop 1")
-    o.e(f"v_permlane32_swap_b32 v{LRUN}, v{MB}")
+    o.e(f"v_permlane32_swap_b32 v{f.LRUN}, v{f.MB}")
     o.e("s_nop 1")
-    o.e(f"v_add_f32 v{S[0] + 1}, v{LRUN}, v{MB}")
-    o.e(f"v_mov_b32 v{S[0]}, v{MC}")
-    o.e(f"v_lshlrev_b32 v{VT0}, 3, v{VN}")
-    o.e(f"v_lshlrev_b32 v{PTMP}, 4, v{VN}")
-    o.e(f"v_lshl_add_u32 v{PTMP}, v{V4H}, 7, v{PTMP}")      # 16 times the lane
-    for g in range(16):
+    o.e(f"v_add_f32 v{f.S[0] + 1}, v{f.LRUN}, v{f.MB}")
+    o.e(f"v_mov_b32 v{f.S[0]}, v{f.MC}")
+    o.e(f"v_lshlrev_b32 v{f.VT0}, 3, v{f.VN}")
+    o.e(f"v_lshlrev_b32 v{f.PTMP}, 4, v{f.VN}")
+    o.e(f"v_lshl_add_u32 v{f.PTMP}, v{f.V4H}, 7, v{f.PTMP}")      # 16 times the lane
+    for g in range(f.d // 8):
         if g and g % 4 == 0:
             o.e("s_add_u32 s38, s38, 4096")
             o.e("s_addc_u32 s39, s39, 0")
-        o.e(f"global_store_dwordx4 v{PTMP}, v[{4 * g}:{4 * g + 3}], {S_PART} offset:{1024 * (g % 4)}")
-    o.e(f"global_store_dwordx2 v{VT0}, v[{S[0]}:{S[0] + 1}], {S_STATS}")   # (both lanes of a row: the same values)
+        o.e(f"global_store_dwordx4 v{f.PTMP}, {vr(f.ACC[0] + 4 * g, 4, f.acc_file)}, {S_PART} offset:{1024 * (g % 4)}")
+    o.e(f"global_store_dwordx2 v{f.VT0}, v[{f.S[0]}:{f.S[0] + 1}], {S_STATS}")   # (both lanes of a row: the same values)
 
 
 def last_epilogue(o, f):
     if f.parts:
         o.e(f"s_cmp_lg_u64 {S_PART}, 0")
         o.e("s_cbranch_scc1 L_partial%=")
-    epilogue(o)
+    epilogue(o, f)
     if f.parts:
         o.e("s_branch L_done%=")
         o.label("L_partial")
-        partial_epilogue(o)
+        partial_epilogue(o, f)
         o.label("L_done")
 
 
@@ -654,17 +702,17 @@ def next_item(o, f):
     o.e("s_sub_u32 s88, s88, 1")
     o.e(f"s_lshl_b32 {S_ROW0}, s88, 5")                 # (the finished item's pointers and store mask stay in registers)
     o.e("s_barrier")                                    # everybody has left the rings
-    o.e(f"v_add_u32 v{VROW}, {S_ROW0}, v{VN}")
+    o.e(f"v_add_u32 v{f.VROW}, {S_ROW0}, v{f.VN}")
     o.e(f"s_sub_u32 s88, {S_SQ}, 1")
-    o.e(f"v_min_i32 v{VROW}, s88, v{VROW}")
-    o.e(f"v_mad_u64_u32 v[{PTMP}:{PTMP + 1}], s[92:93], v{VROW}, {S_QTS}, v[{QBASE}:{QBASE + 1}]")
-    for ks in range(8):
-        o.e(f"global_load_dwordx4 {vr(QF + 4 * ks, 4)}, v[{PTMP}:{PTMP + 1}], off offset:{32 * ks}")
+    o.e(f"v_min_i32 v{f.VROW}, s88, v{f.VROW}")
+    o.e(f"v_mad_u64_u32 v[{f.PTMP}:{f.PTMP + 1}], s[92:93], v{f.VROW}, {S_QTS}, v[{f.QBASE}:{f.QBASE + 1}]")
+    for ks in range(f.d // 16):
+        o.e(f"global_load_dwordx4 {vr(f.QF + 4 * ks, 4)}, v[{f.PTMP}:{f.PTMP + 1}], off offset:{32 * ks}")
     item_blocks(o)
     if paged:
         o.e("s_mov_b64 s[84:85], s[50:51]")
         o.e("s_mov_b64 s[86:87], s[52:53]")
-        o.e(f"v_mov_b32 v{PTREQ}, s54")
+        o.e(f"v_mov_b32 v{f.PTREQ}, s54")
         o.e(f"s_mov_b32 {S_CIN}, s55")
         o.e(f"s_mov_b32 {S_RIN}, s56")
         o.e("s_mov_b64 s[82:83], s[58:59]")
@@ -678,14 +726,19 @@ def next_item(o, f):
         o.e("s_mov_b64 s[66:67], s[52:53]")
     for ln in generate_first(f, "nx"):
         o.lines.append(ln)
-    epilogue(o)
-    item_setup(o, "nx")
+    epilogue(o, f)
+    item_setup(o, f, "nx")
     o.e("s_branch L_item_top%=")
     o.label("L_last_item")
     last_epilogue(o, f)
 
 
-FIRST32 = ("s[50:51]", "s[52:53]", "s[58:59]", "s[84:85]", "s[98:99]")  # blocks of 32: the first five byte offsets
+def first_offsets(f):
+    """Paged: the registers of the first byte offsets, one per tile of 64 keys (`paged` 64) or per block of 32.  The loop
+    goes on with the last two: K's and V's tiles, or the next two V blocks."""
+    if f.paged == 64:
+        return ([S_OFF0] if f.ns == 5 else []) + [S_OFFV, S_OFFK]
+    return ["s[50:51]", "s[52:53]"] + (["s[58:59]"] if f.ns == 5 else []) + [S_OFFV, S_OFF0]
 
 
 def generate_first(f, suffix=""):
@@ -694,37 +747,37 @@ def generate_first(f, suffix=""):
     o = Out()
     paged = f.paged
     for j in range(f.ns):
-        if paged:  # tiles 0, 1, 2 at S_OFF0, S_OFFV, S_OFFK; blocks of 32: 0 .. 4
-            src = ("s[98:99]", S_OFFV, S_OFFK)[j // 2] if paged == 64 else FIRST32[j]
+        if paged:
+            src = first_offsets(f)[j // 2 if paged == 64 else j]
             lo = int(src[2:4])
             o.e(f"s_cmp_eq_u32 {S_KLEFT}, 0")
             o.e(f"s_cbranch_scc1 L_noK_pro{j}{suffix}%=")
             o.e(f"s_add_u32 s90, s64, s{lo}")
             o.e(f"s_addc_u32 s91, s65, s{lo + 1}")
             if j % 2 and paged == 64:
-                o.e(f"s_add_u32 s90, s90, {SLOT}")
+                o.e(f"s_add_u32 s90, s90, {f.SLOT}")
                 o.e("s_addc_u32 s91, s91, 0")
-            o.e(f"s_add_u32 m0, {S_M0B}, {j * SLOT}")
+            o.e(f"s_add_u32 m0, {S_M0B}, {j * f.SLOT}")
             o.e("s_nop 0")
-            two_loads(o, LDK, "s[90:91]")
+            block_loads(o, f, f.LDK, "s[90:91]")
             o.e(f"s_sub_u32 {S_KLEFT}, {S_KLEFT}, 1")
             o.label(f"L_noK_pro{j}{suffix}")
         else:
             request_block(o, f, "K", j, f"pro{j}{suffix}", 0)
     for j in range(f.ns - 2):
         if paged:
-            src = ("s[98:99]", S_OFFV)[j // 2] if paged == 64 else FIRST32[j]
+            src = first_offsets(f)[j // 2 if paged == 64 else j]
             lo = int(src[2:4])
             o.e(f"s_cmp_eq_u32 {S_VLEFT}, 0")
             o.e(f"s_cbranch_scc1 L_noV_pro{j}{suffix}%=")
             o.e(f"s_add_u32 s90, s66, s{lo}")
             o.e(f"s_addc_u32 s91, s67, s{lo + 1}")
             if j % 2 and paged == 64:
-                o.e(f"s_add_u32 s90, s90, {SLOT}")
+                o.e(f"s_add_u32 s90, s90, {f.SLOT}")
                 o.e("s_addc_u32 s91, s91, 0")
-            o.e(f"s_add_u32 m0, {S_M0B}, {f.vring + j * SLOT}")
+            o.e(f"s_add_u32 m0, {S_M0B}, {f.vring + j * f.SLOT}")
             o.e("s_nop 0")
-            two_loads(o, LDV, "s[90:91]")
+            block_loads(o, f, f.LDV, "s[90:91]")
             o.e(f"s_sub_u32 {S_VLEFT}, {S_VLEFT}, 1")
             o.label(f"L_noV_pro{j}{suffix}")
         else:
@@ -735,20 +788,21 @@ def generate_first(f, suffix=""):
 def generate(f):
     o = Out()
     assert (f.ns, f.unroll) in ((5, 10), (4, 4))
-    o.e(f"v_mov_b32 v{VZERO}, 0")
-    item_setup(o, "first")
+    o.e(f"v_mov_b32 v{f.VZERO}, 0")
+    item_setup(o, f, "first")
     o.label("L_item_top")
     o.e("s_waitcnt vmcnt(0)")
     o.e("s_barrier")
     # ---- S(0) from K block 0; behind it the fragments of iteration 0 (K block 1) ------------------
     pairs = score_pairs(0, 0, f)
     it0 = iteration_pairs(0, f, has_pv=False)
-    phase = stream(o, pairs, [[] for _ in pairs], 0, False, [frag for _, frag in it0[:NSLOT]])
+    behind = [frag for _, frag in it0] + first_frags(1, f)
+    phase = stream(o, f, pairs, [[] for _ in pairs], 0, False, behind[:NSLOT])
     # ---- iteration 0: S(1), sm(0) ---------------------------------------------------------------
     o.e("s_nop 7")
     iteration_head(o, f, 0, "i0")
-    phase = stream(o, it0, spread(softmax_ops(0), len(it0)), phase, True, first_frags(1, f))
-    iteration_tail(o, "i0", "L_exit0")
+    phase = stream(o, f, it0, spread(softmax_ops(f, 0), len(it0)), phase, True, first_frags(1, f))
+    iteration_tail(o, f, "i0", "L_exit0")
     phases = {0: phase}  # ring slot of the next iteration's first fragment, behind iteration p
     # ---- iterations 1 .. : `unroll` in a row, then round again -----------------------------------------
     for k in range(f.unroll):
@@ -756,9 +810,9 @@ def generate(f):
         o.label(f"L_it{p}")
         iteration_head(o, f, p, f"p{p}")
         pairs = iteration_pairs(p, f)
-        phase = stream(o, pairs, spread(softmax_ops(p % 2), len(pairs)), phase, True, first_frags(p + 1, f))
+        phase = stream(o, f, pairs, spread(softmax_ops(f, p % 2), len(pairs)), phase, True, first_frags(p + 1, f))
         assert phases.setdefault(p, phase) == phase  # (iteration 0 and iteration `unroll` share an exit)
-        iteration_tail(o, f"p{p}", f"L_exit{p}")
+        iteration_tail(o, f, f"p{p}", f"L_exit{p}")
     o.e("s_branch L_it1%=")
 
     # ---- exits: PV of the last block i = p (mod unroll) -----------------------------------------------
@@ -768,19 +822,27 @@ def generate(f):
         o.label(f"L_exit{p}")
         o.e("s_waitcnt lgkmcnt(0)")
         held = {frag: (phases[p] + j) % NSLOT for j, frag in enumerate(first_frags(p + 1, f)) if frag[0] == "V"}
-        wanted = [("V", p % f.ns, x // 4, x % 4) for x in range(8)]
+        db = f.d // 32
+        wanted = [("V", p % f.ns, x // db, x % db) for x in range(2 * db)]
         free = [x for x in range(NSLOT) if x not in held.values()]
         missing = [frag for frag in wanted if frag not in held]
         slots = dict(held)
-        for frag in missing:
-            slots[frag] = free.pop(0)
-            for x in frag_reads(frag, slots[frag]):
+        for k, frag in enumerate(missing[:len(free)]):
+            slots[frag] = free[k]
+            for x in frag_reads(f, frag, slots[frag]):
                 o.e(x)
         for frag in sorted(held, key=wanted.index):
-            o.e(mfma(("PV", frag[3], p % 2, frag[2]), slots[frag]))
-        o.e("s_waitcnt lgkmcnt(0)")
-        for frag in missing:
-            o.e(mfma(("PV", frag[3], p % 2, frag[2]), slots[frag]))
+            o.e(mfma(f, ("PV", frag[3], p % 2, frag[2]), slots[frag]))
+        batch, rest = missing[:len(free)], missing[len(free):]
+        while batch:
+            o.e("s_waitcnt lgkmcnt(0)")
+            for frag in batch:
+                o.e(mfma(f, ("PV", frag[3], p % 2, frag[2]), slots[frag]))
+            batch, rest = rest[:NSLOT], rest[NSLOT:]
+            for k, frag in enumerate(batch):
+                slots[frag] = k
+                for x in frag_reads(f, frag, k):
+                    o.e(x)
         o.e("s_branch L_end%=")
 
     slow_path(o, f, 0, "L_slow_i0", "L_join_i0", first=True)
@@ -796,24 +858,82 @@ def generate(f):
     return o.lines
 
 
+def bind(reg, value, inout=False, file="v", n=1):
+    """An operand bound to a register (a name like "s[64:65]", or the first of `n` of a file)."""
+    return f'"{"+" if inout else ""}{{{vr(reg, n, file) if isinstance(reg, int) else reg}}}"({value})'
+
+
+def operands(f):
+    """(outputs, inputs) of the first requests and of the block behind them, by the names that prefill_kernel
+    in prefill_stream_kernel.h gives the values."""
+    io = lambda reg, value, n=1: bind(reg, value, True, n=n)
+    i = lambda reg, value, n=1: bind(reg, value, n=n)
+    offs = [(reg, f"off[{k}]") for k, reg in enumerate(first_offsets(f))] if f.paged else []
+    loads = [i(f.LDK, "ldk", f.tensor_loads), i(f.LDV, "ldv", f.tensor_loads)]
+    wide_in = [i(f.LDKP, "ldp"), i(S_PSTRIDE, "wide.stride"), i(S_M0P, "wide.m0"), i(S_VSTRIDE, "wide.v_stride")] if f.wide else []
+    wide_io = [io(S_PBASE, "wide.base")] if f.wide else []
+    bases = [(S_KBASE, "req.kbase"), (S_VBASE, "req.vbase")]
+    counts = [io(S_KLEFT, "req.k_requests"), io(S_VLEFT, "req.v_requests")]
+    if f.paged:
+        first = counts, loads + [i(*b) for b in bases] + [i(S_M0B, "req.m0_base")] + [i(*x) for x in offs]
+    else:
+        first = [io(*b) for b in bases] + counts + wide_io, loads + [i(S_STRIDE, "req.stride"), i(S_M0B, "req.m0_base")] + wide_in
+    outs = [io(f.QF + 16 * k, f"q[{k}]", 16) for k in range(f.d // 64)] + [io(*b) for b in bases] + counts + wide_io
+    outs += [io(S_NB, "nblk"), io(S_K, "it.k"), io(S_ROW0, "it.row0"), io(S_KEY0, "it.key0")]
+    ins = [i(f.KOFF, "ko", f.d // 16), i(f.VOFF, "vo", f.d // 32)] + loads + wide_in
+    ins += [i(f.QBASE, "q_base", 2), i(f.OUTBASE, "out_base", 2), i(f.VN, "n"), i(f.V4H, "h4")]
+    ins += [i(S_STRIDE, "req.stride"), i(S_C, "a.scale_log2e"), i(S_M0B, "req.m0_base"), i(S_J, "it.j"), i(S_SPG, "it.spg"), i(S_NQT, "it.nqt"),
+            i(S_SQ, "it.sq"), i(S_SKV, "it.skv"), i(S_OFFSET, "it.offset"), i(S_CAUSAL, "it.causal"), i(S_QTS, "it.q_row_bytes"),
+            i(S_OTS, "it.out_row_bytes")]
+    if f.wide:
+        ins += [i(f.QFP, "q_second", 16), i(f.KOFFP, "po", 4)]
+    if f.window:
+        ins += [i(f.LOWEST, "lowest"), i(S_LOWTO, "low_to")]
+    if f.paged:
+        outs += [io(S_CIN, "tab.read_in_block"), io(S_RIN, "tab.request_in_block"), io(S_RPTR, "tab.entry_ptr"), io(S_RLEFT, "tab.entry_requests"),
+                 io(f.PTREQ, "tab.entry"), io(S_PART, "out_part.acc")] + [io(*x) for x in offs[-2:]]
+        ins += [i(S_HKV, "tab.kv_heads"), i(S_HK, "tab.kv_head"), i(S_NCB, "tab.num_blocks"), i(S_TPB, "tab.per_block"), i(S_STATS, "out_part.stats")]
+        if f.paged == 32:
+            outs += [io(f.PTREQ2, "tab.entry2")]
+    if f.items and f.paged:  # where the items that follow start
+        ins += [i(S_OFF0, "off[0]"), i("s[50:51]", "off[1]"), i("s[52:53]", "off[2]"), i("s54", "tab.entry"), i("s55", "tab.read_in_block"),
+                i("s56", "tab.request_in_block"), i("s[58:59]", "tab.entry_ptr")]
+    elif f.items:
+        ins += [i("s[50:51]", "kbase0"), i("s[52:53]", "vbase0")]
+    return first, (outs, ins)
+
+
+def registers(text):
+    """Every vector, accumulation and scalar register that a text names."""
+    found = set()
+    for file, single, lo, hi in re.findall(r"\b([vas])(?:(\d+)|\[(\d+):(\d+)\])", text):
+        found |= {f"{file}{r}" for r in (range(int(single), int(single) + 1) if single else range(int(lo), int(hi) + 1))}
+    return found
+
+
+def write_asm(out, macro, lines, outs, ins):
+    """An asm statement's text, operands and clobbers (whatever the text names and no operand is bound to)."""
+    bound = [registers(x.split("(")[0]) for x in outs + ins]
+    for k, x in enumerate(bound):
+        assert not any(x & y for y in bound[:k]), (macro, (outs + ins)[k])
+    clobbers = registers("\n".join(lines)) - set().union(*bound)
+    out.write(f"#define {macro} \\\n")
+    for ln in lines:
+        out.write(f'  "{ln}\\n\\t" \\\n')
+    named = sorted(clobbers, key=lambda r: (r[0], int(r[1:])))
+    out.write(f'  "" : {", ".join(outs)} : {", ".join(ins)} : "memory", "vcc", "scc", "m0"' + "".join(f', "{r}"' for r in named) + "\n")
+
+
 def main():
-    out = sys.argv[1] if len(sys.argv) > 1 else "/dev/stdout"
-    with open(out, "w") as f:
-        f.write("// Generated by gen_prefill_stream.py; do not edit.\n#pragma once\n")
+    with open(sys.argv[1] if len(sys.argv) > 1 else "/dev/stdout", "w") as out:
+        out.write("// Generated by gen_prefill_stream.py; do not edit.\n#pragma once\n")
         for form in FORMS:
-            for macro, lines in ((f"TTPA_STREAM_FIRST_TEXT_{form.name}", generate_first(form)),
-                                 (f"TTPA_STREAM_LOOP_TEXT_{form.name}", generate(form))):
-                f.write(f"#define {macro} \\\n")
-                for ln in lines:
-                    f.write(f'  "{ln}\\n\\t" \\\n')
-                f.write('  ""\n')
-        regs = ", ".join([f'"v{r}"' for r in CLOBBERED] + [f'"{r}"' for r in SCALAR_CLOBBERS])
-        f.write(f"#define TTPA_STREAM_LOOP_CLOBBERS {regs}\n")
-        lds = {form.pring + (form.ns * PSLOT if form.wide else 0) for form in FORMS}
-        assert len(lds) == 1  # every form takes half of a CU's LDS
-        wide = next(form for form in FORMS if form.wide)
-        f.write(f"#define TTPA_STREAM_LDS_BYTES {lds.pop()}\n#define TTPA_STREAM_V_RING {FORMS[0].vring}\n"
-                f"#define TTPA_STREAM_WIDE_V_RING {wide.vring}\n#define TTPA_STREAM_WIDE_P_RING {wide.pring}\n")
+            first, loop = operands(form)
+            write_asm(out, f"TTPA_STREAM_FIRST_{form.name}", generate_first(form), *first)
+            write_asm(out, f"TTPA_STREAM_LOOP_{form.name}", generate(form), *loop)
+        out.write(f"#define TTPA_STREAM_SLOTS(d, wide) ((wide) || (d) == 256 ? 4 : 5)\n")
+        for form in FORMS:
+            assert form.ns == (4 if form.wide or form.d == 256 else 5)
 
 
 if __name__ == "__main__":

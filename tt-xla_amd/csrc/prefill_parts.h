@@ -45,7 +45,12 @@ struct SplitRule {
   int known_percent;            // ... or that the caller knows of: copies are better than the shortest split of block-float-8 blocks
   int block_cost;               // of a 32-key block, in hundredths of the streaming loop's
 };
-constexpr SplitRule kStreamSplit = {2, 8, 16, 100, 100, 100};  // (80 KiB of LDS per workgroup)
+// At 64 and 256 the streaming loop keeps the parts of the plain one: with 128's rule (two thirds as many parts) 4 x 64 rows of 8 / 8 heads
+// of 64 behind 1024 tokens took 16.0 us instead of 14.9, and the error against 64 bits was 1 ... 5 % larger, since a part starts from a
+// maximum of its own.
+constexpr SplitRule stream_split(int d) {
+  return d == 128 ? SplitRule{2, 8, 16, 100, 100, 100} : SplitRule{d == 64 ? 2 : 1, 4, 8, 150, 100, d == 64 ? 150 : 300};
+}
 constexpr SplitRule plain_split(int d, bool bfp8) { return {d <= 128 ? 2 : 1, 4, 8, bfp8 ? 125 : 150, bfp8 && d == 128 ? 113 : 100, d == 256 ? 300 : bfp8 ? 225 : 150}; }
 // Parts up to one workgroup per CU; twice as many, which then share a CU's matrix pipes, from this many blocks per part
 // on (128 workgroups, 2 / 4 parts: 64 blocks 35.0 / 35.6 us, 80 blocks 43.5 / 41.5, 96 blocks 43.6 / 40.8, 256 blocks
@@ -59,8 +64,8 @@ constexpr int part_acc_floats(int d) { return kRowsPerWave * d; }  // accumulato
 __device__ __forceinline__ int blocks_per_part(const PrefillArgs &a, int offset) {
   const int most = max(((a.causal ? min(a.skv, offset + a.sq) : a.skv) + kBlockKeys - 1) / kBlockKeys, 1);  // of the last row block
   if (most < a.split_from) return most;
-  const int shared = (most + a.parts - 1) / a.parts;
-  const int share = shared >= kSharedPartBlocks ? shared : max((most + a.parts_one - 1) / a.parts_one, a.part_min);
+  const int shared = quotient(a.by_parts, most + a.parts - 1);
+  const int share = shared >= kSharedPartBlocks ? shared : max(quotient(a.by_parts_one, most + a.parts_one - 1), a.part_min);
   return (share + 1) & ~1;
 }
 
@@ -161,6 +166,7 @@ inline void set_parts(PrefillArgs &a, int heads_per_wg, const SplitRule &rule) {
   a.part_min = rule.min_part;
   a.parts = blocks < a.split_from * (a.keys_known ? rule.known_percent : rule.table_percent) / 100 ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>(rule.wgs_per_cu * cus / wgs, most));
   a.parts_one = (int)std::max<int64_t>(1, std::min<int64_t>(cus / wgs, most));
+  a.by_parts = divisor(a.parts), a.by_parts_one = divisor(a.parts_one);
 }
 
 inline int64_t part_bytes(PrefillArgs a, int heads_per_wg, const SplitRule &rule, int d) {
