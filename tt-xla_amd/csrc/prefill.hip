@@ -148,21 +148,13 @@ __global__ __launch_bounds__(256, prefill_wgs_per_cu<RH>(D, MODE)) void prefill_
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, h = lane >> 5;
   const int n_lane = n;
-  // Workgroups are dealt to the 8 XCDs round-robin by linear id, and each XCD has its own
-  // L2: all query tiles of one (batch, KV-head group) run on the same XCD, one after the
-  // other, so that K/V of a group is fetched from HBM by one L2 only and stays resident there
-  // while its query tiles stream through.
   const int nqt = (a.sq + ROWS * RPW - 1) / (ROWS * RPW);
-  const int groups = a.hq / HPW;
-  const int xcd = wg & 7, slot = wg >> 3;
-  const int yl = slot / nqt;
-  const int y = yl * 8 + xcd;
-  if (y >= a.batch * groups) return;  // grid is padded to a multiple of 8 groups
-  const int qt = nqt - 1 - (slot - yl * nqt);  // heavy (late) tiles are scheduled first
-  const int b = y / groups;
-  const int hq0 = (y - b * groups) * HPW;
-  const int g = a.hq / a.hkv;
-  const int hk = hq0 / g;
+  int y, rank;
+  if (!workgroup_place(a, wg, y, rank)) return;
+  const int qt = nqt - 1 - rank;  // heavy (late) tiles are scheduled first
+  const int b = quotient(a.by_groups, y);
+  const int hq0 = (y - b * a.by_groups.d) * HPW;
+  const int hk = quotient(a.by_group_heads, hq0);
   const int hq = hq0 + wave % HPW;
   const int row0 = (qt * RPW + wave / HPW) * ROWS;  // first query row of the wavefront
   // (the dense form has no chunk_start and at least one tile: without the bounds its code is what it was, 2 % faster at head size 256)
@@ -597,11 +589,11 @@ __global__ __launch_bounds__(256, prefill_wgs_per_cu<RH>(D, MODE)) void prefill_
 
   // ---- normalise and store: lane (n, h) holds head-dim elements 32 db + 8 j + 4 h + i ----
   if constexpr (SPLIT) {
-    if (!whole) {
+    if (!whole && wave_active) {
       // a part's accumulators and (maximum, sum) per row: lane l's four elements of group 4 db + j at float 256 (4 db + j) + 4 l
       // of the row block's, 1 KiB per store of the wavefront.  A row that sees none of the part's keys has maximum -inf, sum 0.
       const float l_tot = l_run[0] + __shfl_xor(l_run[0], 32);
-      const PartLayout lay = part_layout(a, ROWS * RPW);
+      const PartLayout lay = part_layout(a);
       const int64_t at = (((int64_t)part * a.batch + b) * a.hq + hq) * lay.row_blocks + qt * RPW + wave / HPW;
       float *dst = a.part_acc + at * part_acc_floats(D) + 4 * lane;
 #pragma unroll
@@ -649,19 +641,15 @@ int launch_split(PrefillArgs &b, int grid, hipStream_t st) {
 
 template <int D, int HPW, int MODE, int RH>
 int launch_mode(const PrefillArgs &a, hipStream_t st) {
-  constexpr int RPW = 4 / HPW;
-  constexpr int ROWS = kRowsPerWave * RH;
-  const int nqt = (a.sq + ROWS * RPW - 1) / (ROWS * RPW);
-  const int ny8 = (a.batch * (a.hq / HPW) + 7) / 8;
   PrefillArgs b = a;
-  int grid = nqt * ny8 * 8;
+  int grid = lay_out(b, HPW);
   b.parts = 1;
   if constexpr (MODE != 0) {
     constexpr SplitRule kRule = plain_split(D, MODE == 4);
     if (plain_splits(a) && a.part_acc && a.part_bytes >= part_bytes(a, HPW, kRule, D)) set_parts(b, HPW, kRule);
     if (b.parts > 1) {
       if (const int rc = launch_split<D, HPW, MODE, RH, true>(b, grid, st)) return rc;
-      prefill_merge_kernel<D, RPW><<<dim3((b.sq + kRowsPerWave - 1) / kRowsPerWave, b.hq, b.batch), dim3(2 * D), 0, st>>>(b);
+      prefill_merge_kernel<D><<<dim3((b.sq + kRowsPerWave - 1) / kRowsPerWave, b.hq, b.batch), dim3(2 * D), 0, st>>>(b);
       return check_launch("sdpa_prefill (merge of the parts)");
     }
   }

@@ -5,6 +5,8 @@
 
 #include "common.h"
 
+#include <algorithm>
+
 namespace ttpa {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -68,6 +70,10 @@ struct PrefillArgs {
   // The streaming kernel: workgroups per (batch entry, head group), each taking one or several row blocks
   int spg;
   Divisor by_spg, by_groups, by_group_heads;  // spg, head groups of a batch entry, query heads of a KV head
+  // The place of a workgroup (workgroup_place): head groups (batch entries times the groups of one), of which whole rounds of eight
+  // are dealt to one XCD each and the rest over all of them; query heads of a group
+  int full_rounds, rest, head_group;
+  Divisor by_rest, by_head_group;
   int spg_even; // > 0: when the row blocks weigh about the same, only this many of them work (equal shares)
   // ... with keys of 128 + 64 features: the second part of q and k, and V's own strides
   const uint16_t *q2, *k2;
@@ -94,6 +100,46 @@ __device__ __forceinline__ int div_block(const PrefillArgs &a, int key) {
 // row numbers stay small.
 __device__ __forceinline__ int chunk_offset(const int32_t *chunk_start, int sq, int skv) {
   return chunk_start ? min(max(chunk_start[0], -sq), skv) : 0;
+}
+
+// The wavefronts of a workgroup are four consecutive (row block of 32 rows, query head) pairs of a head group, row block by row block:
+// groups of four heads where a KV head has a multiple of four (a workgroup is four heads of one row block), all heads of it otherwise
+// (two heads: two row blocks; five: the heads of one row block and part of the next).  One head per workgroup where their number is no
+// multiple of two left three of four wavefronts without rows in a chunk of 32 and read K and V once per head.
+__device__ __forceinline__ int row_blocks(const PrefillArgs &a) { return (a.sq + kRowsPerWave - 1) / kRowsPerWave; }
+// Row block of the last pair of workgroup `wg` of a head group.
+__device__ __forceinline__ int last_row_block(const PrefillArgs &a, int wg) {
+  return min(quotient(a.by_head_group, 4 * wg + 3), row_blocks(a) - 1);
+}
+
+// Head group y and rank (0: the last row blocks, heavy ones first) of attention workgroup wg.  Workgroups are dealt to the 8 XCDs
+// round-robin by linear id, and each XCD has its own L2: all workgroups of a group run on one XCD, one after the other, so that its
+// K / V is fetched by one L2 only and stays resident there.  The groups left over when the rounds of eight are dealt are spread over all
+// XCDs, one, two or four to each where they are a power of two: on an XCD each they left the others idle (two groups, one prompt of 4096 tokens with
+// 8 / 2 heads of 64: 80 -> 51 us; 1312 rows behind 9152 128 -> 51).
+__device__ __forceinline__ bool workgroup_place(const PrefillArgs &a, int wg, int &y, int &rank) {
+  const int t = wg - a.full_rounds * 8 * a.spg;
+  if (t < 0) {
+    const int slot = wg >> 3, round = quotient(a.by_spg, slot);
+    y = round * 8 + (wg & 7), rank = slot - round * a.spg;
+    return true;
+  }
+  if (a.rest == 0) return false;
+  rank = quotient(a.by_rest, t);
+  y = a.full_rounds * 8 + t - rank * a.rest;
+  return rank < a.spg;
+}
+// ... and the host's side: the fields it reads, for `heads` query heads per head group and `spg` workgroups per group (0: as many as there are row
+// blocks); the grid, a multiple of 8.
+inline int lay_out(PrefillArgs &a, int heads, int spg = 0) {
+  const int groups = a.batch * (a.hq / heads);
+  const int pairs = (a.sq + kRowsPerWave - 1) / kRowsPerWave * heads;
+  a.head_group = heads, a.by_head_group = divisor(heads);
+  a.spg = spg > 0 ? spg : (pairs + 3) / 4;
+  a.full_rounds = groups / 8, a.rest = groups % 8;
+  a.by_spg = divisor(a.spg), a.by_rest = divisor(std::max(a.rest, 1));
+  a.by_groups = divisor(a.hq / heads), a.by_group_heads = divisor(a.hq / a.hkv);
+  return a.full_rounds * 8 * a.spg + (a.rest * a.spg + 7) / 8 * 8;
 }
 
 // LDS geometry of one stage: the K tile (64 rows of D elements) followed by the V tile.

@@ -75,8 +75,8 @@ struct PartLayout {
   int64_t slots;  // (part, batch entry, head, row block) combinations
   int row_blocks;
 };
-__host__ __device__ inline PartLayout part_layout(const PrefillArgs &a, int rows_per_wg) {
-  const int rb = (a.sq + rows_per_wg - 1) / rows_per_wg * (rows_per_wg / kRowsPerWave);
+__host__ __device__ inline PartLayout part_layout(const PrefillArgs &a) {
+  const int rb = (a.sq + kRowsPerWave - 1) / kRowsPerWave;
   return {(int64_t)a.parts * a.batch * a.hq * rb, rb};
 }
 
@@ -86,19 +86,19 @@ __host__ __device__ inline PartLayout part_layout(const PrefillArgs &a, int rows
 // 8 group + 4 (lane / 32) .. + 3): 512 consecutive bytes per read of 32 lanes, whole 32-byte pieces of a row per
 // write.  Memory bound: 34 MB of accumulators (512 rows, 32 heads, 4 parts) in 7.9 us.  Parts past the last are zeros: repeated
 // with weight 0 they needed as long at head sizes 64 and 128 and 5 us more at 256 (128 rows of 16/8 heads behind 2048 tokens 36.7 / 31.7).
-template <int D, int RPW>
+template <int D>
 __global__ __launch_bounds__(2 * D) void prefill_merge_kernel(PrefillArgs a) {
   const int rb = blockIdx.x, hq = blockIdx.y, b = blockIdx.z;
-  const int qt = rb / RPW;
+  const int pair = rb * a.head_group + hq - quotient(a.by_head_group, hq) * a.head_group;
   const int n = threadIdx.x & 31, g = threadIdx.x >> 5;
   const int offset = a.causal ? chunk_offset(a.chunk_start, a.sq, a.skv) : 0;
-  const int wg_last_row = min(a.sq, (qt + 1) * kRowsPerWave * RPW) - 1;
+  const int wg_last_row = min(a.sq, (last_row_block(a, pair >> 2) + 1) * kRowsPerWave) - 1;
   const int kv_end = a.causal ? min(a.skv, offset + wg_last_row + 1) : a.skv;
   const int nblk = (kv_end + kBlockKeys - 1) / kBlockKeys;
   const int share = blocks_per_part(a, offset);
   if (share >= nblk) return;  // one workgroup saw all keys and wrote the output
   const int active = (nblk + share - 1) / share;
-  const PartLayout lay = part_layout(a, kRowsPerWave * RPW);
+  const PartLayout lay = part_layout(a);
   const int64_t step = (int64_t)a.batch * a.hq * lay.row_blocks;
   const int64_t at = ((int64_t)b * a.hq + hq) * lay.row_blocks + rb;
   const float *acc = a.part_acc + at * part_acc_floats(D) + (8 * g) * 64 + 4 * n;
@@ -154,11 +154,11 @@ __global__ __launch_bounds__(2 * D) void prefill_merge_kernel(PrefillArgs a) {
 
 // Workgroups of the launch without a split, and what it may be split into: as many parts as fill the workgroup slots of
 // every CU once, if its row blocks leave at least half of them empty and its page keys may be enough to be split at all.
-inline void set_parts(PrefillArgs &a, int heads_per_wg, const SplitRule &rule) {
+inline void set_parts(PrefillArgs &a, int heads, const SplitRule &rule) {
   int cus = device_cus();
   if (cus <= 0) cus = 256;
-  const int rows = kRowsPerWave * 4 / heads_per_wg;
-  const int64_t wgs = (int64_t)a.batch * (a.hq / heads_per_wg) * ((a.sq + rows - 1) / rows);
+  const int pairs = (a.sq + kRowsPerWave - 1) / kRowsPerWave * heads;
+  const int64_t wgs = (int64_t)a.batch * (a.hq / heads) * ((pairs + 3) / 4);
   const int blocks = (int)((a.keys_bound + kBlockKeys - 1) / kBlockKeys);
   const int most = std::min(kMaxParts, (blocks + rule.min_part - 1) / rule.min_part);
   const int64_t from = 2 * wgs <= cus ? 7 * wgs / 16 : std::min<int64_t>(wgs, rule.wgs_per_cu * cus) / 2;
@@ -169,12 +169,18 @@ inline void set_parts(PrefillArgs &a, int heads_per_wg, const SplitRule &rule) {
   a.by_parts = divisor(a.parts), a.by_parts_one = divisor(a.parts_one);
 }
 
-inline int64_t part_bytes(PrefillArgs a, int heads_per_wg, const SplitRule &rule, int d) {
-  set_parts(a, heads_per_wg, rule);
+inline int64_t part_bytes(PrefillArgs a, int heads, const SplitRule &rule, int d) {
+  set_parts(a, heads, rule);
   if (a.parts <= 1) return 0;
-  return part_layout(a, kRowsPerWave * 4 / heads_per_wg).slots * (part_acc_floats(d) + 2 * kRowsPerWave) * (int64_t)sizeof(float);
+  return part_layout(a).slots * (part_acc_floats(d) + 2 * kRowsPerWave) * (int64_t)sizeof(float);
 }
 
+// Query heads of a head group: the streaming loop's (head_group_size), whose wavefronts may be of different row blocks wherever the
+// heads end, and the plain loop's, whose workgroups take whole row blocks of 4, 2 or 1 heads.
+inline int head_group_size(const PrefillArgs &a) {
+  const int g = a.hq / a.hkv;
+  return g % 4 == 0 ? 4 : g;
+}
 inline int heads_per_workgroup(const PrefillArgs &a) {
   const int g = a.hq / a.hkv;
   return g % 4 == 0 ? 4 : g % 2 == 0 ? 2 : 1;

@@ -3,9 +3,9 @@
 // 16 / 32 v_mfma_f32_32x32x16_bf16 per block of 32 keys and wavefront, with the vector work of the softmax
 // between them.  At 64, where there are 8, that vector work does (busy 58 % of the time, the matrix pipe 39 %, either 78 %).
 //
-// The work split is that of prefill.hip (four wavefronts of 32 query rows share K / V in LDS: HPW
-// heads of one KV head times 4 / HPW row blocks; all row blocks of a (batch entry, head group) on one
-// XCD, heavy ones first).  The whole life of a workgroup behind its address set-up is one block of
+// The work split: four wavefronts of 32 query rows share K / V in LDS, four consecutive (row block, head) pairs of a KV head
+// (row_blocks in prefill_common.h); where a group's workgroups run says workgroup_place.  Five heads per KV head, 40 / 8 of 128: 6 x 32 rows behind
+// 7232 tokens 140 -> 60 us, 2 x 1152 tokens 50 -> 43, 1 x 224 behind 1216 26.6 -> 28.0 (all workgroups of a KV head read the same keys at once).  The whole life of a workgroup behind its address set-up is one block of
 // assembly, written by gen_prefill_stream.py, which documents the schedule and the state on entry.
 // Against the compiler-scheduled loop of prefill.hip on the same shapes (a whole pass): window of 1024
 // keys, 2 x 4096 tokens, 32 / 8 heads 160 -> 137 us; 4 x 2048 tokens, 16 / 16 heads 118 -> 98 us and 16 / 8
@@ -34,7 +34,7 @@ bool stream_serves(const PrefillArgs &a) {
 }
 
 int64_t stream_part_bytes(const PrefillArgs &a, int head_size) {
-  return a.pt && stream_serves(a) ? part_bytes(a, heads_per_workgroup(a), stream_split(head_size), head_size) : 0;
+  return a.pt && stream_serves(a) ? part_bytes(a, head_group_size(a), stream_split(head_size), head_size) : 0;
 }
 
 // Whether a block-float-8 pass reads bfloat16 copies, written by a launch in front of it, or expands blocks on their way into
@@ -56,17 +56,11 @@ bool stream_expands(const PrefillArgs &a, int head_size, int64_t room) {
   const bool splits = parts > 0 && parts <= room;
   // (a table has room for more keys than the chunk's: 8192 rows of it)
   const bool few = a.batch * a.keys_bound * a.hkv <= (a.keys_known ? 5120 : 8192);
-  const bool pays = (row_blocks > 1 && (readers > 2 || a.keys_bound >= 512)) || few || part_bytes(a, hpw, stream_split(head_size), head_size) > 0 || (readers > (splits ? 3 : 2) && a.keys_bound >= 512);
+  const bool pays = (row_blocks > 1 && (readers > 2 || a.keys_bound >= 512)) || few || part_bytes(a, head_group_size(a), stream_split(head_size), head_size) > 0 || (readers > (splits ? 3 : 2) && a.keys_bound >= 512);
   return pays && !(splits && readers <= 2);
 }
 
-int launch_stream_wide(const PrefillArgs &a, hipStream_t st) {
-  switch (heads_per_workgroup(a)) {
-    case 4: return launch_form<128, 4, kDenseWide>(a, st);
-    case 2: return launch_form<128, 2, kDenseWide>(a, st);
-    default: return launch_form<128, 1, kDenseWide>(a, st);
-  }
-}
+int launch_stream_wide(const PrefillArgs &a, hipStream_t st) { return launch_form<128, kDenseWide>(a, st); }
 
 int launch_stream(const PrefillArgs &a, int head_size, hipStream_t st) {
   switch (head_size) {

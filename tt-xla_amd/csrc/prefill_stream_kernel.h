@@ -95,9 +95,8 @@ constexpr int stream_v_ring(int d, bool wide) { return TTPA_STREAM_SLOTS(d, wide
 constexpr int stream_p_ring(int d, bool wide) { return 2 * stream_v_ring(d, wide); }
 constexpr int stream_lds_bytes(int d, bool wide) { return stream_p_ring(d, wide) + (wide ? TTPA_STREAM_SLOTS(d, wide) * kBlockKeys * 128 : 0); }
 
-template <int D, int HPW, int FORM>
+template <int D, int FORM>
 __global__ __launch_bounds__(256, stream_wgs_per_cu(D)) void prefill_stream_kernel(PrefillArgs a) {
-  constexpr int RPW = 4 / HPW;  // row blocks per workgroup
   constexpr bool PAGED = FORM == kPaged || FORM == kPaged32, WIDE = FORM == kDenseWide;
   using T = Tile<D>;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
@@ -110,29 +109,26 @@ __global__ __launch_bounds__(256, stream_wgs_per_cu(D)) void prefill_stream_kern
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int n = lane & 31, h = lane >> 5;
-  const int nqt = (a.sq + kRowsPerWave * RPW - 1) / (kRowsPerWave * RPW);
-  const int groups = a.hq / HPW;
+  const int nqt = (row_blocks(a) * a.head_group + 3) / 4;  // workgroups of a head group, one after the other in row blocks
   // The part is the slowest index: the workgroups of part 0, the only ones with work where the keys are few, are dealt over the
   // XCDs and CUs as in a launch that is not split.  (As the fastest index, they met on half of the CUs or a quarter: 256
   // workgroups over 512 keys 20.5 us, 16.3 this way.)
   const int part = PAGED ? blockIdx.y : 0;
-  const int xcd = wg & 7, slot = wg >> 3;
-  const int yl = quotient(a.by_spg, slot);
-  const int y = yl * 8 + xcd;
-  if (y >= a.batch * groups) return;  // grid is padded to a multiple of 8 groups
-  const int item0 = slot - yl * a.spg;
+  int y, item0;
+  if (!workgroup_place(a, wg, y, item0)) return;
   const int qt = nqt - 1 - item0;
   const int b = quotient(a.by_groups, y);
-  const int hq0 = (y - b * groups) * HPW;
+  const int hq0 = (y - b * a.by_groups.d) * a.head_group;
   const int hk = quotient(a.by_group_heads, hq0);
-  const int hq = hq0 + wave % HPW;
-  const int row0 = (qt * RPW + wave / HPW) * kRowsPerWave;  // first query row of the wavefront
+  const int row_block = quotient(a.by_head_group, 4 * qt + wave);
+  const int hq = hq0 + 4 * qt + wave - row_block * a.head_group;
+  const int row0 = row_block * kRowsPerWave;  // first query row of the wavefront
   const int offset = a.causal ? chunk_offset(a.chunk_start, a.sq, a.skv) : 0;
 
   // keys the workgroup can see, in blocks of 32
-  const int wg_last_row = min(a.sq, (qt + 1) * kRowsPerWave * RPW) - 1;
+  const int wg_last_row = min(a.sq, (last_row_block(a, qt) + 1) * kRowsPerWave) - 1;
   const int kv_end = a.causal ? min(a.skv, offset + wg_last_row + 1) : a.skv;
-  int first_block = FORM == kDenseWindow ? max(0, offset + qt * kRowsPerWave * RPW - a.window + 1) / kBlockKeys : 0;
+  int first_block = FORM == kDenseWindow ? max(0, offset + quotient(a.by_head_group, 4 * qt) * kRowsPerWave - a.window + 1) / kBlockKeys : 0;
   // (at least one: the loop counts blocks down to zero.  Where no row sees a key, a chunk that starts at a negative
   // position, block 0 is read and masked, and the rows come out as NaN, softmax over nothing)
   int nblk = __builtin_amdgcn_readfirstlane(max((kv_end + kBlockKeys - 1) / kBlockKeys - first_block, 1));
@@ -230,9 +226,9 @@ __global__ __launch_bounds__(256, stream_wgs_per_cu(D)) void prefill_stream_kern
     else if constexpr (D == 64) asm volatile(TTPA_STREAM_FIRST_PAGED32_64);
     else if constexpr (D == 128) asm volatile(TTPA_STREAM_FIRST_PAGED32_128);
     else asm volatile(TTPA_STREAM_FIRST_PAGED32_256);
-    if (!whole) {
-      const PartLayout lay = part_layout(a, kRowsPerWave * RPW);
-      const int64_t at = (((int64_t)part * a.batch + b) * a.hq + hq) * lay.row_blocks + qt * RPW + wave / HPW;
+    if (!whole && row0 < a.sq) {
+      const PartLayout lay = part_layout(a);
+      const int64_t at = (((int64_t)part * a.batch + b) * a.hq + hq) * lay.row_blocks + row_block;
       out_part.acc = uni(reinterpret_cast<uint64_t>(a.part_acc + at * part_acc_floats(D)));
       out_part.stats = uni(reinterpret_cast<uint64_t>(a.part_acc + lay.slots * part_acc_floats(D) + at * (2 * kRowsPerWave)));
     }
@@ -305,65 +301,53 @@ __global__ __launch_bounds__(256, stream_wgs_per_cu(D)) void prefill_stream_kern
   else asm volatile(TTPA_STREAM_LOOP_PAGED32_256);
 }
 
-template <int D, int HPW, int FORM>
+template <int D, int FORM>
 int launch_form(const PrefillArgs &a, hipStream_t st) {
-  constexpr int RPW = 4 / HPW, lds = stream_lds_bytes(D, FORM == kDenseWide);
-  const int nqt = (a.sq + kRowsPerWave * RPW - 1) / (kRowsPerWave * RPW);
+  constexpr int lds = stream_lds_bytes(D, FORM == kDenseWide);
+  constexpr bool PAGED = FORM == kPaged || FORM == kPaged32;
   static std::atomic<uint64_t> lds_ready{0};
-  if (!ensure_dynamic_lds(reinterpret_cast<const void *>(&prefill_stream_kernel<D, HPW, FORM>), lds, lds_ready))
+  if (!ensure_dynamic_lds(reinterpret_cast<const void *>(&prefill_stream_kernel<D, FORM>), lds, lds_ready))
     return fail(TTPA_ERR_LAUNCH, "prefill: cannot reserve %d bytes of LDS", lds);
-  const int ny8 = (a.batch * (a.hq / HPW) + 7) / 8;
   PrefillArgs b = a;
+  b.spg_even = 0, b.parts = 1;
+  const int heads = head_group_size(a);
   // One workgroup per row block and head group, heavy blocks first, and the dispatcher deals them to the CUs
   // as slots free up: the loop can also give a workgroup several row blocks (spg workgroups per group,
   // TTPA_PREFILL_WGS_PER_GROUP), but one round of two workgroups per CU measured 204 us against 150 on
   // the 4 x 2048-token causal workload (a change of row block costs a workgroup about 4 us in which
   // nothing of its own overlaps, and a static deal cannot make up for workgroups that start late).
-  b.spg = nqt, b.spg_even = 0;
-  b.parts = 1;
-  constexpr bool PAGED = FORM == kPaged || FORM == kPaged32;
-  constexpr bool ITEMS = D == 128 && HPW == 4 && (FORM == kDense || FORM == kPaged);  // the loop can go on with another row block
+  const bool items = D == 128 && heads == 4 && (FORM == kDense || FORM == kPaged);  // the loop can go on with another row block
   // (read on every call) an experiment's override: several row blocks per workgroup, each over all of its keys
-  const char *e = ITEMS ? getenv("TTPA_PREFILL_WGS_PER_GROUP") : nullptr;
+  const char *e = items ? getenv("TTPA_PREFILL_WGS_PER_GROUP") : nullptr;
   const int per_group = e ? atoi(e) : 0;
-  if (PAGED && per_group <= 0 && a.part_acc && a.part_bytes >= part_bytes(a, HPW, stream_split(D), D)) set_parts(b, HPW, stream_split(D));
+  if (PAGED && per_group <= 0 && a.part_acc && a.part_bytes >= part_bytes(a, heads, stream_split(D), D)) set_parts(b, heads, stream_split(D));
+  int grid = lay_out(b, heads);
   if (per_group > 0) {
-    b.spg = std::min(nqt, per_group);
-  } else if (ITEMS && b.parts == 1) {
+    grid = lay_out(b, heads, std::min(b.spg, per_group));
+  } else if (items && b.parts == 1) {
     // Row blocks of nearly one weight (a chunk far into its sequence, or no causal mask) that fill the
     // chip more than once: one round of workgroups with equal shares instead, which saves the later
     // rounds' start-up (267 -> 261 us on 4 x 512-token chunks behind 4096 tokens, 64 heads).  The
     // chunk's start is in device memory, so the kernel decides: the workgroups past the round exit.
     int cus = device_cus();
     if (cus <= 0) cus = 256;
-    const int one_round = (2 * cus + ny8 * 8 - 1) / (ny8 * 8);
-    b.spg_even = one_round < nqt && nqt % one_round == 0 ? one_round : 0;
+    const int groups = a.batch * (a.hq / heads), one_round = (2 * cus + groups - 1) / groups;
+    b.spg_even = one_round < b.spg && b.spg % one_round == 0 ? one_round : 0;
   }
-  b.by_spg = divisor(b.spg), b.by_groups = divisor(a.hq / HPW), b.by_group_heads = divisor(a.hq / a.hkv);
-  int grid = b.spg * ny8 * 8;
   if (!PAGED && FORM != kDenseWide && a.fill_kc) grid = grid_with_fill(b, grid, D);
-  launch_dominant(&prefill_stream_kernel<D, HPW, FORM>, dim3(grid, b.parts), dim3(256), (size_t)lds, st, b);
+  launch_dominant(&prefill_stream_kernel<D, FORM>, dim3(grid, b.parts), dim3(256), (size_t)lds, st, b);
   if (const int rc = check_launch("sdpa_prefill")) return rc;
   if (b.parts > 1) {
-    prefill_merge_kernel<D, RPW><<<dim3((b.sq + kRowsPerWave - 1) / kRowsPerWave, b.hq, b.batch), dim3(2 * D), 0, st>>>(b);
+    prefill_merge_kernel<D><<<dim3((b.sq + kRowsPerWave - 1) / kRowsPerWave, b.hq, b.batch), dim3(2 * D), 0, st>>>(b);
     return check_launch("sdpa_prefill (merge of the parts)");
   }
   return TTPA_OK;
 }
 
-template <int D, int HPW>
-int launch_heads(const PrefillArgs &a, hipStream_t st) {
-  if (a.pt) return a.bs % kKeysPerTile == 0 ? launch_form<D, HPW, kPaged>(a, st) : launch_form<D, HPW, kPaged32>(a, st);
-  return a.window > 0 ? launch_form<D, HPW, kDenseWindow>(a, st) : launch_form<D, HPW, kDense>(a, st);
-}
-
 template <int D>
 int launch_stream_d(const PrefillArgs &a, hipStream_t st) {
-  switch (heads_per_workgroup(a)) {
-    case 4: return launch_heads<D, 4>(a, st);
-    case 2: return launch_heads<D, 2>(a, st);
-    default: return launch_heads<D, 1>(a, st);
-  }
+  if (a.pt) return a.bs % kKeysPerTile == 0 ? launch_form<D, kPaged>(a, st) : launch_form<D, kPaged32>(a, st);
+  return a.window > 0 ? launch_form<D, kDenseWindow>(a, st) : launch_form<D, kDense>(a, st);
 }
 
 }  // namespace
