@@ -46,9 +46,8 @@ reads, the first fragments of K block i + 2 and V block i.  Its barrier, at its 
 nobody reads K block i and V block i - 2 any more; K block i + NS and V block i + NS - 2 are
 requested into their slots (LDS-DMA loads, two per tensor and wavefront).  A request has to have
 landed NS - 2 barriers later: the wait in front of a barrier lets the requests of the last NS - 3
-barriers stay in flight (vmcnt(8)), so a tile has three iterations to arrive with NS = 5, where
-two stages of whole tiles gave it two.  Once requests have been skipped (no such block) the wait
-is for everything.  Dense K / V: a block is `stride` bytes behind the one before.  Paged (block
+barriers stay in flight (vmcnt(8), less near the end, where there are fewer), so a tile has three iterations to arrive with NS = 5, where
+two stages of whole tiles gave it two.  Dense K / V: a block is `stride` bytes behind the one before.  Paged (block
 size a multiple of 64): two blocks are a tile, a tile lies in one cache block; the table entry of
 the tile K enters two iterations from now is requested in front of the tile requests of every
 odd iteration (so the same wait covers it) and read at the next odd one.  Entries outside
@@ -73,9 +72,9 @@ key blocks.  The launcher's default is one item per workgroup (spg = nqt: the ha
 workgroups as slots free up, which measured faster than one static round), several when the row
 blocks weigh the same and divide evenly over one round.  (Only where the four wavefronts share their
 rows, and not with a window, whose row blocks start at different keys.)  Per item the block does everything
-between the Q fragments and the stored output rows: its first requests (K blocks 0..NS-1, V blocks
-0..NS-3; for the first item they are a block of assembly of their own, so that the caller's Q loads
-overlap them), all blocks, the last PV, normalisation and store; then the next item's Q fragments
+between the Q rows and the stored output rows: its first requests (K blocks 0..NS-1, V blocks
+0..NS-3; for the first item they are a block of assembly of their own, one block less of each, in front of the
+caller's set-up), all blocks, the last PV, normalisation and store; then the next item's Q fragments
 and first requests go out in front of the store of the finished one.
 
 Matrix-to-vector hazards the hardware does not interlock are kept by construction: the vector
@@ -121,7 +120,8 @@ class Registers:
         self.PTREQ2 = take(1)                      # blocks of 32: the entry requested in odd iterations
         self.LIMIT = take(1)                       # last visible key of the lane's row, minus 4 h
         self.LIMREL, self.NEGINF, self.VZERO = (take(1) for _ in range(3))
-        self.QBASE, self.OUTBASE = take(2), take(2)  # per lane, 64-bit: q / out of row 0 of the lane's head, at the lane's 8 h elements
+        # items: per lane, 64-bit: q / out of row 0 of the lane's head, at the lane's 8 h elements
+        self.QBASE, self.OUTBASE = take(2), take(2)
         self.VN, self.V4H = take(1), take(1)       # lane % 32 and 4 (lane / 32)
         self.OUTP, self.PTMP = take(2), take(2)
         self.VT0, self.VROW = take(1), take(1)
@@ -166,6 +166,9 @@ S_QTS, S_OTS = "s48", "s49"    # bytes from a query / output row to the next
 # and 4 (later: the next two V blocks), s[86:87] the K block's; S_TPB, S_CIN, S_RIN count 32-key blocks
 S_ROW0 = "s57"                 # first query row of the item
 S_STOREMASK = "s[60:61]"
+# LDS offset of the slot with the wavefront's Q rows; LDS offset and address of the slot its output rows go through; output of the
+# wavefront's head, row 0
+S_QSLOT, S_OUTSLOT, S_OUTADDR, S_OUT = "s25", "s26", "s27", "s[28:29]"
 # temporaries s[88:95], s[62:63]
 
 PSLOT = 4096                   # bytes of a block of the second part of K
@@ -529,18 +532,24 @@ def next_block(o, f, p, tag):
     o.label(f"L_noreq_{tag}")
 
 
+def in_flight(f, left):
+    """Loads of the ns - 3 iterations in front of one with `left` blocks left (itself among them): iteration j has requested K block
+    j + ns and V block j + ns - 2 if they exist."""
+    k, v = f.loads - f.tensor_loads, f.tensor_loads
+    return sum(k * (left > f.ns - back) + v * (left > f.ns - 2 - back) for back in range(1, f.ns - 2))
+
+
 def iteration_head(o, f, p, tag):
     """Mask, barrier and requests of iteration i = p (mod f.unroll)."""
     paged, ns = f.paged, f.ns
     mask_block(o, f, p % 2, tag)
-    # requests of the last ns - 3 barriers may stay in flight, unless some were skipped
-    o.e(f"s_cmp_eq_u32 {S_KLEFT}, 0")
-    o.e(f"s_cbranch_scc1 L_all_{tag}%=")
-    o.e(f"s_waitcnt vmcnt({(ns - 3) * f.loads})")
-    o.e(f"s_branch L_bar_{tag}%=")
-    o.label(f"L_all_{tag}")
-    o.e("s_waitcnt vmcnt(0)")
-    o.label(f"L_bar_{tag}")
+    # requests of the last ns - 3 iterations may stay in flight; near the end they are fewer.  (Iteration 0 needs blocks that have landed
+    # in front of it.)  A wait for everything from the last K request on cost a workgroup three waits of half a memory trip.
+    if tag != "i0":
+        o.e(f"s_cmp_ge_u32 {S_NB}, {ns}")
+        o.e(f"s_cbranch_scc0 L_few_{tag}%=")
+        o.e(f"s_waitcnt vmcnt({in_flight(f, ns)})")
+        o.label(f"L_bar_{tag}")
     o.e("s_barrier")
     if paged == 64 and (p + ns) % 2 == 0:
         next_tile(o, f, tag)
@@ -553,6 +562,19 @@ def iteration_head(o, f, p, tag):
     if paged == 32:
         o.e("s_mov_b64 s[84:85], s[98:99]")
         o.e("s_mov_b64 s[98:99], s[86:87]")
+
+
+def few_left(o, f, tag):
+    """The wait of an iteration with less than ns blocks left."""
+    o.label(f"L_few_{tag}")
+    for left in range(1, f.ns - 1):
+        o.e(f"s_cmp_lg_u32 {S_NB}, {left}")
+        o.e(f"s_cbranch_scc1 L_few{left}_{tag}%=")
+        o.e(f"s_waitcnt vmcnt({in_flight(f, left)})")
+        o.e(f"s_branch L_bar_{tag}%=")
+        o.label(f"L_few{left}_{tag}")
+    o.e(f"s_waitcnt vmcnt({in_flight(f, f.ns - 1)})")
+    o.e(f"s_branch L_bar_{tag}%=")
 
 
 def iteration_tail(o, f, tag, exit_label):
@@ -573,8 +595,9 @@ def item_setup(o, f, tag):
     """Per-item state from S_ROW0: output pointers, the rows' key limits, the mask threshold, cleared
     accumulators and softmax state."""
     o.e(f"v_add_u32 v{f.VROW}, {S_ROW0}, v{f.VN}")                                   # the lane's query row
-    o.e(f"v_mad_u64_u32 v[{f.OUTP}:{f.OUTP + 1}], s[92:93], v{f.VROW}, {S_OTS}, v[{f.OUTBASE}:{f.OUTBASE + 1}]")
-    o.e(f"v_cmp_gt_i32_e64 {S_STOREMASK}, {S_SQ}, v{f.VROW}")                      # rows that exist are stored
+    if f.items:
+        o.e(f"v_mad_u64_u32 v[{f.OUTP}:{f.OUTP + 1}], s[92:93], v{f.VROW}, {S_OTS}, v[{f.OUTBASE}:{f.OUTBASE + 1}]")
+        o.e(f"v_cmp_gt_i32_e64 {S_STOREMASK}, {S_SQ}, v{f.VROW}")                  # rows that exist are stored
     o.e(f"s_sub_u32 s88, {S_SQ}, 1")
     o.e(f"v_min_i32 v{f.VT0}, s88, v{f.VROW}")                                       # rows past the end repeat the last one
     o.e(f"v_add_u32 v{f.VT0}, {S_OFFSET}, v{f.VT0}")
@@ -612,10 +635,10 @@ def item_blocks(o):
     o.e(f"s_mov_b32 {S_VLEFT}, {S_NB}")
 
 
-def epilogue(o, f):
-    """Normalises the item's accumulators and stores its rows: lane (n, h) holds, in accumulator
-    register 16 db + 4 j + i, head-dim element 32 db + 8 j + 4 h + i of query row n.  The output pointer
-    of lane (n, h) is row n's plus 16 h bytes."""
+def normalise(o, f):
+    """Normalises the item's accumulators and packs them: lane (n, h) holds, in accumulator
+    register 16 db + 4 j + i, head-dim element 32 db + 8 j + 4 h + i of query row n, and ends with 16-byte chunk 4 db + 2 jp + h
+    of the row in registers S[0] + 8 db + 4 jp ..."""
     o.e(f"v_mov_b32 v{f.MB}, v{f.LRUN}")
     o.e("s_nop 1")
     o.e(f"v_permlane32_swap_b32 v{f.LRUN}, v{f.MB}")
@@ -635,14 +658,19 @@ def epilogue(o, f):
                 o.e(f"v_mul_f32 v{t[k]}, v{f.ALPHA}, v{t[k]}")
             o.e(f"v_cvt_pk_bf16_f32 v{f.S[0] + i}, v{t[0]}, v{t[1]}")
     o.e("s_nop 1")
-    # The two lanes of a row trade halves, so that each stores 16 consecutive bytes (a row's 32 bytes per
-    # instruction): lane (n, 0) keeps its block j and takes (n, 1)'s, lane (n, 1) ends with both blocks j + 1.
+    # The two lanes of a row trade halves, so that each holds 16 consecutive bytes: lane (n, 0) keeps its block j and
+    # takes (n, 1)'s, lane (n, 1) ends with both blocks j + 1.
     for db in range(f.d // 32):
         for jp in range(2):
             x = f.S[0] + 8 * db + 4 * jp
             o.e(f"v_permlane32_swap_b32 v{x}, v{x + 2}")
             o.e(f"v_permlane32_swap_b32 v{x + 1}, v{x + 3}")
     o.e("s_nop 3")
+
+
+def direct_store(o, f):
+    """From the lanes as they are, a row's 32 bytes per instruction (the rings belong to the next item already).  The output pointer of
+    lane (n, h) is row n's plus 16 h bytes."""
     o.e(f"s_and_saveexec_b64 s[62:63], {S_STOREMASK}")
     o.e("s_nop 1")
     for db in range(f.d // 32):
@@ -650,6 +678,66 @@ def epilogue(o, f):
             src = f.S[0] + 8 * db + 4 * jp
             o.e(f"global_store_dwordx4 v[{f.OUTP}:{f.OUTP + 1}], v[{src}:{src + 3}], off offset:{64 * db + 32 * jp} nt")   # written once, read by a later kernel
     o.e("s_mov_b64 exec, s[62:63]")
+    o.e("s_nop 1")
+
+
+def store_rows(o, f):
+    """The packed rows through LDS, so that a store writes whole rows (1 KiB) and not 32 bytes of each of 32 rows: a short pass waited
+    0.85 us for those.  Slot w of the K ring (nobody reads it behind the last barrier) takes the 32 rows of wavefront w in the layout of a K
+    block: chunk 2 s + h of row n lies where the lane's K fragment s does."""
+    rpi, chunks = 512 // f.d, f.d // 8  # rows per instruction, 16-byte chunks per row
+    swizzle = lambda r: r & 15 if f.d >= 128 else r >> 1 & 7
+    for s in range(f.d // 16):
+        o.e(f"v_add_u32 v{f.T[s % 4]}, {S_OUTSLOT}, v{f.KOFF + s}")
+        o.e(f"ds_write_b128 v{f.T[s % 4]}, {vr(f.S[0] + 4 * s, 4)}")
+    # lane l reads and stores chunk l % chunks of row rpi i + l / chunks
+    lane, row, off = f.LIMREL, f.VROW, f.VT0
+    o.e(f"v_lshl_add_u32 v{lane}, v{f.V4H}, 3, v{f.VN}")
+    o.e(f"v_lshrrev_b32 v{row}, {chunks.bit_length() - 1}, v{lane}")
+    o.e(f"v_and_b32 v{off}, {chunks - 1}, v{lane}")
+    if f.d >= 128:
+        o.e(f"v_xor_b32 v{f.MB}, v{off}, v{row}")
+    else:
+        o.e(f"v_lshrrev_b32 v{f.MB}, 1, v{row}")
+        o.e(f"v_xor_b32 v{f.MB}, v{off}, v{f.MB}")
+    o.e(f"v_lshlrev_b32 v{f.MB}, 4, v{f.MB}")
+    o.e(f"v_lshl_add_u32 v{f.MB}, v{row}, {(2 * f.d).bit_length() - 1}, v{f.MB}")
+    o.e(f"v_add_u32 v{f.MB}, {S_OUTADDR}, v{f.MB}")
+    n = 32 // rpi
+    for i in range(n):
+        x = 16 * swizzle(rpi * i)
+        if x:
+            o.e(f"v_xor_b32 v{f.T[i % 4]}, 0x{x:x}, v{f.MB}")
+        o.e(f"ds_read_b128 {vr(f.S[0] + 4 * i, 4)}, v{f.T[i % 4] if x else f.MB} offset:{1024 * i}")
+    o.e(f"v_add_u32 v{f.MCN}, {S_ROW0}, v{row}")
+    o.e(f"v_mov_b32 v{f.PTMP}, s28")
+    o.e(f"v_mov_b32 v{f.PTMP + 1}, s29")
+    o.e(f"v_mad_u64_u32 v[{f.PTMP}:{f.PTMP + 1}], s[92:93], v{f.MCN}, {S_OTS}, v[{f.PTMP}:{f.PTMP + 1}]")
+    o.e(f"v_mad_u64_u32 v[{f.PTMP}:{f.PTMP + 1}], s[92:93], v{off}, 16, v[{f.PTMP}:{f.PTMP + 1}]")
+    o.e(f"s_mul_hi_u32 s89, {S_OTS}, {rpi}")
+    o.e(f"s_mul_i32 s88, {S_OTS}, {rpi}")
+    o.e(f"s_sub_u32 s94, {S_SQ}, {S_ROW0}")                       # rows that exist
+    o.e("s_mov_b64 s[62:63], exec")
+    o.e("s_cmp_lt_i32 s94, 32")
+    o.e("s_cbranch_scc1 L_some_rows%=")
+    for some in (False, True):
+        for i in range(n):
+            if some:
+                o.e(f"v_cmp_gt_i32_e64 s[92:93], s94, v{row}")
+                o.e(f"s_sub_u32 s94, s94, {rpi}")
+            o.e(f"s_waitcnt lgkmcnt({min(n - 1 - i, 15)})" if not some or i == 0 else "s_nop 0")
+            if some:
+                o.e("s_mov_b64 exec, s[92:93]")
+                o.e("s_nop 1")
+            o.e(f"global_store_dwordx4 v[{f.PTMP}:{f.PTMP + 1}], {vr(f.S[0] + 4 * i, 4)}, off nt")   # written once, read by a later kernel
+            if some:
+                o.e("s_mov_b64 exec, s[62:63]")
+            o.e(f"v_lshl_add_u64 v[{f.PTMP}:{f.PTMP + 1}], v[{f.PTMP}:{f.PTMP + 1}], 0, s[88:89]")
+        if not some:
+            o.e("s_branch L_stored%=")
+            o.label("L_some_rows")
+            o.e("s_waitcnt lgkmcnt(0)")
+    o.label("L_stored")
     o.e("s_nop 1")
 
 
@@ -677,7 +765,8 @@ def last_epilogue(o, f):
     if f.parts:
         o.e(f"s_cmp_lg_u64 {S_PART}, 0")
         o.e("s_cbranch_scc1 L_partial%=")
-    epilogue(o, f)
+    normalise(o, f)
+    store_rows(o, f)
     if f.parts:
         o.e("s_branch L_done%=")
         o.label("L_partial")
@@ -724,9 +813,10 @@ def next_item(o, f):
     else:
         o.e("s_mov_b64 s[64:65], s[50:51]")
         o.e("s_mov_b64 s[66:67], s[52:53]")
-    for ln in generate_first(f, "nx"):
+    for ln in generate_first(f, "nx", f.ns):
         o.lines.append(ln)
-    epilogue(o, f)
+    normalise(o, f)
+    direct_store(o, f)
     item_setup(o, f, "nx")
     o.e("s_branch L_item_top%=")
     o.label("L_last_item")
@@ -741,47 +831,36 @@ def first_offsets(f):
     return ["s[50:51]", "s[52:53]"] + (["s[58:59]"] if f.ns == 5 else []) + [S_OFFV, S_OFF0]
 
 
-def generate_first(f, suffix=""):
-    """The first requests: K blocks 0 .. ns - 1, V blocks 0 .. ns - 3 (a block of its own, so that
-    the caller can put its Q loads behind them)."""
+def first_request(o, f, which, j, tag):
+    """K or V block j, one of the first, into slot j."""
+    if not f.paged:
+        request_block(o, f, which, j, tag, 0)
+        return
+    left, lane, base, ring = (S_KLEFT, f.LDK, 64, 0) if which == "K" else (S_VLEFT, f.LDV, 66, f.vring)
+    lo = int(first_offsets(f)[j // 2 if f.paged == 64 else j][2:4])
+    o.e(f"s_cmp_eq_u32 {left}, 0")
+    o.e(f"s_cbranch_scc1 L_no{which}_{tag}%=")
+    o.e(f"s_add_u32 s90, s{base}, s{lo}")
+    o.e(f"s_addc_u32 s91, s{base + 1}, s{lo + 1}")
+    if j % 2 and f.paged == 64:
+        o.e(f"s_add_u32 s90, s90, {f.SLOT}")
+        o.e("s_addc_u32 s91, s91, 0")
+    o.e(f"s_add_u32 m0, {S_M0B}, {ring + j * f.SLOT}")
+    o.e("s_nop 0")
+    block_loads(o, f, lane, "s[90:91]")
+    o.e(f"s_sub_u32 {left}, {left}, 1")
+    o.label(f"L_no{which}_{tag}")
+
+
+def generate_first(f, suffix="", blocks=0):
+    """The first requests: K blocks 0 .. blocks - 1, V blocks 0 .. blocks - 3 (a block of assembly of its own, so that the caller can
+    put its set-up behind them).  At first ns - 1: the slots of the next ones, and those that no V block is in yet, hold Q rows."""
     o = Out()
-    paged = f.paged
-    for j in range(f.ns):
-        if paged:
-            src = first_offsets(f)[j // 2 if paged == 64 else j]
-            lo = int(src[2:4])
-            o.e(f"s_cmp_eq_u32 {S_KLEFT}, 0")
-            o.e(f"s_cbranch_scc1 L_noK_pro{j}{suffix}%=")
-            o.e(f"s_add_u32 s90, s64, s{lo}")
-            o.e(f"s_addc_u32 s91, s65, s{lo + 1}")
-            if j % 2 and paged == 64:
-                o.e(f"s_add_u32 s90, s90, {f.SLOT}")
-                o.e("s_addc_u32 s91, s91, 0")
-            o.e(f"s_add_u32 m0, {S_M0B}, {j * f.SLOT}")
-            o.e("s_nop 0")
-            block_loads(o, f, f.LDK, "s[90:91]")
-            o.e(f"s_sub_u32 {S_KLEFT}, {S_KLEFT}, 1")
-            o.label(f"L_noK_pro{j}{suffix}")
-        else:
-            request_block(o, f, "K", j, f"pro{j}{suffix}", 0)
-    for j in range(f.ns - 2):
-        if paged:
-            src = first_offsets(f)[j // 2 if paged == 64 else j]
-            lo = int(src[2:4])
-            o.e(f"s_cmp_eq_u32 {S_VLEFT}, 0")
-            o.e(f"s_cbranch_scc1 L_noV_pro{j}{suffix}%=")
-            o.e(f"s_add_u32 s90, s66, s{lo}")
-            o.e(f"s_addc_u32 s91, s67, s{lo + 1}")
-            if j % 2 and paged == 64:
-                o.e(f"s_add_u32 s90, s90, {f.SLOT}")
-                o.e("s_addc_u32 s91, s91, 0")
-            o.e(f"s_add_u32 m0, {S_M0B}, {f.vring + j * f.SLOT}")
-            o.e("s_nop 0")
-            block_loads(o, f, f.LDV, "s[90:91]")
-            o.e(f"s_sub_u32 {S_VLEFT}, {S_VLEFT}, 1")
-            o.label(f"L_noV_pro{j}{suffix}")
-        else:
-            request_block(o, f, "V", j, f"pro{j}{suffix}", 0)
+    blocks = blocks or f.ns - 1
+    for j in range(blocks):
+        first_request(o, f, "K", j, f"pro{j}{suffix}")
+    for j in range(blocks - 2):
+        first_request(o, f, "V", j, f"pro{j}{suffix}")
     return o.lines
 
 
@@ -790,9 +869,22 @@ def generate(f):
     assert (f.ns, f.unroll) in ((5, 10), (4, 4))
     o.e(f"v_mov_b32 v{f.VZERO}, 0")
     item_setup(o, f, "first")
-    o.label("L_item_top")
+    # The Q rows of wavefront w lie, in the layout of a K block, in the slot of K block ns - 1 or of V blocks ns - 3 ...: fragment ks at
+    # the lane's K fragment's place.  Once all wavefronts have them, the blocks of those slots are requested.
     o.e("s_waitcnt vmcnt(0)")
+    for ks in range(f.d // 16):
+        o.e(f"v_add_u32 v{f.T[ks % 4]}, {S_QSLOT}, v{f.KOFF + ks}")
+        o.e(f"ds_read_b128 {vr(f.QF + 4 * ks, 4)}, v{f.T[ks % 4]}")
+    o.e("s_waitcnt lgkmcnt(0)")
     o.e("s_barrier")
+    first_request(o, f, "K", f.ns - 1, "late")
+    first_request(o, f, "V", f.ns - 3, "late")
+    if f.items:
+        o.e("s_branch L_start%=")
+        o.label("L_item_top")
+        o.e("s_waitcnt vmcnt(0)")
+        o.e("s_barrier")
+        o.label("L_start")
     # ---- S(0) from K block 0; behind it the fragments of iteration 0 (K block 1) ------------------
     pairs = score_pairs(0, 0, f)
     it0 = iteration_pairs(0, f, has_pv=False)
@@ -848,6 +940,7 @@ def generate(f):
     slow_path(o, f, 0, "L_slow_i0", "L_join_i0", first=True)
     for p in range(f.unroll):
         slow_path(o, f, p % 2, f"L_slow_p{p}", f"L_join_p{p}")
+        few_left(o, f, f"p{p}")
     o.label("L_end")
     o.e("s_nop 15")
     o.e("s_nop 15")
@@ -878,10 +971,12 @@ def operands(f):
         first = counts, loads + [i(*b) for b in bases] + [i(S_M0B, "req.m0_base")] + [i(*x) for x in offs]
     else:
         first = [io(*b) for b in bases] + counts + wide_io, loads + [i(S_STRIDE, "req.stride"), i(S_M0B, "req.m0_base")] + wide_in
-    outs = [io(f.QF + 16 * k, f"q[{k}]", 16) for k in range(f.d // 64)] + [io(*b) for b in bases] + counts + wide_io
+    outs = [io(*b) for b in bases] + counts + wide_io
     outs += [io(S_NB, "nblk"), io(S_K, "it.k"), io(S_ROW0, "it.row0"), io(S_KEY0, "it.key0")]
     ins = [i(f.KOFF, "ko", f.d // 16), i(f.VOFF, "vo", f.d // 32)] + loads + wide_in
-    ins += [i(f.QBASE, "q_base", 2), i(f.OUTBASE, "out_base", 2), i(f.VN, "n"), i(f.V4H, "h4")]
+    ins += [i(f.VN, "n"), i(f.V4H, "h4"), i(S_QSLOT, "q_slot"), i(S_OUTSLOT, "out_slot"), i(S_OUTADDR, "out_address"), i(S_OUT, "out_row0")]
+    if f.items:
+        ins += [i(f.QBASE, "q_base", 2), i(f.OUTBASE, "out_base", 2)]
     ins += [i(S_STRIDE, "req.stride"), i(S_C, "a.scale_log2e"), i(S_M0B, "req.m0_base"), i(S_J, "it.j"), i(S_SPG, "it.spg"), i(S_NQT, "it.nqt"),
             i(S_SQ, "it.sq"), i(S_SKV, "it.skv"), i(S_OFFSET, "it.offset"), i(S_CAUSAL, "it.causal"), i(S_QTS, "it.q_row_bytes"),
             i(S_OTS, "it.out_row_bytes")]
@@ -895,6 +990,7 @@ def operands(f):
         ins += [i(S_HKV, "tab.kv_heads"), i(S_HK, "tab.kv_head"), i(S_NCB, "tab.num_blocks"), i(S_TPB, "tab.per_block"), i(S_STATS, "out_part.stats")]
         if f.paged == 32:
             outs += [io(f.PTREQ2, "tab.entry2")]
+            ins += [i(*offs[f.ns - 3])]
     if f.items and f.paged:  # where the items that follow start
         ins += [i(S_OFF0, "off[0]"), i("s[50:51]", "off[1]"), i("s[52:53]", "off[2]"), i("s54", "tab.entry"), i("s55", "tab.read_in_block"),
                 i("s56", "tab.request_in_block"), i("s[58:59]", "tab.entry_ptr")]

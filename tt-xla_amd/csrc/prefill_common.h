@@ -22,18 +22,17 @@ typedef uint32_t u32x16 __attribute__((ext_vector_type(16)));
 constexpr int kKeysPerTile = 64;
 constexpr int kRowsPerWave = 32;
 
-// x / d for 0 <= x < 2^31 without a division, which is a chain of about 30 vector instructions also where all operands are scalar:
-// magic = floor(2^32 / d) + 1 gives the quotient or, for large x d, one more.  The set-up of a workgroup has eight of them, two behind
+// x / d for 0 <= x < 2^31 without a division, which is a chain of about 30 vector instructions also where all operands are scalar, and without
+// a branch: magic = floor(2^32 / d) (one less for d = 1) gives the quotient or one less.  The set-up of a workgroup has eight of them, two behind
 // each other in front of its first request (a chunk of 32 rows behind 256 tokens, 8 / 8 heads of 64: 11.8 -> 11.2 us a pass).
 struct Divisor {
   int d;
   uint32_t magic;
 };
-inline Divisor divisor(int d) { return {d, d > 1 ? (uint32_t)((1ull << 32) / (uint32_t)d) + 1u : 0u}; }
+inline Divisor divisor(int d) { return {d, d > 1 ? (uint32_t)((1ull << 32) / (uint32_t)d) : ~0u}; }
 __device__ __forceinline__ int quotient(const Divisor &v, int x) {
-  if (v.d == 1) return x;
-  const int q = (int)__umulhi((uint32_t)x, v.magic);
-  return q - ((int64_t)q * v.d > x ? 1 : 0);
+  const uint32_t q = __umulhi((uint32_t)x, v.magic);
+  return (int)(q + ((uint32_t)x - q * (uint32_t)v.d >= (uint32_t)v.d ? 1u : 0u));
 }
 
 struct PrefillArgs {

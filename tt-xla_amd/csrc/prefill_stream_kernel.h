@@ -101,6 +101,12 @@ __global__ __launch_bounds__(256, stream_wgs_per_cu(D)) void prefill_stream_kern
   using T = Tile<D>;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
 
+  // The arguments that the set-up needs arrive as one batch (the compiler would wait for a first one to find the workgroup's place and then for
+  // a second: a trip of a short pass's few), and the chunk's start is asked for before anything else is worked out.
+  asm volatile("" ::"s"(a.q), "s"(a.k), "s"(a.v), "s"(a.pt), "s"(a.q_bs), "s"(a.q_hs), "s"(a.q_ts), "s"(a.pt_rs), "s"(a.out), "s"(a.out_bs),
+               "s"(a.out_hs), "s"(a.out_ts), "s"(a.scale_log2e));
+  if constexpr (!PAGED) asm volatile("" ::"s"(a.kv_bs), "s"(a.kv_hs), "s"(a.kv_ts));
+  const int offset = a.causal ? chunk_offset(a.chunk_start, a.sq, a.skv) : 0;
   int wg = blockIdx.x;
   if constexpr (!PAGED && !WIDE) {
     wg = attention_workgroup<D>(a, wg);
@@ -123,7 +129,6 @@ __global__ __launch_bounds__(256, stream_wgs_per_cu(D)) void prefill_stream_kern
   const int row_block = quotient(a.by_head_group, 4 * qt + wave);
   const int hq = hq0 + 4 * qt + wave - row_block * a.head_group;
   const int row0 = row_block * kRowsPerWave;  // first query row of the wavefront
-  const int offset = a.causal ? chunk_offset(a.chunk_start, a.sq, a.skv) : 0;
 
   // keys the workgroup can see, in blocks of 32
   const int wg_last_row = min(a.sq, (last_row_block(a, qt) + 1) * kRowsPerWave) - 1;
@@ -167,6 +172,19 @@ __global__ __launch_bounds__(256, stream_wgs_per_cu(D)) void prefill_stream_kern
     lane_v[j] = (uint32_t)r * (WIDE ? 2u * (uint32_t)a.v_ts : row_bytes) + 16u * (uint32_t)(cp ^ T::swz_v(r)) + 1024u - 1024u * j;
   }
   const auto ldk = Words<LOADS>::of(lane_k), ldv = Words<LOADS>::of(lane_v);
+  // The wavefront's 32 Q rows, whole rows per load, go to the slot that K block ns - 1 (wavefront 0) or V block ns - 4 + wave takes later,
+  // in the layout of a K block.  Loaded to registers by the lanes that hold them, 32 bytes of each of 32 rows per instruction, they cost a short pass
+  // 0.65 us more.
+  constexpr int SLOTS = TTPA_STREAM_SLOTS(D, WIDE);
+  const int q_slot = (wave == 0 ? SLOTS - 1 : 2 * SLOTS - 4 + wave) * (kBlockKeys * T::RB);
+  {
+    const uint16_t *qp = a.q + b * a.q_bs + hq * a.q_hs;
+#pragma unroll
+    for (int j = 0; j < kRowsPerWave / T::RPI; ++j) {
+      const int r = j * T::RPI + lane / T::CPR;
+      dma16_lane(qp + (int64_t)min(row0 + r, a.sq - 1) * a.q_ts + 8 * ((lane % T::CPR) ^ T::swz_k(r)), uni(lds0 + q_slot + 1024u * j));
+    }
+  }
   StreamWide wide;
   uint32_t ldp = 0;
   if constexpr (WIDE) {
@@ -197,7 +215,7 @@ __global__ __launch_bounds__(256, stream_wgs_per_cu(D)) void prefill_stream_kern
     // keys that share a table entry are a multiple of a unit (a 64-key tile, a 32-key block); the first FIRST
     // units are requested here, the loop takes raw entries from there on
     constexpr int UNIT = FORM == kPaged ? kKeysPerTile : kBlockKeys;
-    constexpr int SLOTS = TTPA_STREAM_SLOTS(D, false), FIRST = FORM == kPaged ? (SLOTS + 1) / 2 : SLOTS, RAW = FORM == kPaged ? 1 : 2;
+    constexpr int FIRST = FORM == kPaged ? (SLOTS + 1) / 2 : SLOTS, RAW = FORM == kPaged ? 1 : 2;
     const int per = a.bs / UNIT, last = a.w * per - 1;  // (entries exist for every unit of the table)
     const int unit0 = first_block * kBlockKeys / UNIT;
     auto column = [&](int unit) { return div_block(a, unit * UNIT); };
@@ -233,17 +251,6 @@ __global__ __launch_bounds__(256, stream_wgs_per_cu(D)) void prefill_stream_kern
       out_part.stats = uni(reinterpret_cast<uint64_t>(a.part_acc + lay.slots * part_acc_floats(D) + at * (2 * kRowsPerWave)));
     }
   }
-  // Q fragments behind the requests (B operand: lane n = query row, 8 head-dim elements per k-step)
-  u32x16 q[D / 64];
-  {
-    const int qrow = min(row0 + n, a.sq - 1);
-    const uint16_t *qp = a.q + b * a.q_bs + hq * a.q_hs + (int64_t)qrow * a.q_ts + 8 * h;
-#pragma unroll
-    for (int s = 0; s < D / 16; ++s) {
-      const uint4 x = *reinterpret_cast<const uint4 *>(qp + 16 * s);
-      q[s / 4][4 * (s % 4)] = x.x, q[s / 4][4 * (s % 4) + 1] = x.y, q[s / 4][4 * (s % 4) + 2] = x.z, q[s / 4][4 * (s % 4) + 3] = x.w;
-    }
-  }
   u32x16 q_second;
   u32x4 po;
   if constexpr (WIDE) {
@@ -276,7 +283,10 @@ __global__ __launch_bounds__(256, stream_wgs_per_cu(D)) void prefill_stream_kern
   it.q_row_bytes = uni(2u * (uint32_t)a.q_ts), it.out_row_bytes = uni(2u * (uint32_t)a.out_ts);
   it.row0 = __builtin_amdgcn_readfirstlane(row0);
   it.key0 = uni(first_block * kBlockKeys);
-  // per lane: row 0 of the lane's head, at the lane's 8 (lane / 32) / 4 (lane / 32) elements
+  const int out_slot = wave * (kBlockKeys * T::RB);
+  const uint32_t out_address = uni(lds0 + out_slot);
+  const uint64_t out_row0 = uni(reinterpret_cast<uint64_t>(a.out + b * a.out_bs + hq * a.out_hs));
+  // per lane: row 0 of the lane's head, at the lane's 8 (lane / 32) elements
   const uint64_t q_base = reinterpret_cast<uint64_t>(a.q + b * a.q_bs + hq * a.q_hs + 8 * h);
   const uint64_t out_base = reinterpret_cast<uint64_t>(a.out + b * a.out_bs + hq * a.out_hs + 8 * h);
   const int h4 = 4 * h;
