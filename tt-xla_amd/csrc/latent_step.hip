@@ -56,6 +56,7 @@ struct StepArgs {
   const void *pos;
   int pos_i64;
   int users, heads, bs, w, nb;
+  int tiles;  // blocks of 32 users per workgroup of latent_value_kernel
   // prompt: the rows are tokens, `seq` to a user, and belong to positions 0 .. seq - 1 of the users' table rows
   int seq, table_rows;
   uint16_t *k_lat;  // [rows][kRow]
@@ -89,11 +90,32 @@ __device__ __forceinline__ void load_columns(bf16x8 (&w)[8], const uint16_t *col
   for (int s = 0; s < 8; ++s) w[s] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(column + 16 * s));
 }
 
+// Activation rows travel memory -> LDS in whole rows of 256 bytes, four to an instruction, and results leave as whole rows: as 16 bytes of each of
+// 32 rows per instruction (8 bytes for the results), each wavefront for itself, they were half of the query's time (128 heads,
+// 75 users 14.9 -> 10.8 us; 16 heads, 128 users 7.6 -> 6.8; a prompt of 32 tokens of 16 heads 24.2 -> 22.8 for the whole pass).
+// 16-byte chunk c of row r lies at chunk position c ^ (r % 16): the lanes of a fragment read find their rows in different banks.
+constexpr int kRowPitch = 272;  // of result rows: 8-byte writes of 32 rows spread over the banks
+
+// Pieces first ... first + count - 1 (four rows each) of the 32 rows of 128 elements from user u0 on, `us` elements apart.  Users past the
+// last repeat it in the last piece, and nothing is read for further ones: a column of the products is a user's, and theirs are not stored.
+__device__ __forceinline__ void request_rows(const uint16_t *src, int64_t us, int u0, int users, unsigned char *rows, int first, int count) {
+  const int lane = threadIdx.x & 63;
+  for (int j = first; j < min(first + count, (users - u0 + 3) >> 2); ++j) {
+    const int r = 4 * j + (lane >> 4);
+    dma16_lane(src + min(u0 + r, users - 1) * us + 8 * ((lane & 15) ^ (r & 15)),
+               (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds_address(rows) + 1024u * (uint32_t)j)));
+  }
+}
+__device__ __forceinline__ bf16x8 read_row(const unsigned char *rows, int r, int chunk) {
+  return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(rows + r * 256 + 16 * (chunk ^ (r & 15))));
+}
+
 // COLUMNS: the weight's contracted dimension is contiguous (else its columns are).  PROMPT: the rows' latent keys go to a.k_lat
 // as well, in one piece for the attention.
 template <bool COLUMNS, bool PROMPT = false>
 __global__ __launch_bounds__(256) void latent_query_kernel(StepArgs a) {
   __shared__ __attribute__((aligned(1024))) unsigned char tile[COLUMNS ? 1024 : kNope * 256];  // 128 rows of 128 columns
+  __shared__ __attribute__((aligned(1024))) unsigned char rows[kUsers * kRowPitch];            // the users' query rows, then their result rows
   const int col0 = blockIdx.x * 128, head = blockIdx.y, u0 = blockIdx.z * kUsers;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -113,11 +135,7 @@ __global__ __launch_bounds__(256) void latent_query_kernel(StepArgs a) {
       dma16_uniform(w + (int64_t)(4 * seg) * a.uk_ld, lane_bytes, lds_address(tile) + 1024u * (uint32_t)seg);
     }
   }
-  const int u = min(u0 + n, a.users - 1);
-  bf16x8 q[8];
-  const uint16_t *qp = a.q_nope + u * a.qn_us + head * a.qn_hs + 8 * h;
-#pragma unroll
-  for (int s = 0; s < 8; ++s) q[s] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(qp + 16 * s));
+  request_rows(a.q_nope + head * a.qn_hs, a.qn_us, u0, a.users, rows, 2 * wave, 2);
 
   if (blockIdx.x == 0) {  // the rotary part of the query, as it is: 8 chunks per user
     const int v = u0 + (tid >> 3), c = 8 * (tid & 7);
@@ -144,10 +162,11 @@ __global__ __launch_bounds__(256) void latent_query_kernel(StepArgs a) {
       *reinterpret_cast<uint4 *>(a.cache + ((int64_t)phys * a.bs + row) * kRow + at) = piece;
     }
   }
-  if constexpr (!COLUMNS) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's segments have landed
-    __syncthreads();
-  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's rows and segments have landed
+  __syncthreads();
+  bf16x8 q[8];
+#pragma unroll
+  for (int s = 0; s < 8; ++s) q[s] = read_row(rows, n, 2 * s + h);
 
   floatx16 acc;
 #pragma unroll
@@ -162,65 +181,82 @@ __global__ __launch_bounds__(256) void latent_query_kernel(StepArgs a) {
     else w = read_transposed(first + s * 16 * 256, 4 * 256);
     acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, q[s], acc, 0, 0, 0);
   }
-  if (u0 + n >= a.users) return;
-  uint16_t *dst = a.q_lat + ((int64_t)(u0 + n) * a.heads + head) * kRow + col0 + 32 * wave + 4 * h;
+  __syncthreads();  // everybody has its query rows
 #pragma unroll
   for (int j = 0; j < 4; ++j)
-    *reinterpret_cast<uint2 *>(dst + 8 * j) = make_uint2(pack_bf16x2(acc[4 * j], acc[4 * j + 1]), pack_bf16x2(acc[4 * j + 2], acc[4 * j + 3]));
+    *reinterpret_cast<uint2 *>(rows + n * kRowPitch + 64 * wave + 16 * j + 8 * h) =
+        make_uint2(pack_bf16x2(acc[4 * j], acc[4 * j + 1]), pack_bf16x2(acc[4 * j + 2], acc[4 * j + 3]));
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kUsers / 16; ++i) {
+    const int v = 16 * i + (tid >> 4), c = tid & 15;
+    if (u0 + v < a.users)
+      *reinterpret_cast<uint4 *>(a.q_lat + ((int64_t)(u0 + v) * a.heads + head) * kRow + col0 + 8 * c) =
+          *reinterpret_cast<const uint4 *>(rows + v * kRowPitch + 16 * c);
+  }
 }
 
+// A workgroup takes a.tiles blocks of 32 users: the weight goes to registers once, and the rows of the next block are on their way while
+// one is worked on.  128 heads, 75 users: 21.0 us with one block per workgroup (the weights read once per 32 users, three rounds of
+// workgroups), 12.9.  (The query's kernel, which writes more than it reads, lost by the same: 10.8 / 16.2 us.)
 template <bool COLUMNS>
 __global__ __launch_bounds__(256) void latent_value_kernel(StepArgs a) {
   constexpr int kPitch = 36;  // floats of a user's partial sums: rows of 16-byte writes in different banks
-  __shared__ __attribute__((aligned(1024))) unsigned char tile[COLUMNS ? 1024 : kLatent * 64];  // 512 rows of 32 columns, 128 per wavefront
-  __shared__ __attribute__((aligned(16))) float sums[4][kUsers * kPitch];
-  const int col0 = blockIdx.x * 32, head = blockIdx.y, u0 = blockIdx.z * kUsers;
+  // Per wavefront 128 latent values of the users, then its partial sums, in two buffers in turn; the second holds the weight at first (512 rows
+  // of 32 columns, 128 per wavefront), until it is in registers.
+  __shared__ __attribute__((aligned(1024))) unsigned char buffer[2][4][kUsers * 256];
+  static_assert(kUsers * kPitch * 4 <= kUsers * 256, "a wavefront's sums take its rows' place");
+  const int col0 = blockIdx.x * 32, head = blockIdx.y, first_user = blockIdx.z * a.tiles * kUsers;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, h = lane >> 5;
   // weights: 8 segments of sixteen 64-byte rows per wavefront (four rows of a transposing read are 256 consecutive bytes)
-  bf16x8 columns[8];
+  bf16x8 w[8];
   if constexpr (COLUMNS) {
-    load_columns(columns, a.w_uv + head * a.uv_hs + (int64_t)(col0 + n) * a.uv_ld + 128 * wave + 8 * h);
+    load_columns(w, a.w_uv + head * a.uv_hs + (int64_t)(col0 + n) * a.uv_ld + 128 * wave + 8 * h);
   } else {
-    const uint16_t *w = a.w_uv + head * a.uv_hs + (int64_t)(128 * wave) * a.uv_ld + col0;
+    const uint16_t *weight = a.w_uv + head * a.uv_hs + (int64_t)(128 * wave) * a.uv_ld + col0;
     const uint32_t lane_bytes = (uint32_t)(lane >> 2) * (uint32_t)(2 * a.uv_ld) + 16u * (uint32_t)(lane & 3);
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      dma16_uniform(w + (int64_t)(16 * j) * a.uv_ld, lane_bytes, lds_address(tile) + 8192u * (uint32_t)wave + 1024u * j);
+    for (int j = 0; j < 8; ++j) dma16_uniform(weight + (int64_t)(16 * j) * a.uv_ld, lane_bytes, lds_address(buffer[1][wave]) + 1024u * j);
   }
-  const int u = min(u0 + n, a.users - 1);
-  bf16x8 o[8];
-  const uint16_t *op = a.o_lat + ((int64_t)u * a.heads + head) * kLatent + 128 * wave + 8 * h;
+  auto request = [&](int t) {
+    request_rows(a.o_lat + (int64_t)head * kLatent + 128 * wave, (int64_t)a.heads * kLatent, first_user + t * kUsers, a.users, buffer[t & 1][wave], 0, 8);
+  };
+  request(0);
+  const int tiles = min(a.tiles, (a.users - first_user + kUsers - 1) / kUsers);
+  for (int t = 0; t < tiles; ++t) {
+    const int u0 = first_user + t * kUsers;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // a wavefront reads the rows and segments that it requested
+    if (!COLUMNS && t == 0) {
+      const int grp = lane >> 4, a16 = lane & 15;
+      const unsigned char *first = buffer[1][wave] + (8 * (grp >> 1) + (a16 >> 2)) * 64 + 32 * (grp & 1) + 8 * (a16 & 3);
 #pragma unroll
-  for (int s = 0; s < 8; ++s) o[s] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(op + 16 * s));
-  if constexpr (!COLUMNS) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // a wavefront reads the segments that it requested
-
-  floatx16 acc;
+      for (int s = 0; s < 8; ++s) w[s] = read_transposed(first + s * 16 * 64, 4 * 64);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+    if (t + 1 < tiles) request(t + 1);  // (its buffer: the weight is in registers, the sums of block t - 1 were read in front of a barrier)
+    floatx16 acc;
 #pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-  const int grp = lane >> 4, a16 = lane & 15;
-  const unsigned char *first = tile + 8192 * wave + (8 * (grp >> 1) + (a16 >> 2)) * 64 + 32 * (grp & 1) + 8 * (a16 & 3);
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
 #pragma unroll
-  for (int s = 0; s < 8; ++s) {
-    bf16x8 w;
-    if constexpr (COLUMNS) w = columns[s];
-    else w = read_transposed(first + s * 16 * 64, 4 * 64);
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, o[s], acc, 0, 0, 0);
+    for (int s = 0; s < 8; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[s], read_row(buffer[t & 1][wave], n, 2 * s + h), acc, 0, 0, 0);
+    auto sums = [&](int k) { return reinterpret_cast<float *>(buffer[t & 1][k]); };
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      *reinterpret_cast<float4 *>(sums(wave) + n * kPitch + 8 * j + 4 * h) = make_float4(acc[4 * j], acc[4 * j + 1], acc[4 * j + 2], acc[4 * j + 3]);
+    __syncthreads();
+    const int v = tid >> 3, c = 4 * (tid & 7);
+    float4 x = *reinterpret_cast<const float4 *>(sums(0) + v * kPitch + c);
+#pragma unroll
+    for (int k = 1; k < 4; ++k) {
+      const float4 y = *reinterpret_cast<const float4 *>(sums(k) + v * kPitch + c);
+      x.x += y.x, x.y += y.y, x.z += y.z, x.w += y.w;
+    }
+    if (u0 + v < a.users)
+      *reinterpret_cast<uint2 *>(a.out + (u0 + v) * a.out_us + head * a.out_hs + col0 + c) = make_uint2(pack_bf16x2(x.x, x.y), pack_bf16x2(x.z, x.w));
+    if (t + 1 < tiles) __syncthreads();
   }
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-    *reinterpret_cast<float4 *>(&sums[wave][n * kPitch + 8 * j + 4 * h]) = make_float4(acc[4 * j], acc[4 * j + 1], acc[4 * j + 2], acc[4 * j + 3]);
-  __syncthreads();
-  const int v = tid >> 3, c = 4 * (tid & 7);
-  if (u0 + v >= a.users) return;
-  float4 t = *reinterpret_cast<const float4 *>(&sums[0][v * kPitch + c]);
-#pragma unroll
-  for (int k = 1; k < 4; ++k) {
-    const float4 x = *reinterpret_cast<const float4 *>(&sums[k][v * kPitch + c]);
-    t.x += x.x, t.y += x.y, t.z += x.z, t.w += x.w;
-  }
-  *reinterpret_cast<uint2 *>(a.out + (u0 + v) * a.out_us + head * a.out_hs + col0 + c) = make_uint2(pack_bf16x2(t.x, t.y), pack_bf16x2(t.z, t.w));
 }
 
 // K and V of a prompt, expanded per head, and the fill of the cache in the same launch (34 GFLOP at 8192 tokens of 16 heads, 75 MB
@@ -380,6 +416,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   else expand_item<false>(a, ring, head, part, row0);
 }
 
+// Blocks of 32 users per workgroup of latent_value_kernel, and how many workgroups share them: as many as keep two workgroups on every CU (their
+// LDS), one where that leaves CUs idle.
+inline unsigned lay_out_tiles(StepArgs &a) {
+  const int64_t tiles = (a.users + kUsers - 1) / kUsers, wgs = 4 * (int64_t)a.heads * tiles;
+  a.tiles = (int)std::min<int64_t>((wgs + 511) / 512, tiles);
+  return (unsigned)((tiles + a.tiles - 1) / a.tiles);
+}
+
 inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 }  // namespace
@@ -451,8 +495,7 @@ extern "C" int ttpa_latent_decode_step_strided(TTPA_LATENT_STEP_HEAD, int64_t w_
   a.pt = page_table, a.pt_rs = page_table_row_stride, a.pos = cur_pos, a.pos_i64 = cur_pos_is_i64;
   a.users = users, a.heads = heads, a.bs = block_size, a.w = table_width, a.nb = num_blocks;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const unsigned tiles = (unsigned)((users + kUsers - 1) / kUsers);
-  const dim3 query_grid(kLatent / 128, (unsigned)heads, tiles), value_grid(kValue / 32, (unsigned)heads, tiles);
+  const dim3 query_grid(kLatent / 128, (unsigned)heads, (unsigned)((a.users + kUsers - 1) / kUsers)), value_grid(kValue / 32, (unsigned)heads, lay_out_tiles(a));
   if (uk_columns) latent_query_kernel<true><<<query_grid, dim3(256), 0, st>>>(a);
   else latent_query_kernel<false><<<query_grid, dim3(256), 0, st>>>(a);
   if (int rc = check_launch("latent_decode_step (query)")) return rc;
@@ -545,8 +588,7 @@ extern "C" int ttpa_latent_prompt(void *out, int64_t out_token_stride, int64_t o
   a.k_lat = reinterpret_cast<uint16_t *>(ws);
   a.q_lat = reinterpret_cast<uint16_t *>(ws + align256((size_t)rows * kRow * 2));
   a.o_lat = reinterpret_cast<uint16_t *>(reinterpret_cast<unsigned char *>(a.q_lat) + align256((size_t)rows * heads * kRow * 2));
-  const unsigned tiles = (unsigned)((rows + kUsers - 1) / kUsers);
-  const dim3 query_grid(kLatent / 128, (unsigned)heads, tiles), value_grid(kValue / 32, (unsigned)heads, tiles);
+  const dim3 query_grid(kLatent / 128, (unsigned)heads, (unsigned)((a.users + kUsers - 1) / kUsers)), value_grid(kValue / 32, (unsigned)heads, lay_out_tiles(a));
   if (uk_columns) latent_query_kernel<true, true><<<query_grid, dim3(256), 0, st>>>(a);
   else latent_query_kernel<false, true><<<query_grid, dim3(256), 0, st>>>(a);
   if (int rc = check_launch("latent_prompt (query)")) return rc;
