@@ -389,7 +389,7 @@ int ttpa_sdpa_prefill_format(void *out, int64_t out_batch_stride, int64_t out_he
 /*
  * ttpa_sdpa_prefill_format with scratch memory from the caller.  With kv_format = TTPA_KV_BFP8 and
  * at least ttpa_sdpa_prefill_workspace_bytes(...) bytes of 16-byte aligned device memory, a pass
- * over head size 128, block_size a multiple of 32, no window and no mask, for which copies are the faster form (few rows in all,
+ * over head size 64 or 128, block_size a multiple of 32, no window and no mask, for which copies are the faster form (few rows in all,
  * several workgroups to a block, keys that can be split only that way or parts that find no room behind them),
  * first expands the block-float-8 blocks it will read into bfloat16 copies
  * in the scratch (one launch; the decode is exact, so the result is the same) and then runs the

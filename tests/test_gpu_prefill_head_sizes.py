@@ -9,6 +9,7 @@ import pytest
 import torch
 
 import test_gpu_prefill as P
+from oracle import bfp8_codec
 from oracle import paged_ops as O
 
 pytestmark = pytest.mark.gpu
@@ -74,3 +75,29 @@ def test_error_against_64_bits(d, window, monkeypatch):
         got = torch.ops.tt.scaled_dot_product_attention(q, k, v, is_causal=True, sliding_window_size=window or None)
         error[stream] = float((got.double() - exact).norm() / exact.norm())
     assert error["1"] <= 1.02 * error["0"], error
+
+
+@pytest.mark.parametrize("users,hq,hkv,bs,start,lc,copies", [
+    (1, 8, 8, 64, 100, 1024, True), (1, 8, 8, 32, 100, 1000, True), (1, 8, 8, 64, 100, 896, False),   # eight workgroups per head group, seven
+    (4, 8, 2, 32, 64, 256, True), (3, 8, 2, 32, 64, 256, False), (1, 64, 8, 64, 70, 250, True),        # 64 workgroups in all, 48
+])
+def test_block_float_8_chunks_of_64_features(monkeypatch, users, hq, hkv, bs, start, lc, copies):
+    """On either side of the line from which on a pass reads bfloat16 copies of its blocks."""
+    from tt_xla_amd import _native as N
+
+    g = torch.Generator().manual_seed(users + hq + lc)
+    nbpu = -(-(start + lc) // bs)
+    key, value, table = P._paged(g, users, nbpu, hkv, bs, 64, False)
+    q = P._bf(g, users, hq, lc, 64)
+    st = torch.tensor([start], dtype=torch.int32)
+    packed = [bfp8_codec.pack_cache(t) for t in (key, value)]
+    want = O.chunked_sdpa(q, *[bfp8_codec.unpack_cache(t, bs).to(torch.bfloat16) for t in packed], table, st, 0.125)
+    room = int(N.lib().ttpa_sdpa_prefill_workspace_bytes(users, hkv, 64, bs, nbpu, 1))
+    blocks = torch.zeros(room, dtype=torch.uint8, device="cuda")
+    call = N.call
+    monkeypatch.setattr(N, "call", lambda name, *a: call(name, *(a[:-3] + (blocks.data_ptr(), room, a[-1]) if name == "ttpa_sdpa_prefill_expanded" else a)))
+    got = torch.ops.tt.chunked_scaled_dot_product_attention(q.cuda(), packed[0].cuda(), packed[1].cuda(), table.cuda(), st.cuda(), 0.125)
+    # (the scratch starts with K's copy of block 0 of user 0, of a pass that is split with float accumulators)
+    k00 = bfp8_codec.unpack_cache(packed[0], bs).to(torch.bfloat16)[int(table[0, 0])]
+    assert torch.equal(blocks[: k00.numel() * 2].view(torch.bfloat16).cpu(), k00.flatten()) == copies
+    P._check(f"bfp8 u{users} h{hq}x{hkv} bs{bs} start{start} len{lc}", got.cpu(), want)

@@ -48,8 +48,16 @@ int64_t stream_part_bytes(const PrefillArgs &a, int head_size) {
 // 1 x 32 rows behind 512 tokens, 64 / 8 heads 23.1 / 18.8; 4 x 32 rows of 32 / 8 behind 1024 32.1 / 25.3, 4096 49.3 / 38.7; 8 x 128 of 16 / 16 behind
 // 4096 167 / 75.6; two row blocks: 4 x 64 of 32 / 8 behind 512 29.5 / 24.9, 8 x 256 of 16 / 16 behind 4096 195 / 128.  Four workgroups: 2 x 64 of
 // 64 / 8 behind 4096 49.5 / 55.6; three: 2 x 96 of 32 / 8 46.7 / 50.0.
+// At head size 64 mode 4 costs less per block and the copies as much: from eight workgroups per head group on, where the launch has 64.  8 / 8 heads,
+// 1 x 1024 rows behind 512 tokens 23.6 / 25.2, 4 x 1024 42.1 / 50.4; 64 / 8, 1 x 256 behind 2048 36.7 / 41.9, 8 x 448 behind 64 44.9 / 64.7; 8 / 2, 4 x 256
+// behind 64 14.2 / 16.6, 512 20.7 / 20.1, 8192 45.8 / 53.7; below either line: 8 / 8, 8 x 448 behind 512 35.2 / 35.4, 4 x 256 33.5 / 30.9; 64 / 8, 8 x 128 behind
+// 512 33.2 / 30.9; 8 / 2, 1 x 512 behind 512 19.2 / 18.3, 1 x 256 behind 8192 31.3 / 28.9.
 bool stream_expands(const PrefillArgs &a, int head_size, int64_t room) {
-  if (head_size != 128 || !stream_serves(a)) return false;
+  if (!stream_serves(a) || head_size == 256) return false;
+  if (head_size == 64) {
+    const int heads = head_group_size(a), per_group = ((a.sq + kRowsPerWave - 1) / kRowsPerWave * heads + 3) / 4;
+    return per_group >= 8 && (int64_t)a.batch * (a.hq / heads) * per_group >= 64;
+  }
   const int hpw = heads_per_workgroup(a), rows = kRowsPerWave * 4 / hpw;
   const int64_t row_blocks = (a.sq + rows - 1) / rows, readers = row_blocks * (a.hq / hpw / a.hkv);
   const int64_t parts = plain_part_bytes(a, head_size, true);
