@@ -262,9 +262,9 @@ __global__ __launch_bounds__(256) void latent_value_kernel(StepArgs a) {
 // K and V of a prompt, expanded per head, and the fill of the cache in the same launch (34 GFLOP at 8192 tokens of 16 heads, 75 MB
 // moved: 52 us, where two library products, a copy of W_UV, the fill and the gaps between them took 61).  Bound by the way of the
 // operands from L2 into LDS, about 44 bytes per ns and CU: without its products the launch takes 45 us.  A workgroup
-// computes 128 tokens x the 128 features of K or of V of a head, in steps of 32 latent values; both operands travel
-// memory -> LDS directly, 16 KiB per step, in a ring of four steps, one barrier per step; 64 KiB, so two workgroups share a CU.  A
-// half step's fragments are read while the products of the half before run.  A wavefront takes 64 x 64 as 2 x 2
+// computes 128 tokens x the 128 features of K or of V of a head, in steps of 32 or 64 latent values (ExpandShape); both operands travel
+// memory -> LDS directly, in a ring of four or two steps, one barrier per step; 64 KiB, so two workgroups share a CU.  A
+// slice's (16 values) fragments are read while the products of the slice before run.  A wavefront takes 64 x 64 as 2 x 2
 // v_mfma_f32_32x32x16_bf16 tiles, features as rows, tokens as columns; the results meet in LDS so that stores are whole rows (57 us
 // with 16 bytes per row and store).  Workgroups are ordered weights first: with the round-robin deal an XCD's L2 holds an
 // eighth of the weights, and the tokens pass through it.  Not better: 256 tokens x K and V per workgroup, with half the bytes
@@ -277,71 +277,100 @@ struct ExpandArgs {
   int items;                 // workgroups behind them write rows of the cache, 8 threads to a row
 };
 
-constexpr int kExpTokens = 128, kExpStep = 32, kExpStages = 4, kExpSteps = kLatent / kExpStep;
-constexpr int kExpHalf = 8192, kExpStage = 2 * kExpHalf;  // bytes of the tokens' and of the weight's part of a step
-constexpr int kExpPitch = 272;    // bytes of a result row in LDS: 8-byte writes of 32 rows spread over the banks
-static_assert(kExpTokens * kExpPitch <= kExpStages * kExpStage, "the results take the ring's place");
+// Steps of 64 latent values in a ring of two where the launch fills the chip: whole 128-byte lines per request instead of halves, which is
+// worth more there than three steps on their way (3 x 1984 tokens of 16 heads, the pass 118.2 / 114.5 us, 3 x 832 of 32 69.7 / 67.6, 1 x 1792 of
+// 16 50.2 / 49.6; 3 x 512 29.7 / 29.4; 2 x 416, which does not, 20.0 / 20.5, 1 x 96 12.4 / 12.9).  256 tokens per workgroup with steps of 32
+// or 64: 4 x 2048 the kernel alone 43.3 and 48.2 us against 45.4 and 41.7 (the two above), 1 x 480 9.7 and 10.3 against 6.2 and 8.1.
+constexpr int kExpTokens = 128;
+template <int STEP, int STAGES>
+struct ExpandShape {
+  static constexpr int kStep = STEP, kStages = STAGES, kSteps = kLatent / STEP;
+  static constexpr int kHalf = kExpTokens * STEP * 2, kStage = 2 * kHalf;  // bytes of the tokens' and of the weight's part of a step
+  static constexpr int kPitch = 272;  // bytes of a result row in LDS: 8-byte writes of 32 rows spread over the banks
+  static constexpr int kLds = kStages * kStage;
+  static constexpr int kPieces = kHalf / 1024 / 2;  // requests of a wavefront per step
+  static_assert(kExpTokens * kPitch <= kLds, "the results take the ring's place");
+};
 
-// Rows of 64 bytes (32 values of the contracted dimension): 16-byte chunk c of row r lies at chunk position c ^ (r / 4 % 4),
-// so the 16 lanes that LDS serves together find their chunks in different banks.
+// Rows of 2 STEP bytes: 16-byte chunk c of row r lies at chunk position c ^ (r / 4 % 4) (64 bytes) or c ^ (r / 2 % 8) (128), so the lanes that
+// LDS serves together find their chunks in different banks.
+template <int STEP>
+__device__ __forceinline__ int row_swizzle(int row) { return STEP == 32 ? (row >> 2) & 3 : (row >> 1) & 7; }
+template <int STEP>
 __device__ __forceinline__ bf16x8 read_row_chunk(const unsigned char *tile, int row, int chunk) {
-  return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(tile + row * 64 + 16 * (chunk ^ ((row >> 2) & 3))));
+  return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(tile + row * (2 * STEP) + 16 * (chunk ^ row_swizzle<STEP>(row))));
 }
 
 // part: 0 for K, 1 for V; ROWS: its weight's contracted dimension is contiguous.
-template <bool ROWS>
+template <class S, bool ROWS>
 __device__ __forceinline__ void expand_item(const ExpandArgs &a, unsigned char *ring, int head, int part, int row0) {
   const StepArgs &p = a.s;
+  constexpr int STEP = S::kStep;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-  // Requests: the first two wavefronts bring the tokens' part of a step, the others the weight's, 4 KiB each as four
-  // consecutive pieces.  Piece i of rows of 64 bytes holds rows 16 i ..., of rows of 256 bytes rows 4 i ...
-  const int first = 4 * (wave & 1);
+  // Requests: the first two wavefronts bring the tokens' part of a step, the others the weight's.  A piece is 1 KiB, whole rows of 2 STEP bytes
+  // or (a weight whose features are contiguous) four rows of 256.
   const bool weights = wave >= 2, by_row = !weights || ROWS;
+  const int first = S::kPieces * (wave & 1);
   const int64_t ld = part ? p.uv_ld : p.uk_ld;
   const uint16_t *weight = part ? p.w_uv + head * p.uv_hs : p.w_uk + head * p.uk_hs;
   const uint64_t at = reinterpret_cast<uint64_t>(weights ? weight : p.latent + row0 * p.latent_us);
   const unsigned char *base = reinterpret_cast<const unsigned char *>(
       address_from_words(__builtin_amdgcn_readfirstlane((int)(uint32_t)at), __builtin_amdgcn_readfirstlane((int)(uint32_t)(at >> 32))));
-  const int64_t step_bytes = by_row ? 2 * kExpStep : 2 * ld * kExpStep;
-  uint32_t lane_bytes[4];
+  const int64_t step_bytes = by_row ? 2 * STEP : 2 * ld * STEP;
+  uint32_t lane_bytes[S::kPieces];
   {
+    constexpr int kLanes = STEP / 8, kRows = 64 / kLanes;  // lanes per row, rows per piece
     const uint32_t pitch = (uint32_t)(weights ? 2 * ld : 2 * p.latent_us);
     const int last = weights ? kLatent : min(kExpTokens, p.users - row0) - 1;  // (rows behind the prompt repeat its last)
-    const int per = by_row ? 16 : 4, in = by_row ? lane >> 2 : lane >> 4;
-    const uint32_t chunk = by_row ? (lane & 3) ^ ((lane >> 4) & 3) : (lane & 15) ^ (4 * (lane >> 4));
+    const int per = by_row ? kRows : 4, in = by_row ? lane / kLanes : lane >> 4;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) lane_bytes[i] = (uint32_t)min(per * (first + i) + in, last) * pitch + 16u * chunk;
+    for (int i = 0; i < S::kPieces; ++i) {
+      const int r = per * (first + i) + in;
+      const uint32_t chunk = by_row ? (lane % kLanes) ^ row_swizzle<STEP>(r) : (lane & 15) ^ (4 * (lane >> 4));
+      lane_bytes[i] = (uint32_t)min(r, last) * pitch + 16u * chunk;
+    }
   }
-  const uint32_t to = lds_address(ring) + 1024u * (uint32_t)first + (weights ? kExpHalf : 0u);
+  const uint32_t to = lds_address(ring) + 1024u * (uint32_t)first + (weights ? (uint32_t)S::kHalf : 0u);
   auto request = [&](int step) {  // called for the steps in turn
-    const void *const bases[4] = {base, base - 1024, base - 2048, base - 3072};
-    dma16_quad(bases, lane_bytes, (uint32_t)__builtin_amdgcn_readfirstlane((int)(to + (uint32_t)(step % kExpStages) * kExpStage)));
+    const uint32_t dst = to + (uint32_t)(step % S::kStages) * S::kStage;
+#pragma unroll
+    for (int i = 0; i < S::kPieces; i += 4) {
+      const void *const bases[4] = {base, base - 1024, base - 2048, base - 3072};
+      const uint32_t lanes[4] = {lane_bytes[i], lane_bytes[i + 1], lane_bytes[i + 2], lane_bytes[i + 3]};
+      dma16_quad(bases, lanes, (uint32_t)__builtin_amdgcn_readfirstlane((int)(dst + 1024u * i)));
+    }
     base += step_bytes;
   };
 
   const int n = lane & 31, h = lane >> 5, grp = lane >> 4, a16 = lane & 15;
   const int f0 = 64 * (wave & 1), t0 = 64 * (wave >> 1);  // the wavefront's features and tokens
   const int trow = 8 * (grp >> 1) + (a16 >> 2), tchunk = f0 / 8 + 2 * (grp & 1) + ((a16 & 3) >> 1);
+  constexpr int kSlices = STEP / 16;  // products of a step
   floatx16 acc[2][2];
-  bf16x8 w[2][2], x[2][2];  // the fragments of a step's two halves
-  auto read = [&](int step, int half) {
-    const unsigned char *tokens = ring + step % kExpStages * kExpStage, *wtile = tokens + kExpHalf;
+  bf16x8 w[2][2], x[2][2];  // the fragments of two slices in turn
+  auto read = [&](int step, int slice) {
+    const unsigned char *tokens = ring + step % S::kStages * S::kStage, *wtile = tokens + S::kHalf;
+    const int to = slice & 1;
 #pragma unroll
-    for (int g = 0; g < 2; ++g) x[half][g] = read_row_chunk(tokens, t0 + 32 * g + n, 2 * half + h);
+    for (int g = 0; g < 2; ++g) x[to][g] = read_row_chunk<STEP>(tokens, t0 + 32 * g + n, 2 * slice + h);
 #pragma unroll
     for (int f = 0; f < 2; ++f)
-      if constexpr (ROWS) w[half][f] = read_row_chunk(wtile, f0 + 32 * f + n, 2 * half + h);
-      else w[half][f] = read_transposed(wtile + (16 * half + trow) * 256 + 16 * ((tchunk + 4 * f) ^ (4 * (trow & 3))) + 8 * (a16 & 1), 4 * 256);
+      if constexpr (ROWS) w[to][f] = read_row_chunk<STEP>(wtile, f0 + 32 * f + n, 2 * slice + h);
+      else w[to][f] = read_transposed(wtile + (16 * slice + trow) * 256 + 16 * ((tchunk + 4 * f) ^ (4 * (trow & 3))) + 8 * (a16 & 1), 4 * 256);
   };
   auto products = [&](int half) {
-    __builtin_amdgcn_sched_barrier(0);  // (the scheduler would put the reads of the other half behind these products)
+    __builtin_amdgcn_sched_barrier(0);  // (the scheduler would put the reads of the next slice behind these products)
 #pragma unroll
     for (int f = 0; f < 2; ++f)
 #pragma unroll
       for (int g = 0; g < 2; ++g) acc[f][g] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[half][f], x[half][g], acc[f][g], 0, 0, 0);
     __builtin_amdgcn_sched_barrier(0);
+  };
+  // at most `steps` steps' requests of this wavefront are still under way, and its reads have returned
+  auto wait = [&](auto steps) {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(decltype(steps)::value * S::kPieces) : "memory");
   };
 #pragma unroll
   for (int f = 0; f < 2; ++f)
@@ -350,27 +379,30 @@ __device__ __forceinline__ void expand_item(const ExpandArgs &a, unsigned char *
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[f][g][r] = 0.f;
 #pragma unroll
-  for (int step = 0; step < kExpStages; ++step) request(step);
-  asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+  for (int step = 0; step < S::kStages; ++step) request(step);
+  wait(std::integral_constant<int, S::kStages - 1>{});
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   read(0, 0);
 #pragma unroll
-  for (int step = 0; step < kExpSteps; ++step) {
-    read(step, 1);
-    products(0);
-    if (step + 1 < kExpSteps) {
+  for (int step = 0; step < S::kSteps; ++step) {
+#pragma unroll
+    for (int slice = 0; slice + 1 < kSlices; ++slice) {
+      read(step, slice + 1);
+      products(slice & 1);
+    }
+    if (step + 1 < S::kSteps) {
       // This wavefront's requests of the next step have landed and its reads of this one have returned; behind the
       // barrier that holds for everybody: the next step can be read, and this one's place filled.
-      if (step + 3 < kExpSteps) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
-      else if (step + 2 < kExpSteps) asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
-      else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      if (step + S::kStages - 1 < S::kSteps) wait(std::integral_constant<int, S::kStages - 2>{});
+      else if (step + 2 < S::kSteps && S::kStages > 3) wait(std::integral_constant<int, 1>{});
+      else wait(std::integral_constant<int, 0>{});
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
-      if (step + kExpStages < kExpSteps) request(step + kExpStages);
+      if (step + S::kStages < S::kSteps) request(step + S::kStages);
       read(step + 1, 0);
     }
-    products(1);
+    products((kSlices - 1) & 1);
   }
   // lane (n, h) holds features 8 j + 4 h ... + 3 of token n; the results meet in LDS so that stores are whole rows
   __syncthreads();
@@ -380,7 +412,7 @@ __device__ __forceinline__ void expand_item(const ExpandArgs &a, unsigned char *
     for (int g = 0; g < 2; ++g)
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        *reinterpret_cast<uint2 *>(ring + (t0 + 32 * g + n) * kExpPitch + 2 * (f0 + 32 * f + 8 * j + 4 * h)) =
+        *reinterpret_cast<uint2 *>(ring + (t0 + 32 * g + n) * S::kPitch + 2 * (f0 + 32 * f + 8 * j + 4 * h)) =
             make_uint2(pack_bf16x2(acc[f][g][4 * j], acc[f][g][4 * j + 1]), pack_bf16x2(acc[f][g][4 * j + 2], acc[f][g][4 * j + 3]));
   __syncthreads();
   uint16_t *out = (part ? a.v : a.k) + head * 128 + 8 * (tid & 15);
@@ -388,10 +420,11 @@ __device__ __forceinline__ void expand_item(const ExpandArgs &a, unsigned char *
   for (int i = 0; i < kExpTokens / 16; ++i) {
     const int r = (tid >> 4) + 16 * i;
     if (row0 + r < p.users)
-      *reinterpret_cast<uint4 *>(out + (int64_t)(row0 + r) * p.heads * 128) = *reinterpret_cast<const uint4 *>(ring + r * kExpPitch + 16 * (tid & 15));
+      *reinterpret_cast<uint4 *>(out + (int64_t)(row0 + r) * p.heads * 128) = *reinterpret_cast<const uint4 *>(ring + r * S::kPitch + 16 * (tid & 15));
   }
 }
 
+template <class S>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void latent_expand_kernel(ExpandArgs a) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char ring[];
   const StepArgs &p = a.s;
@@ -412,8 +445,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
   const int wt = 2 * p.heads, which = (int)blockIdx.x % wt, row0 = (int)blockIdx.x / wt * kExpTokens;
   const int head = which >> 1, part = which & 1;
-  if (part ? a.uv_rows : a.uk_rows) expand_item<true>(a, ring, head, part, row0);
-  else expand_item<false>(a, ring, head, part, row0);
+  if (part ? a.uv_rows : a.uk_rows) expand_item<S, true>(a, ring, head, part, row0);
+  else expand_item<S, false>(a, ring, head, part, row0);
+}
+
+template <class S>
+int launch_expand(ExpandArgs &e, hipStream_t st) {
+  static std::atomic<uint64_t> lds_ready{0};
+  if (!ensure_dynamic_lds(reinterpret_cast<const void *>(&latent_expand_kernel<S>), S::kLds, lds_ready))
+    return fail(TTPA_ERR_LAUNCH, "latent prompt: cannot configure the expansion kernel");
+  const int64_t groups = e.items + (e.s.cache ? ((int64_t)e.s.users + 31) / 32 : 0);
+  latent_expand_kernel<S><<<dim3((unsigned)groups), dim3(256), S::kLds, st>>>(e);
+  return check_launch("latent_prompt (expansion)");
 }
 
 // Blocks of 32 users per workgroup of latent_value_kernel, and how many workgroups share them: as many as keep two workgroups on every CU (their
@@ -572,13 +615,8 @@ extern "C" int ttpa_latent_prompt(void *out, int64_t out_token_stride, int64_t o
     e.k = reinterpret_cast<uint16_t *>(ws), e.v = reinterpret_cast<uint16_t *>(ws + align256((size_t)rows * heads * 256));
     e.uk_rows = !uk_columns, e.uv_rows = uv_columns;
     e.items = (int)(token_tiles * 2 * heads);
-    const int64_t groups = e.items + (cache ? (rows + 31) / 32 : 0);
-    constexpr size_t kLds = (size_t)kExpStages * kExpStage;
-    static std::atomic<uint64_t> lds_ready{0};
-    if (!ensure_dynamic_lds(reinterpret_cast<const void *>(&latent_expand_kernel), kLds, lds_ready))
-      return fail(TTPA_ERR_LAUNCH, "latent prompt: cannot configure the expansion kernel");
-    latent_expand_kernel<<<dim3((unsigned)groups), dim3(256), kLds, st>>>(e);
-    if (int rc = check_launch("latent_prompt (expansion)")) return rc;
+    const bool fills = e.items >= 384;  // (of 512 places)
+    if (int rc = fills ? launch_expand<ExpandShape<64, 2>>(e, st) : launch_expand<ExpandShape<32, 4>>(e, st)) return rc;
     const int64_t hd = (int64_t)heads * 128, sl = seq_len;
     return ttpa_split_key_prefill(out, sl * out_token_stride, out_head_stride, out_token_stride, q_nope, sl * q_nope_token_stride,
                                   q_nope_head_stride, q_nope_token_stride, q_rope, sl * q_rope_token_stride, q_rope_head_stride,
