@@ -60,6 +60,19 @@ def test_scores_that_force_a_rescale(d):
     P._check("rescale", got.cpu(), O.sdpa(q, k, v, None, True, None))
 
 
+@pytest.mark.parametrize("hq", [2, 4, 6, 8])
+@pytest.mark.parametrize("window", [31, 32, 33, 64, 100, 190])
+def test_window_scores_that_force_a_rescale(hq, window):
+    """The same behind a window's lower edge, with workgroups of several row blocks: rows whose first keys come blocks
+    after the workgroup's first have nothing to rescale, the others have it in the same wavefront."""
+    g = torch.Generator().manual_seed(window)
+    q, k, v = (torch.randn(1, h, 256, 256, generator=g) for h in (hq, 2, 2))
+    k = k + q[:, :: hq // 2].mean(2, keepdim=True) * torch.linspace(0, 6, 256).view(1, 1, 256, 1)
+    q, k, v = q.to(torch.bfloat16), k.to(torch.bfloat16), v.to(torch.bfloat16)
+    got = torch.ops.tt.scaled_dot_product_attention(q.cuda(), k.cuda(), v.cuda(), is_causal=True, sliding_window_size=window)
+    P._check(f"rescale h{hq} window{window}", got.cpu(), O.sdpa_windowed(q, k, v, sliding_window=window))
+
+
 @pytest.mark.parametrize("d,window", [(64, 0), (64, 300), (256, 0), (256, 300)])
 def test_error_against_64_bits(d, window, monkeypatch):
     g = torch.Generator().manual_seed(d + window)
