@@ -333,7 +333,7 @@ void paged_decode_mfma16_kernel(
       const u32x4 lo = fresh.part[0], hi = fresh.part[NF - 1];
       const uint32_t w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
       uint32_t out[4];
-      e = bfp8_encode16(w, out);
+      e = bfp8_encode16<D == 256>(w, out);
       val = u32x4{out[0], out[1], out[2], out[3]};
     }
 #pragma unroll
