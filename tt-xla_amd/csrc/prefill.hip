@@ -57,45 +57,70 @@ struct ExpandArgs {
   int64_t pt_rs;
   const int32_t *chunk_start;
   int batch, w, hkv, bs, nb, sq, causal;
+  Divisor by_pieces, by_slabs;  // pieces of a slab, slabs of a block
 };
 
+// Bound by memory.  A wavefront's piece is 64 groups in halves: 8 bytes of a half become 16, so that an instruction writes 1 KiB in
+// one piece; it asks for its next piece before it writes the one it has.  3 x 992 rows behind 1024 tokens of 8 heads of 128 (37 MB) 12.0 -> 9.4 us,
+// 3 x 1728 behind 4096 (110 MB) 27.3 -> 22.3, against a workgroup per slab in turn and 16 bytes of every 32 per store (10.2 and 26.3 with
+// whole groups); the passes 71.3 -> 68.5 and 272.6 -> 271.3, for of the copies that exceed the caches the attention waits for what is left
+// to write.
 template <int D>
 __global__ __launch_bounds__(256) void bfp8_expand_kernel(ExpandArgs e) {
   const int skv = e.w * e.bs;
   const int kv_end = e.causal ? min(skv, chunk_offset(e.chunk_start, e.sq, skv) + e.sq) : skv;
   const int cols = (kv_end + e.bs - 1) / e.bs;  // page-table columns that the pass reads
-  const int blocks = e.batch * cols, items = kv_end > 0 ? blocks * 2 * e.hkv : 0;
-  for (int item = blockIdx.x; item < items; item += gridDim.x) {
-    const int part = item / blocks, r = item - part * blocks;  // (K or V, KV head); block of the pass
-    const int b = r / cols, j = r - b * cols, x = b * e.w + j;
-    const int h = part >> 1;
-    const bool is_v = part & 1;
-    if (part == 0 && threadIdx.x == 0) e.table[x] = x;
+  const int pieces = kv_end > 0 ? e.batch * cols * e.by_slabs.d * e.by_pieces.d : 0;
+  const int lane = threadIdx.x & 63;
+  struct Piece {
+    uint2 bytes[2];
+    uint32_t exponent[2];
+    uint16_t *dst;
+  };
+  auto request = [&](int at) {
+    const int item = quotient(e.by_pieces, at), r = quotient(e.by_slabs, item);  // slab and block of the pass
+    const int part = item - r * e.by_slabs.d, b = r / cols, j = r - b * cols, x = b * e.w + j;
+    const bool is_v = part >= e.hkv;
+    const int h = part - (is_v ? e.hkv : 0), half = 128 * (at - item * e.by_pieces.d) + lane;
     int phys = e.pt[(int64_t)b * e.pt_rs + j];
     if ((unsigned)phys >= (unsigned)e.nb) phys = 0;  // (as the attention kernels treat a bad entry)
-    const int64_t slab = (int64_t)(e.bs + e.bs / 16) * D;
-    const uint8_t *src = (is_v ? e.vc : e.kc) + ((int64_t)phys * e.hkv + h) * slab;
-    const uint8_t *exps = src + (int64_t)e.bs * D;
-    uint16_t *dst = (is_v ? e.v : e.k) + ((int64_t)x * e.hkv + h) * e.bs * D;
-    const int groups = e.bs * D / 16;
-    for (int g = threadIdx.x; g < groups; g += 256) {
-      const u32x4 bytes = *reinterpret_cast<const u32x4 *>(src + 16 * g);
-      const float sc = bfp8_group_scale(exps[g]), off = -128.f * sc;
-      u32x4 lo, hi;
+    if (part == 0 && half == 0) e.table[x] = x;
+    const uint8_t *src = (is_v ? e.vc : e.kc) + ((int64_t)phys * e.hkv + h) * ((int64_t)(e.bs + e.bs / 16) * D);
+    Piece p;
 #pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        const uint32_t v = bytes[w];
+    for (int i = 0; i < 2; ++i) {
+      p.bytes[i] = *reinterpret_cast<const uint2 *>(src + 8 * (half + 64 * i));
+      p.exponent[i] = src[(int64_t)e.bs * D + (half + 64 * i) / 2];
+    }
+    p.dst = (is_v ? e.v : e.k) + ((int64_t)x * e.hkv + h) * e.bs * D + 8 * half;
+    return p;
+  };
+  const int step = (int)gridDim.x * 4;
+  int at = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  if (at >= pieces) return;
+  Piece p = request(at);
+  for (;;) {
+    at += step;
+    const bool more = at < pieces;
+    Piece next = p;
+    if (more) next = request(at);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const float sc = bfp8_group_scale(p.exponent[i]), off = -128.f * sc;
+      u32x4 out;
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {
+        const uint32_t v = w ? p.bytes[i].y : p.bytes[i].x;
         const float f0 = fmaf((float)(v & 0xffu), sc, off), f1 = fmaf((float)((v >> 8) & 0xffu), sc, off);
         const float f2 = fmaf((float)((v >> 16) & 0xffu), sc, off), f3 = fmaf((float)(v >> 24), sc, off);
         // the products are exact in bfloat16: their upper halves are the elements
-        const uint32_t p0 = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, f1), __builtin_bit_cast(uint32_t, f0), 0x07060302u);
-        const uint32_t p1 = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, f3), __builtin_bit_cast(uint32_t, f2), 0x07060302u);
-        if (w < 2) lo[2 * w] = p0, lo[2 * w + 1] = p1;
-        else hi[2 * (w - 2)] = p0, hi[2 * (w - 2) + 1] = p1;
+        out[2 * w] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, f1), __builtin_bit_cast(uint32_t, f0), 0x07060302u);
+        out[2 * w + 1] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, f3), __builtin_bit_cast(uint32_t, f2), 0x07060302u);
       }
-      *reinterpret_cast<u32x4 *>(dst + 16 * g) = lo;
-      *reinterpret_cast<u32x4 *>(dst + 16 * g + 8) = hi;
+      *reinterpret_cast<u32x4 *>(p.dst + 512 * i) = out;
     }
+    if (!more) return;
+    p = next;
   }
 }
 
@@ -688,10 +713,11 @@ int launch(const PrefillArgs &a, hipStream_t st) {
       e.table = reinterpret_cast<int32_t *>(e.v + cache_elems);
       e.pt = a.pt, e.pt_rs = a.pt_rs, e.chunk_start = a.chunk_start;
       e.batch = a.batch, e.w = a.w, e.hkv = a.hkv, e.bs = a.bs, e.nb = a.nb, e.sq = a.sq, e.causal = a.causal;
+      e.by_pieces = divisor(a.bs * D / 1024), e.by_slabs = divisor(2 * a.hkv);  // (blocks are multiples of 32 tokens: stream_serves)
       // armed events: the pair brackets both launches
       hipEvent_t before, after;
       take_profile_events(before, after);
-      const dim3 grid((unsigned)std::min<int64_t>(blocks * 2 * a.hkv, kExpandWorkgroups));
+      const dim3 grid((unsigned)std::min<int64_t>((blocks * 2 * a.hkv * e.by_pieces.d + 3) / 4, kExpandWorkgroups));
       if (before)
         hipExtLaunchKernelGGL(bfp8_expand_kernel<D>, grid, dim3(256), 0u, st, before, nullptr, 0u, e);
       else
