@@ -171,8 +171,29 @@ PyObject *attention_pass(PyObject *, PyObject *const *v, Py_ssize_t n) {
   const at::Tensor *fill = p.table(v[7]), *bidx = p.numbers(v[8], users);
   if (!fill || !bidx || fill->size(0) == 0 || s > fill->size(1) * bs) Py_RETURN_NONE;
   const int32_t *fill_pt = static_cast<const int32_t *>(fill->data_ptr());
+  const auto fill_caches = [&] {
+    RECORD_FUNCTION("tt::paged_fill_kv_cache_", std::vector<c10::IValue>());
+    const Unlocked unlocked;
+    return ttpa_paged_fill_cache_kv(
+        kc->data_ptr(), vc->data_ptr(), k->data_ptr(), val->data_ptr(), s * k->stride(0), d, k->stride(0), fill_pt, fill->stride(0),
+        bidx->data_ptr(), is_i64(bidx), (int32_t)users, (int32_t)fill->size(0), (int32_t)hkv, (int32_t)s, (int32_t)bs, (int32_t)d,
+        (int32_t)fill->size(1), (int32_t)nb, fmt, stream);
+  };
   if (v[9] == Py_None) {
-    if (bfp8 || s % 32) Py_RETURN_NONE;
+    if (s % 32) Py_RETURN_NONE;
+    if (bfp8) {  // (a quantising fill is a launch of its own)
+      written(kc), written(vc), written(out);
+      if (const int rc = fill_caches()) return result("ttpa_paged_fill_cache_kv", rc);
+      RECORD_FUNCTION("tt::scaled_dot_product_attention_out", std::vector<c10::IValue>());
+      const auto launch = [&] {
+        const Unlocked unlocked;
+        return ttpa_sdpa_prefill_expanded(
+            out->data_ptr(), s * hq * d, d, hq * d, q->data_ptr(), s * q->stride(0), d, q->stride(0), k->data_ptr(), val->data_ptr(),
+            s * k->stride(0), d, k->stride(0), nullptr, 0, nullptr, nullptr, 0, 0, (int32_t)users, (int32_t)hq, (int32_t)hkv, (int32_t)s,
+            (int32_t)s, (int32_t)d, 0, 0, 0, 1, scale, (int32_t)window, TTPA_KV_BF16, nullptr, 0, stream);
+      };
+      return result("ttpa_sdpa_prefill_expanded", launch());
+    }
     RECORD_FUNCTION("tt::paged_fill_kv_prefill_out_", std::vector<c10::IValue>());
     written(kc), written(vc), written(out);
     const auto launch = [&] {
@@ -193,17 +214,7 @@ PyObject *attention_pass(PyObject *, PyObject *const *v, Py_ssize_t n) {
                                                           (int32_t)pt->size(1), fmt, most_keys);
   if (bytes < 0 || bytes > kScratchLimit) bytes = 0;
   written(kc), written(vc), written(out);
-  {
-    RECORD_FUNCTION("tt::paged_fill_kv_cache_", std::vector<c10::IValue>());
-    const auto launch = [&] {
-      const Unlocked unlocked;
-      return ttpa_paged_fill_cache_kv(
-          kc->data_ptr(), vc->data_ptr(), k->data_ptr(), val->data_ptr(), s * k->stride(0), d, k->stride(0), fill_pt, fill->stride(0),
-          bidx->data_ptr(), is_i64(bidx), (int32_t)users, (int32_t)fill->size(0), (int32_t)hkv, (int32_t)s, (int32_t)bs, (int32_t)d,
-          (int32_t)fill->size(1), (int32_t)nb, fmt, stream);
-    };
-    if (const int rc = launch()) return result("ttpa_paged_fill_cache_kv", rc);
-  }
+  if (const int rc = fill_caches()) return result("ttpa_paged_fill_cache_kv", rc);
   RECORD_FUNCTION("tt::chunked_scaled_dot_product_attention_out", std::vector<c10::IValue>());
   const auto launch = [&] {
     const Unlocked unlocked;
