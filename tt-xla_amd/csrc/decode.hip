@@ -379,13 +379,24 @@ using namespace ttpa::decode;
 // 512 KB: 11.2 / 15.0).  Eight wavefronts hide more of a tile's chain (one user over 1024 block-float-8 tokens 18.2 / 15.2
 // with four / eight), but four leave room for two workgroups on a CU, which more segments than CUs need (296
 // segments of 128 tokens: 10.7 / 14.7); a segment of four tiles has no work for more.
+//
+// Head size 256 (tiles of 32 tokens, one wavefront per SIMD and so one workgroup of four per CU): as long as every segment has a CU,
+// up to a tile per wavefront, or two where at least half of the CUs have a segment and ranges are short of a second tile themselves.
+// us per layer, cut / whole, 16/8 heads: 64 tokens, one user 10.9 / 7.4, 16 users 12.2 / 8.5; 128 tokens, 5 users 12.1 / 9.5, 32 users
+// 15.6 / 11.4, block-float-8 14.6 / 11.0; 256 tokens, 16 users 15.5 / 13.1, 32 users 19.1 / 15.5, block-float-8 18.0 / 14.4; beyond:
+// 3 users 130 ... 250 tokens of 8/8 11.9 / 12.3, 5 users 384 12.6 / 15.0, 16 users 200 ... 510 16.9 / 18.3, 100 users 64 23.0 / 28.4.  Relative error
+// against 64 bits, whole over cut: 1 up to 128 tokens, 0.996 (28 passes of 150 ... 256 tokens, half of the CUs); few segments of 140 ... 192
+// tokens, 2 - 6 % faster, 1.003: a wavefront's second tile shares its first one's maximum.
+static int segment_tile_tokens(int head_size) { return head_size <= 128 ? 4096 / head_size : 32; }
 static int direct_waves(int users, int kv_heads, int head_size, int kv_format, int64_t tokens, bool forced) {
-  const int tile_tokens = 4096 / head_size;
-  const int64_t bytes = tokens * head_size * (kv_format == TTPA_KV_BFP8 ? 2 : 4);
-  if (!forced && bytes > 272 * 1024) return 0;
   int cus = device_cus();
   if (cus <= 0) cus = 256;
-  return (int64_t)users * kv_heads > cus || tokens <= 4 * tile_tokens ? 4 : 8;
+  const int64_t segments = (int64_t)users * kv_heads;
+  if (head_size > 128) return forced || (segments <= cus && tokens <= (2 * segments >= cus ? 256 : 128)) ? 4 : 0;
+  const int64_t bytes = tokens * head_size * (kv_format == TTPA_KV_BFP8 ? 2 : 4);
+  if (!forced && bytes > 272 * 1024) return 0;
+  const int tile_tokens = segment_tile_tokens(head_size);
+  return segments > cus || tokens <= 4 * tile_tokens ? 4 : 8;
 }
 
 // wavefronts per CU of the largest grid a decode launch uses (the VALU kernel on a block-float-8 cache)
@@ -524,7 +535,7 @@ static int decode_impl(void *out, int64_t out_user_stride, int64_t out_head_stri
   // Whole segments are for the groups that the kernel serves anyway: the attention alone over two or three heads per group of a
   // bfloat16 cache stays with the dot-product kernel, whose error against 64 bits is the smaller one (1.95e-3; whole segments
   // 2.03e-3 ... 2.13e-3, over 128 ... 1001 tokens).  (An explicit grid asks for ranges.)
-  if (!mask && use_mfma16 && head_size <= 128 && block_size % (4096 / head_size / 2) == 0 &&
+  if (!mask && use_mfma16 && block_size % (segment_tile_tokens(head_size) / 2) == 0 &&
       (forced == 5 || ((forced == 0 || forced == 3) && !getenv("TTPA_DECODE_WAVES_PER_CU")))) {
     int64_t tokens = (int64_t)table_width * block_size;
     if (sliding_window > 0) tokens = std::min<int64_t>(tokens, sliding_window);

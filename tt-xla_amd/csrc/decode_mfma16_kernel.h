@@ -702,8 +702,8 @@ template <int D, bool BFP8, bool FUSED>
 bool launch_form(const DecodeArgs &a, hipStream_t st) {
   constexpr bool kOneHead = !BFP8;  // one query head per KV head has kernels of its own
   const bool one = kOneHead && a.hq == a.hkv;
+  if (a.direct == 4) return one ? launch_runs<D, BFP8, FUSED, 4, false, kOneHead>(a, st) : launch_runs<D, BFP8, FUSED, 4, false, false>(a, st);
   if constexpr (D <= 128) {
-    if (a.direct == 4) return one ? launch_runs<D, BFP8, FUSED, 4, false, kOneHead>(a, st) : launch_runs<D, BFP8, FUSED, 4, false, false>(a, st);
     if (a.direct == 8) return one ? launch_runs<D, BFP8, FUSED, 8, false, kOneHead>(a, st) : launch_runs<D, BFP8, FUSED, 8, false, false>(a, st);
   }
   if constexpr (D == 128 && BFP8)
