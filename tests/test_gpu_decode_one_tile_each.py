@@ -1,0 +1,47 @@
+"""Decode at head size 256 on either side of the lists that have a range for every tile (three and four wavefronts per CU: 768 and 1024 tiles on 256
+CUs), of the group width and of the number of segments from which they do.  Outputs against the fp32 oracle, tolerance as in
+test_gpu_decode_units.py; the caller's grid of three per CU gives the same sums in other groups of tiles."""
+
+import pytest
+import torch
+
+import __graft_entry__ as entry
+from oracle import paged_ops as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _pkg():
+    entry.ensure_built()
+    import tt_xla_amd  # noqa: F401
+
+
+@pytest.mark.parametrize("hq,hkv,bs,pos,window", [
+    (16, 8, 32, [1535, 1535], 0), (16, 8, 32, [1535, 1536], 0), (16, 8, 64, [2047, 2047], 0), (8, 8, 32, [2047, 2048], 0),
+    (16, 8, 16, [2047, -1, 0, 2000], 0), (16, 8, 8, [1800, 1700], 0), (32, 8, 32, [1800, 1800], 0), (4, 4, 32, [2600, 2600], 0), (6, 3, 32, [2500] * 4, 0),
+    (16, 8, 32, [5119, 40, 3999, 2047], 1024), (16, 8, 32, [300 + 2 * i for i in range(11)], 0),
+])
+def test_one_tile_each(hq, hkv, bs, pos, window, monkeypatch):
+    gen = torch.Generator().manual_seed(hq + bs + len(pos) + max(pos))
+    users, width, d = len(pos), max(pos) // bs + 1, 256
+    k = torch.randn(width * 2, hkv, bs, d, generator=gen).to(torch.bfloat16)
+    v = torch.randn(width * 2, hkv, bs, d, generator=gen).to(torch.bfloat16)
+    table = torch.randint(0, width * 2, (users, width), generator=gen).to(torch.int32)
+    q = torch.randn(1, users, hq, d, generator=gen).to(torch.bfloat16)
+    cur = torch.tensor(pos, dtype=torch.int32)
+    print(f"one tile each h{hq}x{hkv} bs{bs} users{users} longest{max(pos)} window{window}", flush=True)
+
+    def step():
+        return torch.ops.tt.paged_scaled_dot_product_attention_decode(
+            q.cuda(), k.cuda(), v.cuda(), table.cuda(), is_causal=True, cur_pos_tensor=cur.cuda(), scale=d**-0.5,
+            sliding_window_size=window or None).cpu()
+
+    got = step()
+    monkeypatch.setenv("TTPA_DECODE_WAVES_PER_CU", "3")
+    three = step()
+    live = [u for u, p in enumerate(pos) if p >= 0]
+    assert got[:, [u for u in range(users) if u not in live]].isnan().all()
+    want = O.paged_sdpa_decode_windowed(q[:, live], k, v, table[live], cur[live], d**-0.5, window, None)
+    for t in (got, three):
+        torch.testing.assert_close(t[:, live].float(), want.reshape(t[:, live].shape).float(), atol=2e-2, rtol=2e-2)

@@ -46,8 +46,8 @@ struct DecodeArgs {
   // k_new / v_new [users][>= hkv heads][head_size] instead of the cache, and written to it.
   const uint16_t *k_new = nullptr, *v_new = nullptr;
   int64_t new_us, new_hs;
-  int few_ranges = 0;  // > 0: lists of fewer than `many_from` tiles are cut into that many ranges instead of n_waves
-  int64_t many_from = 0;
+  int few_ranges = 0;  // > 0: lists of `few_from` to fewer than `many_from` tiles are cut into that many ranges instead of n_waves
+  int64_t few_from = 0, many_from = 0;
   int long_tiles = 0;  // 16x16x32 kernel, block-float-8 at head size 128: tiles of 64 tokens instead of 32
   int direct = 0;  // wavefronts of the workgroup that owns a whole segment (16x16x32 kernel: the step, or the attention alone), or 0
   // Additive mask on the scaled scores (bfloat16, natural-log units), or null: the element for
@@ -153,12 +153,12 @@ __device__ inline void build_prefix(const DecodeArgs &a, const void *__restrict_
 // 146 ... 1229 50.1 / 36.7, 16 of 200 ... 3000 57.3 / 50.3, 7 of 1384 ... 7377 54.1 / 49.7; 32 heads, 6 of 500 ... 5000
 // 41.4 / 30.1; 16 heads, one user over 1000 27.9 / 21.3, 8 of 300 ... 3000 28.7 / 27.2.  With none throughout: 30 users of
 // 500 ... 4000, 128 heads 75.6 instead of 64.4 with three; one user over 16000, 16 heads 38.4 instead of 32.3.
-// FEW: n_ranges, a.n_waves on entry, becomes a.few_ranges for a short list (above 64 users by its units).
+// FEW: n_ranges, a.n_waves on entry, becomes a.few_ranges for a list of such a length (above 64 users by its units).
 template <int TILE = kTile, bool FEW = false>
 __device__ __forceinline__ int build_prefix_units(const DecodeArgs &a, const void *__restrict__ cur, int *pref, int *lens, int *wave_sums,
                                                   int &n_ranges) {
   const auto choose = [&](int64_t tiles) {
-    if (FEW && a.few_ranges > 0 && tiles < a.many_from) n_ranges = a.few_ranges;
+    if (FEW && a.few_ranges > 0 && tiles >= a.few_from && tiles < a.many_from) n_ranges = a.few_ranges;
   };
   if (a.seg_free_tiles < 0 || a.users > kWave) {
     build_prefix<TILE>(a, cur, pref, lens, wave_sums, a.seg_units);
@@ -558,7 +558,7 @@ inline int combine_pieces(int n, int slices) {
 // 32 users of 8/2 heads at head size 64 56.2 / 49.8 / 49.9, 16 users with 2048 tokens 117.5 / 117.1 / 119.9, 24 with
 // 1024 tokens 100.4 / 100.3 / 105.4: below eight the segments' workgroups fill the chip as they are, and cutting
 // them only makes more of them.  One user with 512 tokens, whose partials are one batch, 45.2 -> 44.1.
-inline bool combine_sliced(const DecodeArgs &a, int segments) { return a.n_waves >= 8 * segments; }
+inline bool combine_sliced(const DecodeArgs &a, int segments) { return (a.few_from > 0 ? a.few_ranges : a.n_waves) >= 8 * segments; }
 
 // What the weights of the partials seen so far are relative to.  With an explicit mask they may all be fully
 // masked (maximum -inf) where their segment is not: their weights are zeros, not exp2(-inf + inf).
@@ -658,7 +658,7 @@ template <bool PARKED = false>
 inline void launch_combine(const DecodeArgs &a, int segments, int g, int d, hipStream_t st) {
   // (a block-float-8 list may have filled half of the ranges only: not where the slices' workgroups do not fit the chip at once, nine
   // per CU, either: 32 users of 32/8 heads, 3000 ... 24000 tiles, sliced / not 18.2 / 16.7 ... 48.2 / 46.8 us per layer; 18 users 17.4 / 17.1, 46.4 / 46.7)
-  const bool fits = a.few_ranges == 0 || (int64_t)segments * combine_pieces(g * d, kCombineSlices) <= 9 * 256;
+  const bool fits = a.few_ranges == 0 || a.few_from > 0 || (int64_t)segments * combine_pieces(g * d, kCombineSlices) <= 9 * 256;
   if (combine_sliced(a, segments) && fits)
     decode_combine_kernel<kCombineSlices, PARKED><<<dim3(segments, combine_pieces(g * d, kCombineSlices)), dim3(256), 0, st>>>(a, g, d);
   else

@@ -188,7 +188,7 @@ void paged_decode_mfma16_kernel(
   extern __shared__ __attribute__((aligned(16))) uint8_t tiles[];
 
   int seg_units = 0, n_ranges = a.n_waves;
-  if constexpr (DIRECT == 0) seg_units = build_prefix_units<TILE, BFP8 && D <= 128 && !LONG>(a, cur_pos, s_pref, s_len, s_wsum, n_ranges);
+  if constexpr (DIRECT == 0) seg_units = build_prefix_units<TILE, BFP8 ? D <= 128 && !LONG : D == 256 && !MASKED && !ONE>(a, cur_pos, s_pref, s_len, s_wsum, n_ranges);
   const int lane = threadIdx.x & 63;
   const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 15, quad = lane >> 4;
