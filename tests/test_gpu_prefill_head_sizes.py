@@ -49,6 +49,15 @@ def test_paged(d, users, hq, hkv, bs, start, lc):
     P._check(f"paged h{hq}x{hkv} d{d} bs{bs} start{start} len{lc}", got.cpu(), want)
 
 
+@pytest.mark.parametrize("users,hq,hkv,bs,start,lc", [
+    (1, 8, 8, 32, 256, 32), (4, 8, 8, 64, 512, 64), (1, 8, 8, 32, 256, 65), (5, 8, 8, 32, 64, 32), (4, 16, 8, 32, 1024, 32), (2, 2, 1, 32, 1472, 32),
+    (2, 2, 1, 32, 1504, 32), (1, 3, 1, 32, 96, 32), (32, 2, 1, 64, 100, 20),
+])
+def test_few_rows_of_64_features(users, hq, hkv, bs, start, lc):
+    """On either side of the line between the two loops where a group has one or two (row block, head) pairs."""
+    test_paged(64, users, hq, hkv, bs, start, lc)
+
+
 @pytest.mark.parametrize("d", [64, 256])
 def test_scores_that_force_a_rescale(d):
     """The running maximum moves by more than the lazy threshold again and again."""

@@ -684,7 +684,7 @@ int launch_mode(const PrefillArgs &a, hipStream_t st) {
 
 template <int D, int HPW, int RH>
 int launch_rh(const PrefillArgs &a, hipStream_t st) {
-  if (stream_serves(a)) return launch_stream(a, D, st);
+  if (stream_serves(a, D)) return launch_stream(a, D, st);
   if (!a.pt) return launch_mode<D, HPW, 0, RH>(a, st);
   if (a.bs % kKeysPerTile == 0) return launch_mode<D, HPW, 1, RH>(a, st);
   if (a.bs % Tile<D>::RPI == 0) return launch_mode<D, HPW, 3, RH>(a, st);
@@ -924,7 +924,7 @@ extern "C" int64_t ttpa_sdpa_prefill_bounded_scratch_bytes(int32_t batch, int32_
     if (!stream_expands(a, head_size, INT64_MAX)) return plain_part_bytes(a, head_size, true);
     return ttpa_sdpa_prefill_workspace_bytes(batch, kv_heads, head_size, block_size, table_width, kv_format) + stream_part_bytes(a, head_size);
   }
-  return stream_serves(a) ? stream_part_bytes(a, head_size) : plain_part_bytes(a, head_size, false);
+  return stream_serves(a, head_size) ? stream_part_bytes(a, head_size) : plain_part_bytes(a, head_size, false);
 }
 
 extern "C" int ttpa_sdpa_prefill_fill(

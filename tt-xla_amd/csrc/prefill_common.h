@@ -237,7 +237,7 @@ inline int grid_with_fill(PrefillArgs &b, int grid, int d) {
 }
 
 // prefill_stream.hip: whether the streaming kernel serves this launch, and the launch.
-bool stream_serves(const PrefillArgs &a);
+bool stream_serves(const PrefillArgs &a, int head_size);
 // Whether a pass over block-float-8 caches, with `room` bytes of scratch, is worth expanding into bfloat16 copies for it.
 bool stream_expands(const PrefillArgs &a, int head_size, int64_t room);
 // Bytes of scratch with which it splits the launch over the keys (0: it would not); stream_serves launches only.

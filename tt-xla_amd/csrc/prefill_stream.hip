@@ -26,15 +26,22 @@ namespace ttpa {
 
 // The line lies where the loop's unit does: whole blocks of 32 keys that lie in one piece.  A dense K / V that ends inside a block, smaller cache blocks,
 // windows over a paged cache and explicit masks are the plain loop's.  Wherever both run, this one is
-// faster (above) or, on passes of a few microseconds, equal.
-bool stream_serves(const PrefillArgs &a) {
+// faster (above) or, on passes of a few microseconds, equal, but for one corner: at head size 64, where half of the wavefronts have no rows
+// (two (row block, head) pairs in a group), a few such groups over a few keys end sooner on the other loop, whose start is shorter.  us per pass, this
+// loop / the other: 8 / 8 heads, 1 x 32 rows behind 256 tokens 11.5 / 11.2, 1 x 64 behind 512 12.6 / 12.2, 4 x 32 behind 1024 13.0 / 12.5, 4 x 64 behind 256
+// 12.4 / 12.0, 16 / 8, 4 x 32 behind 512 13.5 / 12.8; beyond: 1 x 32 behind 2048 13.1 / 13.5, 4 x 64 behind 8192 27.0 / 29.0, 8 x 32 behind 512 13.3 / 16.0,
+// 1 x 96 behind 256 12.2 / 13.2, 16 / 8, 1 x 64 behind 2048 15.0 / 15.6.
+bool stream_serves(const PrefillArgs &a, int head_size) {
   if (!a.stream || a.mask != nullptr) return false;
-  if (a.pt) return a.bs % kBlockKeys == 0 && a.window == 0;
-  return a.skv % kBlockKeys == 0;
+  if (!a.pt) return a.skv % kBlockKeys == 0;
+  if (a.bs % kBlockKeys != 0 || a.window != 0) return false;
+  const int heads = head_group_size(a);
+  const bool corner = head_size == 64 && (a.sq + kRowsPerWave - 1) / kRowsPerWave * heads <= 2 && (int64_t)a.batch * (a.hq / heads) <= 32 && a.keys_bound < 1536;
+  return !corner;
 }
 
 int64_t stream_part_bytes(const PrefillArgs &a, int head_size) {
-  return a.pt && stream_serves(a) ? part_bytes(a, head_group_size(a), stream_split(head_size), head_size) : 0;
+  return a.pt && stream_serves(a, head_size) ? part_bytes(a, head_group_size(a), stream_split(head_size), head_size) : 0;
 }
 
 // Whether a block-float-8 pass reads bfloat16 copies, written by a launch in front of it, or expands blocks on their way into
@@ -53,7 +60,7 @@ int64_t stream_part_bytes(const PrefillArgs &a, int head_size) {
 // behind 64 14.2 / 16.6, 512 20.7 / 20.1, 8192 45.8 / 53.7; below either line: 8 / 8, 8 x 448 behind 512 35.2 / 35.4, 4 x 256 33.5 / 30.9; 64 / 8, 8 x 128 behind
 // 512 33.2 / 30.9; 8 / 2, 1 x 512 behind 512 19.2 / 18.3, 1 x 256 behind 8192 31.3 / 28.9.
 bool stream_expands(const PrefillArgs &a, int head_size, int64_t room) {
-  if (!stream_serves(a) || head_size == 256) return false;
+  if (!stream_serves(a, head_size) || head_size == 256) return false;
   if (head_size == 64) {
     const int heads = head_group_size(a), per_group = ((a.sq + kRowsPerWave - 1) / kRowsPerWave * heads + 3) / 4;
     return per_group >= 8 && (int64_t)a.batch * (a.hq / heads) * per_group >= 64;
