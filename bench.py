@@ -46,19 +46,19 @@ KERNEL_SOURCES = {
     "paged_decode_latent16_kernel": ["decode_wide.hip", "decode_common.h", "common.h"],
     "paged_decode_latent128_kernel": ["decode_wide.hip", "gen_latent_frag.py", "decode_common.h", "common.h"],
     "latent_prefill_kernel": ["decode_wide.hip", "gen_latent_frag.py", "decode_common.h", "common.h"],
-    "prefill_stream_kernel": ["prefill_stream.hip", "prefill_parts.h", "prefill_common.h", "gen_prefill_stream.py", "common.h"],
+    "prefill_stream_kernel": ["prefill_stream.hip", "prefill_stream_kernel.h", "prefill_parts.h", "prefill_common.h", "gen_prefill_stream.py", "common.h"],
 }
 MEASURED_TRAFFIC = {
     # workload: (kernel, hash of its sources, HBM bytes per launch: FETCH_SIZE and WRITE_SIZE of the
     # kernel, each scaled by what the same counter reads for a plain copy of known size, mean over
     # the rotating workload copies; the summaries under profiles/ hold the runs)
-    "config2": ("paged_decode_mfma16_kernel", "d1ad07dcf65d7c97", 310416888),
-    "config5": ("paged_decode_mfma16_kernel", "d1ad07dcf65d7c97", 169724320),
-    "config4": ("paged_decode_mfma16_kernel", "d1ad07dcf65d7c97", 3415572133),
-    "config3": ("prefill_stream_kernel", "9100e82cd57f3c5b", 244747201),
-    "latent": ("paged_decode_latent16_kernel", "ce690ec22bd340ff", 654190843),
-    "latent128": ("paged_decode_latent128_kernel", "c74b75a4a905f438", 739359376),
-    "latent-prefill": ("latent_prefill_kernel", "c74b75a4a905f438", 332218599),
+    "config2": ("paged_decode_mfma16_kernel", "b05dcbf5a01a1cd1", 310428209),
+    "config5": ("paged_decode_mfma16_kernel", "b05dcbf5a01a1cd1", 169649630),
+    "config4": ("paged_decode_mfma16_kernel", "b05dcbf5a01a1cd1", 3415545175),
+    "config3": ("prefill_stream_kernel", "b6b6dbc7e8cc05b2", 233195745),
+    "latent": ("paged_decode_latent16_kernel", "5e6a63311c628267", 654182677),
+    "latent128": ("paged_decode_latent128_kernel", "59aea2ac54ae75ed", 739351149),
+    "latent-prefill": ("latent_prefill_kernel", "59aea2ac54ae75ed", 332224843),
 }
 DECODE_KERNEL_NAME = {"config2": "paged_decode_mfma16_kernel", "config4": "paged_decode_mfma16_kernel",
                       "config5": "paged_decode_mfma16_kernel"}
