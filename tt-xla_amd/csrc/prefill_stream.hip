@@ -31,8 +31,12 @@ namespace ttpa {
 // loop / the other: 8 / 8 heads, 1 x 32 rows behind 256 tokens 11.5 / 11.2, 1 x 64 behind 512 12.6 / 12.2, 4 x 32 behind 1024 13.0 / 12.5, 4 x 64 behind 256
 // 12.4 / 12.0, 16 / 8, 4 x 32 behind 512 13.5 / 12.8; beyond: 1 x 32 behind 2048 13.1 / 13.5, 4 x 64 behind 8192 27.0 / 29.0, 8 x 32 behind 512 13.3 / 16.0,
 // 1 x 96 behind 256 12.2 / 13.2, 16 / 8, 1 x 64 behind 2048 15.0 / 15.6.
+// (And the block of assembly steps from row to row of the queries and of the output by an unsigned 32-bit number of bytes: rows in descending order or
+// further apart are the plain loop's, which has 64 bits for them.)
 bool stream_serves(const PrefillArgs &a, int head_size) {
   if (!a.stream || a.mask != nullptr) return false;
+  for (const int64_t rows : {a.q_ts, a.out_ts})
+    if (rows < 0 || rows >= (int64_t)1 << 31) return false;
   if (!a.pt) return a.skv % kBlockKeys == 0;
   if (a.bs % kBlockKeys != 0 || a.window != 0) return false;
   const int heads = head_group_size(a);
