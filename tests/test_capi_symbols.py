@@ -54,6 +54,15 @@ def test_abi_version_and_error_string(native):
         native.call("ttpa_bfp8_quantize", 16, 16, 16, 17, None)
 
 
+def test_split_key_prefill_refuses_descending_rows(native):
+    lib = native.lib()
+    for operand in (0, 3, 4, 5):  # out, the two parts of the keys, v (the queries are read by 64-bit addresses)
+        strides = [[16, 8, 8, 8] for _ in range(6)]
+        strides[operand][3] = -8
+        rc = lib.ttpa_split_key_prefill(*[x for s in strides for x in s], 1, 2, 1, 32, 1.0, None)
+        assert rc == native.ERR_INVALID_ARGUMENT and b"token stride" in lib.ttpa_last_error()
+
+
 def test_workspace_size_is_positive_and_monotone(native):
     lib = native.lib()
     a = lib.ttpa_paged_decode_workspace_bytes(32, 32, 8, 128)

@@ -974,8 +974,10 @@ extern "C" int ttpa_split_key_prefill(
   for (int64_t s : strides) TTPA_REQUIRE(s % 8 == 0, "split-key prefill: operand strides must be multiples of 8 elements");
   TTPA_REQUIRE(out_batch_stride % 4 == 0 && out_head_stride % 4 == 0 && out_token_stride % 4 == 0,
                "split-key prefill: out strides must be multiples of 4 elements");
-  TTPA_REQUIRE(k_nope_token_stride < (1 << 24) && k_rope_token_stride < (1 << 24) && v_token_stride < (1 << 24) &&
-                   q_nope_token_stride < (1ll << 31) && out_token_stride < (1ll << 31),
+  // (but for the queries', token strides are unsigned 32-bit numbers of bytes in the kernel)
+  TTPA_REQUIRE(k_nope_token_stride >= 0 && k_nope_token_stride < (1 << 24) && k_rope_token_stride >= 0 && k_rope_token_stride < (1 << 24) &&
+                   v_token_stride >= 0 && v_token_stride < (1 << 24) && q_nope_token_stride < (1ll << 31) && out_token_stride >= 0 &&
+                   out_token_stride < (1ll << 31),
                "split-key prefill: token stride out of range");
   TTPA_REQUIRE((int64_t)batch * q_heads * ((seq_len + 31) / 32) < (1ll << 30),
                "split-key prefill: batch * heads * query tiles too large for one launch");
