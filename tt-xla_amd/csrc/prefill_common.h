@@ -30,8 +30,8 @@ struct Divisor {
   uint32_t magic;
 };
 inline Divisor divisor(int d) { return {d, d > 1 ? (uint32_t)((1ull << 32) / (uint32_t)d) : ~0u}; }
-__device__ __forceinline__ int quotient(const Divisor &v, int x) {
-  const uint32_t q = __umulhi((uint32_t)x, v.magic);
+__host__ __device__ __forceinline__ int quotient(const Divisor &v, int x) {
+  const uint32_t q = (uint32_t)(((uint64_t)(uint32_t)x * v.magic) >> 32);
   return (int)(q + ((uint32_t)x - q * (uint32_t)v.d >= (uint32_t)v.d ? 1u : 0u));
 }
 
@@ -70,8 +70,8 @@ struct PrefillArgs {
   int spg;
   Divisor by_spg, by_groups, by_group_heads;  // spg, head groups of a batch entry, query heads of a KV head
   // The place of a workgroup (workgroup_place): head groups (batch entries times the groups of one), of which whole rounds of eight
-  // are dealt to one XCD each and the rest over all of them; query heads of a group
-  int full_rounds, rest, head_group;
+  // are dealt to one XCD each and the rest over all of them, group by group if `spread`; query heads of a group
+  int full_rounds, rest, spread, head_group;
   Divisor by_rest, by_head_group;
   int spg_even; // > 0: when the row blocks weigh about the same, only this many of them work (equal shares)
   // ... with keys of 128 + 64 features: the second part of q and k, and V's own strides
@@ -115,8 +115,9 @@ __device__ __forceinline__ int last_row_block(const PrefillArgs &a, int wg) {
 // round-robin by linear id, and each XCD has its own L2: all workgroups of a group run on one XCD, one after the other, so that its
 // K / V is fetched by one L2 only and stays resident there.  The groups left over when the rounds of eight are dealt are spread over all
 // XCDs, one, two or four to each where they are a power of two: on an XCD each they left the others idle (two groups, one prompt of 4096 tokens with
-// 8 / 2 heads of 64: 80 -> 51 us; 1312 rows behind 9152 128 -> 51).
-__device__ __forceinline__ bool workgroup_place(const PrefillArgs &a, int wg, int &y, int &rank) {
+// 8 / 2 heads of 64: 80 -> 51 us; 1312 rows behind 9152 128 -> 51).  `spread` (spreads_groups in prefill_parts.h) deals all groups
+// over all XCDs, the workgroups of one after the other's, so that few of an XCD's are of one group.
+__host__ __device__ __forceinline__ bool workgroup_place(const PrefillArgs &a, int wg, int &y, int &rank) {
   const int t = wg - a.full_rounds * 8 * a.spg;
   if (t < 0) {
     const int slot = wg >> 3, round = quotient(a.by_spg, slot);
@@ -124,19 +125,20 @@ __device__ __forceinline__ bool workgroup_place(const PrefillArgs &a, int wg, in
     return true;
   }
   if (a.rest == 0) return false;
-  rank = quotient(a.by_rest, t);
-  y = a.full_rounds * 8 + t - rank * a.rest;
-  return rank < a.spg;
+  const int q = quotient(a.by_rest, t), r = t - q * a.by_rest.d;
+  rank = a.spread ? r : q;
+  y = a.full_rounds * 8 + (a.spread ? q : r);
+  return q < (a.spread ? a.rest : a.spg);
 }
 // ... and the host's side: the fields it reads, for `heads` query heads per head group and `spg` workgroups per group (0: as many as there are row
 // blocks); the grid, a multiple of 8.
-inline int lay_out(PrefillArgs &a, int heads, int spg = 0) {
+inline int lay_out(PrefillArgs &a, int heads, int spg = 0, bool spread = false) {
   const int groups = a.batch * (a.hq / heads);
   const int pairs = (a.sq + kRowsPerWave - 1) / kRowsPerWave * heads;
   a.head_group = heads, a.by_head_group = divisor(heads);
   a.spg = spg > 0 ? spg : (pairs + 3) / 4;
-  a.full_rounds = groups / 8, a.rest = groups % 8;
-  a.by_spg = divisor(a.spg), a.by_rest = divisor(std::max(a.rest, 1));
+  a.spread = spread, a.full_rounds = spread ? 0 : groups / 8, a.rest = spread ? groups : groups % 8;
+  a.by_spg = divisor(a.spg), a.by_rest = divisor(spread ? a.spg : std::max(a.rest, 1));
   a.by_groups = divisor(a.hq / heads), a.by_group_heads = divisor(a.hq / a.hkv);
   return a.full_rounds * 8 * a.spg + (a.rest * a.spg + 7) / 8 * 8;
 }

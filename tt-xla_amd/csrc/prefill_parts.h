@@ -61,12 +61,14 @@ constexpr int kBlockKeys = 32;
 constexpr int part_acc_floats(int d) { return kRowsPerWave * d; }  // accumulators of one (part, head, row block)
 
 // Blocks of a part (whole 64-key tiles) in a launch whose first query row is at `offset`; a row block of no more is not split.
-__device__ __forceinline__ int blocks_per_part(const PrefillArgs &a, int offset) {
-  const int most = max(((a.causal ? min(a.skv, offset + a.sq) : a.skv) + kBlockKeys - 1) / kBlockKeys, 1);  // of the last row block
+__host__ __device__ __forceinline__ int part_of_blocks(const PrefillArgs &a, int most) {
   if (most < a.split_from) return most;
-  const int shared = quotient(a.by_parts, most + a.parts - 1);
-  const int share = shared >= kSharedPartBlocks ? shared : max(quotient(a.by_parts_one, most + a.parts_one - 1), a.part_min);
+  const int shared = quotient(a.by_parts, most + a.parts - 1), one = quotient(a.by_parts_one, most + a.parts_one - 1);
+  const int share = shared >= kSharedPartBlocks ? shared : one > a.part_min ? one : a.part_min;
   return (share + 1) & ~1;
+}
+__device__ __forceinline__ int blocks_per_part(const PrefillArgs &a, int offset) {
+  return part_of_blocks(a, max(((a.causal ? min(a.skv, offset + a.sq) : a.skv) + kBlockKeys - 1) / kBlockKeys, 1));  // (of the last row block)
 }
 
 // Accumulators and (reference, sum) rows of the parts: [part][batch][head][row block], the statistics
@@ -175,15 +177,60 @@ inline int64_t part_bytes(PrefillArgs a, int heads, const SplitRule &rule, int d
   return part_layout(a).slots * (part_acc_floats(d) + 2 * kRowsPerWave) * (int64_t)sizeof(float);
 }
 
-// Query heads of a head group: the streaming loop's (head_group_size), whose wavefronts may be of different row blocks wherever the
-// heads end, and the plain loop's, whose workgroups take whole row blocks of 4, 2 or 1 heads.
-inline int head_group_size(const PrefillArgs &a) {
-  const int g = a.hq / a.hkv;
-  return g % 4 == 0 ? 4 : g;
-}
+// Query heads of a workgroup of the plain loop, which takes whole row blocks of 4, 2 or 1 heads.
 inline int heads_per_workgroup(const PrefillArgs &a) {
   const int g = a.hq / a.hkv;
   return g % 4 == 0 ? 4 : g % 2 == 0 ? 2 : 1;
+}
+
+// What a launch of `heads` query heads per head group is cut into for the most keys that it may see: its workgroups, the blocks of a part.
+struct Cut {
+  int64_t workgroups;  // of all parts
+  int part, parts;
+};
+inline Cut cut(PrefillArgs a, int heads, const SplitRule &rule) {
+  set_parts(a, heads, rule);
+  const int pairs = (a.sq + kRowsPerWave - 1) / kRowsPerWave * heads, blocks = (int)((a.keys_bound + kBlockKeys - 1) / kBlockKeys);
+  const int part = a.parts > 1 ? part_of_blocks(a, blocks) : blocks, parts = (blocks + part - 1) / part;
+  return {(int64_t)a.batch * (a.hq / heads) * ((pairs + 3) / 4) * parts, part, parts};
+}
+
+// Query heads of a head group of the streaming loop, whose wavefronts may be of different row blocks wherever the heads end: four, or all of a KV
+// head's where these are no multiple of four, but for a chunk of one row block that the plain loop's groups, a workgroup for every one or two heads, leave
+// as short: each of those has a CU to itself (13 of 16 are taken at most), and its one or two wavefronts with rows wait for no others.  A split costs
+// about what eleven blocks do.  us per pass, pairs / a workgroup per head, 40 / 8 of 128: 1 x 32 rows behind 512 tokens 15.8 / 15.3, 832 16.1 / 15.5,
+// 2 x 32 behind 512, which then is not split, 16.6 / 15.5; 24 / 8, 3 x 32 behind 512 16.3 / 15.3; 10 / 2 of 64, 1 x 32 behind 512 12.3 / 11.3;
+// beyond: 40 / 8, 1 x 32 behind 2432 18.9 / 21.8, 2 x 32 behind 640 16.7 / 18.0, 3 x 32 behind 512 15.7 / 16.8.
+constexpr int kSplitBlocks = 11;
+inline int head_group_size(const PrefillArgs &a, int d) {
+  const int g = a.hq / a.hkv, fewer = heads_per_workgroup(a);
+  if (g % 4 == 0) return 4;
+  if (!a.pt || a.sq > kRowsPerWave || g == fewer) return g;
+  int cus = device_cus();
+  if (cus <= 0) cus = 256;
+  const Cut pairs = cut(a, g, stream_split(d)), heads = cut(a, fewer, stream_split(d));
+  const bool as_short = heads.part + (heads.parts > 1 ? kSplitBlocks : 0) <= pairs.part + kSplitBlocks;
+  return pairs.parts > 1 && as_short && 16 * heads.workgroups <= 13 * cus ? fewer : g;
+}
+
+// Whether the workgroups of a KV head's pairs are spread over the XCDs: three quarters of the CUs or more have a part each, all of a KV head's, which ask
+// for the same blocks at the same time, would be on one or two XCDs, and the caches are small enough for several XCDs to read the same.  (One row block has too
+// few workgroups per KV head for that, and at head size 64 there was nothing in it.)  us per pass of 40 / 8 heads of 128, a KV head on one XCD / spread (before
+// pairs, whole row blocks of single heads, five KV heads on an XCD): 1 x 96 rows behind 1600 tokens 23.1 / 21.1 (21.3), 1 x 128 behind 2432
+// 26.7 / 24.6 (24.3), 1 x 256 behind 1216 28.9 / 26.3 (25.8), 2 x 96 behind 832 23.9 / 21.7 (22.8), 1 x 384 behind 1600 36.1 / 33.8
+// (33.6); 28 / 4, 1 x 256 behind 2432 29.7 / 27.0 (27.0).  Fewer workgroups: 1 x 128 behind 832 20.4 / 20.9; more keys: 1 x 192 behind 5504
+// 39.9 / 46.5, 2 x 96 behind 3200 30.1 / 31.5; head size 64: 1 x 256 behind 512 17.9 / 17.9.
+constexpr int64_t kSpreadBytes = 14 << 20;
+inline bool spreads_groups(const PrefillArgs &a, int heads, int d) {
+  if (a.parts <= 1 || heads == heads_per_workgroup(a) || a.sq <= kRowsPerWave || d < 128 || 4 * a.batch * a.hkv * a.keys_bound * d > kSpreadBytes) return false;
+  int cus = device_cus();
+  if (cus <= 0) cus = 256;
+  // (a caller's bound may be a few blocks beyond the chunk: parts that two workgroups of a CU would only just share count as not shared)
+  const int64_t blocks = (a.keys_bound + kBlockKeys - 1) / kBlockKeys;
+  if ((blocks + a.parts - 1) / a.parts >= kSharedPartBlocks + 2) return false;
+  const int64_t part = (std::max<int64_t>((blocks + a.parts_one - 1) / a.parts_one, a.part_min) + 1) & ~1;
+  const int64_t pairs = (a.sq + kRowsPerWave - 1) / kRowsPerWave * heads, workgroups = a.batch * (a.hq / heads) * ((pairs + 3) / 4) * ((blocks + part - 1) / part);
+  return 4 * workgroups >= 3 * cus && workgroups <= cus;
 }
 
 // Whether the plain loop may split the keys of this launch: paged, each row sees all keys up to its own.

@@ -4,8 +4,8 @@
 // between them.  At 64, where there are 8, that vector work does (busy 58 % of the time, the matrix pipe 39 %, either 78 %).
 //
 // The work split: four wavefronts of 32 query rows share K / V in LDS, four consecutive (row block, head) pairs of a KV head
-// (row_blocks in prefill_common.h); where a group's workgroups run says workgroup_place.  Five heads per KV head, 40 / 8 of 128: 6 x 32 rows behind
-// 7232 tokens 140 -> 60 us, 2 x 1152 tokens 50 -> 43, 1 x 224 behind 1216 26.6 -> 28.0 (all workgroups of a KV head read the same keys at once).  The whole life of a workgroup behind its address set-up is one block of
+// (row_blocks in prefill_common.h); where a group's workgroups run say workgroup_place and spreads_groups.  Five heads per KV head, 40 / 8 of 128: 6 x 32
+// rows behind 7232 tokens 140 -> 60 us, 2 x 1152 tokens 50 -> 43, 1 x 256 behind 1216 26.9 -> 26.6 (28.9 with a KV head's workgroups on one XCD).  The whole life of a workgroup behind its address set-up is one block of
 // assembly, written by gen_prefill_stream.py, which documents the schedule and the state on entry.
 // Against the compiler-scheduled loop of prefill.hip on the same shapes (a whole pass): window of 1024
 // keys, 2 x 4096 tokens, 32 / 8 heads 160 -> 137 us; 4 x 2048 tokens, 16 / 16 heads 118 -> 98 us and 16 / 8
@@ -39,13 +39,13 @@ bool stream_serves(const PrefillArgs &a, int head_size) {
     if (rows < 0 || rows >= (int64_t)1 << 31) return false;
   if (!a.pt) return a.skv % kBlockKeys == 0;
   if (a.bs % kBlockKeys != 0 || a.window != 0) return false;
-  const int heads = head_group_size(a);
+  const int heads = head_group_size(a, head_size);
   const bool corner = head_size == 64 && (a.sq + kRowsPerWave - 1) / kRowsPerWave * heads <= 2 && (int64_t)a.batch * (a.hq / heads) <= 32 && a.keys_bound < 1536;
   return !corner;
 }
 
 int64_t stream_part_bytes(const PrefillArgs &a, int head_size) {
-  return a.pt && stream_serves(a, head_size) ? part_bytes(a, head_group_size(a), stream_split(head_size), head_size) : 0;
+  return a.pt && stream_serves(a, head_size) ? part_bytes(a, head_group_size(a, head_size), stream_split(head_size), head_size) : 0;
 }
 
 // Whether a block-float-8 pass reads bfloat16 copies, written by a launch in front of it, or expands blocks on their way into
@@ -66,7 +66,7 @@ int64_t stream_part_bytes(const PrefillArgs &a, int head_size) {
 bool stream_expands(const PrefillArgs &a, int head_size, int64_t room) {
   if (!stream_serves(a, head_size) || head_size == 256) return false;
   if (head_size == 64) {
-    const int heads = head_group_size(a), per_group = ((a.sq + kRowsPerWave - 1) / kRowsPerWave * heads + 3) / 4;
+    const int heads = head_group_size(a, head_size), per_group = ((a.sq + kRowsPerWave - 1) / kRowsPerWave * heads + 3) / 4;
     return per_group >= 8 && (int64_t)a.batch * (a.hq / heads) * per_group >= 64;
   }
   const int hpw = heads_per_workgroup(a), rows = kRowsPerWave * 4 / hpw;
@@ -75,7 +75,7 @@ bool stream_expands(const PrefillArgs &a, int head_size, int64_t room) {
   const bool splits = parts > 0 && parts <= room;
   // (a table has room for more keys than the chunk's: 8192 rows of it)
   const bool few = a.batch * a.keys_bound * a.hkv <= (a.keys_known ? 5120 : 8192);
-  const bool pays = (row_blocks > 1 && (readers > 2 || a.keys_bound >= 512)) || few || part_bytes(a, head_group_size(a), stream_split(head_size), head_size) > 0 || (readers > (splits ? 3 : 2) && a.keys_bound >= 512);
+  const bool pays = (row_blocks > 1 && (readers > 2 || a.keys_bound >= 512)) || few || part_bytes(a, head_group_size(a, head_size), stream_split(head_size), head_size) > 0 || (readers > (splits ? 3 : 2) && a.keys_bound >= 512);
   return pays && !(splits && readers <= 2);
 }
 

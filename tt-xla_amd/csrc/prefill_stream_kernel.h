@@ -320,7 +320,7 @@ int launch_form(const PrefillArgs &a, hipStream_t st) {
     return fail(TTPA_ERR_LAUNCH, "prefill: cannot reserve %d bytes of LDS", lds);
   PrefillArgs b = a;
   b.spg_even = 0, b.parts = 1;
-  const int heads = head_group_size(a);
+  const int heads = head_group_size(a, D);
   // One workgroup per row block and head group, heavy blocks first, and the dispatcher deals them to the CUs
   // as slots free up: the loop can also give a workgroup several row blocks (spg workgroups per group,
   // TTPA_PREFILL_WGS_PER_GROUP), but one round of two workgroups per CU measured 204 us against 150 on
@@ -331,7 +331,7 @@ int launch_form(const PrefillArgs &a, hipStream_t st) {
   const char *e = items ? getenv("TTPA_PREFILL_WGS_PER_GROUP") : nullptr;
   const int per_group = e ? atoi(e) : 0;
   if (PAGED && per_group <= 0 && a.part_acc && a.part_bytes >= part_bytes(a, heads, stream_split(D), D)) set_parts(b, heads, stream_split(D));
-  int grid = lay_out(b, heads);
+  int grid = lay_out(b, heads, 0, PAGED && spreads_groups(b, heads, D));
   if (per_group > 0) {
     grid = lay_out(b, heads, std::min(b.spg, per_group));
   } else if (items && b.parts == 1) {
