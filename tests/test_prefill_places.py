@@ -16,12 +16,11 @@ PROGRAM = textwrap.dedent(
     #include <vector>
     #include "prefill_parts.h"
     using namespace ttpa;
-    namespace ttpa { int device_cus() { return 256; } }
 
     static PrefillArgs pass(int batch, int hq, int hkv, int sq, long keys, bool paged) {
       static const int32_t table = 0;
       PrefillArgs a = {};
-      a.batch = batch, a.hq = hq, a.hkv = hkv, a.sq = sq, a.keys_bound = keys, a.keys_known = 1;
+      a.batch = batch, a.hq = hq, a.hkv = hkv, a.sq = sq, a.keys_bound = keys, a.keys_known = 1, a.cus = 256;
       a.pt = paged ? &table : nullptr;
       return a;
     }

@@ -746,6 +746,11 @@ int launch_d(const PrefillArgs &a, hipStream_t st) {
 
 using namespace ttpa;
 
+static int cus_for_rules() {
+  const int cus = device_cus();
+  return cus > 0 ? cus : 256;
+}
+
 // The cache fill that a dense prefill may carry along (ttpa_sdpa_prefill_fill).
 struct FillSpec {
   void *k_cache, *v_cache;
@@ -814,6 +819,7 @@ static int prefill_impl(void *out, int64_t out_batch_stride, int64_t out_head_st
   a.mask_bs = mask_batch_stride, a.mask_rs = mask_row_stride;
   a.batch = batch, a.hq = q_heads, a.hkv = kv_heads, a.sq = q_len, a.skv = kv_len;
   a.bs = block_size, a.w = table_width, a.nb = num_blocks, a.causal = causal ? 1 : 0;
+  a.cus = cus_for_rules();
   a.keys_known = page_table && most_keys > 0, a.keys_bound = a.keys_known ? std::min<int64_t>(most_keys, kv_len) : kv_len;
   a.window = sliding_window;
   a.scale_log2e = scale * 1.4426950408889634f;
@@ -916,7 +922,7 @@ extern "C" int64_t ttpa_sdpa_prefill_bounded_scratch_bytes(int32_t batch, int32_
     return 0;
   const int32_t some_table = 0;
   PrefillArgs a = {};
-  a.pt = &some_table, a.stream = 1;
+  a.pt = &some_table, a.stream = 1, a.cus = cus_for_rules();
   a.batch = batch, a.hq = q_heads, a.hkv = kv_heads, a.sq = q_len, a.bs = block_size, a.w = table_width;
   a.keys_bound = (int64_t)table_width * block_size;
   if (most_keys > 0) a.keys_known = 1, a.keys_bound = std::min(a.keys_bound, most_keys);

@@ -65,13 +65,13 @@ struct PrefillArgs {
   float scale_log2e;
   int kv_bfp8;  // paged form: the caches are block-float-8 (mode 4, or expanded into `expand` first)
   void *expand; // scratch for bfloat16 copies of the block-float-8 blocks of this pass, or null
-  int stream;   // 0: the plain loop whatever the shape (TTPA_PREFILL_STREAM=0)
+  int spread;   // workgroup_place: every head group over all XCDs
   // The streaming kernel: workgroups per (batch entry, head group), each taking one or several row blocks
   int spg;
   Divisor by_spg, by_groups, by_group_heads;  // spg, head groups of a batch entry, query heads of a KV head
   // The place of a workgroup (workgroup_place): head groups (batch entries times the groups of one), of which whole rounds of eight
   // are dealt to one XCD each and the rest over all of them, group by group if `spread`; query heads of a group
-  int full_rounds, rest, spread, head_group;
+  int full_rounds, rest, head_group;
   Divisor by_rest, by_head_group;
   int spg_even; // > 0: when the row blocks weigh about the same, only this many of them work (equal shares)
   // ... with keys of 128 + 64 features: the second part of q and k, and V's own strides
@@ -84,8 +84,11 @@ struct PrefillArgs {
   Divisor by_parts, by_parts_one;
   int split_from;        // launches whose last row block has fewer 32-key blocks are not split
   int part_min;          // 32-key blocks of a part at least
-  int64_t keys_bound;    // keys of the last row at most, as far as the host knows: what the launch is laid out for (set_parts)
+  // The host's alone: what the launch is laid out for (set_parts)
+  int64_t keys_bound;    // keys of the last row at most, as far as the host knows
   int keys_known;        // ... from the caller, and not from the page table's room
+  int cus;               // CUs of the device: asked for once per pass, whose rules need it several times
+  int stream;            // 0: the plain loop whatever the shape (TTPA_PREFILL_STREAM=0)
 };
 
 // key / block_size without a division instruction sequence (about 30 instructions each, and the

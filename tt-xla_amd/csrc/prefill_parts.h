@@ -63,8 +63,8 @@ constexpr int part_acc_floats(int d) { return kRowsPerWave * d; }  // accumulato
 // Blocks of a part (whole 64-key tiles) in a launch whose first query row is at `offset`; a row block of no more is not split.
 __host__ __device__ __forceinline__ int part_of_blocks(const PrefillArgs &a, int most) {
   if (most < a.split_from) return most;
-  const int shared = quotient(a.by_parts, most + a.parts - 1), one = quotient(a.by_parts_one, most + a.parts_one - 1);
-  const int share = shared >= kSharedPartBlocks ? shared : one > a.part_min ? one : a.part_min;
+  const int shared = quotient(a.by_parts, most + a.parts - 1);
+  const int share = shared >= kSharedPartBlocks ? shared : max(quotient(a.by_parts_one, most + a.parts_one - 1), a.part_min);
   return (share + 1) & ~1;
 }
 __device__ __forceinline__ int blocks_per_part(const PrefillArgs &a, int offset) {
@@ -157,17 +157,15 @@ __global__ __launch_bounds__(2 * D) void prefill_merge_kernel(PrefillArgs a) {
 // Workgroups of the launch without a split, and what it may be split into: as many parts as fill the workgroup slots of
 // every CU once, if its row blocks leave at least half of them empty and its page keys may be enough to be split at all.
 inline void set_parts(PrefillArgs &a, int heads, const SplitRule &rule) {
-  int cus = device_cus();
-  if (cus <= 0) cus = 256;
   const int pairs = (a.sq + kRowsPerWave - 1) / kRowsPerWave * heads;
   const int64_t wgs = (int64_t)a.batch * (a.hq / heads) * ((pairs + 3) / 4);
   const int blocks = (int)((a.keys_bound + kBlockKeys - 1) / kBlockKeys);
   const int most = std::min(kMaxParts, (blocks + rule.min_part - 1) / rule.min_part);
-  const int64_t from = 2 * wgs <= cus ? 7 * wgs / 16 : std::min<int64_t>(wgs, rule.wgs_per_cu * cus) / 2;
+  const int64_t from = 2 * wgs <= a.cus ? 7 * wgs / 16 : std::min<int64_t>(wgs, rule.wgs_per_cu * a.cus) / 2;
   a.split_from = (int)std::max<int64_t>(rule.min_split, 100 * from / rule.block_cost);
   a.part_min = rule.min_part;
-  a.parts = blocks < a.split_from * (a.keys_known ? rule.known_percent : rule.table_percent) / 100 ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>(rule.wgs_per_cu * cus / wgs, most));
-  a.parts_one = (int)std::max<int64_t>(1, std::min<int64_t>(cus / wgs, most));
+  a.parts = blocks < a.split_from * (a.keys_known ? rule.known_percent : rule.table_percent) / 100 ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>(rule.wgs_per_cu * a.cus / wgs, most));
+  a.parts_one = (int)std::max<int64_t>(1, std::min<int64_t>(a.cus / wgs, most));
   a.by_parts = divisor(a.parts), a.by_parts_one = divisor(a.parts_one);
 }
 
@@ -206,11 +204,9 @@ inline int head_group_size(const PrefillArgs &a, int d) {
   const int g = a.hq / a.hkv, fewer = heads_per_workgroup(a);
   if (g % 4 == 0) return 4;
   if (!a.pt || a.sq > kRowsPerWave || g == fewer) return g;
-  int cus = device_cus();
-  if (cus <= 0) cus = 256;
   const Cut pairs = cut(a, g, stream_split(d)), heads = cut(a, fewer, stream_split(d));
   const bool as_short = heads.part + (heads.parts > 1 ? kSplitBlocks : 0) <= pairs.part + kSplitBlocks;
-  return pairs.parts > 1 && as_short && 16 * heads.workgroups <= 13 * cus ? fewer : g;
+  return pairs.parts > 1 && as_short && 16 * heads.workgroups <= 13 * a.cus ? fewer : g;
 }
 
 // Whether the workgroups of a KV head's pairs are spread over the XCDs: three quarters of the CUs or more have a part each, all of a KV head's, which ask
@@ -223,14 +219,12 @@ inline int head_group_size(const PrefillArgs &a, int d) {
 constexpr int64_t kSpreadBytes = 14 << 20;
 inline bool spreads_groups(const PrefillArgs &a, int heads, int d) {
   if (a.parts <= 1 || heads == heads_per_workgroup(a) || a.sq <= kRowsPerWave || d < 128 || 4 * a.batch * a.hkv * a.keys_bound * d > kSpreadBytes) return false;
-  int cus = device_cus();
-  if (cus <= 0) cus = 256;
   // (a caller's bound may be a few blocks beyond the chunk: parts that two workgroups of a CU would only just share count as not shared)
   const int64_t blocks = (a.keys_bound + kBlockKeys - 1) / kBlockKeys;
   if ((blocks + a.parts - 1) / a.parts >= kSharedPartBlocks + 2) return false;
   const int64_t part = (std::max<int64_t>((blocks + a.parts_one - 1) / a.parts_one, a.part_min) + 1) & ~1;
   const int64_t pairs = (a.sq + kRowsPerWave - 1) / kRowsPerWave * heads, workgroups = a.batch * (a.hq / heads) * ((pairs + 3) / 4) * ((blocks + part - 1) / part);
-  return 4 * workgroups >= 3 * cus && workgroups <= cus;
+  return 4 * workgroups >= 3 * a.cus && workgroups <= a.cus;
 }
 
 // Whether the plain loop may split the keys of this launch: paged, each row sees all keys up to its own.

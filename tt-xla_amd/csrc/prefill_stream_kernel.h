@@ -339,9 +339,7 @@ int launch_form(const PrefillArgs &a, hipStream_t st) {
     // chip more than once: one round of workgroups with equal shares instead, which saves the later
     // rounds' start-up (267 -> 261 us on 4 x 512-token chunks behind 4096 tokens, 64 heads).  The
     // chunk's start is in device memory, so the kernel decides: the workgroups past the round exit.
-    int cus = device_cus();
-    if (cus <= 0) cus = 256;
-    const int groups = a.batch * (a.hq / heads), one_round = (2 * cus + groups - 1) / groups;
+    const int groups = a.batch * (a.hq / heads), one_round = (2 * a.cus + groups - 1) / groups;
     b.spg_even = one_round < b.spg && b.spg % one_round == 0 ? one_round : 0;
   }
   if (!PAGED && FORM != kDenseWide && a.fill_kc) grid = grid_with_fill(b, grid, D);
