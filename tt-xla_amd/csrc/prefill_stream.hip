@@ -26,11 +26,12 @@ namespace ttpa {
 
 // The line lies where the loop's unit does: whole blocks of 32 keys that lie in one piece.  A dense K / V that ends inside a block, smaller cache blocks,
 // windows over a paged cache and explicit masks are the plain loop's.  Wherever both run, this one is
-// faster (above) or, on passes of a few microseconds, equal, but for one corner: at head size 64, where half of the wavefronts have no rows
-// (two (row block, head) pairs in a group), a few such groups over a few keys end sooner on the other loop, whose start is shorter.  us per pass, this
-// loop / the other: 8 / 8 heads, 1 x 32 rows behind 256 tokens 11.5 / 11.2, 1 x 64 behind 512 12.6 / 12.2, 4 x 32 behind 1024 13.0 / 12.5, 4 x 64 behind 256
-// 12.4 / 12.0, 16 / 8, 4 x 32 behind 512 13.5 / 12.8; beyond: 1 x 32 behind 2048 13.1 / 13.5, 4 x 64 behind 8192 27.0 / 29.0, 8 x 32 behind 512 13.3 / 16.0,
-// 1 x 96 behind 256 12.2 / 13.2, 16 / 8, 1 x 64 behind 2048 15.0 / 15.6.
+// faster (above) or equal, but for launches at head size 64 that are split and in which half of the wavefronts or more have no rows (one or two
+// (row block, head) pairs in a group): over few keys, while the groups are few, the other loop's parts start and end sooner, and with one pair
+// two workgroups of a CU, which wait for memory together, hold longer tiles there.  us per pass, this loop / the other: 8 / 8 heads, 1 x 32 rows behind
+// 256 tokens 11.4 / 11.0, 1 x 64 behind 512 12.5 / 12.2, 4 x 32 behind 1024 13.0 / 12.5, 6 x 64 behind 512 14.1 / 13.6, 16 / 8, 4 x 32 behind 512 13.3 / 12.9;
+// two on a CU: 5 x 32 behind 8192 26.2 / 24.5, 12 x 32 behind 4096 28.2 / 26.8.  Beyond: not split, 1 x 32 behind 64 7.7 / 9.2, 5 x 64 behind 256 10.7 / 12.5;
+// more keys, 1 x 32 behind 2048 13.0 / 13.4, 4 x 64 behind 8192 26.1 / 28.6; more groups, 8 x 64 behind 512 14.3 / 14.6; more pairs, 1 x 96 behind 256 11.8 / 13.1.
 // (And the block of assembly steps from row to row of the queries and of the output by an unsigned 32-bit number of bytes: rows in descending order or
 // further apart are the plain loop's, which has 64 bits for them.)
 bool stream_serves(const PrefillArgs &a, int head_size) {
@@ -39,9 +40,12 @@ bool stream_serves(const PrefillArgs &a, int head_size) {
     if (rows < 0 || rows >= (int64_t)1 << 31) return false;
   if (!a.pt) return a.skv % kBlockKeys == 0;
   if (a.bs % kBlockKeys != 0 || a.window != 0) return false;
-  const int heads = head_group_size(a, head_size);
-  const bool corner = head_size == 64 && (a.sq + kRowsPerWave - 1) / kRowsPerWave * heads <= 2 && (int64_t)a.batch * (a.hq / heads) <= 32 && a.keys_bound < 1536;
-  return !corner;
+  if (head_size != 64 || a.sq > 2 * kRowsPerWave) return true;
+  const int heads = head_group_size(a, head_size), pairs = (a.sq + kRowsPerWave - 1) / kRowsPerWave * heads;
+  const bool few_keys = a.keys_bound < 1536 && (int64_t)a.batch * (a.hq / heads) <= 48;
+  if (pairs > 2 || !(few_keys || pairs == 1)) return true;
+  const Cut c = cut(a, heads, stream_split(head_size));
+  return c.parts == 1 || !(few_keys || (c.part >= kSharedPartBlocks && c.workgroups > a.cus));
 }
 
 int64_t stream_part_bytes(const PrefillArgs &a, int head_size) {
