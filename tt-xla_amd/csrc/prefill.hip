@@ -691,13 +691,6 @@ int launch_rh(const PrefillArgs &a, hipStream_t st) {
   return launch_mode<D, HPW, 2, RH>(a, st);
 }
 
-// Bytes of the scratch an expanded block-float-8 pass needs: K and V copies of batch * width blocks
-// and their table.
-inline int64_t expand_bytes(int batch, int width, int kv_heads, int block_size, int d) {
-  const int64_t blocks = (int64_t)batch * width;
-  return 2 * blocks * kv_heads * block_size * d * 2 + ((blocks * 4 + 255) & ~int64_t(255));
-}
-
 template <int D, int HPW>
 int launch(const PrefillArgs &a, hipStream_t st) {
   if (a.pt && a.kv_bfp8) {

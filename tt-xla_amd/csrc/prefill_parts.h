@@ -175,6 +175,13 @@ inline int64_t part_bytes(PrefillArgs a, int heads, const SplitRule &rule, int d
   return part_layout(a).slots * (part_acc_floats(d) + 2 * kRowsPerWave) * (int64_t)sizeof(float);
 }
 
+// Bytes of the scratch an expanded block-float-8 pass needs: K and V copies of batch * width blocks
+// and their table.
+inline int64_t expand_bytes(int batch, int width, int kv_heads, int block_size, int d) {
+  const int64_t blocks = (int64_t)batch * width;
+  return 2 * blocks * kv_heads * block_size * d * 2 + ((blocks * 4 + 255) & ~int64_t(255));
+}
+
 // Query heads of a workgroup of the plain loop, which takes whole row blocks of 4, 2 or 1 heads.
 inline int heads_per_workgroup(const PrefillArgs &a) {
   const int g = a.hq / a.hkv;

@@ -64,14 +64,20 @@ int64_t stream_part_bytes(const PrefillArgs &a, int head_size) {
 // 4096 167 / 75.6; two row blocks: 4 x 64 of 32 / 8 behind 512 29.5 / 24.9, 8 x 256 of 16 / 16 behind 4096 195 / 128.  Four workgroups: 2 x 64 of
 // 64 / 8 behind 4096 49.5 / 55.6; three: 2 x 96 of 32 / 8 46.7 / 50.0.
 // At head size 64 mode 4 costs less per block and the copies as much: from eight workgroups per head group on, where the launch has 64.  8 / 8 heads,
-// 1 x 1024 rows behind 512 tokens 23.6 / 25.2, 4 x 1024 42.1 / 50.4; 64 / 8, 1 x 256 behind 2048 36.7 / 41.9, 8 x 448 behind 64 44.9 / 64.7; 8 / 2, 4 x 256
-// behind 64 14.2 / 16.6, 512 20.7 / 20.1, 8192 45.8 / 53.7; below either line: 8 / 8, 8 x 448 behind 512 35.2 / 35.4, 4 x 256 33.5 / 30.9; 64 / 8, 8 x 128 behind
-// 512 33.2 / 30.9; 8 / 2, 1 x 512 behind 512 19.2 / 18.3, 1 x 256 behind 8192 31.3 / 28.9.
+// 1 x 1024 rows behind 512 tokens 22.1 / 24.7, 4 x 1024 35.1 / 49.2; 64 / 8, 1 x 256 behind 2048 35.1 / 41.0, 8 x 448 behind 64 42.6 / 63.6; 8 / 2, 5 x 256
+// behind 512 21.7 / 21.9, 4 x 256 behind 64 13.9 / 16.1, 192 15.6 / 17.7, 768 21.4 / 21.5, 8192 43.2 / 51.9, but behind 320 and 512 19.1 / 18.8 and 20.4 / 19.9 (16 / 8
+// 1 x 512, with as many workgroups and blocks read as often, 19.5 / 20.1 there: no line in these numbers parts the two); below either line: 8 / 8,
+// 4 x 256 behind 512 21.8 / 20.7, 8192 56.6 / 50.4; 64 / 8, 8 x 128 behind 512 31.3 / 29.5; 8 / 2, 1 x 512 behind 512 18.8 / 17.6, 1 x 256 behind 8192 30.3 / 28.3.
+// (Launches below the line that are large and not split would gain: 8 / 8, 8 x 448 behind 512 28.2 / 33.5, 2048 54.4 / 56.4.)
 bool stream_expands(const PrefillArgs &a, int head_size, int64_t room) {
   if (!stream_serves(a, head_size) || head_size == 256) return false;
   if (head_size == 64) {
     const int heads = head_group_size(a, head_size), per_group = ((a.sq + kRowsPerWave - 1) / kRowsPerWave * heads + 3) / 4;
-    return per_group >= 8 && (int64_t)a.batch * (a.hq / heads) * per_group >= 64;
+    if (per_group < 8 || (int64_t)a.batch * (a.hq / heads) * per_group < 64) return false;
+    // a caller's scratch may hold mode 4's parts, but not the copies and the parts behind them: unsplit copies are the slower form (4 x 256 rows of 8 / 2 behind
+    // 8700 tokens, the operator with that scratch, 123 us, mode 4 split 55)
+    const int64_t parts = plain_part_bytes(a, head_size, true);
+    return parts == 0 || parts > room || expand_bytes(a.batch, a.w, a.hkv, a.bs, head_size) + stream_part_bytes(a, head_size) <= room;
   }
   const int hpw = heads_per_workgroup(a), rows = kRowsPerWave * 4 / hpw;
   const int64_t row_blocks = (a.sq + rows - 1) / rows, readers = row_blocks * (a.hq / hpw / a.hkv);
