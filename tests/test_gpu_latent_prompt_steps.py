@@ -1,4 +1,4 @@
-"""Latent prompts on either side of the line from which their expansion takes 64 latent values per step (384 workgroups): both layouts of
+"""Latent prompts on either side of the line from which their expansion takes 64 latent values per step (800 workgroups), and at sizes of a part of a round: both layouts of
 either weight, activations as slices, a last tile of one row block; one call against the operators in turn, as test_gpu_latent_prompt.py
 has it."""
 
@@ -16,6 +16,9 @@ def _pkg():
 
 
 @pytest.mark.parametrize("joint,slices", [(None, False), ("latent first", True), ("heads first", False)])
-@pytest.mark.parametrize("n,users,s", [(96, 1, 256), (95, 1, 256), (64, 3, 96), (64, 2, 160)])  # 384 workgroups, 380, 384, 384
+@pytest.mark.parametrize("n,users,s", [
+    (96, 1, 256), (95, 1, 256), (64, 3, 96), (64, 2, 160),  # 384 workgroups, 380, 384, 384
+    (100, 1, 480), (99, 1, 512), (64, 7, 160), (128, 1, 512),  # 800 workgroups, 792, 1152, 1024
+])
 def test_either_step(n, users, s, joint, slices):
     L.test_one_call_equals_the_operators(n, users, s, 32, joint, slices)

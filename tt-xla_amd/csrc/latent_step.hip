@@ -277,10 +277,14 @@ struct ExpandArgs {
   int items;                 // workgroups behind them write rows of the cache, 8 threads to a row
 };
 
-// Steps of 64 latent values in a ring of two where the launch fills the chip: whole 128-byte lines per request instead of halves, which is
-// worth more there than three steps on their way (3 x 1984 tokens of 16 heads, the pass 118.2 / 114.5 us, 3 x 832 of 32 69.7 / 67.6, 1 x 1792 of
-// 16 50.2 / 49.6; 3 x 512 29.7 / 29.4; 2 x 416, which does not, 20.0 / 20.5, 1 x 96 12.4 / 12.9).  256 tokens per workgroup with steps of 32
-// or 64: 4 x 2048 the kernel alone 43.3 and 48.2 us against 45.4 and 41.7 (the two above), 1 x 480 9.7 and 10.3 against 6.2 and 8.1.
+// Steps of 64 latent values in a ring of two where the second round of the chip's 512 places is more than half full: whole 128-byte lines per request
+// instead of halves, which is worth more there than three steps on their way; with fewer workgroups the last ones have the chip to themselves, and what
+// each has on its way counts.  us per pass, steps of 32 / 64 (workgroups): 16 heads, 2 x 1568 tokens 62.9 / 61.1 (800), 2 x 1760 71.1 / 69.6 (896), 2 x 2048
+// 88.3 / 86.6 (1024), 3 x 1824 107.7 / 105.1 (1376), 4 x 2048 150.5 / 148.9 (2048; from card to card 145.0 / 149.3 to 150.6 / 147.9), 32 heads, 3 x 832 69.1 / 67.1
+// (1280), 128 heads, 1 x 416 46.6 / 44.7 (1024).  Below: 16 heads, 1 x 96 12.5 / 12.9 (32), 1 x 1280 39.2 / 38.6 (320), 1 x 1920 51.6 / 51.6 (480), 2 x 1024 38.6 / 40.6 (512),
+// 2 x 1088 45.0 / 46.6 (544), 1 x 2432 70.9 / 74.5 (608), 2 x 1440 58.3 / 58.4 (720), 32 heads, 4 x 256 27.0 / 28.3 (512), 128 heads, 1 x 352 37.5 / 38.2 (768).
+// 256 tokens per workgroup with steps of 32 or 64: 4 x 2048 the kernel alone 43.3 and 48.2 us against 45.4 and 41.7 (the two above), 1 x 480
+// 9.7 and 10.3 against 6.2 and 8.1.
 constexpr int kExpTokens = 128;
 template <int STEP, int STAGES>
 struct ExpandShape {
@@ -615,7 +619,7 @@ extern "C" int ttpa_latent_prompt(void *out, int64_t out_token_stride, int64_t o
     e.k = reinterpret_cast<uint16_t *>(ws), e.v = reinterpret_cast<uint16_t *>(ws + align256((size_t)rows * heads * 256));
     e.uk_rows = !uk_columns, e.uv_rows = uv_columns;
     e.items = (int)(token_tiles * 2 * heads);
-    const bool fills = e.items >= 384;  // (of 512 places)
+    const bool fills = e.items >= 800;  // (of 512 places: ExpandShape)
     if (int rc = fills ? launch_expand<ExpandShape<64, 2>>(e, st) : launch_expand<ExpandShape<32, 4>>(e, st)) return rc;
     const int64_t hd = (int64_t)heads * 128, sl = seq_len;
     return ttpa_split_key_prefill(out, sl * out_token_stride, out_head_stride, out_token_stride, q_nope, sl * q_nope_token_stride,
