@@ -570,11 +570,12 @@ static int decode_impl(void *out, int64_t out_user_stride, int64_t out_head_stri
   if (two_per_cu) a.few_ranges = waves_for_device(4.0);
   // Head size 256, whose tiles are 16 KiB: a list of no more tiles than four wavefronts per CU has a range for each of them, so that none
   // waits for a second tile (how long it is the kernel knows, and leaves a quarter of a longer list's ranges empty).  us per layer, three /
-  // four per CU, 820, 900 and 1000 tiles of 16/8 heads 15.6 / 13.2, 15.9 / 13.7, 16.0 / 14.5; 760 and 1100 tiles 13.2 / 13.2 and 16.0 / 16.0.  More
-  // partials cost the merge more: not with wider groups (32/4 heads 16.9 / 17.1 ... 17.6 / 18.7) or where few segments have
-  // hundreds.  One head per group gains as much (7 users of 408 ... 707 tokens 16.3 / 14.2), but its kernel pays 1 % for the choice on every
-  // other list, and at 64 and 128, for 2 - 8 % of the same lists, longer ones lose up to 2 %.
-  const bool one_each = use_mfma16 && kv_format == TTPA_KV_BF16 && head_size == 256 && !mask && !a.direct && segments >= 12 && g == 2 &&
+  // four per CU, 820, 900 and 1000 tiles of 16/8 heads 15.6 / 13.2, 15.9 / 13.7, 16.0 / 14.5; 760 and 1100 tiles 13.2 / 13.2 and 16.0 / 16.0; 780 ... 1000
+  // of 24/8 15.8 ... 16.6 / 13.9 ... 14.9, of 32/8 16.0 ... 17.1 / 14.4 ... 16.0.  More partials cost the merge more: not with wider groups (64/8 heads
+  // 17.1 ... 20.0 / 16.9 ... 20.2, 12 segments of 32/4 17.9 / 19.3) or where few segments have hundreds; above 64 users a list is cut by its
+  // units, which leave no tile a range of its own.  One head per group gains as much (7 users of 408 ... 707 tokens 16.3 / 14.2), but its kernel pays 1 %
+  // for the choice on every other list, and at 64 and 128, for 2 - 8 % of the same lists, longer ones lose up to 2 %.
+  const bool one_each = use_mfma16 && kv_format == TTPA_KV_BF16 && head_size == 256 && !mask && !a.direct && users <= kWave && segments >= 12 && g >= 2 && g <= 4 &&
                         segments * (seen / segment_tile_tokens(head_size) + 1) > waves_for_device(3.0);
   if (one_each) a.few_ranges = waves_for_device(3.0), a.few_from = (int64_t)waves_for_device(4.0) + 1, a.many_from = INT64_MAX;
   a.n_waves = waves_for_device(use_mfma16 && kv_format == TTPA_KV_BF16 && !one_each ? 3.0
