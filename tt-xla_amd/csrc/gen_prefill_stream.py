@@ -77,10 +77,13 @@ between the Q rows and the stored output rows: its first requests (K blocks 0..N
 caller's set-up), all blocks, the last PV, normalisation and store; then the next item's Q fragments
 and first requests go out in front of the store of the finished one.
 
-Matrix-to-vector hazards the hardware does not interlock are kept by construction: the vector
-instructions that read a score bank start two matrix instructions after the last one that wrote
-it (the mask waits explicitly); a bank of probabilities is rewritten three matrix instructions
-after the last one that read it; the slow path and the exit wait out the matrix pipe with s_nop.
+Matrix-to-vector hazards the hardware does not interlock are kept by construction and checked in the
+text of every form (check_distances): the vector instructions that read a score bank start two matrix
+instructions or more after the last one that wrote it (a result is there about a dozen wait states after
+its instruction, of which the next one's eight passes are eight; the mask waits explicitly); a register
+of probabilities is rewritten five matrix instructions (head size 64), ten (128) or nineteen (256) after
+the last one that read it, which read it as it started; the slow path and the exit wait out the
+matrix pipe with s_nop.
 """
 
 import re
@@ -883,6 +886,44 @@ def generate_first(f, suffix="", blocks=0):
     return o.lines
 
 
+READ_AFTER_WRITE, WRITE_AFTER_READ = 2, 2  # matrix instructions in between, at least (see the top)
+
+
+def vector_registers(operand):
+    """The numbers of the vector registers that an operand names."""
+    m = re.match(r"-?v(?:(\d+)|\[(\d+):(\d+)\])$", operand)
+    return range(0) if not m else range(int(m[1]), int(m[1]) + 1) if m[1] else range(int(m[2]), int(m[3]) + 1)
+
+
+def check_distances(f, lines):
+    """(fewest matrix instructions between the last write of a score register and a vector instruction that reads it, and between
+    the last read of a probability register and one that writes it) in the unrolled iterations, taken twice round.  The mask of a block, behind its
+    branch, waits by itself."""
+    top, end = lines.index("L_it1%=:"), lines.index("s_branch L_it1%=")
+    scores = {r for bank in f.S for r in range(bank, bank + 16)}
+    probabilities = {r for bank in f.P for r in range(bank, bank + 8)}
+    written, read, n, masked = {}, {}, 0, False
+    fewest = [len(lines), len(lines)]
+    for line in lines[top:end] * 2:
+        if line.startswith("s_cbranch_scc1 L_nomask"):
+            masked = True
+        if line.startswith("L_nomask"):
+            masked = False
+        name, _, rest = line.partition(" ")
+        operands = [x.strip() for x in rest.split(",")]
+        if name.startswith("v_mfma"):
+            n += 1
+            written.update((r, n) for r in vector_registers(operands[0]) if r in scores)
+            read.update((r, n) for r in vector_registers(operands[2]) if r in probabilities)
+        elif name.startswith("v_") and not masked:
+            for r in (r for x in operands[1:] for r in vector_registers(x) if r in written):
+                fewest[0] = min(fewest[0], n - written[r])
+            for r in (r for r in vector_registers(operands[0]) if r in read):
+                fewest[1] = min(fewest[1], n - read[r])
+    assert fewest[0] >= READ_AFTER_WRITE and fewest[1] >= WRITE_AFTER_READ, (f.name, fewest)
+    return tuple(fewest)
+
+
 def generate(f):
     o = Out()
     assert (f.ns, f.unroll) in ((5, 10), (4, 4))
@@ -967,6 +1008,7 @@ def generate(f):
         next_item(o, f)
     else:
         last_epilogue(o, f)
+    check_distances(f, o.lines)
     return o.lines
 
 
