@@ -142,20 +142,19 @@ __global__ __launch_bounds__(256) void bfp8_expand_kernel(ExpandArgs e) {
 // barrier too.  LDS operand reads run a few fragments ahead of the matrix instructions that
 // consume them.
 //
-// RH: blocks of 32 query rows per wavefront; only 1 is built (a form with two, one workgroup per
-// CU and every K / V fragment feeding two matrix instructions, measured slower: with one wavefront
-// per SIMD nobody fills the waits for fragments and barriers).
+// A wavefront has one block of 32 query rows, as workgroup_place and the parts know it (two, one workgroup per CU and every K / V
+// fragment feeding two matrix instructions, measured slower: with one wavefront per SIMD nobody fills the waits for fragments and barriers).
 //
 // SPLIT: the keys of a row block are shared by a.parts > 1 workgroups (prefill_parts.h).  A kernel of its own: with the parts' way
 // out as a run-time branch an unsplit launch was 0.1 ... 0.7 us longer than without (1 x 512 rows of 64 / 8 heads of 64 behind 512
 // tokens 28.3 / 27.7 us, 8 x 256 of 16 / 8 of 256 behind 512 55.3 / 54.3), and a split one 0.3 us (1 x 32 of 16 / 8 of 256 22.5 / 22.2).
-template <int RH>
-constexpr int prefill_wgs_per_cu(int d, int mode) { return RH == 1 && d <= 128 ? 2 : 1; }
+constexpr int prefill_wgs_per_cu(int d) { return d <= 128 ? 2 : 1; }
 
-template <int D, int HPW, int MODE, int RH, bool SPLIT>
-__global__ __launch_bounds__(256, prefill_wgs_per_cu<RH>(D, MODE)) void prefill_kernel(PrefillArgs a) {
+template <int D, int HPW, int MODE, bool SPLIT>
+__global__ __launch_bounds__(256, prefill_wgs_per_cu(D)) void prefill_kernel(PrefillArgs a) {
   constexpr int RPW = 4 / HPW;            // wavefront row slots per workgroup
-  constexpr int ROWS = kRowsPerWave * RH;  // query rows per wavefront
+  constexpr int RH = 1;                   // blocks of query rows per wavefront
+  constexpr int ROWS = kRowsPerWave * RH;
   constexpr int KSTEPS = D / 16;          // MFMA k-steps over the head dimension
   constexpr int DBLK = D / 32;            // 32-wide output blocks over the head dimension
   using T = Tile<D>;
@@ -207,7 +206,6 @@ __global__ __launch_bounds__(256, prefill_wgs_per_cu<RH>(D, MODE)) void prefill_
   }
 
   // ---- Q fragments (B operand: lane n = query row, 8 head-dim elements per k-step) -----
-  static_assert(RH == 1, "one block of 32 query rows per wavefront");
   bf16x8 qf[RH][KSTEPS];
 #pragma unroll
   for (int s = 0; s < KSTEPS; ++s) {
@@ -654,17 +652,17 @@ __global__ __launch_bounds__(256, prefill_wgs_per_cu<RH>(D, MODE)) void prefill_
   }
 }
 
-template <int D, int HPW, int MODE, int RH, bool SPLIT>
+template <int D, int HPW, int MODE, bool SPLIT>
 int launch_split(PrefillArgs &b, int grid, hipStream_t st) {
   const size_t lds = 2 * Tile<D>::STAGE_BYTES;  // two stages of a K and a V tile
   static std::atomic<uint64_t> lds_ready{0};
-  if (!ensure_dynamic_lds(reinterpret_cast<const void *>(&prefill_kernel<D, HPW, MODE, RH, SPLIT>), lds, lds_ready))
+  if (!ensure_dynamic_lds(reinterpret_cast<const void *>(&prefill_kernel<D, HPW, MODE, SPLIT>), lds, lds_ready))
     return fail(TTPA_ERR_LAUNCH, "prefill: cannot reserve %zu bytes of LDS", lds);
-  launch_dominant(&prefill_kernel<D, HPW, MODE, RH, SPLIT>, dim3(grid, b.parts), dim3(256), lds, st, b);
+  launch_dominant(&prefill_kernel<D, HPW, MODE, SPLIT>, dim3(grid, b.parts), dim3(256), lds, st, b);
   return check_launch("sdpa_prefill");
 }
 
-template <int D, int HPW, int MODE, int RH>
+template <int D, int HPW, int MODE>
 int launch_mode(const PrefillArgs &a, hipStream_t st) {
   PrefillArgs b = a;
   int grid = lay_out(b, HPW);
@@ -673,22 +671,22 @@ int launch_mode(const PrefillArgs &a, hipStream_t st) {
     constexpr SplitRule kRule = plain_split(D, MODE == 4);
     if (plain_splits(a) && a.part_acc && a.part_bytes >= part_bytes(a, HPW, kRule, D)) set_parts(b, HPW, kRule);
     if (b.parts > 1) {
-      if (const int rc = launch_split<D, HPW, MODE, RH, true>(b, grid, st)) return rc;
+      if (const int rc = launch_split<D, HPW, MODE, true>(b, grid, st)) return rc;
       prefill_merge_kernel<D><<<dim3((b.sq + kRowsPerWave - 1) / kRowsPerWave, b.hq, b.batch), dim3(2 * D), 0, st>>>(b);
       return check_launch("sdpa_prefill (merge of the parts)");
     }
   }
   if (MODE == 0 && a.fill_kc) grid = grid_with_fill(b, grid, D);
-  return launch_split<D, HPW, MODE, RH, false>(b, grid, st);
+  return launch_split<D, HPW, MODE, false>(b, grid, st);
 }
 
-template <int D, int HPW, int RH>
-int launch_rh(const PrefillArgs &a, hipStream_t st) {
+template <int D, int HPW>
+int launch_bf16(const PrefillArgs &a, hipStream_t st) {
   if (stream_serves(a, D)) return launch_stream(a, D, st);
-  if (!a.pt) return launch_mode<D, HPW, 0, RH>(a, st);
-  if (a.bs % kKeysPerTile == 0) return launch_mode<D, HPW, 1, RH>(a, st);
-  if (a.bs % Tile<D>::RPI == 0) return launch_mode<D, HPW, 3, RH>(a, st);
-  return launch_mode<D, HPW, 2, RH>(a, st);
+  if (!a.pt) return launch_mode<D, HPW, 0>(a, st);
+  if (a.bs % kKeysPerTile == 0) return launch_mode<D, HPW, 1>(a, st);
+  if (a.bs % Tile<D>::RPI == 0) return launch_mode<D, HPW, 3>(a, st);
+  return launch_mode<D, HPW, 2>(a, st);
 }
 
 template <int D, int HPW>
@@ -721,9 +719,9 @@ int launch(const PrefillArgs &a, hipStream_t st) {
       b.k = e.k, b.v = e.v, b.pt = e.table, b.pt_rs = a.w, b.nb = (int)blocks, b.kv_bfp8 = 0, b.expand = nullptr;
       return launch_stream(b, D, st);
     }
-    return launch_mode<D, HPW, 4, 1>(a, st);
+    return launch_mode<D, HPW, 4>(a, st);
   }
-  return launch_rh<D, HPW, 1>(a, st);
+  return launch_bf16<D, HPW>(a, st);
 }
 
 template <int D>
