@@ -660,7 +660,8 @@ def item_blocks(o):
 def normalise(o, f):
     """Normalises the item's accumulators and packs them: lane (n, h) holds, in accumulator
     register 16 db + 4 j + i, head-dim element 32 db + 8 j + 4 h + i of query row n, and ends with 16-byte chunk 4 db + 2 jp + h
-    of the row in registers S[0] + 8 db + 4 jp ..."""
+    of the row in registers S[0] + 8 db + 4 jp ...  (The plain loop divides; v_rcp_f32 and the product are within two units of float of
+    that, and the results are rounded to bfloat16, whose unit is 2^16 of those.)"""
     o.e(f"v_mov_b32 v{f.MB}, v{f.LRUN}")
     o.e("s_nop 1")
     o.e(f"v_permlane32_swap_b32 v{f.LRUN}, v{f.MB}")

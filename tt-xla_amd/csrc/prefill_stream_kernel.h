@@ -20,8 +20,8 @@ enum StreamForm { kDense = 0, kDenseWindow = 1, kPaged = 2, kPaged32 = 3, kDense
 
 // The assembly is bound to the registers its text names through constraint strings (both written by
 // gen_prefill_stream.py, with the names that the kernel below gives the values); everything else it
-// touches is on the clobber list.  The requests of a workgroup's first blocks are a block of assembly of their own, issued in front
-// of the Q loads so that the two round trips to memory overlap.  (Scalars only: with the per-lane
+// touches is on the clobber list.  The requests of a workgroup's first blocks are a block of assembly of their own, issued right
+// behind those of its Q rows so that the two round trips to memory overlap.  (Scalars only: with the per-lane
 // offsets in the same struct the compiler keeps the whole of it in vector registers.)
 struct StreamRequests {
   uint64_t kbase, vbase;       // dense: the first block of K / V; paged: the caches (both minus 1024 bytes)
@@ -158,7 +158,7 @@ __global__ __launch_bounds__(256, stream_wgs_per_cu(D)) void prefill_stream_kern
     }
   }
 
-  // ---- first requests, in front of the Q loads ----------------------------------------------------
+  // ---- first requests: the Q rows, then the first blocks -------------------------------------------
   StreamRequests req;
   constexpr int LOADS = D / 64;  // of a wavefront per block and tensor
   uint32_t lane_k[LOADS], lane_v[LOADS];
@@ -174,7 +174,8 @@ __global__ __launch_bounds__(256, stream_wgs_per_cu(D)) void prefill_stream_kern
   const auto ldk = Words<LOADS>::of(lane_k), ldv = Words<LOADS>::of(lane_v);
   // The wavefront's 32 Q rows, whole rows per load, go to the slot that K block ns - 1 (wavefront 0) or V block ns - 4 + wave takes later,
   // in the layout of a K block.  Loaded to registers by the lanes that hold them, 32 bytes of each of 32 rows per instruction, they cost a short pass
-  // 0.65 us more.
+  // 0.65 us more.  (Where three of four wavefronts have no rows, one head per KV head and prompts of 32, the second trip through LDS, of the output,
+  // outweighs that from five users on: 5 ... 8 x 32 tokens of 16 / 16 heads of 128 5.95 -> 6.05 us; 3 x 32 5.3 -> 5.05.)
   constexpr int SLOTS = TTPA_STREAM_SLOTS(D, WIDE);
   const int q_slot = (wave == 0 ? SLOTS - 1 : 2 * SLOTS - 4 + wave) * (kBlockKeys * T::RB);
   {
