@@ -389,12 +389,11 @@ using namespace ttpa::decode;
 // tokens, 2 - 6 % faster, 1.003: a wavefront's second tile shares its first one's maximum.
 static int segment_tile_tokens(int head_size) { return head_size <= 128 ? 4096 / head_size : 32; }
 static int direct_waves(int users, int kv_heads, int head_size, int kv_format, int64_t tokens, bool forced) {
+  const int64_t segments = (int64_t)users * kv_heads, bytes = tokens * head_size * (kv_format == TTPA_KV_BFP8 ? 2 : 4);
+  if (!forced && (head_size > 128 ? tokens > 256 : bytes > 272 * 1024)) return 0;  // (before the device is asked: a long context pays for no rule)
   int cus = device_cus();
   if (cus <= 0) cus = 256;
-  const int64_t segments = (int64_t)users * kv_heads;
   if (head_size > 128) return forced || (segments <= cus && tokens <= (2 * segments >= cus ? 256 : 128)) ? 4 : 0;
-  const int64_t bytes = tokens * head_size * (kv_format == TTPA_KV_BFP8 ? 2 : 4);
-  if (!forced && bytes > 272 * 1024) return 0;
   const int tile_tokens = segment_tile_tokens(head_size);
   return segments > cus || tokens <= 4 * tile_tokens ? 4 : 8;
 }
