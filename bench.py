@@ -52,10 +52,10 @@ MEASURED_TRAFFIC = {
     # workload: (kernel, hash of its sources, HBM bytes per launch: FETCH_SIZE and WRITE_SIZE of the
     # kernel, each scaled by what the same counter reads for a plain copy of known size, mean over
     # the rotating workload copies; the summaries under profiles/ hold the runs)
-    "config2": ("paged_decode_mfma16_kernel", "b05dcbf5a01a1cd1", 310428209),
-    "config5": ("paged_decode_mfma16_kernel", "b05dcbf5a01a1cd1", 169649630),
-    "config4": ("paged_decode_mfma16_kernel", "b05dcbf5a01a1cd1", 3415545175),
-    "config3": ("prefill_stream_kernel", "b6b6dbc7e8cc05b2", 233195745),
+    "config2": ("paged_decode_mfma16_kernel", "825dec6881a8b0dc", 310427720),
+    "config5": ("paged_decode_mfma16_kernel", "825dec6881a8b0dc", 169646686),
+    "config4": ("paged_decode_mfma16_kernel", "825dec6881a8b0dc", 3415544644),
+    "config3": ("prefill_stream_kernel", "77381a1fc5000224", 233177265),
     "latent": ("paged_decode_latent16_kernel", "5e6a63311c628267", 654182677),
     "latent128": ("paged_decode_latent128_kernel", "59aea2ac54ae75ed", 739351149),
     "latent-prefill": ("latent_prefill_kernel", "59aea2ac54ae75ed", 332224843),
