@@ -323,7 +323,8 @@ int ttpa_profile_next_attention(void *before, void *after);
  *   tt::chunked_scaled_dot_product_attention (custom_ops.py:1334-1431; CPU :1376-1429).
  *   out[b, hq, i, :] = softmax_j( scale * q[b,hq,i,:] . K[b, hq/G, j, :] + mask ) . V[b, hq/G, j, :]
  * Dense form: page_table == NULL, k / v are [batch, kv_heads, kv_len, head_size]
- *   addressed by the kv_* strides.
+ *   addressed by the kv_* strides (a token stride that is not negative, with 64 rows inside
+ *   4 GiB).
  * Paged form: page_table != NULL, k / v are caches (bf16 layout above), kv_len is
  *   ignored and the keys of user b are positions 0 .. table_width*block_size-1.
  * Masking: causal != 0 allows key j for query row i iff j <= offset + i, where offset
@@ -512,7 +513,7 @@ int ttpa_latent_prefill(void *out, int64_t out_batch_stride, int64_t out_head_st
  * have been expanded per head (head_size 192, head_dim_v 128; a k_rope that the heads share has head
  * stride 0), and tt::flash_mla_prefill with a V of its own at that size (reference custom_ops.py:223-378).
  * All operands bfloat16 [batch, heads, seq_len, part] by element strides (multiples of 8, out's of 4; innermost
- * dimension contiguous); seq_len a multiple of 32.
+ * dimension contiguous; out's, k's and v's token strides are not negative); seq_len a multiple of 32.
  */
 int ttpa_split_key_prefill(void *out, int64_t out_batch_stride, int64_t out_head_stride, int64_t out_token_stride,
                            const void *q_nope, int64_t q_nope_batch_stride, int64_t q_nope_head_stride,

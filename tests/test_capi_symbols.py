@@ -63,6 +63,14 @@ def test_split_key_prefill_refuses_descending_rows(native):
         assert rc == native.ERR_INVALID_ARGUMENT and b"token stride" in lib.ttpa_last_error()
 
 
+@pytest.mark.parametrize("stride, kv_len", [(-128, 2), (-128, 4096), (1 << 31, 2), (1 << 26, 33), (1 << 26, 64), (34087040, 64)])
+def test_dense_prefill_refuses_key_rows_beyond_its_distances(native, stride, kv_len):
+    """K / V rows of a tile of 64 are reached by unsigned 32-bit numbers of bytes; nothing else is wrong with these calls."""
+    lib = native.lib()
+    args = [16, 128 * 64, 128, 128, 16, 128 * 64, 128, 128, 16, 16, 128, 128, stride, None, 0, None, None, 0, 0, 1, 1, 1, 32, kv_len, 128, 0, 0, 0]
+    assert lib.ttpa_sdpa_prefill(*args, 1, 1.0, None) == native.ERR_INVALID_ARGUMENT and b"token stride" in lib.ttpa_last_error()
+
+
 def test_workspace_size_is_positive_and_monotone(native):
     lib = native.lib()
     a = lib.ttpa_paged_decode_workspace_bytes(32, 32, 8, 128)

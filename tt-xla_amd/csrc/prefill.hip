@@ -786,6 +786,10 @@ static int prefill_impl(void *out, int64_t out_batch_stride, int64_t out_head_st
     TTPA_REQUIRE(kv_len > 0, "dense form needs kv_len > 0");
     TTPA_REQUIRE(kv_batch_stride % 8 == 0 && kv_head_stride % 8 == 0 && kv_token_stride % 8 == 0,
                  "prefill: k / v strides must be multiples of 8 elements");
+    // (both loops reach a tile's rows by unsigned 32-bit numbers of bytes from the first)
+    TTPA_REQUIRE(kv_len == 1 || (kv_token_stride >= 0 && kv_token_stride < (1ll << 31) &&
+                                 (std::min(kv_len, 64) - 1) * kv_token_stride < (1ll << 31) - 1024),
+                 "prefill: k / v token stride %lld is negative, or a tile of 64 rows reaches over 4 GiB", (long long)kv_token_stride);
     TTPA_REQUIRE(chunk_start == nullptr, "chunk_start applies to the paged form only");
   }
   TTPA_REQUIRE(aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out),
