@@ -1,6 +1,6 @@
-"""The cache rows that a dense prefill writes beside its attention, around the lengths at which its workgroups take another quarter of their
-passes (128 rows, 64 at head size 256) and another workgroup starts (512, 256): copied bit for bit, and no others touched.  The kernel is the same
-on the plain loop, which takes the lengths that are no multiple of 32."""
+"""The cache rows that a dense prefill writes beside its attention, around the length up to which its workgroups take a quarter of their
+passes (128 rows, but for head size 256) and those at which another workgroup starts (512, 256): copied bit for bit, and no others touched.  The
+fill is the same on the plain loop, which takes the lengths that are no multiple of 32."""
 
 import pytest
 import torch

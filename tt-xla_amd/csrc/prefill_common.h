@@ -195,16 +195,17 @@ __device__ __forceinline__ void fill_workgroup(const PrefillArgs &a, int f) {
   // every load (rows and table entries) is requested before the first store: the compiler
   // cannot move a load across a store that might alias it, and a table entry per pass would
   // otherwise cost a round trip each
-  // A quarter of the passes at a time, as far as the prompt has rows: the whole of them, 30 of 32 the last row of a prompt of 32 tokens again, were a
-  // fifth of a short launch once it has more workgroups than the chip CUs (16 / 16 heads of 128, 5 x 32 tokens 5.8 -> 4.9 us, 8 x 32 5.95 -> 5.0, 8 x 64
-  // 6.0 -> 5.7; 4 x 32, with a CU for each, 4.9, 8 x 128 and more rows as before).  A branch per pass cost long prompts 0.3 %.
+  // A prompt of a quarter of the passes takes no more: 30 of 32 were the last row of 32 tokens again, and a fifth of a short launch that has more
+  // workgroups than there are CUs (16 / 16 heads of 128, 5 x 32 tokens 5.8 -> 4.9 us, 8 x 32 5.95 -> 5.0, 8 x 64 6.0 -> 5.7; 4 x 32, with a CU for each,
+  // 4.9).  Not so for the rest of longer ones, whose attention workgroups start less well behind fills that end early: 7 x 256 13.0 / 13.2, 7 x 640
+  // 35.0 / 35.3, 4 x 640 of 16 / 8 heads of 256 39.3 / 40.1; nor at 256, where a CU has one workgroup: 8 x 64 7.73 / 7.80.
   constexpr int NQ = NP / 4;
-  const int rows = a.skv - c0 * kFillRows;
+  const int quarters = D <= 128 && a.skv <= NQ * RPP ? 1 : 4;
   u32x4 val[NP];
   int phys[NP];
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    if (q * NQ * RPP >= rows) break;
+    if (q >= quarters) break;
 #pragma unroll
     for (int p = q * NQ; p < (q + 1) * NQ; ++p) {
       const int t = min(t0 + p * RPP, a.skv - 1);
@@ -214,7 +215,7 @@ __device__ __forceinline__ void fill_workgroup(const PrefillArgs &a, int f) {
   }
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    if (q * NQ * RPP >= rows) break;
+    if (q >= quarters) break;
 #pragma unroll
     for (int p = q * NQ; p < (q + 1) * NQ; ++p) {
       const int t = t0 + p * RPP;
