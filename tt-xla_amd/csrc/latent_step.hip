@@ -277,14 +277,16 @@ struct ExpandArgs {
   int items;                 // workgroups behind them write rows of the cache, 8 threads to a row
 };
 
-// Steps of 64 latent values in a ring of two where the second round of the chip's 512 places is more than half full: whole 128-byte lines per request
-// instead of halves, which is worth more there than three steps on their way; with fewer workgroups the last ones have the chip to themselves, and what
-// each has on its way counts.  us per pass, steps of 32 / 64 (workgroups): 16 heads, 2 x 1568 tokens 62.9 / 61.1 (800), 2 x 1760 71.1 / 69.6 (896), 2 x 2048
-// 88.3 / 86.6 (1024), 3 x 1824 107.7 / 105.1 (1376), 4 x 2048 150.5 / 148.9 (2048; from card to card 145.0 / 149.3 to 150.6 / 147.9), 32 heads, 3 x 832 69.1 / 67.1
-// (1280), 128 heads, 1 x 416 46.6 / 44.7 (1024).  Below: 16 heads, 1 x 96 12.5 / 12.9 (32), 1 x 1280 39.2 / 38.6 (320), 1 x 1920 51.6 / 51.6 (480), 2 x 1024 38.6 / 40.6 (512),
-// 2 x 1088 45.0 / 46.6 (544), 1 x 2432 70.9 / 74.5 (608), 2 x 1440 58.3 / 58.4 (720), 32 heads, 4 x 256 27.0 / 28.3 (512), 128 heads, 1 x 352 37.5 / 38.2 (768).
-// 256 tokens per workgroup with steps of 32 or 64: 4 x 2048 the kernel alone 43.3 and 48.2 us against 45.4 and 41.7 (the two above), 1 x 480
-// 9.7 and 10.3 against 6.2 and 8.1.
+// Steps of 64 latent values in a ring of two where workgroups share CUs, in most of one round of the chip's 512 places or in two with the second more than
+// half full: whole 128-byte lines per request instead of halves, which is worth more there than three steps on their way; a workgroup with a CU to itself, all
+// of them up to 256 and the last ones of a launch that is a little over a round (the cache rows' workgroups come on top), depends on what it has on its
+// way.  us per pass, steps of 32 / 64 (workgroups), / on another card: 16 heads, 1 x 1152 tokens 36.8 / 36.1, 37.7 / 36.1 (288), 4 x 320 24.1 / 23.4, 24.7 / 23.8 (320),
+// 1 x 1536 43.9 / 43.4 (384), 4 x 448 27.2 / 26.2 (448); 2 x 1568 62.9 / 61.1 (800), 2 x 1760 71.1 / 69.6 (896), 2 x 2048 88.3 / 86.6 (1024), 3 x 1824 107.7 / 105.1 (1376),
+// 4 x 2048 150.5 / 148.9, 145.0 / 149.3 (2048), 32 heads, 3 x 832 69.1 / 67.1 (1280), 128 heads, 1 x 416 46.6 / 44.7 (1024).  Neither: 16 heads, 1 x 96 12.5 / 12.9 (32),
+// 1 x 512 21.3 / 22.3 (128), 1 x 896 28.9 / 29.9 (224); 1 x 1920 51.6 / 51.6, 50.6 / 49.8 (480), 2 x 1024 38.6 / 40.6,
+// 36.2 / 36.1 (512), 2 x 1088 45.0 / 46.6, 43.3 / 43.1 (544), 1 x 2432 70.9 / 74.5, 67.4 / 67.6 (608), 2 x 1440 58.3 / 58.4 (720), 32 heads, 4 x 256 27.0 / 28.3, 25.4 / 25.4
+// (512), 128 heads, 1 x 352 37.5 / 38.2 (768).  256 tokens per workgroup with steps of 32 or 64: 4 x 2048 the kernel alone 43.3 and 48.2 us against 45.4 and 41.7
+// (the two above), 1 x 480 9.7 and 10.3 against 6.2 and 8.1.
 constexpr int kExpTokens = 128;
 template <int STEP, int STAGES>
 struct ExpandShape {
@@ -619,8 +621,8 @@ extern "C" int ttpa_latent_prompt(void *out, int64_t out_token_stride, int64_t o
     e.k = reinterpret_cast<uint16_t *>(ws), e.v = reinterpret_cast<uint16_t *>(ws + align256((size_t)rows * heads * 256));
     e.uk_rows = !uk_columns, e.uv_rows = uv_columns;
     e.items = (int)(token_tiles * 2 * heads);
-    const bool fills = e.items >= 800;  // (of 512 places: ExpandShape)
-    if (int rc = fills ? launch_expand<ExpandShape<64, 2>>(e, st) : launch_expand<ExpandShape<32, 4>>(e, st)) return rc;
+    const bool shared = (e.items > 256 && e.items < 480) || e.items >= 800;  // (of 512 places, two on a CU: ExpandShape)
+    if (int rc = shared ? launch_expand<ExpandShape<64, 2>>(e, st) : launch_expand<ExpandShape<32, 4>>(e, st)) return rc;
     const int64_t hd = (int64_t)heads * 128, sl = seq_len;
     return ttpa_split_key_prefill(out, sl * out_token_stride, out_head_stride, out_token_stride, q_nope, sl * q_nope_token_stride,
                                   q_nope_head_stride, q_nope_token_stride, q_rope, sl * q_rope_token_stride, q_rope_head_stride,
