@@ -55,7 +55,7 @@ MEASURED_TRAFFIC = {
     "config2": ("paged_decode_mfma16_kernel", "825dec6881a8b0dc", 310427720),
     "config5": ("paged_decode_mfma16_kernel", "825dec6881a8b0dc", 169646686),
     "config4": ("paged_decode_mfma16_kernel", "825dec6881a8b0dc", 3415544644),
-    "config3": ("prefill_stream_kernel", "77381a1fc5000224", 233177265),
+    "config3": ("prefill_stream_kernel", "ec3db3393ba4b856", 233202960),
     "latent": ("paged_decode_latent16_kernel", "5e6a63311c628267", 654182677),
     "latent128": ("paged_decode_latent128_kernel", "59aea2ac54ae75ed", 739351149),
     "latent-prefill": ("latent_prefill_kernel", "59aea2ac54ae75ed", 332224843),

@@ -175,7 +175,7 @@ __global__ __launch_bounds__(256, stream_wgs_per_cu(D)) void prefill_stream_kern
   // The wavefront's 32 Q rows, whole rows per load, go to the slot that K block ns - 1 (wavefront 0) or V block ns - 4 + wave takes later,
   // in the layout of a K block.  Loaded to registers by the lanes that hold them, 32 bytes of each of 32 rows per instruction, they cost a short pass
   // 0.65 us more.  (Where three of four wavefronts have no rows, one head per KV head and prompts of 32, the second trip through LDS, of the output,
-  // outweighs that from five users on: 5 ... 8 x 32 tokens of 16 / 16 heads of 128 5.95 -> 6.05 us; 3 x 32 5.3 -> 5.05.)
+  // cost as much again from five users on: 5 x 32 tokens of 16 / 16 heads of 128 5.72 / 5.80 us, 3 x 32 5.15 / 4.85.)
   constexpr int SLOTS = TTPA_STREAM_SLOTS(D, WIDE);
   const int q_slot = (wave == 0 ? SLOTS - 1 : 2 * SLOTS - 4 + wave) * (kBlockKeys * T::RB);
   {
